@@ -35,34 +35,56 @@ __device__ __forceinline__ uint32_t hash3(uint32_t a, uint32_t b, uint32_t c) {
   return h;
 }
 
-__global__ void __launch_bounds__(256) sample_partial_kernel(
-    float* __restrict__ pv, i32* __restrict__ pi, const u16* __restrict__ logits,
-    const float* __restrict__ temp, const uint32_t* __restrict__ step,
-    uint32_t seed, int V) {
-  const int b = blockIdx.x, split = blockIdx.y;
-  const int chunk = (V + SMP_SPLITS - 1) / SMP_SPLITS;
-  const int v0 = split * chunk, v1 = min(V, v0 + chunk);
-  const float t = temp[b];
-  const float invt = (t > 0.f) ? 1.f / t : 0.f;
-  const uint32_t st = *step;
-
-  float best = AF_NEG_INF;
-  int bidx = 0;
-  const u16* row = logits + (size_t)b * V;
-  for (int v = v0 + threadIdx.x; v < v1; v += 256) {
-    float x = bf2f(row[v]);
-    if (t > 0.f) {
-      const float u = u32_to_unit(hash3(seed ^ st, (uint32_t)b, (uint32_t)v));
-      x = x * invt + gumbel_of(u);
+// Rows are read 16 bytes per lane.  V need not be a multiple of 8 (nor the row
+// 16-byte aligned: an odd V shifts every row), so up to 7 values in front of
+// the first 16-byte boundary and up to 7 behind the last go one by one, to
+// split 0.  Four loads are in flight per thread: a split is ~1000 vectors at
+// V = 128k, i.e. one round trip to memory instead of four.
+template <class F>
+__device__ __forceinline__ void each_logit(const u16* __restrict__ row, int V,
+                                           int split, int nsplit, F f) {
+  const int head =
+      min(V, (int)(((16u - ((uint32_t)(uintptr_t)row & 15u)) & 15u) >> 1));
+  const int nvec = (V - head) >> 3;
+  const int per = (nvec + nsplit - 1) / nsplit;
+  const int i0 = split * per, i1 = min(nvec, i0 + per);
+  const u16* body = row + head;
+  for (int i = i0 + (int)threadIdx.x; i < i1; i += 4 * 256) {
+    s16x8 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      v[u] = *reinterpret_cast<const s16x8*>(
+          body + (size_t)min(i + u * 256, i1 - 1) * 8);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (i + u * 256 >= i1) break;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        f(bf2f((u16)v[u][j]), head + (i + u * 256) * 8 + j);
     }
-    if (x > best) { best = x; bidx = v; }
   }
-  // wave then block argmax
+  if (split == 0) {
+    const int t = threadIdx.x, tail = head + nvec * 8;
+    if (t < head) f(bf2f(row[t]), t);
+    if (tail + t < V) f(bf2f(row[tail + t]), tail + t);
+  }
+}
+
+// Larger value wins, equal values go to the smaller index: the order in which
+// threads and splits see a row does not matter.
+__device__ __forceinline__ void take_best(float ov, int oi, float& best,
+                                          int& bidx) {
+  if (ov > best || (ov == best && oi < bidx)) { best = ov; bidx = oi; }
+}
+
+__device__ __forceinline__ void store_best(float best, int bidx,
+                                           float* __restrict__ pv,
+                                           i32* __restrict__ pi, int at) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     const float ov = __shfl_xor(best, o, 64);
     const int oi = __shfl_xor(bidx, o, 64);
-    if (ov > best || (ov == best && oi < bidx)) { best = ov; bidx = oi; }
+    take_best(ov, oi, best, bidx);
   }
   __shared__ float sv[4];
   __shared__ int si[4];
@@ -71,31 +93,53 @@ __global__ void __launch_bounds__(256) sample_partial_kernel(
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int w = 1; w < 4; ++w)
-      if (sv[w] > best || (sv[w] == best && si[w] < bidx)) { best = sv[w]; bidx = si[w]; }
-    pv[b * SMP_SPLITS + split] = best;
-    pi[b * SMP_SPLITS + split] = bidx;
+    for (int w = 1; w < 4; ++w) take_best(sv[w], si[w], best, bidx);
+    pv[at] = best;
+    pi[at] = bidx;
   }
 }
 
-__global__ void __launch_bounds__(64) sample_combine_kernel(
-    i32* __restrict__ out, const float* __restrict__ pv, const i32* __restrict__ pi) {
-  const int b = blockIdx.x;
-  if (threadIdx.x != 0) return;
+__global__ void __launch_bounds__(256) sample_partial_kernel(
+    float* __restrict__ pv, i32* __restrict__ pi, const u16* __restrict__ logits,
+    const float* __restrict__ temp, const uint32_t* __restrict__ step,
+    uint32_t seed, int V) {
+  const int b = blockIdx.x, split = blockIdx.y;
+  const float t = temp[b];
+  const float invt = (t > 0.f) ? 1.f / t : 0.f;
+  const uint32_t st = *step;
   float best = AF_NEG_INF;
   int bidx = 0;
-  for (int s = 0; s < SMP_SPLITS; ++s) {
-    const float v = pv[b * SMP_SPLITS + s];
-    if (v > best || (v == best && pi[b * SMP_SPLITS + s] < bidx)) {
-      best = v;
-      bidx = pi[b * SMP_SPLITS + s];
+  each_logit(logits + (size_t)b * V, V, split, SMP_SPLITS, [&](float x, int v) {
+    if (t > 0.f) {
+      const float u = u32_to_unit(hash3(seed ^ st, (uint32_t)b, (uint32_t)v));
+      x = x * invt + gumbel_of(u);
     }
-  }
-  out[b] = bidx;
+    if (x > best || (x == best && v < bidx)) { best = x; bidx = v; }
+  });
+  store_best(best, bidx, pv, pi, b * SMP_SPLITS + split);
 }
 
-__global__ void step_inc_kernel(uint32_t* step) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *step += 1u;
+// The last kernel of a draw: every reader of *step has finished, so it also
+// moves the counter (one launch less, ~4.6 us each in a captured step).
+__global__ void __launch_bounds__(64) sample_combine_kernel(
+    i32* __restrict__ out, const float* __restrict__ pv,
+    const i32* __restrict__ pi, uint32_t* __restrict__ step) {
+  const int b = blockIdx.x;
+  float best = AF_NEG_INF;
+  int bidx = 0;
+  if (threadIdx.x < SMP_SPLITS)
+    take_best(pv[b * SMP_SPLITS + threadIdx.x],
+              pi[b * SMP_SPLITS + threadIdx.x], best, bidx);
+#pragma unroll
+  for (int o = SMP_SPLITS / 2; o > 0; o >>= 1) {
+    const float ov = __shfl_xor(best, o, 64);
+    const int oi = __shfl_xor(bidx, o, 64);
+    take_best(ov, oi, best, bidx);
+  }
+  if (threadIdx.x == 0) {
+    out[b] = bidx;
+    if (b == 0) *step += 1u;
+  }
 }
 
 // ---- top-k / top-p restriction --------------------------------------------
@@ -104,155 +148,186 @@ __global__ void step_inc_kernel(uint32_t* step) {
 // or top-p probability mass is reached; the Gumbel-max draw then ignores
 // logits below the threshold.  Boundary-bin granularity is SPAN/256 ~ 0.08
 // logits — the standard approximation for GPU nucleus sampling.
+//
+// Every pass runs SMP_SPLITS blocks per row: a row is 256 KB, and one block a
+// row (64 of them on 256 CUs, one bin conflict after the other) took 173 us
+// for the histogram and 52 us for the maximum at 64 x 128256.  The passes after
+// the first fold the per-split results of the pass before in their prologue, so
+// nothing but the four reads of the row is launched: 346 us -> 28 us.
 #define TKP_BINS 256
 #define TKP_SPAN 20.0f
 
-// pass A: row max (reuses partial scratch pv/pi from the argmax machinery)
+// pass A: maximum of each split
 __global__ void __launch_bounds__(256) row_max_kernel(
     float* __restrict__ rmax, const u16* __restrict__ logits, int V) {
-  const int b = blockIdx.x;
+  const int b = blockIdx.x, split = blockIdx.y;
   float best = AF_NEG_INF;
-  const u16* row = logits + (size_t)b * V;
-  for (int v = threadIdx.x; v < V; v += 256) best = fmaxf(best, bf2f(row[v]));
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) best = fmaxf(best, __shfl_xor(best, o, 64));
+  each_logit(logits + (size_t)b * V, V, split, SMP_SPLITS,
+             [&](float x, int) { best = fmaxf(best, x); });
+  best = wave_max_f32(best);
   __shared__ float sv[4];
   if ((threadIdx.x & 63) == 0) sv[threadIdx.x >> 6] = best;
   __syncthreads();
   if (threadIdx.x == 0)
-    rmax[b] = fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));
+    rmax[b * SMP_SPLITS + split] =
+        fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3]));
 }
 
-// pass B: histogram of counts and exp-mass per bin (temperature applied)
+__device__ __forceinline__ float row_max_of(const float* __restrict__ rmax,
+                                            int b) {
+  float m = rmax[b * SMP_SPLITS];
+#pragma unroll
+  for (int s = 1; s < SMP_SPLITS; ++s)
+    m = fmaxf(m, rmax[b * SMP_SPLITS + s]);
+  return m;
+}
+
+// pass B: histogram of counts and exp-mass per bin (temperature applied) of
+// each split.  What bounds it is LDS atomics: at 64 x 128256 a float add per
+// value takes 41 us and an integer one 2 us, whatever the conflicts.  So a value
+// adds one 64-bit integer: 1 in the upper 20 bits, and below them its mass
+// relative to its bin's upper edge (0.92..1) in units of 2^-24, which loses no
+// more per value than a float does and nothing in the sum.  Every bin has 16
+// copies, one per lane of a group of 16, which also keeps a count within its
+// field for rows of up to 2^28 values (45 us -> 8 us).
+#define TKP_COPIES 16
+#define TKP_MASS_BITS 44
 __global__ void __launch_bounds__(256) tkp_hist_kernel(
     i32* __restrict__ hist_n, float* __restrict__ hist_m,
     const u16* __restrict__ logits, const float* __restrict__ rmax,
     const float* __restrict__ temp, int V) {
-  const int b = blockIdx.x;
-  __shared__ i32 hn[TKP_BINS];
-  __shared__ float hm[TKP_BINS];
-  for (int i = threadIdx.x; i < TKP_BINS; i += 256) { hn[i] = 0; hm[i] = 0.f; }
+  const int b = blockIdx.x, split = blockIdx.y;
+  const int copy = threadIdx.x & (TKP_COPIES - 1);
+  __shared__ unsigned long long h[TKP_BINS * TKP_COPIES];
+#pragma unroll
+  for (int c = 0; c < TKP_COPIES; ++c) h[c * 256 + threadIdx.x] = 0;
   __syncthreads();
   const float t = temp[b];
   const float invt = (t > 0.f) ? 1.f / t : 1.f;
-  const float mx = rmax[b] * invt;
-  const u16* row = logits + (size_t)b * V;
-  for (int v = threadIdx.x; v < V; v += 256) {
-    const float x = bf2f(row[v]) * invt;
+  const float mx = row_max_of(rmax, b) * invt;
+  constexpr float STEP = TKP_SPAN / TKP_BINS;
+  bool odd = false;  // a value that is not a number makes the mass one too
+  each_logit(logits + (size_t)b * V, V, split, SMP_SPLITS, [&](float l, int) {
+    const float x = l * invt;
+    odd |= (x - mx) != (x - mx);
     int bin = (int)((x - (mx - TKP_SPAN)) * (TKP_BINS / TKP_SPAN));
-    if (bin < 0) continue;  // below span: negligible mass
+    if (bin < 0) return;  // below span: negligible mass
     if (bin > TKP_BINS - 1) bin = TKP_BINS - 1;
-    atomicAdd(&hn[bin], 1);
-    atomicAdd(&hm[bin], __expf(x - mx));
+    const float r = __expf(x - mx + (float)(TKP_BINS - 1 - bin) * STEP);
+    atomicAdd(&h[bin * TKP_COPIES + copy],
+              (1ull << TKP_MASS_BITS) +
+                  (unsigned long long)(uint32_t)(r * 16777216.f + 0.5f));
+  });
+  odd = __syncthreads_or(odd);
+  const int first = threadIdx.x * TKP_COPIES;
+  int n = 0;
+  unsigned long long m = 0;
+#pragma unroll
+  for (int c = 0; c < TKP_COPIES; ++c) {
+    const unsigned long long q =
+        h[first + ((c + threadIdx.x) & (TKP_COPIES - 1))];
+    n += (int)(q >> TKP_MASS_BITS);
+    m += q & ((1ull << TKP_MASS_BITS) - 1);
   }
-  __syncthreads();
-  for (int i = threadIdx.x; i < TKP_BINS; i += 256) {
-    hist_n[b * TKP_BINS + i] = hn[i];
-    hist_m[b * TKP_BINS + i] = hm[i];
-  }
+  const size_t at = ((size_t)b * SMP_SPLITS + split) * TKP_BINS + threadIdx.x;
+  hist_n[at] = n;
+  hist_m[at] = odd ? __builtin_nanf("")
+                   : __expf((float)((int)threadIdx.x - (TKP_BINS - 1)) * STEP) *
+                         ((float)m * (1.f / 16777216.f));
 }
 
-// pass C: per row, walk bins from the top until top-k count / top-p mass is
-// covered -> threshold (in temperature-scaled logit space)
-__global__ void __launch_bounds__(64) tkp_threshold_kernel(
-    float* __restrict__ thresh, const i32* __restrict__ hist_n,
-    const float* __restrict__ hist_m, const float* __restrict__ rmax,
-    const float* __restrict__ temp, const i32* __restrict__ topk,
-    const float* __restrict__ topp, int V) {
-  const int b = blockIdx.x;
-  if (threadIdx.x != 0) return;
-  const float t = temp[b];
-  const float invt = (t > 0.f) ? 1.f / t : 1.f;
-  const float mx = rmax[b] * invt;
-  float total = 0.f;
-  for (int i = 0; i < TKP_BINS; ++i) total += hist_m[b * TKP_BINS + i];
-  const int k = (topk[b] > 0) ? topk[b] : V;
-  const float p = (topp[b] > 0.f && topp[b] < 1.f) ? topp[b] : 1.f;
-  if (k == 1) {  // exact: only the argmax survives
-    thresh[b] = mx;
-    return;
-  }
+// The threshold of a row (in temperature-scaled logit space): bins from the
+// top until top-k count / top-p mass is covered.  Thread i holds bin 255 - i;
+// an inclusive scan over the block gives count and mass down to that bin.
+__device__ __forceinline__ float tkp_threshold(
+    const i32* __restrict__ hist_n, const float* __restrict__ hist_m,
+    float mx, int k, float p, int b) {
+  const int i = threadIdx.x, lane = i & 63, wid = i >> 6;
+  const size_t at = (size_t)b * SMP_SPLITS * TKP_BINS + (TKP_BINS - 1 - i);
   int cnt = 0;
   float mass = 0.f;
-  float th = mx - TKP_SPAN;
-  for (int i = TKP_BINS - 1; i >= 0; --i) {
-    cnt += hist_n[b * TKP_BINS + i];
-    mass += hist_m[b * TKP_BINS + i];
-    if (cnt >= k || mass >= p * total) {
-      th = mx - TKP_SPAN + (float)i * (TKP_SPAN / TKP_BINS);
-      break;
-    }
+#pragma unroll
+  for (int s = 0; s < SMP_SPLITS; ++s) {
+    cnt += hist_n[at + s * TKP_BINS];
+    mass += hist_m[at + s * TKP_BINS];
   }
-  thresh[b] = th;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int c = __shfl_up(cnt, o, 64);
+    const float m = __shfl_up(mass, o, 64);
+    if (lane >= o) { cnt += c; mass += m; }
+  }
+  __shared__ i32 wc[4];
+  __shared__ float wm[4];
+  __shared__ i32 hit[4];
+  if (lane == 63) { wc[wid] = cnt; wm[wid] = mass; }
+  __syncthreads();
+  float total = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    if (w < wid) { cnt += wc[w]; mass += wm[w]; }
+    total += wm[w];
+  }
+  const unsigned long long full = __ballot(cnt >= k || mass >= p * total);
+  if (lane == 0) hit[wid] = full ? wid * 64 + (int)__ffsll(full) - 1 : TKP_BINS;
+  __syncthreads();
+  const int first = min(min(hit[0], hit[1]), min(hit[2], hit[3]));
+  if (k == 1) return mx;  // exact: only the argmax survives
+  return first < TKP_BINS
+             ? mx - TKP_SPAN + (float)(TKP_BINS - 1 - first) *
+                                   (TKP_SPAN / TKP_BINS)
+             : mx - TKP_SPAN;
 }
 
-// pass D: Gumbel-argmax over {x/T >= thresh}
+// pass C: Gumbel-argmax over {x/T >= threshold}
 __global__ void __launch_bounds__(256) tkp_sample_kernel(
     float* __restrict__ pv, i32* __restrict__ pi, const u16* __restrict__ logits,
-    const float* __restrict__ temp, const float* __restrict__ thresh,
+    const float* __restrict__ temp, const float* __restrict__ rmax,
+    const i32* __restrict__ hist_n, const float* __restrict__ hist_m,
+    const i32* __restrict__ topk, const float* __restrict__ topp,
     const uint32_t* __restrict__ step, uint32_t seed, int V) {
   const int b = blockIdx.x, split = blockIdx.y;
-  const int chunk = (V + SMP_SPLITS - 1) / SMP_SPLITS;
-  const int v0 = split * chunk, v1 = min(V, v0 + chunk);
   const float t = temp[b];
   const float invt = (t > 0.f) ? 1.f / t : 1.f;
-  const float th = thresh[b];
+  const int k = (topk[b] > 0) ? topk[b] : V;
+  const float p = (topp[b] > 0.f && topp[b] < 1.f) ? topp[b] : 1.f;
+  const float th =
+      tkp_threshold(hist_n, hist_m, row_max_of(rmax, b) * invt, k, p, b);
   const uint32_t st = *step;
   float best = AF_NEG_INF;
   int bidx = 0;
-  const u16* row = logits + (size_t)b * V;
-  for (int v = v0 + threadIdx.x; v < v1; v += 256) {
-    float x = bf2f(row[v]) * invt;
-    if (x < th) continue;
+  each_logit(logits + (size_t)b * V, V, split, SMP_SPLITS, [&](float l, int v) {
+    float x = l * invt;
+    if (x < th) return;
     if (t > 0.f) {
       const float u = u32_to_unit(hash3(seed ^ st, (uint32_t)b, (uint32_t)v));
       x += gumbel_of(u);
     }
-    if (x > best) { best = x; bidx = v; }
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(best, o, 64);
-    const int oi = __shfl_xor(bidx, o, 64);
-    if (ov > best || (ov == best && oi < bidx)) { best = ov; bidx = oi; }
-  }
-  __shared__ float sv[4];
-  __shared__ int si[4];
-  if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = best; si[threadIdx.x >> 6] = bidx; }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int w = 1; w < 4; ++w)
-      if (sv[w] > best || (sv[w] == best && si[w] < bidx)) { best = sv[w]; bidx = si[w]; }
-    pv[b * SMP_SPLITS + split] = best;
-    pi[b * SMP_SPLITS + split] = bidx;
-  }
+    if (x > best || (x == best && v < bidx)) { best = x; bidx = v; }
+  });
+  store_best(best, bidx, pv, pi, b * SMP_SPLITS + split);
 }
 
-// scratch layout for af_sample_topkp: caller provides rmax [B], thresh [B],
-// hist_n [B,256] i32, hist_m [B,256] f32 in addition to pv/pi.
+// scratch of af_sample_topkp besides pv / pi: rmax [B, 16] f32,
+// hist_n [B, 16, 256] i32, hist_m [B, 16, 256] f32.
 AF_EXPORT int af_sample_topkp(void* out, void* pv, void* pi, void* rmax,
-                              void* thresh, void* hist_n, void* hist_m,
-                              const void* logits, const void* temp,
-                              const void* topk, const void* topp, void* step,
-                              uint32_t seed, int B, int V, void* stream) {
+                              void* hist_n, void* hist_m, const void* logits,
+                              const void* temp, const void* topk,
+                              const void* topp, void* step, uint32_t seed,
+                              int B, int V, void* stream) {
   if (B == 0) return 0;
   hipStream_t st = (hipStream_t)stream;
-  row_max_kernel<<<B, 256, 0, st>>>((float*)rmax, (const u16*)logits, V);
-  tkp_hist_kernel<<<B, 256, 0, st>>>((i32*)hist_n, (float*)hist_m,
+  dim3 g(B, SMP_SPLITS);
+  row_max_kernel<<<g, 256, 0, st>>>((float*)rmax, (const u16*)logits, V);
+  tkp_hist_kernel<<<g, 256, 0, st>>>((i32*)hist_n, (float*)hist_m,
                                      (const u16*)logits, (const float*)rmax,
                                      (const float*)temp, V);
-  tkp_threshold_kernel<<<B, 64, 0, st>>>(
-      (float*)thresh, (const i32*)hist_n, (const float*)hist_m,
-      (const float*)rmax, (const float*)temp, (const i32*)topk,
-      (const float*)topp, V);
-  dim3 g(B, SMP_SPLITS);
   tkp_sample_kernel<<<g, 256, 0, st>>>(
       (float*)pv, (i32*)pi, (const u16*)logits, (const float*)temp,
-      (const float*)thresh, (const uint32_t*)step, seed, V);
+      (const float*)rmax, (const i32*)hist_n, (const float*)hist_m,
+      (const i32*)topk, (const float*)topp, (const uint32_t*)step, seed, V);
   sample_combine_kernel<<<B, 64, 0, st>>>((i32*)out, (const float*)pv,
-                                          (const i32*)pi);
-  step_inc_kernel<<<1, 64, 0, st>>>((uint32_t*)step);
+                                          (const i32*)pi, (uint32_t*)step);
   return af_last_err();
 }
 
@@ -265,8 +340,8 @@ AF_EXPORT int af_sample(void* out, void* pv, void* pi, const void* logits,
   sample_partial_kernel<<<g1, 256, 0, st>>>(
       (float*)pv, (i32*)pi, (const u16*)logits, (const float*)temp,
       (const uint32_t*)step, seed, V);
-  sample_combine_kernel<<<B, 64, 0, st>>>((i32*)out, (const float*)pv, (const i32*)pi);
-  step_inc_kernel<<<1, 64, 0, st>>>((uint32_t*)step);
+  sample_combine_kernel<<<B, 64, 0, st>>>((i32*)out, (const float*)pv,
+                                          (const i32*)pi, (uint32_t*)step);
   return af_last_err();
 }
 

@@ -377,11 +377,12 @@ class SamplerState:
         self.pi = torch.empty(max_b, 16, dtype=torch.int32, device=device)
         self.step = torch.zeros(1, dtype=torch.int32, device=device)
         self.seed = seed
-        # top-k/top-p scratch (histogram threshold selection)
-        self.rmax = torch.empty(max_b, dtype=torch.float32, device=device)
-        self.thresh = torch.empty(max_b, dtype=torch.float32, device=device)
-        self.hist_n = torch.empty(max_b, 256, dtype=torch.int32, device=device)
-        self.hist_m = torch.empty(max_b, 256, dtype=torch.float32, device=device)
+        # top-k/top-p scratch (histogram threshold selection), per row split
+        self.rmax = torch.empty(max_b, 16, dtype=torch.float32, device=device)
+        self.hist_n = torch.empty(max_b, 16, 256, dtype=torch.int32,
+                                  device=device)
+        self.hist_m = torch.empty(max_b, 16, 256, dtype=torch.float32,
+                                  device=device)
 
 
 def sample(logits: torch.Tensor, temps: torch.Tensor, state: SamplerState,
@@ -407,10 +408,10 @@ def sample(logits: torch.Tensor, temps: torch.Tensor, state: SamplerState,
             topp = torch.ones(B, dtype=torch.float32, device=logits.device)
         rc = _lib.lib().af_sample_topkp(
             _lib.ptr(out), _lib.ptr(state.pv), _lib.ptr(state.pi),
-            _lib.ptr(state.rmax), _lib.ptr(state.thresh),
-            _lib.ptr(state.hist_n), _lib.ptr(state.hist_m), _lib.ptr(logits),
-            _lib.ptr(temps), _lib.ptr(topk), _lib.ptr(topp),
-            _lib.ptr(state.step), state.seed, B, V, _lib.cur_stream())
+            _lib.ptr(state.rmax), _lib.ptr(state.hist_n),
+            _lib.ptr(state.hist_m), _lib.ptr(logits), _lib.ptr(temps),
+            _lib.ptr(topk), _lib.ptr(topp), _lib.ptr(state.step), state.seed,
+            B, V, _lib.cur_stream())
         _lib.check(rc, "af_sample_topkp")
         return out
     rc = _lib.lib().af_sample(

@@ -64,7 +64,7 @@ def _declare(l: ctypes.CDLL) -> None:
     l.af_gemm_skinny.argtypes = [p, p, p, p, p, i, i, i, i, i,
                                  p, f, p, p]
     l.af_sample.argtypes = [p, p, p, p, p, p, u32, i, i, p]
-    l.af_sample_topkp.argtypes = [p, p, p, p, p, p, p, p, p, p, p, p,
+    l.af_sample_topkp.argtypes = [p, p, p, p, p, p, p, p, p, p, p,
                                   u32, i, i, p]
     l.af_gather_rows.argtypes = [p, p, p, i, i, p]
     l.af_mfma_probe.argtypes = [p, p, p, p]

@@ -349,6 +349,39 @@ def test_sample_temperature_varies_with_step():
     assert len(draws) > 1, "uniform logits should sample different tokens per step"
 
 
+@pytest.mark.parametrize("V", [1, 7, 8, 1001, 32003])
+@pytest.mark.parametrize("skip", [0, 1, 3])
+def test_sample_unaligned_rows(V, skip):
+    """Rows that start and end off the 16-byte grid (odd V, shifted base):
+    argmax with the smallest index among equal values, and top-k draws at or
+    above the lower edge of the k-th value's bin."""
+    B = 3
+    flat = rnd(B * V + skip, seed=50 + V + skip, scale=3.0)
+    logits = flat[skip:].view(B, V)
+    lf = logits.float().cpu()
+    st = ops.SamplerState(B, DEV)
+    temps = torch.tensor([0.0, 0.7, 1.3], device=DEV)
+    one = torch.ones(B, dtype=torch.int32, device=DEV)
+    off = torch.ones(B, dtype=torch.float32, device=DEV)
+    greedy = ops.sample(logits, torch.zeros(B, device=DEV), st).cpu()
+    first = ops.sample(logits, temps, st, topk=one, topp=off).cpu()
+    for b in range(B):
+        best = int((lf[b] == lf[b].max()).nonzero()[0])
+        assert int(greedy[b]) == best
+        assert lf[b, int(first[b])] == lf[b].max()
+    k = min(5, V)
+    gran = 20.0 / 256
+    for _ in range(4):
+        t = ops.sample(logits, temps, st, topk=one * k, topp=off).cpu()
+        for b in range(B):
+            T = float(temps[b]) or 1.0
+            x = lf[b] / T
+            kth, mx = x.topk(k).values[-1], x.max()
+            assert x[int(t[b])] >= kth - gran - 1e-3
+            if float(temps[b]) == 0.0:
+                assert x[int(t[b])] == mx
+
+
 def test_embedding_and_gather():
     tab = rnd(64, 256, seed=101)
     ids = torch.randint(0, 64, (10,), dtype=torch.int32, device=DEV)
