@@ -9,248 +9,311 @@
 //         out [B, Hq*D] bf16 (contiguous)
 // GQA group G = Hq/Hk in {1,2,4,8}.  D = 128.
 //
-// Work decomposition (memory-bound; CDNA4-shaped):
-//   grid (B, Hk, NSPLIT), block = 256 threads = 4 waves.
-//   A wave iteration covers EIGHT tokens (two unrolled groups of four):
-//   lane = tg*16 + dl, token subgroup tg = lane>>4, dim-group dl = lane&15
-//   owning dims [dl*8, dl*8+8).  Each K/V row is a 16-lane x 16 B coalesced
-//   read; within-page consecutive tokens make a 4-token group's reads 1 KiB
-//   contiguous.  The score reduction is 4 xor-shuffles within the 16-lane
-//   group + 2 across groups — ~2 shuffles per token vs 6 for a
-//   whole-wave-per-token layout, with 8x the load ILP.
-//   Online softmax state (m, l) is tracked wave-wide over the 4-token tile;
-//   o accumulates per-lane (8 dims) and is tg-reduced once at the end.
-//   Wave partials merge through LDS; split partials merge in a second kernel.
+// The K/V stream is the bound: 512 bytes per token and K/V head, used once.  A
+// CU's share of the memory rate is ~9 bytes per clock, i.e. one token every ~54
+// clocks, so a token may cost at most that in instructions and the loop must
+// keep tens of KB per CU in flight.
+//   grid (B, Hk, NSPLIT), block = 256 threads = 4 waves; a wave iteration takes
+//   16 tokens (4 KB of K, 4 KB of V, 16 B per lane and load), the next tile's
+//   eight loads are issued before the current tile's arithmetic.
+//   Scores come from the matrix cores: K rows are the A operand straight from
+//   the cache (lane = token, quarter of 32 dims), the group's query heads the
+//   B operand (columns repeat when G < 16), accumulated over 4 x 32 dims.  The
+//   result leaves lane (tg, h) = (lane>>4, lane&15) with head h's scores of the
+//   four tokens tg*4..tg*4+3.
+//   Running maximum, sum and output belong to a row of 16 lanes and its tokens
+//   (every fourth group of four): nothing crosses lanes inside the loop but a
+//   DPP broadcast of a head's weight along its row.  P V stays in fp32 vector
+//   arithmetic (weights are never rounded): lane (tg, dl) owns dims
+//   [dl*8, dl*8+8) and reads the same V rows whole, ~13 clocks per token at
+//   G = 4.
+//   Rows, then waves (through LDS), then splits (second kernel) merge once.
+// Measured with 8 K/V heads, G = 4, against one lane group per token with a
+// shuffle reduction per score: 24 sequences of 1800..8100 tokens (513 MB)
+// 225 -> 112 us (4.6 TB/s), 128 of 545 101 -> 56 us (5.1 TB/s), 1 of 8000
+// 58 -> 22 us.
 #include "common.h"
+
+#include <type_traits>
 
 #define AD_D 128
 #define AD_MAXG 8
+#define AD_TILE 16   // tokens per wave iteration
+#define AD_WAVES 4
 
-// Partial layout: po [B, Hk, NSPLIT, G, D] f32; pml [B, Hk, NSPLIT, G, 2] f32.
-template <int G, bool WIDE>
-__global__ void __launch_bounds__(256) attn_decode_kernel(
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8d;
+
+__device__ __forceinline__ bf16x8d as_bf16x8d(s16x8 v) {
+  union { s16x8 s; bf16x8d b; } u;
+  u.s = v;
+  return u.b;
+}
+
+// lane I of each 16-lane row, in all lanes of the row
+template <int I>
+__device__ __forceinline__ float row_bcast(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(
+      0, __float_as_int(v), 0x150 + I, 0xf, 0xf, true));
+}
+
+template <int I, int N, class F>
+__device__ __forceinline__ void each_head(F f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    each_head<I + 1, N>(f);
+  }
+}
+
+// Partial layout: po [B, Hk, NSPLIT, G, D] f32; pml [B, Hk, NSPLIT, G, 2] f32
+// (maximum in units of log2, sum; a split without tokens leaves po unwritten).
+//
+// TILED: page_size is a multiple of AD_TILE, so a tile lies in one page and its
+// index is a scalar load; otherwise every lane looks its tokens' pages up.
+template <int G, bool TILED>
+__global__ void __launch_bounds__(64 * AD_WAVES, G == 8 ? 3 : 4) attn_decode_kernel(
     u16* __restrict__ out, float* __restrict__ po, float* __restrict__ pml,
     const u16* __restrict__ q, const u16* __restrict__ kc, const u16* __restrict__ vc,
     const i32* __restrict__ bt, const i32* __restrict__ len,
-    float scale, int Hk, int page_size, int max_pages, int nsplit, i64 qs,
-    int win) {
+    float scale, int Hk, int page_size, int page_shift, int max_pages,
+    int nsplit, i64 qs, int win) {
   const int b = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z;
-  const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
   const int tg = lane >> 4, dl = lane & 15;
   const int Hq = Hk * G;
 
   const int L = len[b];
   // sliding window (Mistral): only the last `win` tokens are visible
   const int s0 = (win > 0 && L > win) ? L - win : 0;
-  const int chunk = (L - s0 + nsplit - 1) / nsplit;
-  const int t0 = s0 + split * chunk;
-  const int t1 = min(L, t0 + chunk);
-
-  // Q (8 dims per lane per head), pre-scaled
-  float qr[G][8];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const u16* qp = q + (size_t)b * qs + (kvh * G + g) * AD_D + dl * 8;
-    s16x8 qv = *reinterpret_cast<const s16x8*>(qp);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) qr[g][j] = bf2f((u16)qv[j]) * scale;
-  }
-
-  float m[G], l[G], acc[G][8];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    m[g] = AF_NEG_INF;
-    l[g] = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
-  }
-
-  const i32* btrow = bt + (size_t)b * max_pages;
-  if (!WIDE) {
-    // one 4-token tile per wave iteration: wins at LOW grid occupancy
-    // (<= 2 blocks/CU) where the wider loop loses throughput (measured)
-    for (int tb = t0 + wid * 4; tb < t1; tb += 16) {
-      const int t = tb + tg;
-      const bool valid = t < t1;
-      const int tc = valid ? t : (t1 - 1);
-      const i64 page = btrow[tc / page_size];
-      const size_t base = (((size_t)page * Hk + kvh) * page_size +
-                           (tc % page_size)) * AD_D + dl * 8;
-      const s16x8 kv8 = *reinterpret_cast<const s16x8*>(kc + base);
-      const s16x8 vv8 = *reinterpret_cast<const s16x8*>(vc + base);
-      float kf[8], vf[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        kf[j] = bf2f((u16)kv8[j]);
-        vf[j] = bf2f((u16)vv8[j]);
+  const int a0 = s0 & ~(AD_TILE - 1);
+  // splits are whole rounds of the block's waves
+  constexpr int ROUND = AD_TILE * AD_WAVES;
+  const int chunk = ((L - a0 + nsplit - 1) / nsplit + ROUND - 1) & ~(ROUND - 1);
+  const int c0 = a0 + split * chunk;       // tile grid of this split
+  const int t1 = min(L, c0 + chunk);
+  const int t0 = max(s0, c0);              // visible tokens are [t0, t1)
+  if (c0 >= t1) {                          // no tokens (uniform in the block)
+    if (nsplit > 1) {
+      if (threadIdx.x < G) {
+        const size_t at =
+            (((size_t)b * Hk + kvh) * nsplit + split) * G + threadIdx.x;
+        pml[at * 2] = AF_NEG_INF;
+        pml[at * 2 + 1] = 0.f;
       }
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        float d = 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) d += qr[g][j] * kf[j];
-        float s = group16_sum_f32(d);
-        if (!valid) s = AF_NEG_INF;
-        float tm = fmaxf(s, __shfl_xor(s, 16, 64));
-        tm = fmaxf(tm, __shfl_xor(tm, 32, 64));
-        const float mn = fmaxf(m[g], tm);
-        const float corr = (m[g] <= AF_NEG_INF) ? 0.f : __expf(m[g] - mn);
-        const float p = (s <= AF_NEG_INF) ? 0.f : __expf(s - mn);
-        float psum = p + __shfl_xor(p, 16, 64);
-        psum += __shfl_xor(psum, 32, 64);
-        l[g] = l[g] * corr + psum;
-        m[g] = mn;
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          acc[g][j] = acc[g][j] * corr + p * vf[j];
-      }
+    } else {                               // an empty sequence
+      for (int i = threadIdx.x; i < G * AD_D; i += 64 * AD_WAVES)
+        out[(size_t)b * (Hq * AD_D) + kvh * G * AD_D + i] = 0;
     }
-  } else {
-  // wave w handles tokens {i*32 + w*4 + tg} and {i*32 + 16 + w*4 + tg}:
-  // TWO 4-token tiles per iteration with all four 16-B K/V loads issued
-  // before any compute — the kernel is gather-latency-bound, so doubling
-  // the in-flight bytes per wave is the lever (guide: memory-level
-  // parallelism, not arithmetic, sets gather throughput)
-  auto tile_base = [&](int t) {
-    const i64 page = btrow[t / page_size];
-    return (((size_t)page * Hk + kvh) * page_size + (t % page_size)) * AD_D +
-           dl * 8;
-  };
-  for (int tb = t0 + wid * 4; tb < t1; tb += 32) {
-    const int ta = tb + tg, tb2 = tb + 16 + tg;
-    const bool va = ta < t1, vb = tb2 < t1;
-    // unconditional clamped loads: a branch around the second tile's
-    // loads stops the compiler issuing them early, which defeats the
-    // whole point (measured -25% on short chunks)
-    const size_t base_a = tile_base(va ? ta : (t1 - 1));
-    const size_t base_b = tile_base(vb ? tb2 : (t1 - 1));
-    const s16x8 ka8 = *reinterpret_cast<const s16x8*>(kc + base_a);
-    const s16x8 va8 = *reinterpret_cast<const s16x8*>(vc + base_a);
-    const s16x8 kb8 = *reinterpret_cast<const s16x8*>(kc + base_b);
-    const s16x8 vb8 = *reinterpret_cast<const s16x8*>(vc + base_b);
-    float kfa[8], vfa[8], kfb[8], vfb[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      kfa[j] = bf2f((u16)ka8[j]);
-      vfa[j] = bf2f((u16)va8[j]);
-      kfb[j] = bf2f((u16)kb8[j]);
-      vfb[j] = bf2f((u16)vb8[j]);
-    }
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const bool valid = half ? vb : va;
-      const float* kf = half ? kfb : kfa;
-      const float* vf = half ? vfb : vfa;
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        float d = 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) d += qr[g][j] * kf[j];
-        // 16-lane reduce -> s uniform within token group
-        float s = group16_sum_f32(d);
-        if (!valid) s = AF_NEG_INF;
-        // tile max across the 4 token groups
-        float tm = fmaxf(s, __shfl_xor(s, 16, 64));
-        tm = fmaxf(tm, __shfl_xor(tm, 32, 64));
-        if (tm <= AF_NEG_INF) continue;  // whole tile invalid (tail)
-        const float mn = fmaxf(m[g], tm);
-        const float corr = (m[g] <= AF_NEG_INF) ? 0.f : __expf(m[g] - mn);
-        const float p = (s <= AF_NEG_INF) ? 0.f : __expf(s - mn);
-        float psum = p + __shfl_xor(p, 16, 64);
-        psum += __shfl_xor(psum, 32, 64);
-        l[g] = l[g] * corr + psum;
-        m[g] = mn;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[g][j] = acc[g][j] * corr + p * vf[j];
-      }
-    }
+    return;
   }
+
+  // query heads as B operand: lane holds head (lane & 15) % G, dims
+  // 32 c + tg*8 .. +8
+  s16x8 qf[4];
+  {
+    const u16* qp = q + (size_t)b * qs + (kvh * G + (dl & (G - 1))) * AD_D + tg * 8;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) qf[c] = *reinterpret_cast<const s16x8*>(qp + c * 32);
   }
-  // fold the 4 token-groups' partial o (same dims, disjoint tokens)
+  const float sc = scale * 1.44269504088896f;  // softmax in powers of two
+
+  float m = AF_NEG_INF, l = 0.f, acc[G][8];
 #pragma unroll
   for (int g = 0; g < G; ++g)
 #pragma unroll
+    for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
+
+  const i32* btrow = bt + (size_t)b * max_pages;
+  auto page_of = [&](int t) {
+    return btrow[page_shift >= 0 ? t >> page_shift : t / page_size];
+  };
+  auto page_off = [&](int t) {
+    return page_shift >= 0 ? t & (page_size - 1) : t % page_size;
+  };
+  // K rows of tokens behind t1 may be read (their scores are dropped); V rows
+  // are clamped to visible tokens, whose values are finite when weighed by 0
+  auto load_tile = [&](int t, int page, s16x8* kf, s16x8* vf) {
+    if (TILED) {
+      const size_t base =
+          (((size_t)page * Hk + kvh) * page_size + page_off(t)) * AD_D;
+      const u16* kp = kc + base + dl * AD_D + tg * 8;
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        kf[c] = *reinterpret_cast<const s16x8*>(kp + c * 32);
+      const u16* vp = vc + base + dl * 8;
+      const int lo = t0 - t, hi = t1 - 1 - t;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        vf[r] = *reinterpret_cast<const s16x8*>(
+            vp + min(max(tg * 4 + r, lo), hi) * AD_D);
+    } else {
+      auto row = [&](int tok) {
+        const int tc = min(max(tok, t0), t1 - 1);
+        return (((size_t)page_of(tc) * Hk + kvh) * page_size + page_off(tc)) * AD_D;
+      };
+      const u16* kp = kc + row(t + dl) + tg * 8;
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        kf[c] = *reinterpret_cast<const s16x8*>(kp + c * 32);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        vf[r] = *reinterpret_cast<const s16x8*>(vc + row(t + tg * 4 + r) + dl * 8);
+    }
+  };
+
+  s16x8 kf[4], vf[4], kn[4], vn[4];
+  int t = c0 + wid * AD_TILE;
+  int pg_next = 0;
+  if (t < t1) {
+    load_tile(t, TILED ? page_of(t) : 0, kf, vf);
+    if (TILED) pg_next = page_of(min(t + ROUND, t1 - 1));
+  }
+  for (; t < t1; t += ROUND) {
+    if (t + ROUND < t1) {
+      load_tile(t + ROUND, pg_next, kn, vn);
+      if (TILED) pg_next = page_of(min(t + 2 * ROUND, t1 - 1));
+    }
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8d(kf[c]),
+                                                  as_bf16x8d(qf[c]), s, 0, 0, 0);
+    float mn = m;
+    bool ok[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int tok = t + tg * 4 + r;
+      ok[r] = tok >= t0 && tok < t1;
+      s[r] = ok[r] ? s[r] * sc : AF_NEG_INF;
+      mn = fmaxf(mn, s[r]);
+    }
+    float p[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      p[r] = ok[r] ? __builtin_amdgcn_exp2f(s[r] - mn) : 0.f;
+    if (__any(mn > m)) {  // rare once the first tiles have been seen
+      const float corr = __builtin_amdgcn_exp2f(m - mn);
+      l *= corr;
+      each_head<0, G>([&](auto g) {
+        const float cg = row_bcast<g.value>(corr);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[g.value][j] *= cg;
+      });
+      m = mn;
+    }
+    l += (p[0] + p[1]) + (p[2] + p[3]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = bf2f((u16)vf[r][j]);
+      each_head<0, G>([&](auto g) {
+        const float pg = row_bcast<g.value>(p[r]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          acc[g.value][j] = fmaf(pg, v[j], acc[g.value][j]);
+      });
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) { kf[c] = kn[c]; vf[c] = vn[c]; }
+  }
+
+  // fold the four rows (same dims, other tokens)
+  float M = fmaxf(m, __shfl_xor(m, 16, 64));
+  M = fmaxf(M, __shfl_xor(M, 32, 64));
+  const float f = (m <= AF_NEG_INF) ? 0.f : __builtin_amdgcn_exp2f(m - M);
+  l *= f;
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  __shared__ float s_ml[AD_WAVES][G][2];
+  __shared__ float s_o[AD_WAVES][G][AD_D];
+  each_head<0, G>([&](auto g) {
+    const float fg = row_bcast<g.value>(f);
+    float o[8];
+#pragma unroll
     for (int j = 0; j < 8; ++j) {
-      acc[g][j] += __shfl_xor(acc[g][j], 16, 64);
-      acc[g][j] += __shfl_xor(acc[g][j], 32, 64);
+      o[j] = acc[g.value][j] * fg;
+      o[j] += __shfl_xor(o[j], 16, 64);
+      o[j] += __shfl_xor(o[j], 32, 64);
     }
-
-  // ---- merge 4 wave partials through LDS ----
-  __shared__ float s_ml[4][G][2];
-  __shared__ float s_o[4][G][AD_D];
-  if (lane == 0) {
+    if (tg == 0) {
 #pragma unroll
-    for (int g = 0; g < G; ++g) { s_ml[wid][g][0] = m[g]; s_ml[wid][g][1] = l[g]; }
-  }
-  if (tg == 0) {
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) s_o[wid][g][dl * 8 + j] = acc[g][j];
-  }
+      for (int j = 0; j < 8; ++j) s_o[wid][g.value][dl * 8 + j] = o[j];
+    }
+  });
+  if (lane < G) { s_ml[wid][lane][0] = M; s_ml[wid][lane][1] = l; }
   __syncthreads();
-  if (wid != 0) return;
 
+  // merge the waves: two elements per thread
+  for (int i = threadIdx.x; i < G * AD_D / 2; i += 64 * AD_WAVES) {
+    const int g = i / (AD_D / 2), d = (i % (AD_D / 2)) * 2;
+    float Mx = s_ml[0][g][0];
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    float M = AF_NEG_INF;
+    for (int w = 1; w < AD_WAVES; ++w) Mx = fmaxf(Mx, s_ml[w][g][0]);
+    float L2 = 0.f, o0 = 0.f, o1 = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) M = fmaxf(M, s_ml[w][g][0]);
-    float L2 = 0.f, o8[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o8[j] = 0.f;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const float c = (s_ml[w][g][0] <= AF_NEG_INF) ? 0.f : __expf(s_ml[w][g][0] - M);
+    for (int w = 0; w < AD_WAVES; ++w) {
+      const float c = (s_ml[w][g][0] <= AF_NEG_INF)
+                          ? 0.f
+                          : __builtin_amdgcn_exp2f(s_ml[w][g][0] - Mx);
       L2 += s_ml[w][g][1] * c;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) o8[j] += s_o[w][g][dl * 8 + j] * c;
+      o0 += s_o[w][g][d] * c;
+      o1 += s_o[w][g][d + 1] * c;
     }
-    if (tg != 0) continue;
     if (nsplit == 1) {
       const float inv = (L2 > 0.f) ? 1.f / L2 : 0.f;
-      u16* op = out + (size_t)b * (Hq * AD_D) + (kvh * G + g) * AD_D + dl * 8;
-      s16x8 ov;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) ov[j] = (short)f2bf(o8[j] * inv);
-      *reinterpret_cast<s16x8*>(op) = ov;
+      u16x2 ov = {f2bf(o0 * inv), f2bf(o1 * inv)};
+      *reinterpret_cast<u16x2*>(out + (size_t)b * (Hq * AD_D) +
+                                (kvh * G + g) * AD_D + d) = ov;
     } else {
-      const size_t pbase = ((((size_t)b * Hk + kvh) * nsplit + split) * G + g);
-      float* od = po + pbase * AD_D + dl * 8;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) od[j] = o8[j];
-      if (lane == 0) { pml[pbase * 2] = M; pml[pbase * 2 + 1] = L2; }
+      const size_t at = (((size_t)b * Hk + kvh) * nsplit + split) * G + g;
+      *reinterpret_cast<f32x2*>(po + at * AD_D + d) = f32x2{o0, o1};
+      if (d == 0) { pml[at * 2] = Mx; pml[at * 2 + 1] = L2; }
     }
   }
 }
 
-// Combine split partials: grid (B, Hq), 64 threads (one wave, 2 dims/lane).
+// Combine split partials: grid (B, Hq), one wave, 2 dims per lane.  The splits'
+// weights come first, one split per lane, so that the loads of the partial
+// outputs do not wait for each other.
 __global__ void __launch_bounds__(64) attn_decode_combine_kernel(
     u16* __restrict__ out, const float* __restrict__ po, const float* __restrict__ pml,
     int Hq, int G, int nsplit) {
   const int b = blockIdx.x, h = blockIdx.y;
   const int kvh = h / G, g = h % G;
   const int Hk = Hq / G;
-  const int d0 = threadIdx.x * 2;
+  const int lane = threadIdx.x;
+  const size_t first = (((size_t)b * Hk + kvh) * nsplit) * G + g;
 
-  float M = AF_NEG_INF;
-  for (int s = 0; s < nsplit; ++s) {
-    const size_t pbase = ((((size_t)b * Hk + kvh) * nsplit + s) * G + g);
-    M = fmaxf(M, pml[pbase * 2]);
-  }
-  float L2 = 0.f, o0 = 0.f, o1 = 0.f;
-  for (int s = 0; s < nsplit; ++s) {
-    const size_t pbase = ((((size_t)b * Hk + kvh) * nsplit + s) * G + g);
-    const float pm = pml[pbase * 2];
-    const float c = (pm <= AF_NEG_INF) ? 0.f : __expf(pm - M);
-    L2 += pml[pbase * 2 + 1] * c;
-    o0 += po[pbase * AD_D + d0] * c;
-    o1 += po[pbase * AD_D + d0 + 1] * c;
+  float L2 = 0.f, o0 = 0.f, o1 = 0.f, M = AF_NEG_INF;
+  for (int s0 = 0; s0 < nsplit; s0 += 64) {  // one round for nsplit <= 64
+    const int s = s0 + lane;
+    float pm = AF_NEG_INF, pl = 0.f;
+    if (s < nsplit) {
+      pm = pml[(first + (size_t)s * G) * 2];
+      pl = pml[(first + (size_t)s * G) * 2 + 1];
+    }
+    const float Mn = fmaxf(M, wave_max_f32(pm));
+    const float back = (M <= AF_NEG_INF) ? 0.f : __builtin_amdgcn_exp2f(M - Mn);
+    const float c = (pm <= AF_NEG_INF) ? 0.f : __builtin_amdgcn_exp2f(pm - Mn);
+    L2 = L2 * back + wave_sum_f32(pl * c);
+    o0 *= back;
+    o1 *= back;
+    M = Mn;
+    const int n = min(64, nsplit - s0);
+#pragma unroll 8
+    for (int i = 0; i < n; ++i) {
+      const float ci = __shfl(c, i, 64);
+      if (ci == 0.f) continue;  // without tokens: po was not written
+      const f32x2 v = *reinterpret_cast<const f32x2*>(
+          po + (first + (size_t)(s0 + i) * G) * AD_D + lane * 2);
+      o0 += v[0] * ci;
+      o1 += v[1] * ci;
+    }
   }
   const float inv = (L2 > 0.f) ? 1.f / L2 : 0.f;
-  u16* op = out + (size_t)b * (Hq * AD_D) + h * AD_D + d0;
-  op[0] = f2bf(o0 * inv);
-  op[1] = f2bf(o1 * inv);
+  u16x2 ov = {f2bf(o0 * inv), f2bf(o1 * inv)};
+  *reinterpret_cast<u16x2*>(out + (size_t)b * (Hq * AD_D) + h * AD_D + lane * 2) = ov;
 }
 
 AF_EXPORT int af_attn_decode(void* out, void* po, void* pml, const void* q,
@@ -262,21 +325,19 @@ AF_EXPORT int af_attn_decode(void* out, void* po, void* pml, const void* q,
   const int G = Hq / Hk;
   if (G < 1 || G > AD_MAXG || G * Hk != Hq) return 9003;
   if (B == 0) return 0;
-  dim3 grid(B, Hk, nsplit), blk(256);
+  dim3 grid(B, Hk, nsplit), blk(64 * AD_WAVES);
   hipStream_t st = (hipStream_t)stream;
-  const bool wide = (size_t)B * Hk * nsplit >= 1024;  // >= 4 blocks/CU
+  const bool pow2 = (page_size & (page_size - 1)) == 0;
+  const int shift = pow2 ? __builtin_ctz(page_size) : -1;
+#define AF_LAUNCH1(GG, TT)                                                       \
+  attn_decode_kernel<GG, TT><<<grid, blk, 0, st>>>(                              \
+      (u16*)out, (float*)po, (float*)pml, (const u16*)q, (const u16*)kc,         \
+      (const u16*)vc, (const i32*)bt, (const i32*)len, scale, Hk, page_size,     \
+      shift, max_pages, nsplit, qs, win)
 #define AF_LAUNCH(GG)                                                            \
   do {                                                                           \
-    if (wide)                                                                    \
-      attn_decode_kernel<GG, true><<<grid, blk, 0, st>>>(                        \
-          (u16*)out, (float*)po, (float*)pml, (const u16*)q, (const u16*)kc,     \
-          (const u16*)vc, (const i32*)bt, (const i32*)len, scale, Hk,            \
-          page_size, max_pages, nsplit, qs, win);                                \
-    else                                                                         \
-      attn_decode_kernel<GG, false><<<grid, blk, 0, st>>>(                       \
-          (u16*)out, (float*)po, (float*)pml, (const u16*)q, (const u16*)kc,     \
-          (const u16*)vc, (const i32*)bt, (const i32*)len, scale, Hk,            \
-          page_size, max_pages, nsplit, qs, win);                                \
+    if (page_size % AD_TILE == 0) AF_LAUNCH1(GG, true);                          \
+    else AF_LAUNCH1(GG, false);                                                  \
   } while (0)
   switch (G) {
     case 1: AF_LAUNCH(1); break;
@@ -286,6 +347,7 @@ AF_EXPORT int af_attn_decode(void* out, void* po, void* pml, const void* q,
     default: return 9003;
   }
 #undef AF_LAUNCH
+#undef AF_LAUNCH1
   if (nsplit > 1) {
     dim3 g2(B, Hq), b2(64);
     attn_decode_combine_kernel<<<g2, b2, 0, st>>>(

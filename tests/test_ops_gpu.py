@@ -494,3 +494,36 @@ def test_mxfp8_mlp_layer_accuracy():
     # regime (single-GEMM exactness vs the dequantized product is pinned
     # to 5e-3 in test_gemm_mxfp8)
     assert rel.item() < 0.15, rel.item()
+
+
+@pytest.mark.parametrize("page,G,Hk", [(4, 4, 2), (16, 1, 3), (24, 2, 2),
+                                       (48, 8, 1), (64, 4, 2)])
+@pytest.mark.parametrize("nsplit,window", [(1, 0), (3, 0), (16, 0), (1, 37),
+                                           (4, 130)])
+def test_attn_decode_tile_edges(page, G, Hk, nsplit, window):
+    """Lengths around 16-token tiles, 64-token rounds and pages that do or do
+    not hold whole tiles; splits without tokens; everything that is not visible
+    is NaN in the values, so that reading it with weight 0 would show.
+    Tolerance: bf16 rounding of outputs below 4 (2^-9 * 4)."""
+    D = 128
+    lens = [1, 2, 15, 16, 17, 48, 63, 64, 65, 129, 300]
+    B = len(lens)
+    torch.manual_seed(7)
+    maxp = -(-max(lens) // page)
+    bt = (torch.randperm(B * maxp) + 1).view(B, maxp).to(torch.int32)
+    kc = torch.randn(B * maxp + 1, Hk, page, D).bfloat16()
+    vc = torch.randn(B * maxp + 1, Hk, page, D).bfloat16()
+    seen = torch.zeros(B * maxp + 1, page, dtype=torch.bool)
+    for b, n in enumerate(lens):
+        for t in range(max(0, n - window) if window else 0, n):
+            seen[bt[b, t // page], t % page] = True
+    vc = torch.where(seen[:, None, :, None], vc, torch.nan)
+    q = torch.randn(B, Hk * G * D).bfloat16()
+    L = torch.tensor(lens, dtype=torch.int32)
+    got = ops.attn_decode(q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV),
+                          L.to(DEV), nsplit=nsplit, window=window).cpu()
+    want = ref.attn_decode(q.unflatten(-1, (Hk * G, D)), kc,
+                           torch.nan_to_num(vc), bt, L, 1.0 / math.sqrt(D),
+                           window=window).flatten(1)
+    assert torch.isfinite(got.float()).all()
+    assert close(got, want, atol=2 ** -7, rtol=2 ** -8)
