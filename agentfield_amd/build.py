@@ -35,6 +35,7 @@ HIP_SOURCES = [
     "gemm_mxfp8.hip",
     "allreduce.hip",
     "gemm_skinny.hip",
+    "gemm_rows.hip",
     "sampling.hip",
     "probe.hip",
 ]

@@ -1,4 +1,4 @@
-// Paged causal prefill attention (flash-style, GQA) with MFMA 16x16x32 bf16.
+// Paged causal prefill attention (flash-style, GQA) on MFMA 32x32x16 bf16.
 //
 // q      : chunk rows at stride qs (view into the fused QKV buffer), head h
 //          at offset h*D, D=128, packed by sequence (cu_seqlens of the CHUNK).
@@ -8,37 +8,74 @@
 // qstart : per-seq absolute position of the chunk's first row (0 for a
 //          full-prompt prefill; >0 when continuing a chunked prefill).
 // out    : [chunk_T, Hq*D] bf16 contiguous.
-// Host precomputes a flat tile map (tile_seq[i], tile_q0[i]): workgroup i on
-// grid.x handles chunk rows [q0, q0+ROWS) of sequence tile_seq[i];
-// grid.y = kv head.
 //
-// Workgroup = 256 threads = 4 waves.  Each wave owns a 16-row q-tile of one
-// query head in the GQA group:
-//   G>=4 : all waves share one 16-row tile; wave w covers heads g=w, w+4, ...
-//   G<4  : 4/G row-tiles per workgroup; wave w -> (g = w%G, tile = w/G)
-// K/V tiles (KVBLK=64 tokens) are staged in LDS once per workgroup and shared
-// by the 4 waves; 64-token tiles halve the barrier count per token vs 32.
+// The rows of a sequence and the G query heads of one K/V head form G*len
+// columns (column = row*G + head); a wave owns 32 of them.  Both products are
+// computed transposed:
+//   S^T [tokens x columns] = K Q^T: a lane gets 16 tokens of ONE column per 32
+//     tokens, so maximum, sum and rescaling are per-lane values and a row
+//     maximum crosses lanes once per tile (permlane32_swap).
+//   O^T [dims x columns] = V^T P^T: the P fragment is the lane's own S^T
+//     registers, rounded to bf16 in pairs; the contraction's token order inside
+//     16 tokens is the one S^T came out in ({4h..4h+3, 8+4h..8+4h+3} for lane
+//     half h), and V^T comes from row-major LDS by transposing reads
+//     (ds_read_b64_tr_b16) in that order.  P never passes through LDS.
+// K and V tiles go global -> LDS without registers (16 B per lane), chunks of 16 B
+// permuted within the row by the row number, so that neither the b128 reads of K
+// nor the transposing reads of V meet in a bank.
+// Softmax works on powers of two; the running maximum moves only when a tile
+// exceeds it by 2^6, which bounds P by 64 (relative rounding is unchanged) and
+// saves rescaling the 64 output registers on most tiles.
 //
-// CDNA4 specifics (see /opt/skills/guides/cdna_hip_programming.md):
-//  - K LDS tile is XOR-swizzled (byte ^= (row&7)<<4) so the B-fragment
-//    ds_read_b128 is bank-conflict-free (guide §6 G4: row-major [64][128]
-//    would be a 32-way conflict).
-//  - V is stored transposed [D][KVBLK+pad] with token pairs packed as u32
-//    ds_writes (2 tokens per 4 B slot) so staging is 8 b32 writes per two
-//    16 B loads; pad 64->72 spreads banks on the PV-fragment reads.
-//  - P (scores) round-trips through a small per-wave LDS tile to convert the
-//    MFMA C-layout into the A-fragment layout.
-//  - fragment layouts (guide §3, measured, validated by ops.mfma_probe):
-//      A: lane holds A[m=lane&15][k=(lane>>4)*8+j], j=0..7
-//      B: lane holds B[k=(lane>>4)*8+j][n=lane&15]
-//      C: lane reg r holds C[m=(lane>>4)*4+r][n=lane&15]
+//   attn_prefill_kernel  4 waves x 32 columns, K/V tiles of 64 tokens shared by
+//     the block and double-buffered (64 KB, two blocks per CU: one wave's
+//     exponentials run under the other's MFMA).  Bound by vector issue next to
+//     the matrix cores: 32 exponentials per lane and tile alone take half of the
+//     tile's MFMA time.  grid: K/V head fastest, so with 8 of them an XCD's L2
+//     keeps one head's K/V; late (long) tiles start first.
+//   attn_prefill_few_kernel  32 columns per block: sequences whose columns fit
+//     one wave (verification of a few drafted tokens, single fed tokens), or all
+//     of a batch too small to fill the chip with 128-column blocks.  The four
+//     waves split the keys, each with private 32-token double buffers and no
+//     barrier in the loop, and merge through LDS; with fewer than 256 blocks the
+//     keys are also split over blocks and a second kernel merges.  Bound by the
+//     K/V stream, so P is kept to 16 bits more: two bf16 terms, two products.
+// Fragment layouts (measured): A: lane holds A[m=lane&31][k=(lane>>5)*8+j]; B:
+// B[k=(lane>>5)*8+j][n=lane&31]; C: reg r holds C[8*(r/4)+4*(lane>>5)+r%4][lane&31];
+// transposing read: lane i of a group of 16 gets column i of 4 rows x 16 columns
+// whose 8-byte pieces the group's lanes address row by row.
+//
+// Against 16x16x32 tiles of 64 columns with P through LDS and V transposed by
+// scalar writes (one layer, 8 K/V heads, G = 4): one prompt of 8000 rows 2292 ->
+// 679 us (229 -> 772 TFLOP/s), 20 of 300..700 384 -> 110 us, 8 x 2048 at G = 2
+// 992 -> 232 us; 16 sequences of 5 rows behind 2400 tokens 387 -> 51 us.
 #include "common.h"
 
 #define AP_D 128
-#define AP_KVBLK 64
-#define AP_VPAD 72  // 64 tokens padded to 72 (residual 2-way conflicts are free, guide m136)
+#define AP_KV 64          // tokens per shared tile
+#define AP_FEW 32         // tokens per wave-private tile
+#define AP_ROWB 256       // bytes of a K or V row
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((address_space(3))) char lds_char;
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+typedef __attribute__((address_space(3))) s16x8 lds_s16x8;
+
+struct PrefillArgs {
+  u16* out;
+  const u16* q;
+  const u16* kc;
+  const u16* vc;
+  const i32* bt;
+  const i32* qstart;
+  const i32* cu;
+  float scale;
+  int nseq, Hq, Hk;
+  i64 qs;
+  int page_size, page_shift, max_pages, win;
+  int few_cols;     // sequences of up to so many columns go to the few-kernel
+};
 
 __device__ __forceinline__ bf16x8 as_bf16x8(s16x8 v) {
   union { s16x8 s; bf16x8 b; } u;
@@ -46,218 +83,469 @@ __device__ __forceinline__ bf16x8 as_bf16x8(s16x8 v) {
   return u.b;
 }
 
-__device__ __forceinline__ s16x8 lds_read8(const u16* p) {
-  return *reinterpret_cast<const s16x8*>(p);
+__device__ __forceinline__ float swap_max(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(v),
+                                                  __float_as_int(v), false, false);
+  return fmaxf(__int_as_float(r[0]), __int_as_float(r[1]));
+}
+
+// Sequence and place in it of work item `item`: items are pieces of 32 (FEW) or
+// 128 columns, counted over the sequences that the kernel serves.
+template <int G, bool FEW>
+__device__ __forceinline__ int find_item(const PrefillArgs& a, int item, int* at) {
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  for (int s0 = 0; s0 < a.nseq; s0 += 64) {
+    const int s = s0 + lane;
+    int n = 0;
+    if (s < a.nseq) {
+      const int cols = (a.cu[s + 1] - a.cu[s]) * G;
+      if ((cols <= a.few_cols) == FEW) n = FEW ? (cols + 31) / 32 : (cols + 127) / 128;
+    }
+    int incl = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
+    }
+    const unsigned long long hit = __ballot(base + incl > item);
+    if (hit) {
+      const int l = __ffsll(hit) - 1;
+      *at = __builtin_amdgcn_readfirstlane(
+          item - base - (__shfl(incl, l, 64) - __shfl(n, l, 64)));
+      return __builtin_amdgcn_readfirstlane(s0 + l);
+    }
+    base += __shfl(incl, 63, 64);
+  }
+  return -1;
+}
+
+// Rows [row0, row0 + 4*N) of a K and a V tile whose first token is t0 into LDS:
+// every instruction brings 4 rows (1 KB).  Tokens behind the last one repeat it
+// (their weights are 0 and must meet finite values).
+// page: the tile's page when it lies in one (TILED).
+template <bool TILED, int N>
+__device__ __forceinline__ void stage(const PrefillArgs& a, const i32* btrow,
+                                      int kvh, int t0, int row0, int last,
+                                      int page, lds_char* kl, lds_char* vl) {
+  const int lane = threadIdx.x & 63;
+  const int r4 = lane >> 4, slot = lane & 15;
+  const int off0 =
+      TILED ? (a.page_shift >= 0 ? t0 & (a.page_size - 1) : t0 % a.page_size) : 0;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int row = row0 + i * 4 + r4;
+    size_t src;
+    if (TILED) {
+      src = ((size_t)page * a.Hk + kvh) * a.page_size + off0 +
+            min(row, last - t0);
+    } else {
+      const int t = min(t0 + row, last);
+      const int pi = a.page_shift >= 0 ? t >> a.page_shift : t / a.page_size;
+      src = ((size_t)btrow[pi] * a.Hk + kvh) * a.page_size + (t - pi * a.page_size);
+    }
+    src *= AP_D;
+    const int dst = (row0 + i * 4) * AP_ROWB;
+    __builtin_amdgcn_global_load_lds(
+        (const __attribute__((address_space(1))) uint32_t*)(
+            a.kc + src + ((slot ^ (row & 15)) << 3)),
+        (__attribute__((address_space(3))) uint32_t*)(kl + dst), 16, 0, 0);
+    __builtin_amdgcn_global_load_lds(
+        (const __attribute__((address_space(1))) uint32_t*)(
+            a.vc + src + ((slot ^ ((row & 7) << 1)) << 3)),
+        (__attribute__((address_space(3))) uint32_t*)(vl + dst), 16, 0, 0);
+  }
+}
+
+// A wave's columns and their running softmax.
+struct Columns {
+  s16x8 q[8];       // B operand, 8 x 16 dims
+  f32x16 o[4];      // O^T, 4 x 32 dims
+  float m, l;       // maximum of raw scores, sum over this lane half's tokens
+  int qpos;         // absolute position of the column's row
+};
+
+// NB x 32 tokens from t0 of the tile at kl / vl.  masked: some column does not
+// see some of them.  FINE: P as two bf16 terms.
+template <int NB, bool FINE>
+__device__ __forceinline__ void attend(Columns& c, const lds_char* kl,
+                                       const lds_char* vl, int t0, float sc,
+                                       int win, bool masked) {
+  const int lane = threadIdx.x & 63;
+  const int h = lane >> 5, n = lane & 31, i = lane & 15;
+  f32x16 s[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[b][r] = 0.f;
+  // operands are read one step ahead of their MFMA; the scheduling fences keep
+  // the compiler from reading the whole tile ahead (it spilled 70 registers)
+  const int kx = (h ^ (n & 15)) << 4;
+  auto read_k = [&](int d, s16x8* f) {
+    const lds_char* kp = kl + n * AP_ROWB + (kx ^ (d << 5));
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      f[b] = *reinterpret_cast<const lds_s16x8*>(kp + b * 32 * AP_ROWB);
+  };
+  s16x8 kf[2][NB];
+  read_k(0, kf[0]);
+#pragma unroll
+  for (int d = 0; d < 8; ++d) {
+    if (d < 7) read_k(d + 1, kf[(d + 1) & 1]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      s[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          as_bf16x8(kf[d & 1][b]), as_bf16x8(c.q[d]), s[b], 0, 0, 0);
+  }
+  if (masked) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int t = t0 + b * 32 + 8 * (r / 4) + 4 * h + (r % 4);
+        if (t > c.qpos || (win > 0 && t <= c.qpos - win)) s[b][r] = AF_NEG_INF;
+      }
+  }
+  float mx = AF_NEG_INF;
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; r += 2) mx = fmaxf(mx, fmaxf(s[b][r], s[b][r + 1]));
+  mx = swap_max(mx);
+  if (__any((mx - c.m) * sc > 6.f)) {
+    const float mn = fmaxf(c.m, mx);
+    const float corr = __builtin_amdgcn_exp2f((c.m - mn) * sc);
+    c.m = mn;
+    c.l *= corr;
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) c.o[d][r] *= corr;
+  }
+  // a column that has seen nothing yet keeps weight 0 for masked tokens
+  const float mz = (c.m <= AF_NEG_INF) ? 0.f : -c.m * sc;
+  const int vx = ((4 * h + (i >> 2)) << 1);
+  const lds_char* vp = vl + (4 * h + (i >> 2)) * AP_ROWB + (i & 1) * 8;
+  const int ve = ((lane >> 4) & 1) * 2 + ((i & 3) >> 1);
+  union VF { s16x4 half[2]; bf16x8 b; };
+  auto read_v = [&](int k, VF* f) {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const lds_char* at = vp + (((d * 4 + ve) ^ vx) << 4) + k * 16 * AP_ROWB;
+      f[d].half[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)at);
+      f[d].half[1] =
+          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + 8 * AP_ROWB));
+    }
+  };
+  VF vf[2][4];
+  read_v(0, vf[0]);
+  float sum0 = 0.f, sum1 = 0.f;
+#pragma unroll
+  for (int k = 0; k < NB * 2; ++k) {  // 16 tokens
+    if (k + 1 < NB * 2) read_v(k + 1, vf[(k + 1) & 1]);
+    float p[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      p[j] = __builtin_amdgcn_exp2f(fmaf(s[k / 2][(k & 1) * 8 + j], sc, mz));
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) { sum0 += p[j]; sum1 += p[j + 1]; }
+    bf16x8 pf, pr;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      pf[j] = (__bf16)p[j];
+      if (FINE) pr[j] = (__bf16)(p[j] - (float)pf[j]);
+    }
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      c.o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[k & 1][d].b, pf, c.o[d],
+                                                       0, 0, 0);
+      if (FINE)
+        c.o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[k & 1][d].b, pr,
+                                                         c.o[d], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  c.l += sum0 + sum1;
 }
 
 template <int G>
-__global__ void __launch_bounds__(256) attn_prefill_kernel(
-    u16* __restrict__ out, const u16* __restrict__ q,
-    const u16* __restrict__ kc, const u16* __restrict__ vc,
-    const i32* __restrict__ bt, const i32* __restrict__ qstart,
-    const i32* __restrict__ cu_seqlens,
-    const i32* __restrict__ tile_seq, const i32* __restrict__ tile_q0,
-    float scale, int Hq, int Hk, i64 qs, int page_size, int max_pages,
-    int win) {
-  const int tile = blockIdx.x, kvh = blockIdx.y;
-  const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int seq = tile_seq[tile];
-  const int seq_start = cu_seqlens[seq];
-  const int len = cu_seqlens[seq + 1] - seq_start;  // chunk rows
-  const int hist = qstart[seq];                     // cached tokens before chunk
-  const i32* btrow = bt + (size_t)seq * max_pages;
-
-  constexpr int ROWTILES = (G >= 4) ? 1 : (4 / G);   // 16-row tiles per WG
-  constexpr int ROWS = 16 * ROWTILES;
-  constexpr int HLOOP = (G >= 4) ? (G / 4) : 1;      // heads per wave
-
-  const int my_tile = (G >= 4) ? 0 : (wid / G);
-  const int g0 = (G >= 4) ? wid : (wid % G);
-  const int q0 = tile_q0[tile] + my_tile * 16;        // abs q row of wave tile
-
-  __shared__ u16 k_lds[AP_KVBLK * AP_D];              // swizzled rows
-  __shared__ u16 v_lds[AP_D][AP_VPAD];                // transposed, tok-paired
-  __shared__ u16 p_lds[4][16][AP_VPAD];               // per-wave P tile
-
-  // ---- load Q fragments (stay in registers for all KV tiles) ----
-  const int qrow_frag = min(q0 + (lane & 15), len - 1);
-  s16x8 q_frag[HLOOP][4];
+__device__ __forceinline__ void load_columns(const PrefillArgs& a, Columns& c,
+                                             int row, int head, int seq_start,
+                                             int len, int hist) {
+  const int h = (threadIdx.x & 63) >> 5;
+  const u16* qp = a.q + (size_t)(seq_start + min(row, len - 1)) * a.qs +
+                  head * AP_D + h * 8;
 #pragma unroll
-  for (int hl = 0; hl < HLOOP; ++hl) {
-    const int qh = kvh * G + g0 + hl * 4;
-    const u16* qp = q + (size_t)(seq_start + qrow_frag) * qs + qh * AP_D +
-                    (lane >> 4) * 8;
+  for (int d = 0; d < 8; ++d) c.q[d] = *reinterpret_cast<const s16x8*>(qp + d * 16);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) q_frag[hl][c] = lds_read8(qp + c * 32);
+  for (int d = 0; d < 4; ++d)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) c.o[d][r] = 0.f;
+  c.m = AF_NEG_INF;
+  c.l = 0.f;
+  c.qpos = hist + min(row, len - 1);
+}
+
+template <int G, bool TILED>
+__global__ void __launch_bounds__(256, 2) attn_prefill_kernel(PrefillArgs a,
+                                                              int items) {
+  constexpr int ROWS = 128 / G, WROWS = 32 / G;
+  const int kvh = blockIdx.x % a.Hk;
+  int at;
+  const int seq = find_item<G, false>(a, items - 1 - (int)(blockIdx.x / a.Hk), &at);
+  if (seq < 0) return;  // lengths on the device say less than the host's
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int seq_start = a.cu[seq], len = a.cu[seq + 1] - seq_start;
+  const int hist = a.qstart[seq];
+  const i32* btrow = a.bt + (size_t)seq * a.max_pages;
+  const int q0 = at * ROWS;
+
+  __shared__ __attribute__((aligned(16))) char lds[2][2][AP_KV * AP_ROWB];
+  auto kbuf = [&](int i) { return (lds_char*)&lds[i][0][0]; };
+  auto vbuf = [&](int i) { return (lds_char*)&lds[i][1][0]; };
+
+  const int col = lane & 31;
+  const int row = q0 + wid * WROWS + col / G;
+  const int qh = kvh * G + col % G;
+  Columns c;
+  load_columns<G>(a, c, row, qh, seq_start, len, hist);
+  const float sc = a.scale * 1.44269504088896f;
+  // positions of this wave's first and last row (none: no work but staging)
+  const bool some = q0 + wid * WROWS < len;
+  const int p0 = hist + q0 + wid * WROWS;
+  const int p1 = hist + min(q0 + wid * WROWS + WROWS, len) - 1;
+
+  // tokens visible to this block: history + chunk rows up to the causal bound,
+  // and (sliding window) nothing below the first row's window
+  const int last = hist + len - 1;
+  const int ntiles = (min(last + 1, hist + q0 + ROWS) + AP_KV - 1) / AP_KV;
+  int kt = a.win > 0 ? max(0, hist + q0 - a.win + 1) / AP_KV : 0;
+  auto page_of = [&](int tile) {
+    const int t = min(tile, ntiles - 1) * AP_KV;
+    return btrow[a.page_shift >= 0 ? t >> a.page_shift : t / a.page_size];
+  };
+  stage<TILED, 4>(a, btrow, kvh, kt * AP_KV, wid * 16, last,
+                  TILED ? page_of(kt) : 0, kbuf(0), vbuf(0));
+  int page = TILED ? page_of(kt + 1) : 0;
+  int cur = 0;
+  __syncthreads();
+  for (; kt < ntiles; ++kt) {
+    if (kt + 1 < ntiles) {
+      stage<TILED, 4>(a, btrow, kvh, (kt + 1) * AP_KV, wid * 16, last, page,
+                      kbuf(cur ^ 1), vbuf(cur ^ 1));
+      if (TILED) page = page_of(kt + 2);
+    }
+    const int t0 = kt * AP_KV;
+    if (some && t0 <= p1 && (a.win <= 0 || t0 + AP_KV - 1 > p0 - a.win)) {
+      attend<2, false>(c, kbuf(cur), vbuf(cur), t0, sc, a.win,
+                t0 + AP_KV - 1 > p0 || (a.win > 0 && t0 <= p1 - a.win));
+    }
+    __syncthreads();  // next tile has landed, this one is free
+    cur ^= 1;
   }
 
-  float m[HLOOP][4], l[HLOOP][4];
-  f32x4 o_acc[HLOOP][8];  // 8 d-tiles of 16
+  const float l = c.l + __shfl_xor(c.l, 32, 64);
+  if (row >= len) return;
+  const float inv = (l > 0.f) ? 1.f / l : 0.f;
+  u16* op = a.out + (size_t)(seq_start + row) * (a.Hq * AP_D) + qh * AP_D +
+            4 * (lane >> 5);
 #pragma unroll
-  for (int hl = 0; hl < HLOOP; ++hl) {
+  for (int d = 0; d < 4; ++d)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) { m[hl][r] = AF_NEG_INF; l[hl][r] = 0.f; }
+    for (int r = 0; r < 16; r += 4) {
+      s16x4 v;
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) o_acc[hl][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < 4; ++j) v[j] = (short)f2bf(c.o[d][r + j] * inv);
+      *reinterpret_cast<s16x4*>(op + d * 32 + 2 * r) = v;
+    }
+}
+
+// po [items, Hk, nsplit, 32, D] f32, pml [items, Hk, nsplit, 32, 2] f32: used
+// with nsplit > 1 only.
+template <int G, bool TILED>
+__global__ void __launch_bounds__(256, 1) attn_prefill_few_kernel(
+    PrefillArgs a, float* __restrict__ po, float* __restrict__ pml, int nsplit) {
+  const int kvh = blockIdx.x % a.Hk;
+  int at;
+  const int seq = find_item<G, true>(a, blockIdx.x / a.Hk, &at);
+  if (seq < 0) return;  // lengths on the device say less than the host's
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int seq_start = a.cu[seq], len = a.cu[seq + 1] - seq_start;
+  const int hist = a.qstart[seq];
+  const i32* btrow = a.bt + (size_t)seq * a.max_pages;
+
+  constexpr int TILE = AP_FEW * AP_ROWB, WROWS = 32 / G;
+  __shared__ __attribute__((aligned(16))) char lds[4][2][2][TILE];
+  __shared__ float s_m[4][32], s_l[4][32];
+  auto kbuf = [&](int i) { return (lds_char*)&lds[wid][i][0][0]; };
+  auto vbuf = [&](int i) { return (lds_char*)&lds[wid][i][1][0]; };
+
+  const int col = lane & 31;
+  const int row = at * WROWS + col / G, qh = kvh * G + col % G;
+  const int nrows = min(WROWS, len - at * WROWS);
+  Columns c;
+  load_columns<G>(a, c, row, qh, seq_start, len, hist);
+  const float sc = a.scale * 1.44269504088896f;
+  const int last = hist + len - 1;
+  const int p0 = hist + at * WROWS, p1 = p0 + nrows - 1;
+  const int ntiles = (p1 + AP_FEW) / AP_FEW;
+  const int first = a.win > 0 ? max(0, p0 - a.win + 1) / AP_FEW : 0;
+  const int step = 4 * nsplit;
+  auto page_of = [&](int tile) {
+    const int t = min(tile, ntiles - 1) * AP_FEW;
+    return btrow[a.page_shift >= 0 ? t >> a.page_shift : t / a.page_size];
+  };
+  int kt = first + (int)blockIdx.y * 4 + wid, page = 0, cur = 0;
+  if (kt < ntiles) {
+    stage<TILED, 8>(a, btrow, kvh, kt * AP_FEW, 0, last, TILED ? page_of(kt) : 0,
+                    kbuf(0), vbuf(0));
+    if (TILED) page = page_of(kt + step);
+  }
+  for (; kt < ntiles; kt += step) {
+    if (kt + step < ntiles) {
+      stage<TILED, 8>(a, btrow, kvh, (kt + step) * AP_FEW, 0, last, page,
+                      kbuf(cur ^ 1), vbuf(cur ^ 1));
+      if (TILED) page = page_of(kt + 2 * step);
+      // all but the 16 loads just issued have landed
+      asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    const int t0 = kt * AP_FEW;
+    attend<1, true>(c, kbuf(cur), vbuf(cur), t0, sc, a.win,
+                    t0 + AP_FEW - 1 > p0 || (a.win > 0 && t0 <= p1 - a.win));
+    // this tile's reads are done before its buffer is filled again
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    cur ^= 1;
   }
 
-  // tokens visible to this WG: history + chunk rows up to the causal bound,
-  // and (sliding window) nothing below qrow_min - win + 1
-  const int kv_end = min(hist + len, hist + tile_q0[tile] + ROWS);
-  const int n_kv_tiles = (kv_end + AP_KVBLK - 1) / AP_KVBLK;
-  const int kv_total = hist + len;
-  const int kt_first =
-      (win > 0) ? max(0, hist + tile_q0[tile] - win + 1) / AP_KVBLK : 0;
-
-  for (int kt = kt_first; kt < n_kv_tiles; ++kt) {
-    const int kv0 = kt * AP_KVBLK;
-    __syncthreads();  // previous iteration's frag reads done
-    // ---- stage K (swizzled) from the paged cache ----
-    for (int i = threadIdx.x; i < AP_KVBLK * (AP_D / 8); i += 256) {
-      const int tok = i / (AP_D / 8);
-      const int d8 = (i % (AP_D / 8)) * 8;
-      const int tg = min(kv0 + tok, kv_total - 1);
-      const i64 page = btrow[tg / page_size];
-      const size_t src =
-          (((size_t)page * Hk + kvh) * page_size + (tg % page_size)) * AP_D + d8;
-      s16x8 kv8 = lds_read8(kc + src);
-      const int byte = tok * (AP_D * 2) + ((d8 * 2) ^ ((tok & 7) << 4));
-      *reinterpret_cast<s16x8*>(reinterpret_cast<char*>(k_lds) + byte) = kv8;
+  // merge the waves: O^T as [wave][column][dim] in the tile buffers
+  const float l = c.l + __shfl_xor(c.l, 32, 64);
+  __syncthreads();
+  float* so = reinterpret_cast<float*>(&lds[0][0][0][0]);
+  if (lane < 32) { s_m[wid][col] = c.m; s_l[wid][col] = l; }
+  float* mine = so + (size_t)(wid * 32 + col) * AP_D + 4 * (lane >> 5);
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+#pragma unroll
+    for (int r = 0; r < 16; r += 4)
+      *reinterpret_cast<f32x4*>(mine + d * 32 + 2 * r) =
+          f32x4{c.o[d][r], c.o[d][r + 1], c.o[d][r + 2], c.o[d][r + 3]};
+  __syncthreads();
+  for (int i = threadIdx.x; i < nrows * G * (AP_D / 4); i += 256) {
+    const int cc = i / (AP_D / 4), d = (i % (AP_D / 4)) * 4;
+    float M = s_m[0][cc];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) M = fmaxf(M, s_m[w][cc]);
+    float L = 0.f;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float f = (s_m[w][cc] <= AF_NEG_INF)
+                          ? 0.f
+                          : __builtin_amdgcn_exp2f((s_m[w][cc] - M) * sc);
+      L += s_l[w][cc] * f;
+      const f32x4 v = *reinterpret_cast<const f32x4*>(so + (size_t)(w * 32 + cc) * AP_D + d);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] += v[j] * f;
     }
-    // ---- stage V transposed: token pairs -> u32 writes (8 per 2 loads).
-    // Lane decomposition: consecutive lanes take consecutive token pairs at
-    // the SAME d-slice, so the 8 v_lds writes land in consecutive words
-    // (bank-conflict-free).  The d8-major variant put 16 lanes on one bank
-    // (d8 stride x 36-word rows = 0 mod 32): PMC measured 1.7e8
-    // SQ_LDS_BANK_CONFLICT per dispatch (profiles/pmc_r01_counters.txt).
-    for (int i = threadIdx.x; i < (AP_KVBLK / 2) * (AP_D / 8); i += 256) {
-      const int tp = i % (AP_KVBLK / 2);      // token pair (consecutive lanes)
-      const int d8 = (i / (AP_KVBLK / 2)) * 8;
-      const int t0g = kv0 + tp * 2;
-      const int c0 = min(t0g, kv_total - 1), c1 = min(t0g + 1, kv_total - 1);
-      const size_t s0 = (((size_t)btrow[c0 / page_size] * Hk + kvh) * page_size +
-                         (c0 % page_size)) * AP_D + d8;
-      const size_t s1 = (((size_t)btrow[c1 / page_size] * Hk + kvh) * page_size +
-                         (c1 % page_size)) * AP_D + d8;
-      s16x8 a = (t0g < kv_total) ? lds_read8(vc + s0)
-                                 : s16x8{0, 0, 0, 0, 0, 0, 0, 0};
-      s16x8 b = (t0g + 1 < kv_total) ? lds_read8(vc + s1)
-                                     : s16x8{0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const uint32_t packed = (uint32_t)(unsigned short)a[j] |
-                                ((uint32_t)(unsigned short)b[j] << 16);
-        *reinterpret_cast<uint32_t*>(&v_lds[d8 + j][tp * 2]) = packed;
-      }
+    if (nsplit > 1) {
+      const size_t to = ((size_t)blockIdx.x * nsplit + blockIdx.y) * 32 + cc;
+      *reinterpret_cast<f32x4*>(po + to * AP_D + d) = o;
+      if (d == 0) { pml[to * 2] = M; pml[to * 2 + 1] = L; }
+      continue;
     }
-    __syncthreads();
-
+    const float inv = (L > 0.f) ? 1.f / L : 0.f;
+    s16x4 v;
 #pragma unroll
-    for (int hl = 0; hl < HLOOP; ++hl) {
-      // ---- QK^T: four 16-token sub-tiles ----
-      f32x4 s_acc[4];
-#pragma unroll
-      for (int st = 0; st < 4; ++st) {
-        s_acc[st] = f32x4{0, 0, 0, 0};
-        const int tok = st * 16 + (lane & 15);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int byte = tok * (AP_D * 2) +
-                           (((c * 32 + (lane >> 4) * 8) * 2) ^ ((tok & 7) << 4));
-          s16x8 kf = *reinterpret_cast<const s16x8*>(
-              reinterpret_cast<const char*>(k_lds) + byte);
-          s_acc[st] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              as_bf16x8(q_frag[hl][c]), as_bf16x8(kf), s_acc[st], 0, 0, 0);
-        }
-      }
-      // ---- mask + online softmax (C-layout: reg r = qrow (lane>>4)*4+r) ----
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int qrow = hist + q0 + (lane >> 4) * 4 + r;  // absolute position
-        float sr[4];
-        float tmax = AF_NEG_INF;
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-          sr[st] = s_acc[st][r] * scale;
-          const int kpos = kv0 + st * 16 + (lane & 15);
-          if (kpos > qrow || (win > 0 && kpos <= qrow - win))
-            sr[st] = AF_NEG_INF;
-          tmax = fmaxf(tmax, sr[st]);
-        }
-        tmax = group16_max_f32(tmax);
-        const float mn = fmaxf(m[hl][r], tmax);
-        const float corr = (m[hl][r] <= AF_NEG_INF) ? 0.f : __expf(m[hl][r] - mn);
-        float psum = 0.f;
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-          sr[st] = (sr[st] <= AF_NEG_INF) ? 0.f : __expf(sr[st] - mn);
-          psum += sr[st];
-          s_acc[st][r] = sr[st];  // reuse acc regs to carry P
-        }
-        l[hl][r] = l[hl][r] * corr + group16_sum_f32(psum);
-        m[hl][r] = mn;
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) o_acc[hl][dt][r] *= corr;
-      }
-      // ---- P -> per-wave LDS (C-layout -> A-fragment layout) ----
-#pragma unroll
-      for (int st = 0; st < 4; ++st)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          p_lds[wid][(lane >> 4) * 4 + r][st * 16 + (lane & 15)] =
-              f2bf(s_acc[st][r]);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      s16x8 p_frag0 = lds_read8(&p_lds[wid][lane & 15][(lane >> 4) * 8]);
-      s16x8 p_frag1 = lds_read8(&p_lds[wid][lane & 15][32 + (lane >> 4) * 8]);
-      // ---- PV: o_acc[dt] += P(16x64) @ V(64x16), two K=32 chunks ----
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt) {
-        const u16* vrow = &v_lds[dt * 16 + (lane & 15)][0];
-        s16x8 vf0 = lds_read8(vrow + (lane >> 4) * 8);
-        s16x8 vf1 = lds_read8(vrow + 32 + (lane >> 4) * 8);
-        o_acc[hl][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            as_bf16x8(p_frag0), as_bf16x8(vf0), o_acc[hl][dt], 0, 0, 0);
-        o_acc[hl][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            as_bf16x8(p_frag1), as_bf16x8(vf1), o_acc[hl][dt], 0, 0, 0);
-      }
-    }
-  }
-
-  // ---- epilogue: out = o_acc / l ----
-#pragma unroll
-  for (int hl = 0; hl < HLOOP; ++hl) {
-    const int qh = kvh * G + g0 + hl * 4;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int qrow = q0 + (lane >> 4) * 4 + r;
-      if (qrow >= len) continue;
-      const float inv = (l[hl][r] > 0.f) ? 1.f / l[hl][r] : 0.f;
-      u16* op = out + (size_t)(seq_start + qrow) * (Hq * AP_D) + qh * AP_D +
-                (lane & 15);
-#pragma unroll
-      for (int dt = 0; dt < 8; ++dt) op[dt * 16] = f2bf(o_acc[hl][dt][r] * inv);
-    }
+    for (int j = 0; j < 4; ++j) v[j] = (short)f2bf(o[j] * inv);
+    *reinterpret_cast<s16x4*>(a.out +
+                              (size_t)(seq_start + at * WROWS + cc / G) * (a.Hq * AP_D) +
+                              (kvh * G + cc % G) * AP_D + d) = v;
   }
 }
 
-AF_EXPORT int af_attn_prefill(void* out, const void* q, const void* kc,
-                              const void* vc, const void* bt, const void* qstart,
-                              const void* cu_seqlens, const void* tile_seq,
-                              const void* tile_q0, float scale, int ntiles,
-                              int Hq, int Hk, int D, i64 qs, int page_size,
-                              int max_pages, int win, void* stream) {
+// Merge of the few-kernel's key splits; blocks as there.
+template <int G>
+__global__ void __launch_bounds__(256) attn_prefill_merge_kernel(
+    PrefillArgs a, const float* __restrict__ po, const float* __restrict__ pml,
+    int nsplit) {
+  const int kvh = blockIdx.x % a.Hk;
+  int at;
+  const int seq = find_item<G, true>(a, blockIdx.x / a.Hk, &at);
+  if (seq < 0) return;
+  const int seq_start = a.cu[seq], len = a.cu[seq + 1] - seq_start;
+  const int row0 = at * (32 / G), nrows = min(32 / G, len - row0);
+  const float sc = a.scale * 1.44269504088896f;
+  const size_t from = (size_t)blockIdx.x * nsplit * 32;
+  for (int i = threadIdx.x; i < nrows * G * (AP_D / 4); i += 256) {
+    const int cc = i / (AP_D / 4), d = (i % (AP_D / 4)) * 4;
+    float M = AF_NEG_INF;
+    for (int s = 0; s < nsplit; ++s) M = fmaxf(M, pml[(from + s * 32 + cc) * 2]);
+    float L = 0.f;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < nsplit; ++s) {
+      const float m = pml[(from + s * 32 + cc) * 2];
+      const float f = (m <= AF_NEG_INF) ? 0.f : __builtin_amdgcn_exp2f((m - M) * sc);
+      L += pml[(from + s * 32 + cc) * 2 + 1] * f;
+      const f32x4 v =
+          *reinterpret_cast<const f32x4*>(po + (from + s * 32 + cc) * AP_D + d);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] += v[j] * f;
+    }
+    const float inv = (L > 0.f) ? 1.f / L : 0.f;
+    s16x4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = (short)f2bf(o[j] * inv);
+    *reinterpret_cast<s16x4*>(a.out +
+                              (size_t)(seq_start + row0 + cc / G) * (a.Hq * AP_D) +
+                              (kvh * G + cc % G) * AP_D + d) = v;
+  }
+}
+
+// items: 128-column items of the sequences with more than few_cols columns; few:
+// 32-column items of the others, their keys cut nsplit ways with the partial
+// results in po / pml (all per K/V head).
+AF_EXPORT int af_attn_prefill(void* out, void* po, void* pml, const void* q,
+                              const void* kc, const void* vc, const void* bt,
+                              const void* qstart, const void* cu_seqlens,
+                              float scale, int nseq, int items, int few,
+                              int few_cols, int nsplit, int Hq, int Hk, int D,
+                              i64 qs, int page_size, int max_pages, int win,
+                              void* stream) {
   if (D != AP_D) return 9002;
   const int G = Hq / Hk;
   if (G * Hk != Hq) return 9003;
-  if (ntiles == 0) return 0;
-  dim3 grid(ntiles, Hk), blk(256);
   hipStream_t st = (hipStream_t)stream;
+  const bool pow2 = (page_size & (page_size - 1)) == 0;
+  const PrefillArgs a = {(u16*)out, (const u16*)q, (const u16*)kc, (const u16*)vc,
+                         (const i32*)bt, (const i32*)qstart,
+                         (const i32*)cu_seqlens, scale, nseq, Hq, Hk, qs,
+                         page_size, pow2 ? __builtin_ctz(page_size) : -1,
+                         max_pages, win, few_cols};
+  float* fo = (float*)po;
+  float* fm = (float*)pml;
+  const dim3 gf(few * Hk, nsplit);
 #define AF_LAUNCH(GG)                                                           \
-  attn_prefill_kernel<GG><<<grid, blk, 0, st>>>(                                \
-      (u16*)out, (const u16*)q, (const u16*)kc, (const u16*)vc,                 \
-      (const i32*)bt, (const i32*)qstart,                                       \
-      (const i32*)cu_seqlens, (const i32*)tile_seq, (const i32*)tile_q0,        \
-      scale, Hq, Hk, qs, page_size, max_pages, win)
+  do {                                                                          \
+    if (items > 0) {                                                            \
+      if (page_size % AP_KV == 0)                                               \
+        attn_prefill_kernel<GG, true><<<items * Hk, 256, 0, st>>>(a, items);    \
+      else                                                                      \
+        attn_prefill_kernel<GG, false><<<items * Hk, 256, 0, st>>>(a, items);   \
+    }                                                                           \
+    if (few > 0) {                                                              \
+      if (page_size % AP_FEW == 0)                                              \
+        attn_prefill_few_kernel<GG, true><<<gf, 256, 0, st>>>(a, fo, fm, nsplit); \
+      else                                                                      \
+        attn_prefill_few_kernel<GG, false><<<gf, 256, 0, st>>>(a, fo, fm, nsplit); \
+      if (nsplit > 1)                                                           \
+        attn_prefill_merge_kernel<GG><<<few * Hk, 256, 0, st>>>(a, fo, fm, nsplit); \
+    }                                                                           \
+  } while (0)
   switch (G) {
     case 1: AF_LAUNCH(1); break;
     case 2: AF_LAUNCH(2); break;

@@ -1,0 +1,606 @@
+// Weight-streaming GEMMs for up to 128 rows:  Y[M,N] = X[M,K] @ W[N,K]^T with
+// the step that follows it in a decoder layer.
+//
+// A decode step reads every weight once, so a layer's four projections are bound
+// by the weight stream and by what a launch costs (~4.6 us in a captured step).
+// Weights and X travel global -> LDS without registers, a whole 128-byte line per
+// row and load: operand loads straight to registers (16 rows x 64 bytes per
+// instruction) stop at ~7.6 TB/s of requests whatever is asked for, so X at 16
+// rows doubled the time.  16-byte chunks are permuted within a line by the row
+// number (the operand reads then do not meet in a bank), and the loads of the
+// next pieces are in flight while one is multiplied (counted waits).
+//
+// gemm_rows_kernel, up to 32 rows: a block owns one tile of 16 weight rows (N =
+//   4096 gives 256 tiles, one per CU; N = 28672 seven per CU) and K is split over
+//   its 8 WAVES, which take 64-element pieces in turn, each through buffers of its
+//   own: no barrier in the loop, no partial sums in memory and no second launch.
+//   The waves' sums meet once, in LDS, in an order that does not depend on M.
+//   The epilogue is the layer's next step: bf16 store, residual add in place,
+//   SwiGLU (a tile is 8 gate and 8 up rows), or rotary embedding + page append (a
+//   tile is 8 rotation pairs of a head).  RMSNorm (its weight is folded into W):
+//   the loop multiplies every X fragment with itself (diagonal of X X^T, one
+//   MFMA), so nobody has to leave row statistics behind.
+// gemm_tile_kernel, more rows: X would be read once per 16 weight rows, so here
+//   four waves own 16 weight rows each and share X: 64 weight rows per block and
+//   STAGES pieces in a ring with one barrier per piece.  K is split over blocks
+//   where N alone does not fill the chip, the fp32 parts meet in the kernel that
+//   does the next step.
+// Measured in TB/s of weights (us), against the split-K kernel with two-stage
+// buffers and its second launch (in brackets): one row, 6144 x 4096 with rotary
+// and append 11.8 us (21.3 in three launches), 4096 x 4096 8.3, 4096 x 14336 22.4
+// (together 30.7; 44.4), SwiGLU over 28672 x 4096 42.9 = 5.5 TB/s (58.2).  16
+// rows: 13.9, 8.9, 24.7, 47.4.  64 rows, without the closing launches: 13.4, 9.0,
+// 24.8, 53.1 (16.7, o + down 44.8, 62.7).  128 rows: 16.4, 13.0, 28.3, 61.6
+// (library 25.6 and 57.5 + 5.2 for the first and the last, o + down 63.1).
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8r;
+typedef __attribute__((address_space(3))) char lds_b;
+typedef __attribute__((address_space(3))) s16x8 lds_v8;
+
+__device__ __forceinline__ bf16x8r as_bf16x8r(s16x8 v) {
+  union { s16x8 s; bf16x8r b; } u;
+  u.s = v;
+  return u.b;
+}
+
+enum RowsEpi { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_ROPE = 3,
+               EPI_PARTS = 4 };
+
+struct RowsArgs {
+  u16* out;            // [M, N] ([M, N/2] SwiGLU; [M, Hq*128] rope: q only)
+  u16* residual;       // [M, N], updated in place (EPI_RESIDUAL)
+  float* parts;        // [splits, M, N] (EPI_PARTS)
+  const u16* X;
+  const u16* W;
+  int M, N, K;
+  const float* ss;     // [M, 8] row sums of squares of X (norm 1)
+  float eps;
+  // EPI_ROPE
+  const i32* pos;
+  const float* table;  // [positions, 128]: cos | sin
+  u16* kc;
+  u16* vc;
+  const i64* slot;
+  int Hq, Hk, page_size;
+};
+
+// 8 rows x 128 bytes of a row-major matrix into linear LDS: lane l brings chunk
+// (l & 7) ^ (row & 7) of row l >> 3, so that chunk c of row r sits at slot
+// c ^ (r & 7).
+__device__ __forceinline__ void load_line8(const u16* src, lds_b* dst) {
+  __builtin_amdgcn_global_load_lds(
+      (const __attribute__((address_space(1))) uint32_t*)src,
+      (__attribute__((address_space(3))) uint32_t*)dst, 16, 0, 0);
+}
+
+// operand fragment: lane (r = lane & 15, q = lane >> 4) gets k = 32 h + 8 q .. +8
+// of row r of a 16-row piece
+__device__ __forceinline__ bf16x8r frag(const lds_b* piece, int h) {
+  const int lane = threadIdx.x & 63, r = lane & 15;
+  const int c = (h * 4 + (lane >> 4)) ^ (r & 7);
+  return as_bf16x8r(*reinterpret_cast<const lds_v8*>(piece + r * 128 + c * 16));
+}
+
+// W row of row n of a 16-row tile
+template <int EPI>
+__device__ __forceinline__ int weight_row(const RowsArgs& a, int tile, int n) {
+  if (EPI == EPI_SWIGLU) return (n < 8 ? 0 : (a.N >> 1) - 8) + tile * 8 + n;
+  if (EPI == EPI_ROPE) {
+    const int head = tile >> 3, j = tile & 7;
+    return head * 128 + (head >= a.Hq + a.Hk ? j * 16 + n
+                                             : j * 8 + n + (n < 8 ? 0 : 56));
+  }
+  return tile * 16 + n;
+}
+
+// Rotated q / k pair (dims d, d + 64) or plain v pair (dims d, d + 1) of row m to
+// its place.  head counts q, k, v heads in turn.
+__device__ __forceinline__ void put_rope(const RowsArgs& a, int m, int head, int d,
+                                         float x1, float x2) {
+  const bool is_q = head < a.Hq, is_v = head >= a.Hq + a.Hk;
+  const i64 s = a.slot[m];
+  const i64 page = (s >= 0) ? s / a.page_size : 0;
+  const i64 off = (s >= 0) ? s % a.page_size : 0;
+  if (is_v) {
+    if (s < 0) return;
+    u16* row = a.vc + (((size_t)page * a.Hk + head - a.Hq - a.Hk) * a.page_size +
+                       off) * 128 + d;
+    *reinterpret_cast<u16x2*>(row) = u16x2{f2bf(x1), f2bf(x2)};
+    return;
+  }
+  const float* tab = a.table + (size_t)a.pos[m] * 128 + d;
+  const float cs = tab[0], sn = tab[64];
+  const u16 y1 = f2bf(x1 * cs - x2 * sn), y2 = f2bf(x2 * cs + x1 * sn);
+  if (is_q) {
+    u16* row = a.out + (size_t)m * (a.Hq * 128) + head * 128 + d;
+    row[0] = y1;
+    row[64] = y2;
+  } else if (s >= 0) {
+    u16* row = a.kc + (((size_t)page * a.Hk + head - a.Hq) * a.page_size + off) *
+                          128 + d;
+    row[0] = y1;
+    row[64] = y2;
+  }
+}
+
+// NORM: 0 none, 1 from ss, 2 computed from X.  PD pieces per wave in flight.
+template <int MT, int PD, int EPI, int NORM>
+__global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
+  constexpr int NW = 8;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int n = lane & 15;
+  const int tile = blockIdx.x;
+
+  constexpr int PIECE = 2048;                    // 16 rows x 64 elements
+  constexpr int SLOT = PIECE * (1 + MT);
+  constexpr int RS = MT * 16 + 4;                // column stride of the sums
+  constexpr int RING = NW * PD * SLOT;
+  constexpr int SUMS = NW * 16 * RS * 4;
+  __shared__ __attribute__((aligned(16))) char lds[RING > SUMS ? RING : SUMS];
+  __shared__ float rsq[NW][MT * 16];
+  __shared__ float rstd[MT * 16];
+  lds_b* ring = (lds_b*)&lds[wid * PD * SLOT];
+
+  // sources of this lane's chunks
+  const int r8 = lane >> 3, ch = ((lane & 7) ^ r8) * 8 + wid * 64;
+  const u16* wp[2];
+  const u16* xp[MT * 2];
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+    wp[g] = a.W + (size_t)weight_row<EPI>(a, tile, g * 8 + r8) * a.K + ch;
+#pragma unroll
+  for (int g = 0; g < MT * 2; ++g)
+    xp[g] = a.X + (size_t)min(g * 8 + r8, a.M - 1) * a.K + ch;
+  auto load = [&](int i) {
+    lds_b* to = ring + (i % PD) * SLOT;
+    const size_t off = (size_t)i * (NW * 64);
+#pragma unroll
+    for (int g = 0; g < 2; ++g) load_line8(wp[g] + off, to + g * 1024);
+#pragma unroll
+    for (int g = 0; g < MT * 2; ++g)
+      load_line8(xp[g] + off, to + PIECE + g * 1024);
+  };
+  f32x4 acc[MT], sq[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    acc[m] = f32x4{0, 0, 0, 0};
+    sq[m] = f32x4{0, 0, 0, 0};
+  }
+  const int cnt = ((a.K >> 6) - wid + NW - 1) / NW;  // this wave's pieces
+#pragma unroll
+  for (int s = 0; s < PD; ++s)
+    if (s < cnt) load(s);
+  for (int i = 0; i < cnt; ++i) {
+    // piece i has landed when only the loads of the PD - 1 behind it are out
+    if (i + PD <= cnt) {
+      if (PD == 2) {
+        if (MT == 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+      } else if (PD == 3) {
+        if (MT == 1) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+      } else {
+        static_assert(PD <= 4, "wait counts");
+        if (MT == 1) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(18)" ::: "memory");
+      }
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    const lds_b* at = ring + (i % PD) * SLOT;
+    bf16x8r w[2], x[MT][2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      w[h] = frag(at, h);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) x[m][h] = frag(at + PIECE * (1 + m), h);
+    }
+    // the slot is read: fill it again
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (i + PD < cnt) load(i + PD);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[m][h], w[h], acc[m],
+                                                         0, 0, 0);
+        if (NORM == 2)
+          sq[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[m][h], x[m][h], sq[m],
+                                                          0, 0, 0);
+      }
+  }
+
+  // meet in LDS: [wave][tile column][row]; + 4 spreads the columns over banks
+  __syncthreads();
+  float (*red)[16][RS] = reinterpret_cast<float (*)[16][RS]>(lds);
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+    *reinterpret_cast<f32x4*>(&red[wid][n][m * 16 + (lane >> 4) * 4]) = acc[m];
+  if (NORM == 2) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if ((lane >> 4) * 4 + r == n) rsq[wid][m * 16 + n] = sq[m][r];
+  }
+  __syncthreads();
+  if (NORM != 0) {
+    if ((int)threadIdx.x < a.M) {
+      const int m = threadIdx.x;
+      float s = 0.f;
+      if (NORM == 2) {
+#pragma unroll
+        for (int w = 0; w < NW; ++w) s += rsq[w][m];
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s += a.ss[m * 8 + j];
+      }
+      rstd[m] = rsqrtf(s * (1.f / (float)a.K) + a.eps);
+    }
+    __syncthreads();
+  }
+  auto total = [&](int c, int m) {
+    float s = red[0][c][m];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) s += red[w][c][m];
+    return NORM != 0 ? s * rstd[m] : s;
+  };
+
+  // two values per thread: neighbours, or a gate / rotation pair
+  const int m = threadIdx.x >> 3, j = threadIdx.x & 7;
+  if (m >= a.M) return;
+  if (EPI == EPI_SWIGLU) {
+    const float g = total(j, m), u = total(8 + j, m);
+    a.out[(size_t)m * (a.N >> 1) + tile * 8 + j] = f2bf(g / (1.f + __expf(-g)) * u);
+  } else if (EPI == EPI_ROPE) {
+    const int head = tile >> 3, jt = tile & 7;
+    if (head >= a.Hq + a.Hk)
+      put_rope(a, m, head, jt * 16 + 2 * j, total(2 * j, m), total(2 * j + 1, m));
+    else
+      put_rope(a, m, head, jt * 8 + j, total(j, m), total(8 + j, m));
+  } else {
+    const size_t at = (size_t)m * a.N + tile * 16 + 2 * j;
+    float v0 = total(2 * j, m), v1 = total(2 * j + 1, m);
+    if (EPI == EPI_RESIDUAL) {
+      const u16x2 r = *reinterpret_cast<const u16x2*>(a.residual + at);
+      v0 += bf2f(r[0]);
+      v1 += bf2f(r[1]);
+      *reinterpret_cast<u16x2*>(a.residual + at) = u16x2{f2bf(v0), f2bf(v1)};
+      if (a.out == nullptr) return;
+    }
+    *reinterpret_cast<u16x2*>(a.out + at) = u16x2{f2bf(v0), f2bf(v1)};
+  }
+}
+
+// MT 16-row groups of X (even), ring of STAGES pieces of K = 64.  Grid
+// (N / 64, splits).  EPI_PLAIN, EPI_SWIGLU (not split) or EPI_PARTS.
+template <int N>
+__device__ __forceinline__ void wait_loads_and_meet() {
+  if constexpr (N == 0)
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  else if constexpr (N == 3)
+    asm volatile("s_waitcnt vmcnt(3) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  else if constexpr (N == 4)
+    asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  else if constexpr (N == 5)
+    asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  else if constexpr (N == 6)
+    asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  else if constexpr (N == 8)
+    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  else if constexpr (N == 9)
+    asm volatile("s_waitcnt vmcnt(9) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  else if constexpr (N == 10)
+    asm volatile("s_waitcnt vmcnt(10) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  else {
+    static_assert(N == 12, "wait counts");
+    asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+}
+
+template <int MT, int NW, int STAGES, int EPI, int NORM>
+__global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int n = lane & 15;
+  constexpr int PIECE = 2048;
+  constexpr int STAGE = PIECE * (NW + MT);
+  constexpr int XG = 2 * MT / NW;                // 8-row groups of X per wave
+  constexpr int PER = 2 + XG;                    // loads per wave and stage
+  static_assert(XG * NW == 2 * MT, "X rows divide among the waves");
+  __shared__ __attribute__((aligned(16))) char lds[STAGES * STAGE];
+  lds_b* ring = (lds_b*)&lds[0];
+
+  const int tile = blockIdx.x * NW + wid;         // this wave's 16 weight rows
+  const int pieces = a.K >> 6;
+  const int per = (pieces + (int)gridDim.y - 1) / (int)gridDim.y;
+  const int p0 = (int)blockIdx.y * per;
+  const int cnt = min(pieces, p0 + per) - p0;    // none empty (checked at launch)
+  const int r8 = lane >> 3, ch = ((lane & 7) ^ r8) * 8 + p0 * 64;
+  const u16* wp[2];
+  const u16* xp[XG];
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+    wp[g] = a.W + (size_t)weight_row<EPI>(a, tile, g * 8 + r8) * a.K + ch;
+#pragma unroll
+  for (int g = 0; g < XG; ++g)
+    xp[g] = a.X + (size_t)min((wid * XG + g) * 8 + r8, a.M - 1) * a.K + ch;
+  auto load = [&](int i) {
+    lds_b* to = ring + (i % STAGES) * STAGE;
+    const size_t off = (size_t)i * 64;
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+      load_line8(wp[g] + off, to + wid * PIECE + g * 1024);
+#pragma unroll
+    for (int g = 0; g < XG; ++g)
+      load_line8(xp[g] + off, to + NW * PIECE + (wid * XG + g) * 1024);
+  };
+  f32x4 acc[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) acc[m] = f32x4{0, 0, 0, 0};
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < cnt) load(s);
+  for (int i = 0; i < cnt; ++i) {
+    // stage i is complete for everybody, and stage i - 1 read by everybody
+    if (i + STAGES - 2 < cnt) wait_loads_and_meet<PER * (STAGES - 2)>();
+    else wait_loads_and_meet<0>();
+    if (i + STAGES - 1 < cnt) load(i + STAGES - 1);
+    const lds_b* at = ring + (i % STAGES) * STAGE;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const bf16x8r w = frag(at + wid * PIECE, h);
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            frag(at + PIECE * (NW + m), h), w, acc[m], 0, 0, 0);
+    }
+  }
+
+  // lane: column n of the tile, rows m*16 + (lane>>4)*4 + r
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = m * 16 + (lane >> 4) * 4 + r;
+      if (EPI == EPI_PARTS) {
+        if (row < a.M)
+          a.parts[((size_t)blockIdx.y * a.M + row) * a.N + tile * 16 + n] = acc[m][r];
+        continue;
+      }
+      float v = acc[m][r];
+      if (NORM == 1) {
+        const float* sp = a.ss + min(row, a.M - 1) * 8;
+        float s = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s += sp[j];
+        v *= rsqrtf(s * (1.f / (float)a.K) + a.eps);
+      }
+      if (EPI == EPI_SWIGLU) {
+        const float u = __int_as_float(__builtin_amdgcn_update_dpp(
+            0, __float_as_int(v), 0x128, 0xf, 0xf, true));  // row_ror:8
+        if (n < 8 && row < a.M)
+          a.out[(size_t)row * (a.N >> 1) + tile * 8 + n] =
+              f2bf(v / (1.f + __expf(-v)) * u);
+      } else if (row < a.M) {
+        a.out[(size_t)row * a.N + tile * 16 + n] = f2bf(v);
+      }
+    }
+}
+
+// The parts' sum + rotary positions + page append: grid (M, heads / 4), a head
+// per wave, a rotation (or value) pair per lane.
+__global__ void __launch_bounds__(256) rows_rope_kernel(RowsArgs a, int splits) {
+  const int m = blockIdx.x, lane = threadIdx.x & 63;
+  const int head = blockIdx.y * 4 + (threadIdx.x >> 6);
+  if (head >= a.Hq + 2 * a.Hk) return;
+  const bool is_v = head >= a.Hq + a.Hk;
+  const int d = is_v ? 2 * lane : lane, step = is_v ? 1 : 64;
+  float x1 = 0.f, x2 = 0.f;
+  for (int s = 0; s < splits; ++s) {
+    const float* p = a.parts + ((size_t)s * a.M + m) * a.N + head * 128 + d;
+    x1 += p[0];
+    x2 += p[step];
+  }
+  float q = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) q += a.ss[m * 8 + j];
+  const float rstd = rsqrtf(q * (1.f / (float)a.K) + a.eps);
+  put_rope(a, m, head, d, x1 * rstd, x2 * rstd);
+}
+
+// The parts' sum + residual (in place; a copy to `out` if given) + sums of squares
+// of the new rows (if ss is given): grid (M, 8), a block per eighth of a row.
+__global__ void __launch_bounds__(256) rows_residual_kernel(
+    u16* __restrict__ residual, u16* __restrict__ out,
+    const float* __restrict__ parts, float* __restrict__ ss, int M, int N,
+    int splits) {
+  const int m = blockIdx.x, nb = N / 8, c0 = blockIdx.y * nb;
+  __shared__ float red[4];
+  float local = 0.f;
+  for (int c = c0 + threadIdx.x * 2; c < c0 + nb; c += 512) {
+    const u16x2 rv = *reinterpret_cast<const u16x2*>(residual + (size_t)m * N + c);
+    float v0 = 0.f, v1 = 0.f;
+#pragma unroll 4
+    for (int s = 0; s < splits; ++s) {
+      const f32x2 p =
+          *reinterpret_cast<const f32x2*>(parts + ((size_t)s * M + m) * N + c);
+      v0 += p[0];
+      v1 += p[1];
+    }
+    const u16x2 o = {f2bf(v0 + bf2f(rv[0])), f2bf(v1 + bf2f(rv[1]))};
+    *reinterpret_cast<u16x2*>(residual + (size_t)m * N + c) = o;
+    if (out) *reinterpret_cast<u16x2*>(out + (size_t)m * N + c) = o;
+    const float b0 = bf2f(o[0]), b1 = bf2f(o[1]);  // stats of the rounded value
+    local += b0 * b0 + b1 * b1;
+  }
+  if (!ss) return;
+  local = wave_sum_f32(local);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = local;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    ss[m * 8 + blockIdx.y] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// The parts' sum in bf16, rows optionally scaled by the RMSNorm scalar from ss.
+__global__ void __launch_bounds__(256) rows_sum_kernel(
+    u16* __restrict__ out, const float* __restrict__ parts,
+    const float* __restrict__ ss, int M, int N, int splits, float inv_k,
+    float eps) {
+  const int m = blockIdx.x;
+  const int c = (blockIdx.y * 256 + threadIdx.x) * 2;
+  if (c >= N) return;
+  float v0 = 0.f, v1 = 0.f;
+#pragma unroll 4
+  for (int s = 0; s < splits; ++s) {
+    const f32x2 p =
+        *reinterpret_cast<const f32x2*>(parts + ((size_t)s * M + m) * N + c);
+    v0 += p[0];
+    v1 += p[1];
+  }
+  float rstd = 1.f;
+  if (ss) {
+    float q = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) q += ss[m * 8 + j];
+    rstd = rsqrtf(q * inv_k + eps);
+  }
+  *reinterpret_cast<u16x2*>(out + (size_t)m * N + c) =
+      u16x2{f2bf(v0 * rstd), f2bf(v1 * rstd)};
+}
+
+#define ROWS_MAX 16   // rows up to here: gemm_rows_kernel
+
+// Two pieces per wave in flight leave room for a second block per CU, which pays
+// when a CU has several tiles to go through; four are better when it has one:
+// 28672 x 4096 42.9 us against 50.6, 4096 x 14336 22.4 against 24.0 (one row).
+template <int EPI, int NORM>
+static void launch_rows(const RowsArgs& a, hipStream_t st) {
+  const int tiles = a.N / 16;
+  if (tiles > 256) gemm_rows_kernel<1, 2, EPI, NORM><<<tiles, 512, 0, st>>>(a);
+  else gemm_rows_kernel<1, 4, EPI, NORM><<<tiles, 512, 0, st>>>(a);
+}
+
+// Blocks of 128 weight rows (eight waves) halve the reads of X, from 33 rows on
+// for projections so wide that they fill the chip that way, always above 64.
+template <int EPI, int NORM>
+static void launch_tile(const RowsArgs& a, int splits, hipStream_t st) {
+  const dim3 g64(a.N / 64, splits), g128(a.N / 128, splits);
+  if (a.M <= 32) {
+    gemm_tile_kernel<2, 4, 4, EPI, NORM><<<g64, 256, 0, st>>>(a);
+  } else if (a.M <= 64) {
+    if (a.N % 128 == 0 && a.N / 128 >= 192)
+      gemm_tile_kernel<4, 8, 3, EPI, NORM><<<g128, 512, 0, st>>>(a);
+    else
+      gemm_tile_kernel<4, 4, 4, EPI, NORM><<<g64, 256, 0, st>>>(a);
+  } else {
+    if (a.N % 128 == 0)
+      gemm_tile_kernel<8, 8, 3, EPI, NORM><<<g128, 512, 0, st>>>(a);
+    else
+      gemm_tile_kernel<8, 4, 3, EPI, NORM><<<g64, 256, 0, st>>>(a);
+  }
+}
+
+static int check_rows(const RowsArgs& a, int splits) {
+  if (a.M < 1 || a.M > 128) return 9005;
+  if (a.N % 64 || a.K % 64 || a.K < 64) return 9006;
+  const int pieces = a.K / 64;
+  if (splits < 1 || splits > pieces) return 9003;
+  const int per = (pieces + splits - 1) / splits;
+  if ((splits - 1) * per >= pieces) return 9003;  // an empty split
+  return 0;
+}
+
+// mode 0 plain, 1 residual add (in place, also to `out` if given), 2 SwiGLU,
+// 4 residual add + row sums of squares of the result to ss_out [M, 8].
+// norm 0 none, 1 RMSNorm scalar of X from ss [M, 8], 2 computed (<= 16 rows).
+// parts [splits, M, N]: needed unless rows <= 16 (and mode 0..2) or mode 2.
+AF_EXPORT int af_rows_linear(void* out, void* residual, void* parts, void* ss_out,
+                             const void* X, const void* W, int M, int N, int K,
+                             int splits, int mode, int norm, const void* ss,
+                             float eps, void* stream) {
+  RowsArgs a = {};
+  a.out = (u16*)out;
+  a.residual = (u16*)residual;
+  a.parts = (float*)parts;
+  a.X = (const u16*)X;
+  a.W = (const u16*)W;
+  a.M = M; a.N = N; a.K = K;
+  a.ss = (const float*)ss;
+  a.eps = eps;
+  if (const int rc = check_rows(a, splits)) return rc;
+  if (mode != 0 && mode != 2 && norm != 0) return 9008;
+  hipStream_t st = (hipStream_t)stream;
+  if (M <= ROWS_MAX && mode != 4) {
+    if (mode == 0) {
+      if (norm == 0) launch_rows<EPI_PLAIN, 0>(a, st);
+      else if (norm == 1) launch_rows<EPI_PLAIN, 1>(a, st);
+      else launch_rows<EPI_PLAIN, 2>(a, st);
+    } else if (mode == 1) {
+      launch_rows<EPI_RESIDUAL, 0>(a, st);
+    } else if (mode == 2) {
+      if (norm == 0) launch_rows<EPI_SWIGLU, 0>(a, st);
+      else if (norm == 1) launch_rows<EPI_SWIGLU, 1>(a, st);
+      else launch_rows<EPI_SWIGLU, 2>(a, st);
+    } else {
+      return 9008;
+    }
+    return af_last_err();
+  }
+  if (norm == 2) return 9008;
+  if (mode == 2) {
+    if (norm == 0) launch_tile<EPI_SWIGLU, 0>(a, 1, st);
+    else launch_tile<EPI_SWIGLU, 1>(a, 1, st);
+    return af_last_err();
+  }
+  if (!parts) return 9008;
+  launch_tile<EPI_PARTS, 0>(a, splits, st);
+  if (mode == 0) {
+    const dim3 g(M, (N + 511) / 512);
+    rows_sum_kernel<<<g, 256, 0, st>>>(a.out, a.parts, norm ? a.ss : nullptr, M, N,
+                                       splits, 1.f / (float)K, eps);
+  } else if (mode == 1 || mode == 4) {
+    if (mode == 4 && !ss_out) return 9008;
+    rows_residual_kernel<<<dim3(M, 8), 256, 0, st>>>(
+        a.residual, a.out, a.parts, (float*)ss_out, M, N, splits);
+  } else {
+    return 9008;
+  }
+  return af_last_err();
+}
+
+// Fused QKV projection of normed rows + rotary positions + page append: q
+// [M, Hq*128] to `q`, k and v to their pages only.  Up to 16 rows compute the
+// RMSNorm scalar themselves; more take it from ss.
+AF_EXPORT int af_rows_qkv(void* q, void* parts, const void* X, const void* W,
+                          const void* ss, int M, int Hq, int Hk, int K,
+                          int splits, float eps, const void* pos,
+                          const void* table, void* kc, void* vc,
+                          const void* slot, int page_size, void* stream) {
+  RowsArgs a = {};
+  a.out = (u16*)q;
+  a.parts = (float*)parts;
+  a.X = (const u16*)X;
+  a.W = (const u16*)W;
+  a.M = M; a.N = (Hq + 2 * Hk) * 128; a.K = K;
+  a.ss = (const float*)ss;
+  a.eps = eps;
+  a.pos = (const i32*)pos;
+  a.table = (const float*)table;
+  a.kc = (u16*)kc;
+  a.vc = (u16*)vc;
+  a.slot = (const i64*)slot;
+  a.Hq = Hq; a.Hk = Hk; a.page_size = page_size;
+  if (const int rc = check_rows(a, splits)) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  if (M <= ROWS_MAX) {
+    launch_rows<EPI_ROPE, 2>(a, st);
+    return af_last_err();
+  }
+  if (!parts || !ss) return 9008;
+  launch_tile<EPI_PARTS, 0>(a, splits, st);
+  rows_rope_kernel<<<dim3(M, (Hq + 2 * Hk + 3) / 4), 256, 0, st>>>(a, splits);
+  return af_last_err();
+}

@@ -178,8 +178,7 @@ class LlamaAttention(nn.Module):
         self.o = nn.Parameter(torch.empty(H, cfg.q_size))
         self.scale = 1.0 / math.sqrt(D)
 
-    def attend(self, qkv, positions, rope_tab, kv: KVCache, md: AttnMetadata,
-               scale: tuple | None = None):
+    def attend(self, qkv, positions, rope_tab, kv: KVCache, md: AttnMetadata):
         """RoPE + cache append + attention over the fused QKV buffer."""
         cfg = self.cfg
         # strided views straight into the fused projection (no copies)
@@ -187,8 +186,12 @@ class LlamaAttention(nn.Module):
         k = qkv[:, cfg.q_size:cfg.q_size + cfg.kv_size]
         v = qkv[:, cfg.q_size + cfg.kv_size:]
         ops.rope_cache(q, k, v, positions, rope_tab,
-                       kv.k[self.layer_idx], kv.v[self.layer_idx], md.slots,
-                       scale=scale)
+                       kv.k[self.layer_idx], kv.v[self.layer_idx], md.slots)
+        return self.attention(q, kv, md)
+
+    def attention(self, q, kv: KVCache, md: AttnMetadata):
+        """Attention of rotated query rows over the pages."""
+        cfg = self.cfg
         if md.is_prefill:
             return ops.attn_prefill(q, kv.k[self.layer_idx],
                                     kv.v[self.layer_idx], md.block_table,
@@ -301,34 +304,22 @@ class LlamaLayer(nn.Module):
             h = self.mlp(h)
         return h, residual
 
-    def forward_decode_fused(self, residual, ss, ss2, positions, rope_tab,
-                             kv, md):
-        """Decode fast path: RMSNorms fold into the skinny GEMMs — input
-        normalization happens in the GEMM's X staging (from per-row
-        sum-of-squares stats), residual-add + next-norm stats in the GEMM
-        combine.  Zero standalone norm kernels per layer."""
+    def forward_rows_fused(self, residual, ss, positions, rope_tab, kv, md):
+        """Few-row path (decode steps, small prefill steps): norms, rotary
+        positions, page append, SwiGLU and residual adds ride in the
+        weight-streaming GEMMs, nothing runs on its own but attention.
+        `residual` is updated in place; ss [T, 8] holds its rows' sums of
+        squares (None up to ops.ROWS_MAX rows, which need none)."""
         at, mlp = self.attn, self.mlp
-        M = residual.shape[0]
-        K = residual.shape[1]
-        small = M <= 64  # measured crossover vs hipBLASLt (BENCHMARKS.md)
-        if small:
-            qkv = ops.linear_skinny(residual, at.qkv, scale=(ss, self.eps))
-            o = at.attend(qkv, positions, rope_tab, kv, md)
-        else:
-            # blas GEMM on the un-normalized rows; the RMSNorm scalar rides
-            # along in rope_cache (RoPE is linear, so this is exact)
-            qkv = residual @ at.qkv.t()
-            o = at.attend(qkv, positions, rope_tab, kv, md,
-                          scale=(ss, K, self.eps))
-        ops.linear_skinny(o, at.o, mode=4, residual=residual, ss_out=ss2)
-        if small:
-            act = ops.linear_skinny(residual, mlp.gate_up, mode=2,
-                                    scale=(ss2, self.eps))
-        else:
-            act = ops.silu_and_mul(residual @ mlp.gate_up.t(),
-                                   scale=(ss2, K, self.eps))
-        ops.linear_skinny(act, mlp.down, mode=4, residual=residual, ss_out=ss)
-        return residual, ss
+        q = ops.qkv_rope_rows(residual, at.qkv, self.eps, ss, positions,
+                              rope_tab, kv.k[at.layer_idx],
+                              kv.v[at.layer_idx], md.slots)
+        o = at.attention(q, kv, md)
+        mode = 1 if ss is None else 4
+        ops.linear_rows(o, at.o, mode, residual, ss_out=ss, want_out=False)
+        act = ops.linear_rows(residual, mlp.gate_up, 2, scale=(ss, self.eps))
+        ops.linear_rows(act, mlp.down, mode, residual, ss_out=ss,
+                        want_out=False)
 
 
 class LlamaForCausalLM(nn.Module):
@@ -367,8 +358,8 @@ class LlamaForCausalLM(nn.Module):
         """Fold each RMSNorm's elementwise weight into the projection that
         consumes it (qkv <- input_norm, gate_up <- post_norm, lm_head <-
         final_norm), leaving unit norm weights.  Mathematically identical;
-        lets the fused decode path apply the norm as a per-row output
-        scalar in the GEMM combine, keeping the async weight stream."""
+        lets the few-row path apply the norm as a per-row output scalar
+        of the GEMM, keeping the async weight stream."""
         if getattr(self, "_norms_folded", False):
             return self
         for layer in self.layers:
@@ -391,7 +382,7 @@ class LlamaForCausalLM(nn.Module):
         self._norms_folded = True
         return self
 
-    def _can_fuse_decode(self, T: int) -> bool:
+    def _can_fuse_rows(self, T: int) -> bool:
         import os
         if os.environ.get("AF_NO_FUSED_DECODE") == "1":
             return False
@@ -400,6 +391,7 @@ class LlamaForCausalLM(nn.Module):
         cfg = self.cfg
         return (not getattr(self, "no_fused_decode", False) and T <= 128
                 and cfg.num_experts == 1  # MoE routes through the eager path
+                and cfg.head_dim == 128
                 and cfg.hidden_size % 64 == 0
                 and cfg.intermediate_size % 64 == 0
                 and (cfg.q_size + 2 * cfg.kv_size) % 64 == 0
@@ -409,13 +401,15 @@ class LlamaForCausalLM(nn.Module):
                 logit_rows: torch.Tensor | None = None):
         """ids/positions [T] -> logits [T or len(logit_rows), vocab]."""
         T = ids.numel()
-        if not md.is_prefill and ids.is_cuda and self._can_fuse_decode(T):
-            ss = torch.empty(T, 8, dtype=torch.float32, device=ids.device)
-            ss2 = torch.empty_like(ss)
+        if ids.is_cuda and self._can_fuse_rows(T):
+            ss = (torch.empty(T, 8, dtype=torch.float32, device=ids.device)
+                  if T > ops.ROWS_MAX else None)
             residual = ops.embedding(ids, self.embed, ss=ss)
             for layer in self.layers:
-                residual, ss = layer.forward_decode_fused(
-                    residual, ss, ss2, positions, self.rope_tab, kv, md)
+                layer.forward_rows_fused(residual, ss, positions,
+                                         self.rope_tab, kv, md)
+            if logit_rows is not None:
+                residual = ops.gather_rows(residual, logit_rows)
             h = ops.rmsnorm(residual, self.final_norm, self.cfg.rms_eps)
             return self._project_logits(h)
         h = ops.embedding(ids, self.embed)

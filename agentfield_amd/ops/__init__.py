@@ -8,6 +8,7 @@ Every op has two paths:
 """
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -188,14 +189,29 @@ def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
     return out
 
 
-def prefill_tiles(seq_lens: list[int], rows_per_wg: int):
-    """Host-side tile map for varlen prefill: (tile_seq[], tile_q0[])."""
-    ts, tq = [], []
-    for s, ln in enumerate(seq_lens):
-        for q0 in range(0, ln, rows_per_wg):
-            ts.append(s)
-            tq.append(q0)
-    return ts, tq
+def prefill_split(seq_lens: list[int], G: int, Hk: int, max_keys: int):
+    """How a packed prefill step's attention is cut: (few_cols, 128-column
+    items, 32-column items, key splits of the latter).  A sequence has G columns
+    per row; up to few_cols of them go to the kernel with 32 columns per block.
+
+    Sequences of one wave's columns always do.  A batch that would give the
+    128-column kernel fewer than 128 blocks goes there whole (four prompts of
+    60 rows behind 3000 tokens, 8 K/V heads: 59 us against 108).  Steps of a few
+    rows per sequence, i.e. behind a history, also split the keys until there
+    are 256 blocks, at least 256 of the largest possible history each (16 x 5
+    rows behind 2400 tokens: 51 us against 58); prompts only up to 64 blocks,
+    most have no history and a merge costs a launch."""
+    cols = [ln * G for ln in seq_lens if ln > 0]
+    few_cols = 32
+    if sum(-(-c // 128) for c in cols if c > 32) * Hk < 128:
+        few_cols = 1 << 30
+    items = sum(-(-c // 128) for c in cols if c > few_cols)
+    few = sum(-(-c // 32) for c in cols if c <= few_cols)
+    nsplit = 1
+    if few:
+        blocks = 256 if max(seq_lens) <= 16 else 64
+        nsplit = max(1, min(8, blocks // (few * Hk), max_keys // 256))
+    return few_cols, items, few, nsplit
 
 
 def attn_prefill(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
@@ -218,18 +234,21 @@ def attn_prefill(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
                                       block_table, q_start, cu_seqlens,
                                       scale, window=window).flatten(1)
     G = Hq // Hk
-    rows_per_wg = 16 * max(1, 4 // G)
-    ts, tq = prefill_tiles(seq_lens, rows_per_wg)
-    dev = q.device
-    tile_seq = torch.tensor(ts, dtype=torch.int32, device=dev)
-    tile_q0 = torch.tensor(tq, dtype=torch.int32, device=dev)
+    few_cols, items, few, nsplit = prefill_split(
+        seq_lens, G, Hk, block_table.shape[1] * page)
     out = torch.empty(T, Hq * D, dtype=q.dtype, device=q.device)
+    po = pml = None
+    if nsplit > 1:
+        po = torch.empty(few, Hk, nsplit, 32, D, dtype=torch.float32,
+                         device=q.device)
+        pml = torch.empty(few, Hk, nsplit, 32, 2, dtype=torch.float32,
+                          device=q.device)
     rc = _lib.lib().af_attn_prefill(
-        _lib.ptr(out), _lib.ptr(q), _lib.ptr(kcache), _lib.ptr(vcache),
-        _lib.ptr(block_table), _lib.ptr(q_start),
-        _lib.ptr(cu_seqlens), _lib.ptr(tile_seq), _lib.ptr(tile_q0),
-        scale, len(ts), Hq, Hk, D, q.stride(0), page, block_table.shape[1],
-        window, _lib.cur_stream())
+        _lib.ptr(out), _lib.ptr(po), _lib.ptr(pml), _lib.ptr(q),
+        _lib.ptr(kcache), _lib.ptr(vcache), _lib.ptr(block_table),
+        _lib.ptr(q_start), _lib.ptr(cu_seqlens), scale, len(seq_lens), items,
+        few, few_cols, nsplit, Hq, Hk, D, q.stride(0), page,
+        block_table.shape[1], window, _lib.cur_stream())
     _lib.check(rc, "af_attn_prefill")
     return out
 
@@ -243,12 +262,100 @@ def choose_sk(N: int, K: int) -> int:
     return sk
 
 
+@functools.lru_cache(maxsize=None)
+def rows_splits(M: int, N: int, K: int) -> int:
+    """K splits of the row GEMM's 64- or 128-column blocks (M > 16): one block
+    per CU if that comes out nearly full, else two (64-column blocks only, their
+    buffers leave room for that), at least four 64-element pieces each.  Measured
+    at 64 rows: 4096 x 4096 9.0 us in 4 (10.1 in 8, 13.2 in 2), 6144 x 4096
+    13.5 us in 5 (16.9 in 3), 4096 x 14336 24.8 us in 4 (26.7 in 8)."""
+    pieces = K // 64
+    wide = M > 64 and N % 128 == 0
+    blocks = N // 128 if wide else N // 64
+    n = max(1, 256 // blocks)
+    if not wide and n * blocks < 224:
+        n = max(1, 512 // blocks)
+    n = max(1, min(n, 16, pieces // 4))
+    per = -(-pieces // n)
+    return -(-pieces // per)          # no empty split
+
+
+def _rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """What the row GEMMs take: bf16 rows and weights that lie whole and on
+    16-byte boundaries, whole 64 x 64 tiles of weights, 1..128 rows."""
+    return (x.is_cuda and 0 < x.shape[0] <= 128 and w.shape[0] % 64 == 0
+            and w.shape[1] % 64 == 0 and x.is_contiguous()
+            and w.is_contiguous() and x.dtype == w.dtype == torch.bfloat16
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def linear_rows(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
+                residual: torch.Tensor | None = None,
+                scale: tuple | None = None,
+                ss_out: torch.Tensor | None = None,
+                want_out: bool = True) -> torch.Tensor | None:
+    """Weight-streaming GEMM for up to 128 rows with the step behind it; modes
+    and scale=(ss, eps) as in linear_skinny.  scale=(None, eps): the RMSNorm
+    scalar is computed from x itself (up to 16 rows).  want_out=False (modes 1
+    and 4): only the residual is written.  x and residual must not overlap."""
+    M, K = x.shape
+    N = w.shape[0]
+    out = None
+    if want_out:
+        out = torch.empty(M, N // 2 if mode == 2 else N, dtype=x.dtype,
+                          device=x.device)
+    splits, parts = 1, None
+    if mode != 2 and (M > ROWS_MAX or mode == 4):
+        splits = rows_splits(M, N, K)
+        parts = torch.empty(splits, M, N, dtype=torch.float32, device=x.device)
+    norm, ss, eps = 0, None, 0.0
+    if scale is not None:
+        ss, eps = scale
+        norm = 2 if ss is None else 1
+    rc = _lib.lib().af_rows_linear(
+        _lib.ptr(out), _lib.ptr(residual), _lib.ptr(parts), _lib.ptr(ss_out),
+        _lib.ptr(x), _lib.ptr(w), M, N, K, splits, mode, norm, _lib.ptr(ss), eps,
+        _lib.cur_stream())
+    _lib.check(rc, "af_rows_linear")
+    return out
+
+
+# rows up to which the row GEMM needs no partial sums and no row statistics
+ROWS_MAX = 16
+
+
+def qkv_rope_rows(x: torch.Tensor, w: torch.Tensor, eps: float,
+                  ss: torch.Tensor | None, positions: torch.Tensor,
+                  table: torch.Tensor, kcache: torch.Tensor,
+                  vcache: torch.Tensor, slots: torch.Tensor) -> torch.Tensor:
+    """q [M, Hq*128] of up to 128 un-normalised rows: QKV projection (norm weight
+    folded into w), RMSNorm scalar (from ss [M, 8] above 16 rows), rotary
+    positions, and k / v appended to their pages."""
+    M, K = x.shape
+    _, Hk, page, D = kcache.shape
+    N = w.shape[0]
+    Hq = N // D - 2 * Hk
+    q = torch.empty(M, Hq * D, dtype=x.dtype, device=x.device)
+    splits, parts = 1, None
+    if M > ROWS_MAX:
+        splits = rows_splits(M, N, K)
+        parts = torch.empty(splits, M, N, dtype=torch.float32, device=x.device)
+    rc = _lib.lib().af_rows_qkv(
+        _lib.ptr(q), _lib.ptr(parts), _lib.ptr(x), _lib.ptr(w), _lib.ptr(ss), M,
+        Hq, Hk, K, splits, eps, _lib.ptr(positions.int()), _lib.ptr(table),
+        _lib.ptr(kcache), _lib.ptr(vcache), _lib.ptr(slots), page,
+        _lib.cur_stream())
+    _lib.check(rc, "af_rows_qkv")
+    return q
+
+
 def linear_skinny(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
                   residual: torch.Tensor | None = None,
                   sk: int | None = None,
                   scale: tuple | None = None,
                   ss_out: torch.Tensor | None = None) -> torch.Tensor:
-    """Decode-path GEMM (M<=256) via the MFMA weight-streaming kernel.
+    """Decode-path GEMM (M<=256) via the MFMA weight-streaming kernels: up to 128
+    rows linear_rows, more (or an explicit sk) the split-K kernel below.
 
     mode 0: plain; mode 1: +residual (in-place update); mode 2: fused SwiGLU
     (w holds [gate|up] rows, returns [M, N/2]); mode 4: +residual AND
@@ -260,6 +367,10 @@ def linear_skinny(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
     """
     M, K = x.shape
     N = w.shape[0]
+    if sk is None and _rows_ok(x, w) and (mode in (0, 2) or (
+            scale is None and x.untyped_storage().data_ptr()
+            != residual.untyped_storage().data_ptr())):
+        return linear_rows(x, w, mode, residual, scale, ss_out)
     if sk is None:
         sk = choose_sk(N, K)
     cols = N // 2 if mode == 2 else N
@@ -280,20 +391,16 @@ def linear_skinny(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False) -> torch.Tensor:
-    """Linear layer dispatch: hand-written skinny MFMA kernel for decode
-    shapes (M<=64), hipBLASLt (torch.matmul) for prefill GEMMs."""
-    M, K = x.shape
-    N = w.shape[0]
-    # policy from measured MI355X data (profiles/kernel_bench_r01_final.log
-    # + M=128 sweep): the hand-written path wins where work/CU is scarce —
-    # small-M x small-N (qkv/o at M<=64), fused-SwiGLU gate_up at M<=64, and
-    # the K=14336 down-projection at 32<M<=128; hipBLASLt wins larger M and
-    # the 128k-vocab lm_head.
-    ok_shape = (x.is_cuda and N % 64 == 0 and K % 64 == 0
-                and x.is_contiguous() and M <= 128)
-    if ok_shape and ((M <= 64 and (silu_fuse or (N <= 8192 and K <= 8192)))
-                     or (32 < M and K >= 8192 and N <= 8192)):
-        return linear_skinny(x, w, mode=2 if silu_fuse else 0)
+    """Linear layer dispatch: hand-written weight-streaming kernels up to 128
+    rows, hipBLASLt (torch.matmul) for prefill GEMMs and vocabulary-sized N.
+
+    Measured at 128 rows, where the kernels gain least: 6144 x 4096 21 us with
+    the sum of its splits against the library's 26, 4096 x 14336 33 against 45,
+    SwiGLU over 28672 x 4096 62 us against 58 + 5; one row of 128256 x 4096 is at
+    the memory rate in both."""
+    if _rows_ok(x, w) and (silu_fuse or w.shape[0] <= 16384) and not (
+            torch.is_grad_enabled() and x.requires_grad):
+        return linear_rows(x, w, mode=2 if silu_fuse else 0)
     y = x @ w.t()
     if silu_fuse:
         return silu_and_mul(y)

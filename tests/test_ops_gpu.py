@@ -527,3 +527,119 @@ def test_attn_decode_tile_edges(page, G, Hk, nsplit, window):
                            window=window).flatten(1)
     assert torch.isfinite(got.float()).all()
     assert close(got, want, atol=2 ** -7, rtol=2 ** -8)
+
+
+def _rope_rows_reference(x, w, eps, pos, tab, Hq, Hk):
+    """fp32 QKV + norm scalar + rotate-half; q [M, Hq, D], k / v [M, Hk, D]."""
+    xf, D = x.float(), 128
+    rstd = torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + eps)
+    y = (xf @ w.float().t() * rstd).unflatten(-1, (-1, D))
+    c = tab[pos.long()].float()[:, None]
+    cos, sin = c[..., :D // 2], c[..., D // 2:]
+    a, b = y[..., :D // 2], y[..., D // 2:]
+    r = torch.cat([a * cos - b * sin, b * cos + a * sin], -1)
+    return r[:, :Hq], r[:, Hq:Hq + Hk], y[:, Hq + Hk:]
+
+
+ROW_COUNTS = [1, 3, 16, 17, 32, 33, 64, 65, 100, 128]
+
+
+@pytest.mark.parametrize("M", ROW_COUNTS)
+@pytest.mark.parametrize("N,K", [(64, 64), (192, 448), (4096, 512),
+                                 (320, 1088), (32768, 256)])
+def test_linear_rows_modes(M, N, K):
+    """Every epilogue of the row GEMMs at the edges of their row classes, with
+    fewer K pieces than waves, odd piece counts, odd tile counts and both widths
+    of block.  Tolerance: bf16 rounding of the result (2^-8 relative) and fp32
+    sums over K of products of ~0.1 size."""
+    x = rnd(M, K, seed=M + K, scale=0.3)
+    w = rnd(N, K, seed=N, scale=0.3)
+    y = x.float() @ w.float().t()
+    tol = dict(atol=2e-3 * math.sqrt(K) * 0.09, rtol=2 ** -7)
+    assert close(ops.linear_rows(x, w), y, **tol)
+    ss = torch.zeros(M, 8, device=DEV)
+    ss[:, 3] = x.float().pow(2).sum(-1)
+    rstd = torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + 1e-5)
+    g, u = (y * rstd).chunk(2, -1)
+    want = torch.nn.functional.silu(g) * u
+    loose = dict(atol=2e-3 * K ** 0.5, rtol=2 ** -6)
+    assert close(ops.linear_rows(x, w, 2, scale=(ss, 1e-5)), want, **loose)
+    if M <= ops.ROWS_MAX:
+        assert close(ops.linear_rows(x, w, 2, scale=(None, 1e-5)), want, **loose)
+    for mode in (1, 4):
+        res = rnd(M, N, seed=9)
+        want = y + res.float()
+        st = torch.full((M, 8), torch.nan, device=DEV) if mode == 4 else None
+        out = ops.linear_rows(x, w, mode, res, ss_out=st)
+        assert torch.equal(out, res)
+        assert close(res, want, **tol)
+        if mode == 4:
+            assert torch.allclose(st.sum(-1), res.float().pow(2).sum(-1),
+                                  rtol=1e-4)
+
+
+@pytest.mark.parametrize("M", ROW_COUNTS)
+@pytest.mark.parametrize("Hq,Hk,K", [(2, 1, 256), (8, 8, 192), (32, 8, 1024)])
+def test_qkv_rope_rows(M, Hq, Hk, K):
+    """Fused QKV + norm scalar + rotary + page append against fp32; rows without
+    a slot leave the pages alone.  Tolerance: one bf16 rounding of values of a
+    few units."""
+    D, page = 128, 16
+    x = rnd(M, K, seed=M + Hq, scale=0.7)
+    w = rnd((Hq + 2 * Hk) * D, K, seed=Hk, scale=1.0 / math.sqrt(K))
+    tab = ops.rope_table(512, D, device=DEV)
+    pos = torch.randint(0, 512, (M,), dtype=torch.int32, device=DEV)
+    kc = torch.zeros(M // page + 2, Hk, page, D, dtype=torch.bfloat16, device=DEV)
+    vc = torch.zeros_like(kc)
+    slots = torch.randperm(kc.shape[0] * page, device=DEV)[:M].to(torch.int64)
+    if M > 2:
+        slots[1] = -1
+    ss = torch.zeros(M, 8, device=DEV)
+    ss[:, 0] = x.float().pow(2).sum(-1)
+    q = ops.qkv_rope_rows(x, w, 1e-5, ss if M > ops.ROWS_MAX else None, pos, tab,
+                          kc, vc, slots)
+    wq, wk, wv = _rope_rows_reference(x, w, 1e-5, pos, tab, Hq, Hk)
+    tol = dict(atol=2e-2, rtol=2 ** -7)
+    assert close(q.unflatten(-1, (Hq, D)), wq, **tol)
+    kw, vw = torch.zeros_like(kc).float(), torch.zeros_like(vc).float()
+    ok = slots >= 0
+    kw[slots[ok] // page, :, slots[ok] % page] = wk[ok]
+    vw[slots[ok] // page, :, slots[ok] % page] = wv[ok]
+    assert close(kc, kw, **tol) and close(vc, vw, **tol)
+
+
+@pytest.mark.parametrize("page,G,Hk", [(4, 4, 2), (16, 1, 3), (24, 2, 2),
+                                       (32, 8, 1), (64, 4, 2), (64, 1, 2)])
+@pytest.mark.parametrize("window", [0, 50])
+def test_attn_prefill_tile_edges(page, G, Hk, window):
+    """Chunk lengths around one wave's 32 columns and a block's 128, histories
+    around 32- and 64-token tiles, both kernels in one call, an empty chunk;
+    values of positions that do not exist yet are NaN, so that reading them
+    with weight 0 would show.  Tolerance: P and the output are rounded to bf16
+    (2^-9 of values below 4, twice)."""
+    D = 128
+    lens = [1, 32 // G, 32 // G + 1, 0, 5, 64, 65, 130, 3, 200, 1]
+    hist = [0, 31, 0, 7, 64, 0, 63, 65, 300, 100, 129]
+    B = len(lens)
+    torch.manual_seed(11)
+    maxp = -(-max(n + h for n, h in zip(lens, hist)) // page)
+    bt = (torch.randperm(B * maxp) + 1).view(B, maxp).to(torch.int32)
+    kc = torch.randn(B * maxp + 1, Hk, page, D).bfloat16()
+    vc = torch.randn(B * maxp + 1, Hk, page, D).bfloat16()
+    there = torch.zeros(B * maxp + 1, page, dtype=torch.bool)
+    for b in range(B):
+        for t in range(lens[b] + hist[b]):
+            there[bt[b, t // page], t % page] = True
+    vc = torch.where(there[:, None, :, None], vc, torch.nan)
+    q = torch.randn(sum(lens), Hk * G * D).bfloat16()
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    qs = torch.tensor(hist, dtype=torch.int32)
+    scale = 1.0 / math.sqrt(D)
+    got = ops.attn_prefill(q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV),
+                           qs.to(DEV), cu.to(DEV), lens, scale,
+                           window=window).cpu()
+    want = ref.attn_prefill_paged(q.unflatten(-1, (Hk * G, D)), kc,
+                                  torch.nan_to_num(vc), bt, qs, cu, scale,
+                                  window=window).flatten(1)
+    assert torch.isfinite(got.float()).all()
+    assert close(got, want, atol=2 ** -6, rtol=2 ** -7)
