@@ -398,7 +398,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False) -> torch.T
     the sum of its splits against the library's 26, 4096 x 14336 33 against 45,
     SwiGLU over 28672 x 4096 62 us against 58 + 5; one row of 128256 x 4096 is at
     the memory rate in both."""
-    if _rows_ok(x, w) and (silu_fuse or w.shape[0] <= 16384) and not (
+    if _rows_ok(x, w) and (silu_fuse or w.shape[0] <= 12288) and not (
             torch.is_grad_enabled() and x.requires_grad):
         return linear_rows(x, w, mode=2 if silu_fuse else 0)
     y = x @ w.t()

@@ -666,29 +666,35 @@ def softcap(logits: torch.Tensor, cap: float) -> torch.Tensor:
 
 def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
            out: torch.Tensor | None = None) -> torch.Tensor:
-    """x [M, K] @ w [N, K]^T through the vendor GEMM (hipBLASLt / rocBLAS);
-    fp32 operands run in true fp32 (no reduced-precision matrix mode).  out:
-    rows to write to (always the vendor GEMM).
+    """x [M, K] @ w [N, K]^T; fp32 operands run in true fp32 (no reduced-
+    precision matrix mode).  out: rows to write to (always the vendor GEMM).
 
-    AF_MIX_SKINNY=1 sends decode-sized bf16 products (<= 64 rows, N and K
-    multiples of 64) to the framework's MFMA skinny-GEMM kernel instead, with
-    the per-shape policy ops.linear uses for the Llama family.  Measured on
-    MI355X for this family the two are equal in GEMM time (1.33 vs 1.34 ms
-    per 64-row step at width 2048, and the same tokens/s at width 4096) while
-    the skinny path adds a combine launch per product, so the vendor GEMM is
-    the default."""
+    bf16 products of few rows (decode steps) run on the framework's
+    weight-streaming kernels, wider ones and prompts on the vendor GEMM
+    (hipBLASLt / rocBLAS).  Up to 16 rows that is one launch, above a second one
+    adds the K splits up, which wide weights do not earn back.  Measured, vendor
+    against rows in us: 2048 x 2048 11.1 / 4.6 at 4 rows, 11.7 / 8.8 at 64;
+    10240 x 2048 16.3 / 11.5 at 16 rows, 14.5 / 13.4 at 32, 15.9 / 15.7 at 64;
+    6144 x 2048 12.5 / 11.5 at 32, 13.1 / 13.7 at 64; 2048 x 8192 22.5 / 12.4 at
+    64; 14336 x 4096 29.6 / 25.9 at 16, 24.8 / 27.8 at 24.  AF_MIX_SKINNY=1 sends
+    the remaining decode-sized products (up to 64 rows, or 33..128 against a long
+    inner dimension) to the framework's kernels too."""
     if out is not None:
         return torch.mm(x, w.t(), out=out)
     M, K = x.shape
     N = w.shape[0]
-    if (skinny and _SKINNY and x.is_cuda and x.dtype == torch.bfloat16
-            and N % 64 == 0 and K % 64 == 0
-            and ((M <= 64 and K <= 8192)
-                 or (32 < M <= 128 and K >= 8192 and N <= 8192))
-            and x.is_contiguous() and w.is_contiguous()
-            and _lib.main_lib_ready()):
-        from . import linear_skinny
-        return linear_skinny(x, w)
+    if skinny and x.is_cuda and M <= 128 and _lib.main_lib_ready():
+        from . import ROWS_MAX, _rows_ok, linear_rows, linear_skinny
+        if ((M <= ROWS_MAX and N <= 16384 or M <= 32 and N <= 10240
+                or M <= 64 and N <= 4096) and _rows_ok(x, w)
+                and not (torch.is_grad_enabled() and x.requires_grad)):
+            return linear_rows(x, w)
+        if (_SKINNY and x.dtype == torch.bfloat16
+                and N % 64 == 0 and K % 64 == 0
+                and ((M <= 64 and K <= 8192)
+                     or (32 < M <= 128 and K >= 8192 and N <= 8192))
+                and x.is_contiguous() and w.is_contiguous()):
+            return linear_skinny(x, w)
     return x @ w.t()
 
 
