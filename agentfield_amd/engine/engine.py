@@ -9,8 +9,10 @@ loops in hipGraphs).
 """
 from __future__ import annotations
 
+import math
 import time
 
+import numpy as np
 import torch
 
 from .. import ops
@@ -375,40 +377,69 @@ class LLMEngine:
         return self.state_slots.slot_of(seq, live)
 
     def _chunk_batch(self, seqs: list[Sequence], starts: list[int],
-                     token_lists: list[list[int]]):
+                     token_lists: list[list[int]],
+                     rows: list[list[int]] | None = None):
         """Device-side description of one packed step: sequence i runs
         token_lists[i] at absolute positions starts[i].. — prompt portions
         and single decoded tokens alike.  Returns (ids, positions, metadata,
-        row offsets)."""
-        dev = self.device
-        ids, pos, slots, rowseq, bt_rows = [], [], [], [], []
-        for i, (seq, np0, toks) in enumerate(zip(seqs, starts, token_lists)):
-            take = len(toks)
-            ids.extend(toks)
-            pos.extend(range(np0, np0 + take))
-            slots.extend(self._slot(seq, j) for j in range(np0, np0 + take))
-            rowseq.extend([i] * take)
-            row = torch.zeros(self.max_pages_per_seq, dtype=torch.int32)
-            row[:len(seq.pages)] = torch.tensor(seq.pages, dtype=torch.int32)
-            bt_rows.append(row)
+        row offsets, logit rows); rows lists, per sequence, the rows whose
+        logits are wanted (None: no such tensor).
+
+        All of it is laid out in one pinned block and copied without waiting:
+        a tensor built from a list on the device waits for everything queued
+        on the stream, and a step used to build seven to thirteen."""
         chunks = [len(t) for t in token_lists]
         cu_list = [0]
         for ln in chunks:
             cu_list.append(cu_list[-1] + ln)
-        md = AttnMetadata(
-            is_prefill=True,
-            slots=torch.tensor(slots, dtype=torch.int64, device=dev),
-            cu_seqlens=torch.tensor(cu_list, dtype=torch.int32, device=dev),
-            seq_lens=chunks,
-            q_start=torch.tensor(starts, dtype=torch.int32, device=dev),
-            block_table=torch.stack(bt_rows).to(dev))
+        T, B, maxp = cu_list[-1], len(seqs), self.max_pages_per_seq
+        want = None if rows is None else [
+            cu_list[i] + w for i, r in enumerate(rows) for w in r]
+        parts = [("slots", np.int64, (T,)), ("ids", np.int32, (T,)),
+                 ("pos", np.int32, (T,)), ("cu", np.int32, (B + 1,)),
+                 ("start", np.int32, (B,)), ("bt", np.int32, (B, maxp))]
         if self.stateful:
-            md.state_slots = torch.tensor(
-                [self._state_slot(s) for s in seqs], dtype=torch.int32,
-                device=dev)
-            md.row_seq = torch.tensor(rowseq, dtype=torch.int32, device=dev)
-        return (torch.tensor(ids, dtype=torch.int32, device=dev),
-                torch.tensor(pos, dtype=torch.int32, device=dev), md, cu_list)
+            parts += [("sslot", np.int32, (B,)), ("rowseq", np.int32, (T,))]
+        if want is not None:
+            parts.append(("rows", np.int32, (max(1, len(want)),)))
+        sizes = [math.prod(shape) * np.dtype(dt).itemsize
+                 for _, dt, shape in parts]
+        host = torch.empty(sum(sizes), dtype=torch.uint8,
+                           pin_memory=self.is_gpu)
+        raw, h, at = host.numpy(), {}, 0
+        for (name, dt, shape), size in zip(parts, sizes):
+            h[name] = raw[at:at + size].view(dt).reshape(shape)
+            at += size
+        h["bt"].fill(0)
+        for i, (seq, np0, toks) in enumerate(zip(seqs, starts, token_lists)):
+            c = slice(cu_list[i], cu_list[i + 1])
+            pages = np.asarray(seq.pages, dtype=np.int64)
+            pos = np.arange(np0, np0 + len(toks), dtype=np.int64)
+            h["ids"][c] = toks
+            h["pos"][c] = pos
+            h["slots"][c] = (pages[pos // self.page_size] * self.page_size
+                             + pos % self.page_size)
+            h["bt"][i, :len(pages)] = pages
+            if self.stateful:
+                h["rowseq"][c] = i
+        h["cu"][:] = cu_list
+        h["start"][:] = starts
+        if self.stateful:
+            h["sslot"][:] = [self._state_slot(s) for s in seqs]
+        if want is not None:
+            h["rows"][:] = want or [0]
+        dev = host.to(self.device, non_blocking=True)
+        d, at = {}, 0
+        for (name, dt, shape), size in zip(parts, sizes):
+            kind = torch.int64 if dt is np.int64 else torch.int32
+            d[name] = dev[at:at + size].view(kind).view(shape)
+            at += size
+        md = AttnMetadata(
+            is_prefill=True, slots=d["slots"], cu_seqlens=d["cu"],
+            seq_lens=chunks, q_start=d["start"], block_table=d["bt"])
+        if self.stateful:
+            md.state_slots, md.row_seq = d["sslot"], d["rowseq"]
+        return d["ids"], d["pos"], md, cu_list, d.get("rows")
 
     # -- caller-paced requests: tokens are given, logits are returned -------
     def open_request(self) -> Sequence:
@@ -441,21 +472,19 @@ class LLMEngine:
             if seq.num_tokens + len(toks) > self.cfg.max_position:
                 raise ValueError("request exceeds model max_position")
             self.sched.reserve(seq, len(toks))
-        ids_t, pos_t, md, cu_list = self._chunk_batch(
-            seqs, [s.num_tokens for s in seqs], [e[1] for e in entries])
+        ids_t, pos_t, md, cu_list, rows_t = self._chunk_batch(
+            seqs, [s.num_tokens for s in seqs], [e[1] for e in entries],
+            [e[2] for e in entries])
         if self.stateful and all(len(e[1]) == 1 for e in entries):
             # one token per request: the batch a decode step runs
             md.is_prefill, md.seq_lens = False, None
-        rows = [cu_list[i] + w for i, e in enumerate(entries) for w in e[2]]
         self.metrics["steps"] += 1
         self.metrics["prefill_tokens"] += cu_list[-1]
         for seq, toks, _w in entries:
             seq.prompt_ids.extend(toks)
             seq.num_prefilled = seq.num_tokens
-        rows_t = torch.tensor(rows or [0], dtype=torch.int32,
-                              device=self.device)
         logits = self.model(ids_t, pos_t, self.kv, md, logit_rows=rows_t)
-        return logits.float() if rows else None
+        return logits.float() if any(e[2] for e in entries) else None
 
     def close_request(self, seq: Sequence) -> None:
         """Give back the pages and the state slot of an open request."""
@@ -487,24 +516,24 @@ class LLMEngine:
             chunks.append(take)
             known.append(all_ids)
             budget -= take
-        ids_t, pos_t, md, cu_list = self._chunk_batch(
+        # rows to sample: the last one of every prompt that ends here
+        ids_t, pos_t, md, cu_list, last_rows = self._chunk_batch(
             seqs, [s.num_prefilled for s in seqs],
             [a[s.num_prefilled:s.num_prefilled + t]
+             for s, t, a in zip(seqs, chunks, known)],
+            [[t - 1] if s.num_prefilled + t >= len(a) else []
              for s, t, a in zip(seqs, chunks, known)])
         self.metrics["prefill_tokens"] += cu_list[-1]
-        done, done_rows = [], []
-        for i, (seq, take, all_ids) in enumerate(zip(seqs, chunks, known)):
+        done = []
+        for seq, take, all_ids in zip(seqs, chunks, known):
             seq.num_prefilled += take
             if seq.num_prefilled >= len(all_ids):
                 done.append(seq)
-                done_rows.append(cu_list[i + 1] - 1)
         for seq in done:
             self._prefilling.remove(seq)
         if not done:
-            self.model(ids_t, pos_t, self.kv, md,
-                       logit_rows=torch.zeros(1, dtype=torch.int32, device=dev))
+            self.model(ids_t, pos_t, self.kv, md, logit_rows=last_rows)
             return [], []
-        last_rows = torch.tensor(done_rows, dtype=torch.int32, device=dev)
         logits = self._sampler_logits(
             self.model(ids_t, pos_t, self.kv, md, logit_rows=last_rows))
         if any(s.sampling.json_mode for s in done):
