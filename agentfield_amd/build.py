@@ -36,6 +36,7 @@ HIP_SOURCES = [
     "allreduce.hip",
     "gemm_skinny.hip",
     "gemm_rows.hip",
+    "moe.hip",
     "sampling.hip",
     "probe.hip",
 ]

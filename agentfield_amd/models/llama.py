@@ -232,6 +232,8 @@ class MoEMLP(nn.Module):
 
     * prefill (exact, eager): each expert runs the fused gate_up/down on
       its routed token subset — FLOP-proportional, shapes data-dependent.
+      On the GPU the rows are routed and sorted by expert in two kernels, so
+      that a subset is one block of rows (ops.moe_route).
     * decode (static, hipGraph-capturable): every expert runs on every
       token with routing weights zeroed for unrouted pairs.  Decode
       GEMMs are weight-streaming-bound and a top-2-of-8 batch >= ~16
@@ -249,6 +251,8 @@ class MoEMLP(nn.Module):
         self.down = nn.Parameter(torch.empty(E, H, inter))
 
     def forward(self, x, static: bool = False):
+        if not static and self._can_sort(x):
+            return self._forward_sorted(x)
         # fp32 routing (bf16 softmax near-ties destabilize expert choice)
         E = self.router.shape[0]
         probs = torch.softmax(x.float() @ self.router.float().t(), dim=-1)
@@ -275,6 +279,29 @@ class MoEMLP(nn.Module):
                             self.down[e])
             out.index_add_(0, sel, ye.float() * topv[sel, slot].unsqueeze(1))
         return out.to(x.dtype)
+
+
+    def _can_sort(self, x) -> bool:
+        """Rows that the routing kernels take (the loop serves the rest, and
+        anything that autograd has to see)."""
+        return (x.is_cuda and x.dtype == self.router.dtype == torch.bfloat16
+                and x.is_contiguous() and x.shape[1] % 8 == 0
+                and x.data_ptr() % 16 == 0 and x.shape[0] > 0
+                and self.router.shape[0] <= ops.MOE_MAX_EXPERTS
+                and self.top_k <= ops.MOE_MAX_TOP
+                and not torch.is_grad_enabled())
+
+    def _forward_sorted(self, x):
+        weights, row, pos, offs = ops.moe_route(x, self.router, self.top_k)
+        xs = ops.gather_rows(x, row)
+        ys = torch.empty_like(xs)
+        bounds = offs.tolist()       # the one wait: block bounds
+        for e, (a, b) in enumerate(zip(bounds, bounds[1:])):
+            if a == b:
+                continue
+            act = ops.linear(xs[a:b], self.gate_up[e], silu_fuse=True)
+            ops.linear(act, self.down[e], out=ys[a:b])
+        return ops.moe_combine(ys, pos, weights)
 
 
 class LlamaLayer(nn.Module):

@@ -292,16 +292,16 @@ def _rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
 def linear_rows(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
                 residual: torch.Tensor | None = None,
                 scale: tuple | None = None,
-                ss_out: torch.Tensor | None = None,
-                want_out: bool = True) -> torch.Tensor | None:
+                ss_out: torch.Tensor | None = None, want_out: bool = True,
+                out: torch.Tensor | None = None) -> torch.Tensor | None:
     """Weight-streaming GEMM for up to 128 rows with the step behind it; modes
     and scale=(ss, eps) as in linear_skinny.  scale=(None, eps): the RMSNorm
     scalar is computed from x itself (up to 16 rows).  want_out=False (modes 1
-    and 4): only the residual is written.  x and residual must not overlap."""
+    and 4): only the residual is written.  x and residual must not overlap.
+    out: contiguous rows to write to."""
     M, K = x.shape
     N = w.shape[0]
-    out = None
-    if want_out:
+    if want_out and out is None:
         out = torch.empty(M, N // 2 if mode == 2 else N, dtype=x.dtype,
                           device=x.device)
     splits, parts = 1, None
@@ -390,9 +390,11 @@ def linear_skinny(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
     return out
 
 
-def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False) -> torch.Tensor:
+def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
+           out: torch.Tensor | None = None) -> torch.Tensor:
     """Linear layer dispatch: hand-written weight-streaming kernels up to 128
     rows, hipBLASLt (torch.matmul) for prefill GEMMs and vocabulary-sized N.
+    out (without silu_fuse): contiguous rows to write to.
 
     Measured at 128 rows, where the kernels gain least: 6144 x 4096 21 us with
     the sum of its splits against the library's 26, 4096 x 14336 33 against 45,
@@ -400,11 +402,50 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False) -> torch.T
     the memory rate in both."""
     if _rows_ok(x, w) and (silu_fuse or w.shape[0] <= 12288) and not (
             torch.is_grad_enabled() and x.requires_grad):
-        return linear_rows(x, w, mode=2 if silu_fuse else 0)
+        return linear_rows(x, w, mode=2 if silu_fuse else 0, out=out)
+    if out is not None:
+        return torch.mm(x, w.t(), out=out)
     y = x @ w.t()
     if silu_fuse:
         return silu_and_mul(y)
     return y
+
+
+# ---------------------------------------------------------------- mixture
+MOE_MAX_EXPERTS, MOE_MAX_TOP = 64, 8     # limits of the routing kernels
+
+
+def moe_route(x: torch.Tensor, router: torch.Tensor, k: int):
+    """Softmax routing of rows x [T, H] over the experts' router [E, H], the k
+    largest renormalised, and the (row, choice) entries sorted by expert:
+    (weights [T, k] f32, row [T*k] i32 of every sorted position, sorted position
+    [T*k] i32 of every entry, first position of every expert [E+1] i32)."""
+    T, H = x.shape
+    E = router.shape[0]
+    dev = x.device
+    n = T * k
+    topv = torch.empty(T, k, dtype=torch.float32, device=dev)
+    idx = torch.empty(3 * n + E + 1, dtype=torch.int32, device=dev)
+    topi, row, pos, offs = idx.split([n, n, n, E + 1])
+    rc = _lib.lib().af_moe_route(
+        _lib.ptr(topi), _lib.ptr(topv), _lib.ptr(offs), _lib.ptr(row),
+        _lib.ptr(pos), _lib.ptr(x), _lib.ptr(router), T, H, E, k,
+        _lib.cur_stream())
+    _lib.check(rc, "af_moe_route")
+    return topv, row, pos, offs
+
+
+def moe_combine(y: torch.Tensor, pos: torch.Tensor,
+                weights: torch.Tensor) -> torch.Tensor:
+    """out[t] = sum_j weights[t, j] * y[pos[t*k + j]] over the sorted expert rows."""
+    T, k = weights.shape
+    H = y.shape[1]
+    out = torch.empty(T, H, dtype=y.dtype, device=y.device)
+    rc = _lib.lib().af_moe_combine(
+        _lib.ptr(out), _lib.ptr(y), _lib.ptr(pos), _lib.ptr(weights), T, H, k,
+        _lib.cur_stream())
+    _lib.check(rc, "af_moe_combine")
+    return out
 
 
 def gemm_bf16(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
