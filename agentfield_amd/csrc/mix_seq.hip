@@ -527,16 +527,37 @@ __global__ void __launch_bounds__(256) diff_combine_kernel(
 
 // ------------------------------------------------------------- linear scan
 // Workgroup = (sequence, head, 32-column tile of dv); 256 threads = 16 row
-// groups x 16 column pairs.  Thread (r, c) keeps RP consecutive rows
-// r*RP .. r*RP+RP-1 of columns c and c+16 of the state in registers (each
-// q / k / decay value read from LDS feeds two columns).  Tokens are
-// walked serially in blocks of TB: the block's q / k / decay rows are staged
-// into LDS at once (rotary + scaling applied on the way in), every thread
-// then advances its rows through the TB tokens without synchronising and
-// leaves one partial output per token in LDS, and the 16 partials of each
-// (token, column) are summed after one more barrier: two barriers per TB
-// tokens, the recurrence itself strictly token by token in fp32 — so results
-// are bit-identical however a sequence is cut into chunks.
+// groups x 16 column pairs.  A thread keeps RP consecutive rows of two columns of
+// the state in registers (each q / k / decay value read from LDS feeds two
+// columns).  Tokens are walked serially in blocks of TB: the block's q / k / decay
+// rows are staged into LDS at once (rotary + scaling applied on the way in), the
+// recurrence itself is strictly token by token in fp32, and both kernels sum the
+// 16 row groups in the same order — so results do not depend on how a sequence
+// is cut into chunks.
+//
+// linear_scan_kernel, few tokens per sequence: bound by moving the state; thread
+// (r, c) = (tid >> 4, tid & 15) has columns c and c + 16, so that a state row
+// moves in 64-byte pieces; partial outputs meet in LDS after the block of tokens.
+// linear_scan_prompt_kernel: bound by a token's latency on one wave per SIMD (48
+// multiply-adds of four clocks at 128 rows); the row groups are the 16 lanes of a
+// DPP row, so the sum over rows needs no LDS and no second barrier.
+// Six sequences of 500..1900 tokens, 8 heads of 128 x 128, decays per channel:
+// 787 -> 385 us; 16 heads, one decay per head, rotary: 770 -> 497 us
+// (the row layout alone: 711 and 698; element loads that were converted at once
+// made every block wait for its successor).
+// v plus the sum over the other lanes of its 16-lane row, in all of them
+__device__ __forceinline__ float row16_sum_all(float v) {
+#define AFM_ROR(N)                                                           \
+  v += __int_as_float(__builtin_amdgcn_update_dpp(                           \
+      0, __float_as_int(v), 0x120 + N, 0xf, 0xf, true));
+  AFM_ROR(8)
+  AFM_ROR(4)
+  AFM_ROR(2)
+  AFM_ROR(1)
+#undef AFM_ROR
+  return v;
+}
+
 template <typename S, int RP>
 __global__ void __launch_bounds__(256) linear_scan_kernel(
     float* __restrict__ out, float* __restrict__ state,
@@ -711,14 +732,253 @@ __global__ void __launch_bounds__(256) linear_scan_kernel(
       const int tt = e >> 5, ci = e & 31;
       if (c0 + ci < dv) {
         const float* pr = part + tt * 512 + ci;
-        float o = 0.f;
+        float o[16];  // summed in the order of row16_sum_all
 #pragma unroll
-        for (int rr = 0; rr < 16; ++rr) o += pr[rr * 32];
-        out[(size_t)(tb + tt) * H * dv + (size_t)h * dv + c0 + ci] = o;
+        for (int rr = 0; rr < 16; ++rr) o[rr] = pr[rr * 32];
+#pragma unroll
+        for (int n = 8; n > 0; n >>= 1)
+#pragma unroll
+          for (int rr = 0; rr < n; ++rr) o[rr] += o[rr + n];
+        out[(size_t)(tb + tt) * H * dv + (size_t)h * dv + c0 + ci] = o[0];
       }
     }
     // the next block's staging writes `stage`/`vs`, last read before the
     // barrier above; its partials are written after the next barrier
+  }
+#pragma unroll
+  for (int ii = 0; ii < RP; ++ii) {
+    const int i = r * RP + ii;
+    if (i < dk && oka) sbase[(size_t)i * dv + ca] = sta[ii];
+    if (i < dk && okb) sbase[(size_t)i * dv + cb] = stb[ii];
+  }
+}
+
+// The same recurrence for prompts.  A thread stages E consecutive rows of one token
+// (one wide load each for q, k, the rotary partners and the decay logits, kept raw
+// until the block before has been worked through) and computes RP rows of two
+// columns; lane j of a 16-lane row keeps token j's sum.  Two LDS buffers, one
+// barrier per block of tokens.
+template <typename S, int RP>
+__global__ void __launch_bounds__(256, 2) linear_scan_prompt_kernel(
+    float* __restrict__ out, float* __restrict__ state,
+    const S* __restrict__ q, const S* __restrict__ k, const S* __restrict__ v,
+    const S* __restrict__ zl, const float* __restrict__ zbias,
+    const float* __restrict__ head_decay, const float* __restrict__ inv_freq,
+    const i32* __restrict__ positions, const i32* __restrict__ cu,
+    const i32* __restrict__ q_start, const i32* __restrict__ sslot,
+    float q_scale, float k_scale, float inv_tau, int H, int dk, int dv,
+    int rot, i64 ldq, i64 ldk, i64 ldv, i64 ldz) {
+  constexpr int DKP = 16 * RP;
+  constexpr bool FAST = sizeof(S) == 2;
+  constexpr int TB = RP >= 16 ? 8 : 16;
+  constexpr int E = TB * DKP / 256;            // staged rows per thread
+  constexpr int BUF = TB * (3 * DKP + 32);     // [TB][3][DKP], [TB][32]
+  extern __shared__ float smem[];
+  const int b = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * 32;
+  const int t0 = cu[b], t1 = cu[b + 1];
+  if (t1 <= t0) return;
+  const int r = threadIdx.x & 15, cc = threadIdx.x >> 4;
+  const int ca = c0 + 2 * cc, cb = ca + 1;
+  const bool oka = ca < dv, okb = cb < dv;
+  float* sbase = state + (((size_t)sslot[b] * H + h) * dk) * dv;
+  float sta[RP], stb[RP];
+  const bool fresh = q_start[b] == 0;
+#pragma unroll
+  for (int ii = 0; ii < RP; ++ii) {
+    const int i = r * RP + ii;
+    sta[ii] = (!fresh && oka && i < dk) ? sbase[(size_t)i * dv + ca] : 0.f;
+    stb[ii] = (!fresh && okb && i < dk) ? sbase[(size_t)i * dv + cb] : 0.f;
+  }
+
+  // what this thread stages: rows i0 .. i0+E-1 of token st of a block, and two
+  // columns of v of token vt
+  struct Raw { S x[E]; };
+  const int st = threadIdx.x * E / DKP, i0 = threadIdx.x * E % DKP;
+  const int vt = threadIdx.x >> 4, vc = c0 + 2 * (threadIdx.x & 15);
+  const bool have = i0 < dk, turn = i0 < rot;
+  const int half = rot >> 1, ic = have ? i0 : 0;
+  const bool lowh = i0 < half;
+  const int pi = !turn ? ic : lowh ? i0 + half : i0 - half;
+  float frq[E], bias[E];
+#pragma unroll
+  for (int j = 0; j < E; ++j) {
+    frq[j] = turn ? inv_freq[(lowh ? i0 : i0 - half) + j] : 0.f;
+    bias[j] = zl ? zbias[(size_t)h * dk + ic + j] : 0.f;
+  }
+  const float hd = head_decay ? head_decay[h] : 1.0f;
+  const S* qh = q + (size_t)h * dk;
+  const S* kh = k + (size_t)h * dk;
+  const S* zh = zl ? zl + (size_t)h * dk : nullptr;
+  const S* vh = v + (size_t)h * dv;
+  Raw rq, rk, rqp, rkp, rz;
+  S rv[2];
+  int rpos = 0;
+  auto wide = [](const S* p) { return *reinterpret_cast<const Raw*>(
+      __builtin_assume_aligned(p, sizeof(Raw) < 16 ? sizeof(Raw) : 16)); };
+  auto fetch = [&](int tb) {                   // addresses clamped into the chunk
+    const size_t t = min(tb + st, t1 - 1);
+    rq = wide(qh + t * ldq + ic);
+    rk = wide(kh + t * ldk + ic);
+    if (rot > 0) {
+      rqp = wide(qh + t * ldq + pi);
+      rkp = wide(kh + t * ldk + pi);
+      rpos = positions[t];
+    }
+    if (zl) rz = wide(zh + t * ldz + ic);
+    if (vt < TB) {
+      const S* vp = vh + (size_t)min(tb + vt, t1 - 1) * ldv;
+      rv[0] = vp[min(vc, dv - 1)];
+      rv[1] = vp[min(vc + 1, dv - 1)];
+    }
+  };
+  // rotate / scale q and k, evaluate the decays; rows and tokens beyond the end
+  // are zeros
+  auto fill = [&](int nt, float* stage) {
+    float qv[E], kv[E], av[E];
+    const bool valid = have && st < nt;
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      qv[j] = ldf<S>(&rq.x[j]);
+      kv[j] = ldf<S>(&rk.x[j]);
+      av[j] = hd;
+    }
+    if (rot > 0) {
+#pragma unroll
+      for (int j = 0; j < E; ++j) {
+        const float ang = (float)rpos * frq[j];  // 0 where nothing is rotated
+        float sn, cs;
+        if (FAST) { sn = __sinf(ang); cs = __cosf(ang); }
+        else sincosf(ang, &sn, &cs);
+        // pair (u, w) -> (u cos - w sin, w cos + u sin)
+        sn = lowh ? -sn : sn;
+        const float x = qv[j] * cs + ldf<S>(&rqp.x[j]) * sn;
+        const float y = kv[j] * cs + ldf<S>(&rkp.x[j]) * sn;
+        qv[j] = turn ? x : qv[j];
+        kv[j] = turn ? y : kv[j];
+      }
+    }
+    if (zl) {
+#pragma unroll
+      for (int j = 0; j < E; ++j) {
+        const float z = ldf<S>(&rz.x[j]) + bias[j];
+        // log(sigmoid(z)) = min(z, 0) - log(1 + exp(-|z|)), without overflow
+        if (FAST)
+          av[j] = __expf((fminf(z, 0.f) - __logf(1.0f + __expf(-fabsf(z)))) *
+                         inv_tau);
+        else
+          av[j] = expf((fminf(z, 0.f) - log1pf(expf(-fabsf(z)))) * inv_tau);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      qv[j] = valid ? qv[j] * q_scale : 0.f;
+      kv[j] = valid ? kv[j] * k_scale : 0.f;
+      av[j] = valid ? av[j] : 0.f;
+    }
+    // four-row pieces of the 16 row groups side by side: a lane row reads 256
+    // contiguous bytes
+    float* row = stage + (size_t)st * 3 * DKP;
+    if constexpr (RP >= 4) {
+      const int g = i0 / RP, w0 = i0 % RP;
+#pragma unroll
+      for (int w = 0; w < E; w += 4) {
+        const int at = (((w0 + w) >> 2) * 16 + g) * 4;
+        *reinterpret_cast<f32x4*>(row + at) = f32x4{qv[w], qv[w + 1], qv[w + 2], qv[w + 3]};
+        *reinterpret_cast<f32x4*>(row + DKP + at) = f32x4{kv[w], kv[w + 1], kv[w + 2], kv[w + 3]};
+        *reinterpret_cast<f32x4*>(row + 2 * DKP + at) = f32x4{av[w], av[w + 1], av[w + 2], av[w + 3]};
+      }
+    } else {
+#pragma unroll
+      for (int w = 0; w < E; ++w) {
+        row[i0 + w] = qv[w];
+        row[DKP + i0 + w] = kv[w];
+        row[2 * DKP + i0 + w] = av[w];
+      }
+    }
+    if (vt < TB) {
+      float* vr = stage + TB * 3 * DKP + vt * 32 + (vc - c0);
+      vr[0] = vt < nt && vc < dv ? ldf<S>(&rv[0]) : 0.f;
+      vr[1] = vt < nt && vc + 1 < dv ? ldf<S>(&rv[1]) : 0.f;
+    }
+  };
+  fetch(t0);
+  fill(min(TB, t1 - t0), smem);
+  fetch(min(t0 + TB, t1 - 1));
+  __syncthreads();
+  int cur = 0;
+  for (int tb = t0; tb < t1; tb += TB) {
+    const int nt = min(TB, t1 - tb);
+    if (tb + TB < t1) {
+      fill(min(TB, t1 - tb - TB), smem + (cur ^ BUF));
+      fetch(min(tb + 2 * TB, t1 - 1));         // in flight during the arithmetic
+    }
+    const float* sb = smem + cur;
+    const float* vb = sb + TB * 3 * DKP;
+    float oa = 0.f, ob = 0.f;
+    struct Token { float q[RP], k[RP], a[RP]; f32x2 v; };
+    auto read = [&](int tt) {
+      const float* sq = sb + (size_t)tt * 3 * DKP;
+      Token t;
+      if constexpr (RP >= 4) {
+#pragma unroll
+        for (int w = 0; w < RP; w += 4) {
+          const int at = ((w >> 2) * 16 + r) * 4;
+          const f32x4 q4 = *reinterpret_cast<const f32x4*>(sq + at);
+          const f32x4 k4 = *reinterpret_cast<const f32x4*>(sq + DKP + at);
+          const f32x4 a4 = *reinterpret_cast<const f32x4*>(sq + 2 * DKP + at);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            t.q[w + j] = q4[j];
+            t.k[w + j] = k4[j];
+            t.a[w + j] = a4[j];
+          }
+        }
+      } else {
+#pragma unroll
+        for (int w = 0; w < RP; ++w) {
+          t.q[w] = sq[r * RP + w];
+          t.k[w] = sq[DKP + r * RP + w];
+          t.a[w] = sq[2 * DKP + r * RP + w];
+        }
+      }
+      t.v = *reinterpret_cast<const f32x2*>(vb + tt * 32 + 2 * cc);
+      return t;
+    };
+    auto step = [&](int tt, const Token& t) {
+      float pa = 0.f, pb = 0.f;
+#pragma unroll
+      for (int ii = 0; ii < RP; ++ii) {
+        sta[ii] = t.a[ii] * sta[ii] + t.k[ii] * t.v[0];
+        stb[ii] = t.a[ii] * stb[ii] + t.k[ii] * t.v[1];
+        pa += sta[ii] * t.q[ii];
+        pb += stb[ii] * t.q[ii];
+      }
+      pa = row16_sum_all(pa);
+      pb = row16_sum_all(pb);
+      oa = r == tt ? pa : oa;
+      ob = r == tt ? pb : ob;
+    };
+    if (nt == TB) {
+      // the next token's LDS reads run under this one's arithmetic: the fence
+      // keeps them there, a wave has its SIMD to itself and would wait for them
+      Token t[2];
+      t[0] = read(0);
+#pragma unroll
+      for (int tt = 0; tt < TB; ++tt) {
+        if (tt + 1 < TB) t[(tt + 1) & 1] = read(tt + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        step(tt, t[tt & 1]);
+      }
+    } else {
+      for (int tt = 0; tt < nt; ++tt) step(tt, read(tt));
+    }
+    if (r < nt) {
+      float* op = out + (size_t)(tb + r) * H * dv + (size_t)h * dv;
+      if (oka) op[ca] = oa;
+      if (okb) op[cb] = ob;
+    }
+    __syncthreads();  // the next buffer is filled, this one read
+    cur ^= BUF;
   }
 #pragma unroll
   for (int ii = 0; ii < RP; ++ii) {
@@ -923,22 +1183,40 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
                        const float* head_decay, const float* inv_freq,
                        const i32* positions, const i32* cu, const i32* q_start,
                        const i32* sslot, float q_scale, float k_scale,
-                       float inv_tau, int B, int H, int dk, int dv, int rot,
-                       i64 ldq, i64 ldk, i64 ldv, i64 ldz, hipStream_t s) {
+                       float inv_tau, int T, int B, int H, int dk, int dv,
+                       int rot, i64 ldq, i64 ldk, i64 ldv, i64 ldz,
+                       hipStream_t s) {
   dim3 grid(B, H, (dv + 31) / 32);
   const int rp = (dk + 15) / 16;
   const int rpp = rp <= 2 ? 2 : rp <= 4 ? 4 : rp <= 8 ? 8 : 16;
-  const size_t sm = (size_t)(rpp >= 16 ? 8 : 16) * (3 * 16 * rpp + 512 + 32) * sizeof(float);
-#define SCAN(RP)                                                             \
-  linear_scan_kernel<S, RP><<<grid, 256, sm, s>>>(                           \
+  // From a block of tokens per sequence on the prompt kernel is the better one
+  // (see there); its loads take E rows at once, so heads, halves of the rotated
+  // part, strides and bases must be multiples of E elements (16 bytes at most).
+  const int E = rpp >= 8 ? 8 : rpp;
+  const size_t al = E * sizeof(S) < 16 ? E * sizeof(S) : 16;
+  const bool prompt =
+      T >= 16 * B && dk % E == 0 && (rot / 2) % E == 0 && ldq % E == 0 &&
+      ldk % E == 0 && (!zl || ldz % E == 0) && (uintptr_t)q % al == 0 &&
+      (uintptr_t)k % al == 0 && (uintptr_t)zl % al == 0;
+  const size_t sm = (size_t)(rpp >= 16 ? 8 : 16) * sizeof(float) *
+                    (prompt ? 2 * (3 * 16 * rpp + 32) : 3 * 16 * rpp + 512 + 32);
+#define SCAN_ARGS                                                            \
       out, state, (const S*)q, (const S*)k, (const S*)v, (const S*)zl, zbias, \
       head_decay, inv_freq, positions, cu, q_start, sslot, q_scale, k_scale, \
-      inv_tau, H, dk, dv, rot, ldq, ldk, ldv, ldz)
+      inv_tau, H, dk, dv, rot, ldq, ldk, ldv, ldz
+#define SCAN(RP)                                                             \
+  do {                                                                       \
+    if (prompt)                                                              \
+      linear_scan_prompt_kernel<S, RP><<<grid, 256, sm, s>>>(SCAN_ARGS);     \
+    else                                                                     \
+      linear_scan_kernel<S, RP><<<grid, 256, sm, s>>>(SCAN_ARGS);            \
+  } while (0)
   if (rp <= 2) SCAN(2);
   else if (rp <= 4) SCAN(4);
   else if (rp <= 8) SCAN(8);
   else SCAN(16);
 #undef SCAN
+#undef SCAN_ARGS
   return af_last_err();
 }
 
@@ -947,8 +1225,8 @@ AF_EXPORT int afm_linear_scan(
     const void* zl, const void* zbias, const void* head_decay,
     const void* inv_freq, const void* positions, const void* cu,
     const void* q_start, const void* sslot, float q_scale, float k_scale,
-    float inv_tau, int B, int H, int dk, int dv, int rot, i64 ldq, i64 ldk,
-    i64 ldv, i64 ldz, int dt, void* stream) {
+    float inv_tau, int T, int B, int H, int dk, int dv, int rot, i64 ldq,
+    i64 ldk, i64 ldv, i64 ldz, int dt, void* stream) {
   if (B == 0) return 0;
   if (dk > 256 || dk < 1 || dv < 1) return 9003;
   if (rot < 0 || rot > dk || (rot & 1) || (rot && !inv_freq)) return 9003;
@@ -959,13 +1237,13 @@ AF_EXPORT int afm_linear_scan(
     return launch_scan<u16>((float*)out, (float*)state, q, k, v, zl,
         (const float*)zbias, (const float*)head_decay, (const float*)inv_freq,
         (const i32*)positions, (const i32*)cu, (const i32*)q_start,
-        (const i32*)sslot, q_scale, k_scale, inv_tau, B, H, dk, dv, rot, ldq,
-        ldk, ldv, ldz, s);
+        (const i32*)sslot, q_scale, k_scale, inv_tau, T, B, H, dk, dv, rot,
+        ldq, ldk, ldv, ldz, s);
   if (dt == 1)
     return launch_scan<float>((float*)out, (float*)state, q, k, v, zl,
         (const float*)zbias, (const float*)head_decay, (const float*)inv_freq,
         (const i32*)positions, (const i32*)cu, (const i32*)q_start,
-        (const i32*)sslot, q_scale, k_scale, inv_tau, B, H, dk, dv, rot, ldq,
-        ldk, ldv, ldz, s);
+        (const i32*)sslot, q_scale, k_scale, inv_tau, T, B, H, dk, dv, rot,
+        ldq, ldk, ldv, ldz, s);
   return 9002;
 }

@@ -566,7 +566,7 @@ def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         _lib.ptr(decay_logits), _lib.ptr(decay_bias), _lib.ptr(head_decay),
         _lib.ptr(inv_freq), _lib.ptr(positions), _lib.ptr(md.cu_seqlens),
         _lib.ptr(md.q_start), _lib.ptr(md.state_slots),
-        float(q_scale), float(k_scale), float(inv_tau), B, H, dk, dv, rot,
+        float(q_scale), float(k_scale), float(inv_tau), T, B, H, dk, dv, rot,
         _rowstride(q), _rowstride(k), _rowstride(v),
         _rowstride(decay_logits) if decay_logits is not None else 0,
         _code(q), _lib.cur_stream())

@@ -663,3 +663,71 @@ def test_registry_loads_checkpoint_and_trace_cli(tmp_path):
     assert rel_err(g0, wa[[0, 9]]) < 2e-4
     assert rel_err(g1, wb[[5]]) < 2e-4
     assert rel_err(g2, wa[[20]]) < 2e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("dk,dv,rot,pad", [
+    (16, 32, 0, 0), (24, 33, 16, 0), (64, 48, 32, 8), (120, 31, 0, 0),
+    (128, 128, 64, 0), (128, 64, 24, 0), (200, 40, 64, 0), (128, 40, 64, 3)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_scan_prompt_and_token_kernels_agree(dtype, dk, dv, rot, pad, gated):
+    """The prompt kernel (whole prompts of lengths around its token blocks) and
+    the token kernel (the same prompts in portions of one and of nine tokens)
+    give the same outputs and states; padded dims, column tiles, halves that are
+    not a multiple of the wide loads, rows that are not aligned for them.  Both
+    sum in the same order, so only multiply-add contraction may differ: a few
+    fp32 roundings of the largest term."""
+    from agentfield_amd.ops import seqmix as sm
+    from types import SimpleNamespace
+    H, lens = 2, [1, 16, 17, 33, 100]
+    B, T = len(lens), sum(lens)
+    g = torch.Generator(device="cuda").manual_seed(dk + dv)
+
+    def rows(n, s=1.0):
+        wide = torch.randn(T, n + pad, generator=g, device="cuda") * s
+        return wide.to(dtype)[:, pad:] if pad else wide.to(dtype)
+    q, k, v = rows(H * dk, dk ** -0.5), rows(H * dk, 0.3), rows(H * dv)
+    kw = dict(q_scale=0.5, k_scale=0.7)
+    if gated:
+        kw.update(decay_logits=rows(H * dk, 2.0), inv_tau=1 / 16,
+                  decay_bias=torch.ones(H * dk, device="cuda"))
+    else:
+        kw.update(head_decay=torch.tensor([0.9, 0.99], device="cuda"))
+    if rot:
+        kw.update(inv_freq=sm.rotary_inv_freq(rot, 1e4, "cuda"))
+
+    def run(portion):
+        state = torch.full((B + 1, H, dk, dv), torch.nan, device="cuda")
+        out = torch.full((T, H * dv), torch.nan, device="cuda")
+        first = [sum(lens[:i]) for i in range(B)]
+        at = [0] * B
+        while any(a < n for a, n in zip(at, lens)):
+            take = [min(portion, n - a) for a, n in zip(at, lens)]
+            idx = torch.tensor([f + a + j for f, a, t in zip(first, at, take)
+                                for j in range(t)], device="cuda")
+            live = [i for i in range(B) if take[i]]
+            md = SimpleNamespace(
+                cu_seqlens=torch.tensor([0] + [take[i] for i in live],
+                                        device="cuda").cumsum(0).int(),
+                q_start=torch.tensor([at[i] for i in live], device="cuda").int(),
+                state_slots=torch.tensor([i + 1 for i in live],
+                                         device="cuda").int())
+            pos = torch.cat([torch.arange(a, a + t) for a, t in
+                             zip(at, take)]).int().cuda()
+            cut = portion >= max(lens)
+
+            def part(x):
+                return x if cut else x[idx]
+            more = {n: (part(x) if n == "decay_logits" else x)
+                    for n, x in kw.items()}
+            out[idx] = sm.linear_scan(part(q), part(k), part(v), state, md, pos,
+                                      H, **more)
+            at = [a + t for a, t in zip(at, take)]
+        return out, state[1:]
+    whole, S = run(1000)
+    assert torch.isfinite(whole).all() and torch.isfinite(S).all()
+    for portion in (1, 9):
+        o, s = run(portion)
+        assert (o - whole).abs().max() <= 4e-6 * whole.abs().max()
+        assert (s - S).abs().max() <= 4e-6 * S.abs().max()
