@@ -25,13 +25,22 @@
 //   STAGES pieces in a ring with one barrier per piece.  K is split over blocks
 //   where N alone does not fill the chip, the fp32 parts meet in the kernel that
 //   does the next step.
-// Measured in TB/s of weights (us), against the split-K kernel with two-stage
-// buffers and its second launch (in brackets): one row, 6144 x 4096 with rotary
-// and append 11.8 us (21.3 in three launches), 4096 x 4096 8.3, 4096 x 14336 22.4
-// (together 30.7; 44.4), SwiGLU over 28672 x 4096 42.9 = 5.5 TB/s (58.2).  16
-// rows: 13.9, 8.9, 24.7, 47.4.  64 rows, without the closing launches: 13.4, 9.0,
-// 24.8, 53.1 (16.7, o + down 44.8, 62.7).  128 rows: 16.4, 13.0, 28.3, 61.6
-// (library 25.6 and 57.5 + 5.2 for the first and the last, o + down 63.1).
+//
+// Weight rows lie K * 2 bytes apart, usually a multiple of every channel
+// interleave, so the rows of one piece come from the same memory channel and
+// blocks that walk K in step ask the same channel for everything.  Blocks of an
+// XCD therefore start at different pieces (the order of a sum depends on the
+// column, not on M); where K is split the splits do that already and starting
+// elsewhere costs a little (4096 x 4096 in four, 32 rows: 8.0 -> 8.8 us).  SwiGLU over 28672 x 4096: 42.9 -> 40.2 us at one row, 53.4 -> 45.2
+// at 64, 62.3 -> 57.3 at 128; two pieces per wave in flight are then enough (four
+// needed half the CU's buffers: 50.5 us).
+// Measured in us, against the split-K kernel with two-stage buffers and its second
+// launch (in brackets).  One row: 6144 x 4096 with rotary and append 11.2 (21.3 in
+// three launches), 4096 x 4096 7.6 and 4096 x 14336 21.2 (together 44.4), SwiGLU
+// over 28672 x 4096 40.2 = 5.8 TB/s (58.2).  16 rows: 13.4, 8.3, 24.5, 46.0.  64
+// rows, without the closing launches: 13.4, 9.0, 24.8, 45.2 (16.7, o + down 44.8,
+// 62.7).  128 rows: 16.4, 13.0, 28.3, 57.3 (library 25.6 and 57.5 + 5.2 for the
+// first and the last, o + down 63.1).
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8r;
@@ -153,9 +162,12 @@ __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
 #pragma unroll
   for (int g = 0; g < MT * 2; ++g)
     xp[g] = a.X + (size_t)min(g * 8 + r8, a.M - 1) * a.K + ch;
+  const int cnt = ((a.K >> 6) - wid + NW - 1) / NW;  // this wave's pieces
+  const int rot = cnt > 0 ? ((int)blockIdx.x >> 3) % cnt : 0;
   auto load = [&](int i) {
     lds_b* to = ring + (i % PD) * SLOT;
-    const size_t off = (size_t)i * (NW * 64);
+    const int p = i + rot < cnt ? i + rot : i + rot - cnt;
+    const size_t off = (size_t)p * (NW * 64);
 #pragma unroll
     for (int g = 0; g < 2; ++g) load_line8(wp[g] + off, to + g * 1024);
 #pragma unroll
@@ -168,24 +180,15 @@ __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
     acc[m] = f32x4{0, 0, 0, 0};
     sq[m] = f32x4{0, 0, 0, 0};
   }
-  const int cnt = ((a.K >> 6) - wid + NW - 1) / NW;  // this wave's pieces
 #pragma unroll
   for (int s = 0; s < PD; ++s)
     if (s < cnt) load(s);
   for (int i = 0; i < cnt; ++i) {
     // piece i has landed when only the loads of the PD - 1 behind it are out
     if (i + PD <= cnt) {
-      if (PD == 2) {
-        if (MT == 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-      } else if (PD == 3) {
-        if (MT == 1) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
-      } else {
-        static_assert(PD <= 4, "wait counts");
-        if (MT == 1) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(18)" ::: "memory");
-      }
+      static_assert(PD == 2 && MT <= 2, "wait counts");
+      if (MT == 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
     } else {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
@@ -327,9 +330,10 @@ __global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
 #pragma unroll
   for (int g = 0; g < XG; ++g)
     xp[g] = a.X + (size_t)min((wid * XG + g) * 8 + r8, a.M - 1) * a.K + ch;
+  const int rot = cnt == a.K >> 6 ? ((int)blockIdx.x >> 3) * 2 % cnt : 0;
   auto load = [&](int i) {
     lds_b* to = ring + (i % STAGES) * STAGE;
-    const size_t off = (size_t)i * 64;
+    const size_t off = (size_t)(i + rot < cnt ? i + rot : i + rot - cnt) * 64;
 #pragma unroll
     for (int g = 0; g < 2; ++g)
       load_line8(wp[g] + off, to + wid * PIECE + g * 1024);
@@ -473,14 +477,9 @@ __global__ void __launch_bounds__(256) rows_sum_kernel(
 
 #define ROWS_MAX 16   // rows up to here: gemm_rows_kernel
 
-// Two pieces per wave in flight leave room for a second block per CU, which pays
-// when a CU has several tiles to go through; four are better when it has one:
-// 28672 x 4096 42.9 us against 50.6, 4096 x 14336 22.4 against 24.0 (one row).
 template <int EPI, int NORM>
 static void launch_rows(const RowsArgs& a, hipStream_t st) {
-  const int tiles = a.N / 16;
-  if (tiles > 256) gemm_rows_kernel<1, 2, EPI, NORM><<<tiles, 512, 0, st>>>(a);
-  else gemm_rows_kernel<1, 4, EPI, NORM><<<tiles, 512, 0, st>>>(a);
+  gemm_rows_kernel<1, 2, EPI, NORM><<<a.N / 16, 512, 0, st>>>(a);
 }
 
 // Blocks of 128 weight rows (eight waves) halve the reads of X, from 33 rows on
