@@ -10,7 +10,7 @@
 // number (the operand reads then do not meet in a bank), and the loads of the
 // next pieces are in flight while one is multiplied (counted waits).
 //
-// gemm_rows_kernel, up to 32 rows: a block owns one tile of 16 weight rows (N =
+// gemm_rows_kernel, up to 16 rows: a block owns one tile of 16 weight rows (N =
 //   4096 gives 256 tiles, one per CU; N = 28672 seven per CU) and K is split over
 //   its 8 WAVES, which take 64-element pieces in turn, each through buffers of its
 //   own: no barrier in the loop, no partial sums in memory and no second launch.
@@ -21,10 +21,13 @@
 //   the loop multiplies every X fragment with itself (diagonal of X X^T, one
 //   MFMA), so nobody has to leave row statistics behind.
 // gemm_tile_kernel, more rows: X would be read once per 16 weight rows, so here
-//   four waves own 16 weight rows each and share X: 64 weight rows per block and
-//   STAGES pieces in a ring with one barrier per piece.  K is split over blocks
-//   where N alone does not fill the chip, the fp32 parts meet in the kernel that
-//   does the next step.
+//   four or eight waves share 64 or 128 weight rows and X, STAGES pieces in a ring
+//   with one barrier per piece.  A wave multiplies WT tiles of weights with a WT-th
+//   of X's rows: with WT = 1 every wave reads all of X from LDS, 144 KB per piece
+//   at 128 rows, more cycles than the memory takes to deliver the piece; WT = 4
+//   reads 96 KB (SwiGLU at 128 rows 57.3 -> 52.3 us, 4096 x 14336 28.4 -> 27.7).
+//   K is split over blocks where N alone does not fill the chip, the fp32 parts
+//   meet in the kernel that does the next step.
 //
 // Weight rows lie K * 2 bytes apart, usually a multiple of every channel
 // interleave, so the rows of one piece come from the same memory channel and
@@ -38,8 +41,8 @@
 // launch (in brackets).  One row: 6144 x 4096 with rotary and append 11.2 (21.3 in
 // three launches), 4096 x 4096 7.6 and 4096 x 14336 21.2 (together 44.4), SwiGLU
 // over 28672 x 4096 40.2 = 5.8 TB/s (58.2).  16 rows: 13.4, 8.3, 24.5, 46.0.  64
-// rows, without the closing launches: 13.4, 9.0, 24.8, 45.2 (16.7, o + down 44.8,
-// 62.7).  128 rows: 16.4, 13.0, 28.3, 57.3 (library 25.6 and 57.5 + 5.2 for the
+// rows, without the closing launches: 12.2, 9.0, 23.4, 42.9 (16.7, o + down 44.8,
+// 62.7).  128 rows: 15.2, 12.3, 27.7, 52.3 (library 25.6 and 57.5 + 5.2 for the
 // first and the last, o + down 63.1).
 #include "common.h"
 
@@ -303,7 +306,7 @@ __device__ __forceinline__ void wait_loads_and_meet() {
   }
 }
 
-template <int MT, int NW, int STAGES, int EPI, int NORM>
+template <int MT, int NW, int WT, int STAGES, int EPI, int NORM>
 __global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -316,7 +319,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
   __shared__ __attribute__((aligned(16))) char lds[STAGES * STAGE];
   lds_b* ring = (lds_b*)&lds[0];
 
-  const int tile = blockIdx.x * NW + wid;         // this wave's 16 weight rows
+  const int tile = blockIdx.x * NW + wid;         // the 16 weight rows it fetches
   const int pieces = a.K >> 6;
   const int per = (pieces + (int)gridDim.y - 1) / (int)gridDim.y;
   const int p0 = (int)blockIdx.y * per;
@@ -341,9 +344,14 @@ __global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
     for (int g = 0; g < XG; ++g)
       load_line8(xp[g] + off, to + NW * PIECE + (wid * XG + g) * 1024);
   };
-  f32x4 acc[MT];
+  constexpr int MW = MT / WT;
+  static_assert(NW % WT == 0 && MT % WT == 0, "products divide among the waves");
+  const int w0 = wid / WT * WT, m0 = wid % WT * MW;   // the products it computes
+  f32x4 acc[WT][MW];
 #pragma unroll
-  for (int m = 0; m < MT; ++m) acc[m] = f32x4{0, 0, 0, 0};
+  for (int t = 0; t < WT; ++t)
+#pragma unroll
+    for (int m = 0; m < MW; ++m) acc[t][m] = f32x4{0, 0, 0, 0};
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s)
     if (s < cnt) load(s);
@@ -355,41 +363,50 @@ __global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
     const lds_b* at = ring + (i % STAGES) * STAGE;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const bf16x8r w = frag(at + wid * PIECE, h);
+      bf16x8r w[WT];
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
-        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            frag(at + PIECE * (NW + m), h), w, acc[m], 0, 0, 0);
+      for (int t = 0; t < WT; ++t) w[t] = frag(at + (w0 + t) * PIECE, h);
+#pragma unroll
+      for (int m = 0; m < MW; ++m) {
+        const bf16x8r x = frag(at + PIECE * (NW + m0 + m), h);
+#pragma unroll
+        for (int t = 0; t < WT; ++t)
+          acc[t][m] =
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, w[t], acc[t][m], 0, 0, 0);
+      }
     }
   }
 
-  // lane: column n of the tile, rows m*16 + (lane>>4)*4 + r
+  // lane: column n of each tile, rows (m0 + m)*16 + (lane>>4)*4 + r
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
+  for (int m = 0; m < MW; ++m)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int row = m * 16 + (lane >> 4) * 4 + r;
-      if (EPI == EPI_PARTS) {
-        if (row < a.M)
-          a.parts[((size_t)blockIdx.y * a.M + row) * a.N + tile * 16 + n] = acc[m][r];
-        continue;
-      }
-      float v = acc[m][r];
+      const int row = (m0 + m) * 16 + (lane >> 4) * 4 + r;
+      float rstd = 1.f;
       if (NORM == 1) {
         const float* sp = a.ss + min(row, a.M - 1) * 8;
         float s = 0.f;
 #pragma unroll
         for (int j = 0; j < 8; ++j) s += sp[j];
-        v *= rsqrtf(s * (1.f / (float)a.K) + a.eps);
+        rstd = rsqrtf(s * (1.f / (float)a.K) + a.eps);
       }
-      if (EPI == EPI_SWIGLU) {
-        const float u = __int_as_float(__builtin_amdgcn_update_dpp(
-            0, __float_as_int(v), 0x128, 0xf, 0xf, true));  // row_ror:8
-        if (n < 8 && row < a.M)
-          a.out[(size_t)row * (a.N >> 1) + tile * 8 + n] =
-              f2bf(v / (1.f + __expf(-v)) * u);
-      } else if (row < a.M) {
-        a.out[(size_t)row * a.N + tile * 16 + n] = f2bf(v);
+#pragma unroll
+      for (int t = 0; t < WT; ++t) {
+        const int c = (blockIdx.x * NW + w0 + t) * 16;  // first column of the tile
+        const float v = NORM == 1 ? acc[t][m][r] * rstd : acc[t][m][r];
+        if (EPI == EPI_PARTS) {
+          if (row < a.M)
+            a.parts[((size_t)blockIdx.y * a.M + row) * a.N + c + n] = v;
+        } else if (EPI == EPI_SWIGLU) {
+          const float u = __int_as_float(__builtin_amdgcn_update_dpp(
+              0, __float_as_int(v), 0x128, 0xf, 0xf, true));  // row_ror:8
+          if (n < 8 && row < a.M)
+            a.out[(size_t)row * (a.N >> 1) + c / 2 + n] =
+                f2bf(v / (1.f + __expf(-v)) * u);
+        } else if (row < a.M) {
+          a.out[(size_t)row * a.N + c + n] = f2bf(v);
+        }
       }
     }
 }
@@ -482,24 +499,26 @@ static void launch_rows(const RowsArgs& a, hipStream_t st) {
   gemm_rows_kernel<1, 2, EPI, NORM><<<a.N / 16, 512, 0, st>>>(a);
 }
 
-// Blocks of 128 weight rows (eight waves) halve the reads of X, from 33 rows on
-// for projections so wide that they fill the chip that way, always above 64.
+// Blocks of 128 weight rows (eight waves) halve the reads of X.  They pay from 33
+// rows on where they fill the chip with at least 12 pieces of K each (6144 x 4096 in
+// 5 at 64 rows: 12.2 us against 13.4, 4096 x 14336 in 8: 23.4 against 24.9; but
+// 4096 x 4096 in 8, 8 pieces: 9.7 against 9.0 in 4), below that for whole K only
+// (28672 x 4096 at 32 rows: 43.0 against 44.2), always above 64 rows.
 template <int EPI, int NORM>
 static void launch_tile(const RowsArgs& a, int splits, hipStream_t st) {
   const dim3 g64(a.N / 64, splits), g128(a.N / 128, splits);
-  if (a.M <= 32) {
-    gemm_tile_kernel<2, 4, 4, EPI, NORM><<<g64, 256, 0, st>>>(a);
-  } else if (a.M <= 64) {
-    if (a.N % 128 == 0 && a.N / 128 >= 192)
-      gemm_tile_kernel<4, 8, 3, EPI, NORM><<<g128, 512, 0, st>>>(a);
-    else
-      gemm_tile_kernel<4, 4, 4, EPI, NORM><<<g64, 256, 0, st>>>(a);
-  } else {
-    if (a.N % 128 == 0)
-      gemm_tile_kernel<8, 8, 3, EPI, NORM><<<g128, 512, 0, st>>>(a);
-    else
-      gemm_tile_kernel<8, 4, 3, EPI, NORM><<<g64, 256, 0, st>>>(a);
-  }
+  const bool wide = a.N % 128 == 0 && a.N / 128 * splits >= 192 &&
+                    a.K / 64 >= 12 * splits;
+  if (a.M <= 64 && wide && (a.M > 32 || splits == 1))
+    gemm_tile_kernel<4, 8, 4, 3, EPI, NORM><<<g128, 512, 0, st>>>(a);
+  else if (a.M <= 32)
+    gemm_tile_kernel<2, 4, 1, 4, EPI, NORM><<<g64, 256, 0, st>>>(a);
+  else if (a.M <= 64)
+    gemm_tile_kernel<4, 4, 2, 4, EPI, NORM><<<g64, 256, 0, st>>>(a);
+  else if (a.N % 128 == 0)
+    gemm_tile_kernel<8, 8, 4, 3, EPI, NORM><<<g128, 512, 0, st>>>(a);
+  else
+    gemm_tile_kernel<8, 4, 2, 3, EPI, NORM><<<g64, 256, 0, st>>>(a);
 }
 
 static int check_rows(const RowsArgs& a, int splits) {

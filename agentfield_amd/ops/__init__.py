@@ -266,13 +266,18 @@ def choose_sk(N: int, K: int) -> int:
 def rows_splits(M: int, N: int, K: int) -> int:
     """K splits of the row GEMM's 64- or 128-column blocks (M > 16): one block
     per CU if that comes out nearly full, else two (64-column blocks only, their
-    buffers leave room for that), at least four 64-element pieces each.  Measured
-    at 64 rows: 4096 x 4096 9.0 us in 4 (10.1 in 8, 13.2 in 2), 6144 x 4096
-    13.5 us in 5 (16.9 in 3), 4096 x 14336 24.8 us in 4 (26.7 in 8)."""
+    buffers leave room for that), at least four 64-element pieces each.  128
+    columns above 64 rows, and above 32 where that fills the chip with at least
+    12 pieces each.  Measured at 64 rows: 4096 x 4096 9.0 us in 4 (10.1 in 8,
+    13.2 in 2), 6144 x 4096 12.2 us in 5 (13.4 in 64 columns), 4096 x 14336
+    23.4 us in 8 (24.9 in 4 of 64 columns, 28.7 in 7)."""
     pieces = K // 64
-    wide = M > 64 and N % 128 == 0
+    wide = M > 32 and N % 128 == 0
     blocks = N // 128 if wide else N // 64
     n = max(1, 256 // blocks)
+    if wide and M <= 64 and (n * blocks < 192 or pieces < 12 * n):
+        wide, blocks = False, N // 64
+        n = max(1, 256 // blocks)
     if not wide and n * blocks < 224:
         n = max(1, 512 // blocks)
     n = max(1, min(n, 16, pieces // 4))

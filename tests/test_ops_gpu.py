@@ -546,11 +546,12 @@ ROW_COUNTS = [1, 3, 16, 17, 32, 33, 64, 65, 100, 128]
 
 @pytest.mark.parametrize("M", ROW_COUNTS)
 @pytest.mark.parametrize("N,K", [(64, 64), (192, 448), (4096, 512),
-                                 (320, 1088), (32768, 256)])
+                                 (320, 1088), (32768, 256), (3072, 7744),
+                                 (24576, 832)])
 def test_linear_rows_modes(M, N, K):
     """Every epilogue of the row GEMMs at the edges of their row classes, with
     fewer K pieces than waves, odd piece counts, odd tile counts and both widths
-    of block.  Tolerance: bf16 rounding of the result (2^-8 relative) and fp32
+    of block, split and whole.  Tolerance: bf16 rounding of the result (2^-8 relative) and fp32
     sums over K of products of ~0.1 size."""
     x = rnd(M, K, seed=M + K, scale=0.3)
     w = rnd(N, K, seed=N, scale=0.3)
