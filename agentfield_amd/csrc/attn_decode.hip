@@ -30,8 +30,11 @@
 //   Rows, then waves (through LDS), then splits (second kernel) merge once.
 // Measured with 8 K/V heads, G = 4, against one lane group per token with a
 // shuffle reduction per score: 24 sequences of 1800..8100 tokens (513 MB)
-// 225 -> 112 us (4.6 TB/s), 128 of 545 101 -> 56 us (5.1 TB/s), 1 of 8000
-// 58 -> 22 us.
+// 225 -> 108 us (4.7 TB/s), 128 of 545 101 -> 52 us (5.4 TB/s), 1 of 8000
+// 58 -> 22 us.  V is read with nontemporal loads, whole rows per instruction: 114
+// -> 108 and 57.3 -> 52.5 us.  K is not: two instructions share each of its lines,
+// and a line dropped between them is fetched twice (64 ragged sequences of up to
+// 2000 tokens 60 -> 65 us with both, 59 with V only).
 #include "common.h"
 
 #include <type_traits>
@@ -144,8 +147,8 @@ __global__ void __launch_bounds__(64 * AD_WAVES, G == 8 ? 3 : 4) attn_decode_ker
       const int lo = t0 - t, hi = t1 - 1 - t;
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        vf[r] = *reinterpret_cast<const s16x8*>(
-            vp + min(max(tg * 4 + r, lo), hi) * AD_D);
+        vf[r] = __builtin_nontemporal_load(reinterpret_cast<const s16x8*>(
+            vp + min(max(tg * 4 + r, lo), hi) * AD_D));
     } else {
       auto row = [&](int tok) {
         const int tc = min(max(tok, t0), t1 - 1);
@@ -157,7 +160,8 @@ __global__ void __launch_bounds__(64 * AD_WAVES, G == 8 ? 3 : 4) attn_decode_ker
         kf[c] = *reinterpret_cast<const s16x8*>(kp + c * 32);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        vf[r] = *reinterpret_cast<const s16x8*>(vc + row(t + tg * 4 + r) + dl * 8);
+        vf[r] = __builtin_nontemporal_load(
+            reinterpret_cast<const s16x8*>(vc + row(t + tg * 4 + r) + dl * 8));
     }
   };
 
