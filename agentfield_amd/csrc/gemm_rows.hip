@@ -35,14 +35,14 @@
 // XCD therefore start at different pieces (the order of a sum depends on the
 // column, not on M); where K is split the splits do that already and starting
 // elsewhere costs a little (4096 x 4096 in four, 32 rows: 8.0 -> 8.8 us).  SwiGLU over 28672 x 4096: 42.9 -> 40.2 us at one row, 53.4 -> 45.2
-// at 64, 62.3 -> 57.3 at 128; two pieces per wave in flight are then enough (four
+// at 64, 62.3 -> 57.3 at 128 (before the weights were streamed); two pieces per wave in flight are then enough (four
 // needed half the CU's buffers: 50.5 us).
 // Measured in us, against the split-K kernel with two-stage buffers and its second
-// launch (in brackets).  One row: 6144 x 4096 with rotary and append 11.2 (21.3 in
-// three launches), 4096 x 4096 7.6 and 4096 x 14336 21.2 (together 44.4), SwiGLU
-// over 28672 x 4096 40.2 = 5.8 TB/s (58.2).  16 rows: 13.4, 8.3, 24.5, 46.0.  64
-// rows, without the closing launches: 12.2, 9.0, 23.4, 42.9 (16.7, o + down 44.8,
-// 62.7).  128 rows: 15.2, 12.3, 27.7, 52.3 (library 25.6 and 57.5 + 5.2 for the
+// launch (in brackets).  One row: 6144 x 4096 with rotary and append 10.7 (21.3 in
+// three launches), 4096 x 4096 7.3 and 4096 x 14336 19.0 (together 44.4), SwiGLU
+// over 28672 x 4096 37.5 = 6.3 TB/s (58.2).  16 rows: 13.1, 8.1, 23.1, 42.6.  64
+// rows, without the closing launches: 11.2, 8.5, 21.7, 40.1 (16.7, o + down 44.8,
+// 62.7).  128 rows: 14.3, 12.6, 26.8, 50.0 (library 25.6 and 57.5 + 5.2 for the
 // first and the last, o + down 63.1).
 #include "common.h"
 
@@ -80,11 +80,13 @@ struct RowsArgs {
 // 8 rows x 128 bytes of a row-major matrix into linear LDS: lane l brings chunk
 // (l & 7) ^ (row & 7) of row l >> 3, so that chunk c of row r sits at slot
 // c ^ (r & 7).
+template <int AUX>
 __device__ __forceinline__ void load_line8(const u16* src, lds_b* dst) {
   __builtin_amdgcn_global_load_lds(
       (const __attribute__((address_space(1))) uint32_t*)src,
-      (__attribute__((address_space(3))) uint32_t*)dst, 16, 0, 0);
+      (__attribute__((address_space(3))) uint32_t*)dst, 16, 0, AUX);
 }
+constexpr int STREAM = 2, KEEP = 0;   // AUX: nontemporal, cached
 
 // operand fragment: lane (r = lane & 15, q = lane >> 4) gets k = 32 h + 8 q .. +8
 // of row r of a 16-row piece
@@ -137,7 +139,7 @@ __device__ __forceinline__ void put_rope(const RowsArgs& a, int m, int head, int
 }
 
 // NORM: 0 none, 1 from ss, 2 computed from X.  PD pieces per wave in flight.
-template <int MT, int PD, int EPI, int NORM>
+template <int MT, int PD, int EPI, int NORM, int AUX>
 __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
   constexpr int NW = 8;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -172,10 +174,10 @@ __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
     const int p = i + rot < cnt ? i + rot : i + rot - cnt;
     const size_t off = (size_t)p * (NW * 64);
 #pragma unroll
-    for (int g = 0; g < 2; ++g) load_line8(wp[g] + off, to + g * 1024);
+    for (int g = 0; g < 2; ++g) load_line8<AUX>(wp[g] + off, to + g * 1024);
 #pragma unroll
     for (int g = 0; g < MT * 2; ++g)
-      load_line8(xp[g] + off, to + PIECE + g * 1024);
+      load_line8<KEEP>(xp[g] + off, to + PIECE + g * 1024);
   };
   f32x4 acc[MT], sq[MT];
 #pragma unroll
@@ -306,7 +308,7 @@ __device__ __forceinline__ void wait_loads_and_meet() {
   }
 }
 
-template <int MT, int NW, int WT, int STAGES, int EPI, int NORM>
+template <int MT, int NW, int WT, int STAGES, int EPI, int NORM, int AUX>
 __global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -339,10 +341,10 @@ __global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
     const size_t off = (size_t)(i + rot < cnt ? i + rot : i + rot - cnt) * 64;
 #pragma unroll
     for (int g = 0; g < 2; ++g)
-      load_line8(wp[g] + off, to + wid * PIECE + g * 1024);
+      load_line8<AUX>(wp[g] + off, to + wid * PIECE + g * 1024);
 #pragma unroll
     for (int g = 0; g < XG; ++g)
-      load_line8(xp[g] + off, to + NW * PIECE + (wid * XG + g) * 1024);
+      load_line8<KEEP>(xp[g] + off, to + NW * PIECE + (wid * XG + g) * 1024);
   };
   constexpr int MW = MT / WT;
   static_assert(NW % WT == 0 && MT % WT == 0, "products divide among the waves");
@@ -494,9 +496,19 @@ __global__ void __launch_bounds__(256) rows_sum_kernel(
 
 #define ROWS_MAX 16   // rows up to here: gemm_rows_kernel
 
+// Weights from here on are streamed past the caches, and X stays in them: SwiGLU
+// over 28672 x 4096 40.5 -> 37.5 us (6.3 TB/s) at one row, 42.8 -> 40.1 at 64, 52.0
+// -> 50.0 at 128; 4096 x 14336 21.4 -> 19.0, 23.3 -> 21.7, 27.6 -> 26.8.  Smaller
+// ones are bound by latency, which is higher that way (2048 x 2048 5.1 us against
+// 4.1 from memory, 3.9 against 2.9 from the L2).
+static bool streamed(const RowsArgs& a) { return (i64)a.N * a.K >= (8 << 20); }
+
 template <int EPI, int NORM>
 static void launch_rows(const RowsArgs& a, hipStream_t st) {
-  gemm_rows_kernel<1, 2, EPI, NORM><<<a.N / 16, 512, 0, st>>>(a);
+  if (streamed(a))
+    gemm_rows_kernel<1, 2, EPI, NORM, STREAM><<<a.N / 16, 512, 0, st>>>(a);
+  else
+    gemm_rows_kernel<1, 2, EPI, NORM, KEEP><<<a.N / 16, 512, 0, st>>>(a);
 }
 
 // Blocks of 128 weight rows (eight waves) halve the reads of X.  They pay from 33
@@ -504,21 +516,27 @@ static void launch_rows(const RowsArgs& a, hipStream_t st) {
 // 5 at 64 rows: 12.2 us against 13.4, 4096 x 14336 in 8: 23.4 against 24.9; but
 // 4096 x 4096 in 8, 8 pieces: 9.7 against 9.0 in 4), below that for whole K only
 // (28672 x 4096 at 32 rows: 43.0 against 44.2), always above 64 rows.
-template <int EPI, int NORM>
-static void launch_tile(const RowsArgs& a, int splits, hipStream_t st) {
+template <int EPI, int NORM, int AUX>
+static void launch_tile_as(const RowsArgs& a, int splits, hipStream_t st) {
   const dim3 g64(a.N / 64, splits), g128(a.N / 128, splits);
   const bool wide = a.N % 128 == 0 && a.N / 128 * splits >= 192 &&
                     a.K / 64 >= 12 * splits;
   if (a.M <= 64 && wide && (a.M > 32 || splits == 1))
-    gemm_tile_kernel<4, 8, 4, 3, EPI, NORM><<<g128, 512, 0, st>>>(a);
+    gemm_tile_kernel<4, 8, 4, 3, EPI, NORM, AUX><<<g128, 512, 0, st>>>(a);
   else if (a.M <= 32)
-    gemm_tile_kernel<2, 4, 1, 4, EPI, NORM><<<g64, 256, 0, st>>>(a);
+    gemm_tile_kernel<2, 4, 1, 4, EPI, NORM, AUX><<<g64, 256, 0, st>>>(a);
   else if (a.M <= 64)
-    gemm_tile_kernel<4, 4, 2, 4, EPI, NORM><<<g64, 256, 0, st>>>(a);
+    gemm_tile_kernel<4, 4, 2, 4, EPI, NORM, AUX><<<g64, 256, 0, st>>>(a);
   else if (a.N % 128 == 0)
-    gemm_tile_kernel<8, 8, 4, 3, EPI, NORM><<<g128, 512, 0, st>>>(a);
+    gemm_tile_kernel<8, 8, 4, 3, EPI, NORM, AUX><<<g128, 512, 0, st>>>(a);
   else
-    gemm_tile_kernel<8, 4, 2, 3, EPI, NORM><<<g64, 256, 0, st>>>(a);
+    gemm_tile_kernel<8, 4, 2, 3, EPI, NORM, AUX><<<g64, 256, 0, st>>>(a);
+}
+
+template <int EPI, int NORM>
+static void launch_tile(const RowsArgs& a, int splits, hipStream_t st) {
+  if (streamed(a)) launch_tile_as<EPI, NORM, STREAM>(a, splits, st);
+  else launch_tile_as<EPI, NORM, KEEP>(a, splits, st);
 }
 
 static int check_rows(const RowsArgs& a, int splits) {
