@@ -552,7 +552,8 @@ static int check_rows(const RowsArgs& a, int splits) {
 // mode 0 plain, 1 residual add (in place, also to `out` if given), 2 SwiGLU,
 // 4 residual add + row sums of squares of the result to ss_out [M, 8].
 // norm 0 none, 1 RMSNorm scalar of X from ss [M, 8], 2 computed (<= 16 rows).
-// parts [splits, M, N]: needed unless rows <= 16 (and mode 0..2) or mode 2.
+// parts [splits, M, N]: needed unless rows <= 16 (and mode 0..2), mode 2, or mode 0
+// in one split.
 AF_EXPORT int af_rows_linear(void* out, void* residual, void* parts, void* ss_out,
                              const void* X, const void* W, int M, int N, int K,
                              int splits, int mode, int norm, const void* ss,
@@ -589,6 +590,11 @@ AF_EXPORT int af_rows_linear(void* out, void* residual, void* parts, void* ss_ou
   if (mode == 2) {
     if (norm == 0) launch_tile<EPI_SWIGLU, 0>(a, 1, st);
     else launch_tile<EPI_SWIGLU, 1>(a, 1, st);
+    return af_last_err();
+  }
+  if (mode == 0 && splits == 1) {
+    if (norm == 0) launch_tile<EPI_PLAIN, 0>(a, 1, st);
+    else launch_tile<EPI_PLAIN, 1>(a, 1, st);
     return af_last_err();
   }
   if (!parts) return 9008;

@@ -312,7 +312,9 @@ def linear_rows(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
     splits, parts = 1, None
     if mode != 2 and (M > ROWS_MAX or mode == 4):
         splits = rows_splits(M, N, K)
-        parts = torch.empty(splits, M, N, dtype=torch.float32, device=x.device)
+        if splits > 1 or mode != 0:
+            parts = torch.empty(splits, M, N, dtype=torch.float32,
+                                device=x.device)
     norm, ss, eps = 0, None, 0.0
     if scale is not None:
         ss, eps = scale
@@ -398,14 +400,18 @@ def linear_skinny(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
 def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
            out: torch.Tensor | None = None) -> torch.Tensor:
     """Linear layer dispatch: hand-written weight-streaming kernels up to 128
-    rows, hipBLASLt (torch.matmul) for prefill GEMMs and vocabulary-sized N.
-    out (without silu_fuse): contiguous rows to write to.
+    rows, hipBLASLt (torch.matmul) for prefill GEMMs.  out (without silu_fuse):
+    contiguous rows to write to.
 
-    Measured at 128 rows, where the kernels gain least: 6144 x 4096 21 us with
-    the sum of its splits against the library's 26, 4096 x 14336 33 against 45,
-    SwiGLU over 28672 x 4096 62 us against 58 + 5; one row of 128256 x 4096 is at
-    the memory rate in both."""
-    if _rows_ok(x, w) and (silu_fuse or w.shape[0] <= 12288) and not (
+    Plain products of 33..128 rows lose to the library where N fills the chip
+    neither in blocks of 128 columns nor in several splits.  Measured, library
+    against rows in us: 14336 x 4096 25.6 / 21.7 at 32 rows, 26.7 / 30.0 at 48,
+    33.9 / 36.0 at 128; 16384 x 4096 34.3 / 24.7, 34.9 / 38.9, 39.0 / 43.3;
+    28672 x 4096 53.9 / 41.5, 64.0 / 42.1, 56.7 / 51.7; 128256 x 4096 190 / 151
+    at one row, 214 / 184 at 64, 238 / 215 at 128."""
+    M, N = x.shape[0], w.shape[0]
+    if _rows_ok(x, w) and (
+            silu_fuse or M <= 32 or N <= 12288 or N >= 24576) and not (
             torch.is_grad_enabled() and x.requires_grad):
         return linear_rows(x, w, mode=2 if silu_fuse else 0, out=out)
     if out is not None:

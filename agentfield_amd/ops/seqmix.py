@@ -671,12 +671,13 @@ def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
 
     bf16 products of few rows (decode steps) run on the framework's
     weight-streaming kernels, wider ones and prompts on the vendor GEMM
-    (hipBLASLt / rocBLAS).  Up to 16 rows that is one launch, above a second one
-    adds the K splits up, which wide weights do not earn back.  Measured, vendor
-    against rows in us: 2048 x 2048 11.1 / 4.6 at 4 rows, 11.7 / 8.8 at 64;
-    10240 x 2048 16.3 / 11.5 at 16 rows, 14.5 / 13.4 at 32, 15.9 / 15.7 at 64;
-    6144 x 2048 12.5 / 11.5 at 32, 13.1 / 13.7 at 64; 2048 x 8192 22.5 / 12.4 at
-    64; 14336 x 4096 29.6 / 25.9 at 16, 24.8 / 27.8 at 24.  AF_MIX_SKINNY=1 sends
+    (hipBLASLt / rocBLAS).  Above 16 rows a second launch adds the K splits up
+    unless N fills the chip by itself, which middling widths do not earn back.
+    Measured, vendor against rows in us: 4096 x 4096 15.7 / 7.8 at 4 rows, 15.3 /
+    12.7 at 64, 16.2 / 18.2 at 100; 6144 x 2048 12.8 / 11.0 at 32, 13.2 / 13.9 at
+    64; 10240 x 2048 16.4 / 9.6 at 4, 16.4 / 13.9 at 32, 19.6 / 21.3 at 128;
+    14336 x 4096 25.6 / 21.7 at 32, 26.7 / 30.0 at 48; 128256 x 2048 111 / 91 at
+    32, 125 / 124 at 128.  AF_MIX_SKINNY=1 sends
     the remaining decode-sized products (up to 64 rows, or 33..128 against a long
     inner dimension) to the framework's kernels too."""
     if out is not None:
@@ -684,9 +685,8 @@ def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
     M, K = x.shape
     N = w.shape[0]
     if skinny and x.is_cuda and M <= 128 and _lib.main_lib_ready():
-        from . import ROWS_MAX, _rows_ok, linear_rows, linear_skinny
-        if ((M <= ROWS_MAX and N <= 16384 or M <= 32 and N <= 10240
-                or M <= 64 and N <= 4096) and _rows_ok(x, w)
+        from . import _rows_ok, linear_rows, linear_skinny
+        if ((M <= 32 or M <= 64 and N <= 4096 or N >= 24576) and _rows_ok(x, w)
                 and not (torch.is_grad_enabled() and x.requires_grad)):
             return linear_rows(x, w)
         if (_SKINNY and x.dtype == torch.bfloat16
