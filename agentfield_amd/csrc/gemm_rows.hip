@@ -25,7 +25,8 @@
 //   with one barrier per piece.  A wave multiplies WT tiles of weights with a WT-th
 //   of X's rows: with WT = 1 every wave reads all of X from LDS, 144 KB per piece
 //   at 128 rows, more cycles than the memory takes to deliver the piece; WT = 4
-//   reads 96 KB (SwiGLU at 128 rows 57.3 -> 52.3 us, 4096 x 14336 28.4 -> 27.7).
+//   reads 96 KB (SwiGLU at 128 rows 57.3 -> 52.3 us, 4096 x 14336 28.4 -> 27.7,
+//   both before the weights were streamed).
 //   K is split over blocks where N alone does not fill the chip, the fp32 parts
 //   meet in the kernel that does the next step.
 //
@@ -513,9 +514,10 @@ static void launch_rows(const RowsArgs& a, hipStream_t st) {
 
 // Blocks of 128 weight rows (eight waves) halve the reads of X.  They pay from 33
 // rows on where they fill the chip with at least 12 pieces of K each (6144 x 4096 in
-// 5 at 64 rows: 12.2 us against 13.4, 4096 x 14336 in 8: 23.4 against 24.9; but
-// 4096 x 4096 in 8, 8 pieces: 9.7 against 9.0 in 4), below that for whole K only
-// (28672 x 4096 at 32 rows: 43.0 against 44.2), always above 64 rows.
+// 5 at 64 rows: 11.2 us against 12.8, 4096 x 14336 in 8: 21.7 against 23.1; but
+// 4096 x 4096 in 8, 8 pieces: 8.8 against 8.5 in 4), below that for whole K only
+// (28672 x 4096 at 32 rows, weights not streamed: 43.0 against 44.2), always above
+// 64 rows.
 template <int EPI, int NORM, int AUX>
 static void launch_tile_as(const RowsArgs& a, int splits, hipStream_t st) {
   const dim3 g64(a.N / 64, splits), g128(a.N / 128, splits);

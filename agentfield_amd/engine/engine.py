@@ -36,8 +36,9 @@ def _bucket_for(n: int, max_bs: int) -> int:
 def choose_nsplit(bs: int, hk: int) -> int:
     """Decode attention split-K factor: about 512 workgroups, two per CU,
     whose waves keep enough K/V in flight.  Measured, 8 K/V heads: 64 sequences
-    of 540 tokens 30.7 us unsplit (34.4 in two), 8 of 1600 22.5 us in 8 (24.0
-    in 4, 24.9 in 16), 1 of 8000 22.2 us in 16 (28.6 in 8, 23.3 in 32)."""
+    of 545 tokens 28.3 us unsplit (31.8 in two), 8 of 300..3000 20.9 us in 8
+    (21.1 in 4, 23.4 in 16), 24 of 1800..8100 108 us in 2 (158 unsplit, 105 in
+    4 or 8, 111 in 16)."""
     target = 512
     ns = max(1, min(16, target // max(1, bs * hk)))
     return 1 << (ns.bit_length() - 1)

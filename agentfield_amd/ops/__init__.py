@@ -268,9 +268,9 @@ def rows_splits(M: int, N: int, K: int) -> int:
     per CU if that comes out nearly full, else two (64-column blocks only, their
     buffers leave room for that), at least four 64-element pieces each.  128
     columns above 64 rows, and above 32 where that fills the chip with at least
-    12 pieces each.  Measured at 64 rows: 4096 x 4096 9.0 us in 4 (10.1 in 8,
-    13.2 in 2), 6144 x 4096 12.2 us in 5 (13.4 in 64 columns), 4096 x 14336
-    23.4 us in 8 (24.9 in 4 of 64 columns, 28.7 in 7)."""
+    12 pieces each.  Measured at 64 rows: 4096 x 4096 8.5 us in 4 (8.8 in 8 of
+    128 columns), 6144 x 4096 11.2 us in 5 (12.8 in 64 columns), 4096 x 14336
+    21.7 us in 8 (23.1 in 4 of 64 columns)."""
     pieces = K // 64
     wide = M > 32 and N % 128 == 0
     blocks = N // 128 if wide else N // 64
