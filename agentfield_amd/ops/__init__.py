@@ -286,11 +286,15 @@ def rows_splits(M: int, N: int, K: int) -> int:
 
 
 def _rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """What the row GEMMs take: bf16 rows and weights that lie whole and on
-    16-byte boundaries, whole 64 x 64 tiles of weights, 1..128 rows."""
-    return (x.is_cuda and 0 < x.shape[0] <= 128 and w.shape[0] % 64 == 0
-            and w.shape[1] % 64 == 0 and x.is_contiguous()
-            and w.is_contiguous() and x.dtype == w.dtype == torch.bfloat16
+    """What the row GEMMs take: bf16 rows and weights of one length on one GPU,
+    which lie whole and on 16-byte boundaries, whole 64 x 64 tiles of weights,
+    1..128 rows.  The kernels read w by the length of x's rows."""
+    if not x.is_cuda or x.dim() != 2 or w.dim() != 2:
+        return False
+    (M, K), (N, KW) = x.shape, w.shape
+    return (K == KW and 0 < M <= 128 and K > 0 and N > 0 and N % 64 == 0
+            and K % 64 == 0 and x.is_contiguous() and w.is_contiguous()
+            and x.dtype == w.dtype == torch.bfloat16 and x.device == w.device
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
@@ -304,6 +308,9 @@ def linear_rows(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
     scalar is computed from x itself (up to 16 rows).  want_out=False (modes 1
     and 4): only the residual is written.  x and residual must not overlap.
     out: contiguous rows to write to."""
+    if not _rows_ok(x, w):
+        raise AfOpsError(f"row GEMM: {tuple(x.shape)} {x.dtype} rows against "
+                         f"{tuple(w.shape)} {w.dtype} weights")
     M, K = x.shape
     N = w.shape[0]
     if want_out and out is None:
@@ -374,6 +381,8 @@ def linear_skinny(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
     """
     M, K = x.shape
     N = w.shape[0]
+    if w.shape[1] != K:
+        raise AfOpsError(f"linear_skinny: rows of {K} against {w.shape[1]}")
     if sk is None and _rows_ok(x, w) and (mode in (0, 2) or (
             scale is None and x.untyped_storage().data_ptr()
             != residual.untyped_storage().data_ptr())):
@@ -409,7 +418,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
     33.9 / 36.0 at 128; 16384 x 4096 34.3 / 24.7, 34.9 / 38.9, 39.0 / 43.3;
     28672 x 4096 53.9 / 41.5, 64.0 / 42.1, 56.7 / 51.7; 128256 x 4096 190 / 151
     at one row, 214 / 184 at 64, 238 / 215 at 128."""
-    M, N = x.shape[0], w.shape[0]
+    M, _K = x.shape
+    N = w.shape[0]
     if _rows_ok(x, w) and (
             silu_fuse or M <= 32 or N <= 12288 or N >= 24576) and not (
             torch.is_grad_enabled() and x.requires_grad):

@@ -579,6 +579,20 @@ def test_linear_rows_modes(M, N, K):
                                   rtol=1e-4)
 
 
+@pytest.mark.parametrize("M", [1, 17, 128])
+@pytest.mark.parametrize("K,KW", [(512, 448), (448, 512), (64, 4096)])
+def test_row_products_refuse_other_inner_lengths(M, K, KW):
+    """Rows and weights of different length are refused by every way in, as a
+    matrix product refuses them, not read past their end."""
+    from agentfield_amd.ops import seqmix as sm
+    x, w = rnd(M, K, seed=1), rnd(32768, KW, seed=2)
+    for call in (ops.linear, ops.linear_rows, ops.linear_skinny, sm.matmul):
+        with pytest.raises(RuntimeError):
+            call(x, w)
+    with pytest.raises(RuntimeError):
+        ops.linear(x, w, silu_fuse=True)
+
+
 @pytest.mark.parametrize("M", ROW_COUNTS)
 @pytest.mark.parametrize("Hq,Hk,K", [(2, 1, 256), (8, 8, 192), (32, 8, 1024)])
 def test_qkv_rope_rows(M, Hq, Hk, K):
