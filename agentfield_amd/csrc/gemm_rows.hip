@@ -571,6 +571,8 @@ AF_EXPORT int af_rows_linear(void* out, void* residual, void* parts, void* ss_ou
   a.eps = eps;
   if (const int rc = check_rows(a, splits)) return rc;
   if (mode != 0 && mode != 2 && norm != 0) return 9008;
+  if (mode == 0 || mode == 2 ? !out : !residual) return 9008;
+  if ((mode == 4 && !ss_out) || (norm == 1 && !ss)) return 9008;
   hipStream_t st = (hipStream_t)stream;
   if (M <= ROWS_MAX && mode != 4) {
     if (mode == 0) {
@@ -606,7 +608,6 @@ AF_EXPORT int af_rows_linear(void* out, void* residual, void* parts, void* ss_ou
     rows_sum_kernel<<<g, 256, 0, st>>>(a.out, a.parts, norm ? a.ss : nullptr, M, N,
                                        splits, 1.f / (float)K, eps);
   } else if (mode == 1 || mode == 4) {
-    if (mode == 4 && !ss_out) return 9008;
     rows_residual_kernel<<<dim3(M, 8), 256, 0, st>>>(
         a.residual, a.out, a.parts, (float*)ss_out, M, N, splits);
   } else {

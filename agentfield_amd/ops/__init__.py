@@ -298,6 +298,31 @@ def _rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
+def _need(ok: bool, what: str) -> None:
+    if not ok:
+        raise AfOpsError(what)
+
+
+def _whole(t: torch.Tensor | None, x: torch.Tensor, *shape: int) -> bool:
+    """t can be written as x's kind of rows of that shape, two at a time."""
+    return (t is not None and tuple(t.shape) == shape and t.dtype == x.dtype
+            and t.device == x.device and t.is_contiguous()
+            and t.data_ptr() % 4 == 0)
+
+
+def _row_stats(ss: torch.Tensor | None, x: torch.Tensor) -> bool:
+    """ss holds (or takes) eight fp32 sums for each of x's rows."""
+    return (ss is not None and ss.dtype == torch.float32
+            and ss.device == x.device and ss.is_contiguous()
+            and ss.numel() >= 8 * x.shape[0])
+
+
+def _apart(a: torch.Tensor, b: torch.Tensor) -> bool:
+    pa, pb = a.data_ptr(), b.data_ptr()
+    return (pa + a.numel() * a.element_size() <= pb
+            or pb + b.numel() * b.element_size() <= pa)
+
+
 def linear_rows(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
                 residual: torch.Tensor | None = None,
                 scale: tuple | None = None,
@@ -313,9 +338,19 @@ def linear_rows(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
                          f"{tuple(w.shape)} {w.dtype} weights")
     M, K = x.shape
     N = w.shape[0]
-    if want_out and out is None:
-        out = torch.empty(M, N // 2 if mode == 2 else N, dtype=x.dtype,
-                          device=x.device)
+    cols = N // 2 if mode == 2 else N
+    if mode in (1, 4):
+        _need(_whole(residual, x, M, N) and _apart(residual, x),
+              "row GEMM: the residual must be whole rows apart from x")
+        _need(mode == 1 or _row_stats(ss_out, x),
+              "row GEMM: mode 4 leaves fp32 [M, 8] sums in ss_out")
+    else:
+        _need(mode in (0, 2) and want_out, f"row GEMM: mode {mode}")
+    if out is not None:
+        _need(_whole(out, x, M, cols) and _apart(out, x),
+              f"row GEMM: out must be whole [{M}, {cols}] rows apart from x")
+    elif want_out:
+        out = torch.empty(M, cols, dtype=x.dtype, device=x.device)
     splits, parts = 1, None
     if mode != 2 and (M > ROWS_MAX or mode == 4):
         splits = rows_splits(M, N, K)
@@ -326,6 +361,9 @@ def linear_rows(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
     if scale is not None:
         ss, eps = scale
         norm = 2 if ss is None else 1
+        _need(mode in (0, 2) and (M <= ROWS_MAX if ss is None
+                                  else _row_stats(ss, x)),
+              "row GEMM: fp32 [M, 8] sums of the rows for the norm")
     rc = _lib.lib().af_rows_linear(
         _lib.ptr(out), _lib.ptr(residual), _lib.ptr(parts), _lib.ptr(ss_out),
         _lib.ptr(x), _lib.ptr(w), M, N, K, splits, mode, norm, _lib.ptr(ss), eps,
@@ -383,9 +421,12 @@ def linear_skinny(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
     N = w.shape[0]
     if w.shape[1] != K:
         raise AfOpsError(f"linear_skinny: rows of {K} against {w.shape[1]}")
-    if sk is None and _rows_ok(x, w) and (mode in (0, 2) or (
-            scale is None and x.untyped_storage().data_ptr()
-            != residual.untyped_storage().data_ptr())):
+    _need(mode in (0, 2) or residual is not None and mode in (1, 4)
+          and (mode == 1 or ss_out is not None), f"linear_skinny: mode {mode}")
+    if sk is None and _rows_ok(x, w) and (
+            (scale is None or _row_stats(scale[0], x)) if mode in (0, 2) else
+            scale is None and _whole(residual, x, M, N) and _apart(residual, x)
+            and (mode == 1 or _row_stats(ss_out, x))):
         return linear_rows(x, w, mode, residual, scale, ss_out)
     if sk is None:
         sk = choose_sk(N, K)
@@ -410,7 +451,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
            out: torch.Tensor | None = None) -> torch.Tensor:
     """Linear layer dispatch: hand-written weight-streaming kernels up to 128
     rows, hipBLASLt (torch.matmul) for prefill GEMMs.  out (without silu_fuse):
-    contiguous rows to write to.
+    [M, N] rows of x's type to write to.
 
     Plain products of 33..128 rows lose to the library where N fills the chip
     neither in blocks of 128 columns nor in several splits.  Measured, library
@@ -420,7 +461,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
     at one row, 214 / 184 at 64, 238 / 215 at 128."""
     M, _K = x.shape
     N = w.shape[0]
-    if _rows_ok(x, w) and (
+    if out is not None:
+        _need(not silu_fuse and tuple(out.shape) == (M, N),
+              f"linear: out {tuple(out.shape)} for a [{M}, {N}] product")
+    if (out is None or _whole(out, x, M, N)) and _rows_ok(x, w) and (
             silu_fuse or M <= 32 or N <= 12288 or N >= 24576) and not (
             torch.is_grad_enabled() and x.requires_grad):
         return linear_rows(x, w, mode=2 if silu_fuse else 0, out=out)

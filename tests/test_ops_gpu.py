@@ -593,6 +593,48 @@ def test_row_products_refuse_other_inner_lengths(M, K, KW):
         ops.linear(x, w, silu_fuse=True)
 
 
+@pytest.mark.parametrize("M", [3, 40])
+def test_linear_rows_refuses_other_buffers(M):
+    """Outputs, residuals and row sums that are not what the kernels write to:
+    other shapes, types, devices, strides, overlap with the rows."""
+    K = N = 256
+    x, w, res = rnd(M, K, seed=1), rnd(N, K, seed=2), rnd(M, N, seed=3)
+    before = res.clone()
+    st = torch.zeros(M, 8, device=DEV)
+    wide = rnd(M, 2 * N, seed=4)
+    odd = torch.zeros(M * N + 1, dtype=torch.bfloat16, device=DEV)[1:]
+    bad_rows = [rnd(M, N // 2), rnd(M + 1, N), wide[:, :N], odd.view(M, N),
+                res.float(), res.cpu(), res.flatten()]
+    bad = [dict(mode=3), dict(mode=1), dict(mode=1, residual=x),
+           dict(mode=4, residual=res), dict(mode=4, residual=res, ss_out=st.double()),
+           dict(mode=4, residual=res, ss_out=st[:M - 1]),
+           dict(mode=4, residual=res, ss_out=st, scale=(st, 1e-5)),
+           dict(scale=(st.half(), 1e-5)), dict(mode=2, scale=(st[1:], 1e-5)),
+           dict(want_out=False), dict(out=x), dict(mode=2, out=rnd(M, N))]
+    bad += [dict(out=t) for t in bad_rows]
+    bad += [dict(mode=1, residual=t) for t in bad_rows]
+    if M > ops.ROWS_MAX:
+        bad.append(dict(scale=(None, 1e-5)))
+    for kw in bad:
+        with pytest.raises(ops.AfOpsError):
+            ops.linear_rows(x, w, **kw)
+    for kw in (dict(mode=1), dict(mode=4, residual=res), dict(mode=3)):
+        with pytest.raises(ops.AfOpsError):
+            ops.linear_skinny(x, w, **kw)
+    for t in (rnd(M, N // 2), rnd(M + 1, N), res.flatten()):
+        with pytest.raises(ops.AfOpsError):
+            ops.linear(x, w, out=t)
+    assert torch.equal(res, before)
+    # what the kernels do not write to, the library does
+    got = wide[:, :N]
+    assert ops.linear(x, w, out=got) is got
+    assert close(got, x.float() @ w.float().t(), atol=0.2)
+    # residuals of another form still take the split-K kernel
+    r3 = before.view(M, 1, N).clone()
+    assert close(ops.linear_skinny(x, w, 1, r3),
+                 x.float() @ w.float().t() + before.float(), atol=0.2)
+
+
 @pytest.mark.parametrize("M", ROW_COUNTS)
 @pytest.mark.parametrize("Hq,Hk,K", [(2, 1, 256), (8, 8, 192), (32, 8, 1024)])
 def test_qkv_rope_rows(M, Hq, Hk, K):
