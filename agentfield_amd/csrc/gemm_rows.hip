@@ -620,10 +620,12 @@ AF_EXPORT int af_rows_linear(void* out, void* residual, void* parts, void* ss_ou
 // [M, Hq*128] to `q`, k and v to their pages only.  Up to 16 rows compute the
 // RMSNorm scalar themselves; more take it from ss.
 AF_EXPORT int af_rows_qkv(void* q, void* parts, const void* X, const void* W,
-                          const void* ss, int M, int Hq, int Hk, int K,
+                          const void* ss, int M, int Hq, int Hk, int D, int K,
                           int splits, float eps, const void* pos,
                           const void* table, void* kc, void* vc,
                           const void* slot, int page_size, void* stream) {
+  if (D != 128) return 9002;
+  if (Hq < 1 || Hk < 1 || page_size < 1) return 9003;
   RowsArgs a = {};
   a.out = (u16*)q;
   a.parts = (float*)parts;

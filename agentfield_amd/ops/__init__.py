@@ -382,19 +382,33 @@ def qkv_rope_rows(x: torch.Tensor, w: torch.Tensor, eps: float,
                   vcache: torch.Tensor, slots: torch.Tensor) -> torch.Tensor:
     """q [M, Hq*128] of up to 128 un-normalised rows: QKV projection (norm weight
     folded into w), RMSNorm scalar (from ss [M, 8] above 16 rows), rotary
-    positions, and k / v appended to their pages."""
+    positions, and k / v appended to their pages.  Heads of 128 only."""
+    if not _rows_ok(x, w):
+        raise AfOpsError(f"QKV rows: {tuple(x.shape)} {x.dtype} rows against "
+                         f"{tuple(w.shape)} {w.dtype} weights")
     M, K = x.shape
     _, Hk, page, D = kcache.shape
     N = w.shape[0]
     Hq = N // D - 2 * Hk
+    _need(Hq > 0 and N == (Hq + 2 * Hk) * D and table.shape[1] == D
+          and table.dtype == torch.float32 and table.is_contiguous(),
+          f"QKV rows: {N} outputs for {Hk} K/V heads of {D}")
+    _need(kcache.shape == vcache.shape and kcache.dtype == vcache.dtype == x.dtype
+          and kcache.is_contiguous() and vcache.is_contiguous(),
+          "QKV rows: pages must be whole and of x's type")
+    _need(positions.numel() == M and slots.numel() == M
+          and slots.dtype == torch.int64 and slots.is_contiguous(),
+          f"QKV rows: positions and int64 slots of {M} rows")
+    _need(M <= ROWS_MAX or _row_stats(ss, x), "QKV rows: sums of the rows")
     q = torch.empty(M, Hq * D, dtype=x.dtype, device=x.device)
+    pos = positions.int().contiguous()
     splits, parts = 1, None
     if M > ROWS_MAX:
         splits = rows_splits(M, N, K)
         parts = torch.empty(splits, M, N, dtype=torch.float32, device=x.device)
     rc = _lib.lib().af_rows_qkv(
         _lib.ptr(q), _lib.ptr(parts), _lib.ptr(x), _lib.ptr(w), _lib.ptr(ss), M,
-        Hq, Hk, K, splits, eps, _lib.ptr(positions.int()), _lib.ptr(table),
+        Hq, Hk, D, K, splits, eps, _lib.ptr(pos), _lib.ptr(table),
         _lib.ptr(kcache), _lib.ptr(vcache), _lib.ptr(slots), page,
         _lib.cur_stream())
     _lib.check(rc, "af_rows_qkv")

@@ -64,8 +64,8 @@ def _declare(l: ctypes.CDLL) -> None:
     l.af_gemm_skinny.argtypes = [p, p, p, p, p, i, i, i, i, i,
                                  p, f, p, p]
     l.af_rows_linear.argtypes = [p, p, p, p, p, p, i, i, i, i, i, i, p, f, p]
-    l.af_rows_qkv.argtypes = [p, p, p, p, p, i, i, i, i, i, f, p, p, p, p, p, i,
-                              p]
+    l.af_rows_qkv.argtypes = [p, p, p, p, p, i, i, i, i, i, i, f, p, p, p, p, p,
+                              i, p]
     l.af_moe_route.argtypes = [p, p, p, p, p, p, p, i, i, i, i, p]
     l.af_moe_combine.argtypes = [p, p, p, p, i, i, i, p]
     l.af_sample.argtypes = [p, p, p, p, p, p, u32, i, i, p]

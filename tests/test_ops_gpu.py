@@ -665,6 +665,36 @@ def test_qkv_rope_rows(M, Hq, Hk, K):
     assert close(kc, kw, **tol) and close(vc, vw, **tol)
 
 
+@pytest.mark.parametrize("M", [3, 40])
+def test_qkv_rope_rows_refuses_other_geometries(M):
+    """Head sizes other than 128, weights that are not whole heads, pages, stats
+    and slots of other shapes or types."""
+    Hq, Hk, K, page = 4, 2, 256, 16
+    x, w = rnd(M, K, seed=1), rnd((Hq + 2 * Hk) * 128, K, seed=2)
+    kc = torch.zeros(8, Hk, page, 128, dtype=torch.bfloat16, device=DEV)
+    good = dict(x=x, w=w, eps=1e-5, ss=torch.ones(M, 8, device=DEV),
+                positions=torch.arange(M, device=DEV, dtype=torch.int32),
+                table=ops.rope_table(64, 128, device=DEV), kcache=kc,
+                vcache=kc.clone(), slots=torch.arange(M, device=DEV))
+    small = torch.zeros(8, Hk, page, 64, dtype=torch.bfloat16, device=DEV)
+    bad = [dict(kcache=small, vcache=small, table=ops.rope_table(64, 64, device=DEV)),
+           dict(kcache=small, vcache=small), dict(w=w[:-64]), dict(w=w[:512]),
+           dict(w=w[:, :192].contiguous()), dict(x=x.float()),
+           dict(vcache=kc[:, :1].contiguous()), dict(kcache=kc.float()),
+           dict(kcache=kc.transpose(1, 2).contiguous().transpose(1, 2)),
+           dict(slots=torch.arange(M - 1, device=DEV)),
+           dict(slots=torch.arange(M, device=DEV, dtype=torch.int32)),
+           dict(positions=good["positions"][1:]),
+           dict(table=good["table"].double())]
+    if M > ops.ROWS_MAX:
+        bad += [dict(ss=None), dict(ss=good["ss"][1:])]
+    for kw in bad:
+        with pytest.raises(ops.AfOpsError):
+            ops.qkv_rope_rows(**{**good, **kw})
+    assert not kc.any() and not good["vcache"].any()
+    ops.qkv_rope_rows(**good)
+
+
 @pytest.mark.parametrize("page,G,Hk", [(4, 4, 2), (16, 1, 3), (24, 2, 2),
                                        (32, 8, 1), (64, 4, 2), (64, 1, 2)])
 @pytest.mark.parametrize("window", [0, 50])
