@@ -331,6 +331,12 @@ class LlamaLayer(nn.Module):
             h = self.mlp(h)
         return h, residual
 
+    def rows_weights(self) -> tuple:
+        """The weights that forward_rows_fused reads."""
+        at = self._modules["attn"]._parameters
+        mlp = self._modules["mlp"]._parameters
+        return at["qkv"], at["o"], mlp["gate_up"], mlp["down"]
+
     def forward_rows_fused(self, residual, ss, positions, rope_tab, kv, md):
         """Few-row path (decode steps, small prefill steps): norms, rotary
         positions, page append, SwiGLU and residual adds ride in the
@@ -416,13 +422,16 @@ class LlamaForCausalLM(nn.Module):
         if not getattr(self, "_norms_folded", False):
             return False
         cfg = self.cfg
-        return (not getattr(self, "no_fused_decode", False) and T <= 128
+        return (not getattr(self, "no_fused_decode", False) and 0 < T <= 128
                 and cfg.num_experts == 1  # MoE routes through the eager path
                 and cfg.head_dim == 128
                 and cfg.hidden_size % 64 == 0
                 and cfg.intermediate_size % 64 == 0
                 and (cfg.q_size + 2 * cfg.kv_size) % 64 == 0
-                and cfg.q_size % 64 == 0)
+                and cfg.q_size % 64 == 0
+                and self.embed.dtype == torch.bfloat16
+                and ops.rows_operands_ok(w for layer in self.layers
+                                        for w in layer.rows_weights()))
 
     def forward(self, ids, positions, kv: KVCache, md: AttnMetadata,
                 logit_rows: torch.Tensor | None = None):

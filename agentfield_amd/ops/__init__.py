@@ -285,6 +285,15 @@ def rows_splits(M: int, N: int, K: int) -> int:
     return -(-pieces // per)          # no empty split
 
 
+def rows_operands_ok(tensors) -> bool:
+    """Operands as the row GEMMs read them: bf16, whole, on 16-byte boundaries."""
+    bf16 = torch.bfloat16
+    for t in tensors:
+        if t.dtype is not bf16 or not t.is_contiguous() or t.data_ptr() & 15:
+            return False
+    return True
+
+
 def _rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """What the row GEMMs take: bf16 rows and weights of one length on one GPU,
     which lie whole and on 16-byte boundaries, whole 64 x 64 tiles of weights,
@@ -293,9 +302,7 @@ def _rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
         return False
     (M, K), (N, KW) = x.shape, w.shape
     return (K == KW and 0 < M <= 128 and K > 0 and N > 0 and N % 64 == 0
-            and K % 64 == 0 and x.is_contiguous() and w.is_contiguous()
-            and x.dtype == w.dtype == torch.bfloat16 and x.device == w.device
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+            and K % 64 == 0 and rows_operands_ok((x, w)) and x.device == w.device)
 
 
 def _need(ok: bool, what: str) -> None:
