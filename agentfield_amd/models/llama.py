@@ -284,12 +284,13 @@ class MoEMLP(nn.Module):
     def _can_sort(self, x) -> bool:
         """Rows that the routing kernels take (the loop serves the rest, and
         anything that autograd has to see)."""
-        return (x.is_cuda and x.dtype == self.router.dtype == torch.bfloat16
+        return (x.is_cuda and not ops.watched(x, self.router, self.gate_up,
+                                              self.down)
+                and x.dtype == self.router.dtype == torch.bfloat16
                 and x.is_contiguous() and x.shape[1] % 8 == 0
                 and x.data_ptr() % 16 == 0 and x.shape[0] > 0
                 and self.router.shape[0] <= ops.MOE_MAX_EXPERTS
-                and self.top_k <= ops.MOE_MAX_TOP
-                and not torch.is_grad_enabled())
+                and self.top_k <= ops.MOE_MAX_TOP)
 
     def _forward_sorted(self, x):
         weights, row, pos, offs = ops.moe_route(x, self.router, self.top_k)

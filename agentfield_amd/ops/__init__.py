@@ -12,6 +12,7 @@ import functools
 import math
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 from ._lib import AfOpsError, native_loaded
@@ -285,6 +286,21 @@ def rows_splits(M: int, N: int, K: int) -> int:
     return -(-pieces // per)          # no empty split
 
 
+def watched(*tensors: torch.Tensor, grad: bool = True) -> bool:
+    """Whether a product of these must be torch's own: autograd records it
+    (grad), or forward mode, a function transform, a tracer or a tensor subclass
+    has to see it.  Kernels called by address pass all of them by."""
+    grad = grad and torch.is_grad_enabled()
+    for t in tensors:
+        if (grad and t.requires_grad
+                or type(t) not in (torch.Tensor, torch.nn.Parameter)):
+            return True
+    return (forward_ad._current_level >= 0
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._len_torch_dispatch_stack() > 0
+            or torch.compiler.is_compiling())
+
+
 def rows_operands_ok(tensors) -> bool:
     """Operands as the row GEMMs read them: bf16, whole, on 16-byte boundaries."""
     bf16 = torch.bfloat16
@@ -485,9 +501,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
     if out is not None:
         _need(not silu_fuse and tuple(out.shape) == (M, N),
               f"linear: out {tuple(out.shape)} for a [{M}, {N}] product")
-    if (out is None or _whole(out, x, M, N)) and _rows_ok(x, w) and (
-            silu_fuse or M <= 32 or N <= 12288 or N >= 24576) and not (
-            torch.is_grad_enabled() and x.requires_grad):
+    if (x.is_cuda and not watched(x, w, grad=not silu_fuse)
+            and (out is None or _whole(out, x, M, N)) and _rows_ok(x, w)
+            and (silu_fuse or M <= 32 or N <= 12288 or N >= 24576)):
         return linear_rows(x, w, mode=2 if silu_fuse else 0, out=out)
     if out is not None:
         return torch.mm(x, w.t(), out=out)

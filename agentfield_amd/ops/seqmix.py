@@ -685,9 +685,9 @@ def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
     M, K = x.shape
     N = w.shape[0]
     if skinny and x.is_cuda and M <= 128 and _lib.main_lib_ready():
-        from . import _rows_ok, linear_rows, linear_skinny
-        if ((M <= 32 or M <= 64 and N <= 4096 or N >= 24576) and _rows_ok(x, w)
-                and not (torch.is_grad_enabled() and x.requires_grad)):
+        from . import _rows_ok, linear_rows, linear_skinny, watched
+        if ((M <= 32 or M <= 64 and N <= 4096 or N >= 24576)
+                and not watched(x, w) and _rows_ok(x, w)):
             return linear_rows(x, w)
         if (_SKINNY and x.dtype == torch.bfloat16
                 and N % 64 == 0 and K % 64 == 0

@@ -635,6 +635,60 @@ def test_linear_rows_refuses_other_buffers(M):
                  x.float() @ w.float().t() + before.float(), atol=0.2)
 
 
+@pytest.mark.parametrize("M", [4, 64])
+@pytest.mark.parametrize("N", [512, 16384, 32768])
+def test_row_products_under_autograd(M, N):
+    """Products that autograd, forward mode or vmap have to see are torch's own,
+    whichever operand asks for it.  Gradients in bf16 against fp32: two roundings
+    of sums over N or M terms (2^-7 of their rms times 4)."""
+    from torch.autograd import forward_ad
+    from agentfield_amd.ops import seqmix as sm
+    K = 256
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=0.1)
+    gy = rnd(M, N, seed=3)
+
+    def near(a, b):
+        return (a.float() - b).norm() <= 2 ** -7 * b.norm()
+    for call in (ops.linear, sm.matmul):
+        wp = torch.nn.Parameter(w)
+        y = call(x, wp)
+        y.backward(gy)
+        assert near(wp.grad, gy.float().t() @ x.float())
+        xr = x.clone().requires_grad_()
+        call(xr, w).backward(gy)
+        assert near(xr.grad, gy.float() @ w.float())
+        with torch.no_grad():
+            assert not call(x, wp).requires_grad
+        with forward_ad.dual_level():
+            t = forward_ad.unpack_dual(call(forward_ad.make_dual(x, x), w)).tangent
+        assert near(t, x.float() @ w.float().t())
+        v = torch.func.vmap(lambda a: call(a, w))(torch.stack([x, 2 * x]))
+        assert near(v[1], 2 * (x.float() @ w.float().t()))
+
+
+@pytest.mark.parametrize("T", [3, 100])
+def test_moe_dispatch_under_autograd(T):
+    """The mixture layer's exact dispatch leaves weight gradients where its loop
+    over the experts does, and routes alike either way."""
+    from dataclasses import replace
+    from agentfield_amd.models import CONFIGS
+    from agentfield_amd.models.llama import MoEMLP
+    mlp = MoEMLP(replace(CONFIGS["tiny-moe"])).to(DEV, torch.bfloat16)
+    for i, p in enumerate(mlp.parameters()):
+        p.data.copy_(rnd(*p.shape, seed=20 + i, scale=0.05))
+    x = rnd(T, 256, seed=4)
+    with torch.no_grad():
+        quiet = mlp(x)
+    out = mlp(x)
+    assert out.requires_grad and not quiet.requires_grad
+    assert close(out, quiet)
+    out.float().sum().backward()
+    assert mlp.down.grad is not None and mlp.router.grad is not None
+    for p in mlp.parameters():
+        p.requires_grad_(False)
+    assert torch.equal(mlp(x), quiet)      # grad mode alone changes nothing
+
+
 @pytest.mark.parametrize("M", ROW_COUNTS)
 @pytest.mark.parametrize("Hq,Hk,K", [(2, 1, 256), (8, 8, 192), (32, 8, 1024)])
 def test_qkv_rope_rows(M, Hq, Hk, K):

@@ -74,3 +74,39 @@ def test_few_row_path_needs_plain_bf16_weights():
         assert not m._can_fuse_rows(4)
         p.data = flat
         assert m._can_fuse_rows(4)
+
+
+def test_watched_products():
+    """Autograd, forward mode, transforms and tracers see a product; grad mode
+    alone, with nothing that requires a gradient, does not keep it from the
+    kernels."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.autograd import forward_ad
+    x, w = torch.randn(4, 8), torch.randn(6, 8)
+    p = torch.nn.Parameter(w)
+    seen = []
+    assert not ops.watched(x, w)
+    assert ops.watched(x, p) and ops.watched(x.clone().requires_grad_(), w)
+    assert not ops.watched(x, p, grad=False)
+    with torch.no_grad():
+        assert not ops.watched(x, p)
+    with torch.inference_mode():
+        assert not ops.watched(x, p)
+
+    def look(a):
+        seen.append(ops.watched(a, w))
+        return a * 2
+    torch.func.vmap(look)(torch.stack([x, x]))
+    torch.func.grad(lambda a: look(a).sum())(x)
+    torch.func.jvp(look, (x,), (x,))
+    with forward_ad.dual_level(), torch.no_grad():
+        look(forward_ad.make_dual(x, x))
+    with FakeTensorMode() as m:
+        look(m.from_tensor(x))
+    torch.fx.experimental.proxy_tensor.make_fx(look)(x)
+
+    class Sub(torch.Tensor):
+        pass
+    look(x.as_subclass(Sub))
+    assert seen == [True] * 7
+    assert not ops.watched(x, w)
