@@ -70,7 +70,8 @@ struct PrefillArgs {
   const i32* bt;
   const i32* qstart;
   const i32* cu;
-  float scale;
+  float scale;      // positive
+  float qmul;       // factor of q: the sign of the caller's scale, or a zero
   int nseq, Hq, Hk;
   i64 qs;
   int page_size, page_shift, max_pages, win;
@@ -204,7 +205,8 @@ __device__ __forceinline__ void attend(Columns& c, const lds_char* kl,
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int t = t0 + b * 32 + 8 * (r / 4) + 4 * h + (r % 4);
-        if (t > c.qpos || (win > 0 && t <= c.qpos - win)) s[b][r] = AF_NEG_INF;
+        if (t > c.qpos || (win > 0 && t <= c.qpos - win))
+          s[b][r] = -__builtin_inff();  // weight 0 under any positive scale
       }
   }
   float mx = AF_NEG_INF;
@@ -278,6 +280,13 @@ __device__ __forceinline__ void load_columns(const PrefillArgs& a, Columns& c,
                   head * AP_D + h * 8;
 #pragma unroll
   for (int d = 0; d < 8; ++d) c.q[d] = *reinterpret_cast<const s16x8*>(qp + d * 16);
+  if (a.qmul != 1.f) {
+#pragma unroll
+    for (int d = 0; d < 8; ++d)
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        c.q[d][j] = (short)f2bf(bf2f((u16)c.q[d][j]) * a.qmul);
+  }
 #pragma unroll
   for (int d = 0; d < 4; ++d)
 #pragma unroll
@@ -506,6 +515,9 @@ __global__ void __launch_bounds__(256) attn_prefill_merge_kernel(
   }
 }
 
+// The kernels take the maximum of raw scores and mask before they scale, so scale
+// must be positive there: a negative one changes the sign of q (exact), zero makes
+// all scores zero.
 // items: 128-column items of the sequences with more than few_cols columns; few:
 // 32-column items of the others, their keys cut nsplit ways with the partial
 // results in po / pml (all per K/V head).
@@ -523,7 +535,10 @@ AF_EXPORT int af_attn_prefill(void* out, void* po, void* pml, const void* q,
   const bool pow2 = (page_size & (page_size - 1)) == 0;
   const PrefillArgs a = {(u16*)out, (const u16*)q, (const u16*)kc, (const u16*)vc,
                          (const i32*)bt, (const i32*)qstart,
-                         (const i32*)cu_seqlens, scale, nseq, Hq, Hk, qs,
+                         (const i32*)cu_seqlens,
+                         scale > 0.f ? scale : scale < 0.f ? -scale : 1.f,
+                         scale > 0.f ? 1.f : scale < 0.f ? -1.f : scale,
+                         nseq, Hq, Hk, qs,
                          page_size, pow2 ? __builtin_ctz(page_size) : -1,
                          max_pages, win, few_cols};
   float* fo = (float*)po;

@@ -786,6 +786,45 @@ def test_attn_prefill_tile_edges(page, G, Hk, window):
     assert close(got, want, atol=2 ** -6, rtol=2 ** -7)
 
 
+def _cut(monkeypatch, few_cols, nsplit):
+    """Cut prompt attention like this, whatever the rule would choose; returns
+    the (128-column items, 32-column items, key splits) of the calls."""
+    made = []
+
+    def cut(seq_lens, G, Hk, max_keys):
+        cols = [n * G for n in seq_lens if n > 0]
+        items = sum(-(-c // 128) for c in cols if c > few_cols)
+        few = sum(-(-c // 32) for c in cols if c <= few_cols)
+        made.append((items, few, nsplit if few else 1))
+        return few_cols, items, few, nsplit if few else 1
+    monkeypatch.setattr(ops, "prefill_split", cut)
+    return made
+
+
+@pytest.mark.parametrize("few_cols,nsplit", [(0, 1), (1 << 30, 1), (1 << 30, 3)])
+@pytest.mark.parametrize("scale", [-0.1, 0.0, 1e-20, 0.1])
+@pytest.mark.parametrize("window", [0, 50])
+def test_attn_prefill_any_scale(monkeypatch, few_cols, nsplit, scale, window):
+    """Negative, zero and tiny scales, in both kernels: masked keys have no
+    weight whatever the factor of the scores.  Tolerance: P and the output are
+    rounded to bf16 (2^-9 of values below 4, twice)."""
+    _cut(monkeypatch, few_cols, nsplit)
+    D, page, G, Hk, lens, hist = 128, 64, 4, 2, [5, 64, 130], [0, 70, 33]
+    torch.manual_seed(5)
+    B, maxp = len(lens), 4
+    bt = (torch.randperm(B * maxp) + 1).view(B, maxp).to(torch.int32)
+    kc = torch.randn(B * maxp + 1, Hk, page, D).bfloat16()
+    vc = torch.randn(B * maxp + 1, Hk, page, D).bfloat16()
+    q = torch.randn(sum(lens), Hk * G * D).bfloat16()
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    qs = torch.tensor(hist, dtype=torch.int32)
+    got = ops.attn_prefill(q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV),
+                           qs.to(DEV), cu.to(DEV), lens, scale, window=window)
+    want = ref.attn_prefill_paged(q.unflatten(-1, (Hk * G, D)), kc, vc, bt, qs,
+                                  cu, scale, window=window).flatten(1)
+    assert close(got, want, atol=2 ** -6, rtol=2 ** -7)
+
+
 @pytest.mark.parametrize("T,E,k", [(1, 4, 1), (5, 8, 2), (64, 3, 3), (65, 16, 2),
                                    (700, 8, 2), (333, 64, 8), (1500, 33, 5)])
 def test_moe_sorted_dispatch(T, E, k):
