@@ -531,9 +531,10 @@ __global__ void __launch_bounds__(256) diff_combine_kernel(
 // the state in registers (each q / k / decay value read from LDS feeds two
 // columns).  Tokens are walked serially in blocks of TB: the block's q / k / decay
 // rows are staged into LDS at once (rotary + scaling applied on the way in), the
-// recurrence itself is strictly token by token in fp32, and both kernels sum the
-// 16 row groups in the same order — so results do not depend on how a sequence
-// is cut into chunks.
+// recurrence itself is strictly token by token in fp32, and both kernels use the
+// same operations (scan_*) and sum the 16 row groups in the same order — so they
+// give the same bits, and results do not depend on how a sequence is cut into
+// chunks or on what else is in the step.
 //
 // linear_scan_kernel, few tokens per sequence: bound by moving the state; thread
 // (r, c) = (tid >> 4, tid & 15) has columns c and c + 16, so that a state row
@@ -556,6 +557,46 @@ __device__ __forceinline__ float row16_sum_all(float v) {
   AFM_ROR(1)
 #undef AFM_ROR
   return v;
+}
+
+// The arithmetic of both kernels, every rounding spelled out: contraction is the
+// compiler's choice per place otherwise, and a sequence's results must not depend
+// on which kernel its neighbours in the step selected.
+__device__ __forceinline__ void scan_rotate(float& x, float partner, float cs,
+                                            float sn, bool low) {
+#pragma clang fp contract(off)
+  // pair (u, w) -> (u cos - w sin, w cos + u sin)
+  x = fmaf(x, cs, partner * (low ? -sn : sn));
+}
+
+template <bool FAST>
+__device__ __forceinline__ void scan_angle(float pos, float freq, float& sn,
+                                           float& cs) {
+#pragma clang fp contract(off)
+  const float ang = pos * freq;
+  if (FAST) { sn = __sinf(ang); cs = __cosf(ang); }
+  else sincosf(ang, &sn, &cs);
+}
+
+// sigmoid(z)^inv_tau; log(sigmoid(z)) = min(z, 0) - log(1 + exp(-|z|)) does not
+// overflow
+template <bool FAST>
+__device__ __forceinline__ float scan_decay(float z, float inv_tau) {
+#pragma clang fp contract(off)
+  if (FAST) {
+    const float l = __logf(1.0f + __expf(-fabsf(z)));
+    return __expf((fminf(z, 0.f) - l) * inv_tau);
+  }
+  const float l = log1pf(expf(-fabsf(z)));
+  return expf((fminf(z, 0.f) - l) * inv_tau);
+}
+
+// one row of one column, one token: the state, then its share of the output
+__device__ __forceinline__ void scan_row(float& st, float& o, float a, float k,
+                                         float v, float q) {
+#pragma clang fp contract(off)
+  st = fmaf(a, st, k * v);
+  o = fmaf(st, q, o);
 }
 
 template <typename S, int RP>
@@ -659,27 +700,15 @@ __global__ void __launch_bounds__(256) linear_scan_kernel(
         if (i < rot) {
           const bool lowh = i < half;
           float sn, cs;
-          const float ang = rpos[n] * inv_freq[lowh ? i : i - half];
-          if (FAST) { sn = __sinf(ang); cs = __cosf(ang); }
-          else sincosf(ang, &sn, &cs);
-          // pair (u, w) -> (u cos - w sin, w cos + u sin)
-          qv = lowh ? qv * cs - rqp[n] * sn : qv * cs + rqp[n] * sn;
-          kv = lowh ? kv * cs - rkp[n] * sn : kv * cs + rkp[n] * sn;
+          scan_angle<FAST>(rpos[n], inv_freq[lowh ? i : i - half], sn, cs);
+          scan_rotate(qv, rqp[n], cs, sn, lowh);
+          scan_rotate(kv, rkp[n], cs, sn, lowh);
         }
         qv *= q_scale;
         kv *= k_scale;
         a = hd;
         if (zl) {
-          const float z = rz[n] + zbias[(size_t)h * dk + i];
-          // log(sigmoid(z)) = -softplus(-z), evaluated without overflow
-          if (FAST) {
-            const float ls = z >= 0.f ? -__logf(1.0f + __expf(-z))
-                                      : z - __logf(1.0f + __expf(z));
-            a = __expf(ls * inv_tau);
-          } else {
-            const float ls = z >= 0.f ? -log1pf(expf(-z)) : z - log1pf(expf(z));
-            a = expf(ls * inv_tau);
-          }
+          a = scan_decay<FAST>(rz[n] + zbias[(size_t)h * dk + i], inv_tau);
         }
       }
       if (tt < SCAN_TB) {
@@ -709,10 +738,8 @@ __global__ void __launch_bounds__(256) linear_scan_kernel(
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           const int ii = i2 * 2 + j;
-          sta[ii] = a2[j] * sta[ii] + k2[j] * va;
-          stb[ii] = a2[j] * stb[ii] + k2[j] * vb;
-          pa += sta[ii] * q2[j];
-          pb += stb[ii] * q2[j];
+          scan_row(sta[ii], pa, a2[j], k2[j], va, q2[j]);
+          scan_row(stb[ii], pb, a2[j], k2[j], vb, q2[j]);
         }
       }
       part[tt * 512 + r * 32 + cc] = pa;
@@ -845,29 +872,19 @@ __global__ void __launch_bounds__(256, 2) linear_scan_prompt_kernel(
     if (rot > 0) {
 #pragma unroll
       for (int j = 0; j < E; ++j) {
-        const float ang = (float)rpos * frq[j];  // 0 where nothing is rotated
-        float sn, cs;
-        if (FAST) { sn = __sinf(ang); cs = __cosf(ang); }
-        else sincosf(ang, &sn, &cs);
-        // pair (u, w) -> (u cos - w sin, w cos + u sin)
-        sn = lowh ? -sn : sn;
-        const float x = qv[j] * cs + ldf<S>(&rqp.x[j]) * sn;
-        const float y = kv[j] * cs + ldf<S>(&rkp.x[j]) * sn;
+        float sn, cs;                     // angle 0 where nothing is rotated
+        scan_angle<FAST>((float)rpos, frq[j], sn, cs);
+        float x = qv[j], y = kv[j];
+        scan_rotate(x, ldf<S>(&rqp.x[j]), cs, sn, lowh);
+        scan_rotate(y, ldf<S>(&rkp.x[j]), cs, sn, lowh);
         qv[j] = turn ? x : qv[j];
         kv[j] = turn ? y : kv[j];
       }
     }
     if (zl) {
 #pragma unroll
-      for (int j = 0; j < E; ++j) {
-        const float z = ldf<S>(&rz.x[j]) + bias[j];
-        // log(sigmoid(z)) = min(z, 0) - log(1 + exp(-|z|)), without overflow
-        if (FAST)
-          av[j] = __expf((fminf(z, 0.f) - __logf(1.0f + __expf(-fabsf(z)))) *
-                         inv_tau);
-        else
-          av[j] = expf((fminf(z, 0.f) - log1pf(expf(-fabsf(z)))) * inv_tau);
-      }
+      for (int j = 0; j < E; ++j)
+        av[j] = scan_decay<FAST>(ldf<S>(&rz.x[j]) + bias[j], inv_tau);
     }
 #pragma unroll
     for (int j = 0; j < E; ++j) {
@@ -948,10 +965,8 @@ __global__ void __launch_bounds__(256, 2) linear_scan_prompt_kernel(
       float pa = 0.f, pb = 0.f;
 #pragma unroll
       for (int ii = 0; ii < RP; ++ii) {
-        sta[ii] = t.a[ii] * sta[ii] + t.k[ii] * t.v[0];
-        stb[ii] = t.a[ii] * stb[ii] + t.k[ii] * t.v[1];
-        pa += sta[ii] * t.q[ii];
-        pb += stb[ii] * t.q[ii];
+        scan_row(sta[ii], pa, t.a[ii], t.k[ii], t.v[0], t.q[ii]);
+        scan_row(stb[ii], pb, t.a[ii], t.k[ii], t.v[1], t.q[ii]);
       }
       pa = row16_sum_all(pa);
       pb = row16_sum_all(pb);

@@ -674,10 +674,9 @@ def test_registry_loads_checkpoint_and_trace_cli(tmp_path):
 def test_scan_prompt_and_token_kernels_agree(dtype, dk, dv, rot, pad, gated):
     """The prompt kernel (whole prompts of lengths around its token blocks) and
     the token kernel (the same prompts in portions of one and of nine tokens)
-    give the same outputs and states; padded dims, column tiles, halves that are
-    not a multiple of the wide loads, rows that are not aligned for them.  Both
-    sum in the same order, so only multiply-add contraction may differ: a few
-    fp32 roundings of the largest term."""
+    give the same bits, outputs and states; padded dims, column tiles, halves
+    that are not a multiple of the wide loads, rows that are not aligned for
+    them (those stay with the token kernel in all portions)."""
     from agentfield_amd.ops import seqmix as sm
     from types import SimpleNamespace
     H, lens = 2, [1, 16, 17, 33, 100]
@@ -729,5 +728,4 @@ def test_scan_prompt_and_token_kernels_agree(dtype, dk, dv, rot, pad, gated):
     assert torch.isfinite(whole).all() and torch.isfinite(S).all()
     for portion in (1, 9):
         o, s = run(portion)
-        assert (o - whole).abs().max() <= 4e-6 * whole.abs().max()
-        assert (s - S).abs().max() <= 4e-6 * S.abs().max()
+        assert torch.equal(o, whole) and torch.equal(s, S)
