@@ -286,11 +286,7 @@ class MoEMLP(nn.Module):
         anything that autograd has to see)."""
         return (x.is_cuda and not ops.watched(x, self.router, self.gate_up,
                                               self.down)
-                and x.dtype == self.router.dtype == torch.bfloat16
-                and x.is_contiguous() and x.shape[1] % 8 == 0
-                and x.data_ptr() % 16 == 0 and x.shape[0] > 0
-                and self.router.shape[0] <= ops.MOE_MAX_EXPERTS
-                and self.top_k <= ops.MOE_MAX_TOP)
+                and ops.moe_route_ok(x, self.router, self.top_k))
 
     def _forward_sorted(self, x):
         weights, row, pos, offs = ops.moe_route(x, self.router, self.top_k)

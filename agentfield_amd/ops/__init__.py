@@ -517,11 +517,24 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
 MOE_MAX_EXPERTS, MOE_MAX_TOP = 64, 8     # limits of the routing kernels
 
 
+def moe_route_ok(x: torch.Tensor, router: torch.Tensor, k: int) -> bool:
+    """What the routing kernels take: bf16 rows and router rows of one length on
+    one GPU, read 16 bytes at a time, and k of at most MOE_MAX_EXPERTS experts."""
+    if not x.is_cuda or x.dim() != 2 or router.dim() != 2:
+        return False
+    (T, H), (E, HR) = x.shape, router.shape
+    return (H == HR and T > 0 and H % 8 == 0 and 1 <= E <= MOE_MAX_EXPERTS
+            and 1 <= k <= min(E, MOE_MAX_TOP) and x.device == router.device
+            and rows_operands_ok((x, router)))
+
+
 def moe_route(x: torch.Tensor, router: torch.Tensor, k: int):
     """Softmax routing of rows x [T, H] over the experts' router [E, H], the k
     largest renormalised, and the (row, choice) entries sorted by expert:
     (weights [T, k] f32, row [T*k] i32 of every sorted position, sorted position
     [T*k] i32 of every entry, first position of every expert [E+1] i32)."""
+    _need(moe_route_ok(x, router, k),
+          f"routing {tuple(x.shape)} rows over {tuple(router.shape)}, k {k}")
     T, H = x.shape
     E = router.shape[0]
     dev = x.device
@@ -542,6 +555,12 @@ def moe_combine(y: torch.Tensor, pos: torch.Tensor,
     """out[t] = sum_j weights[t, j] * y[pos[t*k + j]] over the sorted expert rows."""
     T, k = weights.shape
     H = y.shape[1]
+    _need(y.is_cuda and y.shape[0] == T * k and H % 8 == 0
+          and rows_operands_ok((y,)) and weights.dtype == torch.float32
+          and weights.is_contiguous() and weights.device == y.device
+          and pos.numel() == T * k and pos.dtype == torch.int32
+          and pos.is_contiguous() and pos.device == y.device,
+          f"combining {tuple(y.shape)} rows by {tuple(weights.shape)} weights")
     out = torch.empty(T, H, dtype=y.dtype, device=y.device)
     rc = _lib.lib().af_moe_combine(
         _lib.ptr(out), _lib.ptr(y), _lib.ptr(pos), _lib.ptr(weights), T, H, k,

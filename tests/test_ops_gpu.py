@@ -851,3 +851,19 @@ def test_moe_sorted_dispatch(T, E, k):
     got = ops.moe_combine(y, pos, w)
     ref_ = (y.float()[pos.long()].view(T, k, H) * w[..., None]).sum(1)
     assert close(got, ref_, atol=2e-2, rtol=2 ** -7)
+
+
+def test_moe_kernels_refuse_other_operands():
+    x, router = rnd(5, 520, seed=1), rnd(8, 520, seed=2)
+    for a, r, k in ((x, rnd(8, 512), 2), (x[:, :512].contiguous(), router, 2),
+                    (x, router.float(), 2), (x, router, 9), (x.float(), router, 2),
+                    (x[:, :512], router[:, :512].contiguous(), 2)):
+        with pytest.raises(ops.AfOpsError):
+            ops.moe_route(a, r, k)
+    w, row, pos, offs = ops.moe_route(x, router, 2)
+    y = rnd(10, 520, seed=3)
+    for args in ((y[:9], pos, w), (y, pos[1:], w), (y, pos.long(), w),
+                 (y, pos, w.double()), (y.float(), pos, w)):
+        with pytest.raises(ops.AfOpsError):
+            ops.moe_combine(*args)
+    ops.moe_combine(y, pos, w)
