@@ -282,10 +282,13 @@ __device__ __forceinline__ void load_columns(const PrefillArgs& a, Columns& c,
   for (int d = 0; d < 8; ++d) c.q[d] = *reinterpret_cast<const s16x8*>(qp + d * 16);
   if (a.qmul != 1.f) {
 #pragma unroll
-    for (int d = 0; d < 8; ++d)
+    for (int d = 0; d < 8; ++d) {
+      union { s16x8 s; bf16x8 b; } u;
+      u.s = c.q[d];
 #pragma unroll
-      for (int j = 0; j < 8; ++j)
-        c.q[d][j] = (short)f2bf(bf2f((u16)c.q[d][j]) * a.qmul);
+      for (int j = 0; j < 8; ++j) u.b[j] = (__bf16)((float)u.b[j] * a.qmul);
+      c.q[d] = u.s;
+    }
   }
 #pragma unroll
   for (int d = 0; d < 4; ++d)

@@ -314,11 +314,11 @@ def _rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """What the row GEMMs take: bf16 rows and weights of one length on one GPU,
     which lie whole and on 16-byte boundaries, whole 64 x 64 tiles of weights,
     1..128 rows.  The kernels read w by the length of x's rows."""
-    if not x.is_cuda or x.dim() != 2 or w.dim() != 2:
-        return False
-    (M, K), (N, KW) = x.shape, w.shape
-    return (K == KW and 0 < M <= 128 and K > 0 and N > 0 and N % 64 == 0
-            and K % 64 == 0 and rows_operands_ok((x, w)) and x.device == w.device)
+    xs, ws = x.shape, w.shape
+    return (x.is_cuda and len(xs) == 2 == len(ws) and xs[1] == ws[1]
+            and 0 < xs[0] <= 128 and ws[0] > 0 and ws[0] % 64 == 0
+            and ws[1] > 0 and ws[1] % 64 == 0 and x.device == w.device
+            and rows_operands_ok((x, w)))
 
 
 def _need(ok: bool, what: str) -> None:
@@ -328,9 +328,9 @@ def _need(ok: bool, what: str) -> None:
 
 def _whole(t: torch.Tensor | None, x: torch.Tensor, *shape: int) -> bool:
     """t can be written as x's kind of rows of that shape, two at a time."""
-    return (t is not None and tuple(t.shape) == shape and t.dtype == x.dtype
-            and t.device == x.device and t.is_contiguous()
-            and t.data_ptr() % 4 == 0)
+    return (t is not None and t.shape == shape and t.dtype is x.dtype
+            and t.is_contiguous() and t.data_ptr() & 3 == 0
+            and t.device == x.device)
 
 
 def _row_stats(ss: torch.Tensor | None, x: torch.Tensor) -> bool:
@@ -342,8 +342,7 @@ def _row_stats(ss: torch.Tensor | None, x: torch.Tensor) -> bool:
 
 def _apart(a: torch.Tensor, b: torch.Tensor) -> bool:
     pa, pb = a.data_ptr(), b.data_ptr()
-    return (pa + a.numel() * a.element_size() <= pb
-            or pb + b.numel() * b.element_size() <= pa)
+    return pa + a.nbytes <= pb if pa < pb else pb + b.nbytes <= pa
 
 
 def linear_rows(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
