@@ -1,6 +1,7 @@
-"""Which products the row GEMMs take.  The rule is about sizes, types and
-addresses, so it is checked here on stand-ins, without a GPU: whatever it takes
-is read by kernels that know only x's sizes and the number of weight rows."""
+"""Which calls the row GEMMs, the routing kernels and the prompt attention kernels
+take.  The rules are about sizes, types and addresses, so they are checked here
+on stand-ins, without a GPU: whatever the row GEMMs take, for instance, is read by
+kernels that know only x's sizes and the number of weight rows."""
 from types import SimpleNamespace
 
 import pytest
@@ -136,3 +137,28 @@ def test_rows_that_the_routing_kernels_take(monkeypatch, ok, x, router, k):
     monkeypatch.setattr(ops, "watched", lambda *t, **kw: False)
     layer = SimpleNamespace(router=router, gate_up=None, down=None, top_k=k)
     assert MoEMLP._can_sort(layer, x) == ok
+
+
+@pytest.mark.parametrize("lens,want", [
+    ([8000], (32, 250, 0, 1)),                     # one long prompt
+    ([700, 3, 8, 500, 9], (32, 39, 2, 4)),         # both kinds of items
+    ([60] * 4, (1 << 30, 0, 32, 1)),               # few 128-column blocks
+    ([5] * 16, (1 << 30, 0, 16, 2)),               # drafts: keys split
+    ([5], (1 << 30, 0, 1, 8)),
+    ([300, 0, 400], (32, 23, 0, 1)),
+    ([], (1 << 30, 0, 0, 1)),
+])
+def test_prefill_split_reaches_every_kernel(lens, want):
+    """The rule by which prompt attention is cut (8 K/V heads, four query heads
+    each, pages for 8192 tokens): a change of it shows which kernels a step
+    still reaches."""
+    assert ops.prefill_split(lens, 4, 8, 8192) == want
+
+
+@pytest.mark.parametrize("K", [64, 128, 832, 4096, 14336, 65536])
+@pytest.mark.parametrize("N", [64, 192, 4096, 6144, 24576, 128256])
+def test_rows_splits_leave_no_split_empty(N, K):
+    for M in (1, 16, 17, 32, 33, 64, 65, 128):
+        n, pieces = ops.rows_splits(M, N, K), K // 64
+        assert 1 <= n <= min(16, pieces)
+        assert (n - 1) * -(-pieces // n) < pieces

@@ -749,15 +749,36 @@ def test_qkv_rope_rows_refuses_other_geometries(M):
     ops.qkv_rope_rows(**good)
 
 
+def _cut(monkeypatch, few_cols, nsplit):
+    """Cut prompt attention like this, whatever the rule would choose; returns
+    the (128-column items, 32-column items, key splits) of the calls."""
+    made = []
+
+    def cut(seq_lens, G, Hk, max_keys):
+        cols = [n * G for n in seq_lens if n > 0]
+        items = sum(-(-c // 128) for c in cols if c > few_cols)
+        few = sum(-(-c // 32) for c in cols if c <= few_cols)
+        made.append((items, few, nsplit if few else 1))
+        return few_cols, items, few, nsplit if few else 1
+    monkeypatch.setattr(ops, "prefill_split", cut)
+    return made
+
+
 @pytest.mark.parametrize("page,G,Hk", [(4, 4, 2), (16, 1, 3), (24, 2, 2),
                                        (32, 8, 1), (64, 4, 2), (64, 1, 2)])
 @pytest.mark.parametrize("window", [0, 50])
-def test_attn_prefill_tile_edges(page, G, Hk, window):
+@pytest.mark.parametrize("few_cols,nsplit", [
+    (0, 1), (32, 1), (32, 3), (1 << 30, 1), (1 << 30, 3), (1 << 30, 8)])
+def test_attn_prefill_tile_edges(monkeypatch, page, G, Hk, window, few_cols,
+                                 nsplit):
     """Chunk lengths around one wave's 32 columns and a block's 128, histories
-    around 32- and 64-token tiles, both kernels in one call, an empty chunk;
-    values of positions that do not exist yet are NaN, so that reading them
-    with weight 0 would show.  Tolerance: P and the output are rounded to bf16
-    (2^-9 of values below 4, twice)."""
+    around 32- and 64-token tiles, an empty chunk; cut into 128-column items
+    only, into both kinds of items in one call, and into 32-column items only,
+    whole and with the keys split (also into splits without a tile, merged by
+    the second kernel).  Values of positions that do not exist yet are NaN, so
+    that reading them with weight 0 would show.  Tolerance: P and the output
+    are rounded to bf16 (2^-9 of values below 4, twice)."""
+    made = _cut(monkeypatch, few_cols, nsplit)
     D = 128
     lens = [1, 32 // G, 32 // G + 1, 0, 5, 64, 65, 130, 3, 200, 1]
     hist = [0, 31, 0, 7, 64, 0, 63, 65, 300, 100, 129]
@@ -779,26 +800,14 @@ def test_attn_prefill_tile_edges(page, G, Hk, window):
     got = ops.attn_prefill(q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV),
                            qs.to(DEV), cu.to(DEV), lens, scale,
                            window=window).cpu()
+    (items, few, splits), = made
+    assert (items > 0) == (few_cols < 1 << 30) and (few > 0) == (few_cols > 0)
+    assert splits == nsplit
     want = ref.attn_prefill_paged(q.unflatten(-1, (Hk * G, D)), kc,
                                   torch.nan_to_num(vc), bt, qs, cu, scale,
                                   window=window).flatten(1)
     assert torch.isfinite(got.float()).all()
     assert close(got, want, atol=2 ** -6, rtol=2 ** -7)
-
-
-def _cut(monkeypatch, few_cols, nsplit):
-    """Cut prompt attention like this, whatever the rule would choose; returns
-    the (128-column items, 32-column items, key splits) of the calls."""
-    made = []
-
-    def cut(seq_lens, G, Hk, max_keys):
-        cols = [n * G for n in seq_lens if n > 0]
-        items = sum(-(-c // 128) for c in cols if c > few_cols)
-        few = sum(-(-c // 32) for c in cols if c <= few_cols)
-        made.append((items, few, nsplit if few else 1))
-        return few_cols, items, few, nsplit if few else 1
-    monkeypatch.setattr(ops, "prefill_split", cut)
-    return made
 
 
 @pytest.mark.parametrize("few_cols,nsplit", [(0, 1), (1 << 30, 1), (1 << 30, 3)])
@@ -823,6 +832,31 @@ def test_attn_prefill_any_scale(monkeypatch, few_cols, nsplit, scale, window):
     want = ref.attn_prefill_paged(q.unflatten(-1, (Hk * G, D)), kc, vc, bt, qs,
                                   cu, scale, window=window).flatten(1)
     assert close(got, want, atol=2 ** -6, rtol=2 ** -7)
+
+
+@pytest.mark.parametrize("G", [1, 2, 4, 8])
+def test_attn_prefill_as_dispatched(G):
+    """A step that the rule itself sends to both kernels, keys split or not."""
+    D, page, Hk = 128, 64, 8
+    torch.manual_seed(13)
+    for lens, hist in (([900, 2, 700, 1], [0, 90, 300, 1000]),
+                       ([3, 5, 2], [1500, 70, 400])):
+        _fc, items, few, nsplit = ops.prefill_split(lens, G, Hk, 2048)
+        long = max(lens) > 100
+        assert (items > 0) == (long and G > 1) and few > 0
+        assert nsplit == (8 if not long else 4 if G > 1 else 1)
+        B, maxp = len(lens), 2048 // page
+        bt = (torch.randperm(B * maxp) + 1).view(B, maxp).to(torch.int32)
+        kc = torch.randn(B * maxp + 1, Hk, page, D, dtype=torch.bfloat16)
+        vc = torch.randn(B * maxp + 1, Hk, page, D, dtype=torch.bfloat16)
+        q = torch.randn(sum(lens), Hk * G * D, dtype=torch.bfloat16)
+        cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+        qs = torch.tensor(hist, dtype=torch.int32)
+        got = ops.attn_prefill(q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV),
+                               qs.to(DEV), cu.to(DEV), lens)
+        want = ref.attn_prefill_paged(q.unflatten(-1, (Hk * G, D)), kc, vc, bt,
+                                      qs, cu, 1.0 / math.sqrt(D)).flatten(1)
+        assert close(got, want, atol=2 ** -6, rtol=2 ** -7)
 
 
 @pytest.mark.parametrize("T,E,k", [(1, 4, 1), (5, 8, 2), (64, 3, 3), (65, 16, 2),
