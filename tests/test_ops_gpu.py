@@ -325,6 +325,86 @@ def test_gemm_skinny_residual_mode():
     assert close(res, want, atol=tol, rtol=5e-2)  # residual updated in place
 
 
+@pytest.mark.parametrize("M,sk", [(1, 1), (16, 3), (100, 2), (128, 16), (129, None),
+                                  (200, 5), (256, None)])
+@pytest.mark.parametrize("N,K", [(192, 448), (4096, 1088)])
+def test_gemm_skinny_epilogues(M, sk, N, K):
+    """The split-K kernel's own epilogues (more than 128 rows, or an explicit
+    split): norm scalar, SwiGLU, residual, residual with row sums.  Tolerance:
+    bf16 rounding (2^-8 relative, through SwiGLU twice) and fp32 sums over K."""
+    x, w = rnd(M, K, seed=M, scale=0.3), rnd(N, K, seed=N, scale=0.3)
+    y = x.float() @ w.float().t()
+    ss = torch.zeros(M, 8, device=DEV)
+    ss[:, 5] = x.float().pow(2).sum(-1)
+    yn = y * torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + 1e-5)
+    tol = dict(atol=2e-3 * math.sqrt(K) * 0.09, rtol=2 ** -7)
+    loose = dict(atol=2e-3 * K ** 0.5, rtol=2 ** -6)
+
+    def run(mode, **kw):
+        return ops.linear_skinny(x, w, mode, sk=sk, **kw)
+    assert close(run(0), y, **tol)
+    assert close(run(0, scale=(ss, 1e-5)), yn, **loose)
+    g, u = y.chunk(2, -1)
+    assert close(run(2), torch.nn.functional.silu(g) * u, **loose)
+    g, u = yn.chunk(2, -1)
+    assert close(run(2, scale=(ss, 1e-5)), torch.nn.functional.silu(g) * u, **loose)
+    for mode in (1, 4):
+        res = rnd(M, N, seed=9)
+        want = y + res.float()
+        st = torch.full((M, 8), torch.nan, device=DEV) if mode == 4 else None
+        out = run(mode, residual=res, ss_out=st)
+        assert torch.equal(out, res) and close(res, want, **tol)
+        if mode == 4:
+            assert torch.allclose(st.sum(-1), res.float().pow(2).sum(-1),
+                                  rtol=1e-4)
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 64, 128])
+@pytest.mark.parametrize("N,K", [(192, 448), (4096, 512), (32768, 256)])
+def test_linear_rows_norm_scalar(M, N, K):
+    """Plain products with the RMSNorm scalar, split (the sums' kernel applies
+    it) and whole, from row sums or, up to 16 rows, from the rows themselves."""
+    x, w = rnd(M, K, seed=M + K, scale=0.3), rnd(N, K, seed=N, scale=0.3)
+    ss = torch.zeros(M, 8, device=DEV)
+    ss[:, 2] = x.float().pow(2).sum(-1)
+    rstd = torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + 1e-5)
+    want = x.float() @ w.float().t() * rstd
+    tol = dict(atol=2e-3 * K ** 0.5, rtol=2 ** -7)
+    assert close(ops.linear_rows(x, w, scale=(ss, 1e-5)), want, **tol)
+    assert close(ops.linear_skinny(x, w, scale=(ss, 1e-5)), want, **tol)
+    if M <= ops.ROWS_MAX:
+        assert close(ops.linear_rows(x, w, scale=(None, 1e-5)), want, **tol)
+
+
+def test_row_scalar_of_rope_and_activation():
+    """rope_cache and silu_and_mul with the RMSNorm scalar of un-normalised rows,
+    against the same on rows that were scaled first."""
+    T, Hq, Hk, D, K = 37, 4, 2, 128, 512
+    ss = torch.rand(T, 8, device=DEV) * K
+    rstd = torch.rsqrt(ss.sum(-1, keepdim=True) / K + 1e-5)
+    qkv = rnd(T, (Hq + 2 * Hk) * D, seed=1)
+    tab = ops.rope_table(64, D, device=DEV)
+    pos = torch.arange(T, device=DEV, dtype=torch.int32)
+    slots = torch.randperm(64, device=DEV)[:T]
+    got, want = [], []
+    for rows, scale, to in ((qkv.clone(), (ss, K, 1e-5), got),
+                            (qkv.double() * rstd, None, want)):
+        dev = DEV if scale else "cpu"
+        rows = rows.to(dev)
+        q, k, v = rows.split([Hq * D, Hk * D, Hk * D], 1)
+        kc = torch.zeros(4, Hk, 16, D, dtype=rows.dtype, device=dev)
+        vc = torch.zeros_like(kc)
+        ops.rope_cache(q, k, v, pos.to(dev), tab.to(dev), kc, vc, slots.to(dev),
+                       scale=scale)
+        to += [q, kc, vc]
+    for g, w_ in zip(got, want):
+        assert close(g, w_, atol=2 ** -7, rtol=2 ** -7)
+    gu = rnd(T, 2 * 768, seed=2)
+    g, u = (gu.float() * rstd).chunk(2, -1)
+    assert close(ops.silu_and_mul(gu, scale=(ss, K, 1e-5)),
+                 torch.nn.functional.silu(g) * u, atol=2 ** -8, rtol=2 ** -7)
+
+
 def test_sample_greedy_matches_argmax():
     torch.manual_seed(99)
     B, V = 5, 128256
