@@ -30,16 +30,23 @@
 //   attn_prefill_kernel  4 waves x 32 columns, K/V tiles of 64 tokens shared by
 //     the block and double-buffered (64 KB, two blocks per CU: one wave's
 //     exponentials run under the other's MFMA).  Bound by vector issue next to
-//     the matrix cores: 32 exponentials per lane and tile alone take half of the
-//     tile's MFMA time.  grid: K/V head fastest, so with 8 of them an XCD's L2
-//     keeps one head's K/V; late (long) tiles start first.
+//     the matrix cores (32 exponentials per lane and tile alone take half of the
+//     tile's MFMA time) and by the transfers, see below.  grid: K/V head fastest,
+//     so with 8 of them an XCD's L2 keeps one head's K/V; late (long) tiles start
+//     first.
 //   attn_prefill_few_kernel  32 columns per block: sequences whose columns fit
 //     one wave (verification of a few drafted tokens, single fed tokens), or all
 //     of a batch too small to fill the chip with 128-column blocks.  The four
 //     waves split the keys, each with private 32-token double buffers and no
 //     barrier in the loop, and merge through LDS; with fewer than 256 blocks the
 //     keys are also split over blocks and a second kernel merges.  Bound by the
-//     K/V stream, so P is kept to 16 bits more: two bf16 terms, two products.
+//     latency of its transfers, which nothing hides (128 KB of LDS, one block per
+//     CU): ~3.5 TB/s of K/V where decode attention reaches 5.  P is kept to 16 bits
+//     more: two bf16 terms, two products.
+// Transfers: where pages hold whole tiles, the page of the tile after next is looked
+// up behind the next tile's loads.  The compiler makes that a vector load, and the
+// wait for it drains the tile's loads with it, before this tile's arithmetic starts:
+// they overlap with the other block of the CU only.
 // Fragment layouts (measured): A: lane holds A[m=lane&31][k=(lane>>5)*8+j]; B:
 // B[k=(lane>>5)*8+j][n=lane&31]; C: reg r holds C[8*(r/4)+4*(lane>>5)+r%4][lane&31];
 // transposing read: lane i of a group of 16 gets column i of 4 rows x 16 columns
@@ -421,7 +428,8 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_few_kernel(
       stage<TILED, 8>(a, btrow, kvh, (kt + step) * AP_FEW, 0, last, page,
                       kbuf(cur ^ 1), vbuf(cur ^ 1));
       if (TILED) page = page_of(kt + 2 * step);
-      // all but the 16 loads just issued have landed
+      // the tile has landed when only the 16 loads just issued are out (with TILED
+      // the wait for the page index has drained those too)
       asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
     } else {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -7,14 +7,17 @@
 // row and load: operand loads straight to registers (16 rows x 64 bytes per
 // instruction) stop at ~7.6 TB/s of requests whatever is asked for, so X at 16
 // rows doubled the time.  16-byte chunks are permuted within a line by the row
-// number (the operand reads then do not meet in a bank), and the loads of the
-// next pieces are in flight while one is multiplied (counted waits).
+// number (the operand reads then do not meet in a bank).  Waits are counted, so that
+// the loads of the next pieces stay in flight while one is multiplied.  That holds
+// for gemm_tile_kernel and for gemm_rows_kernel without a norm scalar (o, down); in
+// its variants with one (qkv, gate/up) the compiler adds a full wait in front of the
+// operand reads, so everything a wave has asked for ahead has to land there first.
 //
 // gemm_rows_kernel, up to 16 rows: a block owns one tile of 16 weight rows (N =
 //   4096 gives 256 tiles, one per CU; N = 28672 seven per CU) and K is split over
 //   its 8 WAVES, which take 64-element pieces in turn, each through buffers of its
 //   own: no barrier in the loop, no partial sums in memory and no second launch.
-//   The waves' sums meet once, in LDS, in an order that does not depend on M.
+//   The waves' sums meet once, in LDS; results do not depend on M within this kernel.
 //   The epilogue is the layer's next step: bf16 store, residual add in place,
 //   SwiGLU (a tile is 8 gate and 8 up rows), or rotary embedding + page append (a
 //   tile is 8 rotation pairs of a head).  RMSNorm (its weight is folded into W):
@@ -33,11 +36,15 @@
 // Weight rows lie K * 2 bytes apart, usually a multiple of every channel
 // interleave, so the rows of one piece come from the same memory channel and
 // blocks that walk K in step ask the same channel for everything.  Blocks of an
-// XCD therefore start at different pieces (the order of a sum depends on the
-// column, not on M); where K is split the splits do that already and starting
-// elsewhere costs a little (4096 x 4096 in four, 32 rows: 8.0 -> 8.8 us).  SwiGLU over 28672 x 4096: 42.9 -> 40.2 us at one row, 53.4 -> 45.2
-// at 64, 62.3 -> 57.3 at 128 (before the weights were streamed); two pieces per wave in flight are then enough (four
-// needed half the CU's buffers: 50.5 us).
+// XCD therefore start at different pieces; where K is split the splits do that
+// already and starting elsewhere costs a little (4096 x 4096 in four, 32 rows: 8.0 ->
+// 8.8 us).  SwiGLU over 28672 x 4096: 42.9 -> 40.2 us at one row, 53.4 -> 45.2 at 64,
+// 62.3 -> 57.3 at 128 (before the weights were streamed).  Four pieces per wave
+// instead of two, which need half the CU's buffers, were slower (50.5 us), but that
+// was measured on the variant whose loads are drained.
+// The order in which a column is summed depends on the kernel, the width of its
+// blocks and the number of splits, and all three on M: the same row may differ by
+// fp32 rounding between steps of different sizes.
 // Measured in us, against the split-K kernel with two-stage buffers and its second
 // launch (in brackets).  One row: 6144 x 4096 with rotary and append 10.7 (21.3 in
 // three launches), 4096 x 4096 7.3 and 4096 x 14336 19.0 (together 44.4), SwiGLU
@@ -140,7 +147,7 @@ __device__ __forceinline__ void put_rope(const RowsArgs& a, int m, int head, int
 }
 
 // NORM: 0 none, 1 from ss, 2 computed from X.  PD pieces per wave in flight.
-template <int MT, int PD, int EPI, int NORM, int AUX>
+template <int PD, int EPI, int NORM, int AUX>
 __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
   constexpr int NW = 8;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -149,25 +156,23 @@ __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
   const int tile = blockIdx.x;
 
   constexpr int PIECE = 2048;                    // 16 rows x 64 elements
-  constexpr int SLOT = PIECE * (1 + MT);
-  constexpr int RS = MT * 16 + 4;                // column stride of the sums
+  constexpr int SLOT = PIECE * 2;                // of W and of X
+  constexpr int RS = 20;                         // column stride of the sums
   constexpr int RING = NW * PD * SLOT;
   constexpr int SUMS = NW * 16 * RS * 4;
   __shared__ __attribute__((aligned(16))) char lds[RING > SUMS ? RING : SUMS];
-  __shared__ float rsq[NW][MT * 16];
-  __shared__ float rstd[MT * 16];
+  __shared__ float rsq[NW][16];
+  __shared__ float rstd[16];
   lds_b* ring = (lds_b*)&lds[wid * PD * SLOT];
 
   // sources of this lane's chunks
   const int r8 = lane >> 3, ch = ((lane & 7) ^ r8) * 8 + wid * 64;
-  const u16* wp[2];
-  const u16* xp[MT * 2];
+  const u16 *wp[2], *xp[2];
 #pragma unroll
-  for (int g = 0; g < 2; ++g)
+  for (int g = 0; g < 2; ++g) {
     wp[g] = a.W + (size_t)weight_row<EPI>(a, tile, g * 8 + r8) * a.K + ch;
-#pragma unroll
-  for (int g = 0; g < MT * 2; ++g)
     xp[g] = a.X + (size_t)min(g * 8 + r8, a.M - 1) * a.K + ch;
+  }
   const int cnt = ((a.K >> 6) - wid + NW - 1) / NW;  // this wave's pieces
   const int rot = cnt > 0 ? ((int)blockIdx.x >> 3) % cnt : 0;
   auto load = [&](int i) {
@@ -177,62 +182,47 @@ __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
 #pragma unroll
     for (int g = 0; g < 2; ++g) load_line8<AUX>(wp[g] + off, to + g * 1024);
 #pragma unroll
-    for (int g = 0; g < MT * 2; ++g)
+    for (int g = 0; g < 2; ++g)
       load_line8<KEEP>(xp[g] + off, to + PIECE + g * 1024);
   };
-  f32x4 acc[MT], sq[MT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    acc[m] = f32x4{0, 0, 0, 0};
-    sq[m] = f32x4{0, 0, 0, 0};
-  }
+  f32x4 acc = {0, 0, 0, 0}, sq = {0, 0, 0, 0};
 #pragma unroll
   for (int s = 0; s < PD; ++s)
     if (s < cnt) load(s);
   for (int i = 0; i < cnt; ++i) {
     // piece i has landed when only the loads of the PD - 1 behind it are out
+    static_assert(PD == 2, "wait count");
     if (i + PD <= cnt) {
-      static_assert(PD == 2 && MT <= 2, "wait counts");
-      if (MT == 1) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+      asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
     } else {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     const lds_b* at = ring + (i % PD) * SLOT;
-    bf16x8r w[2], x[MT][2];
+    bf16x8r w[2], x[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       w[h] = frag(at, h);
-#pragma unroll
-      for (int m = 0; m < MT; ++m) x[m][h] = frag(at + PIECE * (1 + m), h);
+      x[h] = frag(at + PIECE, h);
     }
     // the slot is read: fill it again
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     if (i + PD < cnt) load(i + PD);
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[m][h], w[h], acc[m],
-                                                         0, 0, 0);
-        if (NORM == 2)
-          sq[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[m][h], x[m][h], sq[m],
-                                                          0, 0, 0);
-      }
+    for (int h = 0; h < 2; ++h) {
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[h], w[h], acc, 0, 0, 0);
+      if (NORM == 2)
+        sq = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[h], x[h], sq, 0, 0, 0);
+    }
   }
 
   // meet in LDS: [wave][tile column][row]; + 4 spreads the columns over banks
   __syncthreads();
   float (*red)[16][RS] = reinterpret_cast<float (*)[16][RS]>(lds);
-#pragma unroll
-  for (int m = 0; m < MT; ++m)
-    *reinterpret_cast<f32x4*>(&red[wid][n][m * 16 + (lane >> 4) * 4]) = acc[m];
+  *reinterpret_cast<f32x4*>(&red[wid][n][(lane >> 4) * 4]) = acc;
   if (NORM == 2) {
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if ((lane >> 4) * 4 + r == n) rsq[wid][m * 16 + n] = sq[m][r];
+    for (int r = 0; r < 4; ++r)
+      if ((lane >> 4) * 4 + r == n) rsq[wid][n] = sq[r];
   }
   __syncthreads();
   if (NORM != 0) {
@@ -283,32 +273,25 @@ __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
   }
 }
 
-// MT 16-row groups of X (even), ring of STAGES pieces of K = 64.  Grid
-// (N / 64, splits).  EPI_PLAIN, EPI_SWIGLU (not split) or EPI_PARTS.
+// All but N of a wave's loads have landed, its LDS reads are done, and so it is for
+// every wave of the block.
 template <int N>
 __device__ __forceinline__ void wait_loads_and_meet() {
+  static_assert(N == 0 || N == 3 || N == 4 || N == 6 || N == 8, "wait counts");
   if constexpr (N == 0)
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   else if constexpr (N == 3)
     asm volatile("s_waitcnt vmcnt(3) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   else if constexpr (N == 4)
     asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  else if constexpr (N == 5)
-    asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   else if constexpr (N == 6)
     asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  else if constexpr (N == 8)
+  else
     asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  else if constexpr (N == 9)
-    asm volatile("s_waitcnt vmcnt(9) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  else if constexpr (N == 10)
-    asm volatile("s_waitcnt vmcnt(10) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  else {
-    static_assert(N == 12, "wait counts");
-    asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  }
 }
 
+// MT 16-row groups of X (even), ring of STAGES pieces of K = 64.  Grid
+// (N / (16 NW), splits).  EPI_PLAIN, EPI_SWIGLU (not split) or EPI_PARTS.
 template <int MT, int NW, int WT, int STAGES, int EPI, int NORM, int AUX>
 __global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -507,9 +490,9 @@ static bool streamed(const RowsArgs& a) { return (i64)a.N * a.K >= (8 << 20); }
 template <int EPI, int NORM>
 static void launch_rows(const RowsArgs& a, hipStream_t st) {
   if (streamed(a))
-    gemm_rows_kernel<1, 2, EPI, NORM, STREAM><<<a.N / 16, 512, 0, st>>>(a);
+    gemm_rows_kernel<2, EPI, NORM, STREAM><<<a.N / 16, 512, 0, st>>>(a);
   else
-    gemm_rows_kernel<1, 2, EPI, NORM, KEEP><<<a.N / 16, 512, 0, st>>>(a);
+    gemm_rows_kernel<2, EPI, NORM, KEEP><<<a.N / 16, 512, 0, st>>>(a);
 }
 
 // Blocks of 128 weight rows (eight waves) halve the reads of X.  They pay from 33

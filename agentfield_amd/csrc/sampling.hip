@@ -153,7 +153,9 @@ __global__ void __launch_bounds__(64) sample_combine_kernel(
 // row (64 of them on 256 CUs, one bin conflict after the other) took 173 us
 // for the histogram and 52 us for the maximum at 64 x 128256.  The passes after
 // the first fold the per-split results of the pass before in their prologue, so
-// nothing but the four reads of the row is launched: 346 us -> 28 us.
+// nothing but the three reads of the row and the draw's last step is launched: 346
+// us -> 28 us.  (The draw's blocks fold all 16 histograms of their row each, 32 KB a
+// block; with the two logarithms per value that is what its 15 us go to.)
 #define TKP_BINS 256
 #define TKP_SPAN 20.0f
 
@@ -188,8 +190,8 @@ __device__ __forceinline__ float row_max_of(const float* __restrict__ rmax,
 // adds one 64-bit integer: 1 in the upper 20 bits, and below them its mass
 // relative to its bin's upper edge (0.92..1) in units of 2^-24, which loses no
 // more per value than a float does and nothing in the sum.  Every bin has 16
-// copies, one per lane of a group of 16, which also keeps a count within its
-// field for rows of up to 2^28 values (45 us -> 8 us).
+// copies, one per lane of a group of 16 (45 us -> 8 us).  A copy gets about 1/256 of
+// a split row's values: the 20-bit count and the 44-bit mass hold rows of up to 2^27.
 #define TKP_COPIES 16
 #define TKP_MASS_BITS 44
 __global__ void __launch_bounds__(256) tkp_hist_kernel(
