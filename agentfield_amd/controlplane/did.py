@@ -16,6 +16,7 @@ import hashlib
 import json
 import os
 import secrets
+import tempfile
 import time
 from pathlib import Path
 
@@ -74,15 +75,30 @@ class Keystore:
     @property
     def seed(self) -> bytes:
         if self._seed is None:
-            if self.path and self.path.exists():
-                self._seed = self._decode(self.path.read_text())
-            else:
-                self._seed = secrets.token_bytes(32)
-                if self.path:
-                    self.path.parent.mkdir(parents=True, exist_ok=True)
-                    self.path.write_text(self._encode(self._seed))
-                    os.chmod(self.path, 0o600)
+            if self.path and not self.path.exists():
+                self._create(secrets.token_bytes(32))
+            self._seed = (self._decode(self.path.read_text()) if self.path
+                          else secrets.token_bytes(32))
         return self._seed
+
+    def _create(self, seed: bytes) -> None:
+        """The file appears whole or not at all, and the first of several
+        processes to create it wins: all of them read its seed."""
+        self.path.parent.mkdir(parents=True, exist_ok=True)
+        fd, tmp = tempfile.mkstemp(dir=self.path.parent,
+                                   prefix=self.path.name + ".")
+        try:
+            with os.fdopen(fd, "w") as f:      # mkstemp: mode 0600
+                f.write(self._encode(seed))
+            try:
+                os.link(tmp, self.path)
+            except FileExistsError:
+                pass
+            except OSError:                    # no hard links here
+                if not self.path.exists():
+                    os.replace(tmp, self.path)
+        finally:
+            Path(tmp).unlink(missing_ok=True)
 
 
 def derive_seed(parent: bytes, path: str) -> bytes:

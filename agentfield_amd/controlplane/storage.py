@@ -103,14 +103,29 @@ class Storage:
         self._lock = threading.RLock()
         with self._lock:
             if path != ":memory:":
-                self._db.execute("PRAGMA journal_mode=WAL")
                 # multi-worker planes share one WAL file: writers from
                 # other processes serialize on the WAL write lock; wait
                 # instead of surfacing SQLITE_BUSY
                 self._db.execute("PRAGMA busy_timeout=10000")
+                self._enter_wal()
             self._db.execute("PRAGMA synchronous=NORMAL")
             self._db.executescript(_SCHEMA)
             self._db.commit()
+
+    def _enter_wal(self, timeout: float = 10.0) -> None:
+        """Switch the file to WAL mode.  The switch needs the file to itself
+        and does not wait for other connections (the busy timeout is not
+        asked), so workers that open a new database at the same moment would
+        fail: try again until they are through."""
+        deadline = time.monotonic() + timeout
+        while True:
+            try:
+                self._db.execute("PRAGMA journal_mode=WAL")
+                return
+            except sqlite3.OperationalError as e:
+                if "locked" not in str(e) or time.monotonic() > deadline:
+                    raise
+                time.sleep(0.01)
 
     def _exec(self, sql: str, args=()):
         with self._lock:

@@ -969,3 +969,37 @@ def test_engine_metrics_ride_heartbeats():
     assert summ["engines"]["gpu0"] == {"running": 7,
                                        "kv_free_pages": 1234}
     srv.stop()
+
+
+def _open_at(path, keys, go, out):
+    from agentfield_amd.controlplane.did import DIDService, Keystore
+    from agentfield_amd.controlplane.storage import Storage
+    while time.time() < go:
+        pass
+    try:
+        dids = DIDService(Storage(path), Keystore(keys))
+        out.put((dids.root_did, dids.keystore.seed.hex()))
+    except Exception as e:
+        out.put(repr(e))
+
+
+def test_workers_open_a_new_plane_at_the_same_moment(tmp_path):
+    """Workers of one plane start together: each must get through the new
+    database's switch to WAL mode, and all must end up with one root identity
+    (one of four used to fail here in every second round)."""
+    import multiprocessing as mp
+    ctx = mp.get_context("fork")
+    for n in range(15):
+        d = tmp_path / str(n)
+        out, go = ctx.Queue(), time.time() + 0.05
+        procs = [ctx.Process(target=_open_at, args=(
+            str(d / "af.db"), str(d / "keystore.key"), go, out))
+            for _ in range(4)]
+        for p in procs:
+            p.start()
+        got = [out.get(timeout=30) for _ in procs]
+        for p in procs:
+            p.join()
+        assert len(set(got)) == 1 and isinstance(got[0], tuple), got
+        assert (d / "keystore.key").stat().st_mode & 0o777 == 0o600
+        assert sorted(f.name for f in d.glob("keystore*")) == ["keystore.key"]
