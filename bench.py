@@ -94,17 +94,22 @@ def parse_args():
 
 
 # --------------------------------------------------------------- REST mode
-def _wait_http(url: str, timeout: float = 60.0) -> None:
+def _wait_http(url: str, proc: subprocess.Popen, log: Path,
+               timeout: float) -> None:
+    """Until the server answers; if it does not, or proc ends, raise with the
+    end of its output."""
     import httpx
     deadline = time.time() + timeout
-    while time.time() < deadline:
+    while time.time() < deadline and proc.poll() is None:
         try:
             if httpx.get(url, timeout=2.0).status_code == 200:
                 return
         except Exception:
             pass
         time.sleep(0.1)
-    raise TimeoutError(f"{url} not up")
+    raise TimeoutError(
+        f"{url} not up (exit status {proc.poll()}); its output ends:\n"
+        + log.read_text(errors="replace")[-3000:])
 
 
 class _AgentServer:
@@ -157,6 +162,7 @@ def run_rest(args, world: int, rank: int, dist, device: str, cfg) -> None:
         max(2, min(8, world, (os.cpu_count() or 8) // 4))
     cp_workers = args.cp_workers or auto
 
+    logs = Path(tempfile.mkdtemp(prefix="af-bench-log-"))
     eng_proc = None
     stats_url = None
     if args.engine_proc:
@@ -175,9 +181,10 @@ def run_rest(args, world: int, rank: int, dist, device: str, cfg) -> None:
             eng_argv.append("--no-graphs")
         eng_proc = subprocess.Popen(
             eng_argv, env={**os.environ, "PYTHONPATH": str(root)}, cwd=root,
-            stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL,
+            stdout=open(logs / "engine.log", "w"), stderr=subprocess.STDOUT,
             preexec_fn=_die_with_parent)
-        _wait_http(f"{stats_url}/v1/health", timeout=600.0)
+        _wait_http(f"{stats_url}/v1/health", eng_proc, logs / "engine.log",
+                   timeout=600.0)
         os.environ["AGENTFIELD_ENGINE_URLS"] = stats_url
         runner = None
     else:
@@ -206,10 +213,12 @@ def run_rest(args, world: int, rank: int, dist, device: str, cfg) -> None:
              "--db", f"{tmp}/af.db", "--data-dir", tmp,
              "--workers", str(cp_workers)],
             env={**os.environ, "PYTHONPATH": str(root)}, cwd=root,
-            stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL,
+            stdout=open(logs / "plane.log", "w"), stderr=subprocess.STDOUT,
             preexec_fn=_die_with_parent)
+        # a fresh machine may first have to page the interpreter's packages in
         for i in range(cp_workers):
-            _wait_http(f"http://127.0.0.1:{cp_port + i}/api/v1/health")
+            _wait_http(f"http://127.0.0.1:{cp_port + i}/api/v1/health",
+                       cp_proc, logs / "plane.log", timeout=180.0)
     if dist is not None:
         dist.barrier()
 

@@ -1003,3 +1003,17 @@ def test_workers_open_a_new_plane_at_the_same_moment(tmp_path):
         assert len(set(got)) == 1 and isinstance(got[0], tuple), got
         assert (d / "keystore.key").stat().st_mode & 0o777 == 0o600
         assert sorted(f.name for f in d.glob("keystore*")) == ["keystore.key"]
+
+
+def test_benchmark_says_why_a_server_is_not_up(tmp_path):
+    import subprocess
+    import sys
+    import bench
+    log = tmp_path / "log"
+    proc = subprocess.Popen(
+        [sys.executable, "-c", "print('database is locked'); raise SystemExit(3)"],
+        stdout=open(log, "w"), stderr=subprocess.STDOUT)
+    t0 = time.time()
+    with pytest.raises(TimeoutError, match="status 3.*\n.*database is locked"):
+        bench._wait_http("http://127.0.0.1:9/health", proc, log, timeout=60.0)
+    assert time.time() - t0 < 30
