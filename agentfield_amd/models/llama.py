@@ -328,27 +328,32 @@ class LlamaLayer(nn.Module):
             h = self.mlp(h)
         return h, residual
 
-    def rows_weights(self) -> tuple:
-        """The weights that forward_rows_fused reads."""
+    def rows_weights_ok(self, cfg: LlamaConfig) -> bool:
+        """Whether forward_rows_fused can read this layer's weights."""
         at = self._modules["attn"]._parameters
         mlp = self._modules["mlp"]._parameters
-        return at["qkv"], at["o"], mlp["gate_up"], mlp["down"]
+        qkv, o, gate_up, down = at["qkv"], at["o"], mlp["gate_up"], mlp["down"]
+        H, I, Q = cfg.hidden_size, cfg.intermediate_size, cfg.q_size
+        return (qkv.shape == (Q + 2 * cfg.kv_size, H) and o.shape == (H, Q)
+                and gate_up.shape == (2 * I, H) and down.shape == (H, I)
+                and ops.rows_operands_ok((qkv, o, gate_up, down)))
 
     def forward_rows_fused(self, residual, ss, positions, rope_tab, kv, md):
         """Few-row path (decode steps, small prefill steps): norms, rotary
         positions, page append, SwiGLU and residual adds ride in the
         weight-streaming GEMMs, nothing runs on its own but attention.
         `residual` is updated in place; ss [T, 8] holds its rows' sums of
-        squares (None up to ops.ROWS_MAX rows, which need none)."""
+        squares (None up to ops.ROWS_MAX rows, which need none).  The caller has
+        asked rows_weights_ok; the rows are made here."""
         at, mlp = self.attn, self.mlp
         q = ops.qkv_rope_rows(residual, at.qkv, self.eps, ss, positions,
                               rope_tab, kv.k[at.layer_idx],
                               kv.v[at.layer_idx], md.slots)
         o = at.attention(q, kv, md)
         mode = 1 if ss is None else 4
-        ops.linear_rows(o, at.o, mode, residual, ss_out=ss, want_out=False)
-        act = ops.linear_rows(residual, mlp.gate_up, 2, scale=(ss, self.eps))
-        ops.linear_rows(act, mlp.down, mode, residual, ss_out=ss,
+        ops.launch_rows(o, at.o, mode, residual, ss_out=ss, want_out=False)
+        act = ops.launch_rows(residual, mlp.gate_up, 2, scale=(ss, self.eps))
+        ops.launch_rows(act, mlp.down, mode, residual, ss_out=ss,
                         want_out=False)
 
 
@@ -427,8 +432,7 @@ class LlamaForCausalLM(nn.Module):
                 and (cfg.q_size + 2 * cfg.kv_size) % 64 == 0
                 and cfg.q_size % 64 == 0
                 and self.embed.dtype == torch.bfloat16
-                and ops.rows_operands_ok(w for layer in self.layers
-                                        for w in layer.rows_weights()))
+                and self.embed.shape[1] == cfg.hidden_size)
 
     def forward(self, ids, positions, kv: KVCache, md: AttnMetadata,
                 logit_rows: torch.Tensor | None = None):
@@ -439,8 +443,15 @@ class LlamaForCausalLM(nn.Module):
                   if T > ops.ROWS_MAX else None)
             residual = ops.embedding(ids, self.embed, ss=ss)
             for layer in self.layers:
-                layer.forward_rows_fused(residual, ss, positions,
-                                         self.rope_tab, kv, md)
+                if layer.rows_weights_ok(self.cfg):
+                    layer.forward_rows_fused(residual, ss, positions,
+                                             self.rope_tab, kv, md)
+                    continue
+                h, _ = layer(residual, None, positions, self.rope_tab, kv, md)
+                residual.add_(h)
+                if ss is not None:
+                    ss.zero_()
+                    ss[:, 0] = residual.float().pow(2).sum(-1)
             if logit_rows is not None:
                 residual = ops.gather_rows(residual, logit_rows)
             h = ops.rmsnorm(residual, self.final_norm, self.cfg.rms_eps)

@@ -286,19 +286,22 @@ def rows_splits(M: int, N: int, K: int) -> int:
     return -(-pieces // per)          # no empty split
 
 
+_transform = torch._C._functorch.peek_interpreter_stack
+_modes = torch._C._len_torch_dispatch_stack
+
+
 def watched(*tensors: torch.Tensor, grad: bool = True) -> bool:
     """Whether a product of these must be torch's own: autograd records it
     (grad), or forward mode, a function transform, a tracer or a tensor subclass
     has to see it.  Kernels called by address pass all of them by."""
     grad = grad and torch.is_grad_enabled()
     for t in tensors:
-        if (grad and t.requires_grad
-                or type(t) not in (torch.Tensor, torch.nn.Parameter)):
+        kind = type(t)
+        if (kind is not torch.Tensor and kind is not torch.nn.Parameter
+                or grad and t.requires_grad):
             return True
-    return (forward_ad._current_level >= 0
-            or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch._C._len_torch_dispatch_stack() > 0
-            or torch.compiler.is_compiling())
+    return (forward_ad._current_level >= 0 or _transform() is not None
+            or _modes() > 0 or torch.compiler.is_compiling())
 
 
 def rows_operands_ok(tensors) -> bool:
@@ -358,8 +361,7 @@ def linear_rows(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
     if not _rows_ok(x, w):
         raise AfOpsError(f"row GEMM: {tuple(x.shape)} {x.dtype} rows against "
                          f"{tuple(w.shape)} {w.dtype} weights")
-    M, K = x.shape
-    N = w.shape[0]
+    M, N = x.shape[0], w.shape[0]
     cols = N // 2 if mode == 2 else N
     if mode in (1, 4):
         _need(_whole(residual, x, M, N) and _apart(residual, x),
@@ -371,8 +373,21 @@ def linear_rows(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
     if out is not None:
         _need(_whole(out, x, M, cols) and _apart(out, x),
               f"row GEMM: out must be whole [{M}, {cols}] rows apart from x")
-    elif want_out:
-        out = torch.empty(M, cols, dtype=x.dtype, device=x.device)
+    if scale is not None:
+        _need(mode in (0, 2) and (M <= ROWS_MAX if scale[0] is None
+                                  else _row_stats(scale[0], x)),
+              "row GEMM: fp32 [M, 8] sums of the rows for the norm")
+    return launch_rows(x, w, mode, residual, scale, ss_out, want_out, out)
+
+
+def launch_rows(x, w, mode=0, residual=None, scale=None, ss_out=None,
+                 want_out=True, out=None):
+    """linear_rows for callers that have checked the operands, or made them."""
+    M, K = x.shape
+    N = w.shape[0]
+    if want_out and out is None:
+        out = torch.empty(M, N // 2 if mode == 2 else N, dtype=x.dtype,
+                          device=x.device)
     splits, parts = 1, None
     if mode != 2 and (M > ROWS_MAX or mode == 4):
         splits = rows_splits(M, N, K)
@@ -383,9 +398,6 @@ def linear_rows(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
     if scale is not None:
         ss, eps = scale
         norm = 2 if ss is None else 1
-        _need(mode in (0, 2) and (M <= ROWS_MAX if ss is None
-                                  else _row_stats(ss, x)),
-              "row GEMM: fp32 [M, 8] sums of the rows for the norm")
     rc = _lib.lib().af_rows_linear(
         _lib.ptr(out), _lib.ptr(residual), _lib.ptr(parts), _lib.ptr(ss_out),
         _lib.ptr(x), _lib.ptr(w), M, N, K, splits, mode, norm, _lib.ptr(ss), eps,
@@ -501,9 +513,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
         _need(not silu_fuse and tuple(out.shape) == (M, N),
               f"linear: out {tuple(out.shape)} for a [{M}, {N}] product")
     if (x.is_cuda and not watched(x, w, grad=not silu_fuse)
-            and (out is None or _whole(out, x, M, N)) and _rows_ok(x, w)
+            and (out is None or _whole(out, x, M, N) and _apart(out, x))
+            and _rows_ok(x, w)
             and (silu_fuse or M <= 32 or N <= 12288 or N >= 24576)):
-        return linear_rows(x, w, mode=2 if silu_fuse else 0, out=out)
+        return launch_rows(x, w, 2 if silu_fuse else 0, out=out)
     if out is not None:
         return torch.mm(x, w.t(), out=out)
     y = x @ w.t()

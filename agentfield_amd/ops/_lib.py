@@ -256,8 +256,8 @@ def check(rc: int, name: str) -> None:
 
 
 def main_lib_ready() -> bool:
-    """True when libafops.so is on disk (never triggers a build)."""
-    return _LIB_PATH.exists()
+    """True when libafops.so is loaded or on disk (never triggers a build)."""
+    return lib.cache_info().currsize > 0 or _LIB_PATH.exists()
 
 
 def native_loaded() -> bool:

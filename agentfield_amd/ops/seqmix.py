@@ -22,11 +22,13 @@ from __future__ import annotations
 import ctypes
 import math
 import os
+import sys
 
 import torch
 
 from . import _lib
 
+_ops = sys.modules[__package__]     # it imports this module last
 _DT = {torch.bfloat16: 0, torch.float32: 1}
 # a step whose longest row chunk reaches this many rows runs bf16 attention
 # through the MFMA tile kernel; shorter steps (decode) use one wave per row
@@ -685,16 +687,15 @@ def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
     M, K = x.shape
     N = w.shape[0]
     if skinny and x.is_cuda and M <= 128 and _lib.main_lib_ready():
-        from . import _rows_ok, linear_rows, linear_skinny, watched
         if ((M <= 32 or M <= 64 and N <= 4096 or N >= 24576)
-                and not watched(x, w) and _rows_ok(x, w)):
-            return linear_rows(x, w)
+                and not _ops.watched(x, w) and _ops._rows_ok(x, w)):
+            return _ops.launch_rows(x, w)
         if (_SKINNY and x.dtype == torch.bfloat16
                 and N % 64 == 0 and K % 64 == 0
                 and ((M <= 64 and K <= 8192)
                      or (32 < M <= 128 and K >= 8192 and N <= 8192))
                 and x.is_contiguous() and w.is_contiguous()):
-            return linear_skinny(x, w)
+            return _ops.linear_skinny(x, w)
     return x @ w.t()
 
 

@@ -51,8 +51,9 @@ def test_left_to_the_library(x, w):
 
 
 def test_few_row_path_needs_plain_bf16_weights():
-    """The few-row path of the dense decoder serves models whose weights the row
-    GEMMs read; any other model keeps the general path, prompts included."""
+    """The few-row path of the dense decoder serves bf16 models, and of these the
+    layers whose weights the row GEMMs read; everything else keeps the general
+    path, prompts included."""
     from agentfield_amd.models import CONFIGS
     from agentfield_amd.models.llama import LlamaForCausalLM
 
@@ -61,20 +62,25 @@ def test_few_row_path_needs_plain_bf16_weights():
             0).fold_norm_weights()
     assert not model(torch.float32)._can_fuse_rows(4)
     assert not model(torch.float16)._can_fuse_rows(4)
+    m = model(torch.bfloat16)
+    assert m._can_fuse_rows(1) and m._can_fuse_rows(128)
+    assert not m._can_fuse_rows(129) and not m._can_fuse_rows(0)
+    layer = m.layers[1]
     for part, name in (("attn", "qkv"), ("attn", "o"), ("mlp", "gate_up"),
                        ("mlp", "down")):
-        m = model(torch.bfloat16)
-        assert m._can_fuse_rows(1) and m._can_fuse_rows(128)
-        assert not m._can_fuse_rows(129) and not m._can_fuse_rows(0)
-        p = getattr(getattr(m.layers[1], part), name)
+        assert layer.rows_weights_ok(m.cfg)
+        p = getattr(getattr(layer, part), name)
         flat = p.data.clone()
         p.data = flat.t().contiguous().t()          # strided
-        assert not m._can_fuse_rows(4)
+        assert not layer.rows_weights_ok(m.cfg)
         p.data = torch.cat([flat.flatten()[:1], flat.flatten()])[1:].view_as(
             flat)                                   # off the 16-byte grid
-        assert not m._can_fuse_rows(4)
+        assert not layer.rows_weights_ok(m.cfg)
+        p.data = flat[:-64]                         # of another size
+        assert not layer.rows_weights_ok(m.cfg)
         p.data = flat
-        assert m._can_fuse_rows(4)
+    p.data = flat.float()
+    assert not layer.rows_weights_ok(m.cfg)
 
 
 def test_watched_products():

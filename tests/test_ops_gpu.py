@@ -981,3 +981,42 @@ def test_moe_kernels_refuse_other_operands():
         with pytest.raises(ops.AfOpsError):
             ops.moe_combine(*args)
     ops.moe_combine(y, pos, w)
+
+
+@pytest.mark.parametrize("T", [5, 40])
+@pytest.mark.parametrize("layer", [0, 1])
+@pytest.mark.parametrize("prompt", [True, False])
+def test_few_row_path_with_strided_weights(T, layer, prompt):
+    """A layer whose weights the row GEMMs cannot read runs its general form in
+    the middle of the few-row path, for prompts and decode steps.  Tolerance:
+    both are bf16 roundings of the same two layers, 1% of the logits' rms."""
+    from agentfield_amd.models import CONFIGS
+    from agentfield_amd.models.llama import (AttnMetadata, KVCache,
+                                             LlamaForCausalLM)
+    cfg, page = CONFIGS["tiny"], 16
+    m = LlamaForCausalLM(cfg, device=DEV).init_random(3).fold_norm_weights()
+    ids = torch.randint(0, cfg.vocab_size, (T,), device=DEV, dtype=torch.int32)
+    if prompt:
+        pos = torch.arange(T, device=DEV, dtype=torch.int32)
+        bt = torch.arange(1, 5, device=DEV, dtype=torch.int32)[None]
+        md = AttnMetadata(
+            is_prefill=True, slots=pos.long() + page, seq_lens=[T], block_table=bt,
+            cu_seqlens=torch.tensor([0, T], device=DEV, dtype=torch.int32),
+            q_start=torch.zeros(1, device=DEV, dtype=torch.int32))
+    else:
+        pos = torch.zeros(T, device=DEV, dtype=torch.int32)
+        bt = torch.arange(1, T + 1, device=DEV, dtype=torch.int32)[:, None]
+        md = AttnMetadata(is_prefill=False, slots=bt[:, 0].long() * page,
+                          block_table=bt, seq_lens_t=pos + 1)
+    out = []
+    with torch.no_grad():
+        for strided in (False, True):
+            if strided:
+                for p in (m.layers[layer].attn.o, m.layers[layer].mlp.down):
+                    p.data = p.data.t().contiguous().t()
+            kv = KVCache(cfg, 64, page, DEV)
+            assert m._can_fuse_rows(T)
+            assert m.layers[layer].rows_weights_ok(cfg) != strided
+            out.append(m(ids, pos, kv, md).float())
+    a, b = out
+    assert (a - b).norm() <= 1e-2 * a.norm()
