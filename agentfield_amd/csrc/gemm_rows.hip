@@ -45,8 +45,9 @@
 // The order in which a column is summed depends on the kernel, the width of its
 // blocks and the number of splits, and all three on M: the same row may differ by
 // fp32 rounding between steps of different sizes.
-// Measured in us, against the split-K kernel with two-stage buffers and its second
-// launch (in brackets).  One row: 6144 x 4096 with rotary and append 10.7 (21.3 in
+// Measured in us, alone and repeated (inside a step 5-25% more: 64 rows 13.8, 9.7,
+// 23.1, 41.9), against the split-K kernel with two-stage buffers and its second launch
+// (in brackets).  One row: 6144 x 4096 with rotary and append 10.7 (21.3 in
 // three launches), 4096 x 4096 7.3 and 4096 x 14336 19.0 (together 44.4), SwiGLU
 // over 28672 x 4096 37.5 = 6.3 TB/s (58.2).  16 rows: 13.1, 8.1, 23.1, 42.6.  64
 // rows, without the closing launches: 11.2, 8.5, 21.7, 40.1 (16.7, o + down 44.8,

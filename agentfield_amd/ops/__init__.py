@@ -506,7 +506,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
     against rows in us: 14336 x 4096 25.6 / 21.7 at 32 rows, 26.7 / 30.0 at 48,
     33.9 / 36.0 at 128; 16384 x 4096 34.3 / 24.7, 34.9 / 38.9, 39.0 / 43.3;
     28672 x 4096 53.9 / 41.5, 64.0 / 42.1, 56.7 / 51.7; 128256 x 4096 190 / 151
-    at one row, 214 / 184 at 64, 238 / 215 at 128."""
+    at one row, 214 / 184 at 64, 238 / 215 at 128.  Between 12288 and 24576
+    these two were measured; the limits are the nearest sizes at which rows win."""
     M, _K = x.shape
     N = w.shape[0]
     if out is not None:

@@ -679,9 +679,11 @@ def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
     12.7 at 64, 16.2 / 18.2 at 100; 6144 x 2048 12.8 / 11.0 at 32, 13.2 / 13.9 at
     64; 10240 x 2048 16.4 / 9.6 at 4, 16.4 / 13.9 at 32, 19.6 / 21.3 at 128;
     14336 x 4096 25.6 / 21.7 at 32, 26.7 / 30.0 at 48; 128256 x 2048 111 / 91 at
-    32, 125 / 124 at 128.  AF_MIX_SKINNY=1 sends
-    the remaining decode-sized products (up to 64 rows, or 33..128 against a long
-    inner dimension) to the framework's kernels too."""
+    32, 125 / 124 at 128.  The heads of the hybrid models call with skinny=False,
+    which is always the vendor GEMM.  AF_MIX_SKINNY=1 sends the remaining
+    decode-sized products (up to 64 rows, or 33..128 against a long inner dimension)
+    to the framework's kernels too.  What autograd or a transform has to see is
+    the vendor GEMM's (watched)."""
     if out is not None:
         return torch.mm(x, w.t(), out=out)
     M, K = x.shape
