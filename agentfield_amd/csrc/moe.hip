@@ -59,7 +59,7 @@ __global__ void __launch_bounds__(256) moe_route_kernel(
 #pragma unroll
   for (int j = 0; j < MOE_MAX_K; ++j)
     if (j < k) {
-      best[j] = __expf(best[j] - top);
+      best[j] = expf(best[j] - top);
       sum += best[j];
     }
 #pragma unroll

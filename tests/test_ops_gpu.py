@@ -967,6 +967,23 @@ def test_moe_sorted_dispatch(T, E, k):
     assert close(got, ref_, atol=2e-2, rtol=2 ** -7)
 
 
+@pytest.mark.parametrize("E,k", [(2, 2), (8, 2), (64, 8)])
+def test_moe_weights_to_fp32_rounding(E, k):
+    """Logits that fp32 holds exactly (a row picks one column of the router), up
+    to 80 apart: what is left are the exponential (2 units of 2^-24), k - 1
+    additions and the division (1 each)."""
+    T = H = 512
+    x = torch.eye(T, H, device=DEV, dtype=torch.bfloat16)
+    torch.manual_seed(E)
+    router = torch.randint(0, 320, (E, H), device=DEV).div(8).bfloat16()
+    router[1::2] *= -1
+    w, row, pos, offs = ops.moe_route(x, router, k)
+    tv = torch.softmax(router.double().t(), -1).topk(k, -1).values
+    tv /= tv.sum(-1, keepdim=True)
+    err = ((w.double() - tv).abs() / tv).max().item()
+    assert err <= (2 + 2 + k) * 2 ** -24, err * 2 ** 24
+
+
 def test_moe_kernels_refuse_other_operands():
     x, router = rnd(5, 520, seed=1), rnd(8, 520, seed=2)
     for a, r, k in ((x, rnd(8, 512), 2), (x[:, :512].contiguous(), router, 2),
