@@ -12,7 +12,8 @@
 #define MOE_MAX_K 8
 
 // Router logits in fp32 (products of bf16 are exact), softmax over the k largest:
-// a wave per row, equal logits go to the smaller expert.
+// a wave per row, equal logits go to the smaller expert.  A logit that is not a
+// number counts as the largest, so that the row's weights show it.
 template <int EM>
 __global__ void __launch_bounds__(256) moe_route_kernel(
     i32* __restrict__ topi, float* __restrict__ topv, const u16* __restrict__ x,
@@ -49,7 +50,7 @@ __global__ void __launch_bounds__(256) moe_route_kernel(
 #pragma unroll
     for (int e = 0; e < EM; ++e) {
       if (e >= E || (used >> e & 1)) continue;
-      if (w < 0 || acc[e] > b) { b = acc[e]; w = e; }
+      if (w < 0 || acc[e] > b || acc[e] != acc[e]) { b = acc[e]; w = e; }
     }
     used |= 1ull << w;
     best[j] = b;

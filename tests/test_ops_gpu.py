@@ -984,6 +984,24 @@ def test_moe_weights_to_fp32_rounding(E, k):
     assert err <= (2 + 2 + k) * 2 ** -24, err * 2 ** 24
 
 
+@pytest.mark.parametrize("E", [2, 5, 64])
+def test_moe_routing_shows_bad_numbers(E):
+    """A row with a logit of NaN or +inf gets weights of NaN as a softmax gives
+    them, whichever expert it belongs to, and the sort stays whole; -inf is a
+    weight of zero."""
+    x = torch.eye(1, 64, device=DEV, dtype=torch.bfloat16)
+    for bad in (torch.nan, torch.inf, -torch.inf):
+        for expert in (0, E - 1):
+            router = torch.zeros(E, 64, device=DEV, dtype=torch.bfloat16)
+            router[:, 0] = rnd(E, seed=E)          # the column that x picks
+            router[expert, 0] = bad
+            w, row, pos, offs = ops.moe_route(x, router, 2)
+            want = torch.softmax(router[:, 0].float(), 0).topk(2).values
+            want /= want.sum()
+            assert torch.allclose(w[0], want, atol=1e-6, equal_nan=True)
+            assert sorted(pos.tolist()) == [0, 1] and offs[-1] == 2
+
+
 def test_moe_kernels_refuse_other_operands():
     x, router = rnd(5, 520, seed=1), rnd(8, 520, seed=2)
     for a, r, k in ((x, rnd(8, 512), 2), (x[:, :512].contiguous(), router, 2),
