@@ -240,7 +240,7 @@ class MoEMLP(nn.Module):
       touches essentially every expert anyway, so streaming all expert
       weights costs what exact dispatch costs — while every shape stays
       static: one grouped gate_up GEMM [T, E*2I], one fused SwiGLU over
-      [T*E, 2I], one batched down GEMM, one weighted sum."""
+      [T*E, 2I], the experts' down GEMMs, one weighted sum."""
 
     def __init__(self, cfg: LlamaConfig):
         super().__init__()
@@ -265,10 +265,16 @@ class MoEMLP(nn.Module):
             w.scatter_(1, topi, topv)
             gu = ops.linear(x, self.gate_up.reshape(E * I2, H))
             act = ops.silu_and_mul(gu.reshape(T * E, I2))
-            act = act.reshape(T, E, I2 // 2).transpose(0, 1)  # [E, T, I]
-            ye = torch.bmm(act, self.down.transpose(1, 2))    # [E, T, H]
-            out = (ye.float() * w.t().unsqueeze(-1)).sum(0)
-            return out.to(x.dtype)
+            act = act.reshape(T, E, I2 // 2)
+            if T <= ops.ROWS_MAX:
+                ye = torch.stack([ops.linear(act[:, e].contiguous(), self.down[e])
+                                  for e in range(E)])         # [E, T, H]
+                return (ye.float() * w.t().unsqueeze(-1)).sum(0).to(x.dtype)
+            # weights on the left: torch.bmm has faulted the GPU in bf16 with a
+            # transposed view on its right, which they would be
+            ye = torch.bmm(self.down, act.permute(1, 2, 0).contiguous())
+            out = (ye.float() * w.t().unsqueeze(1)).sum(0)    # [H, T]
+            return out.to(x.dtype).t().contiguous()
         out = torch.zeros(x.shape, dtype=torch.float32, device=x.device)
         for e in range(E):
             sel, slot = (topi == e).nonzero(as_tuple=True)

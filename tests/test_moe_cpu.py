@@ -59,6 +59,33 @@ def test_moe_static_dispatch_matches_exact():
         assert torch.allclose(static.float(), exact.float(), atol=1e-4),             (static - exact).abs().max()
 
 
+@pytest.mark.parametrize("T", [1, 16, 17, 33])
+def test_moe_static_dispatch_batches_no_transposed_view(T):
+    """torch.bmm in bf16 has faulted the GPU with a transposed view on its right:
+    the static dispatch hands it whole operands."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    seen = []
+
+    class Look(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            name = func.overloadpacket.__name__
+            if name in ("bmm", "baddbmm"):
+                assert args[-1].is_contiguous()
+            seen.append(name)
+            return func(*args, **(kwargs or {}))
+
+    cfg = CONFIGS["tiny-moe"]
+    mlp = MoEMLP(cfg)
+    with torch.no_grad():
+        for p in mlp.parameters():
+            p.normal_(0, 0.2)
+        x = torch.randn(T, cfg.hidden_size)
+        with Look():
+            got = mlp(x, static=True)
+        assert "mm" in seen and got.is_contiguous()
+        assert torch.allclose(got, mlp(x), atol=1e-4)
+
+
 def test_moe_router_uses_all_experts():
     cfg = CONFIGS["tiny-moe"]
     torch.manual_seed(1)
