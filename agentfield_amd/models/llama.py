@@ -299,11 +299,12 @@ class MoEMLP(nn.Module):
         xs = ops.gather_rows(x, row)
         ys = torch.empty_like(xs)
         bounds = offs.tolist()       # the one wait: block bounds
-        for e, (a, b) in enumerate(zip(bounds, bounds[1:])):
+        for a, b, gate_up, down in zip(bounds, bounds[1:], self.gate_up.unbind(),
+                                       self.down.unbind()):
             if a == b:
                 continue
-            act = ops.linear(xs[a:b], self.gate_up[e], silu_fuse=True)
-            ops.linear(act, self.down[e], out=ys[a:b])
+            act = ops.linear(xs[a:b], gate_up, silu_fuse=True)
+            ops.linear(act, down, out=ys[a:b])
         return ops.moe_combine(ys, pos, weights)
 
 
@@ -334,33 +335,35 @@ class LlamaLayer(nn.Module):
             h = self.mlp(h)
         return h, residual
 
-    def rows_weights_ok(self, cfg: LlamaConfig) -> bool:
-        """Whether forward_rows_fused can read this layer's weights."""
+    def rows_weights(self, cfg: LlamaConfig):
+        """(qkv, o, gate_up, down) if forward_rows_fused can read them."""
         at = self._modules["attn"]._parameters
         mlp = self._modules["mlp"]._parameters
-        qkv, o, gate_up, down = at["qkv"], at["o"], mlp["gate_up"], mlp["down"]
+        w = qkv, o, gate_up, down = at["qkv"], at["o"], mlp["gate_up"], mlp["down"]
         H, I, Q = cfg.hidden_size, cfg.intermediate_size, cfg.q_size
-        return (qkv.shape == (Q + 2 * cfg.kv_size, H) and o.shape == (H, Q)
+        if (qkv.shape == (Q + 2 * cfg.kv_size, H) and o.shape == (H, Q)
                 and gate_up.shape == (2 * I, H) and down.shape == (H, I)
-                and ops.rows_operands_ok((qkv, o, gate_up, down)))
+                and ops.rows_operands_ok(w)):
+            return w
+        return None
 
-    def forward_rows_fused(self, residual, ss, positions, rope_tab, kv, md):
+    def forward_rows_fused(self, weights, residual, ss, pos, rope_tab, kv, md):
         """Few-row path (decode steps, small prefill steps): norms, rotary
         positions, page append, SwiGLU and residual adds ride in the
         weight-streaming GEMMs, nothing runs on its own but attention.
         `residual` is updated in place; ss [T, 8] holds its rows' sums of
-        squares (None up to ops.ROWS_MAX rows, which need none).  The caller has
-        asked rows_weights_ok; the rows are made here."""
-        at, mlp = self.attn, self.mlp
-        q = ops.qkv_rope_rows(residual, at.qkv, self.eps, ss, positions,
-                              rope_tab, kv.k[at.layer_idx],
-                              kv.v[at.layer_idx], md.slots)
-        o = at.attention(q, kv, md)
+        squares (None up to ops.ROWS_MAX rows, which need none).  weights are
+        rows_weights', pos is ops.qkv_step's; the rows are made here."""
+        qkv, o, gate_up, down = weights
+        at, eps = self._modules["attn"], self.eps
+        i = at.layer_idx
+        q = ops.launch_qkv_rows(residual, qkv, eps, ss, pos, rope_tab, kv.k[i],
+                                kv.v[i], md.slots)
+        y = at.attention(q, kv, md)
         mode = 1 if ss is None else 4
-        ops.launch_rows(o, at.o, mode, residual, ss_out=ss, want_out=False)
-        act = ops.launch_rows(residual, mlp.gate_up, 2, scale=(ss, self.eps))
-        ops.launch_rows(act, mlp.down, mode, residual, ss_out=ss,
-                        want_out=False)
+        ops.launch_rows(y, o, mode, residual, ss_out=ss, want_out=False)
+        act = ops.launch_rows(residual, gate_up, 2, scale=(ss, eps))
+        ops.launch_rows(act, down, mode, residual, ss_out=ss, want_out=False)
 
 
 class LlamaForCausalLM(nn.Module):
@@ -448,9 +451,12 @@ class LlamaForCausalLM(nn.Module):
             ss = (torch.empty(T, 8, dtype=torch.float32, device=ids.device)
                   if T > ops.ROWS_MAX else None)
             residual = ops.embedding(ids, self.embed, ss=ss)
+            pos = ops.qkv_step(T, self.cfg.head_dim, positions, self.rope_tab,
+                               md.slots)
             for layer in self.layers:
-                if layer.rows_weights_ok(self.cfg):
-                    layer.forward_rows_fused(residual, ss, positions,
+                weights = layer.rows_weights(self.cfg)
+                if weights is not None:
+                    layer.forward_rows_fused(weights, residual, ss, pos,
                                              self.rope_tab, kv, md)
                     continue
                 h, _ = layer(residual, None, positions, self.rope_tab, kv, md)

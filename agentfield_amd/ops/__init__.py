@@ -381,7 +381,7 @@ def linear_rows(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
 
 
 def launch_rows(x, w, mode=0, residual=None, scale=None, ss_out=None,
-                 want_out=True, out=None):
+                want_out=True, out=None):
     """linear_rows for callers that have checked the operands, or made them."""
     M, K = x.shape
     N = w.shape[0]
@@ -420,22 +420,38 @@ def qkv_rope_rows(x: torch.Tensor, w: torch.Tensor, eps: float,
     if not _rows_ok(x, w):
         raise AfOpsError(f"QKV rows: {tuple(x.shape)} {x.dtype} rows against "
                          f"{tuple(w.shape)} {w.dtype} weights")
-    M, K = x.shape
-    _, Hk, page, D = kcache.shape
-    N = w.shape[0]
-    Hq = N // D - 2 * Hk
-    _need(Hq > 0 and N == (Hq + 2 * Hk) * D and table.shape[1] == D
-          and table.dtype == torch.float32 and table.is_contiguous(),
+    M, N, (_, Hk, _, D) = x.shape[0], w.shape[0], kcache.shape
+    _need(N // D - 2 * Hk > 0 and N % D == 0,
           f"QKV rows: {N} outputs for {Hk} K/V heads of {D}")
-    _need(kcache.shape == vcache.shape and kcache.dtype == vcache.dtype == x.dtype
-          and kcache.is_contiguous() and vcache.is_contiguous(),
-          "QKV rows: pages must be whole and of x's type")
+    _need(M <= ROWS_MAX or _row_stats(ss, x), "QKV rows: sums of the rows")
+    pos = qkv_step(M, D, positions, table, slots)
+    return launch_qkv_rows(x, w, eps, ss, pos, table, kcache, vcache, slots)
+
+
+def qkv_step(M: int, D: int, positions: torch.Tensor, table: torch.Tensor,
+             slots: torch.Tensor) -> torch.Tensor:
+    """What the QKV rows of all layers of a step share, checked once: int32
+    positions of M rows."""
+    _need(table.shape[1] == D and table.dtype == torch.float32
+          and table.is_contiguous(), f"QKV rows: rotary table for heads of {D}")
     _need(positions.numel() == M and slots.numel() == M
           and slots.dtype == torch.int64 and slots.is_contiguous(),
           f"QKV rows: positions and int64 slots of {M} rows")
-    _need(M <= ROWS_MAX or _row_stats(ss, x), "QKV rows: sums of the rows")
+    return positions.int().contiguous()
+
+
+def launch_qkv_rows(x, w, eps, ss, pos, table, kcache, vcache, slots):
+    """qkv_rope_rows for callers that have checked the rows and weights, or made
+    them, and have pos from qkv_step; the pages are looked at here."""
+    M, K = x.shape
+    pages = kcache.shape
+    _, Hk, page, D = pages
+    _need(pages == vcache.shape and kcache.dtype is vcache.dtype is x.dtype
+          and kcache.is_contiguous() and vcache.is_contiguous(),
+          "QKV rows: pages must be whole and of x's type")
+    N = w.shape[0]
+    Hq = N // D - 2 * Hk
     q = torch.empty(M, Hq * D, dtype=x.dtype, device=x.device)
-    pos = positions.int().contiguous()
     splits, parts = 1, None
     if M > ROWS_MAX:
         splits = rows_splits(M, N, K)

@@ -68,19 +68,19 @@ def test_few_row_path_needs_plain_bf16_weights():
     layer = m.layers[1]
     for part, name in (("attn", "qkv"), ("attn", "o"), ("mlp", "gate_up"),
                        ("mlp", "down")):
-        assert layer.rows_weights_ok(m.cfg)
+        assert layer.rows_weights(m.cfg) is not None
         p = getattr(getattr(layer, part), name)
         flat = p.data.clone()
         p.data = flat.t().contiguous().t()          # strided
-        assert not layer.rows_weights_ok(m.cfg)
+        assert layer.rows_weights(m.cfg) is None
         p.data = torch.cat([flat.flatten()[:1], flat.flatten()])[1:].view_as(
             flat)                                   # off the 16-byte grid
-        assert not layer.rows_weights_ok(m.cfg)
+        assert layer.rows_weights(m.cfg) is None
         p.data = flat[:-64]                         # of another size
-        assert not layer.rows_weights_ok(m.cfg)
+        assert layer.rows_weights(m.cfg) is None
         p.data = flat
     p.data = flat.float()
-    assert not layer.rows_weights_ok(m.cfg)
+    assert layer.rows_weights(m.cfg) is None
 
 
 def test_watched_products():
