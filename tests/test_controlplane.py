@@ -971,38 +971,54 @@ def test_engine_metrics_ride_heartbeats():
     srv.stop()
 
 
-def _open_at(path, keys, go, out):
-    from agentfield_amd.controlplane.did import DIDService, Keystore
-    from agentfield_amd.controlplane.storage import Storage
+_OPEN_PLANES = """
+import json, sys, time
+from agentfield_amd.controlplane.did import DIDService, Keystore
+from agentfield_amd.controlplane.storage import Storage
+print("ready", flush=True)
+for line in sys.stdin:
+    go, path, keys = json.loads(line)
     while time.time() < go:
         pass
     try:
         dids = DIDService(Storage(path), Keystore(keys))
-        out.put((dids.root_did, dids.keystore.seed.hex()))
+        got = [dids.root_did, dids.keystore.seed.hex()]
     except Exception as e:
-        out.put(repr(e))
+        got = repr(e)
+    print(json.dumps(got), flush=True)
+"""
 
 
 def test_workers_open_a_new_plane_at_the_same_moment(tmp_path):
     """Workers of one plane start together: each must get through the new
     database's switch to WAL mode, and all must end up with one root identity
     (one of four used to fail here in every second round)."""
-    import multiprocessing as mp
-    ctx = mp.get_context("fork")
-    for n in range(15):
-        d = tmp_path / str(n)
-        out, go = ctx.Queue(), time.time() + 0.05
-        procs = [ctx.Process(target=_open_at, args=(
-            str(d / "af.db"), str(d / "keystore.key"), go, out))
-            for _ in range(4)]
+    import subprocess
+    import sys
+    from pathlib import Path
+    procs = [subprocess.Popen(
+        [sys.executable, "-c", _OPEN_PLANES], text=True, stdin=subprocess.PIPE,
+        stdout=subprocess.PIPE, cwd=Path(__file__).resolve().parents[1])
+        for _ in range(4)]
+    try:
         for p in procs:
-            p.start()
-        got = [out.get(timeout=30) for _ in procs]
+            assert p.stdout.readline() == "ready\n"
+        for n in range(15):
+            d = tmp_path / str(n)
+            order = json.dumps([time.time() + 0.02, str(d / "af.db"),
+                                str(d / "keystore.key")])
+            for p in procs:
+                p.stdin.write(order + "\n")
+                p.stdin.flush()
+            got = [json.loads(p.stdout.readline()) for p in procs]
+            assert all(g == got[0] for g in got) and len(got[0]) == 2, got
+            assert (d / "keystore.key").stat().st_mode & 0o777 == 0o600
+            assert [f.name for f in d.glob("keystore*")] == ["keystore.key"]
+    finally:
         for p in procs:
-            p.join()
-        assert len(set(got)) == 1 and isinstance(got[0], tuple), got
-        assert (d / "keystore.key").stat().st_mode & 0o777 == 0o600
-        assert sorted(f.name for f in d.glob("keystore*")) == ["keystore.key"]
+            p.stdin.close()
+            p.stdout.close()
+            p.wait(timeout=30)
 
 
 def test_benchmark_says_why_a_server_is_not_up(tmp_path):
