@@ -290,12 +290,13 @@ class MoEMLP(nn.Module):
     def _can_sort(self, x) -> bool:
         """Rows that the routing kernels take (the loop serves the rest, and
         anything that autograd has to see)."""
-        return (x.is_cuda and not ops.watched(x, self.router, self.gate_up,
-                                              self.down)
-                and ops.moe_route_ok(x, self.router, self.top_k))
+        router = self.router
+        return (x.is_cuda and not ops.watched(x, router, self.gate_up, self.down)
+                and ops.moe_route_ok(x, router, self.top_k))
 
     def _forward_sorted(self, x):
-        weights, row, pos, offs = ops.moe_route(x, self.router, self.top_k)
+        weights, row, pos, offs = ops.launch_moe_route(x, self.router,
+                                                       self.top_k)
         xs = ops.gather_rows(x, row)
         ys = torch.empty_like(xs)
         bounds = offs.tolist()       # the one wait: block bounds

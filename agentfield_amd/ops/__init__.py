@@ -524,15 +524,14 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
     28672 x 4096 53.9 / 41.5, 64.0 / 42.1, 56.7 / 51.7; 128256 x 4096 190 / 151
     at one row, 214 / 184 at 64, 238 / 215 at 128.  Between 12288 and 24576
     these two were measured; the limits are the nearest sizes at which rows win."""
-    M, _K = x.shape
-    N = w.shape[0]
-    if out is not None:
-        _need(not silu_fuse and tuple(out.shape) == (M, N),
-              f"linear: out {tuple(out.shape)} for a [{M}, {N}] product")
-    if (x.is_cuda and not watched(x, w, grad=not silu_fuse)
+    M, N = x.shape[0], w.shape[0]
+    if out is not None and (silu_fuse or out.shape != (M, N)):
+        raise AfOpsError(f"linear: out {tuple(out.shape)} for a [{M}, {N}] "
+                         "product")
+    if (M <= 128 and (silu_fuse or M <= 32 or N <= 12288 or N >= 24576)
+            and x.is_cuda and not watched(x, w, grad=not silu_fuse)
             and (out is None or _whole(out, x, M, N) and _apart(out, x))
-            and _rows_ok(x, w)
-            and (silu_fuse or M <= 32 or N <= 12288 or N >= 24576)):
+            and _rows_ok(x, w)):
         return launch_rows(x, w, 2 if silu_fuse else 0, out=out)
     if out is not None:
         return torch.mm(x, w.t(), out=out)
@@ -562,8 +561,14 @@ def moe_route(x: torch.Tensor, router: torch.Tensor, k: int):
     largest renormalised, and the (row, choice) entries sorted by expert:
     (weights [T, k] f32, row [T*k] i32 of every sorted position, sorted position
     [T*k] i32 of every entry, first position of every expert [E+1] i32)."""
-    _need(moe_route_ok(x, router, k),
-          f"routing {tuple(x.shape)} rows over {tuple(router.shape)}, k {k}")
+    if not moe_route_ok(x, router, k):
+        raise AfOpsError(f"routing {tuple(x.shape)} rows over "
+                         f"{tuple(router.shape)}, k {k}")
+    return launch_moe_route(x, router, k)
+
+
+def launch_moe_route(x, router, k):
+    """moe_route for callers that have asked moe_route_ok."""
     T, H = x.shape
     E = router.shape[0]
     dev = x.device
@@ -584,12 +589,13 @@ def moe_combine(y: torch.Tensor, pos: torch.Tensor,
     """out[t] = sum_j weights[t, j] * y[pos[t*k + j]] over the sorted expert rows."""
     T, k = weights.shape
     H = y.shape[1]
-    _need(y.is_cuda and y.shape[0] == T * k and H % 8 == 0
-          and rows_operands_ok((y,)) and weights.dtype == torch.float32
-          and weights.is_contiguous() and weights.device == y.device
-          and pos.numel() == T * k and pos.dtype == torch.int32
-          and pos.is_contiguous() and pos.device == y.device,
-          f"combining {tuple(y.shape)} rows by {tuple(weights.shape)} weights")
+    if not (y.is_cuda and y.shape[0] == T * k and H % 8 == 0
+            and rows_operands_ok((y,)) and weights.dtype == torch.float32
+            and weights.is_contiguous() and weights.device == y.device
+            and pos.numel() == T * k and pos.dtype == torch.int32
+            and pos.is_contiguous() and pos.device == y.device):
+        raise AfOpsError(f"combining {tuple(y.shape)} rows by "
+                         f"{tuple(weights.shape)} weights")
     out = torch.empty(T, H, dtype=y.dtype, device=y.device)
     rc = _lib.lib().af_moe_combine(
         _lib.ptr(out), _lib.ptr(y), _lib.ptr(pos), _lib.ptr(weights), T, H, k,
