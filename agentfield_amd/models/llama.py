@@ -338,9 +338,13 @@ class LlamaLayer(nn.Module):
 
     def rows_weights(self, cfg: LlamaConfig):
         """(qkv, o, gate_up, down) if forward_rows_fused can read them."""
-        at = self._modules["attn"]._parameters
-        mlp = self._modules["mlp"]._parameters
-        w = qkv, o, gate_up, down = at["qkv"], at["o"], mlp["gate_up"], mlp["down"]
+        at, mlp = self._modules["attn"], self._modules["mlp"]
+        try:
+            a, b = at._parameters, mlp._parameters
+            w = a["qkv"], a["o"], b["gate_up"], b["down"]
+        except KeyError:        # parametrized, or not parameters
+            w = at.qkv, at.o, mlp.gate_up, mlp.down
+        qkv, o, gate_up, down = w
         H, I, Q = cfg.hidden_size, cfg.intermediate_size, cfg.q_size
         if (qkv.shape == (Q + 2 * cfg.kv_size, H) and o.shape == (H, Q)
                 and gate_up.shape == (2 * I, H) and down.shape == (H, I)

@@ -81,6 +81,11 @@ def test_few_row_path_needs_plain_bf16_weights():
         p.data = flat
     p.data = flat.float()
     assert layer.rows_weights(m.cfg) is None
+    p.data = flat
+    torch.nn.utils.parametrize.register_parametrization(
+        layer.mlp, "down", torch.nn.Identity())
+    with torch.no_grad():
+        assert torch.equal(layer.rows_weights(m.cfg)[3], flat)
 
 
 def test_watched_products():
