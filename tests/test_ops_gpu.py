@@ -746,6 +746,34 @@ def test_row_products_under_autograd(M, N):
         assert near(v[1], 2 * (x.float() @ w.float().t()))
 
 
+@pytest.mark.parametrize("T", [1, 16, 17, 64, 130])
+def test_moe_static_dispatch(T):
+    """The mixture layer's decode form, both ways to multiply by the experts'
+    down weights, eager and as a replayed graph, against its prompt form.  1%:
+    both round each expert's activations and products to bf16."""
+    from agentfield_amd.models import CONFIGS
+    from agentfield_amd.models.llama import MoEMLP
+    mlp = MoEMLP(CONFIGS["tiny-moe"]).to(DEV, torch.bfloat16)
+    for i, p in enumerate(mlp.parameters()):
+        p.data.copy_(rnd(*p.shape, seed=20 + i, scale=0.05))
+    x = rnd(T, 256, seed=4)
+    with torch.inference_mode():
+        want = [mlp(x), mlp(2 * x), mlp(-x)]
+        buf = x.clone()
+        mlp(buf, static=True)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = mlp(buf, static=True)
+        for f, w in zip((1, 2, -1), want):
+            buf.copy_(f * x)
+            graph.replay()
+            eager = mlp(buf, static=True)
+            torch.cuda.synchronize()
+            assert got.is_contiguous() and torch.equal(got, eager)
+            assert (got - w).float().norm() <= 1e-2 * w.float().norm()
+
+
 @pytest.mark.parametrize("T", [3, 100])
 def test_moe_dispatch_under_autograd(T):
     """The mixture layer's exact dispatch leaves weight gradients where its loop
