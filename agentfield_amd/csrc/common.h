@@ -20,6 +20,7 @@ typedef __attribute__((ext_vector_type(2))) short s16x2;
 typedef __attribute__((ext_vector_type(4))) short s16x4;
 typedef __attribute__((ext_vector_type(8))) short s16x8;  // 8 bf16 = 16 B
 typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
+typedef __attribute__((ext_vector_type(4))) unsigned short u16x4;
 
 // ---- bf16 <-> fp32 (round-to-nearest-even, matches torch semantics) ----
 __device__ __forceinline__ float bf2f(u16 v) {

@@ -8,10 +8,9 @@
 // instruction) stop at ~7.6 TB/s of requests whatever is asked for, so X at 16
 // rows doubled the time.  16-byte chunks are permuted within a line by the row
 // number (the operand reads then do not meet in a bank).  Waits are counted, so that
-// the loads of the next pieces stay in flight while one is multiplied.  That holds
-// for gemm_tile_kernel and for gemm_rows_kernel without a norm scalar (o, down); in
-// its variants with one (qkv, gate/up) the compiler adds a full wait in front of the
-// operand reads, so everything a wave has asked for ahead has to land there first.
+// the loads of the next pieces stay in flight while one is multiplied.  All LDS of a
+// kernel is one array: with a second one the compiler puts a full wait in front of
+// the operand reads (SwiGLU over 28672 x 4096, one row: 38.7 us, 36.0 without it).
 //
 // gemm_rows_kernel, up to 16 rows: a block owns one tile of 16 weight rows (N =
 //   4096 gives 256 tiles, one per CU; N = 28672 seven per CU) and K is split over
@@ -23,15 +22,28 @@
 //   tile is 8 rotation pairs of a head).  RMSNorm (its weight is folded into W):
 //   the loop multiplies every X fragment with itself (diagonal of X X^T, one
 //   MFMA), so nobody has to leave row statistics behind.
-// gemm_tile_kernel, more rows: X would be read once per 16 weight rows, so here
-//   four or eight waves share 64 or 128 weight rows and X, STAGES pieces in a ring
-//   with one barrier per piece.  A wave multiplies WT tiles of weights with a WT-th
-//   of X's rows: with WT = 1 every wave reads all of X from LDS, 144 KB per piece
-//   at 128 rows, more cycles than the memory takes to deliver the piece; WT = 4
-//   reads 96 KB (SwiGLU at 128 rows 57.3 -> 52.3 us, 4096 x 14336 28.4 -> 27.7,
-//   both before the weights were streamed).
-//   K is split over blocks where N alone does not fill the chip, the fp32 parts
-//   meet in the kernel that does the next step.
+// More rows: X would be read once per 16 weight rows, so here four or eight waves
+//   share 64 or 128 weight rows and X, STAGES pieces in a ring with one barrier per
+//   piece.
+// gemm_parts_kernel, K split over blocks because N alone does not fill the chip: a
+//   wave multiplies WT tiles of weights with a WT-th of X's rows (with WT = 1 every
+//   wave reads all of X from LDS, 144 KB per piece at 128 rows; WT = 4 reads 96 KB).
+//   The fp32 parts meet in the kernel that does the next step.  Bound by the parts
+//   (16.8 MB at 128 rows, written at ~2.5 TB/s after the stream has ended: 7 of the 15
+//   us of 4096 x 4096) and by starts, not by its loop: the loop below was no faster.
+// gemm_tile_kernel, whole K (SwiGLU, plain): at 128 rows the loop of the kernel above
+//   takes 0.47 us per piece without any load, nearly what the memory needs for the
+//   128 weight rows of a piece (0.57), and the two did not overlap.  So half of the
+//   waves take one half of a piece's K and half the other, each 64 weight rows by a
+//   half of X's rows (64 KB of LDS reads per piece instead of 96), and the operands
+//   of the next piece are read while one is multiplied: 0.2 us.  Rows of weights are
+//   the first MFMA operand, so that a lane ends with four neighbouring columns of a
+//   row; the norm scalars are made while the first pieces travel.  The epilogue takes
+//   3 us instead of 8 of the 50.
+//   SwiGLU over 28672 x 4096, alone / inside a step: 24 rows 40.1 -> 36.9, 64 rows
+//   41.4 -> 38.9 / 44.2 -> 42.0, 80 rows (96 brought in instead of 128) 46.9 -> 41.8 /
+//   51.7 -> 43.8, 128 rows 50.3 -> 48.0 / 57.2 -> 52.6; 16384 x 2048 at 128 rows 24.5 ->
+//   19.6.  Deeper rings, in all or for the weights only, change nothing.
 //
 // Weight rows lie K * 2 bytes apart, usually a multiple of every channel
 // interleave, so the rows of one piece come from the same memory channel and
@@ -39,21 +51,22 @@
 // XCD therefore start at different pieces; where K is split the splits do that
 // already and starting elsewhere costs a little (4096 x 4096 in four, 32 rows: 8.0 ->
 // 8.8 us).  SwiGLU over 28672 x 4096: 42.9 -> 40.2 us at one row, 53.4 -> 45.2 at 64,
-// 62.3 -> 57.3 at 128 (before the weights were streamed).  Four pieces per wave
-// instead of two, which need half the CU's buffers, were slower (50.5 us), but that
-// was measured on the variant whose loads are drained.
+// 62.3 -> 57.3 at 128 (before the weights were streamed).  Two pieces per wave leave
+// room for two blocks per CU, whose starts and ends overlap; three pieces with 8 rows
+// of X each 36.4, four 43.7 (one block per CU).
 // The order in which a column is summed depends on the kernel, the width of its
 // blocks and the number of splits, and all three on M: the same row may differ by
 // fp32 rounding between steps of different sizes.
-// Measured in us, alone and repeated (inside a step 5-25% more: 64 rows 13.8, 9.7,
-// 23.1, 41.9), against the split-K kernel with two-stage buffers and its second launch
-// (in brackets).  One row: 6144 x 4096 with rotary and append 10.7 (21.3 in
-// three launches), 4096 x 4096 7.3 and 4096 x 14336 19.0 (together 44.4), SwiGLU
-// over 28672 x 4096 37.5 = 6.3 TB/s (58.2).  16 rows: 13.1, 8.1, 23.1, 42.6.  64
-// rows, without the closing launches: 11.2, 8.5, 21.7, 40.1 (16.7, o + down 44.8,
-// 62.7).  128 rows: 14.3, 12.6, 26.8, 50.0 (library 25.6 and 57.5 + 5.2 for the
-// first and the last, o + down 63.1).
+// Measured in us, alone and repeated (inside a step 5-25% more), against the split-K
+// kernel with two-stage buffers and its second launch (in brackets).  One row: 6144 x
+// 4096 with rotary and append 11.4 (21.3 in three launches), 4096 x 4096 7.2 and 4096 x
+// 14336 19.5 (together 44.4), SwiGLU over 28672 x 4096 36.0 = 6.5 TB/s (58.2).  16
+// rows: 13.3, 8.0, 23.3, 41.2.  64 rows, without the closing launches: 13.1, 9.3,
+// 23.3, 38.9 (16.7, o + down 44.8, 62.7).  128 rows: 16.9, 15.0, 27.5, 48.0 (library
+// 25.6 and 57.5 + 5.2 for the first and the last, o + down 63.1).
 #include "common.h"
+
+#include <type_traits>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8r;
 typedef __attribute__((address_space(3))) char lds_b;
@@ -96,6 +109,9 @@ __device__ __forceinline__ void load_line8(const u16* src, lds_b* dst) {
       (__attribute__((address_space(3))) uint32_t*)dst, 16, 0, AUX);
 }
 constexpr int STREAM = 2, KEEP = 0;   // AUX: nontemporal, cached
+
+// s_waitcnt operand: all but n of a wave's vector loads have landed
+constexpr int vmcnt_only(int n) { return (n & 15) | (n >> 4) << 14 | 0x0f70; }
 
 // operand fragment: lane (r = lane & 15, q = lane >> 4) gets k = 32 h + 8 q .. +8
 // of row r of a 16-row piece
@@ -161,9 +177,10 @@ __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
   constexpr int RS = 20;                         // column stride of the sums
   constexpr int RING = NW * PD * SLOT;
   constexpr int SUMS = NW * 16 * RS * 4;
-  __shared__ __attribute__((aligned(16))) char lds[RING > SUMS ? RING : SUMS];
-  __shared__ float rsq[NW][16];
-  __shared__ float rstd[16];
+  // one array for everything: with a second one the compiler waits for all loads
+  // in front of the loop's reads
+  constexpr int TAIL = SUMS + (NW + 1) * 16 * 4;
+  __shared__ __attribute__((aligned(16))) char lds[RING > TAIL ? RING : TAIL];
   lds_b* ring = (lds_b*)&lds[wid * PD * SLOT];
 
   // sources of this lane's chunks
@@ -192,12 +209,11 @@ __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
     if (s < cnt) load(s);
   for (int i = 0; i < cnt; ++i) {
     // piece i has landed when only the loads of the PD - 1 behind it are out
-    static_assert(PD == 2, "wait count");
-    if (i + PD <= cnt) {
-      asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
+    if (i + PD <= cnt)
+      __builtin_amdgcn_s_waitcnt(vmcnt_only(4 * (PD - 1)));
+    else
+      __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
+    asm volatile("" ::: "memory");
     const lds_b* at = ring + (i % PD) * SLOT;
     bf16x8r w[2], x[2];
 #pragma unroll
@@ -219,6 +235,8 @@ __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
   // meet in LDS: [wave][tile column][row]; + 4 spreads the columns over banks
   __syncthreads();
   float (*red)[16][RS] = reinterpret_cast<float (*)[16][RS]>(lds);
+  float (*rsq)[16] = reinterpret_cast<float (*)[16]>(lds + SUMS);
+  float* rstd = rsq[NW];
   *reinterpret_cast<f32x4*>(&red[wid][n][(lane >> 4) * 4]) = acc;
   if (NORM == 2) {
 #pragma unroll
@@ -291,10 +309,10 @@ __device__ __forceinline__ void wait_loads_and_meet() {
     asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// MT 16-row groups of X (even), ring of STAGES pieces of K = 64.  Grid
-// (N / (16 NW), splits).  EPI_PLAIN, EPI_SWIGLU (not split) or EPI_PARTS.
-template <int MT, int NW, int WT, int STAGES, int EPI, int NORM, int AUX>
-__global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
+// Split K: MT 16-row groups of X (even), ring of STAGES pieces of K = 64, the sums to
+// the parts.  Grid (N / (16 NW), splits).
+template <int MT, int NW, int WT, int STAGES, int AUX>
+__global__ void __launch_bounds__(64 * NW) gemm_parts_kernel(RowsArgs a) {
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int n = lane & 15;
@@ -316,7 +334,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
   const u16* xp[XG];
 #pragma unroll
   for (int g = 0; g < 2; ++g)
-    wp[g] = a.W + (size_t)weight_row<EPI>(a, tile, g * 8 + r8) * a.K + ch;
+    wp[g] = a.W + (size_t)weight_row<EPI_PARTS>(a, tile, g * 8 + r8) * a.K + ch;
 #pragma unroll
   for (int g = 0; g < XG; ++g)
     xp[g] = a.X + (size_t)min((wid * XG + g) * 8 + r8, a.M - 1) * a.K + ch;
@@ -370,32 +388,199 @@ __global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = (m0 + m) * 16 + (lane >> 4) * 4 + r;
-      float rstd = 1.f;
-      if (NORM == 1) {
-        const float* sp = a.ss + min(row, a.M - 1) * 8;
-        float s = 0.f;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) s += sp[j];
-        rstd = rsqrtf(s * (1.f / (float)a.K) + a.eps);
+      for (int t = 0; t < WT; ++t)
+        if (row < a.M)
+          a.parts[((size_t)blockIdx.y * a.M + row) * a.N +
+                  (blockIdx.x * NW + w0 + t) * 16 + n] = acc[t][m][r];
+    }
+}
+
+// All but n groups of PER of a wave's loads have landed (n <= 4), its LDS reads are
+// done, and so it is for every wave of the block.  By builtins: the compiler has to
+// know that the operands are there, or it waits for the next ones as well.
+template <int PER>
+__device__ __forceinline__ void meet(int n) {
+  asm volatile("" ::: "memory");
+  if (n >= 4) __builtin_amdgcn_s_waitcnt(vmcnt_only(4 * PER) & ~0x0f00);
+  else if (n == 3) __builtin_amdgcn_s_waitcnt(vmcnt_only(3 * PER) & ~0x0f00);
+  else if (n == 2) __builtin_amdgcn_s_waitcnt(vmcnt_only(2 * PER) & ~0x0f00);
+  else if (n == 1) __builtin_amdgcn_s_waitcnt(vmcnt_only(PER) & ~0x0f00);
+  else __builtin_amdgcn_s_waitcnt(vmcnt_only(0) & ~0x0f00);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Whole K: MT 16-row groups of X (even), NT 16-row tiles of weights (4 or 8), NW
+// waves, a ring of STAGES pieces of K = 64.  Grid N / (16 NT).  EPI_PLAIN, EPI_SWIGLU.
+template <int MT, int NT, int NW, int STAGES, int EPI, int NORM, int AUX>
+__global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int n = lane & 15;
+  constexpr int PIECE = 2048;
+  constexpr int STAGE = PIECE * (NT + MT);
+  constexpr int WG = 2 * NT / NW;                // 8-row lines of W per wave
+  constexpr int XH = 4 * MT / NW;                // 4-row half lines of X per wave
+  constexpr int XG = (XH + 1) / 2;               // X loads, the last may be a half
+  constexpr int PER = WG + XG;                   // loads per wave and stage
+  constexpr int RP = NW / 2 / (NT / 4);          // parts of X's groups
+  constexpr int MW = MT / RP;                    // X groups of a wave's products
+  static_assert(WG * NW == 2 * NT && XH * NW == 4 * MT && MW * RP == MT, "shares");
+  static_assert(NW * 2 * MW * 1024 <= STAGES * STAGE, "half of the sums fit");
+  static_assert(STAGES >= 2 && STAGES <= 6 && PER * 4 < 64, "wait counts");
+  // one array for everything: with a second one the compiler waits for all loads
+  // in front of the loop's reads
+  __shared__ __attribute__((aligned(16))) char lds[STAGES * STAGE + MT * 64];
+  lds_b* const ring = (lds_b*)&lds[0];
+  float* const rstd = reinterpret_cast<float*>(lds + STAGES * STAGE);
+
+  const int cnt = a.K >> 6;
+  const int r8 = lane >> 3;
+  const u16* wp[WG];
+  const u16* xp[XG];
+#pragma unroll
+  for (int g = 0; g < WG; ++g) {
+    const int line = wid * WG + g;
+    wp[g] = a.W + (size_t)weight_row<EPI>(a, blockIdx.x * NT + line / 2,
+                                          (line & 1) * 8 + r8) * a.K +
+            ((lane & 7) ^ r8) * 8;
+  }
+#pragma unroll
+  for (int g = 0; g < XG; ++g) {
+    const int row = wid * XH * 4 + g * 8 + r8;
+    xp[g] = a.X + (size_t)min(row, a.M - 1) * a.K + ((lane & 7) ^ (row & 7)) * 8;
+  }
+  // the piece and slot to load next
+  int pnext = ((int)blockIdx.x >> 3) * 2 % cnt, snext = 0;
+  auto load = [&]() {
+    lds_b* to = ring + snext * STAGE;
+    const int off = pnext * 64;
+#pragma unroll
+    for (int g = 0; g < WG; ++g)
+      load_line8<AUX>(wp[g] + off, to + (wid * WG + g) * 1024);
+#pragma unroll
+    for (int g = 0; g < XG; ++g)
+      if (2 * g + 2 <= XH || lane < 32)
+        load_line8<KEEP>(xp[g] + off, to + NT * PIECE + wid * XH * 512 + g * 1024);
+    pnext = pnext + 1 == cnt ? 0 : pnext + 1;
+    snext = snext + 1 == STAGES ? 0 : snext + 1;
+  };
+  // products: a half of every piece's K, 4 tiles of weights, a part of X's groups
+  const int kh = wid / (NW / 2), role = wid % (NW / 2);
+  const int w0 = role / RP * 4, m0 = role % RP * MW;
+  f32x4 acc[4][MW];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int m = 0; m < MW; ++m) acc[t][m] = f32x4{0, 0, 0, 0};
+  int slot = 0;                                  // of the piece to read next
+  auto read = [&](bf16x8r (&w)[4], bf16x8r (&x)[MW]) {
+    const lds_b* at = ring + slot * STAGE;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) w[t] = frag(at + (w0 + t) * PIECE, kh);
+#pragma unroll
+    for (int m = 0; m < MW; ++m) x[m] = frag(at + (NT + m0 + m) * PIECE, kh);
+    slot = slot + 1 == STAGES ? 0 : slot + 1;
+  };
+  // piece i + 1 is complete for everybody, and piece i read by everybody: its slot
+  // is filled again, and while i is multiplied the operands of i + 1 are read
+  auto step = [&](int i, const bf16x8r (&w)[4], const bf16x8r (&x)[MW],
+                  bf16x8r (&wn)[4], bf16x8r (&xn)[MW]) {
+    if (i + 1 < cnt) {
+      meet<PER>(min(STAGES - 2, cnt - 2 - i));
+      if (i + STAGES < cnt) load();
+      read(wn, xn);
+    } else {
+      __builtin_amdgcn_s_waitcnt(vmcnt_only(0) & ~0x0f00);
+    }
+#pragma unroll
+    for (int m = 0; m < MW; ++m)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        acc[t][m] =
+            __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t], x[m], acc[t][m], 0, 0, 0);
+  };
+#pragma unroll 1
+  for (int s = 0; s < min(STAGES, cnt); ++s) load();
+  if (NORM == 1) {
+    const int row = threadIdx.x;
+    if (row < MT * 16) {
+      const float* sp = a.ss + (size_t)min(row, a.M - 1) * 8;
+      float s = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s += sp[j];
+      rstd[row] = rsqrtf(s * (1.f / (float)a.K) + a.eps);
+    }
+  }
+  bf16x8r wa[4], xa[MW], wb[4], xb[MW];
+  meet<PER>(min(STAGES, cnt) - 1);
+  read(wa, xa);
+#pragma unroll 1
+  for (int i = 0; i < cnt; i += 2) {
+    step(i, wa, xa, wb, xb);
+    if (i + 1 < cnt) step(i + 1, wb, xb, wa, xa);
+  }
+
+  // the two waves of a product swap sums: each finishes two of its tiles
+  __syncthreads();
+  f32x4* give = reinterpret_cast<f32x4*>(lds) + (wid * 2 * MW) * 64 + lane;
+  const f32x4* take = reinterpret_cast<const f32x4*>(lds) +
+                      ((wid ^ (NW / 2)) * 2 * MW) * 64 + lane;
+  f32x4 sum[2][MW];
+  auto swap = [&](auto upper) {
+    constexpr int U = decltype(upper)::value;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int m = 0; m < MW; ++m) {
+        give[(t * MW + m) * 64] = acc[2 - 2 * U + t][m];
+        sum[t][m] = acc[2 * U + t][m];
       }
+  };
+  if (kh == 0) swap(std::integral_constant<int, 0>{});
+  else swap(std::integral_constant<int, 1>{});
+  __syncthreads();
 #pragma unroll
-      for (int t = 0; t < WT; ++t) {
-        const int c = (blockIdx.x * NW + w0 + t) * 16;  // first column of the tile
-        const float v = NORM == 1 ? acc[t][m][r] * rstd : acc[t][m][r];
-        if (EPI == EPI_PARTS) {
-          if (row < a.M)
-            a.parts[((size_t)blockIdx.y * a.M + row) * a.N + c + n] = v;
-        } else if (EPI == EPI_SWIGLU) {
-          const float u = __int_as_float(__builtin_amdgcn_update_dpp(
-              0, __float_as_int(v), 0x128, 0xf, 0xf, true));  // row_ror:8
-          if (n < 8 && row < a.M)
-            a.out[(size_t)row * (a.N >> 1) + c / 2 + n] =
-                f2bf(v / (1.f + __expf(-v)) * u);
-        } else if (row < a.M) {
-          a.out[(size_t)row * a.N + c + n] = f2bf(v);
-        }
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int m = 0; m < MW; ++m) sum[t][m] += take[(t * MW + m) * 64];
+
+  // lane: row n of each group, columns (lane >> 4) * 4 .. + 4 of each tile
+  const int tile = blockIdx.x * NT + w0 + kh * 2;
+#pragma unroll
+  for (int m = 0; m < MW; ++m) {
+    const int row = (m0 + m) * 16 + n;
+    if (NORM == 1) {
+      const float f = rstd[row];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) sum[t][m] *= f;
+    }
+    if (EPI == EPI_SWIGLU) {
+      // gate rows lie in the lower lanes and up rows in the upper ones: the lower
+      // lanes get both of the first tile, the upper ones both of the second
+      u16x4 o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const auto gu = __builtin_amdgcn_permlane32_swap(
+            __float_as_uint(sum[0][m][r]), __float_as_uint(sum[1][m][r]), false, false);
+        const float v = __uint_as_float(gu[0]), u = __uint_as_float(gu[1]);
+        o[r] = f2bf(v / (1.f + __expf(-v)) * u);
+      }
+      if (row < a.M)
+        *reinterpret_cast<u16x4*>(a.out + (size_t)row * (a.N >> 1) +
+                                  (tile + (lane >> 5)) * 8 + (lane >> 4 & 1) * 4) = o;
+    } else if (row < a.M) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const size_t at = (size_t)row * a.N + (tile + t) * 16 + (lane >> 4) * 4;
+        const f32x4 v = sum[t][m];
+        *reinterpret_cast<u16x4*>(a.out + at) =
+            u16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
       }
     }
+  }
 }
 
 // The parts' sum + rotary positions + page append: grid (M, heads / 4), a head
@@ -482,8 +667,8 @@ __global__ void __launch_bounds__(256) rows_sum_kernel(
 #define ROWS_MAX 16   // rows up to here: gemm_rows_kernel
 
 // Weights from here on are streamed past the caches, and X stays in them: SwiGLU
-// over 28672 x 4096 40.5 -> 37.5 us (6.3 TB/s) at one row, 42.8 -> 40.1 at 64, 52.0
-// -> 50.0 at 128; 4096 x 14336 21.4 -> 19.0, 23.3 -> 21.7, 27.6 -> 26.8.  Smaller
+// over 28672 x 4096 40.5 -> 37.5 us at one row, 42.8 -> 40.1 at 64, 52.0 -> 50.0 at 128
+// (before later changes); 4096 x 14336 21.4 -> 19.0, 23.3 -> 21.7, 27.6 -> 26.8.  Smaller
 // ones are bound by latency, which is higher that way (2048 x 2048 5.1 us against
 // 4.1 from memory, 3.9 against 2.9 from the L2).
 static bool streamed(const RowsArgs& a) { return (i64)a.N * a.K >= (8 << 20); }
@@ -496,33 +681,64 @@ static void launch_rows(const RowsArgs& a, hipStream_t st) {
     gemm_rows_kernel<2, EPI, NORM, KEEP><<<a.N / 16, 512, 0, st>>>(a);
 }
 
-// Blocks of 128 weight rows (eight waves) halve the reads of X.  They pay from 33
-// rows on where they fill the chip with at least 12 pieces of K each (6144 x 4096 in
-// 5 at 64 rows: 11.2 us against 12.8, 4096 x 14336 in 8: 21.7 against 23.1; but
-// 4096 x 4096 in 8, 8 pieces: 8.8 against 8.5 in 4), below that for whole K only
-// (28672 x 4096 at 32 rows, weights not streamed: 43.0 against 44.2), always above
-// 64 rows.
+// Blocks of 128 weight rows halve the reads of X; they pay where they fill the chip
+// (28672 x 4096, 224 blocks: 36.9 us at 24 rows and 48.0 at 128, in 64 columns 41.1 and
+// 63.6), not below (16384 x 2048, 128 blocks: 16.4 and 24.8, in 64 columns 13.8 and 19.6).
 template <int EPI, int NORM, int AUX>
-static void launch_tile_as(const RowsArgs& a, int splits, hipStream_t st) {
+static void launch_tile_as(const RowsArgs& a, hipStream_t st) {
+  if (a.N % 128 == 0 && a.N / 128 >= 192) {
+    const int g = a.N / 128;
+    if (a.M <= 32)
+      gemm_tile_kernel<2, 8, 8, 5, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
+    else if (a.M <= 64)
+      gemm_tile_kernel<4, 8, 8, 4, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
+    else if (a.M <= 96)
+      gemm_tile_kernel<6, 8, 8, 4, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
+    else
+      gemm_tile_kernel<8, 8, 8, 4, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
+  } else {
+    const int g = a.N / 64;
+    if (a.M <= 32)
+      gemm_tile_kernel<2, 4, 4, 5, EPI, NORM, AUX><<<g, 256, 0, st>>>(a);
+    else if (a.M <= 64)
+      gemm_tile_kernel<4, 4, 8, 4, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
+    else if (a.M <= 96)
+      gemm_tile_kernel<6, 4, 4, 3, EPI, NORM, AUX><<<g, 256, 0, st>>>(a);
+    else
+      gemm_tile_kernel<8, 4, 8, 3, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
+  }
+}
+
+template <int EPI, int NORM>
+static void launch_tile(const RowsArgs& a, hipStream_t st) {
+  if (streamed(a)) launch_tile_as<EPI, NORM, STREAM>(a, st);
+  else launch_tile_as<EPI, NORM, KEEP>(a, st);
+}
+
+// Blocks of 128 weight rows pay from 33 rows on where they fill the chip with at least
+// 12 pieces of K each (6144 x 4096 in 5 at 64 rows: 11.2 us against 12.8, 4096 x 14336
+// in 8: 21.7 against 23.1; but 4096 x 4096 in 8, 8 pieces: 8.8 against 8.5 in 4), always
+// above 64 rows.
+template <int AUX>
+static void launch_parts_as(const RowsArgs& a, int splits, hipStream_t st) {
   const dim3 g64(a.N / 64, splits), g128(a.N / 128, splits);
   const bool wide = a.N % 128 == 0 && a.N / 128 * splits >= 192 &&
                     a.K / 64 >= 12 * splits;
   if (a.M <= 64 && wide && (a.M > 32 || splits == 1))
-    gemm_tile_kernel<4, 8, 4, 3, EPI, NORM, AUX><<<g128, 512, 0, st>>>(a);
+    gemm_parts_kernel<4, 8, 4, 3, AUX><<<g128, 512, 0, st>>>(a);
   else if (a.M <= 32)
-    gemm_tile_kernel<2, 4, 1, 4, EPI, NORM, AUX><<<g64, 256, 0, st>>>(a);
+    gemm_parts_kernel<2, 4, 1, 4, AUX><<<g64, 256, 0, st>>>(a);
   else if (a.M <= 64)
-    gemm_tile_kernel<4, 4, 2, 4, EPI, NORM, AUX><<<g64, 256, 0, st>>>(a);
+    gemm_parts_kernel<4, 4, 2, 4, AUX><<<g64, 256, 0, st>>>(a);
   else if (a.N % 128 == 0)
-    gemm_tile_kernel<8, 8, 4, 3, EPI, NORM, AUX><<<g128, 512, 0, st>>>(a);
+    gemm_parts_kernel<8, 8, 4, 3, AUX><<<g128, 512, 0, st>>>(a);
   else
-    gemm_tile_kernel<8, 4, 2, 3, EPI, NORM, AUX><<<g64, 256, 0, st>>>(a);
+    gemm_parts_kernel<8, 4, 2, 3, AUX><<<g64, 256, 0, st>>>(a);
 }
 
-template <int EPI, int NORM>
-static void launch_tile(const RowsArgs& a, int splits, hipStream_t st) {
-  if (streamed(a)) launch_tile_as<EPI, NORM, STREAM>(a, splits, st);
-  else launch_tile_as<EPI, NORM, KEEP>(a, splits, st);
+static void launch_parts(const RowsArgs& a, int splits, hipStream_t st) {
+  if (streamed(a)) launch_parts_as<STREAM>(a, splits, st);
+  else launch_parts_as<KEEP>(a, splits, st);
 }
 
 static int check_rows(const RowsArgs& a, int splits) {
@@ -576,17 +792,17 @@ AF_EXPORT int af_rows_linear(void* out, void* residual, void* parts, void* ss_ou
   }
   if (norm == 2) return 9008;
   if (mode == 2) {
-    if (norm == 0) launch_tile<EPI_SWIGLU, 0>(a, 1, st);
-    else launch_tile<EPI_SWIGLU, 1>(a, 1, st);
+    if (norm == 0) launch_tile<EPI_SWIGLU, 0>(a, st);
+    else launch_tile<EPI_SWIGLU, 1>(a, st);
     return af_last_err();
   }
   if (mode == 0 && splits == 1) {
-    if (norm == 0) launch_tile<EPI_PLAIN, 0>(a, 1, st);
-    else launch_tile<EPI_PLAIN, 1>(a, 1, st);
+    if (norm == 0) launch_tile<EPI_PLAIN, 0>(a, st);
+    else launch_tile<EPI_PLAIN, 1>(a, st);
     return af_last_err();
   }
   if (!parts) return 9008;
-  launch_tile<EPI_PARTS, 0>(a, splits, st);
+  launch_parts(a, splits, st);
   if (mode == 0) {
     const dim3 g(M, (N + 511) / 512);
     rows_sum_kernel<<<g, 256, 0, st>>>(a.out, a.parts, norm ? a.ss : nullptr, M, N,
@@ -631,7 +847,7 @@ AF_EXPORT int af_rows_qkv(void* q, void* parts, const void* X, const void* W,
     return af_last_err();
   }
   if (!parts || !ss) return 9008;
-  launch_tile<EPI_PARTS, 0>(a, splits, st);
+  launch_parts(a, splits, st);
   rows_rope_kernel<<<dim3(M, (Hq + 2 * Hk + 3) / 4), 256, 0, st>>>(a, splits);
   return af_last_err();
 }

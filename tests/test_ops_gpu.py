@@ -659,6 +659,27 @@ def test_linear_rows_modes(M, N, K):
                                   rtol=1e-4)
 
 
+@pytest.mark.parametrize("M", [17, 80, 96, 97])
+@pytest.mark.parametrize("N", [192, 16384, 24576])
+@pytest.mark.parametrize("pieces", [1, 2, 5, 6])
+def test_whole_k_row_products(M, N, pieces):
+    """The kernel of unsplit products: its 96-row class and both block widths, with
+    fewer pieces of K than the ring holds, as many and one more.  Tolerance as in
+    test_linear_rows_modes."""
+    K = 64 * pieces
+    x, w = rnd(M, K, seed=M, scale=0.3), rnd(N, K, seed=N, scale=0.3)
+    ss = torch.zeros(M, 8, device=DEV)
+    ss[:, 6] = x.float().pow(2).sum(-1)
+    rstd = torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + 1e-5)
+    y = x.float() @ w.float().t()
+    assert close(ops.linear(x, w), y, atol=2e-3 * math.sqrt(K) * 0.09, rtol=2 ** -7)
+    for f, scale in ((1, None), (rstd, (ss, 1e-5))):
+        g, u = (y * f).chunk(2, -1)
+        got = ops.linear_rows(x, w, 2, scale=scale)
+        assert close(got, torch.nn.functional.silu(g) * u, atol=2e-3 * K ** 0.5,
+                     rtol=2 ** -6)
+
+
 @pytest.mark.parametrize("M", [1, 17, 128])
 @pytest.mark.parametrize("K,KW", [(512, 448), (448, 512), (64, 4096)])
 def test_row_products_refuse_other_inner_lengths(M, K, KW):
