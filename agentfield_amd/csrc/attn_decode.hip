@@ -13,7 +13,11 @@
 // CU's share of the memory rate is ~9 bytes per clock, i.e. one token every ~54
 // clocks, so a token may cost at most that in instructions and the loop must
 // keep tens of KB per CU in flight.
-//   grid (B, Hk, NSPLIT), block = 256 threads = 4 waves; a wave iteration takes
+//   grid (B x Hk, NSPLIT), K/V head fastest, so that with 8 K/V heads every XCD has one head of all
+//   sequences, long and short (sequence first, an XCD had every eighth sequence: 32 of
+//   300..1500 with 32 heads 91.8 -> 81.5 us, 64 of 200..2000 60.3 -> 57.0, 24 of
+//   1800..8100 in two splits 114.5 -> 110.5).  Block = 256 threads = 4 waves; a wave
+//   iteration takes
 //   16 tokens (4 KB of K, 4 KB of V, 16 B per lane and load), the next tile's
 //   eight loads are issued before the current tile's arithmetic.
 //   Scores come from the matrix cores: K rows are the A operand straight from
@@ -30,11 +34,13 @@
 //   Rows, then waves (through LDS), then splits (second kernel) merge once.
 // Measured with 8 K/V heads, G = 4, against one lane group per token with a
 // shuffle reduction per score: 24 sequences of 1800..8100 tokens (513 MB)
-// 225 -> 108 us (4.7 TB/s), 128 of 545 101 -> 52 us (5.4 TB/s), 1 of 8000
+// 225 -> 108 us (4.7 TB/s), 128 of 545 101 -> 51 us (5.6 TB/s), 1 of 8000
 // 58 -> 22 us.  V is read with nontemporal loads, whole rows per instruction: 114
 // -> 108 and 57.3 -> 52.5 us.  K is not: two instructions share each of its lines,
 // and a line dropped between them is fetched twice (64 ragged sequences of up to
-// 2000 tokens 60 -> 65 us with both, 59 with V only).
+// 2000 tokens 60 -> 65 us with both, 59 with V only).  Not the loads' latency: eight
+// waves per block (114 -> 125 us) and whole rows through LDS with two tiles per wave in
+// flight (110.5 -> 112) do not help, nor do more splits or pages in order.
 #include "common.h"
 
 #include <type_traits>
@@ -79,7 +85,7 @@ __global__ void __launch_bounds__(64 * AD_WAVES, G == 8 ? 3 : 4) attn_decode_ker
     const i32* __restrict__ bt, const i32* __restrict__ len,
     float scale, int Hk, int page_size, int page_shift, int max_pages,
     int nsplit, i64 qs, int win) {
-  const int b = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z;
+  const int kvh = blockIdx.x % Hk, b = blockIdx.x / Hk, split = blockIdx.y;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int tg = lane >> 4, dl = lane & 15;
@@ -329,7 +335,7 @@ AF_EXPORT int af_attn_decode(void* out, void* po, void* pml, const void* q,
   const int G = Hq / Hk;
   if (G < 1 || G > AD_MAXG || G * Hk != Hq) return 9003;
   if (B == 0) return 0;
-  dim3 grid(B, Hk, nsplit), blk(64 * AD_WAVES);
+  dim3 grid(B * Hk, nsplit), blk(64 * AD_WAVES);
   hipStream_t st = (hipStream_t)stream;
   const bool pow2 = (page_size & (page_size - 1)) == 0;
   const int shift = pow2 ? __builtin_ctz(page_size) : -1;
