@@ -64,19 +64,9 @@
 // rows: 13.3, 8.0, 23.3, 41.2.  64 rows, without the closing launches: 13.1, 9.3,
 // 23.3, 38.9 (16.7, o + down 44.8, 62.7).  128 rows: 16.9, 15.0, 27.5, 48.0 (library
 // 25.6 and 57.5 + 5.2 for the first and the last, o + down 63.1).
-#include "common.h"
+#include "mfma_lines.h"
 
 #include <type_traits>
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8r;
-typedef __attribute__((address_space(3))) char lds_b;
-typedef __attribute__((address_space(3))) s16x8 lds_v8;
-
-__device__ __forceinline__ bf16x8r as_bf16x8r(s16x8 v) {
-  union { s16x8 s; bf16x8r b; } u;
-  u.s = v;
-  return u.b;
-}
 
 enum RowsEpi { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_ROPE = 3,
                EPI_PARTS = 4 };
@@ -98,28 +88,6 @@ struct RowsArgs {
   const i64* slot;
   int Hq, Hk, page_size;
 };
-
-// 8 rows x 128 bytes of a row-major matrix into linear LDS: lane l brings chunk
-// (l & 7) ^ (row & 7) of row l >> 3, so that chunk c of row r sits at slot
-// c ^ (r & 7).
-template <int AUX>
-__device__ __forceinline__ void load_line8(const u16* src, lds_b* dst) {
-  __builtin_amdgcn_global_load_lds(
-      (const __attribute__((address_space(1))) uint32_t*)src,
-      (__attribute__((address_space(3))) uint32_t*)dst, 16, 0, AUX);
-}
-constexpr int STREAM = 2, KEEP = 0;   // AUX: nontemporal, cached
-
-// s_waitcnt operand: all but n of a wave's vector loads have landed
-constexpr int vmcnt_only(int n) { return (n & 15) | (n >> 4) << 14 | 0x0f70; }
-
-// operand fragment: lane (r = lane & 15, q = lane >> 4) gets k = 32 h + 8 q .. +8
-// of row r of a 16-row piece
-__device__ __forceinline__ bf16x8r frag(const lds_b* piece, int h) {
-  const int lane = threadIdx.x & 63, r = lane & 15;
-  const int c = (h * 4 + (lane >> 4)) ^ (r & 7);
-  return as_bf16x8r(*reinterpret_cast<const lds_v8*>(piece + r * 128 + c * 16));
-}
 
 // W row of row n of a 16-row tile
 template <int EPI>

@@ -12,19 +12,21 @@
 #define MOE_MAX_K 8
 
 // Router logits in fp32 (products of bf16 are exact), softmax over the k largest:
-// a wave per row, equal logits go to the smaller expert.  A logit that is not a
-// number counts as the largest, so that the row's weights show it.
+// a block per row, equal logits go to the smaller expert.  A logit that is not a
+// number counts as the largest, so that the row's weights show it.  Bound by latency:
+// with a wave per row the loop over the row waited for memory eight times (34 us for 40
+// rows as for 1100); four waves share the row and most of its loads are out at once.
 template <int EM>
 __global__ void __launch_bounds__(256) moe_route_kernel(
     i32* __restrict__ topi, float* __restrict__ topv, const u16* __restrict__ x,
     const u16* __restrict__ router, int T, int H, int E, int k) {
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (t >= T) return;
+  const int t = blockIdx.x, lane = threadIdx.x & 63;
   const u16* xr = x + (size_t)t * H;
   float acc[EM];
 #pragma unroll
   for (int e = 0; e < EM; ++e) acc[e] = 0.f;
-  for (int c = lane * 8; c < H; c += 512) {
+#pragma unroll 2
+  for (int c = threadIdx.x * 8; c < H; c += 2048) {
     const s16x8 xv = *reinterpret_cast<const s16x8*>(xr + c);
     float xf[8];
 #pragma unroll
@@ -37,8 +39,17 @@ __global__ void __launch_bounds__(256) moe_route_kernel(
       for (int j = 0; j < 8; ++j) acc[e] = fmaf(xf[j], bf2f((u16)rv[j]), acc[e]);
     }
   }
+  __shared__ float part[4][EM];
 #pragma unroll
-  for (int e = 0; e < EM; ++e) acc[e] = wave_sum_f32(acc[e]);
+  for (int e = 0; e < EM; ++e) {
+    const float s = wave_sum_f32(acc[e]);
+    if (lane == 0) part[threadIdx.x >> 6][e] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+#pragma unroll
+  for (int e = 0; e < EM; ++e)
+    acc[e] = (part[0][e] + part[1][e]) + (part[2][e] + part[3][e]);
   unsigned long long used = 0;
   float best[MOE_MAX_K], sum = 0.f;
   int who[MOE_MAX_K];
@@ -160,9 +171,8 @@ AF_EXPORT int af_moe_route(void* topi, void* topv, void* offs, void* row, void* 
   if (H % 8 || E < 1 || E > MOE_MAX_E || k < 1 || k > MOE_MAX_K || k > E) return 9001;
   if (T == 0) return 0;
   hipStream_t st = (hipStream_t)stream;
-  const int grid = (T + 3) / 4;
 #define AF_ROUTE(EM)                                                           \
-  moe_route_kernel<EM><<<grid, 256, 0, st>>>((i32*)topi, (float*)topv,         \
+  moe_route_kernel<EM><<<T, 256, 0, st>>>((i32*)topi, (float*)topv,         \
                                              (const u16*)x, (const u16*)router, \
                                              T, H, E, k)
   if (E <= 8) AF_ROUTE(8);

@@ -233,7 +233,8 @@ class MoEMLP(nn.Module):
     * prefill (exact, eager): each expert runs the fused gate_up/down on
       its routed token subset — FLOP-proportional, shapes data-dependent.
       On the GPU the rows are routed and sorted by expert in two kernels, so
-      that a subset is one block of rows (ops.moe_route).
+      that a subset is one block of rows (ops.moe_route), and each projection
+      is one launch over all experts where ops.moe_gemm_ok says so.
     * decode (static, hipGraph-capturable): every expert runs on every
       token with routing weights zeroed for unrouted pairs.  Decode
       GEMMs are weight-streaming-bound and a top-2-of-8 batch >= ~16
@@ -297,6 +298,11 @@ class MoEMLP(nn.Module):
     def _forward_sorted(self, x):
         weights, row, pos, offs = ops.launch_moe_route(x, self.router,
                                                        self.top_k)
+        if ops.moe_gemm_ok(x, self.router, self.gate_up, self.down):
+            act = ops.launch_moe_gemm(x, self.gate_up, offs, row.numel(), row,
+                                      swiglu=True)
+            ys = ops.launch_moe_gemm(act, self.down, offs, row.numel())
+            return ops.moe_combine(ys, pos, weights)
         xs = ops.gather_rows(x, row)
         ys = torch.empty_like(xs)
         bounds = offs.tolist()       # the one wait: block bounds

@@ -604,6 +604,33 @@ def moe_combine(y: torch.Tensor, pos: torch.Tensor,
     return out
 
 
+def moe_gemm_ok(x: torch.Tensor, router: torch.Tensor, gate_up: torch.Tensor,
+                down: torch.Tensor) -> bool:
+    """What the projections over sorted rows take beside moe_route_ok: bf16 weights
+    [E, 2I, H] and [E, H, I] of the router's experts on x's GPU, whole and on 16-byte
+    boundaries, H and I in 64s."""
+    g, d = gate_up.shape, down.shape
+    if len(g) != 3 or len(d) != 3:
+        return False
+    (E, I2, H), I = g, d[2]
+    return (d == (E, H, I) and I2 == 2 * I and x.shape[1] == H
+            and router.shape[0] == E and H > 0 and H % 64 == 0 and I > 0
+            and I % 64 == 0 and x.device == gate_up.device == down.device
+            and rows_operands_ok((x, gate_up, down)))
+
+
+def launch_moe_gemm(x, w, offs, n, row=None, swiglu=False):
+    """n sorted rows against their expert's w [E, N, K], for callers that have asked
+    moe_gemm_ok: x rows through row [n], or x in sorted order."""
+    E, N, K = w.shape
+    out = torch.empty(n, N // 2 if swiglu else N, dtype=x.dtype, device=x.device)
+    rc = _lib.lib().af_moe_gemm(
+        _lib.ptr(out), _lib.ptr(x), _lib.ptr(row), _lib.ptr(w), _lib.ptr(offs), n, E,
+        N, K, 2 if swiglu else 0, _lib.cur_stream())
+    _lib.check(rc, "af_moe_gemm")
+    return out
+
+
 def gemm_bf16(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """C[M,N] = a[M,K] @ w[N,K]^T via the hand-written MFMA kernel."""
     if not _on_gpu(a):

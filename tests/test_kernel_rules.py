@@ -150,6 +150,26 @@ def test_rows_that_the_routing_kernels_take(monkeypatch, ok, x, router, k):
     assert MoEMLP._can_sort(layer, x) == ok
 
 
+@pytest.mark.parametrize("ok,gate_up,down", [
+    (True, mat(4, 128, 64), mat(4, 64, 64)),
+    (True, mat(4, 384, 64), mat(4, 64, 192)),
+    (False, mat(5, 128, 64), mat(5, 64, 64)),         # experts without a router row
+    (False, mat(3, 128, 64), mat(3, 64, 64)),
+    (False, mat(4, 128, 64), mat(3, 64, 64)),
+    (False, mat(4, 192, 64), mat(4, 64, 96)),         # lengths in 64s only
+    (False, mat(4, 128, 128), mat(4, 128, 64)),       # other rows than x's
+    (False, mat(4, 128, 64), mat(4, 64, 128)),
+    (False, mat(4, 128, 64), mat(4, 128, 64)),
+    (False, mat(128, 64), mat(64, 64)),
+    (False, mat(4, 128, 64, contiguous=False), mat(4, 64, 64)),
+    (False, mat(4, 128, 64), mat(4, 64, 64, addr=8)),
+    (False, mat(4, 128, 64), mat(4, 64, 64, dtype=torch.float32)),
+    (False, mat(4, 128, 64), mat(4, 64, 64, device="cuda:1")),
+])
+def test_experts_that_the_sorted_products_take(ok, gate_up, down):
+    assert ops.moe_gemm_ok(mat(5, 64), mat(4, 64), gate_up, down) == ok
+
+
 @pytest.mark.parametrize("lens,want", [
     ([8000], (32, 250, 0, 1)),                     # one long prompt
     ([700, 3, 8, 500, 9], (32, 39, 2, 4)),         # both kinds of items

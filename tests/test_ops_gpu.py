@@ -1067,6 +1067,60 @@ def test_moe_kernels_refuse_other_operands():
     ops.moe_combine(y, pos, w)
 
 
+@pytest.mark.parametrize("counts", [
+    [1], [32, 33], [0, 288, 0, 289, 3], [17, 0, 64, 65, 192, 193, 256, 257],
+    [600, 1, 2, 900], [0] * 63 + [290]])
+@pytest.mark.parametrize("I,H", [(64, 64), (192, 320), (640, 1152)])
+def test_moe_sorted_products(counts, I, H):
+    """Both projections over sorted rows at the edges of their row classes and row
+    tiles, with empty experts, partial blocks of weights and fewer pieces of K than
+    the ring holds.  Tolerance: bf16 rounding of the result (2^-8 relative, 2^-7
+    through SwiGLU) and fp32 sums over K of products of ~0.1 size."""
+    E, n = len(counts), sum(counts)
+    T = n // 2 + 1
+    x = rnd(T, H, seed=n, scale=0.3)
+    gate_up, down = (rnd(E, 2 * I, H, seed=I, scale=0.3),
+                     rnd(E, H, I, seed=H, scale=0.3))
+    offs = torch.tensor([0] + counts, device=DEV).cumsum(0).int()
+    row = torch.randint(0, T, (n,), device=DEV, dtype=torch.int32)
+    act = ops.launch_moe_gemm(x, gate_up, offs, n, row, swiglu=True)
+    y = ops.launch_moe_gemm(act, down, offs, n)
+    at = 0
+    for e, c in enumerate(counts):
+        s = slice(at, at + c)
+        g, u = (x[row[s].long()].float() @ gate_up[e].float().t()).chunk(2, -1)
+        assert close(act[s], torch.nn.functional.silu(g) * u, atol=2e-3 * H ** 0.5,
+                     rtol=2 ** -6)
+        want = act[s].float() @ down[e].float().t()
+        scale = want.abs().max().item() if c else 1.0
+        assert close(y[s], want, atol=2e-5 * scale * I ** 0.5, rtol=2 ** -7)
+        at += c
+
+
+def test_moe_prompt_under_capture():
+    """The mixture's prompt rows need no wait of the host: a captured step gives the
+    eager bits on every replay, with other rows and routes each time."""
+    from agentfield_amd.models import CONFIGS
+    from agentfield_amd.models.llama import MoEMLP
+    mlp = MoEMLP(CONFIGS["tiny-moe"]).to(DEV, torch.bfloat16)
+    with torch.inference_mode():
+        for i, p in enumerate(mlp.parameters()):
+            p.copy_(rnd(*p.shape, seed=i, scale=0.2))
+        x = rnd(75, 256, seed=0)
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            mlp(x)
+        torch.cuda.current_stream().wait_stream(side)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            y = mlp(x)
+        for i in range(4):
+            x.copy_(rnd(75, 256, seed=i + 1))
+            g.replay()
+            assert torch.equal(y, mlp(x))
+
+
 @pytest.mark.parametrize("T", [5, 40])
 @pytest.mark.parametrize("layer", [0, 1])
 @pytest.mark.parametrize("prompt", [True, False])
