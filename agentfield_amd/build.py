@@ -37,6 +37,7 @@ HIP_SOURCES = [
     "gemm_skinny.hip",
     "gemm_rows.hip",
     "moe.hip",
+    "gemm_wide.hip",
     "moe_gemm.hip",
     "sampling.hip",
     "probe.hip",

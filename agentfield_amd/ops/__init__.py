@@ -511,11 +511,57 @@ def linear_skinny(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
     return out
 
 
+def _wide_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """What the wide GEMM takes: bf16 rows and weights of one length on one GPU,
+    whole and on 16-byte boundaries; 256 rows or more, at least 256 weight rows in
+    64s, at least 128 columns in 64s, half of w (the up rows) within 4 GB."""
+    xs, ws = x.shape, w.shape
+    return (x.is_cuda and len(xs) == 2 == len(ws) and xs[1] == ws[1]
+            and 256 <= xs[0] <= 1 << 24 and ws[0] >= 256 and ws[0] % 64 == 0
+            and ws[1] >= 128 and ws[1] % 64 == 0
+            and (ws[0] // 2 + 256) * ws[1] * 2 < 1 << 32
+            and x.device == w.device and rows_operands_ok((x, w)))
+
+
+def _wide_pays(M: int, N: int, K: int, silu_fuse: bool) -> bool:
+    """Whether the wide GEMM beats the library's, by 256 x 256 tiles per round of
+    256 blocks, from 15 projections of four models at 256..9000 rows.
+
+    With SwiGLU behind it, which the library leaves to a pass of its own: from 64
+    tiles on, the fewest measured (library over wide 0.98..1.61, 1.13 in the mean;
+    14336 x 4096 at 2048 rows 364 us / 360, 4096 rows 720 / 668, 5120 rows 1000 /
+    846).
+    Plain: the library is 5-8% ahead in whole rounds (4096 x 4096 at 8000 rows 179
+    us / 189) and draws level below one, but falls back by up to 1.78 where a round
+    is begun (4096 x 14336 at 4352 rows 720 / 410, 8448 rows 1003 / 700; 6144 x 4096
+    at 8448 rows 393 / 310).  Up to half a round the wide GEMM took 34 of 47 sizes
+    and lost 8% at most; with a long K the library stays behind further (4096 x
+    14336 at 6800 rows 920 / 570, at 7400 970 / 600)."""
+    tiles = -(-M // 256) * -(-N // 256)
+    if silu_fuse:
+        return tiles >= 64
+    begun = tiles & 255
+    return tiles > 256 and 0 < begun <= (216 if K >= 2 * N else 128)
+
+
+def launch_wide(x, w, silu_fuse=False, out=None, groups=0):
+    """The wide GEMM itself, for callers that have asked _wide_ok."""
+    (M, K), N = x.shape, w.shape[0]
+    if out is None:
+        out = torch.empty(M, N // 2 if silu_fuse else N, dtype=x.dtype,
+                          device=x.device)
+    rc = _lib.lib().af_gemm_wide(
+        _lib.ptr(out), _lib.ptr(x), _lib.ptr(w), M, N, K, 2 if silu_fuse else 0,
+        groups, _lib.cur_stream())
+    _lib.check(rc, "af_gemm_wide")
+    return out
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
            out: torch.Tensor | None = None) -> torch.Tensor:
     """Linear layer dispatch: hand-written weight-streaming kernels up to 128
-    rows, hipBLASLt (torch.matmul) for prefill GEMMs.  out (without silu_fuse):
-    [M, N] rows of x's type to write to.
+    rows, the wide GEMM or hipBLASLt (torch.matmul) for prefill GEMMs.  out
+    (without silu_fuse): [M, N] rows of x's type to write to.
 
     Plain products of 33..128 rows lose to the library where N fills the chip
     neither in blocks of 128 columns nor in several splits.  Measured, library
@@ -533,6 +579,13 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
             and (out is None or _whole(out, x, M, N) and _apart(out, x))
             and _rows_ok(x, w)):
         return launch_rows(x, w, 2 if silu_fuse else 0, out=out)
+    if (M > 128 and x.is_cuda and x.dim() == 2 == w.dim()
+            and _wide_pays(M, N, x.shape[1], silu_fuse)
+            and not watched(x, w, grad=not silu_fuse)
+            and (out is None or _whole(out, x, M, N) and _apart(out, x)
+                 and out.data_ptr() & 15 == 0)
+            and _wide_ok(x, w)):
+        return launch_wide(x, w, silu_fuse, out)
     if out is not None:
         return torch.mm(x, w.t(), out=out)
     y = x @ w.t()

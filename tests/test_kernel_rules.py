@@ -193,3 +193,39 @@ def test_rows_splits_leave_no_split_empty(N, K):
         n, pieces = ops.rows_splits(M, N, K), K // 64
         assert 1 <= n <= min(16, pieces)
         assert (n - 1) * -(-pieces // n) < pieces
+
+
+@pytest.mark.parametrize("x,w,ok", [
+    (mat(256, 128), mat(256, 128), True),
+    (mat(10077, 4096), mat(28672, 4096), True),
+    (mat(257, 192), mat(320, 192), True),
+    (mat(300, 8192), mat(57344, 8192), True),
+    (mat(255, 128), mat(256, 128), False),        # tiles are 256 rows at most
+    (mat(256, 128), mat(192, 128), False),
+    (mat(256, 128), mat(288, 128), False),
+    (mat(256, 64), mat(256, 64), False),          # two pieces of K are on their way
+    (mat(256, 160), mat(256, 160), False),
+    (mat(256, 128), mat(256, 192), False),
+    (mat(256, 1 << 18), mat(1 << 14, 1 << 18), False),   # offsets of 32 bits
+    (mat(4, 64, 128), mat(256, 128), False),
+    (mat(256, 128, dtype=torch.float16), mat(256, 128, dtype=torch.float16), False),
+    (mat(256, 128, contiguous=False), mat(256, 128), False),
+    (mat(256, 128), mat(256, 128, addr=8), False),
+    (mat(256, 128), mat(256, 128, device="cuda:1"), False),
+    (mat(256, 128, device="cpu"), mat(256, 128, device="cpu"), False),
+])
+def test_wide_gemm_operands(x, w, ok):
+    assert ops._wide_ok(x, w) == ok
+
+
+@pytest.mark.parametrize("M,N,K,glu,pays", [
+    (4096, 28672, 4096, True, True), (256, 16384, 2048, True, True),
+    (256, 8192, 4096, True, False),               # 32 tiles: few blocks at work
+    (4096, 4096, 4096, False, False),             # one whole round
+    (4097, 4096, 4096, False, True),              # a second one begun
+    (6144, 4096, 4096, False, True), (6145, 4096, 4096, False, False),
+    (6145, 4096, 14336, False, True), (7680, 4096, 14336, False, False),
+    (2048, 4096, 4096, False, False),
+])
+def test_wide_gemm_pays(M, N, K, glu, pays):
+    assert ops._wide_pays(M, N, K, glu) == pays

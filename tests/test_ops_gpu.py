@@ -1158,3 +1158,51 @@ def test_few_row_path_with_strided_weights(T, layer, prompt):
             out.append(m(ids, pos, kv, md).float())
     a, b = out
     assert (a - b).norm() <= 1e-2 * a.norm()
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (256, 256, 128),          # one tile, two pieces of K
+    (257, 320, 128),          # both moved back inside the matrix
+    (449, 1088, 192),         # 64 columns of a last tile
+    (1000, 512, 320), (2000, 28672, 256),         # a second round of tiles
+    (4353, 4096, 256),
+])
+@pytest.mark.parametrize("groups", [0, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("glu", [False, True])
+def test_wide_gemm(M, N, K, groups, glu):
+    """Tile edges, remainders and several tiles per block.  bf16 keeps 8 bits: half a
+    unit is at most 2^-8 of a value.  Sums of up to 320 fp32 products, each about
+    0.64 / sqrt(K), differ with their order by at most K^1.5 * 0.64 * 2^-24 = 2.2e-4,
+    which SwiGLU (slope of silu below 1.1) passes on times up or gate."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(N, K, device="cuda", generator=g) / K ** 0.5).bfloat16()
+    got = torch.full((M + 1, N // 2 if glu else N), 7.0, device="cuda",
+                     dtype=torch.bfloat16)
+    ops.launch_wide(x, w, glu, got[:M], groups)
+    y, order = x.float() @ w.float().t(), 2.2e-4
+    if glu:
+        gate, up = y[:, :N // 2], y[:, N // 2:]
+        y = torch.nn.functional.silu(gate) * up
+        order = order * (1.1 * up.abs() + gate.abs() + 1e-2)
+    assert ((got[:M].float() - y).abs() <= 2 ** -8 * y.abs() + order).all()
+    assert (got[M:] == 7.0).all()
+
+
+@pytest.mark.parametrize("glu", [False, True])
+def test_linear_runs_the_wide_gemm(glu):
+    """linear sends what the rule names to the kernel, with and without out, and
+    what torch has to see to torch."""
+    x = torch.randn(4160, 128, device="cuda").bfloat16()
+    w = torch.randn(4096, 128, device="cuda").bfloat16()
+    want = torch.empty(4160, 2048 if glu else 4096, device="cuda").bfloat16()
+    ops.launch_wide(x, w, glu, want)
+    with torch.no_grad():
+        assert torch.equal(ops.linear(x, w, silu_fuse=glu), want)
+        if not glu:
+            out = torch.zeros_like(want)
+            assert ops.linear(x, w, out=out) is out and torch.equal(out, want)
+    if not glu:
+        leaf = w.clone().requires_grad_()
+        ops.linear(x, leaf).float().sum().backward()
+        assert leaf.grad is not None
