@@ -37,42 +37,75 @@ struct WideArgs {
   const u16* X;
   const u16* W;
   int M, N, K, tm, tn;     // tiles of rows and of columns
+  // experts: rows sorted by expert, W [E, N, K]
+  const i32* offs;         // [E + 1] first sorted row
+  const i32* row;          // X row of a sorted row; null: itself
+  int E;
 };
 
-template <int G, int EPI>
-__global__ void __launch_bounds__(256, 1) gemm_wide_kernel(WideArgs a) {
+// All tiles of a block.  EXPERTS: rows of X are gathered and tiles end with their
+// expert's rows; lane e has expert e's first row, rows and the tiles up to its end.
+template <int G, int EPI, bool EXPERTS>
+__device__ __forceinline__ void wide_tiles(const WideArgs& a, char* lds, int first_e,
+                                           int rows_e, int end_e) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int XR = 32 * G, WB = GW_COLS * 128, XB = XR * 128;
   constexpr bool GLU = EPI == WIDE_SWIGLU;
   constexpr int OUT = GLU ? GW_COLS / 2 : GW_COLS;         // output columns per tile
-  __shared__ __attribute__((aligned(16))) char lds[3 * WB + 2 * XB];
   lds_b* const wring = (lds_b*)lds;
   lds_b* const xring = wring + 3 * WB;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, n = lane & 15, q = lane >> 4, r8 = lane >> 3;
-  const int nt = a.tm * a.tn, cnt = a.K >> 6, cols = GLU ? a.N >> 1 : a.N;
+  const int nt = EXPERTS ? __builtin_amdgcn_readlane(end_e, a.E - 1) : a.tm * a.tn;
+  const int cnt = a.K >> 6, cols = GLU ? a.N >> 1 : a.N;
   const unsigned ld = (unsigned)a.K * 2;
 
   // Rounds of 256 tiles; an XCD's 32 blocks take 8 x 4 neighbours, which share their
-  // operands in its L2.  The last tile of a row or column is moved back inside the
-  // matrix (M >= XR, N >= 256) and stores only what the one before it did not.
+  // operands in its L2.  The last tile of a column is moved back inside the matrix (N >=
+  // 256) and stores only what the one before it did not; so is, without experts, the last
+  // tile of a row (M >= XR).
   const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
   auto tile = [&](int round) { return (round * 8 + xcd) * (GW_BLOCKS / 8) + idx; };
-  auto place = [&](int p, int& tm, int& tn) {
-    const int band = p / (8 * a.tn), high = min(8, a.tm - band * 8), in = p - band * 8 * a.tn;
-    tm = band * 8 + in % high;
-    tn = in / high;
+  struct Place { int e, row, rows, fresh, tn; };           // rows from fresh on are new
+  auto place = [&](int p) {
+    Place at = {0, 0, a.M, 0, 0};
+    int tm = a.tm;
+    if (EXPERTS) {
+      at.e = __builtin_ctzll(__ballot(p < end_e));         // the first that ends behind p
+      at.row = __builtin_amdgcn_readlane(first_e, at.e);
+      at.rows = __builtin_amdgcn_readlane(rows_e, at.e);
+      tm = (at.rows + XR - 1) / XR;
+      p -= __builtin_amdgcn_readlane(end_e, at.e) - tm * a.tn;
+    }
+    const int band = p / (8 * a.tn), high = min(8, tm - band * 8), in = p - band * 8 * a.tn;
+    const int t = band * 8 + in % high, r = EXPERTS ? t * XR : min(t * XR, a.M - XR);
+    at.row += r;
+    at.rows -= r;
+    at.fresh = EXPERTS ? 0 : t * XR - r;
+    at.tn = in / high;
+    return at;
   };
-  const char *xb, *wb;                                     // of the tile being loaded
+  const char *xb = (const char*)a.X, *wb;                  // of the tile being loaded
+  unsigned xg[G], xgn[G];                                  // EXPERTS: lanes' rows, bytes
+  auto seek_x = [&](int p) {                               // of the next tile
+    const Place at = place(p);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int r = at.row + min((g * 4 + wid) * 8 + r8, at.rows - 1);
+      xgn[g] = a.row ? a.row[r] : r;
+    }
+  };
   auto aim_x = [&](int p) {
-    int tm, tn;
-    place(p, tm, tn);
-    xb = (const char*)(a.X + (size_t)min(tm * XR, a.M - XR) * a.K);
+    if (EXPERTS) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) xg[g] = xgn[g] * ld + ((lane & 7) ^ r8) * 16;
+    } else {
+      xb = (const char*)(a.X + (size_t)place(p).row * a.K);
+    }
   };
   auto aim_w = [&](int p) {
-    int tm, tn;
-    place(p, tm, tn);
-    wb = (const char*)(a.W + (size_t)min(tn * OUT, cols - OUT) * a.K);
+    const Place at = place(p);
+    wb = (const char*)(a.W + ((size_t)at.e * a.N + min(at.tn * OUT, cols - OUT)) * a.K);
   };
 
   // A wave loads 8 lines (8 rows x 128 bytes) of W and G of X per piece.  Row 16 t + 4 q
@@ -91,7 +124,8 @@ __global__ void __launch_bounds__(256, 1) gemm_wide_kernel(WideArgs a) {
   auto load_x = [&](int g, lds_b* to, int k) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         __builtin_amdgcn_make_buffer_rsrc((void*)xb, 0, 0xffffffffu, 0x00027000),
-        (lds_v*)(to + (g * 4 + wid) * 1024), 16, xo, (g * 4 + wid) * 8 * ld + k, 0, 0);
+        (lds_v*)(to + (g * 4 + wid) * 1024), 16, EXPERTS ? xg[g] : xo,
+        (EXPERTS ? 0 : (g * 4 + wid) * 8 * ld) + k, 0, 0);
   };
   // operands: lane (n, q) has k = 8 q .. + 8 of row n, at the first or second half
   const int wm = wid >> 1, wn = wid & 1;
@@ -108,6 +142,7 @@ __global__ void __launch_bounds__(256, 1) gemm_wide_kernel(WideArgs a) {
 
   int round = 0, p = tile(0);
   if (p >= nt) return;
+  if (EXPERTS) seek_x(p);
   aim_x(p);
   aim_w(p);
 #pragma unroll
@@ -130,6 +165,7 @@ __global__ void __launch_bounds__(256, 1) gemm_wide_kernel(WideArgs a) {
 
   for (;;) {
     const int next = tile(round + 1);
+    if (EXPERTS && next < nt) seek_x(next);
     f32x4 acc[8][G];
 #pragma unroll
     for (int t = 0; t < 8; ++t)
@@ -218,14 +254,13 @@ __global__ void __launch_bounds__(256, 1) gemm_wide_kernel(WideArgs a) {
       for (int m = 0; m < G; ++m) asm volatile("" : "+a"(acc[t][m]));
 
     // lane: row n of each group, columns 8 q .. + 8 of each pair of tiles
-    int tm, tn;
-    place(p, tm, tn);
-    const int r0 = min(tm * XR, a.M - XR) + wm * G * 16 + n;
-    const int c0 = min(tn * OUT, cols - OUT) + wn * (OUT / 2);
-    u16* o = a.out + (size_t)r0 * cols + c0 + q * 8;
+    const Place at = place(p);
+    const int r0 = wm * G * 16 + n;
+    const int c0 = min(at.tn * OUT, cols - OUT) + wn * (OUT / 2);
+    u16* o = a.out + (size_t)(at.row + r0) * cols + c0 + q * 8;
 #pragma unroll
     for (int m = 0; m < G; ++m) {
-      if (r0 + m * 16 >= tm * XR) {
+      if (EXPERTS ? r0 + m * 16 < at.rows : r0 + m * 16 >= at.fresh) {
 #pragma unroll
         for (int t = 0; t < (GLU ? 2 : 4); ++t) {
           bf16x8r v;
@@ -237,7 +272,7 @@ __global__ void __launch_bounds__(256, 1) gemm_wide_kernel(WideArgs a) {
                   acc[(GLU ? 4 : 0) + t * 2 + (j >> 2)][m][j & 3];
             v[j] = (__bf16)f;
           }
-          if (c0 + t * 32 >= tn * OUT) *reinterpret_cast<bf16x8r*>(o + t * 32) = v;
+          if (c0 + t * 32 >= at.tn * OUT) *reinterpret_cast<bf16x8r*>(o + t * 32) = v;
         }
       }
       o += 16 * (size_t)cols;
@@ -250,17 +285,59 @@ __global__ void __launch_bounds__(256, 1) gemm_wide_kernel(WideArgs a) {
 #endif
 }
 
-// G of least cost: microseconds per piece of K for G = 4..8, and per tile beside them,
-// fitted to 2,175 times (15 projections of four models, 256..9000 rows, every G).
-static int wide_groups(int M, int N, int K) {
-  static const float piece[5] = {0.766f, 0.911f, 1.054f, 1.195f, 1.333f};
+template <int G, int EPI>
+__global__ void __launch_bounds__(256, 1) gemm_wide_kernel(WideArgs a) {
+  __shared__ __attribute__((aligned(16))) char lds[(3 * GW_COLS + 2 * 32 * G) * 128];
+  wide_tiles<G, EPI, false>(a, lds, 0, 0, 0);
+}
+
+// Microseconds per piece of K for G = 4..8, and per tile beside them, fitted to 2,175
+// times (15 projections of four models, 256..9000 rows, every G).
+#define GW_PIECE {0.766f, 0.911f, 1.054f, 1.195f, 1.333f}
+#define GW_TILE 3.2f
+
+// The same over rows sorted by expert.  Every block finds G by itself, from the number
+// of tiles that the experts' rows make.
+template <int EPI>
+__global__ void __launch_bounds__(256, 1) gemm_wide_experts_kernel(WideArgs a) {
+  __shared__ __attribute__((aligned(16))) char lds[(3 * GW_COLS + 2 * 256) * 128];
+  const int lane = threadIdx.x & 63;
+  const int first = a.offs[min(lane, a.E)];
+  const int rows = lane < a.E ? a.offs[min(lane + 1, a.E)] - first : 0;
+  constexpr float piece[5] = GW_PIECE;
+  int best = 0, end = 0;
+  float least = 0.f;
+#pragma unroll
+  for (int g = 8; g >= 4; --g) {
+    int sum = (rows + 32 * g - 1) / (32 * g) * a.tn;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(sum, o, 64);
+      if (lane >= o) sum += v;
+    }
+    const int nt = __builtin_amdgcn_readlane(sum, 63);
+    const float us =
+        (float)((nt + GW_BLOCKS - 1) / GW_BLOCKS) * ((a.K >> 6) * piece[g - 4] + GW_TILE);
+    if (best == 0 || us < least) { best = g; least = us; end = sum; }
+  }
+  switch (__builtin_amdgcn_readfirstlane(best)) {
+    case 4: wide_tiles<4, EPI, true>(a, lds, first, rows, end); break;
+    case 5: wide_tiles<5, EPI, true>(a, lds, first, rows, end); break;
+    case 6: wide_tiles<6, EPI, true>(a, lds, first, rows, end); break;
+    case 7: wide_tiles<7, EPI, true>(a, lds, first, rows, end); break;
+    default: wide_tiles<8, EPI, true>(a, lds, first, rows, end);
+  }
+}
+
+static int wide_groups(int M, int N, int K) {   // G of least cost
+  static const float piece[5] = GW_PIECE;
   int best = 0;
   float least = 0.f;
   for (int g = 8; g >= 4; --g) {
     const long long tiles =
         (long long)((M + 32 * g - 1) / (32 * g)) * ((N + GW_COLS - 1) / GW_COLS);
     const float us =
-        (float)((tiles + GW_BLOCKS - 1) / GW_BLOCKS) * (K / 64 * piece[g - 4] + 3.2f);
+        (float)((tiles + GW_BLOCKS - 1) / GW_BLOCKS) * (K / 64 * piece[g - 4] + GW_TILE);
     if (best == 0 || us < least) { best = g; least = us; }
   }
   return best;
@@ -281,7 +358,7 @@ AF_EXPORT int af_gemm_wide(void* out, const void* X, const void* W, int M, int N
   if (groups == 0) groups = wide_groups(M, N, K);
   hipStream_t st = (hipStream_t)stream;
   WideArgs a = {(u16*)out, (const u16*)X, (const u16*)W, M, N, K,
-                (M + 32 * groups - 1) / (32 * groups), (N + GW_COLS - 1) / GW_COLS};
+                (M + 32 * groups - 1) / (32 * groups), (N + GW_COLS - 1) / GW_COLS, nullptr, nullptr, 0};
 #define GW_CASE(g)                                                                \
   case g:                                                                         \
     if (epi == WIDE_SWIGLU) gemm_wide_kernel<g, WIDE_SWIGLU><<<GW_BLOCKS, 256, 0, st>>>(a); \
@@ -292,5 +369,24 @@ AF_EXPORT int af_gemm_wide(void* out, const void* X, const void* W, int M, int N
     default: return 9022;
   }
 #undef GW_CASE
+  return af_last_err();
+}
+
+// Rows sorted by expert, n in all: offs [E + 1], row [n] or null, W [E, N, K], x_rows rows
+// of X.
+AF_EXPORT int af_gemm_wide_experts(void* out, const void* X, const void* row, const void* W,
+                                   const void* offs, int x_rows, int n, int E, int N, int K,
+                                   int epi, void* stream) {
+  if (!wide_ok(256, N, K, epi) || E < 1 || E > 64 || n < 0 || x_rows < 0 ||
+      (long long)x_rows * K * 2 > 0xffffffffll ||
+      ((long long)n / 128 + E) * (N / GW_COLS + 1) > 0x3fffffff)
+    return 9021;
+  if (n == 0) return 0;
+  hipStream_t st = (hipStream_t)stream;
+  WideArgs a = {(u16*)out, (const u16*)X, (const u16*)W, n, N, K, 0,
+                (N + GW_COLS - 1) / GW_COLS, (const i32*)offs, (const i32*)row, E};
+  if (epi == WIDE_SWIGLU)
+    gemm_wide_experts_kernel<WIDE_SWIGLU><<<GW_BLOCKS, 256, 0, st>>>(a);
+  else gemm_wide_experts_kernel<WIDE_PLAIN><<<GW_BLOCKS, 256, 0, st>>>(a);
   return af_last_err();
 }

@@ -16,10 +16,9 @@
 // all (loads alone 541 us of gate/up, products alone 387, both 600).  Weights through
 // registers instead of LDS, 16 rows x 64 bytes per load, were slower (640 us, at half of
 // the rows per wave 1420 with spills).
-// Against one library product per expert and projection, gathered rows and a wait of the
-// host for the block bounds, 4096 x 14336 x 8: 20 rows 505 -> 431 us, 200 589 -> 480,
-// 600 1083 -> 631, 1100 1333 -> 916, 2000 1918 -> 1532, 4096 2940 -> 2760.  Just above
-// 288 rows per expert the second block column pass shows (1150 rows 1137).
+// From 200 rows per expert on (down 250) the wide GEMM takes over.  Against one library
+// product per expert and projection, gathered rows and a wait of the host for the block
+// bounds, 4096 x 14336 x 8: 20 rows 505 -> 431 us, 200 589 -> 480, 600 1083 -> 631.
 #include "mfma_lines.h"
 
 #include <type_traits>

@@ -299,9 +299,9 @@ class MoEMLP(nn.Module):
         weights, row, pos, offs = ops.launch_moe_route(x, self.router,
                                                        self.top_k)
         if ops.moe_gemm_ok(x, self.router, self.gate_up, self.down):
-            act = ops.launch_moe_gemm(x, self.gate_up, offs, row.numel(), row,
-                                      swiglu=True)
-            ys = ops.launch_moe_gemm(act, self.down, offs, row.numel())
+            act = ops.launch_experts(x, self.gate_up, offs, row.numel(), row,
+                                     swiglu=True)
+            ys = ops.launch_experts(act, self.down, offs, row.numel())
             return ops.moe_combine(ys, pos, weights)
         xs = ops.gather_rows(x, row)
         ys = torch.empty_like(xs)

@@ -684,6 +684,41 @@ def launch_moe_gemm(x, w, offs, n, row=None, swiglu=False):
     return out
 
 
+def wide_experts_pay(x_rows: int, n: int, E: int, N: int, K: int,
+                     swiglu: bool) -> bool:
+    """Whether n sorted rows go to the wide GEMM rather than to moe_gemm: what it
+    takes beside moe_gemm_ok (x and half an expert's weights within 4 GB), and rows
+    enough that the matrix cores bound it and not the weight stream.  Measured with 8
+    experts of 4096 x 14336, moe_gemm / wide in us: gate/up 425 / 447 at 175 rows per
+    expert, 475 / 445 at 200, 594 / 522 at 275, 735 / 528 at 300, 1930 / 1593 at
+    1024; down 253 / 272 at 225, 291 / 286 at 250, 378 / 287 at 288, 922 / 809 at
+    1024."""
+    return (n >= (200 if swiglu else 250) * E and N >= 256 and K >= 128
+            and x_rows * K * 2 < 1 << 32 and (N // 2 + 256) * K * 2 < 1 << 32
+            and n <= 1 << 24)
+
+
+def launch_wide_experts(x, w, offs, n, row=None, swiglu=False):
+    """launch_moe_gemm's product by the wide GEMM, for callers that have asked
+    wide_experts_pay."""
+    E, N, K = w.shape
+    out = torch.empty(n, N // 2 if swiglu else N, dtype=x.dtype, device=x.device)
+    rc = _lib.lib().af_gemm_wide_experts(
+        _lib.ptr(out), _lib.ptr(x), _lib.ptr(row), _lib.ptr(w), _lib.ptr(offs),
+        x.shape[0], n, E, N, K, 2 if swiglu else 0, _lib.cur_stream())
+    _lib.check(rc, "af_gemm_wide_experts")
+    return out
+
+
+def launch_experts(x, w, offs, n, row=None, swiglu=False):
+    """n sorted rows against their expert's w by the kernel that suits them, for
+    callers that have asked moe_gemm_ok."""
+    E, N, K = w.shape
+    launch = (launch_wide_experts if wide_experts_pay(x.shape[0], n, E, N, K, swiglu)
+              else launch_moe_gemm)
+    return launch(x, w, offs, n, row, swiglu)
+
+
 def gemm_bf16(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """C[M,N] = a[M,K] @ w[N,K]^T via the hand-written MFMA kernel."""
     if not _on_gpu(a):

@@ -229,3 +229,14 @@ def test_wide_gemm_operands(x, w, ok):
 ])
 def test_wide_gemm_pays(M, N, K, glu, pays):
     assert ops._wide_pays(M, N, K, glu) == pays
+
+
+@pytest.mark.parametrize("x_rows,n,E,N,K,glu,pays", [
+    (800, 1600, 8, 28672, 4096, True, True), (799, 1599, 8, 28672, 4096, True, False),
+    (2000, 2000, 8, 4096, 14336, False, True),
+    (1999, 1999, 8, 4096, 14336, False, False),
+    (800, 1600, 8, 128, 4096, True, False), (800, 2000, 8, 4096, 64, False, False),
+    (1 << 19, 1 << 20, 8, 28672, 4096, True, False),      # 4 GB of rows
+])
+def test_wide_experts_pay(x_rows, n, E, N, K, glu, pays):
+    assert ops.wide_experts_pay(x_rows, n, E, N, K, glu) == pays

@@ -1069,9 +1069,12 @@ def test_moe_kernels_refuse_other_operands():
 
 @pytest.mark.parametrize("counts", [
     [1], [32, 33], [0, 288, 0, 289, 3], [17, 0, 64, 65, 192, 193, 256, 257],
-    [600, 1, 2, 900], [0] * 63 + [290]])
-@pytest.mark.parametrize("I,H", [(64, 64), (192, 320), (640, 1152)])
-def test_moe_sorted_products(counts, I, H):
+    [600, 1, 2, 900], [0] * 63 + [290], [1100, 1090, 1110, 1025]])
+@pytest.mark.parametrize("launch,I,H", [
+    (ops.launch_moe_gemm, 64, 64), (ops.launch_moe_gemm, 192, 320),
+    (ops.launch_moe_gemm, 640, 1152), (ops.launch_wide_experts, 128, 256),
+    (ops.launch_wide_experts, 192, 320), (ops.launch_wide_experts, 640, 1152)])
+def test_moe_sorted_products(counts, launch, I, H):
     """Both projections over sorted rows at the edges of their row classes and row
     tiles, with empty experts, partial blocks of weights and fewer pieces of K than
     the ring holds.  Tolerance: bf16 rounding of the result (2^-8 relative, 2^-7
@@ -1083,8 +1086,8 @@ def test_moe_sorted_products(counts, I, H):
                      rnd(E, H, I, seed=H, scale=0.3))
     offs = torch.tensor([0] + counts, device=DEV).cumsum(0).int()
     row = torch.randint(0, T, (n,), device=DEV, dtype=torch.int32)
-    act = ops.launch_moe_gemm(x, gate_up, offs, n, row, swiglu=True)
-    y = ops.launch_moe_gemm(act, down, offs, n)
+    act = launch(x, gate_up, offs, n, row, swiglu=True)
+    y = launch(act, down, offs, n)
     at = 0
     for e, c in enumerate(counts):
         s = slice(at, at + c)
