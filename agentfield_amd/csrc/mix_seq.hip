@@ -539,13 +539,14 @@ __global__ void __launch_bounds__(256) diff_combine_kernel(
 // linear_scan_kernel, few tokens per sequence: bound by moving the state; thread
 // (r, c) = (tid >> 4, tid & 15) has columns c and c + 16, so that a state row
 // moves in 64-byte pieces; partial outputs meet in LDS after the block of tokens.
-// linear_scan_prompt_kernel: bound by a token's latency on one wave per SIMD (48
-// multiply-adds of four clocks at 128 rows); the row groups are the 16 lanes of a
-// DPP row, so the sum over rows needs no LDS and no second barrier.
+// linear_scan_prompt_kernel: bound by vector instructions, 40 per token and wave on two
+// waves per SIMD beside the staging (a fifth); the row groups are the 16 lanes of a
+// DPP row, so the sum over rows needs no LDS and no second barrier.  A constant decay
+// is not staged.
 // Six sequences of 500..1900 tokens, 8 heads of 128 x 128, decays per channel:
-// 787 -> 385 us; 16 heads, one decay per head, rotary: 770 -> 497 us
-// (the row layout alone: 711 and 698; element loads that were converted at once
-// made every block wait for its successor).
+// 787 -> 336 us; 16 heads, one decay per head, rotary: 770 -> 447 us (one wave per SIMD
+// with two columns per thread 385 and 497; the row layout alone 711 and 698; element
+// loads that were converted at once made every block wait for its successor).
 // v plus the sum over the other lanes of its 16-lane row, in all of them
 __device__ __forceinline__ float row16_sum_all(float v) {
 #define AFM_ROR(N)                                                           \
@@ -780,13 +781,17 @@ __global__ void __launch_bounds__(256) linear_scan_kernel(
   }
 }
 
+// Threads of the prompt kernel: with one column each two waves share a SIMD and fill one
+// another's waits; below 128 rows the staged pieces would be smaller than a load.
+constexpr int scan_threads(int rp) { return rp >= 8 ? 512 : 256; }
+
 // The same recurrence for prompts.  A thread stages E consecutive rows of one token
 // (one wide load each for q, k, the rotary partners and the decay logits, kept raw
 // until the block before has been worked through) and computes RP rows of two
 // columns; lane j of a 16-lane row keeps token j's sum.  Two LDS buffers, one
 // barrier per block of tokens.
-template <typename S, int RP>
-__global__ void __launch_bounds__(256, 2) linear_scan_prompt_kernel(
+template <typename S, int RP, bool ZL>
+__global__ void __launch_bounds__(scan_threads(RP), RP == 8 && sizeof(S) == 2 ? 4 : 2) linear_scan_prompt_kernel(
     float* __restrict__ out, float* __restrict__ state,
     const S* __restrict__ q, const S* __restrict__ k, const S* __restrict__ v,
     const S* __restrict__ zl, const float* __restrict__ zbias,
@@ -798,23 +803,25 @@ __global__ void __launch_bounds__(256, 2) linear_scan_prompt_kernel(
   constexpr int DKP = 16 * RP;
   constexpr bool FAST = sizeof(S) == 2;
   constexpr int TB = RP >= 16 ? 8 : 16;
-  constexpr int E = TB * DKP / 256;            // staged rows per thread
+  constexpr int NT = scan_threads(RP), CPT = 512 / NT;   // columns per thread
+  constexpr int E = TB * DKP / NT;             // staged rows per thread
   constexpr int BUF = TB * (3 * DKP + 32);     // [TB][3][DKP], [TB][32]
   extern __shared__ float smem[];
   const int b = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * 32;
   const int t0 = cu[b], t1 = cu[b + 1];
   if (t1 <= t0) return;
   const int r = threadIdx.x & 15, cc = threadIdx.x >> 4;
-  const int ca = c0 + 2 * cc, cb = ca + 1;
-  const bool oka = ca < dv, okb = cb < dv;
+  const int ca = c0 + CPT * cc;
   float* sbase = state + (((size_t)sslot[b] * H + h) * dk) * dv;
-  float sta[RP], stb[RP];
+  float state_of[CPT][RP];
   const bool fresh = q_start[b] == 0;
 #pragma unroll
   for (int ii = 0; ii < RP; ++ii) {
     const int i = r * RP + ii;
-    sta[ii] = (!fresh && oka && i < dk) ? sbase[(size_t)i * dv + ca] : 0.f;
-    stb[ii] = (!fresh && okb && i < dk) ? sbase[(size_t)i * dv + cb] : 0.f;
+#pragma unroll
+    for (int c = 0; c < CPT; ++c)
+      state_of[c][ii] = (!fresh && ca + c < dv && i < dk)
+                            ? sbase[(size_t)i * dv + ca + c] : 0.f;
   }
 
   // what this thread stages: rows i0 .. i0+E-1 of token st of a block, and two
@@ -830,12 +837,12 @@ __global__ void __launch_bounds__(256, 2) linear_scan_prompt_kernel(
 #pragma unroll
   for (int j = 0; j < E; ++j) {
     frq[j] = turn ? inv_freq[(lowh ? i0 : i0 - half) + j] : 0.f;
-    bias[j] = zl ? zbias[(size_t)h * dk + ic + j] : 0.f;
+    bias[j] = ZL ? zbias[(size_t)h * dk + ic + j] : 0.f;
   }
   const float hd = head_decay ? head_decay[h] : 1.0f;
   const S* qh = q + (size_t)h * dk;
   const S* kh = k + (size_t)h * dk;
-  const S* zh = zl ? zl + (size_t)h * dk : nullptr;
+  const S* zh = ZL ? zl + (size_t)h * dk : nullptr;
   const S* vh = v + (size_t)h * dv;
   Raw rq, rk, rqp, rkp, rz;
   S rv[2];
@@ -851,7 +858,7 @@ __global__ void __launch_bounds__(256, 2) linear_scan_prompt_kernel(
       rkp = wide(kh + t * ldk + pi);
       rpos = positions[t];
     }
-    if (zl) rz = wide(zh + t * ldz + ic);
+    if (ZL) rz = wide(zh + t * ldz + ic);
     if (vt < TB) {
       const S* vp = vh + (size_t)min(tb + vt, t1 - 1) * ldv;
       rv[0] = vp[min(vc, dv - 1)];
@@ -881,7 +888,7 @@ __global__ void __launch_bounds__(256, 2) linear_scan_prompt_kernel(
         kv[j] = turn ? y : kv[j];
       }
     }
-    if (zl) {
+    if (ZL) {
 #pragma unroll
       for (int j = 0; j < E; ++j)
         av[j] = scan_decay<FAST>(ldf<S>(&rz.x[j]) + bias[j], inv_tau);
@@ -902,14 +909,15 @@ __global__ void __launch_bounds__(256, 2) linear_scan_prompt_kernel(
         const int at = (((w0 + w) >> 2) * 16 + g) * 4;
         *reinterpret_cast<f32x4*>(row + at) = f32x4{qv[w], qv[w + 1], qv[w + 2], qv[w + 3]};
         *reinterpret_cast<f32x4*>(row + DKP + at) = f32x4{kv[w], kv[w + 1], kv[w + 2], kv[w + 3]};
-        *reinterpret_cast<f32x4*>(row + 2 * DKP + at) = f32x4{av[w], av[w + 1], av[w + 2], av[w + 3]};
+        if (ZL)
+          *reinterpret_cast<f32x4*>(row + 2 * DKP + at) = f32x4{av[w], av[w + 1], av[w + 2], av[w + 3]};
       }
     } else {
 #pragma unroll
       for (int w = 0; w < E; ++w) {
         row[i0 + w] = qv[w];
         row[DKP + i0 + w] = kv[w];
-        row[2 * DKP + i0 + w] = av[w];
+        if (ZL) row[2 * DKP + i0 + w] = av[w];
       }
     }
     if (vt < TB) {
@@ -931,8 +939,10 @@ __global__ void __launch_bounds__(256, 2) linear_scan_prompt_kernel(
     }
     const float* sb = smem + cur;
     const float* vb = sb + TB * 3 * DKP;
-    float oa = 0.f, ob = 0.f;
-    struct Token { float q[RP], k[RP], a[RP]; f32x2 v; };
+    float o[CPT];
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) o[c] = 0.f;
+    struct Token { float q[RP], k[RP], a[RP], v[CPT]; };
     auto read = [&](int tt) {
       const float* sq = sb + (size_t)tt * 3 * DKP;
       Token t;
@@ -942,7 +952,8 @@ __global__ void __launch_bounds__(256, 2) linear_scan_prompt_kernel(
           const int at = ((w >> 2) * 16 + r) * 4;
           const f32x4 q4 = *reinterpret_cast<const f32x4*>(sq + at);
           const f32x4 k4 = *reinterpret_cast<const f32x4*>(sq + DKP + at);
-          const f32x4 a4 = *reinterpret_cast<const f32x4*>(sq + 2 * DKP + at);
+          f32x4 a4 = {hd, hd, hd, hd};
+          if (ZL) a4 = *reinterpret_cast<const f32x4*>(sq + 2 * DKP + at);
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             t.q[w + j] = q4[j];
@@ -955,23 +966,27 @@ __global__ void __launch_bounds__(256, 2) linear_scan_prompt_kernel(
         for (int w = 0; w < RP; ++w) {
           t.q[w] = sq[r * RP + w];
           t.k[w] = sq[DKP + r * RP + w];
-          t.a[w] = sq[2 * DKP + r * RP + w];
+          t.a[w] = ZL ? sq[2 * DKP + r * RP + w] : hd;
         }
       }
-      t.v = *reinterpret_cast<const f32x2*>(vb + tt * 32 + 2 * cc);
+#pragma unroll
+      for (int c = 0; c < CPT; ++c) t.v[c] = vb[tt * 32 + CPT * cc + c];
       return t;
     };
     auto step = [&](int tt, const Token& t) {
-      float pa = 0.f, pb = 0.f;
+      float part[CPT];
 #pragma unroll
-      for (int ii = 0; ii < RP; ++ii) {
-        scan_row(sta[ii], pa, t.a[ii], t.k[ii], t.v[0], t.q[ii]);
-        scan_row(stb[ii], pb, t.a[ii], t.k[ii], t.v[1], t.q[ii]);
+      for (int c = 0; c < CPT; ++c) part[c] = 0.f;
+#pragma unroll
+      for (int ii = 0; ii < RP; ++ii)
+#pragma unroll
+        for (int c = 0; c < CPT; ++c)
+          scan_row(state_of[c][ii], part[c], t.a[ii], t.k[ii], t.v[c], t.q[ii]);
+#pragma unroll
+      for (int c = 0; c < CPT; ++c) {
+        part[c] = row16_sum_all(part[c]);
+        o[c] = r == tt ? part[c] : o[c];
       }
-      pa = row16_sum_all(pa);
-      pb = row16_sum_all(pb);
-      oa = r == tt ? pa : oa;
-      ob = r == tt ? pb : ob;
     };
     if (nt == TB) {
       // the next token's LDS reads run under this one's arithmetic: the fence
@@ -989,8 +1004,9 @@ __global__ void __launch_bounds__(256, 2) linear_scan_prompt_kernel(
     }
     if (r < nt) {
       float* op = out + (size_t)(tb + r) * H * dv + (size_t)h * dv;
-      if (oka) op[ca] = oa;
-      if (okb) op[cb] = ob;
+#pragma unroll
+      for (int c = 0; c < CPT; ++c)
+        if (ca + c < dv) op[ca + c] = o[c];
     }
     __syncthreads();  // the next buffer is filled, this one read
     cur ^= BUF;
@@ -998,8 +1014,9 @@ __global__ void __launch_bounds__(256, 2) linear_scan_prompt_kernel(
 #pragma unroll
   for (int ii = 0; ii < RP; ++ii) {
     const int i = r * RP + ii;
-    if (i < dk && oka) sbase[(size_t)i * dv + ca] = sta[ii];
-    if (i < dk && okb) sbase[(size_t)i * dv + cb] = stb[ii];
+#pragma unroll
+    for (int c = 0; c < CPT; ++c)
+      if (i < dk && ca + c < dv) sbase[(size_t)i * dv + ca + c] = state_of[c][ii];
   }
 }
 
@@ -1207,7 +1224,7 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
   // From a block of tokens per sequence on the prompt kernel is the better one
   // (see there); its loads take E rows at once, so heads, halves of the rotated
   // part, strides and bases must be multiples of E elements (16 bytes at most).
-  const int E = rpp >= 8 ? 8 : rpp;
+  const int E = rpp >= 4 ? 4 : rpp;
   const size_t al = E * sizeof(S) < 16 ? E * sizeof(S) : 16;
   const bool prompt =
       T >= 16 * B && dk % E == 0 && (rot / 2) % E == 0 && ldq % E == 0 &&
@@ -1221,8 +1238,12 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
       inv_tau, H, dk, dv, rot, ldq, ldk, ldv, ldz
 #define SCAN(RP)                                                             \
   do {                                                                       \
-    if (prompt)                                                              \
-      linear_scan_prompt_kernel<S, RP><<<grid, 256, sm, s>>>(SCAN_ARGS);     \
+    if (prompt && zl)                                                        \
+      linear_scan_prompt_kernel<S, RP, true>                                 \
+          <<<grid, scan_threads(RP), sm, s>>>(SCAN_ARGS);                    \
+    else if (prompt)                                                         \
+      linear_scan_prompt_kernel<S, RP, false>                                \
+          <<<grid, scan_threads(RP), sm, s>>>(SCAN_ARGS);                    \
     else                                                                     \
       linear_scan_kernel<S, RP><<<grid, 256, sm, s>>>(SCAN_ARGS);            \
   } while (0)
