@@ -523,6 +523,10 @@ def _wide_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
             and x.device == w.device and rows_operands_ok((x, w)))
 
 
+def _wide_out_ok(out: torch.Tensor, x: torch.Tensor, M: int, N: int) -> bool:
+    return _whole(out, x, M, N) and _apart(out, x) and out.data_ptr() & 15 == 0
+
+
 def _wide_pays(M: int, N: int, K: int, silu_fuse: bool) -> bool:
     """Whether the wide GEMM beats the library's, by 256 x 256 tiles per round of
     256 blocks, from 15 projections of four models at 256..9000 rows.
@@ -582,8 +586,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
     if (M > 128 and x.is_cuda and x.dim() == 2 == w.dim()
             and _wide_pays(M, N, x.shape[1], silu_fuse)
             and not watched(x, w, grad=not silu_fuse)
-            and (out is None or _whole(out, x, M, N) and _apart(out, x)
-                 and out.data_ptr() & 15 == 0)
+            and (out is None or _wide_out_ok(out, x, M, N))
             and _wide_ok(x, w)):
         return launch_wide(x, w, silu_fuse, out)
     if out is not None:

@@ -669,11 +669,12 @@ def softcap(logits: torch.Tensor, cap: float) -> torch.Tensor:
 def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
            out: torch.Tensor | None = None) -> torch.Tensor:
     """x [M, K] @ w [N, K]^T; fp32 operands run in true fp32 (no reduced-
-    precision matrix mode).  out: rows to write to (always the vendor GEMM).
+    precision matrix mode).  out: rows to write to (above 128 rows, the wide GEMM or
+    the vendor's; below, always the vendor's).
 
     bf16 products of few rows (decode steps) run on the framework's
     weight-streaming kernels, wider ones and prompts on the vendor GEMM
-    (hipBLASLt / rocBLAS).  Above 16 rows a second launch adds the K splits up
+    (hipBLASLt / rocBLAS) or, where that has begun a round, on the wide GEMM.  Above 16 rows a second launch adds the K splits up
     unless N fills the chip by itself, which middling widths do not earn back.
     Measured, vendor against rows in us: 4096 x 4096 15.7 / 7.8 at 4 rows, 15.3 /
     12.7 at 64, 16.2 / 18.2 at 100; 6144 x 2048 12.8 / 11.0 at 32, 13.2 / 13.9 at
@@ -684,10 +685,15 @@ def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
     decode-sized products (up to 64 rows, or 33..128 against a long inner dimension)
     to the framework's kernels too.  What autograd or a transform has to see is
     the vendor GEMM's (watched)."""
-    if out is not None:
-        return torch.mm(x, w.t(), out=out)
     M, K = x.shape
     N = w.shape[0]
+    if (M > 128 and skinny and x.is_cuda and _lib.main_lib_ready()
+            and _ops._wide_pays(M, N, K, False) and not _ops.watched(x, w)
+            and (out is None or _ops._wide_out_ok(out, x, M, N))
+            and _ops._wide_ok(x, w)):
+        return _ops.launch_wide(x, w, out=out)
+    if out is not None:
+        return torch.mm(x, w.t(), out=out)
     if skinny and x.is_cuda and M <= 128 and _lib.main_lib_ready():
         if ((M <= 32 or M <= 64 and N <= 4096 or N >= 24576)
                 and not _ops.watched(x, w) and _ops._rows_ok(x, w)):
