@@ -128,6 +128,22 @@ __device__ __forceinline__ int find_item(const PrefillArgs& a, int item, int* at
   return -1;
 }
 
+// An entry of the block table whose index the wave shares, as a scalar load: after an LDS
+// load the compiler makes it a vector load, and the wait for that drains the tile's loads.
+__device__ __forceinline__ int table_entry(const i32* row, int i) {
+  typedef const __attribute__((address_space(4))) i32 table_t;
+  return ((table_t*)row)[__builtin_amdgcn_readfirstlane(i)];
+}
+
+// All but n of a wave's loads have landed, where the compiler can see it: it would wait
+// for the next tile's loads as well in front of this tile's reads.
+template <int N>
+__device__ __forceinline__ void landed() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4) << 14 | 0x0f70);
+  asm volatile("" ::: "memory");
+}
+
 // Rows [row0, row0 + 4*N) of a K and a V tile whose first token is t0 into LDS:
 // every instruction brings 4 rows (1 KB).  Tokens behind the last one repeat it
 // (their weights are 0 and must meet finite values).
@@ -343,7 +359,7 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_kernel(PrefillArgs a,
   int kt = a.win > 0 ? max(0, hist + q0 - a.win + 1) / AP_KV : 0;
   auto page_of = [&](int tile) {
     const int t = min(tile, ntiles - 1) * AP_KV;
-    return btrow[a.page_shift >= 0 ? t >> a.page_shift : t / a.page_size];
+    return table_entry(btrow, a.page_shift >= 0 ? t >> a.page_shift : t / a.page_size);
   };
   stage<TILED, 4>(a, btrow, kvh, kt * AP_KV, wid * 16, last,
                   TILED ? page_of(kt) : 0, kbuf(0), vbuf(0));
@@ -397,10 +413,11 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_few_kernel(
   const i32* btrow = a.bt + (size_t)seq * a.max_pages;
 
   constexpr int TILE = AP_FEW * AP_ROWB, WROWS = 32 / G;
-  __shared__ __attribute__((aligned(16))) char lds[4][2][2][TILE];
-  __shared__ float s_m[4][32], s_l[4][32];
-  auto kbuf = [&](int i) { return (lds_char*)&lds[wid][i][0][0]; };
-  auto vbuf = [&](int i) { return (lds_char*)&lds[wid][i][1][0]; };
+  // one array: with a second one the compiler waits for all loads before it reads
+  __shared__ __attribute__((aligned(16))) char lds[4 * 4 * TILE + 1024];
+  float (*s_m)[32] = reinterpret_cast<float (*)[32]>(lds + 16 * TILE), (*s_l)[32] = s_m + 4;
+  auto kbuf = [&](int i) { return (lds_char*)&lds[(wid * 4 + i * 2) * TILE]; };
+  auto vbuf = [&](int i) { return (lds_char*)&lds[(wid * 4 + i * 2 + 1) * TILE]; };
 
   const int col = lane & 31;
   const int row = at * WROWS + col / G, qh = kvh * G + col % G;
@@ -415,7 +432,7 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_few_kernel(
   const int step = 4 * nsplit;
   auto page_of = [&](int tile) {
     const int t = min(tile, ntiles - 1) * AP_FEW;
-    return btrow[a.page_shift >= 0 ? t >> a.page_shift : t / a.page_size];
+    return table_entry(btrow, a.page_shift >= 0 ? t >> a.page_shift : t / a.page_size);
   };
   int kt = first + (int)blockIdx.y * 4 + wid, page = 0, cur = 0;
   if (kt < ntiles) {
@@ -428,11 +445,9 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_few_kernel(
       stage<TILED, 8>(a, btrow, kvh, (kt + step) * AP_FEW, 0, last, page,
                       kbuf(cur ^ 1), vbuf(cur ^ 1));
       if (TILED) page = page_of(kt + 2 * step);
-      // the tile has landed when only the 16 loads just issued are out (with TILED
-      // the wait for the page index has drained those too)
-      asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+      landed<16>();      // all but the 16 loads just issued
     } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      landed<0>();
     }
     const int t0 = kt * AP_FEW;
     attend<1, true>(c, kbuf(cur), vbuf(cur), t0, sc, a.win,
@@ -445,7 +460,7 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_few_kernel(
   // merge the waves: O^T as [wave][column][dim] in the tile buffers
   const float l = c.l + __shfl_xor(c.l, 32, 64);
   __syncthreads();
-  float* so = reinterpret_cast<float*>(&lds[0][0][0][0]);
+  float* so = reinterpret_cast<float*>(lds);
   if (lane < 32) { s_m[wid][col] = c.m; s_l[wid][col] = l; }
   float* mine = so + (size_t)(wid * 32 + col) * AP_D + 4 * (lane >> 5);
 #pragma unroll
