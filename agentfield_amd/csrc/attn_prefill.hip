@@ -40,13 +40,15 @@
 //     waves split the keys, each with private 32-token double buffers and no
 //     barrier in the loop, and merge through LDS; with fewer than 256 blocks the
 //     keys are also split over blocks and a second kernel merges.  Bound by the
-//     latency of its transfers, which nothing hides (128 KB of LDS, one block per
-//     CU): ~3.5 TB/s of K/V where decode attention reaches 5.  P is kept to 16 bits
+//     latency of its transfers, which half a tile hides (129 KB of LDS, one block per
+//     CU): ~4.2 TB/s of K/V where decode attention reaches 5.  P is kept to 16 bits
 //     more: two bf16 terms, two products.
-// Transfers: where pages hold whole tiles, the page of the tile after next is looked
-// up behind the next tile's loads.  The compiler makes that a vector load, and the
-// wait for it drains the tile's loads with it, before this tile's arithmetic starts:
-// they overlap with the other block of the CU only.
+// Transfers: where pages hold whole tiles, the page of the tile after next is a scalar
+// lookup behind the next tile's loads (as a vector load its wait drained them before
+// this tile's arithmetic: 672 us and 43.9 against 628 and 37.0, one prompt of 8000 rows
+// and 16 sequences of 5 rows behind up to 3000).  The compiler still waits for them in
+// front of the transposing reads, half a tile later; loads it does not know of changed
+// little (628, 35.9).
 // Fragment layouts (measured): A: lane holds A[m=lane&31][k=(lane>>5)*8+j]; B:
 // B[k=(lane>>5)*8+j][n=lane&31]; C: reg r holds C[8*(r/4)+4*(lane>>5)+r%4][lane&31];
 // transposing read: lane i of a group of 16 gets column i of 4 rows x 16 columns
