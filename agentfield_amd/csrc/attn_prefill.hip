@@ -31,7 +31,7 @@
 //     the block and double-buffered (64 KB, two blocks per CU: one wave's
 //     exponentials run under the other's MFMA).  Bound by vector issue next to
 //     the matrix cores (32 exponentials per lane and tile alone take half of the
-//     tile's MFMA time) and by the transfers, see below.  grid: K/V head fastest,
+//     tile's MFMA time, during which the cores are busy half of the time).  grid: K/V head fastest,
 //     so with 8 of them an XCD's L2 keeps one head's K/V; late (long) tiles start
 //     first.
 //   attn_prefill_few_kernel  32 columns per block: sequences whose columns fit
@@ -46,7 +46,7 @@
 // Transfers: where pages hold whole tiles, the page of the tile after next is a scalar
 // lookup behind the next tile's loads (as a vector load its wait drained them before
 // this tile's arithmetic: 672 us and 43.9 against 628 and 37.0, one prompt of 8000 rows
-// and 16 sequences of 5 rows behind up to 3000).  The compiler still waits for them in
+// and 16 sequences of 5 rows behind up to 3000; with attend() as it is now 544 and 36.6).  The compiler still waits for them in
 // front of the transposing reads, half a tile later; loads it does not know of changed
 // little (628, 35.9).
 // Fragment layouts (measured): A: lane holds A[m=lane&31][k=(lane>>5)*8+j]; B:
@@ -56,8 +56,8 @@
 //
 // Against 16x16x32 tiles of 64 columns with P through LDS and V transposed by
 // scalar writes (one layer, 8 K/V heads, G = 4): one prompt of 8000 rows 2292 ->
-// 679 us (229 -> 772 TFLOP/s), 20 of 300..700 384 -> 110 us, 8 x 2048 at G = 2
-// 992 -> 232 us; 16 sequences of 5 rows behind 2400 tokens 387 -> 51 us.
+// 544 us (229 -> 960 TFLOP/s), 20 of 300..700 384 -> 104 us, 8 x 2048 at G = 2
+// 992 -> 232 us; 16 sequences of 5 rows behind 2400 tokens 387 -> 43 us.
 #include "common.h"
 
 #define AP_D 128
@@ -183,6 +183,20 @@ __device__ __forceinline__ void stage(const PrefillArgs& a, const i32* btrow,
   }
 }
 
+// o += a b, in place: left to itself the compiler puts the result elsewhere and copies 64
+// registers back per tile (together with the maximum in attend() 582 -> 569 us for one
+// prompt of 8000 rows, 105 -> 93 for 20 of 300..700).  Two wait states for operands that were just written; who reads
+// the sums other than as a sum again is behind settled().
+__device__ __forceinline__ void add_product(f32x16& o, bf16x8 a, bf16x8 b) {
+  asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
+               : "+v"(o) : "v"(a), "v"(b));
+}
+
+// The matrix cores are done with the sums.
+__device__ __forceinline__ void settled(f32x16 (&o)[4]) {
+  asm volatile("s_nop 15\n\ts_nop 15" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]));
+}
+
 // A wave's columns and their running softmax.
 struct Columns {
   s16x8 q[8];       // B operand, 8 x 16 dims
@@ -234,14 +248,18 @@ __device__ __forceinline__ void attend(Columns& c, const lds_char* kl,
           s[b][r] = -__builtin_inff();  // weight 0 under any positive scale
       }
   }
-  float mx = AF_NEG_INF;
+  // as a median with infinity: fmaxf first quiets NaNs that cannot signal, one more
+  // instruction per score
+  float mx[2] = {AF_NEG_INF, AF_NEG_INF};
 #pragma unroll
   for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int r = 0; r < 16; r += 2) mx = fmaxf(mx, fmaxf(s[b][r], s[b][r + 1]));
-  mx = swap_max(mx);
-  if (__any((mx - c.m) * sc > 6.f)) {
-    const float mn = fmaxf(c.m, mx);
+    for (int r = 0; r < 16; ++r)
+      mx[r & 1] = __builtin_amdgcn_fmed3f(mx[r & 1], s[b][r], __builtin_inff());
+  const float top = swap_max(fmaxf(mx[0], mx[1]));
+  if (__any((top - c.m) * sc > 6.f)) {
+    settled(c.o);
+    const float mn = fmaxf(c.m, top);
     const float corr = __builtin_amdgcn_exp2f((c.m - mn) * sc);
     c.m = mn;
     c.l *= corr;
@@ -268,31 +286,40 @@ __device__ __forceinline__ void attend(Columns& c, const lds_char* kl,
   VF vf[2][4];
   read_v(0, vf[0]);
   float sum0 = 0.f, sum1 = 0.f;
-#pragma unroll
-  for (int k = 0; k < NB * 2; ++k) {  // 16 tokens
-    if (k + 1 < NB * 2) read_v(k + 1, vf[(k + 1) & 1]);
-    float p[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      p[j] = __builtin_amdgcn_exp2f(fmaf(s[k / 2][(k & 1) * 8 + j], sc, mz));
-#pragma unroll
-    for (int j = 0; j < 8; j += 2) { sum0 += p[j]; sum1 += p[j + 1]; }
-    bf16x8 pf, pr;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      pf[j] = (__bf16)p[j];
-      if (FINE) pr[j] = (__bf16)(p[j] - (float)pf[j]);
+  bf16x8 pf[2], pr[2];
+  auto weigh = [&](int k, int u) {  // tokens 2u, 2u + 1 of the k-th 16
+    const int r = (k & 1) * 8 + 2 * u;
+    const float p0 = __builtin_amdgcn_exp2f(fmaf(s[k / 2][r], sc, mz));
+    const float p1 = __builtin_amdgcn_exp2f(fmaf(s[k / 2][r + 1], sc, mz));
+    sum0 += p0;
+    sum1 += p1;
+    bf16x8 &f = pf[k & 1], &e = pr[k & 1];
+    f[2 * u] = (__bf16)p0;
+    f[2 * u + 1] = (__bf16)p1;
+    if (FINE) {
+      e[2 * u] = (__bf16)(p0 - (float)f[2 * u]);
+      e[2 * u + 1] = (__bf16)(p1 - (float)f[2 * u + 1]);
     }
+  };
+#pragma unroll
+  for (int u = 0; u < 4; ++u) weigh(0, u);
+  // a wave that has its weights goes first, so that the two of a SIMD do not multiply and
+  // exponentiate in step (553 -> 535 us)
+  __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+  for (int k = 0; k < NB * 2; ++k) {  // 16 tokens; the next ones' weights in between, or
+                                      // MFMA and vector unit take turns (569 -> 553 us)
+    if (k + 1 < NB * 2) read_v(k + 1, vf[(k + 1) & 1]);
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
-      c.o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[k & 1][d].b, pf, c.o[d],
-                                                       0, 0, 0);
-      if (FINE)
-        c.o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[k & 1][d].b, pr,
-                                                         c.o[d], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      add_product(c.o[d], vf[k & 1][d].b, pf[k & 1]);
+      if (FINE) add_product(c.o[d], vf[k & 1][d].b, pr[k & 1]);
+      if (k + 1 < NB * 2) weigh(k + 1, d);
     }
     __builtin_amdgcn_sched_barrier(0);
   }
+  __builtin_amdgcn_s_setprio(0);
   c.l += sum0 + sum1;
 }
 
@@ -383,6 +410,7 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_kernel(PrefillArgs a,
     cur ^= 1;
   }
 
+  settled(c.o);
   const float l = c.l + __shfl_xor(c.l, 32, 64);
   if (row >= len) return;
   const float inv = (l > 0.f) ? 1.f / l : 0.f;
@@ -460,6 +488,7 @@ __global__ void __launch_bounds__(256, 1) attn_prefill_few_kernel(
   }
 
   // merge the waves: O^T as [wave][column][dim] in the tile buffers
+  settled(c.o);
   const float l = c.l + __shfl_xor(c.l, 32, 64);
   __syncthreads();
   float* so = reinterpret_cast<float*>(lds);
