@@ -476,9 +476,8 @@ class LlamaForCausalLM(nn.Module):
                     ss.zero_()
                     ss[:, 0] = residual.float().pow(2).sum(-1)
             if logit_rows is not None:
-                residual = ops.gather_rows(residual, logit_rows)
-            h = ops.rmsnorm(residual, self.final_norm, self.cfg.rms_eps)
-            return self._project_logits(h)
+                residual, ss = ops.gather_rows(residual, logit_rows), None
+            return self._logits_rows_fused(residual, ss)
         h = ops.embedding(ids, self.embed)
         residual = None
         for layer in self.layers:
@@ -487,6 +486,19 @@ class LlamaForCausalLM(nn.Module):
         if logit_rows is not None:
             h = ops.gather_rows(h, logit_rows)
         return self._project_logits(h)
+
+    def _logits_rows_fused(self, residual, ss):
+        """Logits of a few residual rows, the final norm (folded) as a scalar of the
+        vocabulary product where that can have it."""
+        few, eps = residual.shape[0] <= ops.ROWS_MAX, self.cfg.rms_eps
+        if ((few or ss is not None)
+                and not getattr(self, "_tp_vocab_parallel", False)
+                and not ops.watched(residual, self.lm_head)
+                and ops.rows_pay(residual.shape[0], self.lm_head.shape[0])
+                and ops._rows_ok(residual, self.lm_head)):
+            return ops.launch_rows(residual, self.lm_head,
+                                   scale=(None if few else ss, eps))
+        return self._project_logits(ops.rmsnorm(residual, self.final_norm, eps))
 
     def _project_logits(self, h: torch.Tensor) -> torch.Tensor:
         """lm_head projection.  Under vocab-parallel TP each rank computes

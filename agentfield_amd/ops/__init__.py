@@ -324,6 +324,17 @@ def _rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
             and rows_operands_ok((x, w)))
 
 
+def rows_pay(M: int, N: int) -> bool:
+    """Whether plain products of up to 128 rows go to the row GEMMs: those of 33..128
+    rows lose to the library where N fills the chip neither in blocks of 128 columns
+    nor in several splits.  Measured, library against rows in us: 14336 x 4096 25.6 / 21.7 at 32 rows, 26.7 / 30.0 at 48,
+    33.9 / 36.0 at 128; 16384 x 4096 34.3 / 24.7, 34.9 / 38.9, 39.0 / 43.3;
+    28672 x 4096 53.9 / 41.5, 64.0 / 42.1, 56.7 / 51.7; 128256 x 4096 190 / 151
+    at one row, 214 / 184 at 64, 238 / 215 at 128.  Between 12288 and 24576
+    these two were measured; the limits are the nearest sizes at which rows win."""
+    return M <= 32 or N <= 12288 or N >= 24576
+
+
 def _need(ok: bool, what: str) -> None:
     if not ok:
         raise AfOpsError(what)
@@ -565,20 +576,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
            out: torch.Tensor | None = None) -> torch.Tensor:
     """Linear layer dispatch: hand-written weight-streaming kernels up to 128
     rows, the wide GEMM or hipBLASLt (torch.matmul) for prefill GEMMs.  out
-    (without silu_fuse): [M, N] rows of x's type to write to.
-
-    Plain products of 33..128 rows lose to the library where N fills the chip
-    neither in blocks of 128 columns nor in several splits.  Measured, library
-    against rows in us: 14336 x 4096 25.6 / 21.7 at 32 rows, 26.7 / 30.0 at 48,
-    33.9 / 36.0 at 128; 16384 x 4096 34.3 / 24.7, 34.9 / 38.9, 39.0 / 43.3;
-    28672 x 4096 53.9 / 41.5, 64.0 / 42.1, 56.7 / 51.7; 128256 x 4096 190 / 151
-    at one row, 214 / 184 at 64, 238 / 215 at 128.  Between 12288 and 24576
-    these two were measured; the limits are the nearest sizes at which rows win."""
+    (without silu_fuse): [M, N] rows of x's type to write to."""
     M, N = x.shape[0], w.shape[0]
     if out is not None and (silu_fuse or out.shape != (M, N)):
         raise AfOpsError(f"linear: out {tuple(out.shape)} for a [{M}, {N}] "
                          "product")
-    if (M <= 128 and (silu_fuse or M <= 32 or N <= 12288 or N >= 24576)
+    if (M <= 128 and (silu_fuse or rows_pay(M, N))
             and x.is_cuda and not watched(x, w, grad=not silu_fuse)
             and (out is None or _whole(out, x, M, N) and _apart(out, x))
             and _rows_ok(x, w)):

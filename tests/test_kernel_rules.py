@@ -240,3 +240,10 @@ def test_wide_gemm_pays(M, N, K, glu, pays):
 ])
 def test_wide_experts_pay(x_rows, n, E, N, K, glu, pays):
     assert ops.wide_experts_pay(x_rows, n, E, N, K, glu) == pays
+
+
+@pytest.mark.parametrize("M,N,pays", [
+    (32, 16384, True), (33, 12288, True), (33, 12352, False), (128, 24512, False),
+    (128, 24576, True)])
+def test_rows_pay(M, N, pays):
+    assert ops.rows_pay(M, N) == pays
