@@ -12,7 +12,8 @@
 // Both operands travel global -> LDS without registers, in whole 128-byte lines, three
 // pieces deep for W and two for X (160 KB).  Loads are spread evenly over the products:
 // asked for at once they come back at 64 bytes per clock and the wave stands (4096 x
-// 14336, 4096 rows: 360 us, spread 320).  One barrier per piece.  The stream of loads
+// 14336, 4096 rows: 360 us, spread 320; those of X every 8 products instead of every 4
+// another 0..3%).  One barrier per piece.  The stream of loads
 // runs on into the block's next tile, so only the stores stand between tiles; a lane
 // stores 16 bytes of a row (weight rows are permuted on their way into LDS so that it
 // has eight neighbours), converted by the hardware (4.7 us less per tile).
@@ -180,7 +181,7 @@ __device__ __forceinline__ void wide_tiles(const WideArgs& a, char* lds, int fir
                : "+a"(acc[(c) & 7][(c) >> 3])                                     \
                : "v"(w[s][(c) & 7]), "v"(x[s][(c) >> 3]))
 #define GW_HERE __builtin_amdgcn_sched_barrier(0)
-    // per half: an LDS read every 2 products, X loads every 4, W loads every G
+    // per half: an LDS read every 2 products, a load of X every 8, of W every G
     static_assert(4 * G >= 8 + G, "all operands are read within a half");
 #pragma unroll 1
     for (int i = 0; i < cnt; ++i) {
@@ -230,9 +231,9 @@ __device__ __forceinline__ void wide_tiles(const WideArgs& a, char* lds, int fir
 #pragma unroll
       for (int c = 0; c < 8 * G; ++c) {
         GW_MUL(1, c);
-        if (c % 4 == 2 && c / 4 < G) {
+        if (c % 8 == 4) {
           GW_HERE;
-          load_x(c / 4, xat, ox);
+          load_x(c / 8, xat, ox);
           GW_HERE;
         }
         if (c % 2 == 1 && c / 2 < 8 + G) {
