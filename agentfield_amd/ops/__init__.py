@@ -539,22 +539,25 @@ def _wide_out_ok(out: torch.Tensor, x: torch.Tensor, M: int, N: int) -> bool:
 
 
 def _wide_pays(M: int, N: int, K: int, silu_fuse: bool) -> bool:
-    """Whether the wide GEMM beats the library's, by 256 x 256 tiles per round of
-    256 blocks, from 15 projections of four models at 256..9000 rows.
+    """Whether the wide GEMM beats the library's, by the tiles that its 256 blocks
+    take, from 15 projections of four models at 256..9000 rows.
 
-    With SwiGLU behind it, which the library leaves to a pass of its own: from 64
-    tiles on, the fewest measured (library over wide 0.98..1.61, 1.13 in the mean;
-    14336 x 4096 at 2048 rows 364 us / 360, 4096 rows 720 / 668, 5120 rows 1000 /
-    846).
-    Plain: the library is 5-8% ahead in whole rounds (4096 x 4096 at 8000 rows 179
-    us / 189) and draws level below one, but falls back by up to 1.78 where a round
-    is begun (4096 x 14336 at 4352 rows 720 / 410, 8448 rows 1003 / 700; 6144 x 4096
-    at 8448 rows 393 / 310).  Up to half a round the wide GEMM took 34 of 47 sizes
-    and lost 8% at most; with a long K the library stays behind further (4096 x
-    14336 at 6800 rows 920 / 570, at 7400 970 / 600)."""
-    tiles = -(-M // 256) * -(-N // 256)
+    With SwiGLU behind it, which the library leaves to a pass of its own: where its
+    smallest tiles, 128 x 256, occupy 172 blocks.  7 projections at 256..2300 rows,
+    weights not in cache, library over wide: 0.70..1.00 up to 168 blocks and K of 4096
+    or more (7168 x 4096 at 513 rows 45.5 us / 51.0, 14336 x 4096 at 320 rows 52.9 /
+    58.5), from 172 on 0.93..1.50, 1.13 in the mean (28672 x 4096 at 448 rows 109 / 91,
+    1024 rows 219 / 191, 4096 rows 720 / 668).
+    Plain, by 256 x 256 tiles: the library is 5-8% ahead in whole rounds (4096 x 4096
+    at 8000 rows 179 us / 189) and draws level below one, but falls back by up to 1.78
+    where a round is begun (4096 x 14336 at 4352 rows 720 / 410, 8448 rows 1003 / 700;
+    6144 x 4096 at 8448 rows 393 / 310).  Up to half a round the wide GEMM took 34 of
+    47 sizes and lost 8% at most; with a long K the library stays behind further (4096
+    x 14336 at 6800 rows 920 / 570, at 7400 970 / 600)."""
+    cols = -(-N // 256)
     if silu_fuse:
-        return tiles >= 64
+        return -(-M // 128) * cols >= 172
+    tiles = -(-M // 256) * cols
     begun = tiles & 255
     return tiles > 256 and 0 < begun <= (216 if K >= 2 * N else 128)
 

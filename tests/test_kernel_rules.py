@@ -219,8 +219,8 @@ def test_wide_gemm_operands(x, w, ok):
 
 
 @pytest.mark.parametrize("M,N,K,glu,pays", [
-    (4096, 28672, 4096, True, True), (256, 16384, 2048, True, True),
-    (256, 8192, 4096, True, False),               # 32 tiles: few blocks at work
+    (4096, 28672, 4096, True, True), (384, 14848, 4096, True, True),
+    (384, 14336, 4096, True, False),              # 168 tiles: few blocks at work
     (4096, 4096, 4096, False, False),             # one whole round
     (4097, 4096, 4096, False, True),              # a second one begun
     (6144, 4096, 4096, False, True), (6145, 4096, 4096, False, False),
