@@ -31,7 +31,7 @@ typedef __attribute__((address_space(3))) void lds_v;
 #define GW_BLOCKS 256
 #define GW_COLS 256
 
-enum WideEpi { WIDE_PLAIN = 0, WIDE_SWIGLU = 2 };
+enum WideEpi { WIDE_PLAIN = 0, WIDE_PARTS = 1, WIDE_SWIGLU = 2 };
 
 struct WideArgs {
   u16* out;
@@ -42,6 +42,9 @@ struct WideArgs {
   const i32* offs;         // [E + 1] first sorted row
   const i32* row;          // X row of a sorted row; null: itself
   int E;
+  // WIDE_PARTS: partial sums [splits, M, N], split s over the s-th share of K
+  float* parts;
+  int splits;
 };
 
 // All tiles of a block.  EXPERTS: rows of X are gathered and tiles end with their
@@ -51,14 +54,15 @@ __device__ __forceinline__ void wide_tiles(const WideArgs& a, char* lds, int fir
                                            int rows_e, int end_e) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int XR = 32 * G, WB = GW_COLS * 128, XB = XR * 128;
-  constexpr bool GLU = EPI == WIDE_SWIGLU;
+  constexpr bool GLU = EPI == WIDE_SWIGLU, PARTS = EPI == WIDE_PARTS;
   constexpr int OUT = GLU ? GW_COLS / 2 : GW_COLS;         // output columns per tile
   lds_b* const wring = (lds_b*)lds;
   lds_b* const xring = wring + 3 * WB;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, n = lane & 15, q = lane >> 4, r8 = lane >> 3;
-  const int nt = EXPERTS ? __builtin_amdgcn_readlane(end_e, a.E - 1) : a.tm * a.tn;
-  const int cnt = a.K >> 6, cols = GLU ? a.N >> 1 : a.N;
+  const int nt = EXPERTS ? __builtin_amdgcn_readlane(end_e, a.E - 1)
+                         : a.tm * a.tn * (PARTS ? a.splits : 1);
+  const int cnt = PARTS ? (a.K >> 6) / a.splits : a.K >> 6, cols = GLU ? a.N >> 1 : a.N;
   const unsigned ld = (unsigned)a.K * 2;
 
   // Rounds of 256 tiles; an XCD's 32 blocks take 8 x 4 neighbours, which share their
@@ -67,9 +71,9 @@ __device__ __forceinline__ void wide_tiles(const WideArgs& a, char* lds, int fir
   // tile of a row (M >= XR).
   const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
   auto tile = [&](int round) { return (round * 8 + xcd) * (GW_BLOCKS / 8) + idx; };
-  struct Place { int e, row, rows, fresh, tn; };           // rows from fresh on are new
+  struct Place { int e, row, rows, fresh, tn, split; };           // rows from fresh on are new
   auto place = [&](int p) {
-    Place at = {0, 0, a.M, 0, 0};
+    Place at = {0, 0, a.M, 0, 0, 0};
     int tm = a.tm;
     if (EXPERTS) {
       at.e = __builtin_ctzll(__ballot(p < end_e));         // the first that ends behind p
@@ -77,6 +81,10 @@ __device__ __forceinline__ void wide_tiles(const WideArgs& a, char* lds, int fir
       at.rows = __builtin_amdgcn_readlane(rows_e, at.e);
       tm = (at.rows + XR - 1) / XR;
       p -= __builtin_amdgcn_readlane(end_e, at.e) - tm * a.tn;
+    }
+    if (PARTS) {
+      at.split = p / (a.tm * a.tn);
+      p -= at.split * a.tm * a.tn;
     }
     const int band = p / (8 * a.tn), high = min(8, tm - band * 8), in = p - band * 8 * a.tn;
     const int t = band * 8 + in % high, r = EXPERTS ? t * XR : min(t * XR, a.M - XR);
@@ -101,12 +109,14 @@ __device__ __forceinline__ void wide_tiles(const WideArgs& a, char* lds, int fir
 #pragma unroll
       for (int g = 0; g < G; ++g) xg[g] = xgn[g] * ld + ((lane & 7) ^ r8) * 16;
     } else {
-      xb = (const char*)(a.X + (size_t)place(p).row * a.K);
+      const Place at = place(p);
+      xb = (const char*)(a.X + (size_t)at.row * a.K + (PARTS ? at.split * cnt * 64 : 0));
     }
   };
   auto aim_w = [&](int p) {
     const Place at = place(p);
-    wb = (const char*)(a.W + ((size_t)at.e * a.N + min(at.tn * OUT, cols - OUT)) * a.K);
+    wb = (const char*)(a.W + ((size_t)at.e * a.N + min(at.tn * OUT, cols - OUT)) * a.K +
+                       (PARTS ? at.split * cnt * 64 : 0));
   };
 
   // A wave loads 8 lines (8 rows x 128 bytes) of W and G of X per piece.  Row 16 t + 4 q
@@ -259,11 +269,19 @@ __device__ __forceinline__ void wide_tiles(const WideArgs& a, char* lds, int fir
     const int r0 = wm * G * 16 + n;
     const int c0 = min(at.tn * OUT, cols - OUT) + wn * (OUT / 2);
     u16* o = a.out + (size_t)(at.row + r0) * cols + c0 + q * 8;
+    float* f4 = a.parts + ((size_t)at.split * a.M + at.row + r0) * cols + c0 + q * 8;
 #pragma unroll
     for (int m = 0; m < G; ++m) {
       if (EXPERTS ? r0 + m * 16 < at.rows : r0 + m * 16 >= at.fresh) {
 #pragma unroll
         for (int t = 0; t < (GLU ? 2 : 4); ++t) {
+          if (PARTS) {
+            if (c0 + t * 32 >= at.tn * OUT) {
+              *reinterpret_cast<f32x4*>(f4 + t * 32) = acc[t * 2][m];
+              *reinterpret_cast<f32x4*>(f4 + t * 32 + 4) = acc[t * 2 + 1][m];
+            }
+            continue;
+          }
           bf16x8r v;
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
@@ -277,6 +295,7 @@ __device__ __forceinline__ void wide_tiles(const WideArgs& a, char* lds, int fir
         }
       }
       o += 16 * (size_t)cols;
+      f4 += 16 * (size_t)cols;
     }
     if (next >= nt) break;
     p = next;
@@ -290,6 +309,28 @@ template <int G, int EPI>
 __global__ void __launch_bounds__(256, 1) gemm_wide_kernel(WideArgs a) {
   __shared__ __attribute__((aligned(16))) char lds[(3 * GW_COLS + 2 * 32 * G) * 128];
   wide_tiles<G, EPI, false>(a, lds, 0, 0, 0);
+}
+
+// out = the sum of the parts, 8 values per thread, splits in their order.
+__global__ void __launch_bounds__(256) wide_sum_kernel(u16* __restrict__ out,
+                                                       const float* __restrict__ parts,
+                                                       long long n8, int splits) {
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n8) return;
+  f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
+#pragma unroll 4
+  for (int s = 0; s < splits; ++s) {
+    const f32x4* at = reinterpret_cast<const f32x4*>(parts + (s * n8 + i) * 8);
+    lo += at[0];
+    hi += at[1];
+  }
+  bf16x8r v;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    v[j] = (__bf16)lo[j];
+    v[j + 4] = (__bf16)hi[j];
+  }
+  *reinterpret_cast<bf16x8r*>(out + i * 8) = v;
 }
 
 // Microseconds per piece of K for G = 4..8, and per tile beside them, fitted to 2,175
@@ -330,15 +371,15 @@ __global__ void __launch_bounds__(256, 1) gemm_wide_experts_kernel(WideArgs a) {
   }
 }
 
-static int wide_groups(int M, int N, int K) {   // G of least cost
+static int wide_groups(int M, int N, int K, int splits) {   // G of least cost
   static const float piece[5] = GW_PIECE;
   int best = 0;
   float least = 0.f;
-  for (int g = 8; g >= 4; --g) {
+  for (int g = M < 256 ? M / 32 : 8; g >= 4; --g) {
     const long long tiles =
-        (long long)((M + 32 * g - 1) / (32 * g)) * ((N + GW_COLS - 1) / GW_COLS);
+        (long long)splits * ((M + 32 * g - 1) / (32 * g)) * ((N + GW_COLS - 1) / GW_COLS);
     const float us =
-        (float)((tiles + GW_BLOCKS - 1) / GW_BLOCKS) * (K / 64 * piece[g - 4] + GW_TILE);
+        (float)((tiles + GW_BLOCKS - 1) / GW_BLOCKS) * (K / 64 / splits * piece[g - 4] + GW_TILE);
     if (best == 0 || us < least) { best = g; least = us; }
   }
   return best;
@@ -356,10 +397,11 @@ static bool wide_ok(int M, int N, int K, int epi) {
 AF_EXPORT int af_gemm_wide(void* out, const void* X, const void* W, int M, int N, int K,
                            int epi, int groups, void* stream) {
   if (!wide_ok(M, N, K, epi)) return 9021;
-  if (groups == 0) groups = wide_groups(M, N, K);
+  if (groups == 0) groups = wide_groups(M, N, K, 1);
   hipStream_t st = (hipStream_t)stream;
   WideArgs a = {(u16*)out, (const u16*)X, (const u16*)W, M, N, K,
-                (M + 32 * groups - 1) / (32 * groups), (N + GW_COLS - 1) / GW_COLS, nullptr, nullptr, 0};
+                (M + 32 * groups - 1) / (32 * groups), (N + GW_COLS - 1) / GW_COLS,
+                nullptr, nullptr, 0, nullptr, 1};
 #define GW_CASE(g)                                                                \
   case g:                                                                         \
     if (epi == WIDE_SWIGLU) gemm_wide_kernel<g, WIDE_SWIGLU><<<GW_BLOCKS, 256, 0, st>>>(a); \
@@ -370,6 +412,55 @@ AF_EXPORT int af_gemm_wide(void* out, const void* X, const void* W, int M, int N
     default: return 9022;
   }
 #undef GW_CASE
+  return af_last_err();
+}
+
+// The number of shares of K, up to 16, that costs least: rounds of 256 blocks as above,
+// but a piece never below 0.95 us while the weights come from HBM, and the parts written
+// and read at 5.5 TB/s.  It names the fastest of 2..16 shares, or one within 6% of it.
+AF_EXPORT int af_gemm_wide_splits(int M, int N, int K) {
+  static const float piece[5] = GW_PIECE;
+  if (M < 128 || N < 64 || K < 1024) return 1;
+  const int pieces = K / 64;
+  int best = 1;
+  float least = 0.f;
+  for (int s = 1; s <= 16 && pieces / s >= 8; ++s) {
+    if (pieces % s) continue;
+    for (int g = M < 256 ? M / 32 : 8; g >= 4; --g) {
+      const long long tiles =
+          (long long)s * ((M + 32 * g - 1) / (32 * g)) * ((N + GW_COLS - 1) / GW_COLS);
+      const float p = piece[g - 4] < 0.95f ? 0.95f : piece[g - 4];
+      const float us = (float)((tiles + GW_BLOCKS - 1) / GW_BLOCKS) * (pieces / s * p + GW_TILE) +
+                       (float)s * M * N * 8e-6f / 5.5f;
+      if (least == 0.f || us < least) { best = s; least = us; }
+    }
+  }
+  return best;
+}
+
+// Plain, K in `splits` shares of whole pieces whose sums meet in parts [splits, M, N]:
+// where the tiles of an output are fewer than the blocks.  14336 -> 4096, weights not in
+// cache, library / this in us: 160 rows 84 / 42, 300 rows 74 / 55, 512 rows 92 / 71, 1000
+// rows 138 / 106, of which the parts' way through memory takes a third.
+AF_EXPORT int af_gemm_wide_split(void* out, void* parts, const void* X, const void* W, int M,
+                                 int N, int K, int splits, int groups, void* stream) {
+  if (M < 128 || splits < 1 || K / 64 % splits || K / 64 / splits < 2 ||
+      !wide_ok(M < 256 ? 256 : M, N, K, WIDE_PLAIN) ||
+      ((long long)M / 128 + 1) * (N / GW_COLS + 1) * splits > 0x3fffffff)
+    return 9021;
+  if (groups == 0) groups = wide_groups(M, N, K, splits);
+  if (groups < 4 || groups > 8 || 32 * groups > M) return 9022;
+  hipStream_t st = (hipStream_t)stream;
+  WideArgs a = {(u16*)out, (const u16*)X, (const u16*)W, M, N, K,
+                (M + 32 * groups - 1) / (32 * groups), (N + GW_COLS - 1) / GW_COLS,
+                nullptr, nullptr, 0, (float*)parts, splits};
+#define GW_CASE(g)                                                                \
+  case g: gemm_wide_kernel<g, WIDE_PARTS><<<GW_BLOCKS, 256, 0, st>>>(a); break
+  switch (groups) { GW_CASE(4); GW_CASE(5); GW_CASE(6); GW_CASE(7); GW_CASE(8); }
+#undef GW_CASE
+  const long long n8 = (long long)M * N / 8;
+  wide_sum_kernel<<<(unsigned)((n8 + 255) / 256), 256, 0, st>>>((u16*)out, (const float*)parts,
+                                                              n8, splits);
   return af_last_err();
 }
 
@@ -385,7 +476,8 @@ AF_EXPORT int af_gemm_wide_experts(void* out, const void* X, const void* row, co
   if (n == 0) return 0;
   hipStream_t st = (hipStream_t)stream;
   WideArgs a = {(u16*)out, (const u16*)X, (const u16*)W, n, N, K, 0,
-                (N + GW_COLS - 1) / GW_COLS, (const i32*)offs, (const i32*)row, E};
+                (N + GW_COLS - 1) / GW_COLS, (const i32*)offs, (const i32*)row, E,
+                nullptr, 1};
   if (epi == WIDE_SWIGLU)
     gemm_wide_experts_kernel<WIDE_SWIGLU><<<GW_BLOCKS, 256, 0, st>>>(a);
   else gemm_wide_experts_kernel<WIDE_PLAIN><<<GW_BLOCKS, 256, 0, st>>>(a);

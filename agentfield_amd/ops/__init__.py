@@ -522,13 +522,13 @@ def linear_skinny(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
     return out
 
 
-def _wide_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+def _wide_ok(x: torch.Tensor, w: torch.Tensor, rows: int = 256) -> bool:
     """What the wide GEMM takes: bf16 rows and weights of one length on one GPU,
-    whole and on 16-byte boundaries; 256 rows or more, at least 256 weight rows in
+    whole and on 16-byte boundaries; 256 rows or more (128 with K split), at least 256 weight rows in
     64s, at least 128 columns in 64s, half of w (the up rows) within 4 GB."""
     xs, ws = x.shape, w.shape
     return (x.is_cuda and len(xs) == 2 == len(ws) and xs[1] == ws[1]
-            and 256 <= xs[0] <= 1 << 24 and ws[0] >= 256 and ws[0] % 64 == 0
+            and rows <= xs[0] <= 1 << 24 and ws[0] >= 256 and ws[0] % 64 == 0
             and ws[1] >= 128 and ws[1] % 64 == 0
             and (ws[0] // 2 + 256) * ws[1] * 2 < 1 << 32
             and x.device == w.device and rows_operands_ok((x, w)))
@@ -575,6 +575,40 @@ def launch_wide(x, w, silu_fuse=False, out=None, groups=0):
     return out
 
 
+def _wide_split_pays(M: int, N: int, K: int) -> bool:
+    """Whether the wide GEMM with K in shares beats the library's: few tiles of 256 x
+    256 and a long K, so that the parts' way through memory is small beside the weights'.
+    10 projections at 129..3000 rows, weights not in cache, library over split: with K
+    >= 2N, K > 8192, up to 128 tiles and tiles * K up to 2^21 0.94..2.28, 1.33 in the
+    mean (14336 -> 4096 at 192 rows 104 us / 48, 640 rows 113 / 84, 1500 rows 170 /
+    155; 28672 -> 8192 at 512 rows 309 / 225); beyond that 0.83..1.06 (14336 -> 4096 at
+    2500 rows 238 / 270, 28672 -> 8192 at 640 rows 275 / 292), 8192 -> 2048 0.93..1.12,
+    K < 2N mostly below 1 (4096 x 4096 at 512 rows 26 / 30).  The shares, which
+    divide K in whole pieces, have to occupy most of the blocks: with the 128 that
+    11008 allows at 129 rows 44 us / 52."""
+    cols = -(-N // 256)
+    tiles = -(-M // 256) * cols
+    if not (M > 128 and K >= 2 * N and K > 8192 and K % 64 == 0 and tiles <= 128
+            and tiles * K <= 1 << 21):
+        return False
+    return -(-M // 128) * cols * _lib.lib().af_gemm_wide_splits(M, N, K) >= 192
+
+
+def launch_wide_split(x, w, out=None, splits=0, groups=0):
+    """The wide GEMM with K in shares (0: as many as cost least), for callers that have
+    asked _wide_ok."""
+    (M, K), N = x.shape, w.shape[0]
+    splits = splits or _lib.lib().af_gemm_wide_splits(M, N, K)
+    if out is None:
+        out = torch.empty(M, N, dtype=x.dtype, device=x.device)
+    parts = torch.empty(splits, M, N, dtype=torch.float32, device=x.device)
+    rc = _lib.lib().af_gemm_wide_split(
+        _lib.ptr(out), _lib.ptr(parts), _lib.ptr(x), _lib.ptr(w), M, N, K, splits,
+        groups, _lib.cur_stream())
+    _lib.check(rc, "af_gemm_wide_split")
+    return out
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
            out: torch.Tensor | None = None) -> torch.Tensor:
     """Linear layer dispatch: hand-written weight-streaming kernels up to 128
@@ -595,6 +629,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
             and (out is None or _wide_out_ok(out, x, M, N))
             and _wide_ok(x, w)):
         return launch_wide(x, w, silu_fuse, out)
+    if (not silu_fuse and x.is_cuda and x.dim() == 2
+            and _wide_split_pays(M, N, x.shape[1])
+            and not watched(x, w)
+            and (out is None or _wide_out_ok(out, x, M, N))
+            and _wide_ok(x, w, 128)):
+        return launch_wide_split(x, w, out)
     if out is not None:
         return torch.mm(x, w.t(), out=out)
     y = x @ w.t()

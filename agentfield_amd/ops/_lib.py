@@ -69,6 +69,8 @@ def _declare(l: ctypes.CDLL) -> None:
     l.af_moe_route.argtypes = [p, p, p, p, p, p, p, i, i, i, i, p]
     l.af_moe_combine.argtypes = [p, p, p, p, i, i, i, p]
     l.af_gemm_wide.argtypes = [p, p, p, i, i, i, i, i, p]
+    l.af_gemm_wide_split.argtypes = [p, p, p, p, i, i, i, i, i, p]
+    l.af_gemm_wide_splits.argtypes = [i, i, i]
     l.af_gemm_wide_experts.argtypes = [p, p, p, p, p, i, i, i, i, i, i, p]
     l.af_moe_gemm.argtypes = [p, p, p, p, p, i, i, i, i, i, p]
     l.af_sample.argtypes = [p, p, p, p, p, p, u32, i, i, p]
@@ -86,7 +88,8 @@ def _declare(l: ctypes.CDLL) -> None:
                "af_attn_prefill", "af_gemm_bf16", "af_gemm_bf16_ring", "af_gemm_bf16_q8", "af_gemm_mxfp8", "af_oneshot_allreduce",
                "af_gemm_skinny", "af_rows_linear", "af_rows_qkv",
                "af_moe_route", "af_moe_combine", "af_moe_gemm", "af_gemm_wide",
-               "af_gemm_wide_experts", "af_sample",
+               "af_gemm_wide_experts", "af_gemm_wide_split",
+               "af_gemm_wide_splits", "af_sample",
                "af_sample_topkp", "af_gather_rows", "af_mfma_probe", "af_mfma_mx_probe", "af_lds_stride_probe", "af_mfma_mx32_probe", "af_axpy",
                "af_device_sync"):
         getattr(l, fn).restype = ctypes.c_int

@@ -231,6 +231,19 @@ def test_wide_gemm_pays(M, N, K, glu, pays):
     assert ops._wide_pays(M, N, K, glu) == pays
 
 
+@pytest.mark.parametrize("M,N,K,pays", [
+    (128, 4096, 14336, False), (257, 4096, 14336, True), (2048, 4096, 14336, True),
+    (2049, 4096, 14336, False),                   # 144 tiles
+    (512, 8192, 28672, True), (513, 8192, 28672, False),
+    (300, 2048, 8192, False), (300, 8192, 14336, False), (300, 4096, 14368, False),
+    (300, 4096, 4096, False),
+    (300, 4096, 8384, False),                     # 131 pieces: no shares
+    (256, 4096, 11008, False), (257, 4096, 11008, True),      # 128 and 192 blocks
+])
+def test_wide_gemm_split_pays(M, N, K, pays):
+    assert ops._wide_split_pays(M, N, K) == pays
+
+
 @pytest.mark.parametrize("x_rows,n,E,N,K,glu,pays", [
     (800, 1600, 8, 28672, 4096, True, True), (799, 1599, 8, 28672, 4096, True, False),
     (2000, 2000, 8, 4096, 14336, False, True),

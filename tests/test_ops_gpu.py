@@ -1192,6 +1192,49 @@ def test_wide_gemm(M, N, K, groups, glu):
     assert (got[M:] == 7.0).all()
 
 
+@pytest.mark.parametrize("M,N,K,splits,groups", [
+    (128, 256, 256, 2, 4),        # one tile per share, two pieces each
+    (129, 320, 1152, 3, 4),       # both moved back inside the matrix
+    (160, 4096, 2048, 16, 5), (255, 1088, 1152, 6, 7), (449, 1088, 1792, 7, 8),
+    (700, 4096, 1024, 8, 6),      # more than a round of tiles
+    (300, 512, 1024, 1, 0), (300, 512, 10240, 0, 0), (2000, 4096, 8320, 0, 0),
+])
+def test_wide_gemm_split(M, N, K, splits, groups):
+    """As test_wide_gemm, for longer sums: 32 products in an instruction, K / 32
+    instructions and the shares are at most K / 32 + 48 roundings of at most the sum of
+    the magnitudes, 0.64 sqrt(K) in the mean, 1.5 times that at most."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(N, K, device="cuda", generator=g) / K ** 0.5).bfloat16()
+    got = torch.full((M + 1, N), 7.0, device="cuda", dtype=torch.bfloat16)
+    ops.launch_wide_split(x, w, got[:M], splits, groups)
+    y = (x.double() @ w.double().t()).float()
+    order = 1.5 * 0.64 * K ** 0.5 * (K / 32 + 48) * 2 ** -24
+    assert ((got[:M].float() - y).abs() <= 2 ** -8 * y.abs() + order).all()
+    assert (got[M:] == 7.0).all()
+
+
+def test_linear_splits_a_long_k():
+    """linear sends what the rule names to the split kernel, also under capture."""
+    x = torch.randn(300, 8320, device="cuda").bfloat16()
+    w = torch.randn(4096, 8320, device="cuda").bfloat16()
+    want = ops.launch_wide_split(x, w)
+    with torch.no_grad():
+        assert torch.equal(ops.linear(x, w), want)
+        out = torch.zeros_like(want)
+        assert ops.linear(x, w, out=out) is out and torch.equal(out, want)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = ops.linear(x, w)
+    for _ in range(3):
+        x.copy_(torch.randn(300, 8320, device="cuda"))
+        graph.replay()
+        assert torch.equal(got, ops.launch_wide_split(x, w))
+    leaf = w.clone().requires_grad_()
+    ops.linear(x, leaf).float().sum().backward()
+    assert leaf.grad is not None
+
+
 @pytest.mark.parametrize("glu", [False, True])
 def test_linear_runs_the_wide_gemm(glu):
     """linear sends what the rule names to the kernel, with and without out, and
