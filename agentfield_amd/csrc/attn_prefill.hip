@@ -31,9 +31,9 @@
 //     the block and double-buffered (64 KB, two blocks per CU: one wave's
 //     exponentials run under the other's MFMA).  Bound by vector issue next to
 //     the matrix cores (32 exponentials per lane and tile alone take half of the
-//     tile's MFMA time, during which the cores are busy half of the time).  grid: K/V head fastest,
-//     so with 8 of them an XCD's L2 keeps one head's K/V; late (long) tiles start
-//     first.
+//     tile's MFMA time, during which the cores are busy half of the time).  grid:
+//     K/V head fastest, so with 8 of them an XCD's L2 keeps one head's K/V; late
+//     (long) tiles start first.
 //   attn_prefill_few_kernel  32 columns per block: sequences whose columns fit
 //     one wave (verification of a few drafted tokens, single fed tokens), or all
 //     of a batch too small to fill the chip with 128-column blocks.  The four
@@ -46,9 +46,9 @@
 // Transfers: where pages hold whole tiles, the page of the tile after next is a scalar
 // lookup behind the next tile's loads (as a vector load its wait drained them before
 // this tile's arithmetic: 672 us and 43.9 against 628 and 37.0, one prompt of 8000 rows
-// and 16 sequences of 5 rows behind up to 3000; with attend() as it is now 544 and 36.6).  The compiler still waits for them in
-// front of the transposing reads, half a tile later; loads it does not know of changed
-// little (628, 35.9).
+// and 16 sequences of 5 rows behind up to 3000; with attend() as it is now 544 and
+// 36.6).  The compiler still waits for them in front of the transposing reads, half a
+// tile later; loads it does not know of changed little (628, 35.9).
 // Fragment layouts (measured): A: lane holds A[m=lane&31][k=(lane>>5)*8+j]; B:
 // B[k=(lane>>5)*8+j][n=lane&31]; C: reg r holds C[8*(r/4)+4*(lane>>5)+r%4][lane&31];
 // transposing read: lane i of a group of 16 gets column i of 4 rows x 16 columns

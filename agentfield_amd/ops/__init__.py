@@ -524,8 +524,9 @@ def linear_skinny(x: torch.Tensor, w: torch.Tensor, mode: int = 0,
 
 def _wide_ok(x: torch.Tensor, w: torch.Tensor, rows: int = 256) -> bool:
     """What the wide GEMM takes: bf16 rows and weights of one length on one GPU,
-    whole and on 16-byte boundaries; 256 rows or more (128 with K split), at least 256 weight rows in
-    64s, at least 128 columns in 64s, half of w (the up rows) within 4 GB."""
+    whole and on 16-byte boundaries; 256 rows or more (128 with K split), at least
+    256 weight rows in 64s, at least 128 columns in 64s, half of w (the up rows)
+    within 4 GB."""
     xs, ws = x.shape, w.shape
     return (x.is_cuda and len(xs) == 2 == len(ws) and xs[1] == ws[1]
             and rows <= xs[0] <= 1 << 24 and ws[0] >= 256 and ws[0] % 64 == 0

@@ -1223,13 +1223,14 @@ def test_linear_splits_a_long_k():
         assert torch.equal(ops.linear(x, w), want)
         out = torch.zeros_like(want)
         assert ops.linear(x, w, out=out) is out and torch.equal(out, want)
+    with torch.inference_mode():
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph):
             got = ops.linear(x, w)
-    for _ in range(3):
-        x.copy_(torch.randn(300, 8320, device="cuda"))
-        graph.replay()
-        assert torch.equal(got, ops.launch_wide_split(x, w))
+        for _ in range(3):
+            x.copy_(torch.randn(300, 8320, device="cuda"))
+            graph.replay()
+            assert torch.equal(got, ops.launch_wide_split(x, w))
     leaf = w.clone().requires_grad_()
     ops.linear(x, leaf).float().sum().backward()
     assert leaf.grad is not None
