@@ -535,6 +535,12 @@ def _wide_ok(x: torch.Tensor, w: torch.Tensor, rows: int = 256) -> bool:
             and x.device == w.device and rows_operands_ok((x, w)))
 
 
+def _launches_here(x: torch.Tensor) -> bool:
+    """x is on the current device, on whose stream a kernel is launched; torch's
+    products go to the device of their operands."""
+    return x.device.index == torch.cuda.current_device()
+
+
 def _wide_out_ok(out: torch.Tensor, x: torch.Tensor, M: int, N: int) -> bool:
     return _whole(out, x, M, N) and _apart(out, x) and out.data_ptr() & 15 == 0
 
@@ -625,13 +631,13 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
             and _rows_ok(x, w)):
         return launch_rows(x, w, 2 if silu_fuse else 0, out=out)
     if (M > 128 and x.is_cuda and x.dim() == 2 == w.dim()
-            and _wide_pays(M, N, x.shape[1], silu_fuse)
+            and _wide_pays(M, N, x.shape[1], silu_fuse) and _launches_here(x)
             and not watched(x, w, grad=not silu_fuse)
             and (out is None or _wide_out_ok(out, x, M, N))
             and _wide_ok(x, w)):
         return launch_wide(x, w, silu_fuse, out)
     if (not silu_fuse and x.is_cuda and x.dim() == 2
-            and _wide_split_pays(M, N, x.shape[1])
+            and _wide_split_pays(M, N, x.shape[1]) and _launches_here(x)
             and not watched(x, w)
             and (out is None or _wide_out_ok(out, x, M, N))
             and _wide_ok(x, w, 128)):

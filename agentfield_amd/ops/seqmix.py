@@ -688,7 +688,8 @@ def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
     M, K = x.shape
     N = w.shape[0]
     if (M > 128 and skinny and x.is_cuda and _lib.main_lib_ready()
-            and _ops._wide_pays(M, N, K, False) and not _ops.watched(x, w)
+            and _ops._wide_pays(M, N, K, False) and _ops._launches_here(x)
+            and not _ops.watched(x, w)
             and (out is None or _ops._wide_out_ok(out, x, M, N))
             and _ops._wide_ok(x, w)):
         return _ops.launch_wide(x, w, out=out)

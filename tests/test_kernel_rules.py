@@ -260,3 +260,33 @@ def test_wide_experts_pay(x_rows, n, E, N, K, glu, pays):
     (128, 24576, True)])
 def test_rows_pay(M, N, pays):
     assert ops.rows_pay(M, N) == pays
+
+
+class Operand(SimpleNamespace):
+    """A stand-in that torch would multiply."""
+
+    def t(self):
+        return self
+
+    def __matmul__(self, other):
+        return "torch"
+
+
+@pytest.mark.parametrize("index,own", [(0, True), (1, False)])
+@pytest.mark.parametrize("M,N,K,glu", [
+    (4353, 4096, 4096, False), (300, 4096, 14336, False),
+    (4096, 28672, 4096, True)])
+def test_wide_products_of_another_device(monkeypatch, index, own, M, N, K, glu):
+    """Operands on another device than the current one, whose stream a launch would
+    take, stay with torch, which goes to theirs."""
+    from agentfield_amd.ops import seqmix
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(ops, "watched", lambda *t, **kw: False)
+    monkeypatch.setattr(ops, "silu_and_mul", lambda y: y)
+    for name in ("launch_wide", "launch_wide_split"):
+        monkeypatch.setattr(ops, name, lambda *a, **kw: "own")
+    x, w = (Operand(**vars(mat(n, K, device=f"cuda:{index}"))) for n in (M, N))
+    want = "own" if own else "torch"
+    assert ops.linear(x, w, silu_fuse=glu) == want
+    if not glu and K == 4096:
+        assert seqmix.matmul(x, w) == want
