@@ -537,8 +537,10 @@ def _wide_ok(x: torch.Tensor, w: torch.Tensor, rows: int = 256) -> bool:
 
 def _launches_here(x: torch.Tensor) -> bool:
     """x is on the current device, on whose stream a kernel is launched; torch's
-    products go to the device of their operands."""
-    return x.device.index == torch.cuda.current_device()
+    products go to the device of their operands.  Nor does autocast choose another
+    type for the product."""
+    return (x.device.index == torch.cuda.current_device()
+            and not torch.is_autocast_enabled("cuda"))
 
 
 def _wide_out_ok(out: torch.Tensor, x: torch.Tensor, M: int, N: int) -> bool:

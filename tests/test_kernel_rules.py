@@ -272,15 +272,19 @@ class Operand(SimpleNamespace):
         return "torch"
 
 
-@pytest.mark.parametrize("index,own", [(0, True), (1, False)])
+@pytest.mark.parametrize("index,cast,own", [
+    (0, False, True), (1, False, False), (0, True, False)])
 @pytest.mark.parametrize("M,N,K,glu", [
     (4353, 4096, 4096, False), (300, 4096, 14336, False),
     (4096, 28672, 4096, True)])
-def test_wide_products_of_another_device(monkeypatch, index, own, M, N, K, glu):
+def test_wide_products_that_stay_with_torch(monkeypatch, index, cast, own, M, N, K,
+                                            glu):
     """Operands on another device than the current one, whose stream a launch would
-    take, stay with torch, which goes to theirs."""
+    take, stay with torch, which goes to theirs; so do products under autocast, which
+    may want another type than the operands'."""
     from agentfield_amd.ops import seqmix
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch, "is_autocast_enabled", lambda kind: cast)
     monkeypatch.setattr(ops, "watched", lambda *t, **kw: False)
     monkeypatch.setattr(ops, "silu_and_mul", lambda y: y)
     for name in ("launch_wide", "launch_wide_split"):
