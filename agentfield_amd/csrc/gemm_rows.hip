@@ -380,6 +380,10 @@ __device__ __forceinline__ void meet(int n) {
   asm volatile("" ::: "memory");
 }
 
+// Four neighbours of a row of the caller's output, whose address is a multiple of 4 bytes
+// only (the hardware needs no more for a store of 8).
+typedef u16x4 __attribute__((aligned(4))) row_u16x4;
+
 // Whole K: MT 16-row groups of X (even), NT 16-row tiles of weights (4 or 8), NW
 // waves, a ring of STAGES pieces of K = 64.  Grid N / (16 NT).  EPI_PLAIN, EPI_SWIGLU.
 template <int MT, int NT, int NW, int STAGES, int EPI, int NORM, int AUX>
@@ -537,14 +541,14 @@ __global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
         o[r] = f2bf(v / (1.f + __expf(-v)) * u);
       }
       if (row < a.M)
-        *reinterpret_cast<u16x4*>(a.out + (size_t)row * (a.N >> 1) +
+        *reinterpret_cast<row_u16x4*>(a.out + (size_t)row * (a.N >> 1) +
                                   (tile + (lane >> 5)) * 8 + (lane >> 4 & 1) * 4) = o;
     } else if (row < a.M) {
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const size_t at = (size_t)row * a.N + (tile + t) * 16 + (lane >> 4) * 4;
         const f32x4 v = sum[t][m];
-        *reinterpret_cast<u16x4*>(a.out + at) =
+        *reinterpret_cast<row_u16x4*>(a.out + at) =
             u16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])};
       }
     }

@@ -680,6 +680,22 @@ def test_whole_k_row_products(M, N, pieces):
                      rtol=2 ** -6)
 
 
+@pytest.mark.parametrize("M", [1, 17, 40, 80, 97])
+@pytest.mark.parametrize("N,mode", [(192, 0), (24576, 0), (192, 2), (24576, 2)])
+def test_row_products_to_an_odd_pair_of_columns(M, N, mode):
+    """A caller's rows need an address that is a multiple of 4 bytes, in every row
+    class and block width: the bits of a product to rows of its own, and nothing
+    beside them."""
+    x, w = rnd(M, 128, seed=M, scale=0.3), rnd(N, 128, seed=N, scale=0.3)
+    want = ops.linear_rows(x, w, mode)
+    buf = torch.full((want.numel() + 4,), 7.0, device=DEV, dtype=torch.bfloat16)
+    out = buf[2:-2].view_as(want)
+    assert out.data_ptr() % 8 == 4
+    assert ops.linear_rows(x, w, mode, out=out) is out
+    assert torch.equal(out, want)
+    assert (buf[:2] == 7.0).all() and (buf[-2:] == 7.0).all()
+
+
 @pytest.mark.parametrize("M", [1, 17, 128])
 @pytest.mark.parametrize("K,KW", [(512, 448), (448, 512), (64, 4096)])
 def test_row_products_refuse_other_inner_lengths(M, K, KW):
