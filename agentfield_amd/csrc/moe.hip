@@ -12,21 +12,26 @@
 #define MOE_MAX_K 8
 
 // Router logits in fp32 (products of bf16 are exact), softmax over the k largest:
-// a block per row, equal logits go to the smaller expert.  A logit that is not a
-// number counts as the largest, so that the row's weights show it.  Bound by latency:
-// with a wave per row the loop over the row waited for memory eight times (34 us for 40
-// rows as for 1100); four waves share the row and most of its loads are out at once.
-template <int EM>
+// equal logits go to the smaller expert.  A logit that is not a number counts as the
+// largest, so that the row's weights show it.
+// Few rows are bound by latency: with a wave per row the loop over the row waits for
+// memory eight times (40 rows of 4096 over 8 experts 18.7 us, sorting included), with
+// WAVES = 4 to a row most of its loads are out at once (10.8).  Many rows are bound by
+// their instructions, and four waves sum every expert's logit four times over: there a
+// wave takes a row.
+template <int EM, int WAVES>
 __global__ void __launch_bounds__(256) moe_route_kernel(
     i32* __restrict__ topi, float* __restrict__ topv, const u16* __restrict__ x,
     const u16* __restrict__ router, int T, int H, int E, int k) {
-  const int t = blockIdx.x, lane = threadIdx.x & 63;
+  const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int t = WAVES == 4 ? blockIdx.x : blockIdx.x * 4 + wid;
+  if (t >= T) return;
   const u16* xr = x + (size_t)t * H;
   float acc[EM];
 #pragma unroll
   for (int e = 0; e < EM; ++e) acc[e] = 0.f;
-#pragma unroll 2
-  for (int c = threadIdx.x * 8; c < H; c += 2048) {
+#pragma unroll WAVES == 4 ? 2 : 1
+  for (int c = (WAVES == 4 ? threadIdx.x : lane) * 8; c < H; c += 512 * WAVES) {
     const s16x8 xv = *reinterpret_cast<const s16x8*>(xr + c);
     float xf[8];
 #pragma unroll
@@ -39,17 +44,19 @@ __global__ void __launch_bounds__(256) moe_route_kernel(
       for (int j = 0; j < 8; ++j) acc[e] = fmaf(xf[j], bf2f((u16)rv[j]), acc[e]);
     }
   }
-  __shared__ float part[4][EM];
 #pragma unroll
-  for (int e = 0; e < EM; ++e) {
-    const float s = wave_sum_f32(acc[e]);
-    if (lane == 0) part[threadIdx.x >> 6][e] = s;
+  for (int e = 0; e < EM; ++e) acc[e] = wave_sum_f32(acc[e]);
+  if constexpr (WAVES == 4) {
+    __shared__ float part[4][EM];
+#pragma unroll
+    for (int e = 0; e < EM; ++e)
+      if (lane == 0) part[wid][e] = acc[e];
+    __syncthreads();
+    if (wid) return;
+#pragma unroll
+    for (int e = 0; e < EM; ++e)
+      acc[e] = (part[0][e] + part[1][e]) + (part[2][e] + part[3][e]);
   }
-  __syncthreads();
-  if (threadIdx.x >= 64) return;
-#pragma unroll
-  for (int e = 0; e < EM; ++e)
-    acc[e] = (part[0][e] + part[1][e]) + (part[2][e] + part[3][e]);
   unsigned long long used = 0;
   float best[MOE_MAX_K], sum = 0.f;
   int who[MOE_MAX_K];
@@ -163,6 +170,19 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(
   }
 }
 
+// Whether four waves share a row (see moe_route_kernel).  Routing, a wave / four waves per
+// row in us: 8 experts, rows of 4096: 18.6 / 11.8 at 300 rows, 24.6 / 22.6 at 2000, 40.9 /
+// 38.8 at 4096, 62 / 70 at 8192; rows of 1024: 12.5 / 12.0 at 1000, 16.8 / 18.4 at 2000; 2
+// experts, rows of 4096: 16.3 / 15.9 at 2000, 17.2 / 20.2 at 3000; 32 experts, rows of
+// 1024: 40.5 / 35.4 at 600, 45.8 / 48.0 at 800; 64 experts, rows of 2048: 95 / 60 at 200,
+// 115 / 157 at 600, rows of 8192: 256 / 271 at 600.  A row of 256 is one load anyway (4 experts, 1000 rows 9.7 / 10.5).
+static bool route_shares_rows(int T, int H, int E) {
+  if (H < 1024) return false;
+  if (E > 32) return T <= min(H / 8, 512);
+  if (E > 16) return T <= min(H / 2, 2048);
+  return T <= min(H, E < 8 ? 2048 : 4096);
+}
+
 // topi [T, k] i32, topv [T, k] f32 (largest first, sum 1); offs / row / pos as
 // moe_sort_kernel leaves them.
 AF_EXPORT int af_moe_route(void* topi, void* topv, void* offs, void* row, void* pos,
@@ -171,15 +191,17 @@ AF_EXPORT int af_moe_route(void* topi, void* topv, void* offs, void* row, void* 
   if (H % 8 || E < 1 || E > MOE_MAX_E || k < 1 || k > MOE_MAX_K || k > E) return 9001;
   if (T == 0) return 0;
   hipStream_t st = (hipStream_t)stream;
-#define AF_ROUTE(EM)                                                           \
-  moe_route_kernel<EM><<<T, 256, 0, st>>>((i32*)topi, (float*)topv,         \
-                                             (const u16*)x, (const u16*)router, \
-                                             T, H, E, k)
+  const bool share = route_shares_rows(T, H, E);
+#define AF_ROUTE_AS(EM, WAVES)                                                 \
+  moe_route_kernel<EM, WAVES><<<WAVES == 4 ? T : (T + 3) / 4, 256, 0, st>>>(   \
+      (i32*)topi, (float*)topv, (const u16*)x, (const u16*)router, T, H, E, k)
+#define AF_ROUTE(EM) (share ? AF_ROUTE_AS(EM, 4) : AF_ROUTE_AS(EM, 1))
   if (E <= 8) AF_ROUTE(8);
   else if (E <= 16) AF_ROUTE(16);
   else if (E <= 32) AF_ROUTE(32);
   else AF_ROUTE(64);
 #undef AF_ROUTE
+#undef AF_ROUTE_AS
   moe_sort_kernel<<<1, 1024, 0, st>>>((i32*)offs, (i32*)row, (i32*)pos,
                                       (const i32*)topi, T * k, k, E);
   return af_last_err();

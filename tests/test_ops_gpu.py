@@ -1032,6 +1032,22 @@ def test_moe_sorted_dispatch(T, E, k):
     assert close(got, ref_, atol=2e-2, rtol=2 ** -7)
 
 
+@pytest.mark.parametrize("T,E,k,H", [
+    (1, 8, 2, 1024), (1032, 8, 2, 1032), (1033, 8, 2, 1032), (516, 32, 4, 1032),
+    (517, 32, 4, 1032), (129, 64, 8, 1032), (130, 64, 8, 1032), (3, 2, 1, 4104)])
+def test_moe_routing_with_shared_rows(T, E, k, H):
+    """Rows that four waves share and, one more of them, rows that do not, with a last
+    piece of 8 columns: weights and choices as softmax and topk have them.  Weights:
+    fp32 sums of 4104 products at most."""
+    x, router = rnd(T, H, seed=T), rnd(E, H, seed=E, scale=0.1)
+    w, row, pos, offs = ops.moe_route(x, router, k)
+    tv, ti = torch.softmax(x.double() @ router.double().t(), -1).topk(k, -1)
+    assert torch.allclose(w.double(), tv / tv.sum(-1, keepdim=True), atol=1e-5)
+    mine = torch.searchsorted(offs, pos, right=True) - 1
+    assert torch.equal(mine.view(T, k), ti)
+    assert torch.equal(row[pos.long()].long(), torch.arange(T * k, device=DEV) // k)
+
+
 @pytest.mark.parametrize("E,k", [(2, 2), (8, 2), (64, 8)])
 def test_moe_weights_to_fp32_rounding(E, k):
     """Logits that fp32 holds exactly (a row picks one column of the router), up
