@@ -609,6 +609,25 @@ def test_attn_decode_tile_edges(page, G, Hk, nsplit, window):
     assert close(got, want, atol=2 ** -7, rtol=2 ** -8)
 
 
+@pytest.mark.parametrize("Hk,nsplit", [(3, 1), (4, 1), (4, 2), (8, 1), (8, 3), (11, 2)])
+def test_attn_decode_orders_of_the_grid(Hk, nsplit):
+    """Heads first and sequences first: every head of every sequence is its own, by
+    the bits of a call with that head alone, which runs sequences first."""
+    B, G, D, page = 13, 2, 128, 16
+    torch.manual_seed(Hk)
+    kc = torch.randn(B * 4, Hk, page, D, device=DEV).bfloat16()
+    vc = torch.randn(B * 4, Hk, page, D, device=DEV).bfloat16()
+    bt = torch.randperm(B * 4, device=DEV).view(B, 4).int()
+    lens = torch.randint(1, 4 * page + 1, (B,), device=DEV).int()
+    q = torch.randn(B, Hk * G * D, device=DEV).bfloat16()
+    got = ops.attn_decode(q, kc, vc, bt, lens, nsplit=nsplit).view(B, Hk, G * D)
+    for h in range(Hk):
+        one = ops.attn_decode(q.view(B, Hk, G * D)[:, h].contiguous(),
+                              kc[:, h:h + 1].contiguous(), vc[:, h:h + 1].contiguous(),
+                              bt, lens, nsplit=nsplit)
+        assert torch.equal(got[:, h], one)
+
+
 def _rope_rows_reference(x, w, eps, pos, tab, Hq, Hk):
     """fp32 QKV + norm scalar + rotate-half; q [M, Hq, D], k / v [M, Hk, D]."""
     xf, D = x.float(), 128
