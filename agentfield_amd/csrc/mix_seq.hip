@@ -527,9 +527,9 @@ __global__ void __launch_bounds__(256) diff_combine_kernel(
 
 // ------------------------------------------------------------- linear scan
 // Workgroup = (sequence, head, 32-column tile of dv); 256 threads = 16 row
-// groups x 16 column pairs.  A thread keeps RP consecutive rows of two columns of
-// the state in registers (each q / k / decay value read from LDS feeds two
-// columns).  Tokens are walked serially in blocks of TB: the block's q / k / decay
+// groups x 16 column pairs, or 512 = 16 x 32 columns.  A thread keeps RP consecutive
+// rows of its columns of the state in registers (each q / k / decay value read from
+// LDS feeds both of two columns).  Tokens are walked serially in blocks of TB: the block's q / k / decay
 // rows are staged into LDS at once (rotary + scaling applied on the way in), the
 // recurrence itself is strictly token by token in fp32, and both kernels use the
 // same operations (scan_*) and sum the 16 row groups in the same order — so they
@@ -539,14 +539,14 @@ __global__ void __launch_bounds__(256) diff_combine_kernel(
 // linear_scan_kernel, few tokens per sequence: bound by moving the state; thread
 // (r, c) = (tid >> 4, tid & 15) has columns c and c + 16, so that a state row
 // moves in 64-byte pieces; partial outputs meet in LDS after the block of tokens.
-// linear_scan_prompt_kernel: bound by vector instructions, 40 per token and wave on two
-// waves per SIMD beside the staging (a fifth); the row groups are the 16 lanes of a
-// DPP row, so the sum over rows needs no LDS and no second barrier.  A constant decay
-// is not staged.
+// linear_scan_prompt_kernel: with few workgroups bound by vector instructions, 40 per
+// token and wave on two waves per SIMD beside the staging (a fifth); the row groups are
+// the 16 lanes of a DPP row, so the sum over rows needs no LDS and no second barrier.  A
+// constant decay is not staged.  Its workgroups are four or eight waves, see launch_scan.
 // Six sequences of 500..1900 tokens, 8 heads of 128 x 128, decays per channel:
-// 787 -> 336 us; 16 heads, one decay per head, rotary: 770 -> 447 us (one wave per SIMD
-// with two columns per thread 385 and 497; the row layout alone 711 and 698; element
-// loads that were converted at once made every block wait for its successor).
+// 787 -> 336 us; 16 heads, one decay per head, rotary: 770 -> 447 us (four waves, two
+// columns per thread, 385 and 497; the row layout alone 711 and 698; element loads that
+// were converted at once made every block wait for its successor).
 // v plus the sum over the other lanes of its 16-lane row, in all of them
 __device__ __forceinline__ float row16_sum_all(float v) {
 #define AFM_ROR(N)                                                           \
@@ -781,17 +781,17 @@ __global__ void __launch_bounds__(256) linear_scan_kernel(
   }
 }
 
-// Threads of the prompt kernel: with one column each two waves share a SIMD and fill one
-// another's waits; below 128 rows the staged pieces would be smaller than a load.
-constexpr int scan_threads(int rp) { return rp >= 8 ? 512 : 256; }
+// Rows of a token that a thread of the prompt kernel stages
+constexpr int scan_rows(int rp, int threads) { return (rp >= 16 ? 8 : 16) * 16 * rp / threads; }
 
 // The same recurrence for prompts.  A thread stages E consecutive rows of one token
 // (one wide load each for q, k, the rotary partners and the decay logits, kept raw
-// until the block before has been worked through) and computes RP rows of two
-// columns; lane j of a 16-lane row keeps token j's sum.  Two LDS buffers, one
-// barrier per block of tokens.
-template <typename S, int RP, bool ZL>
-__global__ void __launch_bounds__(scan_threads(RP), RP == 8 && sizeof(S) == 2 ? 4 : 2) linear_scan_prompt_kernel(
+// until the block before has been worked through) and computes RP rows of one column
+// (NT = 512) or two (256); lane j of a 16-lane row keeps token j's sum.  Two LDS
+// buffers, one barrier per block of tokens.
+template <typename S, int RP, bool ZL, int NT>
+__global__ void __launch_bounds__(NT, NT == 512 && RP == 8 && sizeof(S) == 2 ? 4 : 2)
+linear_scan_prompt_kernel(
     float* __restrict__ out, float* __restrict__ state,
     const S* __restrict__ q, const S* __restrict__ k, const S* __restrict__ v,
     const S* __restrict__ zl, const float* __restrict__ zbias,
@@ -803,8 +803,8 @@ __global__ void __launch_bounds__(scan_threads(RP), RP == 8 && sizeof(S) == 2 ? 
   constexpr int DKP = 16 * RP;
   constexpr bool FAST = sizeof(S) == 2;
   constexpr int TB = RP >= 16 ? 8 : 16;
-  constexpr int NT = scan_threads(RP), CPT = 512 / NT;   // columns per thread
-  constexpr int E = TB * DKP / NT;             // staged rows per thread
+  constexpr int CPT = 512 / NT;                // columns per thread
+  constexpr int E = scan_rows(RP, NT);
   constexpr int BUF = TB * (3 * DKP + 32);     // [TB][3][DKP], [TB][32]
   extern __shared__ float smem[];
   const int b = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * 32;
@@ -969,8 +969,13 @@ __global__ void __launch_bounds__(scan_threads(RP), RP == 8 && sizeof(S) == 2 ? 
           t.a[w] = ZL ? sq[2 * DKP + r * RP + w] : hd;
         }
       }
-#pragma unroll
-      for (int c = 0; c < CPT; ++c) t.v[c] = vb[tt * 32 + CPT * cc + c];
+      if constexpr (CPT == 2) {
+        const f32x2 v = *reinterpret_cast<const f32x2*>(vb + tt * 32 + 2 * cc);
+        t.v[0] = v[0];
+        t.v[1] = v[1];
+      } else {
+        t.v[0] = vb[tt * 32 + cc];
+      }
       return t;
     };
     auto step = [&](int tt, const Token& t) {
@@ -983,14 +988,13 @@ __global__ void __launch_bounds__(scan_threads(RP), RP == 8 && sizeof(S) == 2 ? 
         for (int c = 0; c < CPT; ++c)
           scan_row(state_of[c][ii], part[c], t.a[ii], t.k[ii], t.v[c], t.q[ii]);
 #pragma unroll
-      for (int c = 0; c < CPT; ++c) {
-        part[c] = row16_sum_all(part[c]);
-        o[c] = r == tt ? part[c] : o[c];
-      }
+      for (int c = 0; c < CPT; ++c) part[c] = row16_sum_all(part[c]);
+#pragma unroll
+      for (int c = 0; c < CPT; ++c) o[c] = r == tt ? part[c] : o[c];
     };
     if (nt == TB) {
-      // the next token's LDS reads run under this one's arithmetic: the fence
-      // keeps them there, a wave has its SIMD to itself and would wait for them
+      // the next token's LDS reads run under this one's arithmetic: the fence keeps
+      // them there, the one or two waves of a SIMD do not hide them otherwise
       Token t[2];
       t[0] = read(0);
 #pragma unroll
@@ -1224,26 +1228,46 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
   // From a block of tokens per sequence on the prompt kernel is the better one
   // (see there); its loads take E rows at once, so heads, halves of the rotated
   // part, strides and bases must be multiples of E elements (16 bytes at most).
-  const int E = rpp >= 4 ? 4 : rpp;
-  const size_t al = E * sizeof(S) < 16 ? E * sizeof(S) : 16;
-  const bool prompt =
-      T >= 16 * B && dk % E == 0 && (rot / 2) % E == 0 && ldq % E == 0 &&
-      ldk % E == 0 && (!zl || ldz % E == 0) && (uintptr_t)q % al == 0 &&
-      (uintptr_t)k % al == 0 && (uintptr_t)zl % al == 0;
+  auto loads = [&](int threads) {
+    const int E = scan_rows(rpp, threads);
+    const size_t al = E * sizeof(S) < 16 ? E * sizeof(S) : 16;
+    return T >= 16 * B && dk % E == 0 && (rot / 2) % E == 0 && ldq % E == 0 &&
+           ldk % E == 0 && (!zl || ldz % E == 0) && (uintptr_t)q % al == 0 &&
+           (uintptr_t)k % al == 0 && (uintptr_t)zl % al == 0;
+  };
+  // From 128 rows on with eight waves, which fill one another's waits, while that leaves
+  // a workgroup or two to a CU; beyond, four waves do it with fewer instructions.  Four /
+  // eight waves in us, decays per channel, bf16: 128 rows, 192 groups 110 / 96, 384 groups
+  // 542 / 537, 768 766 / 837, 4096 135 / 150; 256 rows, 64 groups 723 / 673, 384 279 / 348.
+  // fp32: 128 rows, 192 groups 172 / 137, 384 835 / 894; one decay per head 574 / 479 and,
+  // 8192 groups, 1300 / 1199.  What only eight waves can load (rows in fours) is, on many
+  // groups, better off with them than with the token kernel in bf16 at 128 rows (dk 100,
+  // 17 tokens 90 / 75), otherwise for longer prompts (fp32 17 tokens 104 / 151, 75 tokens
+  // 219 / 229, 225 tokens 1148 / 1138).
+  const i64 groups = (i64)B * H * grid.z;
+  const bool few = rpp >= 16 || (sizeof(S) == 4 && zl)
+                       ? groups <= 256 : sizeof(S) == 4 || groups <= 512;
+  const bool eight = rpp >= 8 && loads(512) &&
+                     (few || (!loads(256) && ((rpp == 8 && sizeof(S) == 2) ||
+                                              T >= 128 * B)));
+  const bool prompt = eight || loads(256);
   const size_t sm = (size_t)(rpp >= 16 ? 8 : 16) * sizeof(float) *
                     (prompt ? 2 * (3 * 16 * rpp + 32) : 3 * 16 * rpp + 512 + 32);
 #define SCAN_ARGS                                                            \
       out, state, (const S*)q, (const S*)k, (const S*)v, (const S*)zl, zbias, \
       head_decay, inv_freq, positions, cu, q_start, sslot, q_scale, k_scale, \
       inv_tau, H, dk, dv, rot, ldq, ldk, ldv, ldz
+#define SCAN_PROMPT(RP, NT)                                                  \
+  do {                                                                       \
+    if (zl)                                                                  \
+      linear_scan_prompt_kernel<S, RP, true, NT><<<grid, NT, sm, s>>>(SCAN_ARGS); \
+    else                                                                     \
+      linear_scan_prompt_kernel<S, RP, false, NT><<<grid, NT, sm, s>>>(SCAN_ARGS); \
+  } while (0)
 #define SCAN(RP)                                                             \
   do {                                                                       \
-    if (prompt && zl)                                                        \
-      linear_scan_prompt_kernel<S, RP, true>                                 \
-          <<<grid, scan_threads(RP), sm, s>>>(SCAN_ARGS);                    \
-    else if (prompt)                                                         \
-      linear_scan_prompt_kernel<S, RP, false>                                \
-          <<<grid, scan_threads(RP), sm, s>>>(SCAN_ARGS);                    \
+    if (eight) SCAN_PROMPT((RP >= 8 ? RP : 8), 512);                         \
+    else if (prompt) SCAN_PROMPT(RP, 256);                                   \
     else                                                                     \
       linear_scan_kernel<S, RP><<<grid, 256, sm, s>>>(SCAN_ARGS);            \
   } while (0)
@@ -1252,6 +1276,7 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
   else if (rp <= 8) SCAN(8);
   else SCAN(16);
 #undef SCAN
+#undef SCAN_PROMPT
 #undef SCAN_ARGS
   return af_last_err();
 }

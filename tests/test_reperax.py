@@ -669,14 +669,18 @@ def test_registry_loads_checkpoint_and_trace_cli(tmp_path):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("dk,dv,rot,pad", [
     (16, 32, 0, 0), (24, 33, 16, 0), (64, 48, 32, 8), (120, 31, 0, 0),
-    (128, 128, 64, 0), (128, 64, 24, 0), (200, 40, 64, 0), (128, 40, 64, 3)])
+    (128, 128, 64, 0), (128, 64, 24, 0), (200, 40, 64, 0), (128, 40, 64, 3),
+    # loads of four rows: heads, strides, bases and halves that allow no wider ones, and
+    # a head and a half that allow not even those
+    (100, 40, 0, 0), (196, 33, 8, 4), (128, 64, 8, 4), (122, 64, 0, 0),
+    (128, 64, 20, 0)])
 @pytest.mark.parametrize("gated", [False, True])
 def test_scan_prompt_and_token_kernels_agree(dtype, dk, dv, rot, pad, gated):
     """The prompt kernel (whole prompts of lengths around its token blocks) and
     the token kernel (the same prompts in portions of one and of nine tokens)
-    give the same bits, outputs and states; padded dims, column tiles, halves
-    that are not a multiple of the wide loads, rows that are not aligned for
-    them (those stay with the token kernel in all portions)."""
+    give the same bits, outputs and states; padded dims, column tiles, halves and
+    rows that are not a multiple of the wide loads (those stay with the token
+    kernel in all portions)."""
     from agentfield_amd.ops import seqmix as sm
     from types import SimpleNamespace
     H, lens = 2, [1, 16, 17, 33, 100]
@@ -729,3 +733,46 @@ def test_scan_prompt_and_token_kernels_agree(dtype, dk, dv, rot, pad, gated):
     for portion in (1, 9):
         o, s = run(portion)
         assert torch.equal(o, whole) and torch.equal(s, S)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("dk,dv,rot", [(128, 64, 64), (200, 40, 0), (100, 64, 8)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_scan_bits_do_not_depend_on_the_batch(dtype, dk, dv, rot, gated):
+    """140 prompts of 16..48 tokens at once, more workgroups than eight waves each are
+    used for, and the same 15 at a time, which run on eight: the same bits."""
+    from types import SimpleNamespace
+    from agentfield_amd.ops import seqmix as sm
+    H, B = 2, 140
+    lens = [16 + (i * 13) % 33 for i in range(B)]
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    T = cu[-1]
+    g = torch.Generator(device="cuda").manual_seed(dk)
+
+    def rows(n, s=1.0):
+        return (torch.randn(T, n, generator=g, device="cuda") * s).to(dtype)
+    q, k, v = rows(H * dk, dk ** -0.5), rows(H * dk, 0.3), rows(H * dv)
+    kw = (dict(inv_tau=1 / 16, decay_bias=torch.ones(H * dk, device="cuda")) if gated
+          else dict(head_decay=torch.tensor([0.9, 0.99], device="cuda")))
+    z = rows(H * dk, 2.0) if gated else None
+    if rot:
+        kw.update(inv_freq=sm.rotary_inv_freq(rot, 1e4, "cuda"))
+    state = torch.full((B + 1, H, dk, dv), torch.nan, device="cuda")
+
+    def run(a, b):
+        part = slice(cu[a], cu[b])
+        md = SimpleNamespace(
+            cu_seqlens=torch.tensor(cu[a:b + 1], device="cuda").int() - cu[a],
+            q_start=torch.zeros(b - a, device="cuda", dtype=torch.int32),
+            state_slots=torch.arange(a + 1, b + 1, device="cuda").int())
+        pos = torch.cat([torch.arange(n) for n in lens[a:b]]).int().cuda()
+        return sm.linear_scan(q[part], k[part], v[part], state, md, pos, H,
+                              decay_logits=z[part] if gated else None, **kw)
+    whole = run(0, B)
+    ends = state[1:].clone()
+    assert torch.isfinite(whole).all() and torch.isfinite(ends).all()
+    parts = torch.cat([run(a, min(a + 15, B)) for a in range(0, B, 15)])
+    assert torch.equal(parts, whole) and torch.equal(state[1:], ends)
