@@ -278,8 +278,8 @@ __device__ __forceinline__ void wait_loads_and_meet() {
 }
 
 // Split K: MT 16-row groups of X (even), ring of STAGES pieces of K = 64, the sums to
-// the parts.  Grid (N / (16 NW), splits).
-template <int MT, int NW, int WT, int STAGES, int AUX>
+// the parts (EPI_PARTS); unsplit, EPI_PLAIN.  Grid (N / (16 NW), splits).
+template <int MT, int NW, int WT, int STAGES, int EPI, int NORM, int AUX>
 __global__ void __launch_bounds__(64 * NW) gemm_parts_kernel(RowsArgs a) {
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -356,11 +356,23 @@ __global__ void __launch_bounds__(64 * NW) gemm_parts_kernel(RowsArgs a) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = (m0 + m) * 16 + (lane >> 4) * 4 + r;
+      float rstd = 1.f;
+      if (NORM == 1) {
+        const float* sp = a.ss + (size_t)min(row, a.M - 1) * 8;
+        float s = 0.f;
 #pragma unroll
-      for (int t = 0; t < WT; ++t)
-        if (row < a.M)
-          a.parts[((size_t)blockIdx.y * a.M + row) * a.N +
-                  (blockIdx.x * NW + w0 + t) * 16 + n] = acc[t][m][r];
+        for (int j = 0; j < 8; ++j) s += sp[j];
+        rstd = rsqrtf(s * (1.f / (float)a.K) + a.eps);
+      }
+#pragma unroll
+      for (int t = 0; t < WT; ++t) {
+        const int c = (blockIdx.x * NW + w0 + t) * 16 + n;
+        if (row >= a.M) continue;
+        if (EPI == EPI_PARTS)
+          a.parts[((size_t)blockIdx.y * a.M + row) * a.N + c] = acc[t][m][r];
+        else
+          a.out[(size_t)row * a.N + c] = f2bf(NORM == 1 ? acc[t][m][r] * rstd : acc[t][m][r]);
+      }
     }
 }
 
@@ -637,6 +649,7 @@ __global__ void __launch_bounds__(256) rows_sum_kernel(
 }
 
 #define ROWS_MAX 16   // rows up to here: gemm_rows_kernel
+#define ROWS_CUS 256
 
 // Weights from here on are streamed past the caches, and X stays in them: SwiGLU
 // over 28672 x 4096 40.5 -> 37.5 us at one row, 42.8 -> 40.1 at 64, 52.0 -> 50.0 at 128
@@ -653,24 +666,40 @@ static void launch_rows(const RowsArgs& a, hipStream_t st) {
     gemm_rows_kernel<2, EPI, NORM, KEEP><<<a.N / 16, 512, 0, st>>>(a);
 }
 
-// Blocks of 128 weight rows halve the reads of X; they pay where they fill the chip
-// (28672 x 4096, 224 blocks: 36.9 us at 24 rows and 48.0 at 128, in 64 columns 41.1 and
-// 63.6), not below (16384 x 2048, 128 blocks: 16.4 and 24.8, in 64 columns 13.8 and 19.6).
+// Blocks of 128 weight rows halve the reads of X; they pay where blocks of 64 are more
+// than one to a CU (64 / 128 columns, SwiGLU, in us: 22016 x 4096, 344 or 172 blocks, 38.2
+// / 31.5 at 32 rows, 58.2 / 44.8 at 128; 18432 x 4096 39.3 / 30.0, 57.2 / 43.7; 16384 x
+// 4096, 256 or 128 blocks, 25.3 / 29.6, 34.1 / 43.2).  Up to 64 rows, more than one of them
+// to a CU, the rings are short enough that two have room (57344 x 8192, 17 rows: 156 us in
+// rings of 5, 149 of 3; 128256 x 8192 350, 323), otherwise longer (22016 x 4096 34.6 in 3,
+// 31.5 in 5).  Plain products of 97..128 rows keep the loop of the split ones: 32000 x 2048
+// 28.7 us, 27.2 there; 65536 x 2048 61.4, 58.5; 24576 x 4096 46.4, 45.2; with SwiGLU 47.3 at
+// 28672 x 4096 there and 46.4 here.  Small weights are here and gone: 4096 x 1024 at 32 rows
+// 7.3 us in a ring of 5, 6.9 of 3.
 template <int EPI, int NORM, int AUX>
 static void launch_tile_as(const RowsArgs& a, hipStream_t st) {
-  if (a.N % 128 == 0 && a.N / 128 >= 192) {
+  if (a.N % 128 == 0 && a.N > 64 * ROWS_CUS) {
     const int g = a.N / 128;
-    if (a.M <= 32)
+    if (a.M <= 32 && g <= ROWS_CUS)
       gemm_tile_kernel<2, 8, 8, 5, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
-    else if (a.M <= 64)
+    else if (a.M <= 32)
+      gemm_tile_kernel<2, 8, 8, 3, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
+    else if (a.M <= 64 && g <= ROWS_CUS)
       gemm_tile_kernel<4, 8, 8, 4, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
+    else if (a.M <= 64)
+      gemm_tile_kernel<4, 8, 8, 3, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
     else if (a.M <= 96)
       gemm_tile_kernel<6, 8, 8, 4, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
+    else if constexpr (EPI == EPI_PLAIN)
+      gemm_parts_kernel<8, 8, 4, 3, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
     else
       gemm_tile_kernel<8, 8, 8, 4, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
   } else {
     const int g = a.N / 64;
-    if (a.M <= 32)
+    const bool small = (i64)a.N * a.K <= (4 << 20);
+    if (a.M <= 32 && small)
+      gemm_tile_kernel<2, 4, 4, 3, EPI, NORM, KEEP><<<g, 256, 0, st>>>(a);
+    else if (a.M <= 32)
       gemm_tile_kernel<2, 4, 4, 5, EPI, NORM, AUX><<<g, 256, 0, st>>>(a);
     else if (a.M <= 64)
       gemm_tile_kernel<4, 4, 8, 4, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
@@ -697,15 +726,15 @@ static void launch_parts_as(const RowsArgs& a, int splits, hipStream_t st) {
   const bool wide = a.N % 128 == 0 && a.N / 128 * splits >= 192 &&
                     a.K / 64 >= 12 * splits;
   if (a.M <= 64 && wide && (a.M > 32 || splits == 1))
-    gemm_parts_kernel<4, 8, 4, 3, AUX><<<g128, 512, 0, st>>>(a);
+    gemm_parts_kernel<4, 8, 4, 3, EPI_PARTS, 0, AUX><<<g128, 512, 0, st>>>(a);
   else if (a.M <= 32)
-    gemm_parts_kernel<2, 4, 1, 4, AUX><<<g64, 256, 0, st>>>(a);
+    gemm_parts_kernel<2, 4, 1, 4, EPI_PARTS, 0, AUX><<<g64, 256, 0, st>>>(a);
   else if (a.M <= 64)
-    gemm_parts_kernel<4, 4, 2, 4, AUX><<<g64, 256, 0, st>>>(a);
+    gemm_parts_kernel<4, 4, 2, 4, EPI_PARTS, 0, AUX><<<g64, 256, 0, st>>>(a);
   else if (a.N % 128 == 0)
-    gemm_parts_kernel<8, 8, 4, 3, AUX><<<g128, 512, 0, st>>>(a);
+    gemm_parts_kernel<8, 8, 4, 3, EPI_PARTS, 0, AUX><<<g128, 512, 0, st>>>(a);
   else
-    gemm_parts_kernel<8, 4, 2, 3, AUX><<<g64, 256, 0, st>>>(a);
+    gemm_parts_kernel<8, 4, 2, 3, EPI_PARTS, 0, AUX><<<g64, 256, 0, st>>>(a);
 }
 
 static void launch_parts(const RowsArgs& a, int splits, hipStream_t st) {

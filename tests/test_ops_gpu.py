@@ -699,6 +699,15 @@ def test_whole_k_row_products(M, N, pieces):
                      rtol=2 ** -6)
 
 
+@pytest.mark.parametrize("M", [17, 33, 64, 97, 128])
+@pytest.mark.parametrize("N", [16448, 16512, 32768, 32896])
+@pytest.mark.parametrize("pieces", [1, 2, 3, 4])
+def test_whole_k_row_products_in_shorter_rings(M, N, pieces):
+    """The same where blocks of 128 columns begin, where two of them share a CU and
+    their rings are shorter, and around the length of those."""
+    test_whole_k_row_products(M, N, pieces)
+
+
 @pytest.mark.parametrize("M", [1, 17, 40, 80, 97])
 @pytest.mark.parametrize("N,mode", [(192, 0), (24576, 0), (192, 2), (24576, 2)])
 def test_row_products_to_an_odd_pair_of_columns(M, N, mode):
