@@ -131,8 +131,9 @@ __device__ __forceinline__ void put_rope(const RowsArgs& a, int m, int head, int
   }
 }
 
-// NORM: 0 none, 1 from ss, 2 computed from X.  PD pieces per wave in flight.
-template <int PD, int EPI, int NORM, int AUX>
+// NORM: 0 none, 1 from ss, 2 computed from X.  PD pieces per wave in flight, with DRAIN
+// until the next is needed.
+template <int PD, int EPI, int NORM, int AUX, bool DRAIN>
 __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
   constexpr int NW = 8;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -177,7 +178,7 @@ __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
     if (s < cnt) load(s);
   for (int i = 0; i < cnt; ++i) {
     // piece i has landed when only the loads of the PD - 1 behind it are out
-    if (i + PD <= cnt)
+    if (!DRAIN && i + PD <= cnt)
       __builtin_amdgcn_s_waitcnt(vmcnt_only(4 * (PD - 1)));
     else
       __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
@@ -658,12 +659,20 @@ __global__ void __launch_bounds__(256) rows_sum_kernel(
 // 4.1 from memory, 3.9 against 2.9 from the L2).
 static bool streamed(const RowsArgs& a) { return (i64)a.N * a.K >= (8 << 20); }
 
+// With the norm computed, where some CUs have two blocks and others one, waves that wait
+// for all they have asked for are faster at few rows.  Rotary, in flight / drained in us:
+// 272 blocks, K 4096 11.5 / 10.9 at one row, 11.8 / 11.6 at 8, K 8192 20.0 / 17.7; 384
+// blocks, K 4096 12.6 / 11.9; 448 12.8 / 12.6; but 512 13.6 / 13.6, K 8192 24.1 / 25.7; 256
+// 8.5 / 9.8; 576 16.5 / 18.4; K 2048 from 272 blocks on 0 to 3% slower.
 template <int EPI, int NORM>
 static void launch_rows(const RowsArgs& a, hipStream_t st) {
-  if (streamed(a))
-    gemm_rows_kernel<2, EPI, NORM, STREAM><<<a.N / 16, 512, 0, st>>>(a);
+  const int g = a.N / 16;
+  if (NORM == 2 && g > ROWS_CUS && g <= 448 && a.K >= 4096 && a.M <= 8)
+    gemm_rows_kernel<2, EPI, NORM, STREAM, NORM == 2><<<g, 512, 0, st>>>(a);
+  else if (streamed(a))
+    gemm_rows_kernel<2, EPI, NORM, STREAM, false><<<g, 512, 0, st>>>(a);
   else
-    gemm_rows_kernel<2, EPI, NORM, KEEP><<<a.N / 16, 512, 0, st>>>(a);
+    gemm_rows_kernel<2, EPI, NORM, KEEP, false><<<g, 512, 0, st>>>(a);
 }
 
 // Blocks of 128 weight rows halve the reads of X; they pay where blocks of 64 are more

@@ -892,6 +892,23 @@ def test_qkv_rope_rows(M, Hq, Hk, K):
     assert close(kc, kw, **tol) and close(vc, vw, **tol)
 
 
+@pytest.mark.parametrize("M", [1, 8, 9])
+@pytest.mark.parametrize("heads", [34, 56])
+def test_rows_with_a_norm_between_one_and_two_blocks_per_cu(M, heads):
+    """The waves that drain their loads, and one row more than they are used for:
+    rotary, SwiGLU and plain.  Tolerances as in the tests of each."""
+    K, N = 4096, heads * 128
+    test_qkv_rope_rows(M, heads - 2, 1, K)
+    x, w = rnd(M, K, seed=M, scale=0.3), rnd(N, K, seed=N, scale=0.3)
+    y = (x.float() * torch.rsqrt(x.float().pow(2).mean(-1, keepdim=True) + 1e-5)
+         ) @ w.float().t()
+    g, u = y.chunk(2, -1)
+    assert close(ops.linear_rows(x, w, 2, scale=(None, 1e-5)),
+                 torch.nn.functional.silu(g) * u, atol=2e-3 * K ** 0.5, rtol=2 ** -6)
+    assert close(ops.linear_rows(x, w, scale=(None, 1e-5)), y, atol=2e-3 * K ** 0.5,
+                 rtol=2 ** -7)
+
+
 @pytest.mark.parametrize("M", [3, 40])
 def test_qkv_rope_rows_refuses_other_geometries(M):
     """Head sizes other than 128, weights that are not whole heads, pages, stats
