@@ -549,26 +549,50 @@ def _wide_out_ok(out: torch.Tensor, x: torch.Tensor, M: int, N: int) -> bool:
 
 def _wide_pays(M: int, N: int, K: int, silu_fuse: bool) -> bool:
     """Whether the wide GEMM beats the library's, by the tiles that its 256 blocks
-    take, from 15 projections of four models at 256..9000 rows.
+    take.  Times are the library's over the wide GEMM's, weights not in cache.
 
     With SwiGLU behind it, which the library leaves to a pass of its own: where its
-    smallest tiles, 128 x 256, occupy 172 blocks.  7 projections at 256..2300 rows,
-    weights not in cache, library over wide: 0.70..1.00 up to 168 blocks and K of 4096
-    or more (7168 x 4096 at 513 rows 45.5 us / 51.0, 14336 x 4096 at 320 rows 52.9 /
-    58.5), from 172 on 0.93..1.50, 1.13 in the mean (28672 x 4096 at 448 rows 109 / 91,
-    1024 rows 219 / 191, 4096 rows 720 / 668).
-    Plain, by 256 x 256 tiles: the library is 5-8% ahead in whole rounds (4096 x 4096
-    at 8000 rows 179 us / 189) and draws level below one, but falls back by up to 1.78
-    where a round is begun (4096 x 14336 at 4352 rows 720 / 410, 8448 rows 1003 / 700;
-    6144 x 4096 at 8448 rows 393 / 310).  Up to half a round the wide GEMM took 34 of
-    47 sizes and lost 8% at most; with a long K the library stays behind further (4096
-    x 14336 at 6800 rows 920 / 570, at 7400 970 / 600)."""
+    smallest tiles, 128 x 256, occupy 172 blocks (16 projections at 257..1373 rows:
+    0.89..0.95 up to 168 tiles, 1.18 in the mean from 172 on, 0.96 at least).  Three
+    rows of tiles of a K of 2048..4095 need 200: 16384 x 3072 0.84 at 257 rows, 0.92
+    at 381, 1.11 at 412; 18432 x 2048, 216 tiles, 1.13.  Not 449..512 rows that make
+    one round of 168..192 tall tiles with a longer K: 22016 x 4096 1.09 at 448 rows,
+    0.98 at 512, 1.10 at 513, 24576 x 8192 1.09, 0.91, 0.98, but 20480 x 4096 1.08.
+
+    Plain, by 256 x 256 tiles: the library is ahead in whole rounds (4096 x 4096 at
+    8000 rows 0.95) and draws level below one, but falls back where a round is begun.
+    How far goes with its own choice of tiles; these limits leave 716 of 1374 sizes
+    (23 projections, 263..10284 rows), 1.19 in the mean, 0.96 at least:
+    - K >= 2N, up to 216 tiles begun: 1.0..1.9 (4096 x 14336 at 4353 rows 1.74, 7400
+      rows 1.61).  Not 64 or 128 behind a first round, which the library cuts evenly
+      (8192 x 28672 at 2402 rows 0.89, 4096 x 14336 at 5006 0.96), and above 5120
+      columns not 64 behind two rounds (0.94) or anything beyond (0.90).
+    - up to 5120 columns, 128 begun: 0.96..1.55; 129..216 0.91..1.4.
+    - wider: 63 behind one round (128 0.92 at 12288 x 4096), 128 behind two or four
+      (1.34 at 10240 x 8192, 4076 rows), 95 behind three or five (0.93 beyond that),
+      three not from a K of 8192 on (8192 x 8192 at 6587 rows 0.93), none behind six
+      (0.91) or more.  Above 12288 columns one or two rounds lose (28672 x 4096 at 1100
+      rows 0.95) and 63 is the limit for all (22016 x 4096 at 2560 rows, 92 behind
+      three, 0.86)."""
     cols = -(-N // 256)
     if silu_fuse:
-        return -(-M // 128) * cols >= 172
+        tiles = -(-M // 128) * cols
+        return (tiles >= (200 if M <= 384 and 2048 <= K < 4096 else 172)
+                and not (448 < M <= 512 and 336 <= tiles <= 384 and K >= 4096))
     tiles = -(-M // 256) * cols
-    begun = tiles & 255
-    return tiles > 256 and 0 < begun <= (216 if K >= 2 * N else 128)
+    rounds, begun = tiles >> 8, tiles & 255
+    if rounds < 1 or begun == 0:
+        return False
+    if K >= 2 * N:
+        if rounds == 1 and begun in (64, 128):
+            return False
+        return begun <= 216 and (N <= 5120 or rounds == 1
+                                 or rounds == 2 and begun != 64)
+    if rounds > 5 or rounds < 3 and N > 12288 or rounds == 3 and K >= 8192:
+        return False
+    if N <= 5120 or rounds in (2, 4) and N <= 12288:
+        return begun <= 128
+    return begun < (64 if rounds == 1 or N > 12288 else 96)
 
 
 def launch_wide(x, w, silu_fuse=False, out=None, groups=0):
@@ -594,11 +618,13 @@ def _wide_split_pays(M: int, N: int, K: int) -> bool:
     2500 rows 238 / 270, 28672 -> 8192 at 640 rows 275 / 292), 8192 -> 2048 0.93..1.12,
     K < 2N mostly below 1 (4096 x 4096 at 512 rows 26 / 30).  The shares, which
     divide K in whole pieces, have to occupy most of the blocks: with the 128 that
-    11008 allows at 129 rows 44 us / 52."""
+    11008 allows at 129 rows 44 us / 52.  Many rows of few columns make the parts the
+    larger stream again: 10240 -> 2048 at 1275 rows 79 / 70, at 1458 71 / 75, 2068 rows
+    103 / 114 (but 16384 -> 2048 at 1275 rows 1.17 or more)."""
     cols = -(-N // 256)
     tiles = -(-M // 256) * cols
     if not (M > 128 and K >= 2 * N and K > 8192 and K % 64 == 0 and tiles <= 128
-            and tiles * K <= 1 << 21):
+            and tiles * K <= 1 << 21 and (8 * M <= 5 * N or K >= 16384)):
         return False
     return -(-M // 128) * cols * _lib.lib().af_gemm_wide_splits(M, N, K) >= 192
 

@@ -231,6 +231,36 @@ def test_wide_gemm_pays(M, N, K, glu, pays):
     assert ops._wide_pays(M, N, K, glu) == pays
 
 
+@pytest.mark.parametrize("M,N,K,glu,pays", [
+    (5120, 4096, 14336, False, False),            # 64 begun, even shares of K
+    (5121, 4096, 14336, False, True), (5632, 5120, 13824, False, True),
+    (2500, 8192, 28672, False, False), (2700, 8192, 28672, False, True),
+    (4500, 8192, 28672, False, False), (6300, 8192, 28672, False, False),
+    (2030, 12288, 4096, False, False), (1500, 12288, 4096, False, True),
+    (10077, 12288, 4096, False, False), (9900, 10240, 8192, False, False),
+    (4000, 10240, 8192, False, True), (6500, 8192, 8192, False, False),
+    (6500, 8192, 3584, False, True), (6900, 8192, 3584, False, False),
+    (1100, 28672, 4096, False, False), (2048, 28672, 4096, False, False),
+    (1024, 22016, 4096, False, False), (5000, 14336, 4096, False, False),
+    (257, 16384, 2048, True, False), (384, 16384, 3072, True, False),
+    (385, 16384, 3072, True, True), (257, 20480, 2048, True, True),
+    (384, 16384, 1024, True, True), (257, 22016, 4096, True, True),
+    (448, 22016, 4096, True, True), (449, 22016, 4096, True, False),
+    (512, 24576, 8192, True, False), (513, 22016, 4096, True, True),
+    (512, 22016, 2048, True, True), (512, 20480, 4096, True, True),
+    (2560, 22016, 4096, False, False), (2300, 22016, 4096, False, True),
+])
+def test_wide_gemm_leaves_what_the_library_does_better(M, N, K, glu, pays):
+    assert ops._wide_pays(M, N, K, glu) == pays
+
+
+@pytest.mark.parametrize("M,N,K,pays", [
+    (1280, 2048, 10240, True), (1281, 2048, 10240, False), (2068, 2048, 10240, False),
+    (2048, 2048, 16384, True)])
+def test_wide_gemm_split_of_few_columns(M, N, K, pays):
+    assert ops._wide_split_pays(M, N, K) == pays
+
+
 @pytest.mark.parametrize("M,N,K,pays", [
     (128, 4096, 14336, False), (257, 4096, 14336, True), (2048, 4096, 14336, True),
     (2049, 4096, 14336, False),                   # 144 tiles
