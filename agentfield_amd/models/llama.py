@@ -234,7 +234,8 @@ class MoEMLP(nn.Module):
       its routed token subset — FLOP-proportional, shapes data-dependent.
       On the GPU the rows are routed and sorted by expert in two kernels, so
       that a subset is one block of rows (ops.moe_route), and each projection
-      is one launch over all experts where ops.moe_gemm_ok says so.
+      is one launch over all experts where ops.moe_gemm_ok and moe_gemm_pays
+      say so.
     * decode (static, hipGraph-capturable): every expert runs on every
       token with routing weights zeroed for unrouted pairs.  Decode
       GEMMs are weight-streaming-bound and a top-2-of-8 batch >= ~16
@@ -298,7 +299,8 @@ class MoEMLP(nn.Module):
     def _forward_sorted(self, x):
         weights, row, pos, offs = ops.launch_moe_route(x, self.router,
                                                        self.top_k)
-        if ops.moe_gemm_ok(x, self.router, self.gate_up, self.down):
+        if (ops.moe_gemm_ok(x, self.router, self.gate_up, self.down)
+                and ops.moe_gemm_pays(row.numel(), *self.down.shape)):
             act = ops.launch_experts(x, self.gate_up, offs, row.numel(), row,
                                      swiglu=True)
             ys = ops.launch_experts(act, self.down, offs, row.numel())

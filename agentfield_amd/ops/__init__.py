@@ -756,6 +756,18 @@ def moe_gemm_ok(x: torch.Tensor, router: torch.Tensor, gate_up: torch.Tensor,
             and rows_operands_ok((x, gate_up, down)))
 
 
+def moe_gemm_pays(n: int, E: int, H: int, I: int) -> bool:
+    """Whether one launch per projection beats the row GEMMs expert by expert behind a
+    wait of the host.  Not where the down projection, a block to 128 of its columns and
+    every expert in use, leaves half of the CUs idle through a long K: the whole
+    feed-forward expert by expert / in one launch, us: 2 of 8 experts of 4096 x 14336 at
+    one row 150 / 165, 2 of 4 146 / 165, 4 rows of 4 187 / 195, 6 rows of 8 325 / 304;
+    1 of 2 of 8192 x 28672 247 / 344, 32 rows 529 / 555; but 2 of 8 of 4096 x 7168 103 /
+    100, one of 8192 x 7168 109 / 106."""
+    idle = min(n, E) * -(-H // 128) <= 128
+    return not (idle and (I > 8192 and n <= 4 or I > 16384 and n <= 32 * E))
+
+
 def launch_moe_gemm(x, w, offs, n, row=None, swiglu=False):
     """n sorted rows against their expert's w [E, N, K], for callers that have asked
     moe_gemm_ok: x rows through row [n], or x in sorted order."""
@@ -773,10 +785,13 @@ def wide_experts_pay(x_rows: int, n: int, E: int, N: int, K: int,
     """Whether n sorted rows go to the wide GEMM rather than to moe_gemm: what it
     takes beside moe_gemm_ok (x and half an expert's weights within 4 GB), and rows
     enough that the matrix cores bound it and not the weight stream.  Measured with 8
-    experts of 4096 x 14336, moe_gemm / wide in us: gate/up 425 / 447 at 175 rows per
-    expert, 475 / 445 at 200, 594 / 522 at 275, 735 / 528 at 300, 1930 / 1593 at
-    1024; down 253 / 272 at 225, 291 / 286 at 250, 378 / 287 at 288, 922 / 809 at
-    1024."""
+    experts of 4096 x 14336, moe_gemm / wide in us: gate/up 445 / 454 at 180 rows per
+    expert, 478 / 463 at 200, 589 / 536 at 260, 741 / 598 at 300, 1911 / 1567 at
+    1024; down 242 / 265 at 200, 282 / 279 at 250, 429 / 287 at 288, 915 / 804 at
+    1024.  With 15 shapes of 2..64 experts and 256..6144 x 512..16384 gate/up is ahead
+    from 200 rows on in all (1.0..1.7), down from 250 on in all but the fewest tiles (8
+    experts of 2048 x 1024, 64 of 256 blocks, 25 / 21 at 250 and 25 / 21 at 320; 4 of
+    4096 x 14336 196 / 228 at 320 rows, 241 / 253 at 500, 377 / 253 at 600)."""
     return (n >= (200 if swiglu else 250) * E and N >= 256 and K >= 128
             and x_rows * K * 2 < 1 << 32 and (N // 2 + 256) * K * 2 < 1 << 32
             and n <= 1 << 24)

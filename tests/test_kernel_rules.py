@@ -170,6 +170,15 @@ def test_experts_that_the_sorted_products_take(ok, gate_up, down):
     assert ops.moe_gemm_ok(mat(5, 64), mat(4, 64), gate_up, down) == ok
 
 
+@pytest.mark.parametrize("n,E,H,I,pays", [
+    (2, 8, 4096, 14336, False), (4, 4, 4096, 14336, False),
+    (6, 8, 4096, 14336, True), (8, 4, 4096, 14336, True),
+    (2, 8, 4096, 8192, True), (2, 8, 6144, 16384, False), (4, 8, 6144, 16384, True),
+    (64, 2, 8192, 28672, False), (65, 2, 8192, 28672, True), (2, 4, 256, 512, True)])
+def test_when_one_launch_per_projection_pays(n, E, H, I, pays):
+    assert ops.moe_gemm_pays(n, E, H, I) == pays
+
+
 @pytest.mark.parametrize("lens,want", [
     ([8000], (32, 250, 0, 1)),                     # one long prompt
     ([700, 3, 8, 500, 9], (32, 39, 2, 4)),         # both kinds of items

@@ -1177,6 +1177,30 @@ def test_moe_sorted_products(counts, launch, I, H):
         at += c
 
 
+@pytest.mark.parametrize("T", [1, 2, 75])
+def test_moe_prompt_expert_by_expert(T, monkeypatch):
+    """The same rows by one launch per projection and, where that does not pay, expert
+    by expert: fp32 sums in another order, rounded to bf16 three times (gate/up, down,
+    combination; 2^-9 of a value each)."""
+    from agentfield_amd.models import CONFIGS
+    from agentfield_amd.models.llama import MoEMLP
+    mlp = MoEMLP(CONFIGS["tiny-moe"]).to(DEV, torch.bfloat16)
+    calls = []
+    launch = ops.launch_experts
+    monkeypatch.setattr(ops, "launch_experts",
+                        lambda *a, **kw: calls.append(a) or launch(*a, **kw))
+    with torch.inference_mode():
+        for i, p in enumerate(mlp.parameters()):
+            p.copy_(rnd(*p.shape, seed=i, scale=0.2))
+        x = rnd(T, 256, seed=T)
+        one = mlp(x).float()
+        assert len(calls) == 2
+        monkeypatch.setattr(ops, "moe_gemm_pays", lambda *a: False)
+        each = mlp(x).float()
+    assert len(calls) == 2
+    assert (one - each).norm() <= 3 * 2 ** -8 * one.norm()
+
+
 def test_moe_prompt_under_capture():
     """The mixture's prompt rows need no wait of the host: a captured step gives the
     eager bits on every replay, with other rows and routes each time."""
