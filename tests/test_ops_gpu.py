@@ -1264,6 +1264,59 @@ def test_few_row_path_with_strided_weights(T, layer, prompt):
     assert (a - b).norm() <= 1e-2 * a.norm()
 
 
+@pytest.mark.parametrize("T,rows", [
+    (1, None), (16, None), (17, None), (40, None), (128, None), (40, 1), (40, 16),
+    (40, 17), (128, 20)])
+def test_logits_of_the_few_row_path(T, rows, monkeypatch):
+    """The final norm as a scalar of the vocabulary product, computed by it (up to 16
+    rows) or from the sums that the last layer left, against the general path, whose
+    final norm is a launch of its own: all rows' logits and those of a few.  The
+    residual is small enough that a tenth of the norm is its epsilon.  Tolerance: both
+    are bf16 roundings of the same two layers, 1% of the logits' norm."""
+    from agentfield_amd.models import CONFIGS
+    from agentfield_amd.models.llama import (AttnMetadata, KVCache,
+                                             LlamaForCausalLM)
+    cfg, page = CONFIGS["tiny"], 16
+    m = LlamaForCausalLM(cfg, device=DEV).init_random(4)
+    asked = []
+    launch = ops.launch_rows
+
+    def spy(x, w, *args, scale=None, **kw):
+        if w is m.lm_head:
+            asked.append(scale)
+        return launch(x, w, *args, scale=scale, **kw)
+    monkeypatch.setattr(ops, "launch_rows", spy)
+    pos = torch.arange(T, device=DEV, dtype=torch.int32)
+    md = AttnMetadata(
+        is_prefill=True, slots=pos.long() + page, seq_lens=[T],
+        block_table=torch.arange(1, 10, device=DEV, dtype=torch.int32)[None],
+        cu_seqlens=torch.tensor([0, T], device=DEV, dtype=torch.int32),
+        q_start=torch.zeros(1, device=DEV, dtype=torch.int32))
+    with torch.no_grad():
+        m.embed.mul_(0.5)
+        for layer in m.layers:
+            layer.attn.o.mul_(0.1)
+            layer.mlp.down.mul_(0.1)
+        m.final_norm.copy_(1 + 0.5 * torch.rand(cfg.hidden_size, device=DEV))
+        m.fold_norm_weights()
+        ids = torch.randint(0, cfg.vocab_size, (T,), device=DEV, dtype=torch.int32)
+        pick = None if rows is None else torch.randperm(T, device=DEV)[:rows].int()
+        assert m._can_fuse_rows(T)
+        got = m(ids, pos, KVCache(cfg, 16, page, DEV), md, logit_rows=pick).float()
+        (scale,) = asked
+        few = (rows or T) <= ops.ROWS_MAX
+        if rows is None or few:
+            assert scale[1] == cfg.rms_eps and (scale[0] is None) == few
+        else:
+            assert scale is None          # gathered rows have no sums
+        m.no_fused_decode = True
+        want = m(ids, pos, KVCache(cfg, 16, page, DEV), md, logit_rows=pick).float()
+        resid = m.embed[ids.long()].float()
+    assert 0.05 < cfg.rms_eps / resid.pow(2).mean() < 0.5
+    assert got.shape == (rows or T, cfg.vocab_size)
+    assert (got - want).norm() <= 1e-2 * want.norm()
+
+
 @pytest.mark.parametrize("M,N,K", [
     (256, 256, 128),          # one tile, two pieces of K
     (257, 320, 128),          # both moved back inside the matrix
