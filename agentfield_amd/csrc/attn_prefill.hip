@@ -58,7 +58,7 @@
 // scalar writes (one layer, 8 K/V heads, G = 4): one prompt of 8000 rows 2292 ->
 // 544 us (229 -> 960 TFLOP/s), 20 of 300..700 384 -> 104 us, 8 x 2048 at G = 2
 // 992 -> 232 us; 16 sequences of 5 rows behind 2400 tokens 387 -> 43 us.
-#include "common.h"
+#include "mfma_lines.h"
 
 #define AP_D 128
 #define AP_KV 64          // tokens per shared tile
@@ -142,7 +142,7 @@ __device__ __forceinline__ int table_entry(const i32* row, int i) {
 template <int N>
 __device__ __forceinline__ void landed() {
   asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4) << 14 | 0x0f70);
+  __builtin_amdgcn_s_waitcnt(vmcnt_only(N));
   asm volatile("" ::: "memory");
 }
 

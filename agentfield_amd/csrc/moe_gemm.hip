@@ -21,8 +21,6 @@
 // bounds, 4096 x 14336 x 8: 20 rows 505 -> 431 us, 200 589 -> 480, 600 1083 -> 631.
 #include "mfma_lines.h"
 
-#include <type_traits>
-
 enum MoeEpi { MOE_PLAIN = 0, MOE_SWIGLU = 2 };
 
 #define MG_MT 18                       // 16-row groups of X per block
@@ -45,21 +43,6 @@ struct MoeGemmArgs {
   const i32* offs;   // [E + 1]
   int E, N, K;
 };
-
-// All but n groups of PER of a wave's loads have landed (n <= 4), its LDS reads are
-// done, and so it is for every wave of the block.
-template <int PER>
-__device__ __forceinline__ void moe_meet(int n) {
-  asm volatile("" ::: "memory");
-  if (n >= 4) __builtin_amdgcn_s_waitcnt(vmcnt_only(4 * PER) & ~0x0f00);
-  else if (n == 3) __builtin_amdgcn_s_waitcnt(vmcnt_only(3 * PER) & ~0x0f00);
-  else if (n == 2) __builtin_amdgcn_s_waitcnt(vmcnt_only(2 * PER) & ~0x0f00);
-  else if (n == 1) __builtin_amdgcn_s_waitcnt(vmcnt_only(PER) & ~0x0f00);
-  else __builtin_amdgcn_s_waitcnt(vmcnt_only(0) & ~0x0f00);
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 // Rows pos0 .. pos0 + rows (up to 32 MW) of the sorted order against the weight rows of
 // block column nb.
@@ -122,7 +105,7 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, char* lds, int e,
 #pragma unroll 1
   for (int i = 0; i < cnt; ++i) {
     // piece i is complete for everybody, and piece i - 1 read by everybody
-    moe_meet<PER>(min(STAGES - 2, cnt - 1 - i));
+    meet<PER>(min(STAGES - 2, cnt - 1 - i));
     if (i + STAGES - 1 < cnt) load();
     const lds_b* at = ring + slot * STAGE;
     slot = slot + 1 == STAGES ? 0 : slot + 1;
@@ -153,28 +136,8 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, char* lds, int e,
     }
   }
 
-  // the two waves of a product swap sums: each finishes two of its tiles
-  __syncthreads();
-  f32x4* give = reinterpret_cast<f32x4*>(lds) + wid * 2 * MW * 64 + lane;
-  const f32x4* take = reinterpret_cast<const f32x4*>(lds) + (wid ^ 4) * 2 * MW * 64 + lane;
   f32x4 sum[2][MW];
-  auto swap = [&](auto upper) {
-    constexpr int U = decltype(upper)::value;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int m = 0; m < MW; ++m) {
-        give[(t * MW + m) * 64] = acc[2 - 2 * U + t][m];
-        sum[t][m] = acc[2 * U + t][m];
-      }
-  };
-  if (kh == 0) swap(std::integral_constant<int, 0>{});
-  else swap(std::integral_constant<int, 1>{});
-  __syncthreads();
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int m = 0; m < MW; ++m) sum[t][m] += take[(t * MW + m) * 64];
+  swap_sums<MW>(lds, wid, wid ^ 4, kh, acc, sum);
 
   // lane: row n of each group, columns 4 q .. + 4 of each tile
   const int tile = nb * MG_NT + w0 + kh * 2;
@@ -183,16 +146,7 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, char* lds, int e,
     const int r = (m0 + m) * 16 + n;
     u16* o = a.out + (size_t)(pos0 + r) * (EPI == MOE_SWIGLU ? a.N >> 1 : a.N);
     if (EPI == MOE_SWIGLU) {
-      // gate rows lie in the lower lanes and up rows in the upper ones: the lower
-      // lanes get both of the first tile, the upper ones both of the second
-      u16x4 v;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const auto gu = __builtin_amdgcn_permlane32_swap(
-            __float_as_uint(sum[0][m][j]), __float_as_uint(sum[1][m][j]), false, false);
-        const float g = __uint_as_float(gu[0]), u = __uint_as_float(gu[1]);
-        v[j] = f2bf(g / (1.f + __expf(-g)) * u);
-      }
+      const u16x4 v = swiglu_tiles(sum[0][m], sum[1][m]);
       const int mine = tile + (lane >> 5);
       if (r < rows && mine <= last)
         *reinterpret_cast<u16x4*>(o + mine * 8 + (q & 1) * 4) = v;
