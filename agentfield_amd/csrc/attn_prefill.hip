@@ -185,8 +185,8 @@ __device__ __forceinline__ void stage(const PrefillArgs& a, const i32* btrow,
 
 // o += a b, in place: left to itself the compiler puts the result elsewhere and copies 64
 // registers back per tile (together with the maximum in attend() 582 -> 569 us for one
-// prompt of 8000 rows, 105 -> 93 for 20 of 300..700).  Two wait states for operands that were just written; who reads
-// the sums other than as a sum again is behind settled().
+// prompt of 8000 rows, 105 -> 93 for 20 of 300..700).  Two wait states for operands that
+// were just written; who reads the sums other than as a sum again is behind settled().
 __device__ __forceinline__ void add_product(f32x16& o, bf16x8 a, bf16x8 b) {
   asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0"
                : "+v"(o) : "v"(a), "v"(b));

@@ -31,6 +31,7 @@
 //   The fp32 parts meet in the kernel that does the next step.  Bound by the parts
 //   (16.8 MB at 128 rows, written at ~2.5 TB/s after the stream has ended: 7 of the 15
 //   us of 4096 x 4096) and by starts, not by its loop: the loop below was no faster.
+//   Unsplit, it also serves plain products of 97..128 rows in blocks of 128 columns.
 // gemm_tile_kernel, whole K (SwiGLU, plain): at 128 rows the loop of the kernel above
 //   takes 0.47 us per piece without any load, nearly what the memory needs for the
 //   128 weight rows of a piece (0.57), and the two did not overlap.  So half of the
@@ -59,7 +60,7 @@
 // fp32 rounding between steps of different sizes.
 // Measured in us, alone and repeated (inside a step 5-25% more), against the split-K
 // kernel with two-stage buffers and its second launch (in brackets).  One row: 6144 x
-// 4096 with rotary and append 11.4 (21.3 in three launches), 4096 x 4096 7.2 and 4096 x
+// 4096 with rotary and append 11.3 (21.3 in three launches), 4096 x 4096 7.2 and 4096 x
 // 14336 19.5 (together 44.4), SwiGLU over 28672 x 4096 36.0 = 6.5 TB/s (58.2).  16
 // rows: 13.3, 8.0, 23.3, 41.2.  64 rows, without the closing launches: 13.1, 9.3,
 // 23.3, 38.9 (16.7, o + down 44.8, 62.7).  128 rows: 16.9, 15.0, 27.5, 48.0 (library

@@ -529,9 +529,9 @@ __global__ void __launch_bounds__(256) diff_combine_kernel(
 // Workgroup = (sequence, head, 32-column tile of dv); 256 threads = 16 row
 // groups x 16 column pairs, or 512 = 16 x 32 columns.  A thread keeps RP consecutive
 // rows of its columns of the state in registers (each q / k / decay value read from
-// LDS feeds both of two columns).  Tokens are walked serially in blocks of TB: the block's q / k / decay
-// rows are staged into LDS at once (rotary + scaling applied on the way in), the
-// recurrence itself is strictly token by token in fp32, and both kernels use the
+// LDS feeds both of two columns).  Tokens are walked serially in blocks of TB: the
+// block's q / k / decay rows are staged into LDS at once (rotary + scaling applied on
+// the way in), the recurrence itself is strictly token by token in fp32, and both kernels use the
 // same operations (scan_*) and sum the 16 row groups in the same order — so they
 // give the same bits, and results do not depend on how a sequence is cut into
 // chunks or on what else is in the step.
@@ -782,7 +782,9 @@ __global__ void __launch_bounds__(256) linear_scan_kernel(
 }
 
 // Rows of a token that a thread of the prompt kernel stages
-constexpr int scan_rows(int rp, int threads) { return (rp >= 16 ? 8 : 16) * 16 * rp / threads; }
+constexpr int scan_rows(int rp, int threads) {
+  return (rp >= 16 ? 8 : 16) * 16 * rp / threads;
+}
 
 // The same recurrence for prompts.  A thread stages E consecutive rows of one token
 // (one wide load each for q, k, the rotary partners and the decay logits, kept raw
@@ -1260,9 +1262,11 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
 #define SCAN_PROMPT(RP, NT)                                                  \
   do {                                                                       \
     if (zl)                                                                  \
-      linear_scan_prompt_kernel<S, RP, true, NT><<<grid, NT, sm, s>>>(SCAN_ARGS); \
+      linear_scan_prompt_kernel<S, RP, true, NT>                             \
+          <<<grid, NT, sm, s>>>(SCAN_ARGS);                                  \
     else                                                                     \
-      linear_scan_prompt_kernel<S, RP, false, NT><<<grid, NT, sm, s>>>(SCAN_ARGS); \
+      linear_scan_prompt_kernel<S, RP, false, NT>                            \
+          <<<grid, NT, sm, s>>>(SCAN_ARGS);                                  \
   } while (0)
 #define SCAN(RP)                                                             \
   do {                                                                       \

@@ -175,7 +175,8 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(
 // 38.8 at 4096, 62 / 70 at 8192; rows of 1024: 12.5 / 12.0 at 1000, 16.8 / 18.4 at 2000; 2
 // experts, rows of 4096: 16.3 / 15.9 at 2000, 17.2 / 20.2 at 3000; 32 experts, rows of
 // 1024: 40.5 / 35.4 at 600, 45.8 / 48.0 at 800; 64 experts, rows of 2048: 95 / 60 at 200,
-// 115 / 157 at 600, rows of 8192: 256 / 271 at 600.  A row of 256 is one load anyway (4 experts, 1000 rows 9.7 / 10.5).
+// 115 / 157 at 600, rows of 8192: 256 / 271 at 600.  A row of 256 is one load anyway (4
+// experts, 1000 rows 9.7 / 10.5).
 static bool route_shares_rows(int T, int H, int E) {
   if (H < 1024) return false;
   if (E > 32) return T <= min(H / 8, 512);

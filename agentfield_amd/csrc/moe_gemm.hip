@@ -2,9 +2,10 @@
 // all experts,  Y[rows of e] = X[rows of e] @ W[e]^T, rows gathered through the sorted
 // order where they are still the caller's, SwiGLU in the epilogue.
 //
-// Prompts of up to a few hundred rows per expert are bound by the experts' weights as
-// much as by the matrix cores (1100 rows, 8 experts, 2 per row: 2.8 GB or 435 us at 6.5
-// TB/s, 775 GFLOP or 310 us).  A block takes all rows of an expert, up to 288, against
+// Prompts of up to 200 rows per expert (down 250, above which the wide GEMM takes over)
+// are bound by the experts' weights more than by the matrix cores (600 rows, 8 experts of
+// 4096 x 14336, 2 per row: 2.8 GB or 435 us at 6.5 TB/s, 423 GFLOP or 280 us; 429 us of
+// gate/up and 203 of down).  A block takes all rows of an expert, up to 288, against
 // 128 weight rows, so the weights are read once; more rows are cut evenly, and the cuts
 // of one block column run on one XCD at the same time.  Both operands go global -> LDS
 // without registers, in stages of K = 64 (52 KB at 288 rows, three of them); half of the
@@ -12,13 +13,15 @@
 // half of the rows (144 registers of sums per lane, of the 256 that two waves leave).
 // The loop is unrolled for the number of 16-row groups per wave, so few rows cost few
 // products.
-// What bounds it now, at 1100 rows: the 52 KB per piece, which arrive at 12.3 TB/s in
-// all (loads alone 541 us of gate/up, products alone 387, both 600).  Weights through
-// registers instead of LDS, 16 rows x 64 bytes per load, were slower (640 us, at half of
-// the rows per wave 1420 with spills).
-// From 200 rows per expert on (down 250) the wide GEMM takes over.  Against one library
-// product per expert and projection, gathered rows and a wait of the host for the block
-// bounds, 4096 x 14336 x 8: 20 rows 505 -> 431 us, 200 589 -> 480, 600 1083 -> 631.
+// Where experts' rows are uneven it still sees blocks of 288.  With 275 rows of every
+// expert, more than it is sent now, the 52 KB per piece bounded it, which arrive at 12.3
+// TB/s in all (loads alone 541 us of gate/up, products alone 387, both 600).  Weights
+// through registers instead of LDS, 16 rows x 64 bytes per load, were slower there (640
+// us, at half of the rows per wave 1420 with spills), and so were, at one row, rings
+// short enough for two blocks to a CU (165 -> 182 us of the whole feed-forward).
+// Feed-forward of 8 experts of 4096 x 14336 against one library product per expert and
+// projection, gathered rows and a wait of the host for the block bounds: 20 rows 488 ->
+// 429 us, 200 577 -> 474, 600 1119 -> 639.
 #include "mfma_lines.h"
 
 enum MoeEpi { MOE_PLAIN = 0, MOE_SWIGLU = 2 };
@@ -32,7 +35,8 @@ enum MoeEpi { MOE_PLAIN = 0, MOE_SWIGLU = 2 };
 // Up to 192 rows the weights dominate: they are streamed past the caches, and blocks of
 // an XCD start at different pieces of K, or they ask one memory channel for everything
 // (40 rows: 307 us of gate/up without the first, 341 without the second, 276 with both).
-// Above, pieces in step keep the rows of X in the L2 (4096 rows: 2001 -> 1802 us).
+// Above, pieces in step keep the rows of X in the L2 (512 rows of every expert: 2001 ->
+// 1802 us of gate/up).
 #define MG_FEW 6                       // 16-row groups per wave
 
 struct MoeGemmArgs {

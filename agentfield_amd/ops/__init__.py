@@ -327,10 +327,11 @@ def _rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
 def rows_pay(M: int, N: int) -> bool:
     """Whether plain products of up to 128 rows go to the row GEMMs: those of 33..128
     rows lose to the library where N fills the chip neither in blocks of 128 columns
-    nor in several splits.  Measured, library against rows in us: 14336 x 4096 25.6 / 21.7 at 32 rows, 26.7 / 30.0 at 48,
-    33.9 / 36.0 at 128; 16384 x 4096 34.3 / 24.7, 34.9 / 38.9, 39.0 / 43.3;
-    28672 x 4096 53.9 / 41.5, 64.0 / 42.1, 56.7 / 51.7; 128256 x 4096 190 / 151
-    at one row, 214 / 184 at 64, 238 / 215 at 128.  Between 12288 and 24576
+    nor in several splits.  Measured, library against rows in us: 14336 x 4096
+    25.6 / 21.7 at 32 rows, 26.7 / 30.0 at 48, 33.9 / 36.0 at 128; 16384 x 4096
+    34.3 / 24.7, 34.9 / 38.9, 39.0 / 43.3; 28672 x 4096 53.9 / 41.5, 64.0 / 42.1,
+    56.7 / 51.7; 128256 x 4096 190 / 151 at one row, 214 / 184 at 64, 238 / 215 at
+    128.  Between 12288 and 24576
     these two were measured; the limits are the nearest sizes at which rows win."""
     return M <= 32 or N <= 12288 or N >= 24576
 
@@ -611,8 +612,8 @@ def launch_wide(x, w, silu_fuse=False, out=None, groups=0):
 def _wide_split_pays(M: int, N: int, K: int) -> bool:
     """Whether the wide GEMM with K in shares beats the library's: few tiles of 256 x
     256 and a long K, so that the parts' way through memory is small beside the weights'.
-    10 projections at 129..3000 rows, weights not in cache, library over split: with K
-    >= 2N, K > 8192, up to 128 tiles and tiles * K up to 2^21 0.94..2.28, 1.33 in the
+    21 projections at 129..3000 rows, weights not in cache, library over split: with K
+    >= 2N, K > 8192, up to 128 tiles and tiles * K up to 2^21 0.96..2.8, 1.33 in the
     mean (14336 -> 4096 at 192 rows 104 us / 48, 640 rows 113 / 84, 1500 rows 170 /
     155; 28672 -> 8192 at 512 rows 309 / 225); beyond that 0.83..1.06 (14336 -> 4096 at
     2500 rows 238 / 270, 28672 -> 8192 at 640 rows 275 / 292), 8192 -> 2048 0.93..1.12,

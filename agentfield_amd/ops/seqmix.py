@@ -674,8 +674,9 @@ def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
 
     bf16 products of few rows (decode steps) run on the framework's
     weight-streaming kernels, wider ones and prompts on the vendor GEMM
-    (hipBLASLt / rocBLAS) or, where that has begun a round, on the wide GEMM.  Above 16 rows a second launch adds the K splits up
-    unless N fills the chip by itself, which middling widths do not earn back.
+    (hipBLASLt / rocBLAS) or, where that has begun a round, on the wide GEMM.  Above
+    16 rows a second launch adds the K splits up unless N fills the chip by itself,
+    which middling widths do not earn back.
     Measured, vendor against rows in us: 4096 x 4096 15.7 / 7.8 at 4 rows, 15.3 /
     12.7 at 64, 16.2 / 18.2 at 100; 6144 x 2048 12.8 / 11.0 at 32, 13.2 / 13.9 at
     64; 10240 x 2048 16.4 / 9.6 at 4, 16.4 / 13.9 at 32, 19.6 / 21.3 at 128;
