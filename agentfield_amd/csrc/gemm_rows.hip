@@ -67,6 +67,8 @@
 // 25.6 and 57.5 + 5.2 for the first and the last, o + down 63.1).
 #include "mfma_lines.h"
 
+#include <type_traits>
+
 enum RowsEpi { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_ROPE = 3,
                EPI_PARTS = 4 };
 
@@ -491,8 +493,29 @@ __global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
     if (i + 1 < cnt) step(i + 1, wb, xb, wa, xa);
   }
 
+  // the two waves of a product swap sums: each finishes two of its tiles
+  __syncthreads();
+  f32x4* give = reinterpret_cast<f32x4*>(lds) + (wid * 2 * MW) * 64 + lane;
+  const f32x4* take = reinterpret_cast<const f32x4*>(lds) +
+                      ((wid ^ (NW / 2)) * 2 * MW) * 64 + lane;
   f32x4 sum[2][MW];
-  swap_sums<MW>(lds, wid, wid ^ (NW / 2), kh, acc, sum);
+  auto swap = [&](auto upper) {
+    constexpr int U = decltype(upper)::value;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int m = 0; m < MW; ++m) {
+        give[(t * MW + m) * 64] = acc[2 - 2 * U + t][m];
+        sum[t][m] = acc[2 * U + t][m];
+      }
+  };
+  if (kh == 0) swap(std::integral_constant<int, 0>{});
+  else swap(std::integral_constant<int, 1>{});
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int m = 0; m < MW; ++m) sum[t][m] += take[(t * MW + m) * 64];
 
   // lane: row n of each group, columns (lane >> 4) * 4 .. + 4 of each tile
   const int tile = blockIdx.x * NT + w0 + kh * 2;
@@ -505,7 +528,16 @@ __global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
       for (int t = 0; t < 2; ++t) sum[t][m] *= f;
     }
     if (EPI == EPI_SWIGLU) {
-      const u16x4 o = swiglu_tiles(sum[0][m], sum[1][m]);
+      // gate rows lie in the lower lanes and up rows in the upper ones: the lower
+      // lanes get both of the first tile, the upper ones both of the second
+      u16x4 o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const auto gu = __builtin_amdgcn_permlane32_swap(
+            __float_as_uint(sum[0][m][r]), __float_as_uint(sum[1][m][r]), false, false);
+        const float v = __uint_as_float(gu[0]), u = __uint_as_float(gu[1]);
+        o[r] = f2bf(v / (1.f + __expf(-v)) * u);
+      }
       if (row < a.M)
         *reinterpret_cast<row_u16x4*>(a.out + (size_t)row * (a.N >> 1) +
                                   (tile + (lane >> 5)) * 8 + (lane >> 4 & 1) * 4) = o;

@@ -3,8 +3,6 @@
 #pragma once
 #include "common.h"
 
-#include <type_traits>
-
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8r;
 typedef __attribute__((address_space(3))) char lds_b;
 typedef __attribute__((address_space(3))) s16x8 lds_v8;
@@ -51,46 +49,4 @@ __device__ __forceinline__ void meet(int n) {
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-}
-
-// The two waves of a product, `peer` and wid, swap sums through LDS: each finishes two of
-// its four tiles, the upper wave the last two.
-template <int MW>
-__device__ __forceinline__ void swap_sums(char* lds, int wid, int peer, int upper,
-                                          const f32x4 (&acc)[4][MW], f32x4 (&sum)[2][MW]) {
-  const int lane = threadIdx.x & 63;
-  __syncthreads();
-  f32x4* give = reinterpret_cast<f32x4*>(lds) + wid * 2 * MW * 64 + lane;
-  const f32x4* take = reinterpret_cast<const f32x4*>(lds) + peer * 2 * MW * 64 + lane;
-  auto swap = [&](auto up) {
-    constexpr int U = decltype(up)::value;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int m = 0; m < MW; ++m) {
-        give[(t * MW + m) * 64] = acc[2 - 2 * U + t][m];
-        sum[t][m] = acc[2 * U + t][m];
-      }
-  };
-  if (upper == 0) swap(std::integral_constant<int, 0>{});
-  else swap(std::integral_constant<int, 1>{});
-  __syncthreads();
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int m = 0; m < MW; ++m) sum[t][m] += take[(t * MW + m) * 64];
-}
-
-// SwiGLU of two tiles whose gate rows lie in the lower lanes and up rows in the upper
-// ones: the lower lanes get both of the first tile, the upper ones both of the second.
-__device__ __forceinline__ u16x4 swiglu_tiles(f32x4 first, f32x4 second) {
-  u16x4 o;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const auto gu = __builtin_amdgcn_permlane32_swap(
-        __float_as_uint(first[j]), __float_as_uint(second[j]), false, false);
-    const float g = __uint_as_float(gu[0]), u = __uint_as_float(gu[1]);
-    o[j] = f2bf(g / (1.f + __expf(-g)) * u);
-  }
-  return o;
 }

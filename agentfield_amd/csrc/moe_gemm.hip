@@ -24,6 +24,8 @@
 // 429 us, 200 577 -> 474, 600 1119 -> 639.
 #include "mfma_lines.h"
 
+#include <type_traits>
+
 enum MoeEpi { MOE_PLAIN = 0, MOE_SWIGLU = 2 };
 
 #define MG_MT 18                       // 16-row groups of X per block
@@ -140,8 +142,28 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, char* lds, int e,
     }
   }
 
+  // the two waves of a product swap sums: each finishes two of its tiles
+  __syncthreads();
+  f32x4* give = reinterpret_cast<f32x4*>(lds) + wid * 2 * MW * 64 + lane;
+  const f32x4* take = reinterpret_cast<const f32x4*>(lds) + (wid ^ 4) * 2 * MW * 64 + lane;
   f32x4 sum[2][MW];
-  swap_sums<MW>(lds, wid, wid ^ 4, kh, acc, sum);
+  auto swap = [&](auto upper) {
+    constexpr int U = decltype(upper)::value;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int m = 0; m < MW; ++m) {
+        give[(t * MW + m) * 64] = acc[2 - 2 * U + t][m];
+        sum[t][m] = acc[2 * U + t][m];
+      }
+  };
+  if (kh == 0) swap(std::integral_constant<int, 0>{});
+  else swap(std::integral_constant<int, 1>{});
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int m = 0; m < MW; ++m) sum[t][m] += take[(t * MW + m) * 64];
 
   // lane: row n of each group, columns 4 q .. + 4 of each tile
   const int tile = nb * MG_NT + w0 + kh * 2;
@@ -150,7 +172,16 @@ __device__ __forceinline__ void moe_tile(const MoeGemmArgs& a, char* lds, int e,
     const int r = (m0 + m) * 16 + n;
     u16* o = a.out + (size_t)(pos0 + r) * (EPI == MOE_SWIGLU ? a.N >> 1 : a.N);
     if (EPI == MOE_SWIGLU) {
-      const u16x4 v = swiglu_tiles(sum[0][m], sum[1][m]);
+      // gate rows lie in the lower lanes and up rows in the upper ones: the lower
+      // lanes get both of the first tile, the upper ones both of the second
+      u16x4 v;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const auto gu = __builtin_amdgcn_permlane32_swap(
+            __float_as_uint(sum[0][m][j]), __float_as_uint(sum[1][m][j]), false, false);
+        const float g = __uint_as_float(gu[0]), u = __uint_as_float(gu[1]);
+        v[j] = f2bf(g / (1.f + __expf(-g)) * u);
+      }
       const int mine = tile + (lane >> 5);
       if (r < rows && mine <= last)
         *reinterpret_cast<u16x4*>(o + mine * 8 + (q & 1) * 4) = v;
