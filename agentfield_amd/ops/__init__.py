@@ -670,7 +670,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, silu_fuse: bool = False,
             and not watched(x, w)
             and (out is None or _wide_out_ok(out, x, M, N))
             and _wide_ok(x, w, 128)):
-        return launch_wide_split(x, w, out)
+        try:
+            return launch_wide_split(x, w, out)
+        except torch.OutOfMemoryError:
+            pass              # the library needs no room for parts
     if out is not None:
         return torch.mm(x, w.t(), out=out)
     y = x @ w.t()

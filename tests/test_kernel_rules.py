@@ -333,3 +333,15 @@ def test_wide_products_that_stay_with_torch(monkeypatch, index, cast, own, M, N,
     assert ops.linear(x, w, silu_fuse=glu) == want
     if not glu and K == 4096:
         assert seqmix.matmul(x, w) == want
+
+
+def test_wide_split_without_room_for_its_parts(monkeypatch):
+    """Where the shares' sums find no memory the product is torch's, which needs none."""
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(ops, "watched", lambda *t, **kw: False)
+
+    def full(*a, **kw):
+        raise torch.OutOfMemoryError("full")
+    monkeypatch.setattr(ops, "launch_wide_split", full)
+    x, w = (Operand(**vars(mat(n, 14336))) for n in (300, 4096))
+    assert ops.linear(x, w) == "torch"
