@@ -31,7 +31,8 @@
 //   The fp32 parts meet in the kernel that does the next step.  Bound by the parts
 //   (16.8 MB at 128 rows, written at ~2.5 TB/s after the stream has ended: 7 of the 15
 //   us of 4096 x 4096) and by starts, not by its loop: the loop below was no faster.
-//   Unsplit, it also serves plain products of 97..128 rows in blocks of 128 columns.
+//   Unsplit, it also serves plain products of 97..128 rows without a norm, in blocks of
+//   128 columns.
 // gemm_tile_kernel, whole K (SwiGLU, plain): at 128 rows the loop of the kernel above
 //   takes 0.47 us per piece without any load, nearly what the memory needs for the
 //   128 weight rows of a piece (0.57), and the two did not overlap.  So half of the
@@ -281,7 +282,7 @@ __device__ __forceinline__ void wait_loads_and_meet() {
 
 // Split K: MT 16-row groups of X (even), ring of STAGES pieces of K = 64, the sums to
 // the parts (EPI_PARTS); unsplit, EPI_PLAIN.  Grid (N / (16 NW), splits).
-template <int MT, int NW, int WT, int STAGES, int EPI, int NORM, int AUX>
+template <int MT, int NW, int WT, int STAGES, int EPI, int AUX>
 __global__ void __launch_bounds__(64 * NW) gemm_parts_kernel(RowsArgs a) {
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -358,14 +359,6 @@ __global__ void __launch_bounds__(64 * NW) gemm_parts_kernel(RowsArgs a) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = (m0 + m) * 16 + (lane >> 4) * 4 + r;
-      float rstd = 1.f;
-      if (NORM == 1) {
-        const float* sp = a.ss + (size_t)min(row, a.M - 1) * 8;
-        float s = 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) s += sp[j];
-        rstd = rsqrtf(s * (1.f / (float)a.K) + a.eps);
-      }
 #pragma unroll
       for (int t = 0; t < WT; ++t) {
         const int c = (blockIdx.x * NW + w0 + t) * 16 + n;
@@ -373,7 +366,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_parts_kernel(RowsArgs a) {
         if (EPI == EPI_PARTS)
           a.parts[((size_t)blockIdx.y * a.M + row) * a.N + c] = acc[t][m][r];
         else
-          a.out[(size_t)row * a.N + c] = f2bf(NORM == 1 ? acc[t][m][r] * rstd : acc[t][m][r]);
+          a.out[(size_t)row * a.N + c] = f2bf(acc[t][m][r]);
       }
     }
 }
@@ -666,9 +659,9 @@ static void launch_rows(const RowsArgs& a, hipStream_t st) {
 // 4096, 256 or 128 blocks, 25.3 / 29.6, 34.1 / 43.2).  Up to 64 rows, more than one of them
 // to a CU, the rings are short enough that two have room (57344 x 8192, 17 rows: 156 us in
 // rings of 5, 149 of 3; 128256 x 8192 350, 323), otherwise longer (22016 x 4096 34.6 in 3,
-// 31.5 in 5).  Plain products of 97..128 rows keep the loop of the split ones: 32000 x 2048
-// 28.7 us, 27.2 there; 65536 x 2048 61.4, 58.5; 24576 x 4096 46.4, 45.2; with SwiGLU 47.3 at
-// 28672 x 4096 there and 46.4 here.  Small weights are here and gone: 4096 x 1024 at 32 rows
+// 31.5 in 5).  Plain products of 97..128 rows without a norm keep the loop of the split
+// ones: 32000 x 2048 28.7 us, 27.2 there; 65536 x 2048 61.4, 58.5; 24576 x 4096 46.4, 45.2;
+// but 128256 x 4096 with a norm 211, 215 there, 28672 x 4096 with SwiGLU 46.4, 48.2.  Small weights are here and gone: 4096 x 1024 at 32 rows
 // 7.3 us in a ring of 5, 6.9 of 3.
 template <int EPI, int NORM, int AUX>
 static void launch_tile_as(const RowsArgs& a, hipStream_t st) {
@@ -684,8 +677,8 @@ static void launch_tile_as(const RowsArgs& a, hipStream_t st) {
       gemm_tile_kernel<4, 8, 8, 3, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
     else if (a.M <= 96)
       gemm_tile_kernel<6, 8, 8, 4, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
-    else if constexpr (EPI == EPI_PLAIN)
-      gemm_parts_kernel<8, 8, 4, 3, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
+    else if constexpr (EPI == EPI_PLAIN && NORM == 0)
+      gemm_parts_kernel<8, 8, 4, 3, EPI, AUX><<<g, 512, 0, st>>>(a);
     else
       gemm_tile_kernel<8, 8, 8, 4, EPI, NORM, AUX><<<g, 512, 0, st>>>(a);
   } else {
@@ -720,15 +713,15 @@ static void launch_parts_as(const RowsArgs& a, int splits, hipStream_t st) {
   const bool wide = a.N % 128 == 0 && a.N / 128 * splits >= 192 &&
                     a.K / 64 >= 12 * splits;
   if (a.M <= 64 && wide && (a.M > 32 || splits == 1))
-    gemm_parts_kernel<4, 8, 4, 3, EPI_PARTS, 0, AUX><<<g128, 512, 0, st>>>(a);
+    gemm_parts_kernel<4, 8, 4, 3, EPI_PARTS, AUX><<<g128, 512, 0, st>>>(a);
   else if (a.M <= 32)
-    gemm_parts_kernel<2, 4, 1, 4, EPI_PARTS, 0, AUX><<<g64, 256, 0, st>>>(a);
+    gemm_parts_kernel<2, 4, 1, 4, EPI_PARTS, AUX><<<g64, 256, 0, st>>>(a);
   else if (a.M <= 64)
-    gemm_parts_kernel<4, 4, 2, 4, EPI_PARTS, 0, AUX><<<g64, 256, 0, st>>>(a);
+    gemm_parts_kernel<4, 4, 2, 4, EPI_PARTS, AUX><<<g64, 256, 0, st>>>(a);
   else if (a.N % 128 == 0)
-    gemm_parts_kernel<8, 8, 4, 3, EPI_PARTS, 0, AUX><<<g128, 512, 0, st>>>(a);
+    gemm_parts_kernel<8, 8, 4, 3, EPI_PARTS, AUX><<<g128, 512, 0, st>>>(a);
   else
-    gemm_parts_kernel<8, 4, 2, 3, EPI_PARTS, 0, AUX><<<g64, 256, 0, st>>>(a);
+    gemm_parts_kernel<8, 4, 2, 3, EPI_PARTS, AUX><<<g64, 256, 0, st>>>(a);
 }
 
 static void launch_parts(const RowsArgs& a, int splits, hipStream_t st) {
