@@ -299,8 +299,10 @@ class MoEMLP(nn.Module):
     def _forward_sorted(self, x):
         weights, row, pos, offs = ops.launch_moe_route(x, self.router,
                                                        self.top_k)
+        # (a capture cannot wait for the bounds)
         if (ops.moe_gemm_ok(x, self.router, self.gate_up, self.down)
-                and ops.moe_gemm_pays(row.numel(), *self.down.shape)):
+                and (ops.moe_gemm_pays(row.numel(), *self.down.shape)
+                     or torch.cuda.is_current_stream_capturing())):
             act = ops.launch_experts(x, self.gate_up, offs, row.numel(), row,
                                      swiglu=True)
             ys = ops.launch_experts(act, self.down, offs, row.numel())
