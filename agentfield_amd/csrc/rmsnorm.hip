@@ -5,8 +5,11 @@
 //
 // Replaces the torch composition (add + pow + mean + rsqrt + mul + mul) with
 // a single HBM-bound pass: one read of x (+res +w), one write of out (+res).
-// Vectorized 8x bf16 (16 B/lane) per guide Guideline 13; row kept in
-// registers between the sum-of-squares pass and the scale pass.
+// Vectorized 8x bf16 (16 B/lane); row kept in registers between the sum-of-squares
+// pass and the scale pass.  Many rows are bound by memory (10284 x 4096 with a residual
+// 61 us, 5.4 TB/s), few by one row's latency: a block per row there too, a wave per row
+// that walks it twice is slower from 1024 columns on (with a residual, wave / block in
+// us: 1 x 2048 4.5 / 2.3, 150 x 4096 8.2 / 3.7, 256 x 8192 15.5 / 6.2, 64 x 512 2.5 / 2.5).
 #include "common.h"
 
 template <bool HAS_RES>
@@ -70,74 +73,11 @@ __global__ void __launch_bounds__(256) rmsnorm_kernel(
   }
 }
 
-// Low-latency variant for decode-sized T: one wave per row, no LDS/barriers
-// (the 256-thread block version costs ~14 us at T=64 from barrier latency).
-template <bool HAS_RES>
-__global__ void __launch_bounds__(64) rmsnorm_wave_kernel(
-    u16* __restrict__ out, u16* __restrict__ res_out,
-    const u16* __restrict__ x, const u16* __restrict__ res,
-    const u16* __restrict__ w, float eps, int T, int H) {
-  constexpr int VEC = 8;
-  const int row = blockIdx.x;
-  if (row >= T) return;
-  const int per_row = H / VEC;
-  const u16* xrow = x + (size_t)row * H;
-  const u16* rrow = HAS_RES ? res + (size_t)row * H : nullptr;
-  float ss = 0.f;
-  for (int c = threadIdx.x; c < per_row; c += 64) {
-    s16x8 xv = *reinterpret_cast<const s16x8*>(xrow + c * VEC);
-    float f[VEC];
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) f[j] = bf2f((u16)xv[j]);
-    if (HAS_RES) {
-      s16x8 rv = *reinterpret_cast<const s16x8*>(rrow + c * VEC);
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) f[j] += bf2f((u16)rv[j]);
-    }
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) ss += f[j] * f[j];
-  }
-  const float rstd = rsqrtf(wave_sum_f32(ss) / (float)H + eps);
-  // second pass re-reads from L2 (rows are hot at decode sizes); avoids a
-  // runtime-indexed register cache which would spill to scratch (rule #20)
-  for (int c = threadIdx.x; c < per_row; c += 64) {
-    s16x8 xv = *reinterpret_cast<const s16x8*>(xrow + c * VEC);
-    float f[VEC];
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) f[j] = bf2f((u16)xv[j]);
-    if (HAS_RES) {
-      s16x8 rv = *reinterpret_cast<const s16x8*>(rrow + c * VEC);
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) f[j] += bf2f((u16)rv[j]);
-    }
-    s16x8 wv = *reinterpret_cast<const s16x8*>(w + c * VEC);
-    s16x8 ov, hv;
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) {
-      if (HAS_RES) hv[j] = (short)f2bf(f[j]);
-      ov[j] = (short)f2bf(f[j] * rstd * bf2f((u16)wv[j]));
-    }
-    *reinterpret_cast<s16x8*>(out + (size_t)row * H + c * VEC) = ov;
-    if (HAS_RES)
-      *reinterpret_cast<s16x8*>(res_out + (size_t)row * H + c * VEC) = hv;
-  }
-}
-
 AF_EXPORT int af_rmsnorm(void* out, void* res_out, const void* x, const void* res,
                          const void* w, float eps, int T, int H, void* stream) {
   if (H % 8 || H > 16384) return 9001;
   if (T == 0) return 0;
   hipStream_t st = (hipStream_t)stream;
-  if (T <= 256 && H <= 16384) {
-    if (res)
-      rmsnorm_wave_kernel<true><<<T, 64, 0, st>>>(
-          (u16*)out, (u16*)res_out, (const u16*)x, (const u16*)res,
-          (const u16*)w, eps, T, H);
-    else
-      rmsnorm_wave_kernel<false><<<T, 64, 0, st>>>(
-          (u16*)out, nullptr, (const u16*)x, nullptr, (const u16*)w, eps, T, H);
-    return af_last_err();
-  }
   int blocks = T < 16384 ? T : 16384;  // one row per block fills 256 CUs
   if (res)
     rmsnorm_kernel<true><<<blocks, 256, 0, st>>>(

@@ -75,6 +75,21 @@ def test_rmsnorm_fused_residual():
     assert close(new_res, res_ref)
 
 
+@pytest.mark.parametrize("T", [1, 3, 256, 257])
+@pytest.mark.parametrize("H", [8, 256, 520, 2048, 2056, 8192, 16384])
+def test_rmsnorm_row_lengths(T, H):
+    """Rows shorter than a wave, with a ragged last round of a block and the longest:
+    fp32 inside, so a bf16 rounding of the row and one of the result (2^-8 of values
+    below 8)."""
+    x, w, res = (rnd(*s, seed=i) for i, s in enumerate([(T, H), (H,), (T, H)]))
+    assert close(ops.rmsnorm(x, w, 1e-5), ref.rmsnorm(x.cpu(), w.cpu(), 1e-5),
+                 atol=2 ** -5, rtol=2 ** -7)
+    out, new = ops.rmsnorm(x, w, 1e-5, residual=res.clone())
+    want, want_new = ref.rmsnorm(x.cpu(), w.cpu(), 1e-5, residual=res.cpu().clone())
+    assert torch.equal(new.cpu(), want_new)
+    assert close(out, want, atol=2 ** -5, rtol=2 ** -7)
+
+
 def test_rope_cache_fused_strided():
     """Fused RoPE+cache on strided rows (views of a fused QKV buffer)."""
     T, Hq, Hk, D, page, npages = 9, 4, 2, 128, 4, 8
