@@ -64,6 +64,7 @@
 #define AP_KV 64          // tokens per shared tile
 #define AP_FEW 32         // tokens per wave-private tile
 #define AP_ROWB 256       // bytes of a K or V row
+#define AP_SPLITS 8       // shares of the keys at most
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
@@ -549,18 +550,27 @@ __global__ void __launch_bounds__(256) attn_prefill_merge_kernel(
   const size_t from = (size_t)blockIdx.x * nsplit * 32;
   for (int i = threadIdx.x; i < nrows * G * (AP_D / 4); i += 256) {
     const int cc = i / (AP_D / 4), d = (i % (AP_D / 4)) * 4;
+    // the splits' results are asked for together (those behind the last repeat it)
+    f32x2 ml[AP_SPLITS];
+    f32x4 part[AP_SPLITS];
+#pragma unroll
+    for (int s = 0; s < AP_SPLITS; ++s) {
+      const size_t at = from + min(s, nsplit - 1) * 32 + cc;
+      ml[s] = *reinterpret_cast<const f32x2*>(pml + at * 2);
+      part[s] = *reinterpret_cast<const f32x4*>(po + at * AP_D + d);
+    }
     float M = AF_NEG_INF;
-    for (int s = 0; s < nsplit; ++s) M = fmaxf(M, pml[(from + s * 32 + cc) * 2]);
+#pragma unroll
+    for (int s = 0; s < AP_SPLITS; ++s) M = fmaxf(M, ml[s][0]);
     float L = 0.f;
     f32x4 o = {0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < nsplit; ++s) {
-      const float m = pml[(from + s * 32 + cc) * 2];
-      const float f = (m <= AF_NEG_INF) ? 0.f : __builtin_amdgcn_exp2f((m - M) * sc);
-      L += pml[(from + s * 32 + cc) * 2 + 1] * f;
-      const f32x4 v =
-          *reinterpret_cast<const f32x4*>(po + (from + s * 32 + cc) * AP_D + d);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) o[j] += v[j] * f;
+    for (int s = 0; s < AP_SPLITS; ++s) {
+      if (s >= nsplit) break;
+      const float f = (ml[s][0] <= AF_NEG_INF) ? 0.f : __builtin_amdgcn_exp2f((ml[s][0] - M) * sc);
+      L += ml[s][1] * f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] += part[s][j] * f;
     }
     const float inv = (L > 0.f) ? 1.f / L : 0.f;
     s16x4 v;
@@ -587,7 +597,7 @@ AF_EXPORT int af_attn_prefill(void* out, void* po, void* pml, const void* q,
                               void* stream) {
   if (D != AP_D) return 9002;
   const int G = Hq / Hk;
-  if (G * Hk != Hq) return 9003;
+  if (G * Hk != Hq || (few > 0 && (nsplit < 1 || nsplit > AP_SPLITS))) return 9003;
   hipStream_t st = (hipStream_t)stream;
   const bool pow2 = (page_size & (page_size - 1)) == 0;
   const PrefillArgs a = {(u16*)out, (const u16*)q, (const u16*)kc, (const u16*)vc,

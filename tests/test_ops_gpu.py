@@ -624,6 +624,28 @@ def test_attn_decode_tile_edges(page, G, Hk, nsplit, window):
     assert close(got, want, atol=2 ** -7, rtol=2 ** -8)
 
 
+@pytest.mark.parametrize("nsplit", [2, 4, 5, 8, 9, 16, 17, 35])
+def test_attn_decode_merges_splits(nsplit):
+    """Every width of the merge, and more splits than its widest takes at once; splits
+    without tokens, whose partial outputs nobody writes, are NaN in the scratch.
+    Tolerance: bf16 rounding of outputs below 4 (2^-9 * 4)."""
+    Hk, G, D, page = 2, 4, 128, 16
+    lens = [1, 64, 65, 400, 2300]
+    B, maxp = len(lens), 2300 // page + 1
+    torch.manual_seed(nsplit)
+    bt = (torch.randperm(B * maxp) + 1).view(B, maxp).to(torch.int32)
+    kc, vc = (torch.randn(B * maxp + 1, Hk, page, D).bfloat16() for _ in range(2))
+    q = torch.randn(B, Hk * G * D).bfloat16()
+    L = torch.tensor(lens, dtype=torch.int32)
+    scratch = (torch.full((B, Hk, nsplit, G, D), torch.nan, device=DEV),
+               torch.full((B, Hk, nsplit, G, 2), torch.nan, device=DEV))
+    got = ops.attn_decode(q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV), L.to(DEV),
+                          nsplit=nsplit, scratch=scratch).cpu()
+    want = ref.attn_decode(q.unflatten(-1, (Hk * G, D)), kc, vc, bt, L,
+                           1.0 / math.sqrt(D)).flatten(1)
+    assert close(got, want, atol=2 ** -7, rtol=2 ** -8)
+
+
 @pytest.mark.parametrize("Hk,nsplit", [(3, 1), (4, 1), (4, 2), (8, 1), (8, 3), (11, 2)])
 def test_attn_decode_orders_of_the_grid(Hk, nsplit):
     """Heads first and sequences first: every head of every sequence is its own, by
