@@ -12,6 +12,11 @@
 #include "common.h"
 
 #define SMP_SPLITS 16
+// rows from here on draw behind a bar (Draw): with fewer values a lane has not enough of
+// them for it to pay (all rows unrestricted, a pass of 256 threads in 16 splits: 64 x 32003
+// 18.3 us with the bar, 16.8 without; 64 x 128256 26.3 and 27.9, 128 x 128256 without top-k
+// or top-p 19.5 and 23.5)
+#define SMP_BAR 65536
 
 __device__ __forceinline__ float u32_to_unit(uint32_t x) {
   return (x >> 8) * (1.f / 16777216.f) + (0.5f / 16777216.f);
@@ -70,12 +75,76 @@ __device__ __forceinline__ void each_logit(const u16* __restrict__ row, int V,
   }
 }
 
+// The same with all lanes of a wave in f(value, index, there) together, those without a
+// value of their own with there = false.  Eight values are passed over where the largest of
+// none of the lanes' is `want`ed.
+template <class Want, class F>
+__device__ __forceinline__ void each_logit_in_step(const u16* __restrict__ row, int V,
+                                                   int split, int nsplit, Want want, F f) {
+  const int head =
+      min(V, (int)(((16u - ((uint32_t)(uintptr_t)row & 15u)) & 15u) >> 1));
+  const int nvec = (V - head) >> 3;
+  const int per = (nvec + nsplit - 1) / nsplit;
+  const int i0 = split * per, i1 = min(nvec, i0 + per);
+  const u16* body = row + head;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63);
+  for (int base = i0 + wave; base < i1; base += 4 * 256) {
+    const int i = base + (int)(threadIdx.x & 63);
+    s16x8 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      v[u] = *reinterpret_cast<const s16x8*>(
+          body + (size_t)min(i + u * 256, i1 - 1) * 8);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (base + u * 256 >= i1) break;
+      const bool there = i + u * 256 < i1;
+      float m = AF_NEG_INF;                  // a median with infinity is the larger one
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        m = __builtin_amdgcn_fmed3f(m, bf2f((u16)v[u][j]), __builtin_inff());
+      if (!__any(want(m))) continue;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        f(bf2f((u16)v[u][j]), head + (i + u * 256) * 8 + j, there);
+    }
+  }
+  if (split == 0 && wave == 0) {             // V >= 1
+    const int t = threadIdx.x, tail = head + nvec * 8;
+    if (head > 0) f(bf2f(row[min(t, V - 1)]), t, t < head);
+    if (tail < V) f(bf2f(row[min(tail + t, V - 1)]), tail + t, tail + t < V);
+  }
+}
+
 // Larger value wins, equal values go to the smaller index: the order in which
 // threads and splits see a row does not matter.
 __device__ __forceinline__ void take_best(float ov, int oi, float& best,
                                           int& bidx) {
   if (ov > best || (ov == best && oi < bidx)) { best = ov; bidx = oi; }
 }
+
+// The best of values with Gumbel noise, where a lane has many.  The noise is two
+// logarithms, 22 instructions, that nearly no value needs: with w + 1/2 = 2^24 (1 - u), w a
+// whole number, -log u >= 1 - u, so a value x can only pass the score `top` of another where
+// w < 2^24 exp(x - top).  Eight steps of w (for the rounding of u and of the first
+// logarithm, and the u that rounds to 1) and 2^0.002 make up for rounding.
+struct Draw {
+  float best = AF_NEG_INF, top = -__builtin_inff();   // this lane's, the wave's
+  int bidx = 0;
+  uint32_t seed;
+  int b;
+
+  // all lanes of a wave; x counts where `there`
+  __device__ __forceinline__ void take(float x, int v, bool there) {
+    const uint32_t h = hash3(seed, (uint32_t)b, (uint32_t)v);
+    const float lim = __builtin_amdgcn_exp2f(fmaf(x - top, 1.44269504f, 24.002f)) + 8.f;
+    there = there && !((float)(~h >> 8) >= lim);
+    if (!__any(there)) return;
+    x += gumbel_of(u32_to_unit(h));
+    if (there && (x > best || (x == best && v < bidx))) { best = x; bidx = v; }
+    top = wave_max_f32(best);
+  }
+};
 
 __device__ __forceinline__ void store_best(float best, int bidx,
                                            float* __restrict__ pv,
@@ -99,6 +168,7 @@ __device__ __forceinline__ void store_best(float best, int bidx,
   }
 }
 
+template <bool BAR>
 __global__ void __launch_bounds__(256) sample_partial_kernel(
     float* __restrict__ pv, i32* __restrict__ pi, const u16* __restrict__ logits,
     const float* __restrict__ temp, const uint32_t* __restrict__ step,
@@ -107,6 +177,16 @@ __global__ void __launch_bounds__(256) sample_partial_kernel(
   const float t = temp[b];
   const float invt = (t > 0.f) ? 1.f / t : 0.f;
   const uint32_t st = *step;
+  if (BAR && t > 0.f) {
+    Draw d;
+    d.seed = seed ^ st;
+    d.b = b;
+    each_logit_in_step(logits + (size_t)b * V, V, split, SMP_SPLITS,
+                       [](float) { return true; },
+                       [&](float x, int v, bool there) { d.take(x * invt, v, there); });
+    store_best(d.best, d.bidx, pv, pi, b * SMP_SPLITS + split);
+    return;
+  }
   float best = AF_NEG_INF;
   int bidx = 0;
   each_logit(logits + (size_t)b * V, V, split, SMP_SPLITS, [&](float x, int v) {
@@ -154,8 +234,10 @@ __global__ void __launch_bounds__(64) sample_combine_kernel(
 // for the histogram and 52 us for the maximum at 64 x 128256.  The passes after
 // the first fold the per-split results of the pass before in their prologue, so
 // nothing but the three reads of the row and the draw's last step is launched: 346
-// us -> 28 us.  (The draw's blocks fold all 16 histograms of their row each, 32 KB a
-// block; with the two logarithms per value that is what its 15 us go to.)
+// us -> 27 us; 24 with the bar of Draw, greedy rows without a histogram and the blocks of a
+// CU from different rows.  (A draw to which top-k leaves few values takes 6.8 us, mostly its
+// blocks' folding of all 16 histograms of their row, 32 KB each; one of all values, bound by
+// their hashes, 13.9.)
 #define TKP_BINS 256
 #define TKP_SPAN 20.0f
 
@@ -198,8 +280,9 @@ __global__ void __launch_bounds__(256) tkp_hist_kernel(
     i32* __restrict__ hist_n, float* __restrict__ hist_m,
     const u16* __restrict__ logits, const float* __restrict__ rmax,
     const float* __restrict__ temp, int V) {
-  const int b = blockIdx.x, split = blockIdx.y;
+  const int split = blockIdx.y, b = blockIdx.x;
   const int copy = threadIdx.x & (TKP_COPIES - 1);
+  if (!(temp[b] > 0.f)) return;              // a greedy row takes its largest value
   __shared__ unsigned long long h[TKP_BINS * TKP_COPIES];
 #pragma unroll
   for (int c = 0; c < TKP_COPIES; ++c) h[c * 256 + threadIdx.x] = 0;
@@ -282,29 +365,53 @@ __device__ __forceinline__ float tkp_threshold(
 }
 
 // pass C: Gumbel-argmax over {x/T >= threshold}
+template <bool BAR>
 __global__ void __launch_bounds__(256) tkp_sample_kernel(
     float* __restrict__ pv, i32* __restrict__ pi, const u16* __restrict__ logits,
     const float* __restrict__ temp, const float* __restrict__ rmax,
     const i32* __restrict__ hist_n, const float* __restrict__ hist_m,
     const i32* __restrict__ topk, const float* __restrict__ topp,
     const uint32_t* __restrict__ step, uint32_t seed, int V) {
-  const int b = blockIdx.x, split = blockIdx.y;
+  // a CU's blocks are of different rows, long and short (as blockIdx.x the four of a CU
+  // were of one row: 64 x 128256 25.4 us, 24.2)
+  const int split = blockIdx.y, b = (blockIdx.x + 8 * (split >> 2)) % gridDim.x;
+  const u16* row = logits + (size_t)b * V;
   const float t = temp[b];
-  const float invt = (t > 0.f) ? 1.f / t : 1.f;
+  if (!(t > 0.f)) {
+    float best = AF_NEG_INF;
+    int bidx = 0;
+    each_logit(row, V, split, SMP_SPLITS, [&](float x, int v) {
+      if (x > best || (x == best && v < bidx)) { best = x; bidx = v; }
+    });
+    store_best(best, bidx, pv, pi, b * SMP_SPLITS + split);
+    return;
+  }
+  const float invt = 1.f / t;
   const int k = (topk[b] > 0) ? topk[b] : V;
   const float p = (topp[b] > 0.f && topp[b] < 1.f) ? topp[b] : 1.f;
   const float th =
       tkp_threshold(hist_n, hist_m, row_max_of(rmax, b) * invt, k, p, b);
   const uint32_t st = *step;
+  if (BAR) {
+    Draw d;
+    d.seed = seed ^ st;
+    d.b = b;
+    each_logit_in_step(row, V, split, SMP_SPLITS,
+                       [&](float l) { return !(l * invt < th); },
+                       [&](float l, int v, bool there) {
+      const float x = l * invt;
+      there = there && !(x < th);
+      if (__any(there)) d.take(x, v, there);
+    });
+    store_best(d.best, d.bidx, pv, pi, b * SMP_SPLITS + split);
+    return;
+  }
   float best = AF_NEG_INF;
   int bidx = 0;
-  each_logit(logits + (size_t)b * V, V, split, SMP_SPLITS, [&](float l, int v) {
+  each_logit(row, V, split, SMP_SPLITS, [&](float l, int v) {
     float x = l * invt;
     if (x < th) return;
-    if (t > 0.f) {
-      const float u = u32_to_unit(hash3(seed ^ st, (uint32_t)b, (uint32_t)v));
-      x += gumbel_of(u);
-    }
+    x += gumbel_of(u32_to_unit(hash3(seed ^ st, (uint32_t)b, (uint32_t)v)));
     if (x > best || (x == best && v < bidx)) { best = x; bidx = v; }
   });
   store_best(best, bidx, pv, pi, b * SMP_SPLITS + split);
@@ -324,7 +431,8 @@ AF_EXPORT int af_sample_topkp(void* out, void* pv, void* pi, void* rmax,
   tkp_hist_kernel<<<g, 256, 0, st>>>((i32*)hist_n, (float*)hist_m,
                                      (const u16*)logits, (const float*)rmax,
                                      (const float*)temp, V);
-  tkp_sample_kernel<<<g, 256, 0, st>>>(
+  const auto draw = V >= SMP_BAR ? tkp_sample_kernel<true> : tkp_sample_kernel<false>;
+  draw<<<g, 256, 0, st>>>(
       (float*)pv, (i32*)pi, (const u16*)logits, (const float*)temp,
       (const float*)rmax, (const i32*)hist_n, (const float*)hist_m,
       (const i32*)topk, (const float*)topp, (const uint32_t*)step, seed, V);
@@ -339,7 +447,8 @@ AF_EXPORT int af_sample(void* out, void* pv, void* pi, const void* logits,
   if (B == 0) return 0;
   hipStream_t st = (hipStream_t)stream;
   dim3 g1(B, SMP_SPLITS);
-  sample_partial_kernel<<<g1, 256, 0, st>>>(
+  const auto draw = V >= SMP_BAR ? sample_partial_kernel<true> : sample_partial_kernel<false>;
+  draw<<<g1, 256, 0, st>>>(
       (float*)pv, (i32*)pi, (const u16*)logits, (const float*)temp,
       (const uint32_t*)step, seed, V);
   sample_combine_kernel<<<B, 64, 0, st>>>((i32*)out, (const float*)pv,

@@ -527,6 +527,62 @@ def test_sample_topk_topp():
             assert lf[b, int(t[b])] >= mx[b] - gran - 1e-3
 
 
+def _noise(seed, step, B, V):
+    """The sampler's Gumbel noise [B, V]: its hash in whole numbers, its float steps."""
+    M = 0xFFFFFFFF
+    b, v = (torch.arange(n, device=DEV) for n in (B, V))
+    h = ((seed ^ step) * 0x9E3779B1 & M) + (b * 0x85EBCA77 & M)[:, None] \
+        + (v * 0xC2B2AE3D & M)[None] + 0x27220A95 & M
+    for shift, mul in ((15, 0x2C1B3C6D), (12, 0x297A2D39)):
+        h = (h ^ h >> shift)
+        h = ((h & 0xFFFF) * mul + ((h >> 16) * mul << 16 & M)) & M
+    h = h ^ h >> 15
+    u = (h >> 8).float() * 2.0 ** -24 + 2.0 ** -25
+    return -torch.log(torch.clamp(-torch.log(u), min=1e-30))
+
+
+@pytest.mark.parametrize("V", [65536, 65541, 131073])
+@pytest.mark.parametrize("cut", [False, True])
+def test_sample_behind_a_bar(V, cut):
+    """Wide rows skip the noise of values that cannot win: the token drawn is the best of
+    all values with their noise (two logarithms of 32 bits apart), at temperatures from
+    sharp to flat, with masked, infinite and missing values, greedy rows among them; with
+    top-k / top-p its best of those that can be drawn for sure may not be better."""
+    B = 24
+    st = ops.SamplerState(B, DEV, seed=77)
+    st.step.fill_(5)
+    x = rnd(B, V, seed=V, scale=3.0)
+    x[1, : V // 2] = -1e30
+    x[2] = -1e30
+    x[2, V - 1] = 0.5
+    x[3, 100] = math.inf
+    x[4, ::3] = -math.inf
+    x[5, 7] = math.nan
+    x[6] = 1.0
+    t = torch.tensor([1.0, 0.7, 1.0, 1.0, 1.5, 0.9, 1.0, 0.0] * 3, device=DEV)
+    t[8:16] *= 0.05
+    t[16:] *= 10
+    kw = {}
+    if cut:
+        kw = dict(topk=torch.tensor([0, 40, 1] * 8, device=DEV, dtype=torch.int32),
+                  topp=torch.tensor([1.0, 1.0, 1.0, 0.9] * 6, device=DEV))
+    got = ops.sample(x, t, st, **kw).long()
+    noise = _noise(77, 5, B, V) * (t > 0)[:, None]
+    score = x.float() / torch.where(t > 0, t, 1.0)[:, None]
+    sure = torch.zeros_like(score, dtype=torch.bool)     # drawn from whatever the cut
+    sure[torch.arange(B), torch.nan_to_num(score, nan=-math.inf).argmax(1)] = True
+    if not cut:
+        sure[:] = True
+    total = torch.nan_to_num(score + noise, nan=-math.inf, posinf=3e38)
+    best = torch.where(sure, total, -math.inf).amax(1)
+    mine = total.gather(1, got[:, None])[:, 0]
+    # x * (1 / t) against x / t, and two logarithms
+    assert (mine >= best - 1e-4 - 1e-6 * best.abs()).all(), (mine, best)
+    assert torch.equal(got[t == 0], score[t == 0].argmax(1))
+    if cut:
+        assert (got[2::3] == torch.nan_to_num(score, nan=-math.inf).argmax(1)[2::3]).all()
+
+
 def test_engine_topk_sampling_runs():
     from agentfield_amd.engine import LLMEngine, SamplingParams
     from agentfield_amd.models import CONFIGS
