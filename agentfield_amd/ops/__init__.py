@@ -9,6 +9,7 @@ Every op has two paths:
 from __future__ import annotations
 
 import functools
+import itertools
 import math
 
 import torch
@@ -548,6 +549,37 @@ def _wide_out_ok(out: torch.Tensor, x: torch.Tensor, M: int, N: int) -> bool:
     return _whole(out, x, M, N) and _apart(out, x) and out.data_ptr() & 15 == 0
 
 
+@functools.lru_cache(maxsize=4096)
+def _library_behind(M: int, N: int, K: int) -> bool:
+    """Whether the library's plain product, by what it reaches with 256 x 256 tiles, takes
+    1.16 of the wide GEMM's own estimate.  It gives every block the same number of tiles
+    where some 232..256 of them come out even, and then reaches 1.4 PFLOP/s; where only
+    fewer blocks do, or none of 128 or more, its rate falls with them (means of 1738
+    products: none 0.93, 128 0.95, 160 1.08, 192 1.16, 216 1.25 PFLOP/s).  Of 5,460
+    products (25 projections, 256..14000 rows) this names 378 that the rules of _wide_pays
+    leave to the library, library over wide 1.16 in the mean, 0.965 at least: 4096 x 4096
+    at 10284 rows 351 us / 239, 11000 rows 407 / 283, 8256 x 2048 at 7634 rows 242 / 200,
+    6144 x 4096 at 1500 rows 78 / 68.  With a K beyond 5120 or more than six rounds of
+    tiles it is wrong by more (0.91, 0.93)."""
+    tiles = -(-M // 256) * -(-N // 256)
+    if K > 5120 or N > 24576 or not 128 < tiles <= 1536:
+        return False
+    blocks = next((tiles // r for r in range(-(-tiles // 256), tiles // 128 + 1)
+                   if tiles % r == 0), 0)
+    if blocks >= 232:
+        return False
+    for (lo, a), (hi, b) in itertools.pairwise(_LIBRARY_RATE):
+        if lo <= blocks <= hi:
+            rate = a + (b - a) * (blocks - lo) / (hi - lo)
+            break
+    ns = _lib.lib().af_gemm_wide_ns(M, N, K)
+    return 0 < 1.16 * ns < 2e-6 * M * N * K / rate
+
+
+#: blocks of the library that come out even, PFLOP/s
+_LIBRARY_RATE = ((0, .93), (128, .95), (160, 1.08), (192, 1.16), (216, 1.25), (232, 1.38))
+
+
 def _wide_pays(M: int, N: int, K: int, silu_fuse: bool) -> bool:
     """Whether the wide GEMM beats the library's, by the tiles that its 256 blocks
     take.  Times are the library's over the wide GEMM's, weights not in cache.
@@ -574,7 +606,8 @@ def _wide_pays(M: int, N: int, K: int, silu_fuse: bool) -> bool:
       three not from a K of 8192 on (8192 x 8192 at 6587 rows 0.93), none behind six
       (0.91) or more.  Above 12288 columns one or two rounds lose (28672 x 4096 at 1100
       rows 0.95) and 63 is the limit for all (22016 x 4096 at 2560 rows, 92 behind
-      three, 0.86)."""
+      three, 0.86).
+    - K < 2N beyond these limits and below a round: _library_behind."""
     cols = -(-N // 256)
     if silu_fuse:
         tiles = -(-M // 128) * cols
@@ -582,18 +615,19 @@ def _wide_pays(M: int, N: int, K: int, silu_fuse: bool) -> bool:
                 and not (448 < M <= 512 and 336 <= tiles <= 384 and K >= 4096))
     tiles = -(-M // 256) * cols
     rounds, begun = tiles >> 8, tiles & 255
-    if rounds < 1 or begun == 0:
-        return False
     if K >= 2 * N:
-        if rounds == 1 and begun in (64, 128):
+        if rounds < 1 or begun == 0 or rounds == 1 and begun in (64, 128):
             return False
         return begun <= 216 and (N <= 5120 or rounds == 1
                                  or rounds == 2 and begun != 64)
-    if rounds > 5 or rounds < 3 and N > 12288 or rounds == 3 and K >= 8192:
-        return False
-    if N <= 5120 or rounds in (2, 4) and N <= 12288:
-        return begun <= 128
-    return begun < (64 if rounds == 1 or N > 12288 else 96)
+    if rounds >= 1 and begun and not (
+            rounds > 5 or rounds < 3 and N > 12288 or rounds == 3 and K >= 8192):
+        if N <= 5120 or rounds in (2, 4) and N <= 12288:
+            if begun <= 128:
+                return True
+        elif begun < (64 if rounds == 1 or N > 12288 else 96):
+            return True
+    return M >= 256 and _library_behind(M, N, K)
 
 
 def launch_wide(x, w, silu_fuse=False, out=None, groups=0):

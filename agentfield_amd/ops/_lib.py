@@ -71,6 +71,7 @@ def _declare(l: ctypes.CDLL) -> None:
     l.af_gemm_wide.argtypes = [p, p, p, i, i, i, i, i, p]
     l.af_gemm_wide_split.argtypes = [p, p, p, p, i, i, i, i, i, p]
     l.af_gemm_wide_splits.argtypes = [i, i, i]
+    l.af_gemm_wide_ns.argtypes = [i, i, i]
     l.af_gemm_wide_experts.argtypes = [p, p, p, p, p, i, i, i, i, i, i, p]
     l.af_moe_gemm.argtypes = [p, p, p, p, p, i, i, i, i, i, p]
     l.af_sample.argtypes = [p, p, p, p, p, p, u32, i, i, p]
@@ -89,7 +90,7 @@ def _declare(l: ctypes.CDLL) -> None:
                "af_gemm_skinny", "af_rows_linear", "af_rows_qkv",
                "af_moe_route", "af_moe_combine", "af_moe_gemm", "af_gemm_wide",
                "af_gemm_wide_experts", "af_gemm_wide_split",
-               "af_gemm_wide_splits", "af_sample",
+               "af_gemm_wide_splits", "af_gemm_wide_ns", "af_sample",
                "af_sample_topkp", "af_gather_rows", "af_mfma_probe", "af_mfma_mx_probe", "af_lds_stride_probe", "af_mfma_mx32_probe", "af_axpy",
                "af_device_sync"):
         getattr(l, fn).restype = ctypes.c_int

@@ -264,6 +264,19 @@ def test_wide_gemm_leaves_what_the_library_does_better(M, N, K, glu, pays):
 
 
 @pytest.mark.parametrize("M,N,K,pays", [
+    (10284, 4096, 4096, True), (11000, 4096, 4096, True),    # 219, 229 blocks come out even
+    (7634, 8256, 2048, True), (1500, 6144, 4096, True),      # none; below one round
+    (7634, 8192, 2048, False), (7634, 2048, 2048, False),    # 240 do
+    (10284, 6144, 4096, False), (9000, 10240, 2048, False),  # 246, 240
+    (1500, 4096, 4096, False), (2000, 4096, 4096, False),    # up to 128 tiles
+    (2400, 8192, 8192, False), (11157, 12288, 4096, False),  # a long K; many rounds
+    (255, 6144, 4096, False),
+])
+def test_wide_gemm_where_the_library_cannot_divide(M, N, K, pays):
+    assert ops._wide_pays(M, N, K, False) == pays
+
+
+@pytest.mark.parametrize("M,N,K,pays", [
     (1280, 2048, 10240, True), (1281, 2048, 10240, False), (2068, 2048, 10240, False),
     (2048, 2048, 16384, True)])
 def test_wide_gemm_split_of_few_columns(M, N, K, pays):
