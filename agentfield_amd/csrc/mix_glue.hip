@@ -139,8 +139,10 @@ __global__ void __launch_bounds__(256) add_rows_kernel(
   }
 }
 
-// a = norm(x)(1+w1), b = norm(x)(1+w2), s = a + (a_prev - a)*shift.
-template <typename S, int V>
+// a = norm(x)(1+w1), b = norm(x)(1+w2), s = a + (a_prev - a)*shift.  Rows of up to R * 256
+// * V stay in registers, and all that the step behind the sum reads is asked for before it
+// (rows of 2048, six: 4.7 -> 3.9 us; 7636: 50 -> 38).  R = 0: any length.
+template <typename S, int V, int R>
 __global__ void __launch_bounds__(256) dual_norm_shift_kernel(
     S* __restrict__ a_out, S* __restrict__ s_out, S* __restrict__ b_out,
     float* __restrict__ last, const float* __restrict__ x,
@@ -154,60 +156,97 @@ __global__ void __launch_bounds__(256) dual_norm_shift_kernel(
   // overwritten by the same thread.
   __shared__ float red[8];
   const int t = blockIdx.x;
+  const float* xr = x + (size_t)t * W;
+  const float* xp = xr - W;  // previous row, only touched when !first
+  struct Cols { float x[4], w1[4], w2[4], mix[4], before[4]; };
+  Cols at[R > 0 ? R : 1];
+  // (no branch between the loads: what is not there reads w1 again)
+  const S* w2r = b_out ? w2 : w1;
+  const S* mixr = shift ? shift : w1;
+  auto load = [&](int i, Cols& c) {
+    ldv<float, V>(xr + i, c.x);
+    ldv<S, V>(w1 + i, c.w1);
+    ldv<S, V>(w2r + i, c.w2);
+    ldv<S, V>(mixr + i, c.mix);
+  };
+  if (R > 0) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      load(min((int)(threadIdx.x + r * 256) * V, W - V), at[r]);
+  }
   const int b = row_seq[t];
   const int r0 = cu[b];
   const bool first = (t == r0);
   const bool is_last = (t == cu[b + 1] - 1);
   const int pos = q_start[b] + (t - r0);
-  const float* xr = x + (size_t)t * W;
-  const float* xp = xr - W;  // previous row, only touched when !first
   const bool need_prev_row = shift && !first;
+  // the row before, or what the state slot holds of it
+  const float* bef = need_prev_row ? xp
+                     : (shift && pos > 0) ? prev + (size_t)sslot[b] * W : nullptr;
   float ss[2] = {0.f, 0.f};
-  for (int i = threadIdx.x * V; i < W; i += 256 * V) {
-    float xv[4], pv4[4];
-    ldv<float, V>(xr + i, xv);
+  auto load_before = [&](int i, Cols& c) {
+    c.before[0] = c.before[1] = c.before[2] = c.before[3] = 0.f;
+    if (bef) ldv<float, V>(bef + i, c.before);
+  };
+  auto add = [&](const Cols& c) {
 #pragma unroll
-    for (int j = 0; j < V; ++j) ss[0] += xv[j] * xv[j];
+    for (int j = 0; j < V; ++j) ss[0] = fmaf(c.x[j], c.x[j], ss[0]);
     if (need_prev_row) {
-      ldv<float, V>(xp + i, pv4);
 #pragma unroll
-      for (int j = 0; j < V; ++j) ss[1] += pv4[j] * pv4[j];
+      for (int j = 0; j < V; ++j) ss[1] = fmaf(c.before[j], c.before[j], ss[1]);
+    }
+  };
+  if (R > 0) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      load_before(min((int)(threadIdx.x + r * 256) * V, W - V), at[r]);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if ((int)(threadIdx.x + r * 256) * V < W) add(at[r]);
+  } else {
+    for (int i = threadIdx.x * V; i < W; i += 256 * V) {
+      ldv<float, V>(xr + i, at[0].x);
+      if (need_prev_row) ldv<float, V>(xp + i, at[0].before);
+      add(at[0]);
     }
   }
   block_sum<2>(ss, red);
   const float r = 1.0f / sqrtf(ss[0] / (float)W + eps);
   const float rp = 1.0f / sqrtf(ss[1] / (float)W + eps);
-  const float* pv = (shift && first && pos > 0)
-                        ? prev + (size_t)sslot[b] * W : nullptr;
-  for (int i = threadIdx.x * V; i < W; i += 256 * V) {
-    float xv[4], g1[4], a[4], o[4], tmp[4];
-    ldv<float, V>(xr + i, xv);
-    ldv<S, V>(w1 + i, g1);
+  auto put = [&](int i, const Cols& c) {
+    float g1[4], a[4], o[4];
 #pragma unroll
-    for (int j = 0; j < V; ++j) { g1[j] += 1.0f; a[j] = xv[j] * r * g1[j]; }
+    for (int j = 0; j < V; ++j) { g1[j] = c.w1[j] + 1.0f; a[j] = c.x[j] * r * g1[j]; }
     stv<S, V>(a_out + (size_t)t * W + i, a);
     if (b_out) {
-      ldv<S, V>(w2 + i, tmp);
 #pragma unroll
-      for (int j = 0; j < V; ++j) o[j] = xv[j] * r * (1.0f + tmp[j]);
+      for (int j = 0; j < V; ++j) o[j] = c.x[j] * r * (1.0f + c.w2[j]);
       stv<S, V>(b_out + (size_t)t * W + i, o);
     }
     if (shift) {
-      float ap[4] = {0.f, 0.f, 0.f, 0.f};
-      if (need_prev_row) {
-        ldv<float, V>(xp + i, tmp);
+      float ap[4];
 #pragma unroll
-        for (int j = 0; j < V; ++j) ap[j] = tmp[j] * rp * g1[j];
-      } else if (pv) {
-        ldv<float, V>(pv + i, ap);
-      }
-      ldv<S, V>(shift + i, tmp);
+      for (int j = 0; j < V; ++j)
+        ap[j] = need_prev_row ? c.before[j] * rp * g1[j] : c.before[j];
 #pragma unroll
-      for (int j = 0; j < V; ++j) o[j] = a[j] + (ap[j] - a[j]) * tmp[j];
+      for (int j = 0; j < V; ++j) o[j] = a[j] + (ap[j] - a[j]) * c.mix[j];
       stv<S, V>(s_out + (size_t)t * W + i, o);
       if (is_last)
         stv<float, V>(last ? last + (size_t)b * W + i
                            : prev + (size_t)sslot[b] * W + i, a);
+    }
+  };
+  if (R > 0) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = (threadIdx.x + r * 256) * V;
+      if (i < W) put(i, at[r]);
+    }
+  } else {
+    for (int i = threadIdx.x * V; i < W; i += 256 * V) {
+      load(i, at[0]);
+      load_before(i, at[0]);
+      put(i, at[0]);
     }
   }
 }
@@ -593,7 +632,9 @@ __global__ void __launch_bounds__(256) headnorm_gate_kernel(
   }
 }
 
-template <typename S, int V>
+// Rows of up to R * 256 * V stay in registers: read once, all loads in flight together (rows
+// of 8192 bf16, six: 6.5 us read twice, 4.4 so; 7636: 58 us, 41).  R = 0: any length.
+template <typename S, int V, int R>
 __global__ void __launch_bounds__(256) polynorm_kernel(
     S* __restrict__ out, const S* __restrict__ z, const float* __restrict__ coef,
     float eps, int F, i64 ldz) {
@@ -601,9 +642,8 @@ __global__ void __launch_bounds__(256) polynorm_kernel(
   const int t = blockIdx.x;
   const S* zr = z + (size_t)t * ldz;
   float s[3] = {0.f, 0.f, 0.f};
-  for (int i = threadIdx.x * V; i < F; i += 256 * V) {
-    float v[4];
-    ldv<S, V>(zr + i, v);
+  float row[R > 0 ? R : 1][4];
+  auto add = [&](const float (&v)[4]) {
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       const float v2 = v[j] * v[j];
@@ -611,21 +651,45 @@ __global__ void __launch_bounds__(256) polynorm_kernel(
       s[1] += v2 * v2;
       s[2] += v2 * v2 * v2;
     }
+  };
+  if (R > 0) {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      ldv<S, V>(zr + min((int)(threadIdx.x + r * 256) * V, F - V), row[r]);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if ((int)(threadIdx.x + r * 256) * V < F) add(row[r]);
+  } else {
+    for (int i = threadIdx.x * V; i < F; i += 256 * V) {
+      ldv<S, V>(zr + i, row[0]);
+      add(row[0]);
+    }
   }
+  const float c0 = coef[0], c1 = coef[1], c2 = coef[2], c3 = coef[3];
   block_sum<3>(s, red);
   const float r1 = 1.0f / sqrtf(s[0] / (float)F + eps);
   const float r2 = 1.0f / sqrtf(s[1] / (float)F + eps);
   const float r3 = 1.0f / sqrtf(s[2] / (float)F + eps);
-  const float c0 = coef[0], c1 = coef[1], c2 = coef[2], c3 = coef[3];
-  for (int i = threadIdx.x * V; i < F; i += 256 * V) {
-    float v[4], o[4];
-    ldv<S, V>(zr + i, v);
+  auto put = [&](int i, const float (&v)[4]) {
+    float o[4];
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       const float v2 = v[j] * v[j];
       o[j] = c0 * (v[j] * r1) + c1 * (v2 * r2) + c2 * (v2 * v[j] * r3) + c3;
     }
     stv<S, V>(out + (size_t)t * F + i, o);
+  };
+  if (R > 0) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int i = (threadIdx.x + r * 256) * V;
+      if (i < F) put(i, row[r]);
+    }
+  } else {
+    for (int i = threadIdx.x * V; i < F; i += 256 * V) {
+      ldv<S, V>(zr + i, row[0]);
+      put(i, row[0]);
+    }
   }
 }
 
@@ -1051,13 +1115,15 @@ AF_EXPORT int afm_dual_norm_shift(
   hipStream_t s = (hipStream_t)stream;
   const bool vec = W % 4 == 0 && aligned16(a, s_out, b, last, x, w1) &&
                    aligned16(w2, shift, prev);
-#define DNS(ST, V)                                                            \
-  dual_norm_shift_kernel<ST, V><<<T, 256, 0, s>>>((ST*)a, (ST*)s_out, (ST*)b, \
+#define DNS(ST, V, R)                                                         \
+  dual_norm_shift_kernel<ST, V, R><<<T, 256, 0, s>>>((ST*)a, (ST*)s_out, (ST*)b, \
       (float*)last, (const float*)x, (const ST*)w1, (const ST*)w2,            \
       (const ST*)shift, (float*)prev, (const i32*)row_seq,                    \
       (const i32*)cu, (const i32*)q_start, (const i32*)sslot, eps, W)
-  if (vec) MIX_DISPATCH(dt, (DNS(u16, 4)), (DNS(float, 4)));
-  else MIX_DISPATCH(dt, (DNS(u16, 1)), (DNS(float, 1)));
+  if (vec && W > 0 && W <= 2048) MIX_DISPATCH(dt, (DNS(u16, 4, 2)), (DNS(float, 4, 2)));
+  else if (vec && W > 0 && W <= 4096) MIX_DISPATCH(dt, (DNS(u16, 4, 4)), (DNS(float, 4, 4)));
+  else if (vec) MIX_DISPATCH(dt, (DNS(u16, 4, 0)), (DNS(float, 4, 0)));
+  else MIX_DISPATCH(dt, (DNS(u16, 1, 0)), (DNS(float, 1, 0)));
 #undef DNS
   return af_last_err();
 }
@@ -1112,11 +1178,13 @@ AF_EXPORT int afm_polynorm(void* out, const void* z, const void* coef,
   if (T == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const bool vec = F % 4 == 0 && ldz % 4 == 0 && aligned16(out, z);
-#define PN(ST, V)                                                     \
-  polynorm_kernel<ST, V><<<T, 256, 0, s>>>((ST*)out, (const ST*)z,    \
+#define PN(ST, V, R)                                                  \
+  polynorm_kernel<ST, V, R><<<T, 256, 0, s>>>((ST*)out, (const ST*)z,    \
       (const float*)coef, eps, F, ldz)
-  if (vec) MIX_DISPATCH(dt, (PN(u16, 4)), (PN(float, 4)));
-  else MIX_DISPATCH(dt, (PN(u16, 1)), (PN(float, 1)));
+  if (vec && F > 0 && F <= 4096) MIX_DISPATCH(dt, (PN(u16, 4, 4)), (PN(float, 4, 4)));
+  else if (vec && F > 0 && F <= 8192) MIX_DISPATCH(dt, (PN(u16, 4, 8)), (PN(float, 4, 8)));
+  else if (vec) MIX_DISPATCH(dt, (PN(u16, 4, 0)), (PN(float, 4, 0)));
+  else MIX_DISPATCH(dt, (PN(u16, 1, 0)), (PN(float, 1, 0)));
 #undef PN
   return af_last_err();
 }

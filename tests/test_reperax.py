@@ -251,6 +251,56 @@ def test_chunk_attention_alone(device, dtype, shape):
     assert rel_err(torch.cat(got), want) < tol(dtype)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("W", [4, 1020, 2048, 2052, 4096, 4100, 8192, 8196, 1023])
+def test_row_kernels_around_their_register_rows(dtype, W):
+    """Rows that stay in registers in whole, in part, or are read again, in steps of four
+    elements and of one; decode steps and chunks.  Against the same formulas in fp32 on
+    the CPU: fp32 sums over W, and where both results are rounded to bf16 they may fall
+    on the two sides of a tie: one step of 8 bits, up to 2^-7 of the value."""
+    torch.manual_seed(W)
+    T, rel = 5, 2 ** -7 if dtype == torch.bfloat16 else W ** 0.5 * 2 ** -22
+
+    def same(got, want, slack=0.0):
+        got, want = got.float().cpu(), want.float()
+        assert ((got - want).abs() <= want.abs() * rel + slack).all()
+
+    z, coef = torch.randn(T, W).to(dtype), torch.tensor([.4, .3, .2, .1])
+    # terms of at most 16 or so cancel
+    same(sm.polynorm(z.cuda(), coef.cuda(), 1e-6), sm.polynorm(z, coef, 1e-6),
+         2 ** -18)
+    x = torch.randn(T, W)
+    w = [torch.rand(W).to(dtype) for _ in range(3)]
+    for lens, starts in (([1] * T, [0, 3, 3, 0, 9]), ([2, 3], [4, 0])):
+        prev = torch.randn(T + 1, W)
+        md, _ = md_for(lens, starts, list(range(1, len(lens) + 1)), "cpu")
+        md.is_prefill = len(lens) < T
+        on = SimpleNamespace(**{k: v.cuda() if torch.is_tensor(v) else v
+                                for k, v in vars(md).items()})
+        there = prev.cuda()
+        got = sm.dual_norm_shift(x.cuda(), *(v.cuda() for v in w), 1e-6, there, on, dtype)
+        want = sm.dual_norm_shift(x, *w, 1e-6, prev, md, dtype)
+        for g, v in zip(got, want):
+            same(g, v, 2 ** -18)
+        same(there, prev, 2 ** -18)
+    if W % 2:
+        return
+    dk, G = W // 2, 2
+    q, k, v = (torch.randn(T, 2 * dk).to(dtype) for _ in range(3))
+    qw, kw = torch.rand(2 * dk).to(dtype), torch.rand(2 * dk).to(dtype)
+    slots = torch.tensor([3, 0, 7, 9, 4])
+    for ws in ((qw, kw), (None, None)):
+        caches = [torch.zeros(3, G, 4, dk, dtype=dtype) for _ in range(2)]
+        onc = [c.cuda() for c in caches]
+        got = sm.qk_norm_cache(q.cuda(), k.cuda(), v.cuda(),
+                               *(None if u is None else u.cuda() for u in ws), 1e-6,
+                               *onc, slots.cuda())
+        same(got, sm.qk_norm_cache(q, k, v, *ws, 1e-6, *caches, slots))
+        same(onc[0], caches[0])
+        assert torch.equal(onc[1].cpu(), caches[1])
+
+
 @pytest.mark.parametrize("device", DEVICES)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_chunk_edge_one_key_stands_out(device, dtype):
