@@ -261,39 +261,86 @@ __global__ void __launch_bounds__(256) masked_attention_kernel(
 // ------------------------------------------------ row attention (decode)
 // One workgroup per (row, K/V head): the GQ query heads of the group share
 // every K and V load.  Keys are walked in super-tiles of `kt`:
-//   A. scores: one key per lane, its row read 16 bytes at a time and dotted
-//      with every head's query (queries sit in LDS, read as broadcasts), so
-//      no cross-lane reduction is needed; one score per (head, key) in LDS;
-//   B. per head: max, exp, sum over the tile (running max / sum / rescale
-//      factor kept in LDS across super-tiles);
+//   A. scores: a key row is read by adjacent lanes, 16 bytes each, as the value
+//      rows are: its lines are fetched whole and once, where one key per lane
+//      walked 64 rows at a time and lost lines between its reads of them.  The
+//      query slices stay in registers; partial dot products meet in lane swaps
+//      and DPP.  One score per (head, key) in LDS, beside the key's page;
+//   B. per head: bias and cap, max, exp, sum over the tile (running max / sum /
+//      rescale factor kept in LDS across super-tiles);
 //   C. P.V: a value row is read by LPV adjacent lanes, each lane accumulates
 //      its 16-byte slice for every head in registers.
-// The partial outputs of the key groups are summed with shuffles, across
+// The partial outputs of the key groups are summed with lane swaps and DPP, across
 // waves through LDS.  Serves decode steps and short prompt portions, bf16
 // and fp32 storage; head sizes up to 64 lanes x 16 bytes.
+// Few rows are bound by the chain position, block table, K, scores, V: its branches
+// on the lane layout and the page size stand outside the unrolled loops, and no
+// division is in it.  Eight key or value rows in flight per lane, or the next value rows
+// asked for ahead, cost more in wavefronts than they hid.  With the merge, heads of 128
+// over 8 K/V heads, one key per lane -> adjacent lanes: 6 rows of up to 512 keys 16.5 ->
+// 10.6 us, of 1000 keys 30.4 -> 17.8; 64 rows of 400 keys 43 -> 28; 128 rows of 3000 keys
+// 398 -> 289 us (5.4 TB/s); fp32, 6 rows of up to 512 keys 15.9 -> 12.3.
+
+// Sixteen bytes of a row in storage type, for loads that stay in flight across other work;
+// zeros past the row's end.
 template <typename S, bool VEC>
-__device__ __forceinline__ void load_slice(const S* row, int e0, int n,
-                                           float (&o)[16 / sizeof(S)]) {
-  constexpr int EPL = 16 / sizeof(S);
-  if (VEC) {
-    if (e0 < n) {
-      if constexpr (sizeof(S) == 2) {
-        const s16x8 v = *reinterpret_cast<const s16x8*>(row + e0);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) o[j] = bf2f((u16)v[j]);
-      } else {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(row + e0);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o[j] = v[j];
-      }
+struct RawSlice {
+  static constexpr int EPL = 16 / sizeof(S);
+  union { f32x4 v; S e[EPL]; };
+  __device__ __forceinline__ void load(const S* row, int e0, int n, bool wide = true) {
+    if (VEC && wide) {
+      v = *reinterpret_cast<const f32x4*>(row + min(e0, n - EPL));
     } else {
 #pragma unroll
-      for (int j = 0; j < EPL; ++j) o[j] = 0.f;
+      for (int j = 0; j < EPL; ++j) e[j] = row[min(e0 + j, n - 1)];
     }
-  } else {
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) o[j] = (e0 + j < n) ? ldf<S>(row + e0 + j) : 0.f;
   }
+  __device__ __forceinline__ void floats(int e0, int n, float (&o)[EPL]) const {
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) o[j] = e0 + (VEC ? 0 : j) < n ? ldf<S>(e + j) : 0.f;
+  }
+};
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float add_half_f32(float v) {      // the other 32 lanes
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v),
+                                                  false, false);
+  return __uint_as_float(a[0]) + __uint_as_float(a[1]);
+}
+__device__ __forceinline__ float add_quarter_f32(float v) {   // the other 16 of 32 lanes
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v),
+                                                  false, false);
+  return __uint_as_float(a[0]) + __uint_as_float(a[1]);
+}
+
+// Each value's sum over groups of 1 << log2 adjacent lanes, in each of them (the branches,
+// which all lanes take together, once for all N values).
+template <int N>
+__device__ __forceinline__ void group_sums(float (&v)[N], int log2) {
+#define EACH(...) do { _Pragma("unroll") for (int i = 0; i < N; ++i) __VA_ARGS__; } while (0)
+  if (log2 > 0) EACH(v[i] += dpp_f32<0xB1>(v[i]));    // lanes 1 apart
+  if (log2 > 1) EACH(v[i] += dpp_f32<0x4E>(v[i]));    // 2 apart
+  if (log2 > 2) EACH(v[i] += dpp_f32<0x141>(v[i]));   // the other half of 8, mirrored
+  if (log2 > 3) EACH(v[i] += dpp_f32<0x140>(v[i]));   // the other half of 16, mirrored
+  if (log2 > 4) EACH(v[i] = add_quarter_f32(v[i]));
+  if (log2 > 5) EACH(v[i] = add_half_f32(v[i]));
+}
+
+// Each value's sum over the lanes with the same low log2 bits of their number, in each of them.
+template <int N>
+__device__ __forceinline__ void strided_sums(float (&v)[N], int log2) {
+  if (log2 < 6) EACH(v[i] = add_half_f32(v[i]));
+  if (log2 < 5) EACH(v[i] = add_quarter_f32(v[i]));
+  // rotations within 16 lanes, whose halves, quarters, ... are alike by then
+  if (log2 < 4) EACH(v[i] += dpp_f32<0x128>(v[i]));
+  if (log2 < 3) EACH(v[i] += dpp_f32<0x124>(v[i]));
+  if (log2 < 2) EACH(v[i] += dpp_f32<0x122>(v[i]));
+  if (log2 < 1) EACH(v[i] += dpp_f32<0x121>(v[i]));
+#undef EACH
 }
 
 // NK = 2 (differential attention, ex.vshare == 2): the workgroup's heads are
@@ -305,14 +352,15 @@ __global__ void __launch_bounds__(256) attn_rows_kernel(
     S* __restrict__ out, const S* __restrict__ q, const S* __restrict__ kc,
     const S* __restrict__ vc, const i32* __restrict__ bt,
     const i32* __restrict__ row_seq, const i32* __restrict__ positions,
-    float scale, int H, int G, int dk, int dv, int page, int maxp, int chunk,
-    int window, i64 ldq, int lpk_log2, int lpv_log2, int kt, int nsplit,
+    float scale, int H, int G, int hpg, int dk, int dv, int page, int page_log2,
+    int q_wide, int maxp, int chunk, int window, i64 ldq, int lpk_log2, int lpv_log2, int kt, int nsplit,
     float* __restrict__ part_o, float* __restrict__ part_ml, AttnExtra ex) {
   // nsplit > 1: the visible keys are cut into nsplit ranges, one workgroup
   // each (grid.z = head blocks x nsplit).  With part_o, unnormalised outputs
   // and (max, sum) go to part_o [T, H, nsplit, dv] / part_ml [T, H, nsplit,
   // 2] for attn_split_combine_kernel (or diff_combine_kernel) to merge.
   constexpr int EPL = 16 / sizeof(S);
+  constexpr int UK = 4, UV = 4;                // key and value rows in flight per lane
   extern __shared__ float smem[];
   const int dvp = EPL << lpv_log2;             // padded value width
   float* sc = smem;                            // [GQ][kt] scores, then probabilities
@@ -322,15 +370,24 @@ __global__ void __launch_bounds__(256) attn_rows_kernel(
   float* corr = l_run + 8;                     // [8]
   float* r1s = corr + 8;                       // [8] distance-bias factors
   float* r2s = r1s + 8;                        // [8]
-  const int dkp = (dk + EPL - 1) / EPL * EPL;
-  float* qs = r2s + 8;                         // [GQ][dkp] scaled queries
+  i32* pgs = reinterpret_cast<i32*>(r2s + 8);  // [kt] pages of the tile's keys
   const int t = blockIdx.x, g = blockIdx.y;
-  const int GV = NK == 2 ? G : G / ex.vshare, gv = NK == 2 ? g : g / ex.vshare;
-  const int hpg = H / G;
-  const int zh = blockIdx.z / nsplit, sp = blockIdx.z % nsplit;
+  const bool own = NK == 2 || ex.vshare == 1;
+  const int GV = own ? G : G / ex.vshare, gv = own ? g : g / ex.vshare;
+  const int zh = (int)gridDim.z == nsplit ? 0 : blockIdx.z / nsplit;
+  const int sp = blockIdx.z - zh * nsplit;
   const int h0 = g * hpg + zh * GQ;
   const int nh = min(GQ, hpg - zh * GQ);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int lik = lane & ((1 << lpk_log2) - 1), kik = lane >> lpk_log2;
+  const int kpk = 64 >> lpk_log2;
+  const int liv = lane & ((1 << lpv_log2) - 1), kiv = lane >> lpv_log2;
+  const int kpv = 64 >> lpv_log2;
+  RawSlice<S, VEC> qr[GQ];                     // the lane's slice of each query
+#pragma unroll
+  for (int gg = 0; gg < GQ; ++gg)
+    qr[gg].load(q + (size_t)t * ldq + (size_t)(h0 + min(gg, nh - 1)) * dk, lik * EPL, dk,
+                q_wide);
   int pos = positions[t];
   const int qpos = pos;
   const i32* btr = bt + (size_t)row_seq[t] * maxp;
@@ -348,14 +405,20 @@ __global__ void __launch_bounds__(256) attn_rows_kernel(
     pos = min(pos, lo + per - 1);
   }
 
-  const int liv = lane & ((1 << lpv_log2) - 1), kiv = lane >> lpv_log2;
-  const int kpv = 64 >> lpv_log2;
-
-  for (int i = threadIdx.x; i < GQ * dkp; i += 256) {
-    const int gg = i / dkp, d = i % dkp;
-    qs[i] = (gg < nh && d < dk)
-        ? ldf<S>(q + (size_t)t * ldq + (size_t)(h0 + gg) * dk + d) * scale : 0.f;
-  }
+  // where keys of the tile (virtual indexes, see above) lie: their page's place in the
+  // block table and the place in it.  A page is a power of two of keys as a rule.
+  auto places = [&](auto& jv, auto& at) {
+    constexpr int N = sizeof(jv) / sizeof(int);
+#pragma unroll
+    for (int u = 0; u < N; ++u) jv[u] = jv[u] < wlo ? jv[u] - vsh : jv[u];
+    if (page_log2 >= 0) {
+#pragma unroll
+      for (int u = 0; u < N; ++u) { at[u] = jv[u] & (page - 1); jv[u] >>= page_log2; }
+    } else {
+#pragma unroll
+      for (int u = 0; u < N; ++u) { at[u] = jv[u] % page; jv[u] /= page; }
+    }
+  };
   float acc[GQ][EPL];
 #pragma unroll
   for (int gg = 0; gg < GQ; ++gg)
@@ -373,46 +436,72 @@ __global__ void __launch_bounds__(256) attn_rows_kernel(
 
   for (int tile0 = lo; tile0 <= pos; tile0 += kt) {
     const int nk = min(kt, pos + 1 - tile0);
-    // ---- A: scores, one key per lane ----
-    if (tile0 == lo) __syncthreads();          // queries are in LDS
-    for (int kidx = threadIdx.x; kidx < nk; kidx += 256) {
-      const int jv = tile0 + kidx;
-      const int j = jv < wlo ? jv - vsh : jv;
-      const S* kr = kc + (((size_t)btr[j / page] * G + g) * NK * page + (j % page)) * dk;
-      const S* kr1 = kr + (size_t)(NK - 1) * page * dk;    // the second map's
-      float sco[GQ];
+    // ---- A: scores, a key's row over adjacent lanes ----
+    int pgk[UK], atk[UK];
+    auto look_up = [&](int kb) {
+      int pi[UK];
 #pragma unroll
-      for (int gg = 0; gg < GQ; ++gg) sco[gg] = 0.f;
-#pragma unroll 4
-      for (int e0 = 0; e0 < dk; e0 += EPL) {
-        float kv[EPL];
-        load_slice<S, VEC>(kr, e0, dk, kv);
+      for (int u = 0; u < UK; ++u) pi[u] = tile0 + min(kb + u * 4 * kpk + kik, nk - 1);
+      places(pi, atk);
 #pragma unroll
-        for (int gg = 0; gg < GQ / NK; ++gg)
+      for (int u = 0; u < UK; ++u) pgk[u] = btr[pi[u]];
+    };
+    if (wave * kpk < nk) look_up(wave * kpk);
+    for (int kb = wave * kpk; kb < nk; kb += 4 * UK * kpk) {
+      RawSlice<S, VEC> kk[UK][NK];
 #pragma unroll
-          for (int e = 0; e < EPL; ++e) sco[gg] += qs[gg * dkp + e0 + e] * kv[e];
-        if constexpr (NK == 2) {
-          load_slice<S, VEC>(kr1, e0, dk, kv);
+      for (int u = 0; u < UK; ++u) {
+        const S* kr = kc + (((size_t)pgk[u] * G + g) * NK * page + atk[u]) * dk;
 #pragma unroll
-          for (int gg = GQ / 2; gg < GQ; ++gg)
+        for (int m = 0; m < NK; ++m)           // the second map's rows lie behind the first's
+          kk[u][m].load(kr + (size_t)m * page * dk, lik * EPL, dk);
+        if (lik == 0) pgs[min(kb + u * 4 * kpk + kik, nk - 1)] = pgk[u];
+      }
+      if (kb + 4 * UK * kpk < nk) look_up(kb + 4 * UK * kpk);
+      float qv[GQ][EPL];
 #pragma unroll
-            for (int e = 0; e < EPL; ++e) sco[gg] += qs[gg * dkp + e0 + e] * kv[e];
+      for (int gg = 0; gg < GQ; ++gg) qr[gg].floats(lik * EPL, dk, qv[gg]);
+      float a[UK * GQ];
+#pragma unroll
+      for (int u = 0; u < UK; ++u) {
+        float kf[NK][EPL];
+#pragma unroll
+        for (int m = 0; m < NK; ++m) kk[u][m].floats(lik * EPL, dk, kf[m]);
+#pragma unroll
+        for (int gg = 0; gg < GQ; ++gg) {
+          const float (&kg)[EPL] = kf[gg / (GQ / NK)];
+          a[u * GQ + gg] = 0.f;
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) a[u * GQ + gg] += qv[gg][e] * kg[e];
         }
       }
+      group_sums(a, lpk_log2);
+      if (lik == 0) {
 #pragma unroll
-      for (int gg = 0; gg < GQ; ++gg)
-        if (gg < nh) {
-          float sv = attn_softcap(sco[gg], ex.cap);
-          if (ex.r1) sv -= attn_dist_bias(r1s[gg], r2s[gg], qpos - j);
-          sc[gg * kt + kidx] = sv;
+        for (int u = 0; u < UK; ++u) {
+          const int kidx = kb + u * 4 * kpk + kik;
+          if (kidx < nk) {
+#pragma unroll
+            for (int gg = 0; gg < GQ; ++gg) sc[gg * kt + kidx] = a[u * GQ + gg] * scale;
+          }
         }
+      }
     }
     __syncthreads();
     // ---- B: softmax statistics, wave w takes heads w, w+4, ... ----
     for (int gg = wave; gg < nh; gg += 4) {
       float* sr = sc + gg * kt;
       float mx = AF_NEG_INF;
-      for (int i = lane; i < nk; i += 64) mx = fmaxf(mx, sr[i]);
+      for (int i = lane; i < nk; i += 64) {
+        float sv = sr[i];
+        if (ex.cap > 0.f || ex.r1) {
+          const int jv = tile0 + i;
+          sv = attn_softcap(sv, ex.cap);
+          if (ex.r1) sv -= attn_dist_bias(r1s[gg], r2s[gg], qpos - (jv < wlo ? jv - vsh : jv));
+          sr[i] = sv;
+        }
+        mx = fmaxf(mx, sv);
+      }
       mx = wave_max_f32(mx);
       const float m_old = m_run[gg];
       const float m_new = fmaxf(m_old, mx);
@@ -440,24 +529,28 @@ __global__ void __launch_bounds__(256) attn_rows_kernel(
         for (int e = 0; e < EPL; ++e) acc[gg][e] *= c;
       }
     }
-    for (int kb = wave * kpv; kb < nk; kb += 16 * kpv) {
-      float vv[4][EPL];
+    for (int kb = wave * kpv; kb < nk; kb += 4 * UV * kpv) {
+      RawSlice<S, VEC> vv[UV];
+      int pi[UV], at[UV];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int jv = tile0 + min(kb + u * 4 * kpv + kiv, nk - 1);
-        const int j = jv < wlo ? jv - vsh : jv;
-        const S* vr = vc + (((size_t)btr[j / page] * GV + gv) * page + (j % page)) * ex.ldv;
-        load_slice<S, VEC>(vr, liv * EPL, dv, vv[u]);
+      for (int u = 0; u < UV; ++u) pi[u] = tile0 + min(kb + u * 4 * kpv + kiv, nk - 1);
+      places(pi, at);
+#pragma unroll
+      for (int u = 0; u < UV; ++u) {
+        const int pg = pgs[min(kb + u * 4 * kpv + kiv, nk - 1)];
+        vv[u].load(vc + (((size_t)pg * GV + gv) * page + at[u]) * ex.ldv, liv * EPL, dv);
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < UV; ++u) {
         const int kidx = kb + u * 4 * kpv + kiv;
         const bool valid = kidx < nk;
+        float vf[EPL];
+        vv[u].floats(liv * EPL, dv, vf);
 #pragma unroll
         for (int gg = 0; gg < GQ; ++gg) {
           const float p = (valid && gg < nh) ? sc[gg * kt + kidx] : 0.f;
 #pragma unroll
-          for (int e = 0; e < EPL; ++e) acc[gg][e] += p * vv[u][e];
+          for (int e = 0; e < EPL; ++e) acc[gg][e] += p * vf[e];
         }
       }
     }
@@ -465,13 +558,14 @@ __global__ void __launch_bounds__(256) attn_rows_kernel(
   }
   // ---- sum the key groups of a wave, then the 4 waves ----
 #pragma unroll
-  for (int gg = 0; gg < GQ; ++gg)
+  for (int gg = 0; gg < GQ; ++gg) strided_sums(acc[gg], lpv_log2);
+  if (kiv == 0) {
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      float a = acc[gg][e];
-      for (int o = 1 << lpv_log2; o < 64; o <<= 1) a += __shfl_xor(a, o, 64);
-      if (kiv == 0) red[(wave * GQ + gg) * dvp + liv * EPL + e] = a;
-    }
+    for (int gg = 0; gg < GQ; ++gg)
+#pragma unroll
+      for (int e = 0; e < EPL; ++e)
+        red[(wave * GQ + gg) * dvp + liv * EPL + e] = acc[gg][e];
+  }
   __syncthreads();
   for (int i = threadIdx.x; i < nh * dv; i += 256) {
     const int gg = i / dv, d = i % dv;
@@ -492,8 +586,8 @@ __global__ void __launch_bounds__(256) attn_rows_kernel(
 }
 
 // One wave per (row, head): merge the nsplit (<= 64) partial softmaxes.
-// Lane s weighs split s once; empty splits (max = -inf) weigh nothing and
-// their partial outputs are never read.
+// Lane s weighs split s once; empty splits (max = -inf) weigh nothing and their partial
+// outputs are not added.  Eight splits' are asked for together: one wait, not one each.
 template <typename S>
 __global__ void __launch_bounds__(256) attn_split_combine_kernel(
     S* __restrict__ out, const float* __restrict__ part_o,
@@ -512,11 +606,17 @@ __global__ void __launch_bounds__(256) attn_split_combine_kernel(
   S* orow = out + (size_t)t * ex.ldo + (size_t)h * dv;
   for (int d0 = 0; d0 < dv; d0 += 64) {
     const int d = d0 + lane;
+    const float* po = part_o + (size_t)rh * nsplit * dv + min(d, dv - 1);
     float o = 0.f;
-    for (int s = 0; s < nsplit; ++s) {
-      const float ws = __shfl(w, s, 64);
-      if (ws > 0.f && d < dv)
-        o += part_o[((size_t)rh * nsplit + s) * dv + d] * ws;
+    for (int s0 = 0; s0 < nsplit; s0 += 8) {
+      float p[8];   // an empty split's may hold anything, and is not added
+#pragma unroll
+      for (int u = 0; u < 8; ++u) p[u] = po[(size_t)min(s0 + u, nsplit - 1) * dv];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float ws = s0 + u < nsplit ? __shfl(w, s0 + u, 64) : 0.f;
+        if (ws > 0.f) o += p[u] * ws;
+      }
     }
     if (d < dv) stf<S>(orow + d, o * inv);
   }
@@ -549,13 +649,22 @@ __global__ void __launch_bounds__(256) diff_combine_kernel(
     const float m = wave_max_f32(ms);
     const float w = ms > AF_NEG_INF ? expf(ms - m) : 0.f;
     const float ws = (mp ? -lam : 1.0f) * w / wave_sum_f32(w * ls);
-    for (int s = 0; s < nsplit; ++s) {
-      if (__shfl(w, s, 64) <= 0.f) continue;   // empty splits are never read
-      const float wv = __shfl(ws, s, 64);
-      const float* p = part_o + (ph * nsplit + s) * dv;
+    for (int s0 = 0; s0 < nsplit; s0 += 4) {
+      float p[4][NV];                          // empty splits' are not added
 #pragma unroll
-      for (int i = 0; i < NV; ++i)
-        if (i * 64 + lane < dv) o[i] += wv * p[i * 64 + lane];
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+          p[u][i] = part_o[(ph * nsplit + min(s0 + u, nsplit - 1)) * dv +
+                           min(i * 64 + lane, dv - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (s0 + u >= nsplit || __shfl(w, s0 + u, 64) <= 0.f) continue;
+        const float wv = __shfl(ws, s0 + u, 64);
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+          if (i * 64 + lane < dv) o[i] += wv * p[u][i];
+      }
     }
   }
   float ss = 0.f;
@@ -1129,17 +1238,18 @@ static int launch_attention(void* out, const void* q, const void* kc,
     const int gq = hpg >= 8 ? 8 : hpg > 2 ? 4 : hpg;   // 1, 2, 4 or 8
     const int dvp = EPL << lpv;
     const int kt = dvp <= 128 ? 1024 : 512;
-    const int dkp = (dk + EPL - 1) / EPL * EPL;
-    const size_t sm = ((size_t)gq * kt + 4 * gq * dvp + 40 +
-                       (size_t)gq * dkp) * sizeof(float);
+    const size_t sm = ((size_t)gq * kt + 4 * gq * dvp + 40 + kt) * sizeof(float);
     const bool vec = dk % EPL == 0 && dv % EPL == 0 && ex.ldv % EPL == 0 &&
                      (uintptr_t)kc % 16 == 0 && (uintptr_t)vc % 16 == 0;
+    const int q_wide = ldq % EPL == 0 && (uintptr_t)q % 16 == 0;
+    const int pl2 = page & (page - 1) ? -1 : clog2(page);
     dim3 grid(T, G, ((hpg + gq - 1) / gq) * nsplit);
 #define ROWS(GQ, ...)                                                         \
   attn_rows_kernel<S, GQ, __VA_ARGS__><<<grid, 256, sm, s>>>(                 \
       (S*)out, (const S*)q, (const S*)kc, (const S*)vc, (const i32*)bt,       \
-      (const i32*)row_seq, (const i32*)positions, scale, H, G, dk, dv, page,  \
-      maxp, chunk, window, ldq, lpk, lpv, kt, nsplit, part_o, part_ml, ex)
+      (const i32*)row_seq, (const i32*)positions, scale, H, G, hpg, dk, dv,    \
+      page, pl2, q_wide, maxp, chunk, window, ldq, lpk, lpv, kt, nsplit,      \
+      part_o, part_ml, ex)
     if (both) {
       if (vec) {
         if (gq == 2) ROWS(2, true, 2); else if (gq == 4) ROWS(4, true, 2);

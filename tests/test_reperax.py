@@ -253,6 +253,48 @@ def test_chunk_attention_alone(device, dtype, shape):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,G,dk,dv,page,odd", [
+    (1, 1, 4, 8, 8, 0), (2, 1, 16, 40, 8, 0), (3, 1, 30, 33, 7, 0),
+    (8, 2, 64, 24, 16, 3), (8, 1, 128, 128, 16, 0), (11, 1, 96, 200, 5, 0),
+    (2, 2, 256, 512, 16, 1), (1, 1, 500, 136, 16, 0)])
+def test_row_attention_on_every_lane_layout(dtype, H, G, dk, dv, page, odd, monkeypatch):
+    """Keys and values over 1 to 64 lanes, pages of a power of two of keys and others,
+    queries in rows of an odd stride, one and several key splits, positions around the
+    rounds of 4 waves.  Against the same sums in 64 bits: |scores| < 8 and values of one
+    or so, so 2^-8 of rounding in a bf16 result, and about dk + keys roundings of 2^-24
+    of the scores and the weights in fp32 (so not the kernel of many heads, whose
+    weights are bf16)."""
+    monkeypatch.setattr(sm, "HEADS_MFMA_MIN", 99)
+    torch.manual_seed(dk)
+    pos = [0, 1, 15, 16, 63, 64, 255, 256, 257, 700]
+    T, maxp = len(pos), -(-701 // page)
+    md, _ = md_for([1] * T, pos, [1] * T, "cpu", page, maxp)
+    kc = torch.randn(T * maxp + 1, G, page, dk).to(dtype)
+    vc = torch.randn(T * maxp + 1, G, page, dv).to(dtype)
+    q = torch.randn(T, H * dk + odd).to(dtype)[:, :H * dk]
+    on = SimpleNamespace(**{k: v.cuda() if torch.is_tensor(v) else v
+                            for k, v in vars(md).items()})
+    qd = torch.empty(T, H * dk + odd, dtype=dtype, device="cuda")[:, :H * dk]
+    qd.copy_(q)
+    positions = torch.tensor(pos, dtype=torch.int32)
+    for window in (0, 100):
+        got = sm.masked_attention(qd, kc.cuda(), vc.cuda(), on, positions.cuda(),
+                                  dk ** -0.5, H, window=window).cpu()
+        for t, p in enumerate(pos):
+            js = torch.arange(max(0, p - window + 1) if window else 0, p + 1)
+            pg = md.block_table[t].long()[js // page]
+            k, v = (c[pg, :, js % page].to(F64).repeat_interleave(H // G, 1)
+                    for c in (kc, vc))
+            w = torch.softmax(torch.einsum("nhd,hd->hn", k, q[t].to(F64).view(H, dk))
+                              * dk ** -0.5, -1)
+            want = torch.einsum("hn,nhd->hd", w, v).reshape(-1)
+            err = (got[t].to(F64) - want).abs().max()
+            assert err < (want.abs().max() * 2 ** -8 if dtype == torch.bfloat16
+                          else 0) + (dk + 701) * 2 ** -24
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("W", [4, 1020, 2048, 2052, 4096, 4100, 8192, 8196, 1023])
 def test_row_kernels_around_their_register_rows(dtype, W):
     """Rows that stay in registers in whole, in part, or are read again, in steps of four
