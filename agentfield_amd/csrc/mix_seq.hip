@@ -942,6 +942,33 @@ constexpr int scan_rows(int rp, int threads) {
   return (rp >= 16 ? 8 : 16) * 16 * rp / threads;
 }
 
+// The sequence of a workgroup, and its rows.  The grid walks sequence by sequence, and the
+// longest comes first where that decides what shares a CU and what is left to the end:
+// beyond one workgroup per CU (256).  With a head of every sequence in turn two of the
+// longest met on one CU, or one started last: 6 sequences of 620..1900 tokens in 384
+// workgroups 430 -> 328 us, 32 of up to 1500 in 2048 1173 -> 660 and, with decays per channel,
+// 1312 -> 650.  A lane per sequence finds the ranks; more than 64 sequences keep their order
+// (70 of up to 700 tokens 864 -> 815, 995 -> 900).
+struct ScanRows { int b, t0, t1; };
+__device__ __forceinline__ ScanRows scan_sequence(const i32* __restrict__ cu) {
+  const int B = gridDim.z, turn = blockIdx.z;
+  if (B > 64 || B * gridDim.x * gridDim.y <= 256) return {turn, cu[turn], cu[turn + 1]};
+  const int lane = min((int)threadIdx.x & 63, B - 1);
+  const int from = cu[lane], len = cu[lane + 1] - from;
+  // (lengths alike: nothing to win, and the ranks cost short ones 1 us of 48)
+  if (wave_max_f32((float)len) + wave_max_f32((float)-len) < 64.f)
+    return {turn, __builtin_amdgcn_readlane(from, turn),
+            __builtin_amdgcn_readlane(from, turn) + __builtin_amdgcn_readlane(len, turn)};
+  int rank = 0;
+  for (int j = 0; j < B; ++j) {
+    const int other = __builtin_amdgcn_readlane(len, j);
+    rank += other > len || (other == len && j < lane);
+  }
+  const int b = __ffsll((unsigned long long)__ballot(rank == turn)) - 1;
+  const int t0 = __builtin_amdgcn_readlane(from, b);
+  return {b, t0, t0 + __builtin_amdgcn_readlane(len, b)};
+}
+
 // The same recurrence for prompts.  A thread stages E consecutive rows of one token
 // (one wide load each for q, k, the rotary partners and the decay logits, kept raw
 // until the block before has been worked through) and computes RP rows of one column
@@ -965,8 +992,9 @@ linear_scan_prompt_kernel(
   constexpr int E = scan_rows(RP, NT);
   constexpr int BUF = TB * (3 * DKP + 32);     // [TB][3][DKP], [TB][32]
   extern __shared__ float smem[];
-  const int b = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * 32;
-  const int t0 = cu[b], t1 = cu[b + 1];
+  const ScanRows rows = scan_sequence(cu);
+  const int b = rows.b, t0 = rows.t0, t1 = rows.t1;
+  const int h = blockIdx.x, c0 = blockIdx.y * 32;
   if (t1 <= t0) return;
   const int r = threadIdx.x & 15, cc = threadIdx.x >> 4;
   const int ca = c0 + CPT * cc;
@@ -1391,7 +1419,7 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
                        float inv_tau, int T, int B, int H, int dk, int dv,
                        int rot, i64 ldq, i64 ldk, i64 ldv, i64 ldz,
                        hipStream_t s) {
-  dim3 grid(B, H, (dv + 31) / 32);
+  const dim3 grid(B, H, (dv + 31) / 32), by_sequence(H, grid.z, B);
   const int rp = (dk + 15) / 16;
   const int rpp = rp <= 2 ? 2 : rp <= 4 ? 4 : rp <= 8 ? 8 : 16;
   // From a block of tokens per sequence on the prompt kernel is the better one
@@ -1400,7 +1428,7 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
   auto loads = [&](int threads) {
     const int E = scan_rows(rpp, threads);
     const size_t al = E * sizeof(S) < 16 ? E * sizeof(S) : 16;
-    return T >= 16 * B && dk % E == 0 && (rot / 2) % E == 0 && ldq % E == 0 &&
+    return T >= 16 * B && B <= 65535 && dk % E == 0 && (rot / 2) % E == 0 && ldq % E == 0 &&
            ldk % E == 0 && (!zl || ldz % E == 0) && (uintptr_t)q % al == 0 &&
            (uintptr_t)k % al == 0 && (uintptr_t)zl % al == 0;
   };
@@ -1430,10 +1458,10 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
   do {                                                                       \
     if (zl)                                                                  \
       linear_scan_prompt_kernel<S, RP, true, NT>                             \
-          <<<grid, NT, sm, s>>>(SCAN_ARGS);                                  \
+          <<<by_sequence, NT, sm, s>>>(SCAN_ARGS);                           \
     else                                                                     \
       linear_scan_prompt_kernel<S, RP, false, NT>                            \
-          <<<grid, NT, sm, s>>>(SCAN_ARGS);                                  \
+          <<<by_sequence, NT, sm, s>>>(SCAN_ARGS);                           \
   } while (0)
 #define SCAN(RP)                                                             \
   do {                                                                       \
