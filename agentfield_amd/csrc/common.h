@@ -37,6 +37,21 @@ __device__ __forceinline__ u16 f2bf(float f) {
   return (u16)((c.u + 0x7fffu + lsb) >> 16);
 }
 
+// Reduction within 16-lane groups (used for MFMA 16x16 row reductions), in the order of
+// exchanges over 8, 4, 2 and 1 lanes.
+template <typename F>
+__device__ __forceinline__ float group16_reduce_f32(float v, F f) {
+#define AF_ROTATE(N)                                                                \
+  v = f(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + N, \
+                                                      0xf, 0xf, true)))
+  AF_ROTATE(8);
+  AF_ROTATE(4);
+  AF_ROTATE(2);
+  AF_ROTATE(1);
+#undef AF_ROTATE
+  return v;
+}
+
 // ---- wave (64-lane) reductions: every lane ends with the result ----
 // Over the lanes 32, 16, 8, 4, 2 and 1 apart, in this order.  By lane swaps and DPP
 // operands: a shuffle is a round trip through the LDS unit, and small launches wait for
@@ -50,16 +65,7 @@ __device__ __forceinline__ float wave_reduce_f32(float v, F f) {
   const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v),
                                                   false, false);
   v = f(__uint_as_float(b[0]), __uint_as_float(b[1]));
-  // rotations within 16 lanes: 8, 4, 2, 1
-#define AF_ROTATE(N)                                                                \
-  v = f(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + N, \
-                                                      0xf, 0xf, true)))
-  AF_ROTATE(8);
-  AF_ROTATE(4);
-  AF_ROTATE(2);
-  AF_ROTATE(1);
-#undef AF_ROTATE
-  return v;
+  return group16_reduce_f32(v, f);
 }
 
 __device__ __forceinline__ float wave_sum_f32(float v) {
@@ -70,17 +76,12 @@ __device__ __forceinline__ float wave_max_f32(float v) {
   return wave_reduce_f32(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
-// Reduction within 16-lane groups (used for MFMA 16x16 row reductions).
 __device__ __forceinline__ float group16_max_f32(float v) {
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  return group16_reduce_f32(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 __device__ __forceinline__ float group16_sum_f32(float v) {
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  return group16_reduce_f32(v, [](float a, float b) { return a + b; });
 }
 
 #define AF_NEG_INF (-3.0e38f)

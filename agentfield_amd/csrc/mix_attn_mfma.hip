@@ -13,6 +13,16 @@
 // intersect the rows' visible range are visited: for chunk-local attention
 // that is at most chunk/64 + 1 tiles per workgroup.
 //
+// A tile is a chain: pages, rows, LDS, scores, softmax, P V.  What shortens it: pages are
+// looked up two tiles ahead; two workgroups of two heads share a CU (128 registers); the
+// row maxima and sums are DPP; tiles that a wave sees whole are not masked; divisions by the
+// chunk and by a page of a power of two of keys are not in the walk.  16 heads of 128 over 8
+// K/V heads, 7636 rows of six prompts: chunks of 512 152 -> 77 us, windows of 256 132 -> 68,
+// causal 302 -> 210; one K/V head per head 164 -> 113 (rows fetched a tile ahead, 142
+// without; for two heads per workgroup that costs the second workgroup, 77 -> 107); heads of
+// 256 226 -> 165; one latent of 576 for 16 heads 1081 -> 974.  Vector instructions are half of
+// what is left.
+//
 // Fragment layouts of v_mfma_f32_16x16x32_bf16 (64-lane wave):
 //   A: lane holds A[m = lane&15][k = (lane>>4)*8 + j], j = 0..7
 //   B: lane holds B[k = (lane>>4)*8 + j][n = lane&15]
@@ -28,6 +38,13 @@ __device__ __forceinline__ bf16x8 as_bf16x8(s16x8 v) {
   union { s16x8 s; bf16x8 b; } u;
   u.s = v;
   return u.b;
+}
+
+// round to nearest even, by the instruction (TIGHT: by integers, around which the widest
+// instances are not scheduled into 160 spilled registers)
+template <bool TIGHT>
+__device__ __forceinline__ u16 to_bf16(float f) {
+  return TIGHT ? f2bf(f) : __builtin_bit_cast(u16, (__bf16)f);
 }
 
 // 8 consecutive bf16 starting at element e0 of a row of n valid elements;
@@ -46,60 +63,113 @@ __device__ __forceinline__ s16x8 load8(const u16* row, int e0, int n) {
   return v;
 }
 
-// Stage one tile of KT keys: K rows row-major into k_lds, V rows transposed into
-// v_lds ([d][token], token pairs packed into 32-bit writes).  The page walk
-// is done once per key (row_lds[tok] = row index in the pages, -1 for keys
-// past `last`; vrow_lds the value row, whose pages may have fewer heads), so
-// the tile's loads depend on nothing but LDS and are issued back to back.
-// NK = 2 stages the rows of the key heads g and g + 1, one tile behind the
-// other, over one value tile.
-template <int DKC, int DVT, bool VEC, int NT = 256, int KT = 64, int NK = 1>
-__device__ __forceinline__ void stage_kv_tile(
-    u16* k_lds, u16* v_lds, i32* row_lds, i32* vrow_lds,
-    const u16* __restrict__ kc, const u16* __restrict__ vc,
-    const i32* __restrict__ btr, int kv0, int last, int G, int g, int GV,
-    int gv, int page, int dk, int dv, i64 ldv) {
-  constexpr int KS = DKC * 32 + 8;
-  constexpr int VS = KT + 8;
-  constexpr int TP = KT / 2;                  // token pairs
-  if (threadIdx.x < KT) {
-    const int j = kv0 + threadIdx.x;
-    const int pg = j <= last ? btr[j / page] : 0, off = j % page;
-    row_lds[threadIdx.x] = j <= last ? (pg * G + g) * page + off : -1;
-    vrow_lds[threadIdx.x] = j <= last ? (pg * GV + gv) * page + off : -1;
-  }
-  __syncthreads();
-  constexpr int KIT = (NK * KT * DKC * 4 + NT - 1) / NT;
-#pragma unroll
-  for (int it = 0; it < KIT; ++it) {
-    const int i = it * NT + threadIdx.x;
-    if (i >= NK * KT * DKC * 4) break;
+// A tile of KT keys on its way into LDS: K rows row-major into k_lds, V rows transposed into
+// v_lds ([d][token], token pairs packed into 32-bit writes).  The page walk is done once
+// per key (row_lds[tok] = row index in the pages, -1 for keys past the last; vrow_lds the
+// value row, whose pages may have fewer heads), so the tile's loads depend on nothing but
+// LDS and are issued back to back.  NK = 2 stages the rows of the key heads g and g + 1, one
+// tile behind the other, over one value tile.
+template <int DKC, int DVT, bool VEC, int NT, int KT, int NK>
+struct StagedTile {
+  static constexpr int KS = DKC * 32 + 8, VS = KT + 8;
+  static constexpr int TP = KT / 2;           // token pairs
+  static constexpr int KN = NK * KT * DKC * 4, VN = TP * DVT * 2;
+  static constexpr int KIT = (KN + NT - 1) / NT, VIT = (VN + NT - 1) / NT;
+  s16x8 k[KIT], va[VIT], vb[VIT];
+
+  struct From {
+    const u16 *kc, *vc;
+    int page, dk, dv;
+    i64 ldv;
+  };
+  __device__ __forceinline__ void fetch_k(int it, const From& f, const i32* row_lds) {
+    const int i = min(it * NT + (int)threadIdx.x, KN - 1);
     const int tok = i / (DKC * 4), e0 = (i % (DKC * 4)) * 8;
     const int row = row_lds[NK == 1 ? tok : tok % KT];
-    s16x8 v8 = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (row >= 0)
-      v8 = load8<VEC>(kc + (size_t)(NK == 1 ? row : row + tok / KT * page) * dk,
-                      e0, dk);
-    *reinterpret_cast<s16x8*>(k_lds + tok * KS + e0) = v8;
+    const int at = max(row, 0) + (NK == 1 ? 0 : tok / KT * f.page);
+    k[it] = load8<VEC>(f.kc + (size_t)at * f.dk, VEC ? min(e0, f.dk - 8) : e0, f.dk);
+    if (row < 0 || e0 >= f.dk) k[it] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
   }
-  constexpr int VIT = (TP * DVT * 2 + NT - 1) / NT;
-#pragma unroll
-  for (int it = 0; it < VIT; ++it) {
-    const int i = it * NT + threadIdx.x;
-    if (i >= TP * DVT * 2) break;
-    const int tp = i % TP, e0 = (i / TP) * 8;
+  __device__ __forceinline__ void fetch_v(int it, const From& f, const i32* vrow_lds) {
+    const int i = min(it * NT + (int)threadIdx.x, VN - 1);
+    const int tp = i % TP, e0 = (i / TP) * 8, e = VEC ? min(e0, f.dv - 8) : e0;
     const int ra = vrow_lds[tp * 2], rb = vrow_lds[tp * 2 + 1];
-    s16x8 a = {0, 0, 0, 0, 0, 0, 0, 0}, c8 = a;
-    if (ra >= 0) a = load8<VEC>(vc + (size_t)ra * ldv, e0, dv);
-    if (rb >= 0) c8 = load8<VEC>(vc + (size_t)rb * ldv, e0, dv);
+    va[it] = load8<VEC>(f.vc + (size_t)max(ra, 0) * f.ldv, e, f.dv);
+    vb[it] = load8<VEC>(f.vc + (size_t)max(rb, 0) * f.ldv, e, f.dv);
+    if (ra < 0 || e0 >= f.dv) va[it] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    if (rb < 0 || e0 >= f.dv) vb[it] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
+  }
+  __device__ __forceinline__ void store_k(int it, u16* k_lds) const {
+    const int i = it * NT + threadIdx.x;
+    if (i >= KN) return;
+    *reinterpret_cast<s16x8*>(k_lds + i / (DKC * 4) * KS + (i % (DKC * 4)) * 8) = k[it];
+  }
+  __device__ __forceinline__ void store_v(int it, u16* v_lds) const {
+    const int i = it * NT + threadIdx.x;
+    if (i >= VN) return;
+    const int tp = i % TP, e0 = (i / TP) * 8;
 #pragma unroll
     for (int jj = 0; jj < 8; ++jj) {
-      const uint32_t packed = (uint32_t)(unsigned short)a[jj] |
-                              ((uint32_t)(unsigned short)c8[jj] << 16);
+      const uint32_t packed = (uint32_t)(unsigned short)va[it][jj] |
+                              ((uint32_t)(unsigned short)vb[it][jj] << 16);
       *reinterpret_cast<uint32_t*>(v_lds + (e0 + jj) * VS + tp * 2) = packed;
     }
   }
-}
+
+  __device__ __forceinline__ void fetch(const From& f, const i32* row_lds,
+                                        const i32* vrow_lds) {
+#pragma unroll
+    for (int it = 0; it < KIT; ++it) fetch_k(it, f, row_lds);
+#pragma unroll
+    for (int it = 0; it < VIT; ++it) fetch_v(it, f, vrow_lds);
+  }
+  __device__ __forceinline__ void store(u16* k_lds, u16* v_lds) const {
+#pragma unroll
+    for (int it = 0; it < KIT; ++it) store_k(it, k_lds);
+#pragma unroll
+    for (int it = 0; it < VIT; ++it) store_v(it, v_lds);
+  }
+  // both, where registers are short: a few rows at a time, absent ones behind a branch
+  __device__ __forceinline__ void pass_tight(const From& f, const i32* row_lds,
+                                             const i32* vrow_lds, u16* k_lds, u16* v_lds) {
+    const s16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int it = 0; it < KIT; ++it) {
+      const int i = it * NT + threadIdx.x;
+      if (i >= KN) break;
+      const int tok = i / (DKC * 4), e0 = (i % (DKC * 4)) * 8;
+      const int row = row_lds[NK == 1 ? tok : tok % KT];
+      s16x8 v8 = zero;
+      if (row >= 0)
+        v8 = load8<VEC>(f.kc + (size_t)(NK == 1 ? row : row + tok / KT * f.page) * f.dk, e0, f.dk);
+      *reinterpret_cast<s16x8*>(k_lds + tok * KS + e0) = v8;
+    }
+#pragma unroll
+    for (int it = 0; it < VIT; ++it) {
+      const int i = it * NT + threadIdx.x;
+      if (i >= VN) break;
+      const int tp = i % TP, e0 = (i / TP) * 8;
+      const int ra = vrow_lds[tp * 2], rb = vrow_lds[tp * 2 + 1];
+      va[0] = zero, vb[0] = zero;
+      if (ra >= 0) va[0] = load8<VEC>(f.vc + (size_t)ra * f.ldv, e0, f.dv);
+      if (rb >= 0) vb[0] = load8<VEC>(f.vc + (size_t)rb * f.ldv, e0, f.dv);
+#pragma unroll
+      for (int jj = 0; jj < 8; ++jj) {
+        const uint32_t packed = (uint32_t)(unsigned short)va[0][jj] |
+                                ((uint32_t)(unsigned short)vb[0][jj] << 16);
+        *reinterpret_cast<uint32_t*>(v_lds + (e0 + jj) * VS + tp * 2) = packed;
+      }
+    }
+  }
+  // both, a few rows at a time
+  __device__ __forceinline__ void pass(const From& f, const i32* row_lds,
+                                       const i32* vrow_lds, u16* k_lds, u16* v_lds) {
+#pragma unroll
+    for (int it = 0; it < KIT; ++it) { fetch_k(it, f, row_lds); store_k(it, k_lds); }
+#pragma unroll
+    for (int it = 0; it < VIT; ++it) { fetch_v(it, f, vrow_lds); store_v(it, v_lds); }
+  }
+};
 
 // NH = 2: two query heads of one K/V group per workgroup (eight waves), so a
 // staged tile serves both and one head's LDS / MFMA waits hide behind the
@@ -117,8 +187,8 @@ struct DiffTail {
   float lam, diff, eps;
 };
 
-// LITE 1: no chunk, soft cap, distance bias or kept keys (window and sink
-// stay): what those terms keep alive costs the wide instances registers.  LITE
+// LITE 1: no soft cap, distance bias or kept keys (chunk, window and sink
+// stay): what those terms keep alive costs the instances registers.  LITE
 // 2: every earlier key, no distance bias (cap and sink stay): a wave compares
 // positions only in the tiles that reach past its first row.
 template <int DKC, int DVT, bool VEC, int NH, int KT, bool DIFF = false,
@@ -136,7 +206,10 @@ __device__ __forceinline__ void attn_prefill_mfma_body(
   constexpr int NST = KT / 16;       // 16-key sub-tiles
   constexpr int NHF = KT / 32;       // 32-key halves of P V
   constexpr int NK = DIFF ? 2 : 1;
-  const int chunk = LITE ? 0 : chunk_in, first = LITE ? 0 : ex.first;
+  // a tile's rows are fetched while the one before is worked on, where the registers are
+  // there for it; the widest heads keep nothing that can be computed again
+  constexpr bool AHEAD = DKC <= 4 && NH == 1, TIGHT = DKC > 10;
+  const int chunk = LITE == 2 ? 0 : chunk_in, first = LITE ? 0 : ex.first;
   const int window = LITE == 2 ? 0 : window_in;
   const bool biased = !LITE && ex.r1, capped = LITE != 1 && ex.cap > 0.f;
   constexpr int XS = DVT * 16 + 4;   // row stride of the maps' exchange (floats)
@@ -149,7 +222,7 @@ __device__ __forceinline__ void attn_prefill_mfma_body(
   __shared__ u16 p_lds[NH * 4 * 16 * VS];
   __shared__ float bias_lds[LITE ? 1 : NH * 128];  // distance bias of this tile's distances
   // page rows of every key of the tile
-  __shared__ i32 row_lds[KT], vrow_lds[KT];
+  __shared__ i32 row_lds[2][KT], vrow_lds[2][KT];
 
   const int hsel = threadIdx.x >> 8;           // which of the NH heads (maps)
   // DIFF: H, G count heads and K/V heads, blockIdx.y is the head; h and g are
@@ -207,12 +280,65 @@ __device__ __forceinline__ void attn_prefill_mfma_body(
   const int nfirst = (first > 0 && lo > 0) ? min(first, lo) : 0;
   const int a_end = (nfirst + KT - 1) / KT * KT;
   const int b0 = max(lo, a_end);
-  for (int kv0 = nfirst > 0 ? 0 : lo; kv0 <= p_last;
-       kv0 = (kv0 < a_end && kv0 + KT >= a_end) ? b0 : kv0 + KT) {
+  auto after = [&](int kv0) {
+    return kv0 < a_end && kv0 + KT >= a_end ? b0 : kv0 + KT;
+  };
+  // a key's rows in the pages, for the threads that look one up per tile
+  const int sh = page & (page - 1) ? -1 : __ffs(page) - 1;
+  i32 krow = -1, vrow = -1;
+  auto look_up = [&](int kv0) {
+    const int j = kv0 + threadIdx.x;
+    krow = vrow = -1;
+    if ((int)threadIdx.x >= KT || j > p_last) return;
+    const int pi = sh >= 0 ? j >> sh : j / page, off = j - pi * page, pg = btr[pi];
+    krow = (pg * GK + g) * page + off;
+    vrow = (pg * GV + gv) * page + off;
+  };
+  auto note = [&](int at) {
+    if (threadIdx.x < KT) {
+      row_lds[at][threadIdx.x] = krow;
+      vrow_lds[at][threadIdx.x] = vrow;
+    }
+  };
+  using Staged = StagedTile<DKC, DVT, VEC, 256 * NH, KT, NK>;
+  const typename Staged::From from{kc, vc, page, dk, dv, ex.ldv};
+  Staged staged;
+  // what a row (of the wave) sees first of its chunk and window
+  auto sees_from = [&](int p) {
+    const int c = chunk > 0 ? p / chunk * chunk : 0;
+    return window > 0 ? max(c, p - window + 1) : c;
+  };
+  int rows_from[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) rows_from[r] = sees_from(wp0 + (lane >> 4) * 4 + r);
+  const int wave_from = sees_from(wp_last);
+  // Pages are looked up two tiles ahead and (AHEAD) rows fetched one ahead, both while the
+  // tile before is worked on.
+  int kv0 = nfirst > 0 ? 0 : lo, at = 0;
+  if (!TIGHT) {
+    look_up(kv0);
+    note(0);
+    look_up(after(kv0));
+    note(1);
+    __syncthreads();
+  }
+  if (AHEAD) staged.fetch(from, row_lds[0], vrow_lds[0]);
+  for (; kv0 <= p_last; kv0 = after(kv0), at ^= 1) {
     __syncthreads();   // fragment reads of the previous tile are done
-    stage_kv_tile<DKC, DVT, VEC, 256 * NH, KT, NK>(
-        k_lds, v_lds, row_lds, vrow_lds, kc, vc, btr, kv0, p_last, GK, g, GV,
-        gv, page, dk, dv, ex.ldv);
+    if (AHEAD) {
+      staged.store(k_lds, v_lds);
+      if (after(kv0) <= p_last) staged.fetch(from, row_lds[at ^ 1], vrow_lds[at ^ 1]);
+    } else {
+      if (TIGHT) {
+        look_up(kv0);
+        note(at);
+        __syncthreads();
+        staged.pass_tight(from, row_lds[at], vrow_lds[at], k_lds, v_lds);
+      } else {
+        staged.pass(from, row_lds[at], vrow_lds[at], k_lds, v_lds);
+      }
+    }
+    if (!TIGHT) look_up(after(after(kv0)));
     // distance bias for every distance between a row and a key of the tile:
     // entry i is distance i + (p0 - kv0 - (KT-1)); keys ahead of a row are masked
     if (biased && (threadIdx.x & 255) < 63 + KT) {     // each head its own table
@@ -221,6 +347,8 @@ __device__ __forceinline__ void attn_prefill_mfma_body(
           dist > 0 ? attn_dist_bias(r1, r2, dist) : 0.f;
     }
     __syncthreads();
+    // the tile's own rows have been fetched: their place is free
+    if (!TIGHT) note(at);
     // keys of this tile that any row of the wave may see
     if (!wave_live || kv0 > wp_last) continue;
     if (window > 0 && kv0 + KT - 1 <= wp0 - window && kv0 >= first) continue;
@@ -240,13 +368,12 @@ __device__ __forceinline__ void attn_prefill_mfma_body(
       }
     }
     // ---- mask + online softmax; reg r is row (lane>>4)*4 + r ----
-    const bool all_seen = LITE == 2 && kv0 + KT - 1 <= wp0;
+    const bool all_seen = kv0 + KT - 1 <= wp0 &&
+                          (LITE == 2 || (!TIGHT && kv0 >= wave_from));
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int p = wp0 + (lane >> 4) * 4 + r;
-      int rlo = 0;
-      if (chunk > 0) rlo = (p / chunk) * chunk;
-      if (window > 0) rlo = max(rlo, p - window + 1);
+      const int from_r = TIGHT ? sees_from(p) : rows_from[r];
       float sr[NST];
       float tmax = AF_NEG_INF;
 #pragma unroll
@@ -255,8 +382,9 @@ __device__ __forceinline__ void attn_prefill_mfma_body(
         float sv = s_acc[st][r] * scale;
         if (capped) sv = attn_softcap_fast(sv, inv_cap, ex.cap);
         if (biased) sv -= bias_lds[hsel * 128 + (p - p0) - (j - kv0) + KT - 1];
-        sr[st] = (all_seen || (j <= p && (LITE == 2 || j >= rlo || j < first)))
-                     ? sv : AF_NEG_INF;
+        sr[st] = sv;
+        if (!all_seen)
+          sr[st] = j <= p && (LITE == 2 || j >= from_r || j < first) ? sv : AF_NEG_INF;
         tmax = fmaxf(tmax, sr[st]);
       }
       tmax = group16_max_f32(tmax);
@@ -279,7 +407,7 @@ __device__ __forceinline__ void attn_prefill_mfma_body(
     for (int st = 0; st < NST; ++st)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        pw[((lane >> 4) * 4 + r) * VS + st * 16 + (lane & 15)] = f2bf(s_acc[st][r]);
+        pw[((lane >> 4) * 4 + r) * VS + st * 16 + (lane & 15)] = to_bf16<TIGHT>(s_acc[st][r]);
     __builtin_amdgcn_wave_barrier();
     s16x8 pf[NHF];
 #pragma unroll
@@ -335,7 +463,7 @@ __device__ __forceinline__ void attn_prefill_mfma_body(
         if (d < dv) {
           float v = o_acc[dt][r] * f;
           if (df.gate) v *= __frcp_rn(1.0f + __expf(-bf2f(gp[d])));
-          op[d] = f2bf(v);
+          op[d] = to_bf16<TIGHT>(v);
         }
       }
     }
@@ -351,7 +479,7 @@ __device__ __forceinline__ void attn_prefill_mfma_body(
 #pragma unroll
     for (int dt = 0; dt < DVT; ++dt) {
       const int d = dt * 16 + (lane & 15);
-      if (d < dv) op[d] = f2bf(o_acc[dt][r] * inv);
+      if (d < dv) op[d] = to_bf16<TIGHT>(o_acc[dt][r] * inv);
     }
   }
 }
@@ -368,7 +496,7 @@ __device__ __forceinline__ void attn_prefill_mfma_body(
     page, maxp, chunk, window, ldq, ex
 
 template <int DKC, int DVT, bool VEC, int NH, int KT = 64, int LITE = 0>
-__global__ void __launch_bounds__(256 * NH) attn_prefill_mfma_kernel(AF_APM_PARAMS) {
+__global__ void __launch_bounds__(256 * NH, (DKC <= 4 && NH == 2 ? 4 : 1)) attn_prefill_mfma_kernel(AF_APM_PARAMS) {
   attn_prefill_mfma_body<DKC, DVT, VEC, NH, KT, false, LITE>(AF_APM_ARGS);
 }
 
@@ -638,8 +766,8 @@ AF_EXPORT int afm_attn_prefill_mfma(
                      cap, ldv, keep_first, vshare, gate, ldg, ldo};
   // two heads per workgroup when a K/V group has an even number of them
   const bool pair = vec && (H / G) % 2 == 0;
-  const bool plain = chunk <= 0 && !r1 && keep_first == 0;
-  const bool lite = plain && cap <= 0.f, causal = plain && window <= 0;
+  const bool plain = !r1 && keep_first == 0;
+  const bool lite = plain && cap <= 0.f, causal = plain && chunk <= 0 && window <= 0;
   hipStream_t s = (hipStream_t)stream;
 #define APM(DKC, DVT, VEC, NH, ...)                                            \
   attn_prefill_mfma_kernel<DKC, DVT, VEC, NH, ##__VA_ARGS__>                   \
@@ -669,6 +797,7 @@ AF_EXPORT int afm_attn_prefill_mfma(
   else if (small && vec) APM(2, 4, true, 1);
   else if (small) APM(2, 4, false, 1);
   else if (pair && causal) APM(4, 8, true, 2, 64, 2);
+  else if (pair && lite) APM(4, 8, true, 2, 64, 1);
   else if (pair) APM(4, 8, true, 2);
   else if (vec) APM(4, 8, true, 1);
   else APM(4, 8, false, 1);

@@ -294,6 +294,35 @@ def test_row_attention_on_every_lane_layout(dtype, H, G, dk, dv, page, odd, monk
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,G,dk,dv,page", [
+    (4, 2, 128, 128, 16), (3, 3, 128, 128, 8), (4, 2, 64, 64, 16), (3, 1, 64, 56, 5),
+    (2, 1, 100, 90, 7), (2, 1, 256, 256, 16), (1, 1, 264, 136, 6), (2, 1, 576, 512, 16),
+    (1, 1, 576, 512, 16)])
+@pytest.mark.parametrize("chunk,window,cap", [(0, 0, 0.), (96, 0, 0.), (0, 70, 0.),
+                                              (64, 40, 0.), (100, 0, 5.)])
+def test_prompt_attention_of_every_instance(H, G, dk, dv, page, chunk, window, cap):
+    """Prompts that end inside and on a tile, behind a history or not, through every
+    instance of the tile kernel: chunks and windows that begin inside and on a tile, pages of
+    a power of two of keys and others.  Weights are rounded to bf16 (2^-9 of values below
+    max |v|), and so is the result."""
+    torch.manual_seed(dk + chunk)
+    lens, starts = [64, 130, 33], [0, 37, 200]
+    B, T, maxp = len(lens), sum(lens), 260 // page + 1
+    kc = torch.randn(B * maxp + 1, G, page, dk).bfloat16()
+    vc = torch.randn(B * maxp + 1, G, page, dv).bfloat16()
+    q = torch.randn(T, H * dk).bfloat16()
+    md, pos = md_for(lens, starts, [1] * B, "cpu", page, maxp)
+    on = SimpleNamespace(**{k: v.cuda() if torch.is_tensor(v) else v
+                            for k, v in vars(md).items()})
+    got = sm.masked_attention(q.cuda(), kc.cuda(), vc.cuda(), on, pos.cuda(), dk ** -0.5,
+                              H, chunk=chunk, window=window, softcap=cap).cpu()
+    want = sm.masked_attention(q, kc, vc, md, pos, dk ** -0.5, H, chunk=chunk,
+                               window=window, softcap=cap)
+    assert ((got.float() - want.float()).abs()
+            <= 2 ** -9 * vc.abs().max() + 2 ** -8 * want.abs()).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("W", [4, 1020, 2048, 2052, 4096, 4100, 8192, 8196, 1023])
 def test_row_kernels_around_their_register_rows(dtype, W):
