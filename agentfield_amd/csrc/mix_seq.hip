@@ -695,26 +695,56 @@ __global__ void __launch_bounds__(256) diff_combine_kernel(
 // linear_scan_kernel, few tokens per sequence: bound by moving the state; thread
 // (r, c) = (tid >> 4, tid & 15) has columns c and c + 16, so that a state row
 // moves in 64-byte pieces; partial outputs meet in LDS after the block of tokens.
-// linear_scan_prompt_kernel: with few workgroups bound by vector instructions, 40 per
-// token and wave on two waves per SIMD beside the staging (a fifth); the row groups are
+// linear_scan_prompt_kernel: with few workgroups bound by vector instructions, 28 per
+// token and wave on two waves per SIMD beside the staging (a quarter); the row groups are
 // the 16 lanes of a DPP row, so the sum over rows needs no LDS and no second barrier.  A
 // constant decay is not staged.  Its workgroups are four or eight waves, see launch_scan.
-// Six sequences of 500..1900 tokens, 8 heads of 128 x 128, decays per channel:
-// 787 -> 336 us; 16 heads, one decay per head, rotary: 770 -> 447 us (four waves, two
-// columns per thread, 385 and 497; the row layout alone 711 and 698; element loads that
-// were converted at once made every block wait for its successor).
-// v plus the sum over the other lanes of its 16-lane row, in all of them
+// Six sequences of 620..1900 tokens, 8 heads of 128 x 128, decays per channel:
+// 787 -> 308 us; 16 heads, one decay per head, rotary: 770 -> 296 us (the row layout alone
+// 711 and 698; four waves, two columns per thread, 350 and 333; element loads that were
+// converted at once made every block wait for its successor).
+// The 16 row groups of a token are summed as a tree: j with 15 - j, of the eight sums j with
+// 7 - j, of the four 0 with 2 and 1 with 3, then the two.  In a 16-lane row these are mirrors
+// and exchanges within quads; row16_sum_all leaves the sum in all lanes.
 __device__ __forceinline__ float row16_sum_all(float v) {
-#define AFM_ROR(N)                                                           \
-  v += __int_as_float(__builtin_amdgcn_update_dpp(                           \
-      0, __float_as_int(v), 0x120 + N, 0xf, 0xf, true));
-  AFM_ROR(8)
-  AFM_ROR(4)
-  AFM_ROR(2)
-  AFM_ROR(1)
-#undef AFM_ROR
+  v += dpp_f32<0x140>(v);
+  v += dpp_f32<0x141>(v);
+  v += dpp_f32<0x4E>(v);
+  v += dpp_f32<0xB1>(v);
   return v;
 }
+
+// The same sums of a block of tokens, each lane one token's: of every two tokens (then sums of
+// two, four and eight lanes) a lane hands its partner the one that the partner goes on with,
+// 15 additions for 16 tokens instead of 64.  DPP operands run at half rate, so the sums were a
+// quarter of the prompt kernel's vector time: one sequence of 1900 tokens, 16 heads of 128
+// 284 -> 240 us; 6 of 620..1900, 8 heads with decays per channel 337 -> 308.  (Each two tokens
+// at once, with three values waiting instead of eight, 315.)
+template <int TB>
+struct Row16Sums {
+  float p[8], sum;
+  // tokens tt = 0 .. TB-1 in turn, tt known when compiled; sum is the lane's after the last
+  __device__ __forceinline__ void add(int tt, float part, int lane) {
+    const bool b3 = lane & 8, b2 = lane & 4, b1 = lane & 2, b0 = lane & 1;
+    p[tt & 7] = part;
+    if ((tt & 7) != 7) return;
+    float s[4], u[2];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      s[t] = (b3 ? p[2 * t + 1] : p[2 * t]) + dpp_f32<0x140>(b3 ? p[2 * t] : p[2 * t + 1]);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      u[t] = (b2 ? s[2 * t + 1] : s[2 * t]) + dpp_f32<0x141>(b2 ? s[2 * t] : s[2 * t + 1]);
+    const float v = (b1 ? u[1] : u[0]) + dpp_f32<0x4E>(b1 ? u[0] : u[1]);
+    if (TB == 8) sum = v + dpp_f32<0xB1>(v);
+    else if (!(tt & 8)) sum = v;
+    else sum = (b0 ? v : sum) + dpp_f32<0xB1>(b0 ? sum : v);
+  }
+  // the token whose sum a lane has (TB == 8: from 8 on, nobody's)
+  static __device__ __forceinline__ int token_of(int lane) {
+    return (lane >> 3 & 1) | (lane >> 1 & 2) | (lane << 1 & 4) | (lane << 3 & 8);
+  }
+};
 
 // The arithmetic of both kernels, every rounding spelled out: contraction is the
 // compiler's choice per place otherwise, and a sequence's results must not depend
@@ -920,10 +950,11 @@ __global__ void __launch_bounds__(256) linear_scan_kernel(
 #pragma unroll
         for (int rr = 0; rr < 16; ++rr) o[rr] = pr[rr * 32];
 #pragma unroll
-        for (int n = 8; n > 0; n >>= 1)
+        for (int rr = 0; rr < 8; ++rr) o[rr] += o[15 - rr];
 #pragma unroll
-          for (int rr = 0; rr < n; ++rr) o[rr] += o[rr + n];
-        out[(size_t)(tb + tt) * H * dv + (size_t)h * dv + c0 + ci] = o[0];
+        for (int rr = 0; rr < 4; ++rr) o[rr] += o[7 - rr];
+        out[(size_t)(tb + tt) * H * dv + (size_t)h * dv + c0 + ci] =
+            (o[0] + o[2]) + (o[1] + o[3]);
       }
     }
     // the next block's staging writes `stage`/`vs`, last read before the
@@ -956,7 +987,8 @@ __device__ __forceinline__ ScanRows scan_sequence(const i32* __restrict__ cu) {
   const int lane = min((int)threadIdx.x & 63, B - 1);
   const int from = cu[lane], len = cu[lane + 1] - from;
   // (lengths alike: nothing to win, and the ranks cost short ones 1 us of 48)
-  if (wave_max_f32((float)len) + wave_max_f32((float)-len) < 64.f)
+  if (__builtin_amdgcn_readfirstlane(wave_max_f32((float)len) +
+                                     wave_max_f32((float)-len) < 64.f))
     return {turn, __builtin_amdgcn_readlane(from, turn),
             __builtin_amdgcn_readlane(from, turn) + __builtin_amdgcn_readlane(len, turn)};
   int rank = 0;
@@ -972,10 +1004,10 @@ __device__ __forceinline__ ScanRows scan_sequence(const i32* __restrict__ cu) {
 // The same recurrence for prompts.  A thread stages E consecutive rows of one token
 // (one wide load each for q, k, the rotary partners and the decay logits, kept raw
 // until the block before has been worked through) and computes RP rows of one column
-// (NT = 512) or two (256); lane j of a 16-lane row keeps token j's sum.  Two LDS
+// (NT = 512) or two (256); each lane of a 16-lane row keeps one token's sum.  Two LDS
 // buffers, one barrier per block of tokens.
 template <typename S, int RP, bool ZL, int NT>
-__global__ void __launch_bounds__(NT, NT == 512 && RP == 8 && sizeof(S) == 2 ? 4 : 2)
+__global__ void __launch_bounds__(NT, RP == 8 && sizeof(S) == 2 ? (NT == 512 ? 4 : 3) : 2)
 linear_scan_prompt_kernel(
     float* __restrict__ out, float* __restrict__ state,
     const S* __restrict__ q, const S* __restrict__ k, const S* __restrict__ v,
@@ -993,7 +1025,9 @@ linear_scan_prompt_kernel(
   constexpr int BUF = TB * (3 * DKP + 32);     // [TB][3][DKP], [TB][32]
   extern __shared__ float smem[];
   const ScanRows rows = scan_sequence(cu);
-  const int b = rows.b, t0 = rows.t0, t1 = rows.t1;
+  const int b = __builtin_amdgcn_readfirstlane(rows.b);   // (known to be alike in all lanes)
+  const int t0 = __builtin_amdgcn_readfirstlane(rows.t0);
+  const int t1 = __builtin_amdgcn_readfirstlane(rows.t1);
   const int h = blockIdx.x, c0 = blockIdx.y * 32;
   if (t1 <= t0) return;
   const int r = threadIdx.x & 15, cc = threadIdx.x >> 4;
@@ -1007,7 +1041,7 @@ linear_scan_prompt_kernel(
 #pragma unroll
     for (int c = 0; c < CPT; ++c)
       state_of[c][ii] = (!fresh && ca + c < dv && i < dk)
-                            ? sbase[(size_t)i * dv + ca + c] : 0.f;
+                            ? sbase[i * dv + ca + c] : 0.f;
   }
 
   // what this thread stages: rows i0 .. i0+E-1 of token st of a block, and two
@@ -1164,8 +1198,7 @@ linear_scan_prompt_kernel(
       }
       return t;
     };
-    auto step = [&](int tt, const Token& t) {
-      float part[CPT];
+    auto step = [&](const Token& t, float (&part)[CPT]) {
 #pragma unroll
       for (int c = 0; c < CPT; ++c) part[c] = 0.f;
 #pragma unroll
@@ -1173,27 +1206,39 @@ linear_scan_prompt_kernel(
 #pragma unroll
         for (int c = 0; c < CPT; ++c)
           scan_row(state_of[c][ii], part[c], t.a[ii], t.k[ii], t.v[c], t.q[ii]);
-#pragma unroll
-      for (int c = 0; c < CPT; ++c) part[c] = row16_sum_all(part[c]);
-#pragma unroll
-      for (int c = 0; c < CPT; ++c) o[c] = r == tt ? part[c] : o[c];
     };
+    // a lane keeps the sums of token `mine`
+    const int mine = Row16Sums<TB>::token_of(r);
     if (nt == TB) {
       // the next token's LDS reads run under this one's arithmetic: the fence keeps
       // them there, the one or two waves of a SIMD do not hide them otherwise
       Token t[2];
+      Row16Sums<TB> sums[CPT];
       t[0] = read(0);
 #pragma unroll
       for (int tt = 0; tt < TB; ++tt) {
         if (tt + 1 < TB) t[(tt + 1) & 1] = read(tt + 1);
         __builtin_amdgcn_sched_barrier(0);
-        step(tt, t[tt & 1]);
+        float part[CPT];
+        step(t[tt & 1], part);
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) sums[c].add(tt, part[c], r);
       }
+#pragma unroll
+      for (int c = 0; c < CPT; ++c) o[c] = sums[c].sum;
     } else {
-      for (int tt = 0; tt < nt; ++tt) step(tt, read(tt));
+      for (int tt = 0; tt < nt; ++tt) {
+        float part[CPT];
+        step(read(tt), part);
+#pragma unroll
+        for (int c = 0; c < CPT; ++c) {
+          part[c] = row16_sum_all(part[c]);
+          o[c] = mine == tt ? part[c] : o[c];
+        }
+      }
     }
-    if (r < nt) {
-      float* op = out + (size_t)(tb + r) * H * dv + (size_t)h * dv;
+    if (mine < nt) {
+      float* op = out + (size_t)(tb + mine) * H * dv + (size_t)h * dv;
 #pragma unroll
       for (int c = 0; c < CPT; ++c)
         if (ca + c < dv) op[ca + c] = o[c];
@@ -1206,7 +1251,7 @@ linear_scan_prompt_kernel(
     const int i = r * RP + ii;
 #pragma unroll
     for (int c = 0; c < CPT; ++c)
-      if (i < dk && ca + c < dv) sbase[(size_t)i * dv + ca + c] = state_of[c][ii];
+      if (i < dk && ca + c < dv) sbase[i * dv + ca + c] = state_of[c][ii];
   }
 }
 
@@ -1434,16 +1479,16 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
   };
   // From 128 rows on with eight waves, which fill one another's waits, while that leaves
   // a workgroup or two to a CU; beyond, four waves do it with fewer instructions.  Four /
-  // eight waves in us, decays per channel, bf16: 128 rows, 192 groups 110 / 96, 384 groups
-  // 542 / 537, 768 766 / 837, 4096 135 / 150; 256 rows, 64 groups 723 / 673, 384 279 / 348.
-  // fp32: 128 rows, 192 groups 172 / 137, 384 835 / 894; one decay per head 574 / 479 and,
-  // 8192 groups, 1300 / 1199.  What only eight waves can load (rows in fours) is, on many
-  // groups, better off with them than with the token kernel in bf16 at 128 rows (dk 100,
-  // 17 tokens 90 / 75), otherwise for longer prompts (fp32 17 tokens 104 / 151, 75 tokens
-  // 219 / 229, 225 tokens 1148 / 1138).
+  // eight waves in us, sequences of 300 tokens, 128 rows: decays per channel, 192 groups
+  // 67 / 61, 384 95 / 97 (of 50..1900 tokens 350 / 318), 768 133 / 149, 4096 585 / 679; one
+  // decay per head 61 / 50, 85 / 80, 118 / 122, 530 / 579; 256 rows, 64 groups 113 / 107,
+  // 384 179 / 221.  fp32: 128 rows, 192 groups 101 / 82, 384 140 / 153; one decay per head
+  // 73 / 55, 96 / 88, 768 133 / 136, 4096 609 / 640.  What only eight waves can load (rows in
+  // fours) is, on many groups, better off with them than with the token kernel in bf16 at 128
+  // rows (dk 100, 17 tokens 27 / 25), otherwise for longer prompts (fp32 17 tokens 32 / 44, 75
+  // tokens 97 / 98, 225 tokens 265 / 253).
   const i64 groups = (i64)B * H * grid.z;
-  const bool few = rpp >= 16 || (sizeof(S) == 4 && zl)
-                       ? groups <= 256 : sizeof(S) == 4 || groups <= 512;
+  const bool few = groups <= (rpp >= 16 || (sizeof(S) == 4 && zl) ? 256 : 512);
   const bool eight = rpp >= 8 && loads(512) &&
                      (few || (!loads(256) && ((rpp == 8 && sizeof(S) == 2) ||
                                               T >= 128 * B)));
