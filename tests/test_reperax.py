@@ -324,6 +324,27 @@ def test_prompt_attention_of_every_instance(H, G, dk, dv, page, chunk, window, c
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dv", [4, 20, 64, 68, 128, 132, 256, 260, 33])
+def test_headnorm_gate_on_its_lanes(dtype, dv):
+    """Heads on 16, 32 and 64 lanes, in part and in whole, and the lengths beyond; more
+    and fewer heads than a block takes.  Both results are rounded (2^-7 of the value in bf16,
+    as two may fall on the sides of a tie), sums and exponentials in fp32."""
+    torch.manual_seed(dv)
+    rel = 2 ** -7 if dtype == torch.bfloat16 else 2 ** -18
+    for T, H in ((1, 1), (7, 3), (33, 8)):
+        o = torch.randn(T, H * dv)
+        g = torch.randn(T, H * dv + 8).to(dtype)[:, :H * dv]
+        for w in (None, torch.randn(dv).to(dtype)):
+            for act in ("silu", "sigmoid"):
+                want = sm.headnorm_gate(o, g, w, 1e-6, H, dtype, act).float()
+                gd = torch.empty(T, H * dv + 8, dtype=dtype, device="cuda")[:, :H * dv]
+                got = sm.headnorm_gate(o.cuda(), gd.copy_(g), None if w is None else w.cuda(),
+                                       1e-6, H, dtype, act).float().cpu()
+                assert ((got - want).abs() <= want.abs() * rel + 2 ** -20).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("W", [4, 1020, 2048, 2052, 4096, 4100, 8192, 8196, 1023])
 def test_row_kernels_around_their_register_rows(dtype, W):
     """Rows that stay in registers in whole, in part, or are read again, in steps of four
