@@ -148,6 +148,7 @@ class AttnMetadata:
     decode_scratch: tuple | None = None
     state_slots: torch.Tensor | None = None
     row_seq: torch.Tensor | None = None
+    step_tiles: tuple | None = None     # row tiles that the step's layers share
 
 
 class KVCache:

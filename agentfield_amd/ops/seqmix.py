@@ -249,6 +249,18 @@ def qk_norm_cache(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     return out
 
 
+def _on_device(device, *lists):
+    """Equally long int32 lists on the device, without waiting for what is queued on the
+    stream: a tensor built there from a list waits for all of it.  Not while a graph is
+    recorded, whose copy would outlive the host's memory: built as any other there, which
+    the recording refuses."""
+    if device.type != "cuda" or torch.cuda.is_current_stream_capturing():
+        return [torch.tensor(v, dtype=torch.int32, device=device) for v in lists]
+    host = torch.empty(len(lists), len(lists[0]), dtype=torch.int32, pin_memory=True)
+    host.numpy()[:] = lists
+    return host.to(device, non_blocking=True).unbind(0)
+
+
 def _row_tiles(lens, rows: int, device):
     """Tile map of packed chunks for the tile kernels: (tiles, sequence of
     every tile, its first row inside the chunk).  Late rows see the most keys
@@ -256,11 +268,23 @@ def _row_tiles(lens, rows: int, device):
     which spreads them over the XCDs and keeps each one's keys in few L2s."""
     tiles = sorted((-q0, b) for b, ln in enumerate(lens)
                    for q0 in range(0, ln, rows))
-    return (len(tiles),
-            torch.tensor([b for _q, b in tiles], dtype=torch.int32,
-                         device=device),
-            torch.tensor([-q for q, _b in tiles], dtype=torch.int32,
-                         device=device))
+    return (len(tiles), *_on_device(device, [b for _q, b in tiles],
+                                    [-q for q, _b in tiles]))
+
+
+def _step_tiles(md, rows: int, device):
+    """_row_tiles of the step that md describes, which its layers share: kept there for
+    the lengths, the device and the stream they were made for.  Six prompts of 7636 rows of
+    the 1b hybrid: the host waited for each of the eight attention layers, 12 ms for
+    the step that now takes it 4.1, and with six decode steps behind it the host was what
+    28.7 ms were spent on, 28.0 now (19 of them the host's)."""
+    if device.type != "cuda" or torch.cuda.is_current_stream_capturing():
+        return _row_tiles(md.seq_lens, rows, device)
+    key = (tuple(md.seq_lens), rows, device, _lib.cur_stream())
+    kept = getattr(md, "step_tiles", None)
+    if kept is None or kept[0] != key:
+        kept = md.step_tiles = (key, _row_tiles(md.seq_lens, rows, device))
+    return kept[1]
 
 
 def masked_attention(q: torch.Tensor, kcache: torch.Tensor,
@@ -341,7 +365,7 @@ def masked_attention(q: torch.Tensor, kcache: torch.Tensor,
     if (q.dtype == torch.bfloat16 and lens is not None and dk <= 576
             and dv <= 512 and max(lens) >= MFMA_MIN_ROWS):
         # prompt portions: 64-row tiles on the matrix cores
-        nt, tile_seq, tile_q0 = _row_tiles(lens, 64, q.device)
+        nt, tile_seq, tile_q0 = _step_tiles(md, 64, q.device)
         rc = _L().afm_attn_prefill_mfma(
             _lib.ptr(out), _lib.ptr(q), _lib.ptr(kcache), _lib.ptr(vsrc),
             _lib.ptr(md.block_table), _lib.ptr(md.cu_seqlens),
@@ -444,7 +468,7 @@ def diff_attention(q: torch.Tensor, kcache: torch.Tensor,
             and dv <= 256 and max(lens) >= MFMA_MIN_ROWS):
         # prompt portions: both maps of a head in one workgroup, combined,
         # normed and gated before they leave it
-        nt, tile_seq, tile_q0 = _row_tiles(lens, 64, q.device)
+        nt, tile_seq, tile_q0 = _step_tiles(md, 64, q.device)
         rc = _L().afm_diff_prefill_mfma(
             _lib.ptr(out), _lib.ptr(q), _lib.ptr(kcache), _lib.ptr(vcache),
             _lib.ptr(md.block_table), _lib.ptr(md.cu_seqlens),
@@ -1224,8 +1248,7 @@ def sigmoid_attention(q: torch.Tensor, kcache: torch.Tensor,
             for q0 in range(0, ln, 16):
                 ts.append(b)
                 tq.append(q0)
-        tile_seq = torch.tensor(ts, dtype=torch.int32, device=q.device)
-        tile_q0 = torch.tensor(tq, dtype=torch.int32, device=q.device)
+        tile_seq, tile_q0 = _on_device(q.device, ts, tq)
         rc = _L().afm_sigattn_prefill_mfma(
             _lib.ptr(out), _lib.ptr(q), _lib.ptr(kcache), _lib.ptr(vcache),
             _lib.ptr(md.block_table), _lib.ptr(md.cu_seqlens),

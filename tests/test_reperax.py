@@ -323,6 +323,28 @@ def test_prompt_attention_of_every_instance(H, G, dk, dv, page, chunk, window, c
 
 
 @pytest.mark.gpu
+def test_row_tiles_of_a_step():
+    """The tile map that a step's layers share is that of its own lengths, stream and
+    device, whatever was asked before, and the one a call without a step makes."""
+    md = SimpleNamespace(seq_lens=[130, 1, 64])
+
+    def tiles(got):
+        return got[0], got[1].tolist(), got[2].tolist()
+    dev = torch.device("cuda", 0)
+    first = sm._step_tiles(md, 64, dev)
+    assert sm._step_tiles(md, 64, dev) is first
+    assert tiles(first) == tiles(sm._row_tiles([130, 1, 64], 64, torch.device("cpu")))
+    assert tiles(first) == (5, [0, 0, 0, 1, 2], [128, 64, 0, 0, 0])
+    md.seq_lens[1] = 70                      # in place
+    assert tiles(sm._step_tiles(md, 64, dev)) == (
+        6, [0, 0, 1, 0, 1, 2], [128, 64, 64, 0, 0, 0])
+    assert tiles(sm._step_tiles(md, 16, dev))[0] == 18
+    kept = sm._step_tiles(md, 64, dev)
+    with torch.cuda.stream(torch.cuda.Stream()):
+        assert sm._step_tiles(md, 64, dev) is not kept
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("dv", [4, 20, 64, 68, 128, 132, 256, 260, 33])
 def test_headnorm_gate_on_its_lanes(dtype, dv):
