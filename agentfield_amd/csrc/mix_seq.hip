@@ -792,7 +792,10 @@ __device__ __forceinline__ void scan_row(float& st, float& o, float a, float k,
   o = fmaf(st, q, o);
 }
 
-template <typename S, int RP>
+// SCAN_TB: tokens of a block, 16 (8: keeps LDS under 64 KB), or one for decode steps, which
+// staged the other 15 for nothing and held LDS for them (16 heads of 128 x 128, 6 rows 6.6 ->
+// 5.2 us, 64 rows 39.8 -> 26.8, 5 TB/s).
+template <typename S, int RP, int SCAN_TB>
 __global__ void __launch_bounds__(256) linear_scan_kernel(
     float* __restrict__ out, float* __restrict__ state,
     const S* __restrict__ q, const S* __restrict__ k, const S* __restrict__ v,
@@ -806,7 +809,6 @@ __global__ void __launch_bounds__(256) linear_scan_kernel(
   // bf16 operands carry 2^-9 relative rounding already: hardware
   // transcendentals there; fp32 storage keeps the precise library forms
   constexpr bool FAST = sizeof(S) == 2;
-  constexpr int SCAN_TB = RP >= 16 ? 8 : 16;  // keeps LDS under 64 KB
   extern __shared__ float smem[];      // [TB][3][DKP] + [TB][16][32] + [TB][32]
   const int b = blockIdx.x, h = blockIdx.y, c0 = blockIdx.z * 32;
   const int t0 = cu[b], t1 = cu[b + 1];
@@ -829,7 +831,7 @@ __global__ void __launch_bounds__(256) linear_scan_kernel(
   const float hd = head_decay ? head_decay[h] : 1.0f;
   const int half = rot >> 1;
   // raw operands of the next block, fetched while the current one computes
-  constexpr int EPT = SCAN_TB * DKP / 256;   // staged elements per thread
+  constexpr int EPT = (SCAN_TB * DKP + 255) / 256;   // staged elements per thread
   float rq[EPT], rk[EPT], rqp[EPT], rkp[EPT], rz[EPT], rpos[EPT];
   float rv[(SCAN_TB * 32 + 255) / 256];
   // Every load is unconditional on a clamped address (invalid lanes are
@@ -1499,7 +1501,8 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
                      (few || (!loads(256) && ((rpp == 8 && sizeof(S) == 2) ||
                                               T >= 128 * B)));
   const bool prompt = eight || loads(256);
-  const size_t sm = (size_t)(rpp >= 16 ? 8 : 16) * sizeof(float) *
+  const bool single = !prompt && T <= B;   // a token per sequence, as a rule
+  const size_t sm = (size_t)(single ? 1 : rpp >= 16 ? 8 : 16) * sizeof(float) *
                     (prompt ? 2 * (3 * 16 * rpp + 32) : 3 * 16 * rpp + 512 + 32);
 #define SCAN_ARGS                                                            \
       out, state, (const S*)q, (const S*)k, (const S*)v, (const S*)zl, zbias, \
@@ -1518,8 +1521,11 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
   do {                                                                       \
     if (eight) SCAN_PROMPT((RP >= 8 ? RP : 8), 512);                         \
     else if (prompt) SCAN_PROMPT(RP, 256);                                   \
+    else if (single)                                                         \
+      linear_scan_kernel<S, RP, 1><<<grid, 256, sm, s>>>(SCAN_ARGS);         \
     else                                                                     \
-      linear_scan_kernel<S, RP><<<grid, 256, sm, s>>>(SCAN_ARGS);            \
+      linear_scan_kernel<S, RP, (RP >= 16 ? 8 : 16)>                         \
+          <<<grid, 256, sm, s>>>(SCAN_ARGS);                                 \
   } while (0)
   if (rp <= 2) SCAN(2);
   else if (rp <= 4) SCAN(4);

@@ -979,3 +979,42 @@ def test_scan_order_of_the_sequences(B, H, dv):
         if lens[a]:
             assert torch.equal(run(a, a + 1, alone), whole[cu[a]:cu[a + 1]])
     assert torch.equal(together, alone)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dk", [30, 64, 128, 200])
+@pytest.mark.parametrize("gated", [False, True])
+def test_scan_of_few_tokens(dtype, dk, gated):
+    """Blocks of one token, also for sequences of several next to empty ones: the bits of
+    the larger blocks, which the same tokens take in a step of more tokens than
+    sequences."""
+    from types import SimpleNamespace
+    from agentfield_amd.ops import seqmix as sm
+    H, dv, lens = 3, 40, [1, 3, 0, 0, 1]
+    g = torch.Generator(device="cuda").manual_seed(dk)
+
+    def rows(n, s=1.0):
+        return (torch.randn(5, n, generator=g, device="cuda") * s).to(dtype)
+    q, k, v, z = rows(H * dk, dk ** -0.5), rows(H * dk, 0.3), rows(H * dv), rows(H * dk)
+    before = torch.randn(9, H, dk, dv, generator=g, device="cuda")
+
+    def run(which, state):
+        cu = torch.tensor([0] + lens).cumsum(0)
+        idx = torch.cat([torch.arange(cu[i], cu[i + 1]) for i in which]).cuda()
+        n = [lens[i] for i in which]
+        md = SimpleNamespace(
+            cu_seqlens=torch.tensor([0] + n).cumsum(0).int().cuda(),
+            q_start=torch.tensor([4 * i for i in which]).int().cuda(),
+            state_slots=torch.tensor([i + 1 for i in which]).int().cuda())
+        pos = torch.cat([torch.arange(lens[i]) + 4 * i for i in which]).int().cuda()
+        kw = (dict(decay_logits=z[idx], decay_bias=torch.ones(H * dk, device="cuda"),
+                   inv_tau=0.25) if gated
+              else dict(head_decay=torch.tensor([.9, .99, .5], device="cuda")))
+        return sm.linear_scan(q[idx], k[idx], v[idx], state, md, pos, H,
+                              inv_freq=sm.rotary_inv_freq(8, 1e4, "cuda"), **kw)
+    whole, state = None, before.clone()
+    whole = run([0, 1, 2, 3, 4], state)          # as many tokens as sequences
+    other = before.clone()
+    parts = torch.cat([run([0], other), run([1], other), run([4], other)])
+    assert torch.equal(whole, parts) and torch.equal(state, other)
