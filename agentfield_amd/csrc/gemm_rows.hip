@@ -68,6 +68,7 @@
 // 25.6 and 57.5 + 5.2 for the first and the last, o + down 63.1).
 #include "mfma_lines.h"
 
+#include <climits>
 #include <type_traits>
 
 enum RowsEpi { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_ROPE = 3,
@@ -136,12 +137,11 @@ __device__ __forceinline__ void put_rope(const RowsArgs& a, int m, int head, int
 // NORM: 0 none, 1 from ss, 2 computed from X.  PD pieces per wave in flight, with DRAIN
 // until the next is needed.
 template <int PD, int EPI, int NORM, int AUX, bool DRAIN>
-__global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
+__device__ __forceinline__ void rows_block(const RowsArgs& a, const int tile) {
   constexpr int NW = 8;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int n = lane & 15;
-  const int tile = blockIdx.x;
 
   constexpr int PIECE = 2048;                    // 16 rows x 64 elements
   constexpr int SLOT = PIECE * 2;                // of W and of X
@@ -163,7 +163,7 @@ __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
     xp[g] = a.X + (size_t)min(g * 8 + r8, a.M - 1) * a.K + ch;
   }
   const int cnt = ((a.K >> 6) - wid + NW - 1) / NW;  // this wave's pieces
-  const int rot = cnt > 0 ? ((int)blockIdx.x >> 3) % cnt : 0;
+  const int rot = cnt > 0 ? (tile >> 3) % cnt : 0;
   auto load = [&](int i) {
     lds_b* to = ring + (i % PD) * SLOT;
     const int p = i + rot < cnt ? i + rot : i + rot - cnt;
@@ -261,6 +261,42 @@ __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
     }
     *reinterpret_cast<u16x2*>(a.out + at) = u16x2{f2bf(v0), f2bf(v1)};
   }
+}
+
+template <int PD, int EPI, int NORM, int AUX, bool DRAIN>
+__global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
+  rows_block<PD, EPI, NORM, AUX, DRAIN>(a, blockIdx.x);
+}
+
+// Several plain products of as many rows in one launch, the longest inner dimension first:
+// alone, those of small weights are launches and latency (rows against 2048 x 2048 4.1 us).
+// Of a 1b hybrid layer, 6 rows: 8192 x 2048, 10240 x 2048 and 2048 x 2048 20.5 us in three
+// launches, 15.2 in one (5.5 TB/s); 2048 x 8192, 2048 x 2048 and 2048 x 1024 17.0, 12.8; one
+// row 19.6, 15.3 and 16.2, 10.5.  Two of larger weights gain the launch, 4096 x 4096 and
+// 4096 x 14336 28.0, 26.4.
+#define GROUP_MAX 4
+struct RowsGroup {
+  struct Part {
+    u16* out;
+    const u16 *X, *W;
+    int N, K, tile0;
+  } part[GROUP_MAX];
+  int parts, M;
+};
+
+template <int AUX>
+__global__ void __launch_bounds__(512) gemm_rows_group_kernel(RowsGroup g) {
+  int i = 0;
+  while (i + 1 < g.parts && (int)blockIdx.x >= g.part[i + 1].tile0) ++i;
+  const RowsGroup::Part& p = g.part[i];
+  RowsArgs a = {};
+  a.out = p.out;
+  a.X = p.X;
+  a.W = p.W;
+  a.M = g.M;
+  a.N = p.N;
+  a.K = p.K;
+  rows_block<2, EPI_PLAIN, 0, AUX, false>(a, blockIdx.x - p.tile0);
 }
 
 // All but N of a wave's loads have landed, its LDS reads are done, and so it is for
@@ -801,6 +837,42 @@ AF_EXPORT int af_rows_linear(void* out, void* residual, void* parts, void* ss_ou
   } else {
     return 9008;
   }
+  return af_last_err();
+}
+
+// Up to GROUP_MAX plain products of M <= 16 rows each: out [M, N] = X [M, K] @ W [N, K]^T,
+// described by n times (out, X, W, N, K).
+AF_EXPORT int af_rows_group(const i64* desc, int n, int M, void* stream) {
+  if (n < 1 || n > GROUP_MAX || M < 1 || M > ROWS_MAX) return 9008;
+  RowsGroup g = {};
+  g.parts = n;
+  g.M = M;
+  int order[GROUP_MAX] = {0, 1, 2, 3}, tiles = 0;
+  for (int i = 1; i < n; ++i)
+    for (int j = i; j > 0 && desc[order[j] * 5 + 4] > desc[order[j - 1] * 5 + 4]; --j) {
+      const int t = order[j];
+      order[j] = order[j - 1];
+      order[j - 1] = t;
+    }
+  bool stream_past = false;
+  for (int i = 0; i < n; ++i) {
+    const i64* d = desc + order[i] * 5;
+    RowsArgs a = {};
+    a.out = (u16*)d[0];
+    a.X = (const u16*)d[1];
+    a.W = (const u16*)d[2];
+    a.M = M;
+    a.N = (int)d[3];
+    a.K = (int)d[4];
+    if (!a.out || d[3] < 64 || d[3] > INT_MAX || d[4] > INT_MAX) return 9008;
+    if (const int rc = check_rows(a, 1)) return rc;
+    g.part[i] = {a.out, a.X, a.W, a.N, a.K, tiles};
+    tiles += a.N / 16;
+    stream_past = stream_past || streamed(a);
+  }
+  hipStream_t st = (hipStream_t)stream;
+  if (stream_past) gemm_rows_group_kernel<STREAM><<<tiles, 512, 0, st>>>(g);
+  else gemm_rows_group_kernel<KEEP><<<tiles, 512, 0, st>>>(g);
   return af_last_err();
 }
 

@@ -298,14 +298,17 @@ class ChunkedAttention(nn.Module):
         return [("q", s.heads * s.dim), ("k", s.kv_heads * s.dim),
                 ("v", s.kv_heads * s.vdim)]
 
-    def forward(self, p: dict, cache: HybridCache, run: int, md, positions):
+    def rows(self, p: dict, cache: HybridCache, run: int, md, positions):
+        """What the output projection reads."""
         s = self.spec
         q = sm.qk_norm_cache(p["q"], p["k"], p["v"], self.q_norm, self.k_norm,
                              self.eps, cache.k[run], cache.v[run], md.slots)
-        o = sm.masked_attention(q, cache.k[run], cache.v[run], md, positions,
-                                s.scale, s.heads, chunk=s.chunk,
-                                window=s.window)
-        return sm.matmul(o, self.o)
+        return sm.masked_attention(q, cache.k[run], cache.v[run], md, positions,
+                                   s.scale, s.heads, chunk=s.chunk,
+                                   window=s.window)
+
+    def forward(self, p: dict, cache: HybridCache, run: int, md, positions):
+        return sm.matmul(self.rows(p, cache, run, md, positions), self.o)
 
 
 class GatedLinearAttention(nn.Module):
@@ -329,16 +332,19 @@ class GatedLinearAttention(nn.Module):
                 ("v", s.heads * s.vdim), ("g", s.heads * s.vdim),
                 ("a1", s.rank)]
 
-    def forward(self, p: dict, cache: HybridCache, run: int, md, positions):
+    def rows(self, p: dict, cache: HybridCache, run: int, md, positions):
+        """What the output projection reads."""
         s = self.spec
         z = sm.matmul(p["a1"], self.a2)
         o = sm.linear_scan(p["q"], p["k"], p["v"], cache.rec[run], md,
                            positions, s.heads, q_scale=s.dim ** -0.5,
                            decay_logits=z, decay_bias=self.a2_b,
                            inv_tau=1.0 / s.tau)
-        y = sm.headnorm_gate(o, p["g"], self.norm, self.eps, s.heads,
-                             self.o.dtype)
-        return sm.matmul(y, self.o)
+        return sm.headnorm_gate(o, p["g"], self.norm, self.eps, s.heads,
+                                self.o.dtype)
+
+    def forward(self, p: dict, cache: HybridCache, run: int, md, positions):
+        return sm.matmul(self.rows(p, cache, run, md, positions), self.o)
 
 
 class Retention(nn.Module):
@@ -364,13 +370,16 @@ class Retention(nn.Module):
         return [("q", s.heads * s.dim), ("k", s.heads * s.dim),
                 ("v", s.heads * s.vdim), ("g", s.heads * s.vdim)]
 
-    def forward(self, p: dict, cache: HybridCache, run: int, md, positions):
+    def rows(self, p: dict, cache: HybridCache, run: int, md, positions):
+        """What the output projection reads."""
         s = self.spec
         o = sm.linear_scan(p["q"], p["k"], p["v"], cache.rec[run], md,
                            positions, s.heads, k_scale=s.dim ** -0.5,
                            head_decay=self.decay, inv_freq=self.inv_freq)
-        y = sm.headnorm_gate(o, p["g"], None, self.eps, s.heads, self.o.dtype)
-        return sm.matmul(y, self.o)
+        return sm.headnorm_gate(o, p["g"], None, self.eps, s.heads, self.o.dtype)
+
+    def forward(self, p: dict, cache: HybridCache, run: int, md, positions):
+        return sm.matmul(self.rows(p, cache, run, md, positions), self.o)
 
 
 class PolyNormMLP(nn.Module):
@@ -383,8 +392,27 @@ class PolyNormMLP(nn.Module):
         self.down = nn.Parameter(torch.empty(width, ff))
         self.register_buffer("act", torch.zeros(4, dtype=torch.float32))
 
+    def rows(self, z):
+        """What the down projection reads."""
+        return sm.polynorm(z, self.act, self.eps)
+
     def forward(self, z):
-        return sm.matmul(sm.polynorm(z, self.act, self.eps), self.down)
+        return sm.matmul(self.rows(z), self.down)
+
+
+_ROWS_OF = {ChunkedAttention, GatedLinearAttention, Retention, PolyNormMLP}
+
+
+def _as_written(*modules) -> bool:
+    """Whether calling these modules is their own forward and nothing else: no
+    subclass, and no hooks that a call would run."""
+    if torch.nn.modules.module._has_any_global_hook():
+        return False
+    for m in modules:
+        if (type(m) not in _ROWS_OF or m._forward_hooks or m._forward_pre_hooks
+                or m._backward_hooks or m._backward_pre_hooks):
+            return False
+    return True
 
 
 class ReperaxLayer(nn.Module):
@@ -427,18 +455,39 @@ class ReperaxLayer(nn.Module):
         dt = self.mix_in.dtype
         a, s, b = sm.dual_norm_shift(x, self.norm1, self.norm2, self.shift,
                                      self.eps, cache.shift[run], md, dt)
-        proj = sm.matmul(s, self.mix_in)
+        # decode steps: what reads the norms in one launch, and what writes the
+        # residual in another (prompts keep their order, and with it their memory)
+        mods = [*self.mixers.values()] + ([self.mlp] if self.mlp is not None else [])
+        reads = [(s, self.mix_in), (a, self.rg1)]
+        if self.mlp is not None:
+            reads.append((b, self.ff_in))
+        read = sm.matmul_group(reads) if _as_written(*mods) else None
+        proj = sm.matmul(s, self.mix_in) if read is None else read[0]
         views, c0 = {}, 0
         for mn, bn, rows in self.blocks:
             views.setdefault(mn, {})[bn] = proj[:, c0:c0 + rows]
             c0 += rows
-        outs = [m(views[mn], cache, run, md, positions)
-                for mn, m in self.mixers.items()]
-        g1 = sm.matmul(a, self.rg1)
-        m_out = g2 = b2 = None
+        m_out = g2 = b2 = u = None
+        if read is None:
+            outs = [m(views[mn], cache, run, md, positions)
+                    for mn, m in self.mixers.items()]
+            g1 = sm.matmul(a, self.rg1)
+            if self.mlp is not None:
+                u = sm.matmul(b, self.ff_in)
+                m_out = self.mlp(u[:, :self.spec.ff])
+        else:
+            _, g1, *rest = read
+            writes = [(m.rows(views[mn], cache, run, md, positions), m.o)
+                      for mn, m in self.mixers.items()]
+            if self.mlp is not None:
+                u, = rest
+                writes.append((self.mlp.rows(u[:, :self.spec.ff]), self.mlp.down))
+            outs = sm.matmul_group(writes)
+            if outs is None:
+                outs = [sm.matmul(*w) for w in writes]
+            if self.mlp is not None:
+                *outs, m_out = outs
         if self.mlp is not None:
-            u = sm.matmul(b, self.ff_in)
-            m_out = self.mlp(u[:, :self.spec.ff])
             g2 = u[:, self.spec.ff:self.spec.ff + x.shape[1]]
             b2 = self.rg2_b
         sm.gated_residual(x, outs[0], self.scales[0],

@@ -9,6 +9,7 @@ Every op has two paths:
 from __future__ import annotations
 
 import functools
+import ctypes
 import itertools
 import math
 
@@ -421,6 +422,22 @@ def launch_rows(x, w, mode=0, residual=None, scale=None, ss_out=None,
 
 # rows up to which the row GEMM needs no partial sums and no row statistics
 ROWS_MAX = 16
+# plain products of so few rows that one launch takes
+ROWS_GROUP = 4
+
+
+def launch_rows_group(pairs) -> list:
+    """[x @ w^T for x, w in pairs], at most ROWS_GROUP of as many rows, ROWS_MAX at
+    most, in one launch; for callers that have checked the operands."""
+    outs, desc = [], []
+    for x, w in pairs:
+        out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
+        outs.append(out)
+        desc += (out.data_ptr(), x.data_ptr(), w.data_ptr(), *w.shape)
+    rc = _lib.lib().af_rows_group((ctypes.c_int64 * len(desc))(*desc), len(pairs),
+                                  pairs[0][0].shape[0], _lib.cur_stream())
+    _lib.check(rc, "af_rows_group")
+    return outs
 
 
 def qkv_rope_rows(x: torch.Tensor, w: torch.Tensor, eps: float,

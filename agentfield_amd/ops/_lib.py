@@ -64,6 +64,7 @@ def _declare(l: ctypes.CDLL) -> None:
     l.af_gemm_skinny.argtypes = [p, p, p, p, p, i, i, i, i, i,
                                  p, f, p, p]
     l.af_rows_linear.argtypes = [p, p, p, p, p, p, i, i, i, i, i, i, p, f, p]
+    l.af_rows_group.argtypes = [p, i, i, p]
     l.af_rows_qkv.argtypes = [p, p, p, p, p, i, i, i, i, i, i, f, p, p, p, p, p,
                               i, p]
     l.af_moe_route.argtypes = [p, p, p, p, p, p, p, i, i, i, i, p]
@@ -87,7 +88,7 @@ def _declare(l: ctypes.CDLL) -> None:
     for fn in ("af_rmsnorm", "af_rope_cache", "af_silu_mul", "af_add",
                "af_reshape_and_cache", "af_embedding", "af_attn_decode",
                "af_attn_prefill", "af_gemm_bf16", "af_gemm_bf16_ring", "af_gemm_bf16_q8", "af_gemm_mxfp8", "af_oneshot_allreduce",
-               "af_gemm_skinny", "af_rows_linear", "af_rows_qkv",
+               "af_gemm_skinny", "af_rows_linear", "af_rows_group", "af_rows_qkv",
                "af_moe_route", "af_moe_combine", "af_moe_gemm", "af_gemm_wide",
                "af_gemm_wide_experts", "af_gemm_wide_split",
                "af_gemm_wide_splits", "af_gemm_wide_ns", "af_sample",

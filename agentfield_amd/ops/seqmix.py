@@ -733,6 +733,22 @@ def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
     return x @ w.t()
 
 
+def matmul_group(pairs) -> list | None:
+    """[x @ w^T for x, w in pairs] in one launch, by the kernel and with the bits of
+    matmul: bf16 products of as many rows each, up to 16, on one GPU.  None where they
+    are not, and where matmul leaves one of them to torch."""
+    x0 = pairs[0][0]
+    M = x0.shape[0]
+    if not (x0.is_cuda and 0 < M <= _ops.ROWS_MAX and len(pairs) <= _ops.ROWS_GROUP
+            and _lib.main_lib_ready()):
+        return None
+    for x, w in pairs:
+        if (x.shape[0] != M or x.device != x0.device or _ops.watched(x, w)
+                or not _ops._rows_ok(x, w)):
+            return None
+    return _ops.launch_rows_group(pairs)
+
+
 # few rows against a weight whose inner dimension is the long one: from this
 # inner dimension on the split-K kernel streams the weight about twice as fast
 # as the vendor GEMM (42 against 93 us for 64 rows of 36864 -> 2048)

@@ -1018,3 +1018,68 @@ def test_scan_of_few_tokens(dtype, dk, gated):
     other = before.clone()
     parts = torch.cat([run([0], other), run([1], other), run([4], other)])
     assert torch.equal(whole, parts) and torch.equal(state, other)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 6, 16])
+@pytest.mark.parametrize("shapes", [
+    [(64, 64)], [(64, 640), (192, 64), (64, 1024), (128, 576)],
+    [(2048, 1024), (2048, 4096), (2048, 2048)], [(4160, 2048), (64, 64)]])
+def test_products_of_few_rows_in_one_launch(M, shapes):
+    """In any order of inner dimensions, weights past the caches and not: the bits of a
+    launch each."""
+    g = torch.Generator(device="cuda").manual_seed(M)
+    pairs = [tuple(torch.randn(n, k, generator=g, device="cuda").bfloat16()
+                   for n in (M, rows)) for rows, k in shapes]
+    got = sm.matmul_group(pairs)
+    assert len(got) == len(pairs)
+    for y, (x, w) in zip(got, pairs):
+        assert torch.equal(y, sm.matmul(x, w))
+
+
+@pytest.mark.gpu
+def test_products_of_few_rows_left_alone():
+    """What one launch does not take is None: other row counts, types, strides, sizes,
+    places, more products than it has room for, and what autograd has to see."""
+    def t(*s, dtype=torch.bfloat16):
+        return torch.ones(*s, device="cuda", dtype=dtype)
+    good = (t(4, 64), t(128, 64))
+    assert sm.matmul_group([good] * 4) is not None
+    for pairs in ([good] * 5, [good, (t(5, 64), t(64, 64))], [(t(17, 64), t(64, 64))],
+                  [good, (t(4, 64, dtype=torch.float32), t(64, 64, dtype=torch.float32))],
+                  [good, (t(4, 96), t(64, 96))], [good, (t(4, 64), t(100, 64))],
+                  [good, (t(4, 128)[:, :64], t(64, 64))], [good, (t(4, 64), t(64, 128))],
+                  [(x.cpu(), w.cpu()) for x, w in [good]], [(t(0, 64), t(64, 64))],
+                  [good, (t(4, 64), t(64, 64).requires_grad_())]):
+        assert sm.matmul_group(pairs) is None
+
+
+@pytest.mark.gpu
+def test_grouped_layer_and_its_hooks():
+    """A layer of few rows gives the bits of its projections one by one, which is how it
+    runs while a hook wants to see its mixers' or unit's calls."""
+    from agentfield_amd.models.hybrid import HYBRID_CONFIGS
+    cfg = HYBRID_CONFIGS["reperax-tiny"]
+    torch.manual_seed(0)
+    model = cfg.build_model("cuda")
+    for p in model.parameters():
+        p.data.normal_(0, 0.05)
+    seen = []
+
+    def logits():
+        eng = LLMEngine(cfg, device="cuda", page_size=8, num_pages=32, max_num_seqs=3,
+                        model=model, enable_graphs=False, caller_paced=True)
+        reqs = [eng.open_request() for _ in range(3)]
+        eng.feed_step([(r, [5, 6, 7, 8][:i + 1], [i]) for i, r in enumerate(reqs)])
+        return torch.stack([eng.feed_step([(r, [n + i], [0]) for i, r in enumerate(reqs)])
+                            for n in (3, 9, 11)])
+    plain = logits()
+    handles = [m.register_forward_hook(lambda m, a, y: seen.append(type(m).__name__))
+               for layer in model.layers for m in (*layer.mixers.values(), layer.mlp)]
+    assert torch.equal(logits(), plain)
+    runs = len(cfg.runs)
+    assert len(seen) >= 4 * 2 * runs
+    for h in handles:
+        h.remove()
+    n = len(seen)
+    assert torch.equal(logits(), plain) and len(seen) == n
