@@ -666,6 +666,54 @@ __global__ void __launch_bounds__(256) headnorm_gate_lanes_kernel(
   if (d < dv && rh < n_rh) stv<S, 4>(out + (size_t)rh * dv + d, r);
 }
 
+// out [M, N] = x [M, K] @ w [N, K]^T for an inner dimension of at most KP (the upper half of a
+// low-rank projection): bound by writing out.  A thread keeps the weights of two columns, a
+// block R rows of x in LDS, read as broadcasts; sums in fp32 in the order of K.
+// Two rows per block while that gives no more than a few rounds of them (1000 x 1024 3.7 us,
+// 16 rows 5.6; 600 x 8192 9.3, 7.7).  Library / here, K 16: 6 x 1024 5.2 / 2.7 us, 210 x 1024
+// 4.1 / 2.8, 7636 x 1024 12.7 / 9.7, 30000 x 8192 198 / 159, 6 x 256 5.1 / 2.5.  With K 24 or
+// 32 the library is the faster one from 64 rows on (256 columns 4.2 / 7.1).
+template <int KP, int R>
+__global__ void __launch_bounds__(256) narrow_product_kernel(
+    u16* __restrict__ out, const u16* __restrict__ x, const u16* __restrict__ w, int M, int N,
+    int K, i64 ldx) {
+  __shared__ __attribute__((aligned(16))) float xs[R][KP];
+  const int m0 = blockIdx.y * R, c = (blockIdx.x * 256 + threadIdx.x) * 2;
+  const int rows = min(R, M - m0);
+  s16x8 raw[2][KP / 8];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < KP / 8; ++j)
+      raw[h][j] = *reinterpret_cast<const s16x8*>(w + (size_t)min(c + h, N - 1) * K +
+                                                  min(j * 8, K - 8));
+  for (int i = threadIdx.x; i < rows * KP; i += 256) {
+    const int r = i / KP, k = i % KP;
+    xs[r][k] = k < K ? bf2f(x[(size_t)(m0 + r) * ldx + k]) : 0.f;
+  }
+  float wf[2][KP];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int k = 0; k < KP; ++k) wf[h][k] = k < K ? bf2f((u16)raw[h][k / 8][k % 8]) : 0.f;
+  __syncthreads();
+  if (c >= N) return;
+  for (int r = 0; r < rows; ++r) {
+    float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+    for (int k = 0; k < KP; k += 4) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(&xs[r][k]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        s0 = fmaf(v[j], wf[0][k + j], s0);
+        s1 = fmaf(v[j], wf[1][k + j], s1);
+      }
+    }
+    *reinterpret_cast<uint32_t*>(out + (size_t)(m0 + r) * N + c) =
+        (uint32_t)f2bf(s0) | ((uint32_t)f2bf(s1) << 16);
+  }
+}
+
 // Rows of up to R * 256 * V stay in registers: read once, all loads in flight together (rows
 // of 8192 bf16, six: 6.5 us read twice, 4.4 so; 7636: 58 us, 41).  R = 0: any length.
 template <typename S, int V, int R>
@@ -1212,6 +1260,23 @@ AF_EXPORT int afm_headnorm_gate(void* out, const void* o, const void* g,
 #undef HGS
 #undef HGL
 #undef HG
+  return af_last_err();
+}
+
+// bf16; K 8 or 16, N even, w and its rows on 16-byte boundaries, out whole rows.
+AF_EXPORT int afm_narrow_product(void* out, const void* x, const void* w, int M, int N, int K,
+                                 i64 ldx, void* stream) {
+  if (M == 0) return 0;
+  if (M < 0 || N < 2 || N % 2 || (K != 8 && K != 16) || ldx < K ||
+      (uintptr_t)w % 16 || (uintptr_t)out % 4 || (M + 15) / 16 > 65535)
+    return 9003;
+  hipStream_t s = (hipStream_t)stream;
+#define NARROW(R)                                                              \
+  narrow_product_kernel<16, R><<<dim3((N + 511) / 512, (M + R - 1) / R), 256, 0, s>>>( \
+      (u16*)out, (const u16*)x, (const u16*)w, M, N, K, ldx)
+  if ((i64)M * N <= (4 << 20)) NARROW(2);
+  else NARROW(16);
+#undef NARROW
   return af_last_err();
 }
 

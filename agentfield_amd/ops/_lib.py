@@ -155,6 +155,7 @@ def _mix_sigs() -> dict:
             "afm_relu2": [p, i64, p, i64, p, i64, i, i, i, i, i, p],
             "afm_xielu": [p, p, i64, p, i, i, i, p],
             "afm_headnorm_gate": [p, p, p, p, f, i, i, i, i64, i, i, p],
+            "afm_narrow_product": [p, p, p, i, i, i, i64, p],
             "afm_polynorm": [p, p, p, f, i, i, i64, i, p],
             "afm_gated_residual": [p, p, f, p, f, p, i64, p, p, p, i64, p,
                                    i, i, i, p],

@@ -698,7 +698,8 @@ def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
 
     bf16 products of few rows (decode steps) run on the framework's
     weight-streaming kernels, wider ones and prompts on the vendor GEMM
-    (hipBLASLt / rocBLAS) or, where that has begun a round, on the wide GEMM.  Above
+    (hipBLASLt / rocBLAS) or, where that has begun a round, on the wide GEMM; an inner
+    dimension of up to 16 has a kernel of its own (_narrow).  Above
     16 rows a second launch adds the K splits up unless N fills the chip by itself,
     which middling widths do not earn back.
     Measured, vendor against rows in us: 4096 x 4096 15.7 / 7.8 at 4 rows, 15.3 /
@@ -712,6 +713,9 @@ def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
     the vendor GEMM's (watched)."""
     M, K = x.shape
     N = w.shape[0]
+    if (K <= 16 and skinny and out is None and x.is_cuda
+            and _narrow_ok(x, w) and not _ops.watched(x, w)):
+        return _narrow(x, w)
     if (M > 128 and skinny and x.is_cuda and _lib.main_lib_ready()
             and _ops._wide_pays(M, N, K, False) and _ops._launches_here(x)
             and not _ops.watched(x, w)
@@ -731,6 +735,29 @@ def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
                 and x.is_contiguous() and w.is_contiguous()):
             return _ops.linear_skinny(x, w)
     return x @ w.t()
+
+
+def _narrow_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """What the narrow product takes: bf16 rows of any stride against whole weights on
+    16-byte boundaries, an inner dimension of 8 or 16, an even N from 256 on."""
+    M, K = x.shape
+    return (w.dim() == 2 and w.shape[1] == K and K in (8, 16)
+            and w.shape[0] % 2 == 0 and w.shape[0] >= 256 and 0 < M < 1 << 20
+            and x.dtype == torch.bfloat16 == w.dtype and x.device == w.device
+            and x.stride(1) == 1 and (M == 1 or x.stride(0) >= K)
+            and w.is_contiguous() and w.data_ptr() % 16 == 0
+            and _ops._launches_here(x))
+
+
+def _narrow(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x [M, K] @ w [N, K]^T with an inner dimension of 8 or 16."""
+    M, K = x.shape
+    out = torch.empty(M, w.shape[0], dtype=x.dtype, device=x.device)
+    rc = _L().afm_narrow_product(_lib.ptr(out), _lib.ptr(x), _lib.ptr(w), M,
+                                 w.shape[0], K, max(x.stride(0), K),
+                                 _lib.cur_stream())
+    _lib.check(rc, "afm_narrow_product")
+    return out
 
 
 def matmul_group(pairs) -> list | None:

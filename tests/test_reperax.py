@@ -1083,3 +1083,32 @@ def test_grouped_layer_and_its_hooks():
         h.remove()
     n = len(seen)
     assert torch.equal(logits(), plain) and len(seen) == n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2, 3, 17, 16385])
+@pytest.mark.parametrize("N,K,step", [(256, 16, 16), (258, 8, 40), (1000, 16, 33),
+                                      (514, 16, 17)])
+def test_narrow_product(M, N, K, step):
+    """Rows of any stride and address, columns around a block's 512, both block heights.
+    fp32 sums of K exact products (K * 2^-24 of their magnitudes), rounded to bf16."""
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn(M, step, generator=g, device="cuda").bfloat16()[:, step - K:]
+    w = torch.randn(N, K, generator=g, device="cuda").bfloat16()
+    assert sm._narrow_ok(x, w)
+    got = sm.matmul(x, w).double()
+    want = x.double() @ w.double().t()
+    bound = want.abs() * 2 ** -8 + x.double().abs() @ w.double().abs().t() * K * 2 ** -24
+    assert ((got - want).abs() <= bound).all()
+    for bad in (w[:, :K // 2], w[:254], w.float(), w.cpu(),
+                torch.empty(N * K + 1, device="cuda").bfloat16()[1:].view(N, K)):
+        assert not sm._narrow_ok(x, bad)
+    assert not sm._narrow_ok(x.t()[:, :0].t(), w)
+
+
+@pytest.mark.gpu
+def test_narrow_product_is_seen_by_autograd():
+    x = torch.randn(4, 16, device="cuda").bfloat16()
+    w = torch.randn(256, 16, device="cuda").bfloat16().requires_grad_()
+    sm.matmul(x, w).float().sum().backward()
+    assert torch.isfinite(w.grad).all() and w.grad.abs().sum() > 0
