@@ -283,7 +283,11 @@ def _step_tiles(md, rows: int, device):
     key = (tuple(md.seq_lens), rows, device, _lib.cur_stream())
     kept = getattr(md, "step_tiles", None)
     if kept is None or kept[0] != key:
-        kept = md.step_tiles = (key, _row_tiles(md.seq_lens, rows, device))
+        kept = (key, _row_tiles(md.seq_lens, rows, device))
+        try:
+            md.step_tiles = kept
+        except AttributeError:      # a description that takes no more attributes
+            pass
     return kept[1]
 
 

@@ -342,6 +342,9 @@ def test_row_tiles_of_a_step():
     kept = sm._step_tiles(md, 64, dev)
     with torch.cuda.stream(torch.cuda.Stream()):
         assert sm._step_tiles(md, 64, dev) is not kept
+    from collections import namedtuple
+    fixed = namedtuple("Fixed", "seq_lens")([130, 70, 64])
+    assert tiles(sm._step_tiles(fixed, 64, dev)) == tiles(kept)
 
 
 @pytest.mark.gpu
