@@ -1117,6 +1117,30 @@ def test_attn_prefill_any_scale(monkeypatch, few_cols, nsplit, scale, window):
     assert close(got, want, atol=2 ** -6, rtol=2 ** -7)
 
 
+@pytest.mark.parametrize("B", [1, 16, 17, 32, 33, 64, 65, 130])
+@pytest.mark.parametrize("few_cols,nsplit", [(0, 1), (32, 2), (1 << 30, 1)])
+def test_attn_prefill_finds_its_items(monkeypatch, B, few_cols, nsplit):
+    """Sequences around the 16 and 64 whose items a wave counts at once, empty ones
+    and such of the other kernel's among them, each with its own keys.  Tolerance as
+    above."""
+    _cut(monkeypatch, few_cols, nsplit)
+    D, G, page, maxp = 128, 4, 16, 4
+    lens = [(3, 0, 9, 40, 1, 8)[i % 6] for i in range(B)]
+    hist = [(i * 5) % 20 for i in range(B)]
+    torch.manual_seed(B)
+    bt = (torch.randperm(B * maxp) + 1).view(B, maxp).to(torch.int32)
+    kc, vc = (torch.randn(B * maxp + 1, 1, page, D).bfloat16() for _ in range(2))
+    q = torch.randn(sum(lens), G * D).bfloat16()
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    qs = torch.tensor(hist, dtype=torch.int32)
+    scale = 1.0 / math.sqrt(D)
+    got = ops.attn_prefill(q.to(DEV), kc.to(DEV), vc.to(DEV), bt.to(DEV), qs.to(DEV),
+                           cu.to(DEV), lens, scale).cpu()
+    want = ref.attn_prefill_paged(q.unflatten(-1, (G, D)), kc, vc, bt, qs, cu,
+                                  scale).flatten(1)
+    assert close(got, want, atol=2 ** -6, rtol=2 ** -7)
+
+
 @pytest.mark.parametrize("G", [1, 2, 4, 8])
 def test_attn_prefill_as_dispatched(G):
     """A step that the rule itself sends to both kernels, keys split or not."""
