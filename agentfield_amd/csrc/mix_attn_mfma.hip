@@ -496,7 +496,8 @@ __device__ __forceinline__ void attn_prefill_mfma_body(
     page, maxp, chunk, window, ldq, ex
 
 template <int DKC, int DVT, bool VEC, int NH, int KT = 64, int LITE = 0>
-__global__ void __launch_bounds__(256 * NH, (DKC <= 4 && NH == 2 ? 4 : 1)) attn_prefill_mfma_kernel(AF_APM_PARAMS) {
+__global__ void __launch_bounds__(256 * NH, DKC <= 4 && NH == 2 ? 4 : 1)
+attn_prefill_mfma_kernel(AF_APM_PARAMS) {
   attn_prefill_mfma_body<DKC, DVT, VEC, NH, KT, false, LITE>(AF_APM_ARGS);
 }
 

@@ -353,7 +353,8 @@ __global__ void __launch_bounds__(256) attn_rows_kernel(
     const S* __restrict__ vc, const i32* __restrict__ bt,
     const i32* __restrict__ row_seq, const i32* __restrict__ positions,
     float scale, int H, int G, int hpg, int dk, int dv, int page, int page_log2,
-    int q_wide, int maxp, int chunk, int window, i64 ldq, int lpk_log2, int lpv_log2, int kt, int nsplit,
+    int q_wide, int maxp, int chunk, int window, i64 ldq, int lpk_log2, int lpv_log2,
+    int kt, int nsplit,
     float* __restrict__ part_o, float* __restrict__ part_ml, AttnExtra ex) {
   // nsplit > 1: the visible keys are cut into nsplit ranges, one workgroup
   // each (grid.z = head blocks x nsplit).  With part_o, unnormalised outputs
