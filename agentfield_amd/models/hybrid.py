@@ -404,12 +404,13 @@ _ROWS_OF = {ChunkedAttention, GatedLinearAttention, Retention, PolyNormMLP}
 
 
 def _as_written(*modules) -> bool:
-    """Whether calling these modules is their own forward and nothing else: no
-    subclass, and no hooks that a call would run."""
+    """Whether calling these modules is their class's forward and nothing else: no
+    subclass, no forward of the instance's own, no hooks that a call would run."""
     if torch.nn.modules.module._has_any_global_hook():
         return False
     for m in modules:
-        if (type(m) not in _ROWS_OF or m._forward_hooks or m._forward_pre_hooks
+        if (type(m) not in _ROWS_OF or "forward" in m.__dict__
+                or m._compiled_call_impl is not None or m._forward_hooks or m._forward_pre_hooks
                 or m._backward_hooks or m._backward_pre_hooks):
             return False
     return True

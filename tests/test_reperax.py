@@ -1086,6 +1086,10 @@ def test_grouped_layer_and_its_hooks():
         h.remove()
     n = len(seen)
     assert torch.equal(logits(), plain) and len(seen) == n
+    mlp = model.layers[0].mlp
+    mlp.forward = lambda z: (seen.append("own"), type(mlp).forward(mlp, z))[1]
+    assert torch.equal(logits(), plain) and seen[n:] == ["own"] * 4 * sum(
+        li == 0 for li, _ in cfg.runs)
 
 
 @pytest.mark.gpu
