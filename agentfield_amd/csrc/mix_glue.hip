@@ -1263,18 +1263,21 @@ AF_EXPORT int afm_headnorm_gate(void* out, const void* o, const void* g,
   return af_last_err();
 }
 
-// bf16; K 8 or 16, N even, w and its rows on 16-byte boundaries, out whole rows.
+// bf16; K 8 or 16, N even, w and its rows on 16-byte boundaries, out whole rows, up to 65535
+// blocks of rows.
 AF_EXPORT int afm_narrow_product(void* out, const void* x, const void* w, int M, int N, int K,
                                  i64 ldx, void* stream) {
   if (M == 0) return 0;
+  const int R = (i64)M * N <= (4 << 20) ? 2 : 16;      // rows of a block
   if (M < 0 || N < 2 || N % 2 || (K != 8 && K != 16) || ldx < K ||
-      (uintptr_t)w % 16 || (uintptr_t)out % 4 || (M + 15) / 16 > 65535)
+      (uintptr_t)w % 16 || (uintptr_t)out % 4 || ((i64)M + R - 1) / R > 65535)
     return 9003;
+  const dim3 grid((N + 511) / 512, (M + R - 1) / R);
   hipStream_t s = (hipStream_t)stream;
-#define NARROW(R)                                                              \
-  narrow_product_kernel<16, R><<<dim3((N + 511) / 512, (M + R - 1) / R), 256, 0, s>>>( \
+#define NARROW(R)                                                 \
+  narrow_product_kernel<16, R><<<grid, 256, 0, s>>>(              \
       (u16*)out, (const u16*)x, (const u16*)w, M, N, K, ldx)
-  if ((i64)M * N <= (4 << 20)) NARROW(2);
+  if (R == 2) NARROW(2);
   else NARROW(16);
 #undef NARROW
   return af_last_err();

@@ -741,12 +741,17 @@ def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
     return x @ w.t()
 
 
+# rows that the narrow product takes: the blocks of a grid's second dimension, 16 rows each
+NARROW_ROWS = 65535 * 16
+
+
 def _narrow_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """What the narrow product takes: bf16 rows of any stride against whole weights on
-    16-byte boundaries, an inner dimension of 8 or 16, an even N from 256 on."""
+    16-byte boundaries, an inner dimension of 8 or 16, an even N from 256 on, up to
+    NARROW_ROWS rows."""
     M, K = x.shape
     return (w.dim() == 2 and w.shape[1] == K and K in (8, 16)
-            and w.shape[0] % 2 == 0 and w.shape[0] >= 256 and 0 < M < 1 << 20
+            and w.shape[0] % 2 == 0 and w.shape[0] >= 256 and 0 < M <= NARROW_ROWS
             and x.dtype == torch.bfloat16 == w.dtype and x.device == w.device
             and x.stride(1) == 1 and (M == 1 or x.stride(0) >= K)
             and w.is_contiguous() and w.data_ptr() % 16 == 0

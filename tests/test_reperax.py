@@ -1113,6 +1113,20 @@ def test_narrow_product(M, N, K, step):
     assert not sm._narrow_ok(x.t()[:, :0].t(), w)
 
 
+def test_narrow_product_takes_what_its_grid_holds(monkeypatch):
+    """Up to 65535 blocks of 16 rows, in the predicate as in the entry point, which refuses
+    more before it launches, whichever block height it takes; nothing runs here."""
+    monkeypatch.setattr(sm._ops, "_launches_here", lambda x: True)
+    w = torch.zeros(256, 8, dtype=torch.bfloat16)
+    most = 65535 * 16
+    for M in (1, most - 1, most, most + 1, most + 15, 1 << 20):
+        assert sm._narrow_ok(torch.empty(M, 8, dtype=torch.bfloat16), w) == (M <= most)
+    entry = sm._L().afm_narrow_product
+    for M, N in ((most + 1, 256), (1 << 20, 256), (2 * 65535 + 1, 2), (4 << 18, 4),
+                 (2 ** 31 - 1, 2)):
+        assert entry(0, 0, 0, M, N, 8, 8, None) == 9003
+
+
 @pytest.mark.gpu
 def test_narrow_product_is_seen_by_autograd():
     x = torch.randn(4, 16, device="cuda").bfloat16()
