@@ -31,6 +31,17 @@ __device__ __forceinline__ float gumbel_of(float u) {
   return -__logf(nl);
 }
 
+// A value and its noise, with the rounding spelled out (contraction is the compiler's
+// choice per place otherwise, and equal values are told apart by the last bit): the draw
+// without top-k and top-p in one step, the other, which compares x first, in two.
+__device__ __forceinline__ float scaled_sum(float l, float invt, float g) {
+  return fmaf(l, invt, g);
+}
+__device__ __forceinline__ float plain_sum(float x, float g) {
+#pragma clang fp contract(off)
+  return x + g;
+}
+
 __device__ __forceinline__ uint32_t hash3(uint32_t a, uint32_t b, uint32_t c) {
   // Wang/xxhash-style avalanche mix
   uint32_t h = a * 0x9E3779B1u + b * 0x85EBCA77u + c * 0xC2B2AE3Du + 0x27220A95u;
@@ -127,22 +138,28 @@ __device__ __forceinline__ void take_best(float ov, int oi, float& best,
 // logarithms, 22 instructions, that nearly no value needs: with w + 1/2 = 2^24 (1 - u), w a
 // whole number, -log u >= 1 - u, so a value x can only pass the score `top` of another where
 // w < 2^24 exp(x - top).  Eight steps of w (for the rounding of u and of the first
-// logarithm, and the u that rounds to 1) and 2^0.002 make up for rounding.
+// logarithm, and the u that rounds to 1) and 2^0.002 make up for rounding of the noise;
+// that of the scores themselves, which decides between equal values where 1/T is large, is
+// up to 2^-24 of them for the sum and as much for a product that is rounded first: 2^-22
+// of `top`.
 struct Draw {
   float best = AF_NEG_INF, top = -__builtin_inff();   // this lane's, the wave's
+  float lift = __builtin_inff();                      // 24 and what makes up for rounding
   int bidx = 0;
   uint32_t seed;
   int b;
 
-  // all lanes of a wave; x counts where `there`
-  __device__ __forceinline__ void take(float x, int v, bool there) {
+  // all lanes of a wave; x counts where `there`, and `sum` adds noise to it
+  template <class Sum>
+  __device__ __forceinline__ void take(float x, int v, bool there, Sum sum) {
     const uint32_t h = hash3(seed, (uint32_t)b, (uint32_t)v);
-    const float lim = __builtin_amdgcn_exp2f(fmaf(x - top, 1.44269504f, 24.002f)) + 8.f;
+    const float lim = __builtin_amdgcn_exp2f(fmaf(x - top, 1.44269504f, lift)) + 8.f;
     there = there && !((float)(~h >> 8) >= lim);
     if (!__any(there)) return;
-    x += gumbel_of(u32_to_unit(h));
+    x = sum(gumbel_of(u32_to_unit(h)));
     if (there && (x > best || (x == best && v < bidx))) { best = x; bidx = v; }
     top = wave_max_f32(best);
+    lift = fmaf(fabsf(top), 1.44269504f * 0x1p-22f, 24.002f);
   }
 };
 
@@ -183,7 +200,9 @@ __global__ void __launch_bounds__(256) sample_partial_kernel(
     d.b = b;
     each_logit_in_step(logits + (size_t)b * V, V, split, SMP_SPLITS,
                        [](float) { return true; },
-                       [&](float x, int v, bool there) { d.take(x * invt, v, there); });
+                       [&](float l, int v, bool there) {
+      d.take(l * invt, v, there, [&](float g) { return scaled_sum(l, invt, g); });
+    });
     store_best(d.best, d.bidx, pv, pi, b * SMP_SPLITS + split);
     return;
   }
@@ -192,7 +211,7 @@ __global__ void __launch_bounds__(256) sample_partial_kernel(
   each_logit(logits + (size_t)b * V, V, split, SMP_SPLITS, [&](float x, int v) {
     if (t > 0.f) {
       const float u = u32_to_unit(hash3(seed ^ st, (uint32_t)b, (uint32_t)v));
-      x = x * invt + gumbel_of(u);
+      x = scaled_sum(x, invt, gumbel_of(u));
     }
     if (x > best || (x == best && v < bidx)) { best = x; bidx = v; }
   });
@@ -401,7 +420,7 @@ __global__ void __launch_bounds__(256) tkp_sample_kernel(
                        [&](float l, int v, bool there) {
       const float x = l * invt;
       there = there && !(x < th);
-      if (__any(there)) d.take(x, v, there);
+      if (__any(there)) d.take(x, v, there, [&](float g) { return plain_sum(x, g); });
     });
     store_best(d.best, d.bidx, pv, pi, b * SMP_SPLITS + split);
     return;
@@ -411,7 +430,7 @@ __global__ void __launch_bounds__(256) tkp_sample_kernel(
   each_logit(row, V, split, SMP_SPLITS, [&](float l, int v) {
     float x = l * invt;
     if (x < th) return;
-    x += gumbel_of(u32_to_unit(hash3(seed ^ st, (uint32_t)b, (uint32_t)v)));
+    x = plain_sum(x, gumbel_of(u32_to_unit(hash3(seed ^ st, (uint32_t)b, (uint32_t)v))));
     if (x > best || (x == best && v < bidx)) { best = x; bidx = v; }
   });
   store_best(best, bidx, pv, pi, b * SMP_SPLITS + split);

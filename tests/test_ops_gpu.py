@@ -583,6 +583,29 @@ def test_sample_behind_a_bar(V, cut):
         assert (got[2::3] == torch.nan_to_num(score, nan=-math.inf).argmax(1)[2::3]).all()
 
 
+@pytest.mark.parametrize("T", [1.0, 0.3, 1e-3, 3e-4, 1e-5, 1e-6, 1e-9])
+@pytest.mark.parametrize("topk", [0, 50000])
+def test_sample_behind_a_bar_when_sharp(T, topk):
+    """Temperatures at which the rounding of the scores decides between many equal
+    values: the token of a row that is drawn behind a bar is that of the same row without
+    its masked end, which is short enough to be drawn without."""
+    B, short, wide = 64, 60000, 65600
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.full((B, wide), -math.inf, device=DEV)
+    t = torch.full((B,), T, device=DEV)
+    kw = {}
+    if topk:
+        kw = dict(topk=torch.full((B,), topk, device=DEV, dtype=torch.int32),
+                  topp=torch.ones(B, device=DEV))
+    for seed in range(20):
+        x[:, :short] = torch.randn(B, short, generator=g, device=DEV)
+        x[:, :short][torch.rand(B, short, generator=g, device=DEV) < 0.01] = 40.0
+        y = x.bfloat16()
+        got, want = (ops.sample(rows, t, ops.SamplerState(B, DEV, seed=seed), **kw)
+                     for rows in (y, y[:, :short].contiguous()))
+        assert torch.equal(got, want)
+
+
 def test_engine_topk_sampling_runs():
     from agentfield_amd.engine import LLMEngine, SamplingParams
     from agentfield_amd.models import CONFIGS
