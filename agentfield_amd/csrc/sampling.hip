@@ -15,7 +15,10 @@
 // rows from here on draw behind a bar (Draw): with fewer values a lane has not enough of
 // them for it to pay (all rows unrestricted, a pass of 256 threads in 16 splits: 64 x 32003
 // 18.3 us with the bar, 16.8 without; 64 x 128256 26.3 and 27.9, 128 x 128256 without top-k
-// or top-p 19.5 and 23.5)
+// or top-p 19.5 and 23.5).  With top-k or top-p two vectors a lane are too few as well (16 x
+// 65536, top-p 0.9, 14.6 and 14.0; 64 x 128256 0.9 of the time without), and a row whose
+// top-k leaves fewer than one value in 64 draws without (all rows of 128256 with top-k 50, 64
+// rows 18.8 and 18.0, 16 rows 14.6 and 14.1).
 #define SMP_BAR 65536
 
 __device__ __forceinline__ float u32_to_unit(uint32_t x) {
@@ -411,7 +414,7 @@ __global__ void __launch_bounds__(256) tkp_sample_kernel(
   const float th =
       tkp_threshold(hist_n, hist_m, row_max_of(rmax, b) * invt, k, p, b);
   const uint32_t st = *step;
-  if (BAR) {
+  if (BAR && k >= (V >> 6)) {                // of few values a bar spares nothing
     Draw d;
     d.seed = seed ^ st;
     d.b = b;
@@ -450,7 +453,7 @@ AF_EXPORT int af_sample_topkp(void* out, void* pv, void* pi, void* rmax,
   tkp_hist_kernel<<<g, 256, 0, st>>>((i32*)hist_n, (float*)hist_m,
                                      (const u16*)logits, (const float*)rmax,
                                      (const float*)temp, V);
-  const auto draw = V >= SMP_BAR ? tkp_sample_kernel<true> : tkp_sample_kernel<false>;
+  const auto draw = V > SMP_BAR ? tkp_sample_kernel<true> : tkp_sample_kernel<false>;
   draw<<<g, 256, 0, st>>>(
       (float*)pv, (i32*)pi, (const u16*)logits, (const float*)temp,
       (const float*)rmax, (const i32*)hist_n, (const float*)hist_m,

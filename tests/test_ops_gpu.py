@@ -584,11 +584,12 @@ def test_sample_behind_a_bar(V, cut):
 
 
 @pytest.mark.parametrize("T", [1.0, 0.3, 1e-3, 3e-4, 1e-5, 1e-6, 1e-9])
-@pytest.mark.parametrize("topk", [0, 50000])
+@pytest.mark.parametrize("topk", [0, 50000, 1024, 1025])
 def test_sample_behind_a_bar_when_sharp(T, topk):
     """Temperatures at which the rounding of the scores decides between many equal
     values: the token of a row that is drawn behind a bar is that of the same row without
-    its masked end, which is short enough to be drawn without."""
+    its masked end, which is short enough to be drawn without; with a top-k on both sides of
+    one value in 64 as well."""
     B, short, wide = 64, 60000, 65600
     g = torch.Generator(device=DEV).manual_seed(3)
     x = torch.full((B, wide), -math.inf, device=DEV)
