@@ -304,13 +304,13 @@ __global__ void __launch_bounds__(256) tkp_hist_kernel(
     const float* __restrict__ temp, int V) {
   const int split = blockIdx.y, b = blockIdx.x;
   const int copy = threadIdx.x & (TKP_COPIES - 1);
-  if (!(temp[b] > 0.f)) return;              // a greedy row takes its largest value
+  const float t = temp[b];
+  if (!(t > 0.f)) return;    // a greedy row takes its largest value: its histogram is not written
   __shared__ unsigned long long h[TKP_BINS * TKP_COPIES];
 #pragma unroll
   for (int c = 0; c < TKP_COPIES; ++c) h[c * 256 + threadIdx.x] = 0;
   __syncthreads();
-  const float t = temp[b];
-  const float invt = (t > 0.f) ? 1.f / t : 1.f;
+  const float invt = 1.f / t;
   const float mx = row_max_of(rmax, b) * invt;
   constexpr float STEP = TKP_SPAN / TKP_BINS;
   bool odd = false;  // a value that is not a number makes the mass one too
