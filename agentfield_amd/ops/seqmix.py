@@ -256,7 +256,8 @@ def _on_device(device, *lists):
     the recording refuses."""
     if device.type != "cuda" or torch.cuda.is_current_stream_capturing():
         return [torch.tensor(v, dtype=torch.int32, device=device) for v in lists]
-    host = torch.empty(len(lists), len(lists[0]), dtype=torch.int32, pin_memory=True)
+    host = torch.empty(len(lists), len(lists[0]), dtype=torch.int32, device="cpu",
+                       pin_memory=True)
     host.numpy()[:] = lists
     return host.to(device, non_blocking=True).unbind(0)
 

@@ -348,6 +348,17 @@ def test_row_tiles_of_a_step():
 
 
 @pytest.mark.gpu
+def test_row_tiles_under_a_default_device():
+    """A program that makes its tensors on the GPU by default: the lists pass through host
+    memory all the same."""
+    dev = torch.device("cuda", 0)
+    want = [t.tolist() for t in sm._row_tiles([130, 1, 64], 64, torch.device("cpu"))[1:]]
+    with dev:
+        got = sm._row_tiles([130, 1, 64], 64, dev)[1:]
+    assert [t.tolist() for t in got] == want and all(t.device == dev for t in got)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("dv", [4, 20, 64, 68, 128, 132, 256, 260, 33])
 def test_headnorm_gate_on_its_lanes(dtype, dv):
