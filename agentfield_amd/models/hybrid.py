@@ -400,16 +400,20 @@ class PolyNormMLP(nn.Module):
         return sm.matmul(self.rows(z), self.down)
 
 
-_ROWS_OF = {ChunkedAttention, GatedLinearAttention, Retention, PolyNormMLP}
+#: mixers and units whose forward is a product with what their `rows` returns, so written
+_ROWS_OF = {c: (c.forward, c.__call__)
+            for c in (ChunkedAttention, GatedLinearAttention, Retention, PolyNormMLP)}
 
 
 def _as_written(*modules) -> bool:
-    """Whether calling these modules is their class's forward and nothing else: no
-    subclass, no forward of the instance's own, no hooks that a call would run."""
+    """Whether calling these modules is their forward as written here and nothing else: no
+    subclass, no forward that the class or the instance was given later, no hooks that a call
+    would run."""
     if torch.nn.modules.module._has_any_global_hook():
         return False
     for m in modules:
-        if (type(m) not in _ROWS_OF or "forward" in m.__dict__
+        c = type(m)
+        if (_ROWS_OF.get(c) != (c.forward, c.__call__) or "forward" in m.__dict__
                 or m._compiled_call_impl is not None or m._forward_hooks or m._forward_pre_hooks
                 or m._backward_hooks or m._backward_pre_hooks):
             return False

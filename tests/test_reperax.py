@@ -1068,6 +1068,30 @@ def test_products_of_few_rows_left_alone():
         assert sm.matmul_group(pairs) is None
 
 
+def test_grouped_layer_only_as_written(monkeypatch):
+    """Mixers and units whose calls are not their forward as written run one by one: a
+    forward of the class's, given later, as one of the instance's, a subclass or a hook."""
+    from agentfield_amd.models import hybrid
+    model = hybrid.HYBRID_CONFIGS["reperax-tiny"].build_model("cpu")
+    layers = [[*layer.mixers.values(), layer.mlp] for layer in model.layers]
+    mods = [m for ms in layers for m in ms if m is not None]
+    assert hybrid._as_written(*mods)
+    for c in {type(m) for m in mods}:
+        for name in ("forward", "__call__"):
+            with monkeypatch.context() as patch:
+                patch.setattr(c, name, lambda self, *a, **kw: None)
+                assert not hybrid._as_written(*mods)
+        assert hybrid._as_written(*mods)
+    handle = mods[-1].register_forward_pre_hook(lambda m, a: None)
+    assert not hybrid._as_written(*mods)
+    handle.remove()
+    mods[0].forward = mods[0].forward
+    assert not hybrid._as_written(*mods)
+    del mods[0].forward
+    mods[0].__class__ = type("Own", (type(mods[0]),), {})
+    assert not hybrid._as_written(*mods)
+
+
 @pytest.mark.gpu
 def test_grouped_layer_and_its_hooks():
     """A layer of few rows gives the bits of its projections one by one, which is how it
