@@ -1471,7 +1471,7 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
                        const i32* positions, const i32* cu, const i32* q_start,
                        const i32* sslot, float q_scale, float k_scale,
                        float inv_tau, int T, int B, int H, int dk, int dv,
-                       int rot, i64 ldq, i64 ldk, i64 ldv, i64 ldz,
+                       int rot, i64 ldq, i64 ldk, i64 ldv, i64 ldz, bool one,
                        hipStream_t s) {
   const dim3 grid(B, H, (dv + 31) / 32), by_sequence(H, grid.z, B);
   const int rp = (dk + 15) / 16;
@@ -1502,7 +1502,9 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
                      (few || (!loads(256) && ((rpp == 8 && sizeof(S) == 2) ||
                                               T >= 128 * B)));
   const bool prompt = eight || loads(256);
-  const bool single = !prompt && T <= B;   // a token per sequence, as a rule
+  // Only where the caller says so: as many tokens as sequences may be one sequence's (50 of 51
+  // sequences, 16 heads of 16 x 32 11 us in blocks of 16, 47 one by one).
+  const bool single = !prompt && one;
   const size_t sm = (size_t)(single ? 1 : rpp >= 16 ? 8 : 16) * sizeof(float) *
                     (prompt ? 2 * (3 * 16 * rpp + 32) : 3 * 16 * rpp + 512 + 32);
 #define SCAN_ARGS                                                            \
@@ -1538,13 +1540,14 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
   return af_last_err();
 }
 
+// one: at most a token per sequence, as the caller knows it (any lengths are right).
 AF_EXPORT int afm_linear_scan(
     void* out, void* state, const void* q, const void* k, const void* v,
     const void* zl, const void* zbias, const void* head_decay,
     const void* inv_freq, const void* positions, const void* cu,
     const void* q_start, const void* sslot, float q_scale, float k_scale,
     float inv_tau, int T, int B, int H, int dk, int dv, int rot, i64 ldq,
-    i64 ldk, i64 ldv, i64 ldz, int dt, void* stream) {
+    i64 ldk, i64 ldv, i64 ldz, int dt, int one, void* stream) {
   if (B == 0) return 0;
   if (dk > 256 || dk < 1 || dv < 1) return 9003;
   if (rot < 0 || rot > dk || (rot & 1) || (rot && !inv_freq)) return 9003;
@@ -1556,12 +1559,12 @@ AF_EXPORT int afm_linear_scan(
         (const float*)zbias, (const float*)head_decay, (const float*)inv_freq,
         (const i32*)positions, (const i32*)cu, (const i32*)q_start,
         (const i32*)sslot, q_scale, k_scale, inv_tau, T, B, H, dk, dv, rot,
-        ldq, ldk, ldv, ldz, s);
+        ldq, ldk, ldv, ldz, one, s);
   if (dt == 1)
     return launch_scan<float>((float*)out, (float*)state, q, k, v, zl,
         (const float*)zbias, (const float*)head_decay, (const float*)inv_freq,
         (const i32*)positions, (const i32*)cu, (const i32*)q_start,
         (const i32*)sslot, q_scale, k_scale, inv_tau, T, B, H, dk, dv, rot,
-        ldq, ldk, ldv, ldz, s);
+        ldq, ldk, ldv, ldz, one, s);
   return 9002;
 }

@@ -188,7 +188,7 @@ def _mix_sigs() -> dict:
             "afm_attn_split_combine": [p, p, p, i, i, i, i, p, i64, i64, i,
                                        p],
             "afm_linear_scan": [p, p, p, p, p, p, p, p, p, p, p, p, p, f, f, f,
-                                i, i, i, i, i, i, i64, i64, i64, i64, i, p],
+                                i, i, i, i, i, i, i64, i64, i64, i64, i, i, p],
         },
         "conv": {
             "afm_causal_conv": [p, p, i64, p, p, p, p, p, p, p, p, i, i, i, i,

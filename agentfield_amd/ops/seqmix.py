@@ -600,9 +600,16 @@ def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         float(q_scale), float(k_scale), float(inv_tau), T, B, H, dk, dv, rot,
         _rowstride(q), _rowstride(k), _rowstride(v),
         _rowstride(decay_logits) if decay_logits is not None else 0,
-        _code(q), _lib.cur_stream())
+        _code(q), _one_each(md, T, B), _lib.cur_stream())
     _lib.check(rc, "afm_linear_scan")
     return out
+
+
+def _one_each(md, T: int, B: int) -> bool:
+    """Whether no sequence of the step has more than one row, as far as the host knows."""
+    lens = getattr(md, "seq_lens", None)
+    return T <= B and (not getattr(md, "is_prefill", True)
+                       or lens is not None and max(lens, default=0) <= 1)
 
 
 def headnorm_gate(o: torch.Tensor, g: torch.Tensor,

@@ -1034,6 +1034,47 @@ def test_scan_of_few_tokens(dtype, dk, gated):
     assert torch.equal(whole, parts) and torch.equal(state, other)
 
 
+def test_scan_knows_steps_of_one_token():
+    """Blocks of one token are for steps in which no sequence has more: decode steps and
+    chunks known to be as short, not any step of as many tokens as sequences."""
+    def one(T, B, **md):
+        return bool(sm._one_each(SimpleNamespace(**md), T, B))
+    assert one(6, 6, is_prefill=False) and one(6, 6, is_prefill=False, seq_lens=None)
+    assert one(2, 3, is_prefill=True, seq_lens=[1, 0, 1]) and one(0, 1, seq_lens=[])
+    assert not one(50, 51) and not one(50, 51, is_prefill=True)
+    assert not one(50, 51, is_prefill=True, seq_lens=[0] * 50 + [50])
+    assert not one(7, 6, is_prefill=False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dk", [30, 64, 128, 200])
+@pytest.mark.parametrize("lens", [[1] * 5, [1, 3, 0, 0, 1]])
+def test_scan_in_blocks_of_one_token(dtype, dk, lens):
+    """Bits of the larger blocks, in decode steps and, were one described as such, where a
+    sequence has several."""
+    H, dv = 3, 40
+    g = torch.Generator(device="cuda").manual_seed(dk)
+    q, k, v, z = ((torch.randn(5, n, generator=g, device="cuda") * s).to(dtype)
+                  for n, s in ((H * dk, dk ** -0.5), (H * dk, 0.3), (H * dv, 1.0),
+                               (H * dk, 1.0)))
+    before = torch.randn(6, H, dk, dv, generator=g, device="cuda")
+    pos = torch.cat([torch.arange(n) + 4 * i for i, n in enumerate(lens)]).int().cuda()
+    for kw in (dict(decay_logits=z, decay_bias=torch.ones(H * dk, device="cuda"),
+                    inv_tau=0.25),
+               dict(head_decay=torch.tensor([.9, .99, .5], device="cuda"))):
+        got = []
+        for prefill in (True, False):
+            md = SimpleNamespace(
+                is_prefill=prefill,
+                cu_seqlens=torch.tensor([0] + lens).cumsum(0).int().cuda(),
+                q_start=torch.tensor([4 * i for i in range(5)]).int().cuda(),
+                state_slots=torch.tensor([3, 1, 2, 5, 4]).int().cuda())
+            state = before.clone()
+            got.append((sm.linear_scan(q, k, v, state, md, pos, H, **kw), state))
+        assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 6, 16])
 @pytest.mark.parametrize("shapes", [
