@@ -1493,13 +1493,15 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
   // decay per head 61 / 50, 85 / 80, 118 / 122, 530 / 579; 256 rows, 64 groups 113 / 107,
   // 384 179 / 221.  fp32: 128 rows, 192 groups 101 / 82, 384 140 / 153; one decay per head
   // 73 / 55, 96 / 88, 768 133 / 136, 4096 609 / 640.  What only eight waves can load (rows in
-  // fours) is, on many groups, better off with them than with the token kernel in bf16 at 128
-  // rows (dk 100, 17 tokens 27 / 25), otherwise for longer prompts (fp32 17 tokens 32 / 44, 75
-  // tokens 97 / 98, 225 tokens 265 / 253).
+  // fours) is, on many groups, better off with them than with the token kernel at 128 rows in
+  // bf16 (dk 100, 17 tokens 27 / 25) and with one decay per head (fp32, dk 100, 560 groups, 17
+  // tokens 22 / 19, 50 tokens 47 / 31, 100 tokens 87 / 47; dk 124 breaks even at 24),
+  // otherwise for longer prompts (fp32 17 tokens 32 / 44, 75 tokens 97 / 98, 225 tokens
+  // 265 / 253).
   const i64 groups = (i64)B * H * grid.z;
   const bool few = groups <= (rpp >= 16 || (sizeof(S) == 4 && zl) ? 256 : 512);
   const bool eight = rpp >= 8 && loads(512) &&
-                     (few || (!loads(256) && ((rpp == 8 && sizeof(S) == 2) ||
+                     (few || (!loads(256) && ((rpp == 8 && (sizeof(S) == 2 || !zl)) ||
                                               T >= 128 * B)));
   const bool prompt = eight || loads(256);
   // Only where the caller says so: as many tokens as sequences may be one sequence's (50 of 51
