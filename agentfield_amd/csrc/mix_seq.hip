@@ -988,7 +988,11 @@ constexpr int scan_rows(int rp, int threads) {
 // longest met on one CU, or one started last: 6 sequences of 620..1900 tokens in 384
 // workgroups 430 -> 328 us, 32 of up to 1500 in 2048 1173 -> 660 and, with decays per channel,
 // 1312 -> 650.  A lane per sequence finds the ranks; more than 64 sequences keep their order
-// (70 of up to 700 tokens 864 -> 815, 995 -> 900).
+// (70 of up to 700 tokens 864 -> 815, 995 -> 900).  Steps of fewer than 64 tokens per sequence
+// walk a head of every sequence in turn (by_sequence, the host's word, is false): there a look
+// at the lengths, a load that the workgroup waits for, costs 1 us of 13 and the order as much
+// (8 sequences of 16 tokens, 16 heads of 128 x 128 12.8 -> 14.0, now 13.6; of 3, 17 and 40, 16
+// heads of 256 x 256 42 -> 47, now 42).
 struct ScanRows { int b, t0, t1; };
 __device__ __forceinline__ ScanRows scan_sequence(const i32* __restrict__ cu) {
   const int B = gridDim.z, turn = blockIdx.z;
@@ -1025,7 +1029,7 @@ linear_scan_prompt_kernel(
     const i32* __restrict__ positions, const i32* __restrict__ cu,
     const i32* __restrict__ q_start, const i32* __restrict__ sslot,
     float q_scale, float k_scale, float inv_tau, int H, int dk, int dv,
-    int rot, i64 ldq, i64 ldk, i64 ldv, i64 ldz) {
+    int rot, i64 ldq, i64 ldk, i64 ldv, i64 ldz, bool by_sequence) {
   constexpr int DKP = 16 * RP;
   constexpr bool FAST = sizeof(S) == 2;
   constexpr int TB = RP >= 16 ? 8 : 16;
@@ -1033,11 +1037,13 @@ linear_scan_prompt_kernel(
   constexpr int E = scan_rows(RP, NT);
   constexpr int BUF = TB * (3 * DKP + 32);     // [TB][3][DKP], [TB][32]
   extern __shared__ float smem[];
-  const ScanRows rows = scan_sequence(cu);
+  const ScanRows rows = by_sequence ? scan_sequence(cu)
+                                    : ScanRows{(int)blockIdx.x, cu[blockIdx.x], cu[blockIdx.x + 1]};
   const int b = __builtin_amdgcn_readfirstlane(rows.b);   // (known to be alike in all lanes)
   const int t0 = __builtin_amdgcn_readfirstlane(rows.t0);
   const int t1 = __builtin_amdgcn_readfirstlane(rows.t1);
-  const int h = blockIdx.x, c0 = blockIdx.y * 32;
+  const int h = by_sequence ? blockIdx.x : blockIdx.y;
+  const int c0 = (by_sequence ? blockIdx.y : blockIdx.z) * 32;
   if (t1 <= t0) return;
   const int r = threadIdx.x & 15, cc = threadIdx.x >> 4;
   const int ca = c0 + CPT * cc;
@@ -1473,7 +1479,7 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
                        float inv_tau, int T, int B, int H, int dk, int dv,
                        int rot, i64 ldq, i64 ldk, i64 ldv, i64 ldz, bool one,
                        hipStream_t s) {
-  const dim3 grid(B, H, (dv + 31) / 32), by_sequence(H, grid.z, B);
+  const dim3 grid(B, H, (dv + 31) / 32), ordered(H, grid.z, B);
   const int rp = (dk + 15) / 16;
   const int rpp = rp <= 2 ? 2 : rp <= 4 ? 4 : rp <= 8 ? 8 : 16;
   // From a block of tokens per sequence on the prompt kernel is the better one
@@ -1504,6 +1510,7 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
                      (few || (!loads(256) && ((rpp == 8 && (sizeof(S) == 2 || !zl)) ||
                                               T >= 128 * B)));
   const bool prompt = eight || loads(256);
+  const bool order = (i64)T >= 64 * (i64)B;    // see scan_sequence
   // Only where the caller says so: as many tokens as sequences may be one sequence's (50 of 51
   // sequences, 16 heads of 16 x 32 11 us in blocks of 16, 47 one by one).
   const bool single = !prompt && one;
@@ -1517,10 +1524,10 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
   do {                                                                       \
     if (zl)                                                                  \
       linear_scan_prompt_kernel<S, RP, true, NT>                             \
-          <<<by_sequence, NT, sm, s>>>(SCAN_ARGS);                           \
+          <<<order ? ordered : grid, NT, sm, s>>>(SCAN_ARGS, order);         \
     else                                                                     \
       linear_scan_prompt_kernel<S, RP, false, NT>                            \
-          <<<by_sequence, NT, sm, s>>>(SCAN_ARGS);                           \
+          <<<order ? ordered : grid, NT, sm, s>>>(SCAN_ARGS, order);         \
   } while (0)
 #define SCAN(RP)                                                             \
   do {                                                                       \
