@@ -955,11 +955,9 @@ __global__ void __launch_bounds__(256) linear_scan_kernel(
       const int tt = e >> 5, ci = e & 31;
       if (c0 + ci < dv) {
         const float* pr = part + tt * 512 + ci;
-        float o[16];  // summed in the order of row16_sum_all
+        float o[8];   // summed in the order of row16_sum_all
 #pragma unroll
-        for (int rr = 0; rr < 16; ++rr) o[rr] = pr[rr * 32];
-#pragma unroll
-        for (int rr = 0; rr < 8; ++rr) o[rr] += o[15 - rr];
+        for (int rr = 0; rr < 8; ++rr) o[rr] = pr[rr * 32] + pr[(15 - rr) * 32];
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) o[rr] += o[7 - rr];
         out[(size_t)(tb + tt) * H * dv + (size_t)h * dv + c0 + ci] =
