@@ -141,8 +141,10 @@ __global__ void __launch_bounds__(256) add_rows_kernel(
 
 // a = norm(x)(1+w1), b = norm(x)(1+w2), s = a + (a_prev - a)*shift.  Rows of up to R * 256
 // * V stay in registers, and all that the step behind the sum reads is asked for before it
-// (rows of 2048, six: 4.7 -> 3.9 us; 7636: 50 -> 38).  R = 0: any length.
-template <typename S, int V, int R>
+// (rows of 2048, six: 4.7 -> 3.9 us; 7636: 50 -> 38).  R = 1: threads past the row load
+// nothing (7636 rows of 64 8.8 us in the loop, 12.4 with all threads loading).  R = 0: any
+// length.  MORE: a second norm or the shift.
+template <typename S, int V, int R, bool MORE>
 __global__ void __launch_bounds__(256) dual_norm_shift_kernel(
     S* __restrict__ a_out, S* __restrict__ s_out, S* __restrict__ b_out,
     float* __restrict__ last, const float* __restrict__ x,
@@ -160,16 +162,17 @@ __global__ void __launch_bounds__(256) dual_norm_shift_kernel(
   const float* xp = xr - W;  // previous row, only touched when !first
   struct Cols { float x[4], w1[4], w2[4], mix[4], before[4]; };
   Cols at[R > 0 ? R : 1];
-  // (no branch between the loads: what is not there reads w1 again)
+  // (R > 0: no branch between the loads, what is not there reads w1 again)
   const S* w2r = b_out ? w2 : w1;
   const S* mixr = shift ? shift : w1;
   auto load = [&](int i, Cols& c) {
     ldv<float, V>(xr + i, c.x);
     ldv<S, V>(w1 + i, c.w1);
-    ldv<S, V>(w2r + i, c.w2);
-    ldv<S, V>(mixr + i, c.mix);
+    if (MORE && (R > 0 || b_out)) ldv<S, V>(w2r + i, c.w2);
+    if (MORE && (R > 0 || shift)) ldv<S, V>(mixr + i, c.mix);
   };
-  if (R > 0) {
+  const bool mine = R != 1 || (int)threadIdx.x * V < W;
+  if (R > 0 && mine) {
 #pragma unroll
     for (int r = 0; r < R; ++r)
       load(min((int)(threadIdx.x + r * 256) * V, W - V), at[r]);
@@ -179,10 +182,10 @@ __global__ void __launch_bounds__(256) dual_norm_shift_kernel(
   const bool first = (t == r0);
   const bool is_last = (t == cu[b + 1] - 1);
   const int pos = q_start[b] + (t - r0);
-  const bool need_prev_row = shift && !first;
+  const bool need_prev_row = MORE && shift && !first;
   // the row before, or what the state slot holds of it
   const float* bef = need_prev_row ? xp
-                     : (shift && pos > 0) ? prev + (size_t)sslot[b] * W : nullptr;
+                     : (MORE && shift && pos > 0) ? prev + (size_t)sslot[b] * W : nullptr;
   float ss[2] = {0.f, 0.f};
   auto load_before = [&](int i, Cols& c) {
     c.before[0] = c.before[1] = c.before[2] = c.before[3] = 0.f;
@@ -196,14 +199,14 @@ __global__ void __launch_bounds__(256) dual_norm_shift_kernel(
       for (int j = 0; j < V; ++j) ss[1] = fmaf(c.before[j], c.before[j], ss[1]);
     }
   };
-  if (R > 0) {
+  if (R > 0 && mine) {
 #pragma unroll
     for (int r = 0; r < R; ++r)
       load_before(min((int)(threadIdx.x + r * 256) * V, W - V), at[r]);
 #pragma unroll
     for (int r = 0; r < R; ++r)
       if ((int)(threadIdx.x + r * 256) * V < W) add(at[r]);
-  } else {
+  } else if (R == 0) {
     for (int i = threadIdx.x * V; i < W; i += 256 * V) {
       ldv<float, V>(xr + i, at[0].x);
       if (need_prev_row) ldv<float, V>(xp + i, at[0].before);
@@ -218,12 +221,12 @@ __global__ void __launch_bounds__(256) dual_norm_shift_kernel(
 #pragma unroll
     for (int j = 0; j < V; ++j) { g1[j] = c.w1[j] + 1.0f; a[j] = c.x[j] * r * g1[j]; }
     stv<S, V>(a_out + (size_t)t * W + i, a);
-    if (b_out) {
+    if (MORE && b_out) {
 #pragma unroll
       for (int j = 0; j < V; ++j) o[j] = c.x[j] * r * (1.0f + c.w2[j]);
       stv<S, V>(b_out + (size_t)t * W + i, o);
     }
-    if (shift) {
+    if (MORE && shift) {
       float ap[4];
 #pragma unroll
       for (int j = 0; j < V; ++j)
@@ -1197,15 +1200,22 @@ AF_EXPORT int afm_dual_norm_shift(
   hipStream_t s = (hipStream_t)stream;
   const bool vec = W % 4 == 0 && aligned16(a, s_out, b, last, x, w1) &&
                    aligned16(w2, shift, prev);
-#define DNS(ST, V, R)                                                         \
-  dual_norm_shift_kernel<ST, V, R><<<T, 256, 0, s>>>((ST*)a, (ST*)s_out, (ST*)b, \
-      (float*)last, (const float*)x, (const ST*)w1, (const ST*)w2,            \
+#define DNS(ST, V, R, MORE)                                                   \
+  dual_norm_shift_kernel<ST, V, R, MORE><<<T, 256, 0, s>>>((ST*)a, (ST*)s_out, \
+      (ST*)b, (float*)last, (const float*)x, (const ST*)w1, (const ST*)w2,    \
       (const ST*)shift, (float*)prev, (const i32*)row_seq,                    \
       (const i32*)cu, (const i32*)q_start, (const i32*)sslot, eps, W)
-  if (vec && W > 0 && W <= 2048) MIX_DISPATCH(dt, (DNS(u16, 4, 2)), (DNS(float, 4, 2)));
-  else if (vec && W > 0 && W <= 4096) MIX_DISPATCH(dt, (DNS(u16, 4, 4)), (DNS(float, 4, 4)));
-  else if (vec) MIX_DISPATCH(dt, (DNS(u16, 4, 0)), (DNS(float, 4, 0)));
-  else MIX_DISPATCH(dt, (DNS(u16, 1, 0)), (DNS(float, 1, 0)));
+#define DNW(ST, MORE)                                                         \
+  do {                                                                        \
+    if (!vec) DNS(ST, 1, 0, MORE);                                            \
+    else if (W <= 0 || W > 4096) DNS(ST, 4, 0, MORE);                         \
+    else if (W <= 1024) DNS(ST, 4, 1, MORE);                                  \
+    else if (W <= 2048) DNS(ST, 4, 2, MORE);                                  \
+    else DNS(ST, 4, 4, MORE);                                                 \
+  } while (0)
+  if (b || shift) MIX_DISPATCH(dt, DNW(u16, true), DNW(float, true));
+  else MIX_DISPATCH(dt, DNW(u16, false), DNW(float, false));
+#undef DNW
 #undef DNS
   return af_last_err();
 }

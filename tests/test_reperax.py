@@ -429,6 +429,33 @@ def test_row_kernels_around_their_register_rows(dtype, W):
         assert torch.equal(onc[1].cpu(), caches[1])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("W", [8, 1023, 1024, 1028, 4096, 4100])
+@pytest.mark.parametrize("second,shifted", [(False, False), (True, False), (False, True)])
+def test_norms_without_a_second_or_a_shift(dtype, W, second, shifted):
+    """Rows of a register round, around it and beyond, for layers that have one norm or no
+    token shift; tolerance as above."""
+    torch.manual_seed(W)
+    rel = 2 ** -7 if dtype == torch.bfloat16 else W ** 0.5 * 2 ** -22
+    x = torch.randn(5, W)
+    w1, w2, shift = (torch.rand(W).to(dtype) for _ in range(3))
+    args = (w1, w2 if second else None, shift if shifted else None)
+    prev = torch.randn(6, W)
+    md, _ = md_for([2, 3], [4, 0], [1, 2], "cpu")
+    on = SimpleNamespace(**{k: v.cuda() if torch.is_tensor(v) else v
+                            for k, v in vars(md).items()})
+    there = prev.cuda()
+    got = sm.dual_norm_shift(x.cuda(), *(None if a is None else a.cuda() for a in args),
+                             1e-6, there, on, dtype)
+    want = sm.dual_norm_shift(x, *args, 1e-6, prev, md, dtype)
+    for g, v in zip((*got, there), (*want, prev)):
+        assert (g is None) == (v is None)
+        if v is not None:
+            assert ((g.float().cpu() - v.float()).abs()
+                    <= v.float().abs() * rel + 2 ** -18).all()
+
+
 @pytest.mark.parametrize("device", DEVICES)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_chunk_edge_one_key_stands_out(device, dtype):
