@@ -53,11 +53,18 @@ __device__ __forceinline__ void stv(S* p, const float (&o)[4]) {
 }
 
 // Block-wide sum of up to N values per thread (256 threads); every thread
-// gets the totals.  red must hold N*4 floats.
-template <int N>
+// gets the totals.  red must hold N*4 floats.  SHUFFLE: wave_sum_f32's sums, in its order, by
+// the LDS unit, for kernels whose vector ALU many waves share.
+template <int N, bool SHUFFLE = false>
 __device__ __forceinline__ void block_sum(float (&v)[N], float* red) {
 #pragma unroll
-  for (int n = 0; n < N; ++n) v[n] = wave_sum_f32(v[n]);
+  for (int n = 0; n < N; ++n) {
+    if (!SHUFFLE) v[n] = wave_sum_f32(v[n]);
+  }
+#pragma unroll
+  for (int o = 32; SHUFFLE && o > 0; o >>= 1)
+#pragma unroll
+    for (int n = 0; n < N; ++n) v[n] += __shfl_xor(v[n], o, 64);
   const int wave = threadIdx.x >> 6;
   __syncthreads();  // red may still be read from a previous call
   if ((threadIdx.x & 63) == 0) {
@@ -718,8 +725,12 @@ __global__ void __launch_bounds__(256) narrow_product_kernel(
 }
 
 // Rows of up to R * 256 * V stay in registers: read once, all loads in flight together (rows
-// of 8192 bf16, six: 6.5 us read twice, 4.4 so; 7636: 58 us, 41).  R = 0: any length.
-template <typename S, int V, int R>
+// of 8192 bf16, six: 6.5 us read twice, 4.4 so; 7636: 58 us, 41), R = 1 by the threads that
+// the row has work for (7636 rows of 64 read twice 8.6 us, by all threads 11.6).  R = 0: any
+// length.  MANY: from some 2000 rows of 768 on the three sums go by the LDS unit, as the vector
+// ALU is what the blocks of a CU share (7636 x 1024 13.9 -> 12.5 us, x 2048 17.4 -> 16.0; rows of
+// 64 6.9 -> 8.4).
+template <typename S, int V, int R, bool MANY>
 __global__ void __launch_bounds__(256) polynorm_kernel(
     S* __restrict__ out, const S* __restrict__ z, const float* __restrict__ coef,
     float eps, int F, i64 ldz) {
@@ -737,7 +748,12 @@ __global__ void __launch_bounds__(256) polynorm_kernel(
       s[2] += v2 * v2 * v2;
     }
   };
-  if (R > 0) {
+  if (R == 1) {
+    if ((int)threadIdx.x * V < F) {
+      ldv<S, V>(zr + threadIdx.x * V, row[0]);
+      add(row[0]);
+    }
+  } else if (R > 0) {
 #pragma unroll
     for (int r = 0; r < R; ++r)
       ldv<S, V>(zr + min((int)(threadIdx.x + r * 256) * V, F - V), row[r]);
@@ -750,11 +766,11 @@ __global__ void __launch_bounds__(256) polynorm_kernel(
       add(row[0]);
     }
   }
-  const float c0 = coef[0], c1 = coef[1], c2 = coef[2], c3 = coef[3];
-  block_sum<3>(s, red);
+  block_sum<3, MANY>(s, red);
   const float r1 = 1.0f / sqrtf(s[0] / (float)F + eps);
   const float r2 = 1.0f / sqrtf(s[1] / (float)F + eps);
   const float r3 = 1.0f / sqrtf(s[2] / (float)F + eps);
+  const float c0 = coef[0], c1 = coef[1], c2 = coef[2], c3 = coef[3];
   auto put = [&](int i, const float (&v)[4]) {
     float o[4];
 #pragma unroll
@@ -1299,13 +1315,22 @@ AF_EXPORT int afm_polynorm(void* out, const void* z, const void* coef,
   if (T == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const bool vec = F % 4 == 0 && ldz % 4 == 0 && aligned16(out, z);
-#define PN(ST, V, R)                                                  \
-  polynorm_kernel<ST, V, R><<<T, 256, 0, s>>>((ST*)out, (const ST*)z,    \
-      (const float*)coef, eps, F, ldz)
-  if (vec && F > 0 && F <= 4096) MIX_DISPATCH(dt, (PN(u16, 4, 4)), (PN(float, 4, 4)));
-  else if (vec && F > 0 && F <= 8192) MIX_DISPATCH(dt, (PN(u16, 4, 8)), (PN(float, 4, 8)));
-  else if (vec) MIX_DISPATCH(dt, (PN(u16, 4, 0)), (PN(float, 4, 0)));
-  else MIX_DISPATCH(dt, (PN(u16, 1, 0)), (PN(float, 1, 0)));
+#define PN(ST, V, R, MANY)                                            \
+  polynorm_kernel<ST, V, R, MANY><<<T, 256, 0, s>>>((ST*)out,         \
+      (const ST*)z, (const float*)coef, eps, F, ldz)
+#define PNW(ST, MANY)                                                 \
+  do {                                                                \
+    if (!vec) PN(ST, 1, 0, MANY);                                     \
+    else if (F <= 0 || F > 8192) PN(ST, 4, 0, MANY);                  \
+    else if (F <= 1024) PN(ST, 4, 1, MANY);                           \
+    else if (F <= 2048) PN(ST, 4, 2, MANY);                           \
+    else if (F <= 4096) PN(ST, 4, 4, MANY);                           \
+    else PN(ST, 4, 8, MANY);                                          \
+  } while (0)
+  if (T >= 2000 && F >= 768) MIX_DISPATCH(dt, PNW(u16, true), PNW(float, true));
+  else MIX_DISPATCH(dt, PNW(u16, false), PNW(float, false));
+#undef PNW
+#undef PNW
 #undef PN
   return af_last_err();
 }

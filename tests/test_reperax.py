@@ -431,6 +431,17 @@ def test_row_kernels_around_their_register_rows(dtype, W):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("F", [764, 768, 771, 1024, 1028, 2052, 4100, 8196])
+def test_polynorm_of_many_rows(dtype, F):
+    """The sums of steps of many rows go another way in the same order: the bits of fewer."""
+    torch.manual_seed(F)
+    z, coef = torch.randn(2000, F, device="cuda").to(dtype), torch.rand(4, device="cuda")
+    got = sm.polynorm(z, coef, 1e-6)
+    assert torch.equal(got, torch.cat([sm.polynorm(p, coef, 1e-6) for p in z.split(999)]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("W", [8, 1023, 1024, 1028, 4096, 4100])
 @pytest.mark.parametrize("second,shifted", [(False, False), (True, False), (False, True)])
 def test_norms_without_a_second_or_a_shift(dtype, W, second, shifted):
