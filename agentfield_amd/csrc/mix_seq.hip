@@ -58,8 +58,9 @@ __device__ __forceinline__ void stvs(S* p, const float (&o)[4]) {
 
 // Rows of up to R * 256 * V stay in registers, and all that the kernel reads is asked for
 // before the sums (rows of 2048 and 1024: six 4.5 -> 3.5
-// us, 7636 30.3 -> 24.2).  R = 0: any length.
-template <typename S, int V, int R>
+// us, 7636 30.3 -> 24.2).  R = 1: threads past a row load nothing (7636 rows of 64 9.9 us in
+// the loop, 11.6 with all threads loading).  R = 0: any length.  NORM: weights for either.
+template <typename S, int V, int R, bool NORM>
 __global__ void __launch_bounds__(256) qk_norm_cache_kernel(
     S* __restrict__ qout, const S* __restrict__ q, const S* __restrict__ k,
     const S* __restrict__ v, const S* __restrict__ qw, const S* __restrict__ kw,
@@ -71,23 +72,34 @@ __global__ void __launch_bounds__(256) qk_norm_cache_kernel(
   const S* qr = q + (size_t)t * ldq;
   const S* kr = k + (size_t)t * ldk;
   const S* vr = v + (size_t)t * ldv;
-  // (no branch between the loads: without weights they read the rows again)
+  // (no branch between the loads: without weights of its own a side reads its row again)
   const S* qwr = qw ? qw : qr;
   const S* kwr = kw ? kw : kr;
   constexpr int N = R > 0 ? R : 1;
   float fq[N][4], fk[N][4], fv[N][4], wq[N][4], wk[N][4];
   const i64 sl = slots[t];
   float sq = 0.f, sk = 0.f;
-  if (R > 0) {
+  if (R == 1) {
+    const int i = threadIdx.x * V;
+    if (i < nq) ldvs<S, V>(qr + i, fq[0]);
+    if (i < nk) ldvs<S, V>(kr + i, fk[0]);
+    if (i < nv) ldvs<S, V>(vr + i, fv[0]);
+    if (NORM && i < nq) ldvs<S, V>(qwr + i, wq[0]);
+    if (NORM && i < nk) ldvs<S, V>(kwr + i, wk[0]);
+  }
+  if (R > 1) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int i = (threadIdx.x + r * 256) * V;
       ldvs<S, V>(qr + min(i, nq - V), fq[r]);
+      if (NORM) ldvs<S, V>(qwr + min(i, nq - V), wq[r]);
+      if (r > 0 && r * 256 * V >= max(nk, nv)) continue;   // few key heads
       ldvs<S, V>(kr + min(i, nk - V), fk[r]);
       ldvs<S, V>(vr + min(i, nv - V), fv[r]);
-      ldvs<S, V>(qwr + min(i, nq - V), wq[r]);
-      ldvs<S, V>(kwr + min(i, nk - V), wk[r]);
+      if (NORM) ldvs<S, V>(kwr + min(i, nk - V), wk[r]);
     }
+  }
+  if (R > 0) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int i = (threadIdx.x + r * 256) * V;
@@ -120,7 +132,7 @@ __global__ void __launch_bounds__(256) qk_norm_cache_kernel(
   const float rk = kw ? 1.0f / sqrtf((red[4] + red[5] + red[6] + red[7]) / (float)nk + eps) : 1.0f;
   const i64 pg = sl / page, off = sl % page;
   auto put_q = [&](int i, float (&f)[4], const float (&w4)[4]) {
-    if (qw) {
+    if (NORM && qw) {
 #pragma unroll
       for (int j = 0; j < V; ++j) f[j] *= rq * w4[j];
     }
@@ -128,7 +140,7 @@ __global__ void __launch_bounds__(256) qk_norm_cache_kernel(
   };
   auto put_k = [&](int i, float (&f)[4], const float (&w4)[4]) {
     const int g = i / dk, d = i % dk;
-    if (kw) {
+    if (NORM && kw) {
 #pragma unroll
       for (int j = 0; j < V; ++j) f[j] *= rk * w4[j];
     }
@@ -150,13 +162,13 @@ __global__ void __launch_bounds__(256) qk_norm_cache_kernel(
   }
   for (int i = threadIdx.x * V; i < nq; i += 256 * V) {
     ldvs<S, V>(qr + i, fq[0]);
-    ldvs<S, V>(qwr + i, wq[0]);
+    if (NORM) ldvs<S, V>(qwr + i, wq[0]);
     put_q(i, fq[0], wq[0]);
   }
   if (sl < 0) return;
   for (int i = threadIdx.x * V; i < nk; i += 256 * V) {
     ldvs<S, V>(kr + i, fk[0]);
-    ldvs<S, V>(kwr + i, wk[0]);
+    if (NORM) ldvs<S, V>(kwr + i, wk[0]);
     put_k(i, fk[0], wk[0]);
   }
   for (int i = threadIdx.x * V; i < nv; i += 256 * V) {
@@ -1284,21 +1296,22 @@ AF_EXPORT int afm_qk_norm_cache(
                    al(v) && al(qw) && al(kw) && al(kc) && al(vc);
   const int wide = max(nq, max(nk, nv));
   const bool any = nq > 0 && nk > 0 && nv > 0;
-#define QKN(ST, V, R)                                                         \
-  qk_norm_cache_kernel<ST, V, R><<<T, 256, 0, s>>>((ST*)qout, (const ST*)q,   \
+#define QKN(ST, V, R, NORM)                                                   \
+  qk_norm_cache_kernel<ST, V, R, NORM><<<T, 256, 0, s>>>((ST*)qout, (const ST*)q, \
       (const ST*)k, (const ST*)v, (const ST*)qw, (const ST*)kw, (ST*)kc,      \
       (ST*)vc, (const i64*)slots, eps, nq, nk, nv, G, dk, dv, page, ldq, ldk, \
       ldv)
-#define QKR(ST)                                                               \
+#define QKR(ST, NORM)                                                         \
   do {                                                                        \
-    if (vec && any && wide <= 2048) QKN(ST, 4, 2);                            \
-    else if (vec && any && wide <= 4096) QKN(ST, 4, 4);                       \
-    else if (vec) QKN(ST, 4, 0);                                              \
-    else QKN(ST, 1, 0);                                                       \
+    if (!vec) QKN(ST, 1, 0, NORM);                                            \
+    else if (!any || wide > 4096) QKN(ST, 4, 0, NORM);                        \
+    else if (wide <= 1024) QKN(ST, 4, 1, NORM);                               \
+    else if (wide <= 2048) QKN(ST, 4, 2, NORM);                               \
+    else QKN(ST, 4, 4, NORM);                                                 \
   } while (0)
-  if (dt == 0) QKR(u16);
-  else if (dt == 1) QKR(float);
-  else return 9002;
+  if (dt != 0 && dt != 1) return 9002;
+  if (qw || kw) { if (dt == 0) QKR(u16, true); else QKR(float, true); }
+  else { if (dt == 0) QKR(u16, false); else QKR(float, false); }
 #undef QKR
 #undef QKN
   return af_last_err();

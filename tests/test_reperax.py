@@ -442,6 +442,30 @@ def test_polynorm_of_many_rows(dtype, F):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nq,nk,nv", [(1024, 8, 1020), (12, 1024, 4), (3072, 128, 128),
+                                      (128, 4096, 1028), (4, 128, 2052), (4100, 8, 8)])
+@pytest.mark.parametrize("normed", [(1, 1), (1, 0), (0, 1), (0, 0)])
+def test_qk_norm_of_unlike_widths(dtype, nq, nk, nv, normed):
+    """Queries, keys and values of different register rounds, with weights for either, both
+    or none.  Tolerance as above."""
+    torch.manual_seed(nq)
+    rel = 2 ** -7 if dtype == torch.bfloat16 else max(nq, nk) ** 0.5 * 2 ** -22
+    q, k, v = (torch.randn(5, n).to(dtype) for n in (nq, nk, nv))
+    ws = [torch.rand(n).to(dtype) if on else None for n, on in zip((nq, nk), normed)]
+    slots = torch.tensor([3, 0, 7, 9, 4])
+    caches = [torch.zeros(3, 1, 4, n, dtype=dtype) for n in (nk, nv)]
+    onc = [c.cuda() for c in caches]
+    got = sm.qk_norm_cache(q.cuda(), k.cuda(), v.cuda(),
+                           *(None if w is None else w.cuda() for w in ws), 1e-6, *onc,
+                           slots.cuda())
+    want = sm.qk_norm_cache(q, k, v, *ws, 1e-6, *caches, slots)
+    for g, w in zip((got, onc[0]), (want, caches[0])):
+        assert ((g.cpu().float() - w.float()).abs() <= w.float().abs() * rel).all()
+    assert torch.equal(onc[1].cpu(), caches[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("W", [8, 1023, 1024, 1028, 4096, 4100])
 @pytest.mark.parametrize("second,shifted", [(False, False), (True, False), (False, True)])
 def test_norms_without_a_second_or_a_shift(dtype, W, second, shifted):
