@@ -679,10 +679,11 @@ __global__ void __launch_bounds__(256) headnorm_gate_lanes_kernel(
 // out [M, N] = x [M, K] @ w [N, K]^T for an inner dimension of at most KP (the upper half of a
 // low-rank projection): bound by writing out.  A thread keeps the weights of two columns, a
 // block R rows of x in LDS, read as broadcasts; sums in fp32 in the order of K.
-// Two rows per block while that gives no more than a few rounds of them (1000 x 1024 3.7 us,
-// 16 rows 5.6; 600 x 8192 9.3, 7.7).  Library / here, K 16: 6 x 1024 5.2 / 2.7 us, 210 x 1024
-// 4.1 / 2.8, 7636 x 1024 12.7 / 9.7, 30000 x 8192 198 / 159, 6 x 256 5.1 / 2.5.  With K 24 or
-// 32 the library is the faster one from 64 rows on (256 columns 4.2 / 7.1).
+// Two rows per block while that gives no more than a few rounds of them (1000 x 1024 3.4 us,
+// 16 rows 5.3; 5500 x 512 6.0, 5.9; 4000 x 1024 7.4, 6.4).  Library / here, K 16: 6 x 1024
+// 5.2 / 2.7 us, 210 x 1024 4.1 / 2.8, 4000 x 1024 7.0 / 6.4, 7636 x 1024 12.7 / 9.7, 30000 x
+// 8192 198 / 159, 6 x 256 5.1 / 2.5, 60000 x 256 13.5 / 14.4 (256 columns fill half a block).
+// With K 24 or 32 the library is the faster one from 64 rows on (256 columns 4.2 / 7.1).
 template <int KP, int R>
 __global__ void __launch_bounds__(256) narrow_product_kernel(
     u16* __restrict__ out, const u16* __restrict__ x, const u16* __restrict__ w, int M, int N,
@@ -1294,7 +1295,7 @@ AF_EXPORT int afm_headnorm_gate(void* out, const void* o, const void* g,
 AF_EXPORT int afm_narrow_product(void* out, const void* x, const void* w, int M, int N, int K,
                                  i64 ldx, void* stream) {
   if (M == 0) return 0;
-  const int R = (i64)M * N <= (4 << 20) ? 2 : 16;      // rows of a block
+  const int R = (i64)M * N <= (5 << 19) ? 2 : 16;      // rows of a block
   if (M < 0 || N < 2 || N % 2 || (K != 8 && K != 16) || ldx < K ||
       (uintptr_t)w % 16 || (uintptr_t)out % 4 || ((i64)M + R - 1) / R > 65535)
     return 9003;
