@@ -8,6 +8,8 @@
 #include "common.h"
 #include "mix_attn.h"
 
+#include <type_traits>
+
 namespace {
 
 template <typename S> __device__ __forceinline__ float ldf(const S* p);
@@ -277,7 +279,8 @@ __global__ void __launch_bounds__(256) masked_attention_kernel(
 //      rows are: its lines are fetched whole and once, where one key per lane
 //      walked 64 rows at a time and lost lines between its reads of them.  The
 //      query slices stay in registers; partial dot products meet in lane swaps
-//      and DPP.  One score per (head, key) in LDS, beside the key's page;
+//      and DPP, a lane ends with its share of them (scattered_sums).  One score
+//      per (head, key) in LDS, beside the key's page;
 //   B. per head: bias and cap, max, exp, sum over the tile (running max / sum /
 //      rescale factor kept in LDS across super-tiles);
 //   C. P.V: a value row is read by LPV adjacent lanes, each lane accumulates
@@ -288,10 +291,20 @@ __global__ void __launch_bounds__(256) masked_attention_kernel(
 // Few rows are bound by the chain position, block table, K, scores, V: its branches
 // on the lane layout and the page size stand outside the unrolled loops, and no
 // division is in it.  Eight key or value rows in flight per lane, or the next value rows
-// asked for ahead, cost more in wavefronts than they hid.  With the merge, heads of 128
-// over 8 K/V heads, one key per lane -> adjacent lanes: 6 rows of up to 512 keys 16.5 ->
-// 10.6 us, of 1000 keys 30.4 -> 17.8; 64 rows of 400 keys 43 -> 28; 128 rows of 3000 keys
-// 398 -> 289 us (5.4 TB/s); fp32, 6 rows of up to 512 keys 15.9 -> 12.3.
+// asked for ahead, cost more in wavefronts than they hid; with eight heads in bf16 two key
+// rows leave registers for a second wavefront.  Rows of 128 elements with the merge, one
+// key per lane -> adjacent lanes, us (diff: both maps of 16 heads):
+//     query / K/V heads    6 x 300 keys  6 x 1000     6 x 4000     128 x 1000
+//     bf16  8 / 8          14.3 -> 10.9  20.3 -> 12.4 45.6 -> 25.1 142 -> 93
+//          16 / 8          16.2 -> 11.9  22.3 -> 14.0 48.6 -> 26.8 145 -> 95
+//          32 / 8          27.5 -> 14.4  32.9 -> 16.9 66.8 -> 32.0 202 -> 109
+//          diff 16 / 8     32.2 -> 15.1  43.2 -> 21.2 87.7 -> 37.3 498 -> 147
+//          diff 16 / 4     47.6 -> 20.5  54.4 -> 22.7 102 -> 44.5  275 -> 119
+//     fp32 16 / 8          15.7 -> 13.1  26.5 -> 16.9 60.4 -> 38.6 228 -> 178
+//          32 / 8          18.6 -> 15.8  28.9 -> 19.3 62.7 -> 42.5 238 -> 180
+//          16 / 2          38.0 -> 21.3  41.5 -> 21.5 88.2 -> 51.2 123 -> 80
+// 128 rows of 3000 keys, 16 / 8 heads, 398 -> 289 us (5.4 TB/s).  Of 4382 shapes the worst are
+// fp32 heads of 33, 90 or 130 elements in groups of six, up to 1.1 of the time before.
 
 // Sixteen bytes of a row in storage type, for loads that stay in flight across other work;
 // zeros past the row's end.
@@ -329,22 +342,45 @@ __device__ __forceinline__ float add_quarter_f32(float v) {   // the other 16 of
   return __uint_as_float(a[0]) + __uint_as_float(a[1]);
 }
 
-// Each value's sum over groups of 1 << log2 adjacent lanes, in each of them (the branches,
-// which all lanes take together, once for all N values).
-template <int N>
-__device__ __forceinline__ void group_sums(float (&v)[N], int log2) {
-#define EACH(...) do { _Pragma("unroll") for (int i = 0; i < N; ++i) __VA_ARGS__; } while (0)
-  if (log2 > 0) EACH(v[i] += dpp_f32<0xB1>(v[i]));    // lanes 1 apart
-  if (log2 > 1) EACH(v[i] += dpp_f32<0x4E>(v[i]));    // 2 apart
-  if (log2 > 2) EACH(v[i] += dpp_f32<0x141>(v[i]));   // the other half of 8, mirrored
-  if (log2 > 3) EACH(v[i] += dpp_f32<0x140>(v[i]));   // the other half of 16, mirrored
-  if (log2 > 4) EACH(v[i] = add_quarter_f32(v[i]));
-  if (log2 > 5) EACH(v[i] = add_half_f32(v[i]));
+// One level of sums over lanes that differ in bit B of their number (mirrored within 16 lanes):
+// a lane without the bit gets a's sum, one with it b's.
+template <int B>
+__device__ __forceinline__ float meet(float a, float b, int lane) {
+  if constexpr (B == 5 || B == 4) {
+    const uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+    const auto r = B == 5 ? __builtin_amdgcn_permlane32_swap(x, y, false, false)
+                          : __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  } else {
+    const bool has = lane >> B & 1;
+    return (has ? b : a) + dpp_f32<B == 3 ? 0x140 : B == 2 ? 0x141 : B == 1 ? 0x4E : 0xB1>(
+                               has ? a : b);
+  }
 }
 
-// Each value's sum over the lanes with the same low log2 bits of their number, in each of them.
+// Sums of N values over groups of 1 << LOG2 adjacent lanes, each lane's share of them: value
+// i of a lane is that of index i << min(LOG2, log2 N) | its number's low LOG2 bits reversed
+// (the low ones of these where N is smaller).  Of every two values a lane hands its partner the
+// one that the partner goes on with: N additions where every lane's adding up all N takes
+// N * LOG2, half rate most of them (one row of 300 keys, 32 heads of 192 over 8 in fp32 23.8 ->
+// 19.8 us).
+template <int LOG2, int M, int N>
+__device__ __forceinline__ void scattered_sums(float (&v)[N], int lane) {
+  if constexpr (LOG2 > 0) {
+    constexpr int HALF = M > 1 ? M / 2 : 1;
+#pragma unroll
+    for (int i = 0; i < HALF; ++i)
+      v[i] = M > 1 ? meet<LOG2 - 1>(v[2 * i], v[2 * i + 1], lane)
+                   : meet<LOG2 - 1>(v[i], v[i], lane);
+    scattered_sums<LOG2 - 1, HALF>(v, lane);
+  }
+}
+
+// Each value's sum over the lanes with the same low log2 bits of their number, in each of them
+// (the branches, which all lanes take together, once for all N values).
 template <int N>
 __device__ __forceinline__ void strided_sums(float (&v)[N], int log2) {
+#define EACH(...) do { _Pragma("unroll") for (int i = 0; i < N; ++i) __VA_ARGS__; } while (0)
   if (log2 < 6) EACH(v[i] = add_half_f32(v[i]));
   if (log2 < 5) EACH(v[i] = add_quarter_f32(v[i]));
   // rotations within 16 lanes, whose halves, quarters, ... are alike by then
@@ -360,7 +396,7 @@ __device__ __forceinline__ void strided_sums(float (&v)[N], int log2) {
 // 2 gv + 1, so that a value row is read once for both; grid.y and G count
 // value heads, H all query heads.
 template <typename S, int GQ, bool VEC, int NK = 1>
-__global__ void __launch_bounds__(256) attn_rows_kernel(
+__global__ void __launch_bounds__(256, sizeof(S) == 2 && VEC && GQ == 4 ? 3 : 1) attn_rows_kernel(
     S* __restrict__ out, const S* __restrict__ q, const S* __restrict__ kc,
     const S* __restrict__ vc, const i32* __restrict__ bt,
     const i32* __restrict__ row_seq, const i32* __restrict__ positions,
@@ -373,7 +409,8 @@ __global__ void __launch_bounds__(256) attn_rows_kernel(
   // and (max, sum) go to part_o [T, H, nsplit, dv] / part_ml [T, H, nsplit,
   // 2] for attn_split_combine_kernel (or diff_combine_kernel) to merge.
   constexpr int EPL = 16 / sizeof(S);
-  constexpr int UK = 4, UV = 4;                // key and value rows in flight per lane
+  // key and value rows in flight per lane
+  constexpr int UK = sizeof(S) == 2 && GQ == 8 ? 2 : 4, UV = 4;
   extern __shared__ float smem[];
   const int dvp = EPL << lpv_log2;             // padded value width
   float* sc = smem;                            // [GQ][kt] scores, then probabilities
@@ -488,17 +525,28 @@ __global__ void __launch_bounds__(256) attn_rows_kernel(
           for (int e = 0; e < EPL; ++e) a[u * GQ + gg] += qv[gg][e] * kg[e];
         }
       }
-      group_sums(a, lpk_log2);
-      if (lik == 0) {
+      // a lane's share of the sums goes to LDS
+      auto scatter = [&](auto log2) {
+        constexpr int L = decltype(log2)::value, N = UK * GQ;
+        constexpr int LN = N >= 32 ? 5 : N >= 16 ? 4 : N >= 8 ? 3 : 2, LS = L < LN ? L : LN;
+        scattered_sums<L, N>(a, lane);
+        int l = lik;
+        asm volatile("" : "+v"(l));   // places in LDS of no layout are kept across rounds
+        if (L > LN && (l & ((1 << (L - LS)) - 1))) return;
+        const int mine = L > 0 ? (int)(__brev(l) >> (32 - L)) & ((1 << LS) - 1) : 0;
 #pragma unroll
-        for (int u = 0; u < UK; ++u) {
-          const int kidx = kb + u * 4 * kpk + kik;
-          if (kidx < nk) {
-#pragma unroll
-            for (int gg = 0; gg < GQ; ++gg) sc[gg * kt + kidx] = a[u * GQ + gg] * scale;
-          }
+        for (int i = 0; i < N >> LS; ++i) {
+          const int at = i << LS | mine, gg = at % GQ, kidx = kb + at / GQ * 4 * kpk + kik;
+          if (kidx < nk) sc[gg * kt + kidx] = a[i] * scale;
         }
-      }
+      };
+      if (lpk_log2 == 4) scatter(std::integral_constant<int, 4>());
+      else if (lpk_log2 == 3) scatter(std::integral_constant<int, 3>());
+      else if (lpk_log2 == 5) scatter(std::integral_constant<int, 5>());
+      else if (lpk_log2 == 6) scatter(std::integral_constant<int, 6>());
+      else if (lpk_log2 == 2) scatter(std::integral_constant<int, 2>());
+      else if (lpk_log2 == 1) scatter(std::integral_constant<int, 1>());
+      else scatter(std::integral_constant<int, 0>());
     }
     __syncthreads();
     // ---- B: softmax statistics, wave w takes heads w, w+4, ... ----

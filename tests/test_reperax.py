@@ -294,6 +294,16 @@ def test_row_attention_on_every_lane_layout(dtype, H, G, dk, dv, page, odd, monk
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("hpg", [1, 2, 4, 8])
+@pytest.mark.parametrize("dk", [3, 8, 12, 24, 40, 72, 136, 256])
+def test_row_attention_scatters_every_score(dtype, hpg, dk, monkeypatch):
+    """Groups of one to eight heads with key rows on 1 to 64 lanes: more scores than lanes
+    and fewer; against 64 bits as above."""
+    test_row_attention_on_every_lane_layout(dtype, 2 * hpg, 2, dk, 8, 16, 0, monkeypatch)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,G,dk,dv,page", [
     (4, 2, 128, 128, 16), (3, 3, 128, 128, 8), (4, 2, 64, 64, 16), (3, 1, 64, 56, 5),
     (2, 1, 100, 90, 7), (2, 1, 256, 256, 16), (1, 1, 264, 136, 6), (2, 1, 576, 512, 16),
