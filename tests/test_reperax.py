@@ -1106,6 +1106,33 @@ def test_scan_of_few_tokens(dtype, dk, gated):
     assert torch.equal(whole, parts) and torch.equal(state, other)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("step", [False, True])
+def test_decays_add_up_no_bias(step):
+    """Decays from logits in bf16 storage go by exp2 and log2 instructions: a state that only
+    decays, for 200 tokens, shows their mean error.  With exp and log of natural base it is
+    1.9e-9 a token at these logits; roundings of 6e-8 each leave 1e-10 over 400,000 decays."""
+    H, dk, n = 16, 128, 200
+    g = torch.Generator(device="cuda").manual_seed(0)
+    z = (torch.randn(n, H * dk, generator=g, device="cuda") + 3).bfloat16()
+    bias = torch.randn(H * dk, generator=g, device="cuda") * 0.1
+    zero = torch.zeros(n, H * dk, dtype=torch.bfloat16, device="cuda")
+    state = torch.ones(2, H, dk, 8, device="cuda")
+
+    def run(a, b):
+        md = SimpleNamespace(cu_seqlens=torch.tensor([0, b - a]).int().cuda(),
+                             q_start=torch.tensor([a + 1]).int().cuda(),
+                             state_slots=torch.tensor([1]).int().cuda(), is_prefill=not step)
+        sm.linear_scan(zero[a:b], zero[a:b], zero[a:b, :H * 8], state, md,
+                       torch.arange(a, b).int().cuda(), H, decay_logits=z[a:b],
+                       decay_bias=bias)
+    for a in range(0, n, 1 if step else n):
+        run(a, a + (1 if step else n))
+    want = torch.nn.functional.logsigmoid((z.float() + bias).to(F64)).sum(0).view(H, dk)
+    err = (state[1, :, :, 0].to(F64).log() - want).mean() / n
+    assert abs(err) < 1.9e-9
+
+
 def test_scan_knows_steps_of_one_token():
     """Blocks of one token are for steps in which no sequence has more: decode steps and
     chunks known to be as short, not any step of as many tokens as sequences."""
