@@ -55,8 +55,11 @@ __device__ __forceinline__ float group16_reduce_f32(float v, F f) {
 // ---- wave (64-lane) reductions: every lane ends with the result ----
 // Over the lanes 32, 16, 8, 4, 2 and 1 apart, in this order.  By lane swaps and DPP
 // operands: a shuffle is a round trip through the LDS unit, and small launches wait for
-// six of them in a row (RMSNorm of 64 x 4096, a wave per row, 5.93 us with shuffles, 5.78;
-// 64 x 512 2.34 and 2.21).  All lanes of the wave take part.
+// six of them in a row (six rows through a block each, with shuffles / so: a norm of 512
+// 2.74 us / 2.56, with the residual 2.77 / 2.62, with a mean first 3.19 / 2.88; heads of 128
+// normed and rotated 9.8 / 8.8).  Where many waves share a vector ALU it can lose (7636 rows,
+// two branches' norms of 1024 21.5 / 22.3): block_sum of the row kernels has shuffles for
+// those.  All lanes of the wave take part.
 template <class F>
 __device__ __forceinline__ float wave_reduce_f32(float v, F f) {
   const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v),

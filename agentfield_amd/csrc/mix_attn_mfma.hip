@@ -20,8 +20,11 @@
 // K/V heads, 7636 rows of six prompts: chunks of 512 152 -> 77 us, windows of 256 132 -> 68,
 // causal 302 -> 210; one K/V head per head 164 -> 113 (rows fetched a tile ahead, 142
 // without; for two heads per workgroup that costs the second workgroup, 77 -> 107); heads of
-// 256 226 -> 165; one latent of 576 for 16 heads 1081 -> 974.  Vector instructions are half of
-// what is left.
+// 256 226 -> 165; one latent of 576 for 16 heads 1081 -> 974.  The instance with every term
+// keeps 11 values in scratch for its second workgroup and gains as much: cap and window 126 ->
+// 77, bias 372 -> 241, 16 kept keys and a window of 512 209 -> 131, with bias 222 -> 139.
+// By counters, vector instructions fill 64% (chunks) to 72% (causal) of the SIMDs' time, the
+// matrix unit 14 and 15%; a wave waits for 52 to 56% of its own.
 //
 // Fragment layouts of v_mfma_f32_16x16x32_bf16 (64-lane wave):
 //   A: lane holds A[m = lane&15][k = (lane>>4)*8 + j], j = 0..7

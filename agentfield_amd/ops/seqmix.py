@@ -710,8 +710,8 @@ def matmul(x: torch.Tensor, w: torch.Tensor, skinny: bool = True,
 
     bf16 products of few rows (decode steps) run on the framework's
     weight-streaming kernels, wider ones and prompts on the vendor GEMM
-    (hipBLASLt / rocBLAS) or, where that has begun a round, on the wide GEMM; an inner
-    dimension of up to 16 has a kernel of its own (_narrow).  Above
+    (hipBLASLt / rocBLAS) or, where that has begun a round or divides its tiles badly, on
+    the wide GEMM; inner dimensions of 8 and 16 have a kernel of their own (_narrow).  Above
     16 rows a second launch adds the K splits up unless N fills the chip by itself,
     which middling widths do not earn back.
     Measured, vendor against rows in us: 4096 x 4096 15.7 / 7.8 at 4 rows, 15.3 /
