@@ -1048,22 +1048,32 @@ constexpr int scan_rows(int rp, int threads) {
 // The sequence of a workgroup, and its rows.  The grid walks sequence by sequence, and the
 // longest comes first where that decides what shares a CU and what is left to the end:
 // beyond one workgroup per CU (256).  With a head of every sequence in turn two of the
-// longest met on one CU, or one started last: 6 sequences of 620..1900 tokens in 384
-// workgroups 430 -> 328 us, 32 of up to 1500 in 2048 1173 -> 660 and, with decays per channel,
-// 1312 -> 650.  A lane per sequence finds the ranks; more than 64 sequences keep their order
-// (70 of up to 700 tokens 864 -> 815, 995 -> 900).  Steps of fewer than 64 tokens per sequence
-// walk a head of every sequence in turn (by_sequence, the host's word, is false): there a look
-// at the lengths, a load that the workgroup waits for, costs 1 us of 13 and the order as much
-// (8 sequences of 16 tokens, 16 heads of 128 x 128 12.8 -> 14.0, now 13.6; of 3, 17 and 40, 16
-// heads of 256 x 256 42 -> 47, now 42).
+// longest met on one CU, or one started last, and where their number shares a factor with 8
+// an XCD has some of them only: 6 sequences of 620..1900 tokens in 384 workgroups 430 -> 328
+// us, 32 of up to 1500 in 2048 1173 -> 660 and, with decays per channel, 1312 -> 650.  A lane
+// per sequence finds the ranks; more than 64 sequences keep their order (70 of up to 700
+// tokens 864 -> 815, 995 -> 900).
+// Below 64 tokens per sequence the look at the lengths, a load that the workgroup waits for,
+// costs 1 us of 13, and the ranks more with every sequence: the host says where they pay, with
+// up to 16 sequences whose lengths it knows to differ by 16 and up to 32 that differ by 64,
+// unless they fall already (in order / longest first: 8 and 12 of 3..114 in any order 1.05, 17
+// to 24 1.03 to 1.11, 32 1.01, 32 of 3..45 0.93; 8 of falling lengths 0.98, 24 0.94).  Else
+// they keep their order, and up to 256 workgroups a head of every sequence in turn.  1440
+// calls of 3..128 sequences against a head of each in turn everywhere: 0.81 of it in the mean
+// (16 of 10..76, 16 heads of 256 x 256 165 -> 119 us, 64 of 25..75, 16 of 128 x 128 in fp32
+// 257 -> 203), lengths alike 1.00, at most 1.04.
+enum ScanLengths { LENS_UNKNOWN, LENS_ONE, LENS_DIFFER };   // at most a token each, unlike
+enum ScanWalk { HEADS_IN_TURN, IN_ORDER, LONGEST_FIRST, LONGEST_FIRST_SHORT };
 struct ScanRows { int b, t0, t1; };
-__device__ __forceinline__ ScanRows scan_sequence(const i32* __restrict__ cu) {
+__device__ __forceinline__ ScanRows scan_sequence(const i32* __restrict__ cu, int walk) {
   const int B = gridDim.z, turn = blockIdx.z;
-  if (B > 64 || B * gridDim.x * gridDim.y <= 256) return {turn, cu[turn], cu[turn + 1]};
+  if (walk == IN_ORDER || B > 64 || B * gridDim.x * gridDim.y <= 256)
+    return {turn, cu[turn], cu[turn + 1]};
   const int lane = min((int)threadIdx.x & 63, B - 1);
   const int from = cu[lane], len = cu[lane + 1] - from;
   // (lengths alike: nothing to win, and the ranks cost short ones 1 us of 48)
-  if (__builtin_amdgcn_readfirstlane(wave_max_f32((float)len) +
+  if (walk == LONGEST_FIRST &&
+      __builtin_amdgcn_readfirstlane(wave_max_f32((float)len) +
                                      wave_max_f32((float)-len) < 64.f))
     return {turn, __builtin_amdgcn_readlane(from, turn),
             __builtin_amdgcn_readlane(from, turn) + __builtin_amdgcn_readlane(len, turn)};
@@ -1092,7 +1102,7 @@ linear_scan_prompt_kernel(
     const i32* __restrict__ positions, const i32* __restrict__ cu,
     const i32* __restrict__ q_start, const i32* __restrict__ sslot,
     float q_scale, float k_scale, float inv_tau, int H, int dk, int dv,
-    int rot, i64 ldq, i64 ldk, i64 ldv, i64 ldz, bool by_sequence) {
+    int rot, i64 ldq, i64 ldk, i64 ldv, i64 ldz, int walk) {
   constexpr int DKP = 16 * RP;
   constexpr bool FAST = sizeof(S) == 2;
   constexpr int TB = RP >= 16 ? 8 : 16;
@@ -1100,7 +1110,8 @@ linear_scan_prompt_kernel(
   constexpr int E = scan_rows(RP, NT);
   constexpr int BUF = TB * (3 * DKP + 32);     // [TB][3][DKP], [TB][32]
   extern __shared__ float smem[];
-  const ScanRows rows = by_sequence ? scan_sequence(cu)
+  const bool by_sequence = walk != HEADS_IN_TURN;
+  const ScanRows rows = by_sequence ? scan_sequence(cu, walk)
                                     : ScanRows{(int)blockIdx.x, cu[blockIdx.x], cu[blockIdx.x + 1]};
   const int b = __builtin_amdgcn_readfirstlane(rows.b);   // (known to be alike in all lanes)
   const int t0 = __builtin_amdgcn_readfirstlane(rows.t0);
@@ -1541,7 +1552,7 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
                        const i32* positions, const i32* cu, const i32* q_start,
                        const i32* sslot, float q_scale, float k_scale,
                        float inv_tau, int T, int B, int H, int dk, int dv,
-                       int rot, i64 ldq, i64 ldk, i64 ldv, i64 ldz, bool one,
+                       int rot, i64 ldq, i64 ldk, i64 ldv, i64 ldz, int known,
                        hipStream_t s) {
   const dim3 grid(B, H, (dv + 31) / 32), ordered(H, grid.z, B);
   const int rp = (dk + 15) / 16;
@@ -1574,10 +1585,12 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
                      (few || (!loads(256) && ((rpp == 8 && (sizeof(S) == 2 || !zl)) ||
                                               T >= 128 * B)));
   const bool prompt = eight || loads(256);
-  const bool order = (i64)T >= 64 * (i64)B;    // see scan_sequence
+  const int walk = (i64)T >= 64 * (i64)B ? LONGEST_FIRST    // see scan_sequence
+                   : groups <= 256        ? HEADS_IN_TURN
+                   : known == LENS_DIFFER ? LONGEST_FIRST_SHORT : IN_ORDER;
   // Only where the caller says so: as many tokens as sequences may be one sequence's (50 of 51
   // sequences, 16 heads of 16 x 32 11 us in blocks of 16, 47 one by one).
-  const bool single = !prompt && one;
+  const bool single = !prompt && known == LENS_ONE;
   const size_t sm = (size_t)(single ? 1 : rpp >= 16 ? 8 : 16) * sizeof(float) *
                     (prompt ? 2 * (3 * 16 * rpp + 32) : 3 * 16 * rpp + 512 + 32);
 #define SCAN_ARGS                                                            \
@@ -1588,10 +1601,10 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
   do {                                                                       \
     if (zl)                                                                  \
       linear_scan_prompt_kernel<S, RP, true, NT>                             \
-          <<<order ? ordered : grid, NT, sm, s>>>(SCAN_ARGS, order);         \
+          <<<walk ? ordered : grid, NT, sm, s>>>(SCAN_ARGS, walk);           \
     else                                                                     \
       linear_scan_prompt_kernel<S, RP, false, NT>                            \
-          <<<order ? ordered : grid, NT, sm, s>>>(SCAN_ARGS, order);         \
+          <<<walk ? ordered : grid, NT, sm, s>>>(SCAN_ARGS, walk);           \
   } while (0)
 #define SCAN(RP)                                                             \
   do {                                                                       \
@@ -1613,14 +1626,14 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
   return af_last_err();
 }
 
-// one: at most a token per sequence, as the caller knows it (any lengths are right).
+// known: what the caller knows of the lengths (ScanLengths; any lengths are right).
 AF_EXPORT int afm_linear_scan(
     void* out, void* state, const void* q, const void* k, const void* v,
     const void* zl, const void* zbias, const void* head_decay,
     const void* inv_freq, const void* positions, const void* cu,
     const void* q_start, const void* sslot, float q_scale, float k_scale,
     float inv_tau, int T, int B, int H, int dk, int dv, int rot, i64 ldq,
-    i64 ldk, i64 ldv, i64 ldz, int dt, int one, void* stream) {
+    i64 ldk, i64 ldv, i64 ldz, int dt, int known, void* stream) {
   if (B == 0) return 0;
   if (dk > 256 || dk < 1 || dv < 1) return 9003;
   if (rot < 0 || rot > dk || (rot & 1) || (rot && !inv_freq)) return 9003;
@@ -1632,12 +1645,12 @@ AF_EXPORT int afm_linear_scan(
         (const float*)zbias, (const float*)head_decay, (const float*)inv_freq,
         (const i32*)positions, (const i32*)cu, (const i32*)q_start,
         (const i32*)sslot, q_scale, k_scale, inv_tau, T, B, H, dk, dv, rot,
-        ldq, ldk, ldv, ldz, one, s);
+        ldq, ldk, ldv, ldz, known, s);
   if (dt == 1)
     return launch_scan<float>((float*)out, (float*)state, q, k, v, zl,
         (const float*)zbias, (const float*)head_decay, (const float*)inv_freq,
         (const i32*)positions, (const i32*)cu, (const i32*)q_start,
         (const i32*)sslot, q_scale, k_scale, inv_tau, T, B, H, dk, dv, rot,
-        ldq, ldk, ldv, ldz, one, s);
+        ldq, ldk, ldv, ldz, known, s);
   return 9002;
 }

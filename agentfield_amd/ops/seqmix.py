@@ -20,6 +20,7 @@ do not depend on where a prompt was cut into chunks.
 from __future__ import annotations
 
 import ctypes
+import itertools
 import math
 import os
 import sys
@@ -600,7 +601,7 @@ def linear_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         float(q_scale), float(k_scale), float(inv_tau), T, B, H, dk, dv, rot,
         _rowstride(q), _rowstride(k), _rowstride(v),
         _rowstride(decay_logits) if decay_logits is not None else 0,
-        _code(q), _one_each(md, T, B), _lib.cur_stream())
+        _code(q), _known_lens(md, T, B), _lib.cur_stream())
     _lib.check(rc, "afm_linear_scan")
     return out
 
@@ -610,6 +611,19 @@ def _one_each(md, T: int, B: int) -> bool:
     lens = getattr(md, "seq_lens", None)
     return T <= B and (not getattr(md, "is_prefill", True)
                        or lens is not None and max(lens, default=0) <= 1)
+
+
+def _known_lens(md, T: int, B: int) -> int:
+    """What the host knows of a step's lengths, for the recurrence's choice of blocks and
+    of their order: 1 no sequence has more than one row, 2 up to 16 short ones differ by 16
+    rows or more, up to 32 by 64, and a longer one follows a shorter, 0 anything else."""
+    if _one_each(md, T, B):
+        return 1
+    lens = getattr(md, "seq_lens", None)
+    if not lens or B > 32 or T >= 64 * B:
+        return 0
+    unlike = max(lens) - min(lens) >= (16 if B <= 16 else 64)
+    return 2 if unlike and any(a < b for a, b in itertools.pairwise(lens)) else 0
 
 
 def headnorm_gate(o: torch.Tensor, g: torch.Tensor,

@@ -5,6 +5,7 @@ the engine's cache, state slots, batching, scheduler and generation.
 Each test runs on the CPU op path and, marked gpu, on the gfx950 kernels.
 fp32 runs are held to rounding-level agreement; bf16 runs to bf16 rounding.
 """
+import itertools
 import json
 import math
 import subprocess
@@ -1143,6 +1144,51 @@ def test_scan_knows_steps_of_one_token():
     assert not one(50, 51) and not one(50, 51, is_prefill=True)
     assert not one(50, 51, is_prefill=True, seq_lens=[0] * 50 + [50])
     assert not one(7, 6, is_prefill=False)
+
+
+def test_scan_knows_short_prompts_of_unlike_lengths():
+    def known(T, B, **md):
+        return sm._known_lens(SimpleNamespace(**md), T, B)
+    assert known(6, 6, is_prefill=False) == 1 == known(2, 3, seq_lens=[1, 0, 1])
+    assert known(60, 3, seq_lens=[3, 17, 40]) == 2 == known(60, 3, seq_lens=[30, 0, 30])
+    assert known(336, 16, seq_lens=[20] * 15 + [36]) == 2
+    assert known(704, 32, seq_lens=[20] * 31 + [84]) == 2
+    for lens in ([20, 20, 20], [10, 25, 25], [40, 17, 3], [20] * 16 + [83],
+                 [20] * 32 + [84], [40, 200]):
+        assert known(sum(lens), len(lens), seq_lens=lens) == 0
+    assert known(60, 3) == 0 == known(60, 3, seq_lens=None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dk,dv", [(64, 40), (128, 128), (256, 64)])
+@pytest.mark.parametrize("lens", [[20, 17], [20] * 9, [60] * 9, [0, 40, 3, 70, 33, 16, 1, 40, 25],
+                                  [3, 17, 40], [5, 90, 20, 64] * 16, [30, 10] * 35])
+def test_scan_in_any_order_of_its_sequences(dtype, dk, dv, lens):
+    """The bits of each sequence alone, whichever way the grid walks them: few workgroups and
+    many, alike and not, known to be so or not, more sequences than lanes."""
+    H, B, T = 16, len(lens), sum(lens)
+    g = torch.Generator(device="cuda").manual_seed(dk)
+    q, k, v, z = ((torch.randn(T, n, generator=g, device="cuda") * s).to(dtype)
+                  for n, s in ((H * dk, dk ** -0.5), (H * dk, 0.3), (H * dv, 1.0),
+                               (H * dk, 1.0)))
+    before = torch.randn(B, H, dk, dv, generator=g, device="cuda")
+    kw = dict(decay_bias=torch.ones(H * dk, device="cuda"), inv_tau=0.25)
+    cu = [0, *itertools.accumulate(lens)]
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+
+    def run(first, last, state, **known):
+        a, b = cu[first], cu[last]
+        md = SimpleNamespace(cu_seqlens=i32(cu[first:last + 1]) - a,
+                             q_start=i32([4] * (last - first)),
+                             state_slots=i32(range(last - first)), is_prefill=True, **known)
+        return sm.linear_scan(q[a:b], k[a:b], v[a:b], state, md, i32(range(a, b)), H,
+                              decay_logits=z[a:b], **kw)
+    alone = before.clone()
+    want = torch.cat([run(i, i + 1, alone[i:i + 1]) for i in range(B) if lens[i]])
+    for known in ({}, {"seq_lens": lens}):
+        state = before.clone()
+        assert torch.equal(run(0, B, state, **known), want) and torch.equal(state, alone)
 
 
 @pytest.mark.gpu
