@@ -58,11 +58,13 @@ __device__ __forceinline__ void stvs(S* p, const float (&o)[4]) {
   }
 }
 
-// Rows of up to R * 256 * V stay in registers, and all that the kernel reads is asked for
-// before the sums (rows of 2048 and 1024: six 4.5 -> 3.5
-// us, 7636 30.3 -> 24.2).  R = 1: threads past a row load nothing (7636 rows of 64 9.9 us in
-// the loop, 11.6 with all threads loading).  R = 0: any length.  NORM: weights for either.
-template <typename S, int V, int R, bool NORM>
+// Rows of up to R * 256 * V stay in registers, keys and values in the first RK rounds, and all
+// that the kernel reads is asked for before the sums, without a branch between (rows of 2048
+// and 1024: six 4.5 -> 3.6 us, 7636 30.3 -> 23.2; with a branch around the further rounds of
+// the keys 7636 x 4096 / 2048 48, 41 without).  PART: waves past a row load nothing (7636 rows
+// of 64 9.9 us in the loop, 11.6 with all threads loading; from 768 on all have a share, and
+// the branch costs 0.15 us of 3).  R = 0: any length.  NORM: weights for either.
+template <typename S, int V, int R, int RK, bool NORM, bool PART>
 __global__ void __launch_bounds__(256) qk_norm_cache_kernel(
     S* __restrict__ qout, const S* __restrict__ q, const S* __restrict__ k,
     const S* __restrict__ v, const S* __restrict__ qw, const S* __restrict__ kw,
@@ -81,24 +83,16 @@ __global__ void __launch_bounds__(256) qk_norm_cache_kernel(
   float fq[N][4], fk[N][4], fv[N][4], wq[N][4], wk[N][4];
   const i64 sl = slots[t];
   float sq = 0.f, sk = 0.f;
-  if (R == 1) {
-    const int i = threadIdx.x * V;
-    if (i < nq) ldvs<S, V>(qr + i, fq[0]);
-    if (i < nk) ldvs<S, V>(kr + i, fk[0]);
-    if (i < nv) ldvs<S, V>(vr + i, fv[0]);
-    if (NORM && i < nq) ldvs<S, V>(qwr + i, wq[0]);
-    if (NORM && i < nk) ldvs<S, V>(kwr + i, wk[0]);
-  }
-  if (R > 1) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63);
+  if (R > 0 && (!PART || wave * V < max(nq, max(nk, nv)))) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int i = (threadIdx.x + r * 256) * V;
       ldvs<S, V>(qr + min(i, nq - V), fq[r]);
+      if (r < RK) ldvs<S, V>(kr + min(i, nk - V), fk[r]);
+      if (r < RK) ldvs<S, V>(vr + min(i, nv - V), fv[r]);
       if (NORM) ldvs<S, V>(qwr + min(i, nq - V), wq[r]);
-      if (r > 0 && r * 256 * V >= max(nk, nv)) continue;   // few key heads
-      ldvs<S, V>(kr + min(i, nk - V), fk[r]);
-      ldvs<S, V>(vr + min(i, nv - V), fv[r]);
-      if (NORM) ldvs<S, V>(kwr + min(i, nk - V), wk[r]);
+      if (NORM && r < RK) ldvs<S, V>(kwr + min(i, nk - V), wk[r]);
     }
   }
   if (R > 0) {
@@ -108,7 +102,7 @@ __global__ void __launch_bounds__(256) qk_norm_cache_kernel(
 #pragma unroll
       for (int j = 0; j < V; ++j) {
         if (i < nq) sq += fq[r][j] * fq[r][j];
-        if (i < nk) sk += fk[r][j] * fk[r][j];
+        if (r < RK && i < nk) sk += fk[r][j] * fk[r][j];
       }
     }
   } else {
@@ -157,8 +151,8 @@ __global__ void __launch_bounds__(256) qk_norm_cache_kernel(
     for (int r = 0; r < R; ++r) {
       const int i = (threadIdx.x + r * 256) * V;
       if (i < nq) put_q(i, fq[r], wq[r]);
-      if (i < nk && sl >= 0) put_k(i, fk[r], wk[r]);
-      if (i < nv && sl >= 0) put_v(i, fv[r]);
+      if (r < RK && i < nk && sl >= 0) put_k(i, fk[r], wk[r]);
+      if (r < RK && i < nv && sl >= 0) put_v(i, fv[r]);
     }
     return;
   }
@@ -1059,7 +1053,7 @@ constexpr int scan_rows(int rp, int threads) {
 // unless they fall already (in order / longest first: 8 and 12 of 3..114 in any order 1.05, 17
 // to 24 1.03 to 1.11, 32 1.01, 32 of 3..45 0.93; 8 of falling lengths 0.98, 24 0.94).  Else
 // they keep their order, and up to 256 workgroups a head of every sequence in turn.  1440
-// calls of 3..128 sequences against a head of each in turn everywhere: 0.81 of it in the mean
+// calls of 3..128 sequences against a head of each in turn everywhere: 0.80 of it in the mean
 // (16 of 10..76, 16 heads of 256 x 256 165 -> 119 us, 64 of 25..75, 16 of 128 x 128 in fp32
 // 257 -> 203), lengths alike 1.00, at most 1.04.
 enum ScanLengths { LENS_UNKNOWN, LENS_ONE, LENS_DIFFER };   // at most a token each, unlike
@@ -1360,18 +1354,23 @@ AF_EXPORT int afm_qk_norm_cache(
                    al(v) && al(qw) && al(kw) && al(kc) && al(vc);
   const int wide = max(nq, max(nk, nv));
   const bool any = nq > 0 && nk > 0 && nv > 0;
-#define QKN(ST, V, R, NORM)                                                   \
-  qk_norm_cache_kernel<ST, V, R, NORM><<<T, 256, 0, s>>>((ST*)qout, (const ST*)q, \
+  const int narrow = max(nk, nv);
+#define QKN(ST, V, R, RK, NORM, PART)                                         \
+  qk_norm_cache_kernel<ST, V, R, RK, NORM, PART><<<T, 256, 0, s>>>((ST*)qout, (const ST*)q, \
       (const ST*)k, (const ST*)v, (const ST*)qw, (const ST*)kw, (ST*)kc,      \
       (ST*)vc, (const i64*)slots, eps, nq, nk, nv, G, dk, dv, page, ldq, ldk, \
       ldv)
 #define QKR(ST, NORM)                                                         \
   do {                                                                        \
-    if (!vec) QKN(ST, 1, 0, NORM);                                            \
-    else if (!any || wide > 4096) QKN(ST, 4, 0, NORM);                        \
-    else if (wide <= 1024) QKN(ST, 4, 1, NORM);                               \
-    else if (wide <= 2048) QKN(ST, 4, 2, NORM);                               \
-    else QKN(ST, 4, 4, NORM);                                                 \
+    if (!vec) QKN(ST, 1, 0, 0, NORM, false);                                  \
+    else if (!any || wide > 4096) QKN(ST, 4, 0, 0, NORM, false);              \
+    else if (wide <= 768) QKN(ST, 4, 1, 1, NORM, true);                       \
+    else if (wide <= 1024) QKN(ST, 4, 1, 1, NORM, false);                     \
+    else if (wide <= 2048 && narrow <= 1024) QKN(ST, 4, 2, 1, NORM, false);   \
+    else if (wide <= 2048) QKN(ST, 4, 2, 2, NORM, false);                     \
+    else if (narrow <= 1024) QKN(ST, 4, 4, 1, NORM, false);                   \
+    else if (narrow <= 2048) QKN(ST, 4, 4, 2, NORM, false);                   \
+    else QKN(ST, 4, 4, 4, NORM, false);                                       \
   } while (0)
   if (dt != 0 && dt != 1) return 9002;
   if (qw || kw) { if (dt == 0) QKR(u16, true); else QKR(float, true); }

@@ -454,7 +454,9 @@ def test_polynorm_of_many_rows(dtype, F):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("nq,nk,nv", [(1024, 8, 1020), (12, 1024, 4), (3072, 128, 128),
-                                      (128, 4096, 1028), (4, 128, 2052), (4100, 8, 8)])
+                                      (128, 4096, 1028), (4, 128, 2052), (4100, 8, 8),
+                                      (768, 768, 4), (772, 4, 772), (2048, 1028, 8),
+                                      (2052, 1024, 1024), (4096, 8, 1028), (4096, 2052, 4)])
 @pytest.mark.parametrize("normed", [(1, 1), (1, 0), (0, 1), (0, 0)])
 def test_qk_norm_of_unlike_widths(dtype, nq, nk, nv, normed):
     """Queries, keys and values of different register rounds, with weights for either, both
