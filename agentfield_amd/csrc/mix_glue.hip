@@ -150,8 +150,9 @@ __global__ void __launch_bounds__(256) add_rows_kernel(
 // * V stay in registers, and all that the step behind the sum reads is asked for before it
 // (rows of 2048, six: 4.7 -> 3.9 us; 7636: 50 -> 38).  R = 1: threads past the row load
 // nothing (7636 rows of 64 8.8 us in the loop, 12.4 with all threads loading).  R = 0: any
-// length.  MORE: a second norm or the shift.
-template <typename S, int V, int R, bool MORE>
+// length.  SECOND, SHIFTED: with b, with s; a branch around their loads in the loop instead
+// costs rows of 8192 7 to 10% (six 17.8 -> 19.2 us), what is not there read as w1 up to 3%.
+template <typename S, int V, int R, bool SECOND, bool SHIFTED>
 __global__ void __launch_bounds__(256) dual_norm_shift_kernel(
     S* __restrict__ a_out, S* __restrict__ s_out, S* __restrict__ b_out,
     float* __restrict__ last, const float* __restrict__ x,
@@ -169,14 +170,11 @@ __global__ void __launch_bounds__(256) dual_norm_shift_kernel(
   const float* xp = xr - W;  // previous row, only touched when !first
   struct Cols { float x[4], w1[4], w2[4], mix[4], before[4]; };
   Cols at[R > 0 ? R : 1];
-  // (R > 0: no branch between the loads, what is not there reads w1 again)
-  const S* w2r = b_out ? w2 : w1;
-  const S* mixr = shift ? shift : w1;
   auto load = [&](int i, Cols& c) {
     ldv<float, V>(xr + i, c.x);
     ldv<S, V>(w1 + i, c.w1);
-    if (MORE && (R > 0 || b_out)) ldv<S, V>(w2r + i, c.w2);
-    if (MORE && (R > 0 || shift)) ldv<S, V>(mixr + i, c.mix);
+    if (SECOND) ldv<S, V>(w2 + i, c.w2);
+    if (SHIFTED) ldv<S, V>(shift + i, c.mix);
   };
   const bool mine = R != 1 || (int)threadIdx.x * V < W;
   if (R > 0 && mine) {
@@ -189,10 +187,10 @@ __global__ void __launch_bounds__(256) dual_norm_shift_kernel(
   const bool first = (t == r0);
   const bool is_last = (t == cu[b + 1] - 1);
   const int pos = q_start[b] + (t - r0);
-  const bool need_prev_row = MORE && shift && !first;
+  const bool need_prev_row = SHIFTED && !first;
   // the row before, or what the state slot holds of it
   const float* bef = need_prev_row ? xp
-                     : (MORE && shift && pos > 0) ? prev + (size_t)sslot[b] * W : nullptr;
+                     : (SHIFTED && pos > 0) ? prev + (size_t)sslot[b] * W : nullptr;
   float ss[2] = {0.f, 0.f};
   auto load_before = [&](int i, Cols& c) {
     c.before[0] = c.before[1] = c.before[2] = c.before[3] = 0.f;
@@ -228,12 +226,12 @@ __global__ void __launch_bounds__(256) dual_norm_shift_kernel(
 #pragma unroll
     for (int j = 0; j < V; ++j) { g1[j] = c.w1[j] + 1.0f; a[j] = c.x[j] * r * g1[j]; }
     stv<S, V>(a_out + (size_t)t * W + i, a);
-    if (MORE && b_out) {
+    if (SECOND) {
 #pragma unroll
       for (int j = 0; j < V; ++j) o[j] = c.x[j] * r * (1.0f + c.w2[j]);
       stv<S, V>(b_out + (size_t)t * W + i, o);
     }
-    if (MORE && shift) {
+    if (SHIFTED) {
       float ap[4];
 #pragma unroll
       for (int j = 0; j < V; ++j)
@@ -1217,21 +1215,23 @@ AF_EXPORT int afm_dual_norm_shift(
   hipStream_t s = (hipStream_t)stream;
   const bool vec = W % 4 == 0 && aligned16(a, s_out, b, last, x, w1) &&
                    aligned16(w2, shift, prev);
-#define DNS(ST, V, R, MORE)                                                   \
-  dual_norm_shift_kernel<ST, V, R, MORE><<<T, 256, 0, s>>>((ST*)a, (ST*)s_out, \
+#define DNS(ST, V, R, ...)                                                    \
+  dual_norm_shift_kernel<ST, V, R, __VA_ARGS__><<<T, 256, 0, s>>>((ST*)a, (ST*)s_out, \
       (ST*)b, (float*)last, (const float*)x, (const ST*)w1, (const ST*)w2,    \
       (const ST*)shift, (float*)prev, (const i32*)row_seq,                    \
       (const i32*)cu, (const i32*)q_start, (const i32*)sslot, eps, W)
-#define DNW(ST, MORE)                                                         \
+#define DNW(ST, ...)                                                          \
   do {                                                                        \
-    if (!vec) DNS(ST, 1, 0, MORE);                                            \
-    else if (W <= 0 || W > 4096) DNS(ST, 4, 0, MORE);                         \
-    else if (W <= 1024) DNS(ST, 4, 1, MORE);                                  \
-    else if (W <= 2048) DNS(ST, 4, 2, MORE);                                  \
-    else DNS(ST, 4, 4, MORE);                                                 \
+    if (!vec) DNS(ST, 1, 0, __VA_ARGS__);                                     \
+    else if (W <= 0 || W > 4096) DNS(ST, 4, 0, __VA_ARGS__);                  \
+    else if (W <= 1024) DNS(ST, 4, 1, __VA_ARGS__);                           \
+    else if (W <= 2048) DNS(ST, 4, 2, __VA_ARGS__);                           \
+    else DNS(ST, 4, 4, __VA_ARGS__);                                          \
   } while (0)
-  if (b || shift) MIX_DISPATCH(dt, DNW(u16, true), DNW(float, true));
-  else MIX_DISPATCH(dt, DNW(u16, false), DNW(float, false));
+  if (b && shift) MIX_DISPATCH(dt, DNW(u16, true, true), DNW(float, true, true));
+  else if (b) MIX_DISPATCH(dt, DNW(u16, true, false), DNW(float, true, false));
+  else if (shift) MIX_DISPATCH(dt, DNW(u16, false, true), DNW(float, false, true));
+  else MIX_DISPATCH(dt, DNW(u16, false, false), DNW(float, false, false));
 #undef DNW
 #undef DNS
   return af_last_err();
