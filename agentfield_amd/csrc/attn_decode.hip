@@ -38,7 +38,7 @@
 // and a line dropped between them is fetched twice (64 ragged sequences of up to
 // 2000 tokens 60 -> 65 us with both, 59 with V only).  Not the loads' latency: eight
 // waves per block (114 -> 125 us) and whole rows through LDS with two tiles per wave in
-// flight (110.5 -> 112) do not help, nor do more splits or pages in order.
+// flight (110.5 -> 112) do not help, nor do pages in order.
 #include "common.h"
 
 #include <type_traits>
@@ -71,41 +71,131 @@ __device__ __forceinline__ void each_head(F f) {
   }
 }
 
+// splits are whole rounds of the block's waves
+constexpr int ROUND = AD_TILE * AD_WAVES;
+
+// Visible tokens of a sequence are [first, L), its rounds begin at a whole tile.
+struct Visible { int first, tile0, rounds; };
+__device__ __forceinline__ Visible visible(int L, int win) {
+  // sliding window (Mistral): only the last `win` tokens
+  const int s0 = (win > 0 && L > win) ? L - win : 0;
+  const int a0 = s0 & ~(AD_TILE - 1);
+  return {s0, a0, (L - a0 + ROUND - 1) / ROUND};
+}
+
+// How the sequences of a step, a lane's each, are cut.  In nsplit parts each, the longest
+// decide: 24 of 1800..8100 tokens in two are blocks of 900 to 4050 tokens, 105 us where as
+// many tokens in sequences of one length take 86.  Where that leaves enough to win, all of
+// them are cut as one row of rounds into `slots` equal shares instead: a block goes on into
+// the next sequence, and its part of each is a piece, number slot + sequence.  Every block
+// and every merge finds the same cut.  In us, nsplit parts / equal shares: the above 105 / 90
+// (a step of 16 layers 3205 / 2907), 9 of 1600..8000 in four 53 / 44, 24 of 800..4000 in two
+// 57 / 48, 5 of 300..3000 with 32 heads 36 / 31, 30 of up to 8000 with G = 8 113 / 86.  Four
+// rounds are what going on takes (3 us: a merge more, loads from the start); looking at the
+// lengths costs those that stay with nsplit parts 0.3 to 0.8 us (17 of 400 13.5 / 14.3).
+// Loads of a part before the cut is known: 0.2 us less there, 4 us more here.
+struct Cut { int mine, share; };   // rounds of the lane's sequence, of a slot (0: nsplit parts)
+__device__ __forceinline__ Cut find_cut(int L, int B, int nsplit, int slots, int win) {
+  const int mine = (int)(threadIdx.x & 63) < B ? visible(L, win).rounds : 0;
+  const float total = wave_sum_f32((float)mine), most = wave_max_f32((float)mine);
+  // the largest part against a share, in products: this is on the way of every call
+  const int even =
+      most * (float)slots <= (float)nsplit * (total + 4.f * (float)slots);
+  if (__builtin_amdgcn_readfirstlane(even)) return {mine, 0};
+  return {mine, (__builtin_amdgcn_readfirstlane((int)total) + slots - 1) / slots};
+}
+
+// Rounds of each of n parts; n is 2, 3 or 4
+__device__ __forceinline__ int split_rounds(int rounds, int n) {
+  if (n == 3) return (int)(((uint64_t)(uint32_t)(rounds + 2) * 0xAAAAAAABull) >> 33);
+  return n == 2 ? (rounds + 1) >> 1 : (rounds + 3) >> 2;
+}
+
+// Sums over the lanes up to a lane's own
+__device__ __forceinline__ int wave_scan(int v) {
+#define AD_ADD(CTRL, ROWS) \
+  v += __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false)
+  AD_ADD(0x111, 0xf);   // a row's lanes 1, 2, 4 and 8 below
+  AD_ADD(0x112, 0xf);
+  AD_ADD(0x114, 0xf);
+  AD_ADD(0x118, 0xf);
+  AD_ADD(0x142, 0xa);   // the last lane of rows 0 and 2, then of the lower half
+  AD_ADD(0x143, 0xc);
+#undef AD_ADD
+  return v;
+}
+
 // Partial layout: po [B, Hk, NSPLIT, G, D] f32; pml [B, Hk, NSPLIT, G, 2] f32
-// (maximum in units of log2, sum; a split without tokens leaves po unwritten).
+// (maximum in units of log2, sum; a split without tokens leaves po unwritten);
+// CUT: [Hk, cap, G, ..], cap pieces, split s of sequence b at b * nsplit + s.
 //
 // TILED: page_size is a multiple of AD_TILE, so a tile lies in one page and its
 // index is a scalar load; otherwise every lane looks its tokens' pages up.
-template <int G, bool TILED>
-__global__ void __launch_bounds__(64 * AD_WAVES, G == 8 ? 3 : 4) attn_decode_kernel(
+// CUT: with find_cut, where the launcher says so.
+template <int G, bool TILED, bool CUT>
+__global__ void __launch_bounds__(64 * AD_WAVES, (G == 8 ? 3 : 4) - CUT) attn_decode_kernel(
     u16* __restrict__ out, float* __restrict__ po, float* __restrict__ pml,
     const u16* __restrict__ q, const u16* __restrict__ kc, const u16* __restrict__ vc,
     const i32* __restrict__ bt, const i32* __restrict__ len,
-    float scale, int Hk, int page_size, int page_shift, int max_pages,
-    int nsplit, i64 qs, int win, int faster) {
+    float scale, int B, int Hk, int page_size, int page_shift, int max_pages,
+    int nsplit, int slots, int cap, i64 qs, int win, int faster) {
   // `faster`, the number of heads or of sequences, runs within x
   const int hi = blockIdx.x / faster, lo = blockIdx.x - hi * faster, split = blockIdx.y;
-  const int kvh = faster == Hk ? lo : hi, b = faster == Hk ? hi : lo;
+  const int kvh = faster == Hk ? lo : hi;
+  int b = faster == Hk ? hi : lo;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int tg = lane >> 4, dl = lane & 15;
   const int Hq = Hk * G;
 
-  const int L = len[b];
-  // sliding window (Mistral): only the last `win` tokens are visible
-  const int s0 = (win > 0 && L > win) ? L - win : 0;
-  const int a0 = s0 & ~(AD_TILE - 1);
-  // splits are whole rounds of the block's waves
-  constexpr int ROUND = AD_TILE * AD_WAVES;
-  const int chunk = ((L - a0 + nsplit - 1) / nsplit + ROUND - 1) & ~(ROUND - 1);
-  const int c0 = a0 + split * chunk;       // tile grid of this split
-  const int t1 = min(L, c0 + chunk);
-  const int t0 = max(s0, c0);              // visible tokens are [t0, t1)
+  // (constant memory: the compiler looks nothing up by scalar loads behind a store, and a
+  // vector load of a page waits for the tile that was asked for before it)
+  typedef const __attribute__((address_space(4))) i32* pages;
+  const pages tables = (pages)bt, lengths = (pages)len;
+  pages btrow = tables + (size_t)b * max_pages;
+  auto page_of = [&](int t) {
+    return btrow[page_shift >= 0 ? t >> page_shift : t / page_size];
+  };
+  // a part: its visible tokens [t0, t1), tile grid, place; this wave's tile and its page
+  int c0, t0, t1, t, pg_next = 0;
+  size_t piece = CUT ? (size_t)kvh * cap + b * nsplit + split
+                     : ((size_t)b * Hk + kvh) * nsplit + split;
+  auto take = [&](int L, int skip, int rounds) {
+    const Visible v = visible(L, win);
+    c0 = v.tile0 + skip * ROUND;
+    t1 = min(L, c0 + rounds * ROUND);
+    t0 = max(v.first, c0);
+    t = c0 + wid * AD_TILE;
+    if (CUT && TILED) pg_next = page_of(min(t, max(t1 - 1, 0)));
+  };
+  int left = 0;                            // rounds of this slot behind the part
+  {
+    const int lens = CUT ? len[min(lane, B - 1)] : 0;
+    const int L = len[b], rounds = visible(L, win).rounds;
+    const int part = CUT ? split_rounds(rounds, nsplit) : (rounds + nsplit - 1) / nsplit;
+    take(L, split * part, part);
+    if (CUT) {
+      __builtin_amdgcn_sched_barrier(0);   // the page is looked up meanwhile
+      const Cut c = find_cut(lens, B, nsplit, slots, win);
+      if (c.share > 0) {
+        const int slot = split * B + b, at = slot * c.share;
+        const int sum = wave_scan(c.mine);
+        const unsigned long long behind = __ballot(sum > at);
+        if (slot >= slots || behind == 0) return;
+        b = (int)__ffsll(behind) - 1;
+        piece = (size_t)kvh * cap + slot + b;
+        btrow = tables + (size_t)b * max_pages;
+        const int skip = at - __builtin_amdgcn_readlane(sum - c.mine, b);
+        const int now = min(c.share, __builtin_amdgcn_readlane(c.mine, b) - skip);
+        left = c.share - now;
+        take(__builtin_amdgcn_readlane(lens, b), skip, now);
+      }
+    }
+  }
   if (c0 >= t1) {                          // no tokens (uniform in the block)
     if (nsplit > 1) {
       if (threadIdx.x < G) {
-        const size_t at =
-            (((size_t)b * Hk + kvh) * nsplit + split) * G + threadIdx.x;
+        const size_t at = piece * G + threadIdx.x;
         pml[at * 2] = AF_NEG_INF;
         pml[at * 2 + 1] = 0.f;
       }
@@ -119,23 +209,13 @@ __global__ void __launch_bounds__(64 * AD_WAVES, G == 8 ? 3 : 4) attn_decode_ker
   // query heads as B operand: lane holds head (lane & 15) % G, dims
   // 32 c + tg*8 .. +8
   s16x8 qf[4];
-  {
+  auto load_q = [&]() {
     const u16* qp = q + (size_t)b * qs + (kvh * G + (dl & (G - 1))) * AD_D + tg * 8;
 #pragma unroll
     for (int c = 0; c < 4; ++c) qf[c] = *reinterpret_cast<const s16x8*>(qp + c * 32);
-  }
+  };
   const float sc = scale * 1.44269504088896f;  // softmax in powers of two
 
-  float m = AF_NEG_INF, l = 0.f, acc[G][8];
-#pragma unroll
-  for (int g = 0; g < G; ++g)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
-
-  const i32* btrow = bt + (size_t)b * max_pages;
-  auto page_of = [&](int t) {
-    return btrow[page_shift >= 0 ? t >> page_shift : t / page_size];
-  };
   auto page_off = [&](int t) {
     return page_shift >= 0 ? t & (page_size - 1) : t % page_size;
   };
@@ -172,114 +252,144 @@ __global__ void __launch_bounds__(64 * AD_WAVES, G == 8 ? 3 : 4) attn_decode_ker
   };
 
   s16x8 kf[4], vf[4], kn[4], vn[4];
-  int t = c0 + wid * AD_TILE;
-  int pg_next = 0;
-  if (t < t1) {
-    load_tile(t, TILED ? page_of(t) : 0, kf, vf);
+  auto begin = [&]() {                     // the wave's first tile
+    load_q();
+    if (t >= t1) return;
+    load_tile(t, CUT ? pg_next : TILED ? page_of(t) : 0, kf, vf);
     if (TILED) pg_next = page_of(min(t + ROUND, t1 - 1));
-  }
-  for (; t < t1; t += ROUND) {
-    if (t + ROUND < t1) {
-      load_tile(t + ROUND, pg_next, kn, vn);
-      if (TILED) pg_next = page_of(min(t + 2 * ROUND, t1 - 1));
-    }
-    f32x4 s = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8d(kf[c]),
-                                                  as_bf16x8d(qf[c]), s, 0, 0, 0);
-    float mn = m;
-    bool ok[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int tok = t + tg * 4 + r;
-      ok[r] = tok >= t0 && tok < t1;
-      s[r] = ok[r] ? s[r] * sc : AF_NEG_INF;
-      mn = fmaxf(mn, s[r]);
-    }
-    float p[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      p[r] = ok[r] ? __builtin_amdgcn_exp2f(s[r] - mn) : 0.f;
-    if (__any(mn > m)) {  // rare once the first tiles have been seen
-      const float corr = __builtin_amdgcn_exp2f(m - mn);
-      l *= corr;
-      each_head<0, G>([&](auto g) {
-        const float cg = row_bcast<g.value>(corr);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[g.value][j] *= cg;
-      });
-      m = mn;
-    }
-    l += (p[0] + p[1]) + (p[2] + p[3]);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float v[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = bf2f((u16)vf[r][j]);
-      each_head<0, G>([&](auto g) {
-        const float pg = row_bcast<g.value>(p[r]);
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          acc[g.value][j] = fmaf(pg, v[j], acc[g.value][j]);
-      });
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) { kf[c] = kn[c]; vf[c] = vn[c]; }
-  }
-
-  // fold the four rows (same dims, other tokens)
-  float M = fmaxf(m, __shfl_xor(m, 16, 64));
-  M = fmaxf(M, __shfl_xor(M, 32, 64));
-  const float f = (m <= AF_NEG_INF) ? 0.f : __builtin_amdgcn_exp2f(m - M);
-  l *= f;
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  };
   __shared__ float s_ml[AD_WAVES][G][2];
   __shared__ float s_o[AD_WAVES][G][AD_D];
-  each_head<0, G>([&](auto g) {
-    const float fg = row_bcast<g.value>(f);
-    float o[8];
+  begin();
+  for (;;) {
+    float m = AF_NEG_INF, l = 0.f, acc[G][8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      o[j] = acc[g.value][j] * fg;
-      o[j] += __shfl_xor(o[j], 16, 64);
-      o[j] += __shfl_xor(o[j], 32, 64);
-    }
-    if (tg == 0) {
+    for (int g = 0; g < G; ++g)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) s_o[wid][g.value][dl * 8 + j] = o[j];
+      for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
+    for (; t < t1; t += ROUND) {
+      if (t + ROUND < t1) {
+        load_tile(t + ROUND, pg_next, kn, vn);
+        if (TILED) pg_next = page_of(min(t + 2 * ROUND, t1 - 1));
+      }
+      f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8d(kf[c]),
+                                                    as_bf16x8d(qf[c]), s, 0, 0, 0);
+      float mn = m;
+      bool ok[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int tok = t + tg * 4 + r;
+        ok[r] = tok >= t0 && tok < t1;
+        s[r] = ok[r] ? s[r] * sc : AF_NEG_INF;
+        mn = fmaxf(mn, s[r]);
+      }
+      float p[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        p[r] = ok[r] ? __builtin_amdgcn_exp2f(s[r] - mn) : 0.f;
+      if (__any(mn > m)) {  // rare once the first tiles have been seen
+        const float corr = __builtin_amdgcn_exp2f(m - mn);
+        l *= corr;
+        each_head<0, G>([&](auto g) {
+          const float cg = row_bcast<g.value>(corr);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) acc[g.value][j] *= cg;
+        });
+        m = mn;
+      }
+      l += (p[0] + p[1]) + (p[2] + p[3]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = bf2f((u16)vf[r][j]);
+        each_head<0, G>([&](auto g) {
+          const float pg = row_bcast<g.value>(p[r]);
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            acc[g.value][j] = fmaf(pg, v[j], acc[g.value][j]);
+        });
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) { kf[c] = kn[c]; vf[c] = vn[c]; }
     }
-  });
-  if (lane < G) { s_ml[wid][lane][0] = M; s_ml[wid][lane][1] = l; }
-  __syncthreads();
 
-  // merge the waves: two elements per thread
-  for (int i = threadIdx.x; i < G * AD_D / 2; i += 64 * AD_WAVES) {
-    const int g = i / (AD_D / 2), d = (i % (AD_D / 2)) * 2;
-    float Mx = s_ml[0][g][0];
-#pragma unroll
-    for (int w = 1; w < AD_WAVES; ++w) Mx = fmaxf(Mx, s_ml[w][g][0]);
-    float L2 = 0.f, o0 = 0.f, o1 = 0.f;
-#pragma unroll
-    for (int w = 0; w < AD_WAVES; ++w) {
-      const float c = (s_ml[w][g][0] <= AF_NEG_INF)
-                          ? 0.f
-                          : __builtin_amdgcn_exp2f(s_ml[w][g][0] - Mx);
-      L2 += s_ml[w][g][1] * c;
-      o0 += s_o[w][g][d] * c;
-      o1 += s_o[w][g][d + 1] * c;
+    // the slot's next sequence that has tokens: its loads travel while this part is merged
+    const int of = b;
+    const size_t to = piece;
+    bool on = false;
+    if (CUT && left > 0) {
+      int L = 0;
+      while (L <= 0 && b + 1 < B) {
+        L = lengths[++b];
+        ++piece;
+      }
+      on = L > 0;
+      if (on) {
+        const int rounds = min(left, visible(L, win).rounds);
+        left -= rounds;
+        btrow = tables + (size_t)b * max_pages;
+        take(L, 0, rounds);
+        begin();
+      }
     }
-    if (nsplit == 1) {
-      const float inv = (L2 > 0.f) ? 1.f / L2 : 0.f;
-      u16x2 ov = {f2bf(o0 * inv), f2bf(o1 * inv)};
-      *reinterpret_cast<u16x2*>(out + (size_t)b * (Hq * AD_D) +
-                                (kvh * G + g) * AD_D + d) = ov;
-    } else {
-      const size_t at = (((size_t)b * Hk + kvh) * nsplit + split) * G + g;
-      *reinterpret_cast<f32x2*>(po + at * AD_D + d) = f32x2{o0, o1};
-      if (d == 0) { pml[at * 2] = Mx; pml[at * 2 + 1] = L2; }
+
+    // fold the four rows (same dims, other tokens)
+    float M = fmaxf(m, __shfl_xor(m, 16, 64));
+    M = fmaxf(M, __shfl_xor(M, 32, 64));
+    const float f = (m <= AF_NEG_INF) ? 0.f : __builtin_amdgcn_exp2f(m - M);
+    l *= f;
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    each_head<0, G>([&](auto g) {
+      const float fg = row_bcast<g.value>(f);
+      float o[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        o[j] = acc[g.value][j] * fg;
+        o[j] += __shfl_xor(o[j], 16, 64);
+        o[j] += __shfl_xor(o[j], 32, 64);
+      }
+      if (tg == 0) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s_o[wid][g.value][dl * 8 + j] = o[j];
+      }
+    });
+    if (lane < G) { s_ml[wid][lane][0] = M; s_ml[wid][lane][1] = l; }
+    __syncthreads();
+
+    // merge the waves: two elements per thread
+    for (int i = threadIdx.x; i < G * AD_D / 2; i += 64 * AD_WAVES) {
+      const int g = i / (AD_D / 2), d = (i % (AD_D / 2)) * 2;
+      float Mx = s_ml[0][g][0];
+#pragma unroll
+      for (int w = 1; w < AD_WAVES; ++w) Mx = fmaxf(Mx, s_ml[w][g][0]);
+      float L2 = 0.f, o0 = 0.f, o1 = 0.f;
+#pragma unroll
+      for (int w = 0; w < AD_WAVES; ++w) {
+        const float c = (s_ml[w][g][0] <= AF_NEG_INF)
+                            ? 0.f
+                            : __builtin_amdgcn_exp2f(s_ml[w][g][0] - Mx);
+        L2 += s_ml[w][g][1] * c;
+        o0 += s_o[w][g][d] * c;
+        o1 += s_o[w][g][d + 1] * c;
+      }
+      if (nsplit == 1) {
+        const float inv = (L2 > 0.f) ? 1.f / L2 : 0.f;
+        u16x2 ov = {f2bf(o0 * inv), f2bf(o1 * inv)};
+        *reinterpret_cast<u16x2*>(out + (size_t)of * (Hq * AD_D) +
+                                  (kvh * G + g) * AD_D + d) = ov;
+      } else {
+        const size_t at = to * G + g;
+        *reinterpret_cast<f32x2*>(po + at * AD_D + d) = f32x2{o0, o1};
+        if (d == 0) { pml[at * 2] = Mx; pml[at * 2 + 1] = L2; }
+      }
     }
+    if (!on) return;
+    __syncthreads();                         // the sums are read
   }
 }
 
@@ -289,26 +399,48 @@ __global__ void __launch_bounds__(64 * AD_WAVES, G == 8 ? 3 : 4) attn_decode_ker
 // sequence of 387 tokens in 16 splits 1473 -> 1425 us, 12 of 4500..8000 in four 2074 ->
 // 2050).  Splits behind the last repeat it; those without tokens, whose po was not
 // written, are left out of the sum.
-template <int NS>
+// CUT: the parts are asked for as if there were nsplit each, and again where there are
+// shares (find_cut), so that the lengths are not waited for first.
+template <int NS, bool CUT>
 __global__ void __launch_bounds__(64) attn_decode_combine_kernel(
     u16* __restrict__ out, const float* __restrict__ po, const float* __restrict__ pml,
-    int Hq, int G, int nsplit) {
+    const i32* __restrict__ len, int B, int Hq, int G, int nsplit, int slots, int cap,
+    int win) {
   const int b = blockIdx.x, h = blockIdx.y;
   const int kvh = h / G, g = h % G;
   const int Hk = Hq / G;
   const int lane = threadIdx.x;
-  const size_t first = (((size_t)b * Hk + kvh) * nsplit) * G + g;
+  const int lens = CUT ? len[min(lane, B - 1)] : 0;
+  size_t first = CUT ? ((size_t)kvh * cap + b * nsplit) * G + g
+                     : (((size_t)b * Hk + kvh) * nsplit) * G + g;
+  int n = nsplit;
 
-  float L2 = 0.f, o0 = 0.f, o1 = 0.f, M = AF_NEG_INF;
-  for (int s0 = 0; s0 < nsplit; s0 += NS) {
-    const f32x2 ml = *reinterpret_cast<const f32x2*>(
-        pml + (first + (size_t)min(s0 + lane, nsplit - 1) * G) * 2);
-    f32x2 v[NS];
+  f32x2 ml, v[NS];
+  auto ask = [&](int s0) {
+    ml = *reinterpret_cast<const f32x2*>(
+        pml + (first + (size_t)min(s0 + lane, n - 1) * G) * 2);
 #pragma unroll
     for (int i = 0; i < NS; ++i)
       v[i] = *reinterpret_cast<const f32x2*>(
-          po + (first + (size_t)min(s0 + i, nsplit - 1) * G) * AD_D + lane * 2);
-    const bool mine = lane < NS && s0 + lane < nsplit;
+          po + (first + (size_t)min(s0 + i, n - 1) * G) * AD_D + lane * 2);
+  };
+  if (CUT) {
+    ask(0);
+    __builtin_amdgcn_sched_barrier(0);
+    const Cut c = find_cut(lens, B, nsplit, slots, win);
+    if (c.share > 0) {
+      const int sum = wave_scan(c.mine);
+      const int rounds = __builtin_amdgcn_readlane(c.mine, b);
+      const int end = __builtin_amdgcn_readlane(sum, b), slot = (end - rounds) / c.share;
+      n = rounds > 0 ? (end - 1) / c.share - slot + 1 : 0;
+      first = ((size_t)kvh * cap + slot + b) * G + g;
+      if (n > 0) ask(0);
+    }
+  }
+  float L2 = 0.f, o0 = 0.f, o1 = 0.f, M = AF_NEG_INF;
+  for (int s0 = 0; s0 < n; s0 += NS) {
+    if (!CUT || s0 > 0) ask(s0);
+    const bool mine = lane < NS && s0 + lane < n;
     const float pm = mine ? ml[0] : AF_NEG_INF, pl = mine ? ml[1] : 0.f;
     const float Mn = fmaxf(M, wave_max_f32(pm));
     const float back = (M <= AF_NEG_INF) ? 0.f : __builtin_amdgcn_exp2f(M - Mn);
@@ -344,21 +476,34 @@ AF_EXPORT int af_attn_decode(void* out, void* po, void* pml, const void* q,
                              const void* kc, const void* vc, const void* bt,
                              const void* len, float scale, int B, int Hq, int Hk,
                              int D, int page_size, int max_pages, int nsplit,
-                             i64 qs, int win, void* stream) {
+                             int cap, i64 qs, int win, void* stream) {
   if (D != AD_D) return 9002;
   const int G = Hq / Hk;
   if (G < 1 || G > AD_MAXG || G * Hk != Hq) return 9003;
   if (B == 0) return 0;
+  if (nsplit > 1 && cap < B * nsplit) return 9004;
+  // Equal shares: slots + B - 1 pieces at most.  A lane per sequence; all blocks have room
+  // at once, or the dispatch evens them out.  Beyond four parts a sequence is short, or the
+  // step is small (seven of 200..2000 in eight 14.7 us, 16 with a look at the lengths).  Long
+  // sequences behind a window are of one length.
+  const bool cut = nsplit > 1 && nsplit <= 4 && B > 1 && B <= 64 && win <= 0 &&
+                   B * Hk * nsplit <= 256 * (G == 8 ? 2 : 3);
+  const int slots = cut ? max(0, min(B * nsplit, cap - (B - 1))) : 0;
   const int faster = heads_first(Hk, nsplit) ? Hk : B;
   const dim3 grid(B * Hk, nsplit), blk(64 * AD_WAVES);
   hipStream_t st = (hipStream_t)stream;
   const bool pow2 = (page_size & (page_size - 1)) == 0;
   const int shift = pow2 ? __builtin_ctz(page_size) : -1;
-#define AF_LAUNCH1(GG, TT)                                                       \
-  attn_decode_kernel<GG, TT><<<grid, blk, 0, st>>>(                              \
+#define AF_LAUNCH2(GG, TT, CUT)                                                  \
+  attn_decode_kernel<GG, TT, CUT><<<grid, blk, 0, st>>>(                         \
       (u16*)out, (float*)po, (float*)pml, (const u16*)q, (const u16*)kc,         \
-      (const u16*)vc, (const i32*)bt, (const i32*)len, scale, Hk, page_size,     \
-      shift, max_pages, nsplit, qs, win, faster)
+      (const u16*)vc, (const i32*)bt, (const i32*)len, scale, B, Hk, page_size,  \
+      shift, max_pages, nsplit, slots, cap, qs, win, faster)
+#define AF_LAUNCH1(GG, TT)                                                       \
+  do {                                                                           \
+    if (slots > 0) AF_LAUNCH2(GG, TT, true);                                     \
+    else AF_LAUNCH2(GG, TT, false);                                              \
+  } while (0)
 #define AF_LAUNCH(GG)                                                            \
   do {                                                                           \
     if (page_size % AD_TILE == 0) AF_LAUNCH1(GG, true);                          \
@@ -373,11 +518,16 @@ AF_EXPORT int af_attn_decode(void* out, void* po, void* pml, const void* q,
   }
 #undef AF_LAUNCH
 #undef AF_LAUNCH1
+#undef AF_LAUNCH2
   if (nsplit > 1) {
     const dim3 g2(B, Hq);
 #define AF_COMBINE(NS)                                                           \
-  attn_decode_combine_kernel<NS><<<g2, 64, 0, st>>>((u16*)out, (const float*)po, \
-                                                    (const float*)pml, Hq, G, nsplit)
+  do {                                                                           \
+    const auto merge = slots > 0 ? attn_decode_combine_kernel<NS, true>          \
+                                 : attn_decode_combine_kernel<NS, false>;        \
+    merge<<<g2, 64, 0, st>>>((u16*)out, (const float*)po, (const float*)pml,     \
+                             (const i32*)len, B, Hq, G, nsplit, slots, cap, win); \
+  } while (0)
     if (nsplit <= 4) AF_COMBINE(4);
     else if (nsplit <= 8) AF_COMBINE(8);
     else AF_COMBINE(16);

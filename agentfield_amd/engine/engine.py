@@ -971,11 +971,8 @@ class LLMEngine:
             return None
         cfg = self.cfg
         G = cfg.num_heads // cfg.num_kv_heads
-        po = torch.empty(bs, cfg.num_kv_heads, nsplit, G, cfg.head_dim,
-                         dtype=torch.float32, device=self.device)
-        pml = torch.empty(bs, cfg.num_kv_heads, nsplit, G, 2,
-                          dtype=torch.float32, device=self.device)
-        return po, pml
+        return ops.decode_scratch(bs, cfg.num_kv_heads, nsplit, G, self.device,
+                                  cfg.head_dim)
 
     def _get_graph(self, bs: int, tkp: bool, lp: bool = False):
         key = (bs, tkp, lp)

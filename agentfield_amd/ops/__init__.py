@@ -175,21 +175,25 @@ def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
     if out is None:
         out = torch.empty(B, Hq * D, dtype=q.dtype, device=q.device)
     G = Hq // Hk
+    po = pml = None
+    cap = 0
     if nsplit > 1:
-        if scratch is None:
-            po = torch.empty(B, Hk, nsplit, G, D, dtype=torch.float32, device=q.device)
-            pml = torch.empty(B, Hk, nsplit, G, 2, dtype=torch.float32, device=q.device)
-        else:
-            po, pml = scratch
-    else:
-        po = pml = None
+        po, pml = decode_scratch(B, Hk, nsplit, G, q.device) if scratch is None else scratch
+        cap = min(po.numel() // (Hk * G * D), pml.numel() // (Hk * G * 2))
     rc = _lib.lib().af_attn_decode(
         _lib.ptr(out), _lib.ptr(po), _lib.ptr(pml), _lib.ptr(q),
         _lib.ptr(kcache), _lib.ptr(vcache), _lib.ptr(block_table),
         _lib.ptr(seq_lens), scale, B, Hq, Hk, D, page, block_table.shape[1],
-        nsplit, q.stride(0), window, _lib.cur_stream())
+        nsplit, cap, q.stride(0), window, _lib.cur_stream())
     _lib.check(rc, "af_attn_decode")
     return out
+
+
+def decode_scratch(B: int, Hk: int, nsplit: int, G: int, device, D: int = 128):
+    """Scratch of attn_decode: room for nsplit parts of every sequence, and for one more
+    each, with which unlike lengths can be cut evenly."""
+    return tuple(torch.empty(B, Hk, nsplit + 1, G, n, dtype=torch.float32, device=device)
+                 for n in (D, 2))
 
 
 def prefill_split(seq_lens: list[int], G: int, Hk: int, max_keys: int):

@@ -48,7 +48,7 @@ def _declare(l: ctypes.CDLL) -> None:
     l.af_add.argtypes = [p, p, p, i64, p]
     l.af_reshape_and_cache.argtypes = [p, p, p, p, p, i, i, i, i, p]
     l.af_embedding.argtypes = [p, p, p, p, i, i, p]
-    l.af_attn_decode.argtypes = [p, p, p, p, p, p, p, p, f, i, i, i, i, i, i, i,
+    l.af_attn_decode.argtypes = [p, p, p, p, p, p, p, p, f, i, i, i, i, i, i, i, i,
                                  i64, i, p]
     l.af_attn_prefill.argtypes = [p, p, p, p, p, p, p, p, p, f, i, i, i, i, i,
                                   i, i, i, i64, i, i, i, p]

@@ -726,6 +726,60 @@ def test_attn_decode_merges_splits(nsplit):
     assert close(got, want, atol=2 ** -7, rtol=2 ** -8)
 
 
+@pytest.mark.parametrize("G,page,nsplit,lens", [
+    (4, 64, 2, [6000, 1, 700, 64, 65]),            # through three sequences and more
+    (4, 64, 2, [0, 3000, 0, 0, 2, 1100, 0]),       # empty ones first, between and last
+    (1, 16, 3, [5, 4096, 17, 2048]),               # shares that end with a sequence
+    (2, 64, 4, [9000, 300, 300]),
+    (8, 24, 2, [2500, 100, 33]),                   # tiles over two pages
+    (8, 64, 4, [64 * 150, 1, 1, 1, 1, 1]),
+    (4, 32, 2, [2900 if i == 40 else 7 * i for i in range(64)]),   # a lane each
+    (4, 32, 2, [2900 if i == 40 else 7 * i for i in range(65)]),   # one too many
+    (4, 64, 2, [1600, 1500, 1400])])               # alike: nsplit parts each
+def test_attn_decode_shares(G, page, nsplit, lens):
+    """Sequences of unlike lengths, cut in equal shares of all their tokens; replayed with
+    other lengths, and with scratch for nsplit parts of each only.  What is not visible is
+    NaN in the values.  Tolerance: bf16 rounding of outputs below 4 (2^-9 * 4)."""
+    D, Hk, B = 128, 2, len(lens)
+    torch.manual_seed(len(lens) + G)
+    maxp = -(-max(lens) // page)
+    bt = (torch.randperm(B * maxp) + 1).view(B, maxp).to(torch.int32)
+    kc = torch.randn(B * maxp + 1, Hk, page, D).bfloat16()
+    clean = torch.randn(B * maxp + 1, Hk, page, D).bfloat16()
+    q = torch.randn(B, Hk * G * D).bfloat16()
+    btd, kd, qd = bt.to(DEV), kc.to(DEV), q.to(DEV)
+
+    def values(lens):
+        seen = torch.zeros(B * maxp + 1, page, dtype=torch.bool)
+        for b, n in enumerate(lens):
+            t = torch.arange(n)
+            seen[bt[b, t // page].long(), t % page] = True
+        return torch.where(seen[:, None, :, None], clean, torch.nan)
+
+    def check(got, lens):
+        some = [b for b in range(B) if lens[b]]
+        L = torch.tensor(lens, dtype=torch.int32)
+        want = ref.attn_decode(q.unflatten(-1, (Hk * G, D))[some], kc, clean, bt[some],
+                               L[some], 1.0 / math.sqrt(D)).flatten(1)
+        got = got.cpu()
+        assert torch.isfinite(got.float()).all()
+        assert close(got[some], want, atol=2 ** -7, rtol=2 ** -8)
+        assert all((got[b] == 0).all() for b in range(B) if not lens[b])
+
+    vd, L = values(lens).to(DEV), torch.tensor(lens, dtype=torch.int32, device=DEV)
+    check(ops.attn_decode(qd, kd, vd, btd, L, nsplit=nsplit), lens)
+    scratch = tuple(torch.full((B, Hk, nsplit, G, n), torch.nan, device=DEV) for n in (D, 2))
+    check(ops.attn_decode(qd, kd, vd, btd, L, nsplit=nsplit, scratch=scratch), lens)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ops.attn_decode(qd, kd, vd, btd, L, nsplit=nsplit)
+    for turned in (lens[::-1], [min(n, 90) for n in lens], lens):
+        vd.copy_(values(turned))
+        L.copy_(torch.tensor(turned, dtype=torch.int32))
+        graph.replay()
+        check(out, turned)
+
+
 @pytest.mark.parametrize("Hk,nsplit", [(3, 1), (4, 1), (4, 2), (8, 1), (8, 3), (11, 2)])
 def test_attn_decode_orders_of_the_grid(Hk, nsplit):
     """Heads first and sequences first: every head of every sequence is its own, by
