@@ -1056,7 +1056,8 @@ constexpr int scan_rows(int rp, int threads) {
 // calls of 3..128 sequences against a head of each in turn everywhere: 0.80 of it in the mean
 // (16 of 10..76, 16 heads of 256 x 256 165 -> 119 us, 64 of 25..75, 16 of 128 x 128 in fp32
 // 257 -> 203), lengths alike 1.00, at most 1.04.
-enum ScanLengths { LENS_UNKNOWN, LENS_ONE, LENS_DIFFER };   // at most a token each, unlike
+// at most a token each, unlike, the longest 1.25 of the mean (and 256 tokens in the mean)
+enum ScanLengths { LENS_UNKNOWN, LENS_ONE, LENS_DIFFER, LENS_UNEVEN };
 enum ScanWalk { HEADS_IN_TURN, IN_ORDER, LONGEST_FIRST, LONGEST_FIRST_SHORT };
 struct ScanRows { int b, t0, t1; };
 __device__ __forceinline__ ScanRows scan_sequence(const i32* __restrict__ cu, int walk) {
@@ -1086,7 +1087,13 @@ __device__ __forceinline__ ScanRows scan_sequence(const i32* __restrict__ cu, in
 // until the block before has been worked through) and computes RP rows of one column
 // (NT = 512) or two (256); each lane of a 16-lane row keeps one token's sum.  Two LDS
 // buffers, one barrier per block of tokens.
-template <typename S, int RP, bool ZL, int NT>
+// APART (NT = 512, 16 columns): four waves stage and four compute, one of each per SIMD.
+// With few workgroups the longest sequence's tokens follow one another, each the arithmetic
+// of two waves and then their staging (28 vector instructions each and a quarter); so it is
+// the arithmetic of one, beside the staging: 140 -> 100 ns a token with decays per channel,
+// 124 -> 87 with one per head.  Every column is staged for twice as often, which costs where
+// the chip is full.  (All four waves of 16 columns staging 267 -> 226 us.)
+template <typename S, int RP, bool ZL, int NT, int COLS>
 __global__ void __launch_bounds__(NT, RP == 8 && sizeof(S) == 2 ? (NT == 512 ? 4 : 3) : 2)
 linear_scan_prompt_kernel(
     float* __restrict__ out, float* __restrict__ state,
@@ -1100,9 +1107,13 @@ linear_scan_prompt_kernel(
   constexpr int DKP = 16 * RP;
   constexpr bool FAST = sizeof(S) == 2;
   constexpr int TB = RP >= 16 ? 8 : 16;
-  constexpr int CPT = 512 / NT;                // columns per thread
-  constexpr int E = scan_rows(RP, NT);
-  constexpr int BUF = TB * (3 * DKP + 32);     // [TB][3][DKP], [TB][32]
+  constexpr bool APART = COLS == 16 && NT == 512;   // half of the waves stage
+  constexpr int WORK = APART ? NT / 2 : NT;
+  constexpr int CPT = 16 * COLS / WORK;        // columns per thread
+  constexpr int E = scan_rows(RP, WORK);
+  const bool stages = !APART || threadIdx.x >= WORK, walks = !APART || threadIdx.x < WORK;
+  const int tid = APART ? threadIdx.x % WORK : threadIdx.x;
+  constexpr int BUF = TB * (3 * DKP + COLS);   // [TB][3][DKP], [TB][COLS]
   extern __shared__ float smem[];
   const bool by_sequence = walk != HEADS_IN_TURN;
   const ScanRows rows = by_sequence ? scan_sequence(cu, walk)
@@ -1111,9 +1122,9 @@ linear_scan_prompt_kernel(
   const int t0 = __builtin_amdgcn_readfirstlane(rows.t0);
   const int t1 = __builtin_amdgcn_readfirstlane(rows.t1);
   const int h = by_sequence ? blockIdx.x : blockIdx.y;
-  const int c0 = (by_sequence ? blockIdx.y : blockIdx.z) * 32;
+  const int c0 = (by_sequence ? blockIdx.y : blockIdx.z) * COLS;
   if (t1 <= t0) return;
-  const int r = threadIdx.x & 15, cc = threadIdx.x >> 4;
+  const int r = tid & 15, cc = tid >> 4;
   const int ca = c0 + CPT * cc;
   float* sbase = state + (((size_t)sslot[b] * H + h) * dk) * dv;
   float state_of[CPT][RP];
@@ -1130,8 +1141,8 @@ linear_scan_prompt_kernel(
   // what this thread stages: rows i0 .. i0+E-1 of token st of a block, and two
   // columns of v of token vt
   struct Raw { S x[E]; };
-  const int st = threadIdx.x * E / DKP, i0 = threadIdx.x * E % DKP;
-  const int vt = threadIdx.x >> 4, vc = c0 + 2 * (threadIdx.x & 15);
+  const int st = tid * E / DKP, i0 = tid * E % DKP;
+  const int vt = tid / (COLS / 2), vc = c0 + 2 * (tid % (COLS / 2));
   const bool have = i0 < dk, turn = i0 < rot;
   const int half = rot >> 1, ic = have ? i0 : 0;
   const bool lowh = i0 < half;
@@ -1224,22 +1235,25 @@ linear_scan_prompt_kernel(
       }
     }
     if (vt < TB) {
-      float* vr = stage + TB * 3 * DKP + vt * 32 + (vc - c0);
+      float* vr = stage + TB * 3 * DKP + vt * COLS + (vc - c0);
       vr[0] = vt < nt && vc < dv ? ldf<S>(&rv[0]) : 0.f;
       vr[1] = vt < nt && vc + 1 < dv ? ldf<S>(&rv[1]) : 0.f;
     }
   };
-  fetch(t0);
-  fill(min(TB, t1 - t0), smem);
-  fetch(min(t0 + TB, t1 - 1));
+  if (stages) {
+    fetch(t0);
+    fill(min(TB, t1 - t0), smem);
+    fetch(min(t0 + TB, t1 - 1));
+  }
   __syncthreads();
   int cur = 0;
   for (int tb = t0; tb < t1; tb += TB) {
     const int nt = min(TB, t1 - tb);
-    if (tb + TB < t1) {
+    if (stages && tb + TB < t1) {
       fill(min(TB, t1 - tb - TB), smem + (cur ^ BUF));
       fetch(min(tb + 2 * TB, t1 - 1));         // in flight during the arithmetic
     }
+    if (walks) {
     const float* sb = smem + cur;
     const float* vb = sb + TB * 3 * DKP;
     float o[CPT];
@@ -1273,11 +1287,11 @@ linear_scan_prompt_kernel(
         }
       }
       if constexpr (CPT == 2) {
-        const f32x2 v = *reinterpret_cast<const f32x2*>(vb + tt * 32 + 2 * cc);
+        const f32x2 v = *reinterpret_cast<const f32x2*>(vb + tt * COLS + 2 * cc);
         t.v[0] = v[0];
         t.v[1] = v[1];
       } else {
-        t.v[0] = vb[tt * 32 + cc];
+        t.v[0] = vb[tt * COLS + cc];
       }
       return t;
     };
@@ -1326,9 +1340,11 @@ linear_scan_prompt_kernel(
       for (int c = 0; c < CPT; ++c)
         if (ca + c < dv) op[ca + c] = o[c];
     }
+    }
     __syncthreads();  // the next buffer is filled, this one read
     cur ^= BUF;
   }
+  if (!walks) return;
 #pragma unroll
   for (int ii = 0; ii < RP; ++ii) {
     const int i = r * RP + ii;
@@ -1553,7 +1569,7 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
                        float inv_tau, int T, int B, int H, int dk, int dv,
                        int rot, i64 ldq, i64 ldk, i64 ldv, i64 ldz, int known,
                        hipStream_t s) {
-  const dim3 grid(B, H, (dv + 31) / 32), ordered(H, grid.z, B);
+  dim3 grid(B, H, (dv + 31) / 32);
   const int rp = (dk + 15) / 16;
   const int rpp = rp <= 2 ? 2 : rp <= 4 ? 4 : rp <= 8 ? 8 : 16;
   // From a block of tokens per sequence on the prompt kernel is the better one
@@ -1578,12 +1594,30 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
   // tokens 22 / 19, 50 tokens 47 / 31, 100 tokens 87 / 47; dk 124 breaks even at 24),
   // otherwise for longer prompts (fp32 17 tokens 32 / 44, 75 tokens 97 / 98, 225 tokens
   // 265 / 253).
-  const i64 groups = (i64)B * H * grid.z;
+  i64 groups = (i64)B * H * grid.z;
   const bool few = groups <= (rpp >= 16 || (sizeof(S) == 4 && zl) ? 256 : 512);
   const bool eight = rpp >= 8 && loads(512) &&
                      (few || (!loads(256) && ((rpp == 8 && (sizeof(S) == 2 || !zl)) ||
                                               T >= 128 * B)));
   const bool prompt = eight || loads(256);
+  // Half of eight waves staging for the other half, 16 columns to a workgroup, where the
+  // longest sequences decide: up to a workgroup per CU of these, or three where the caller
+  // knows them to be uneven.  All waves staging / apart in us: one sequence of 1900 tokens, 8
+  // heads of 128 x 128 with decays per channel 267 / 190, 16 heads, one decay per head 235 /
+  // 165; 4 of 300..700, 4 heads of 64 x 64 79 / 47, 8 of 256 x 256 222 / 158, in fp32 8 of 128
+  // x 128 161 / 135; 3 of 58..82 19.2 / 18.2, but 4 of 49..58 16.2 / 16.7.  6 of 500..1900,
+  // 384 groups 277 / 228, all of 1900 273 / 287; 768 groups 365 / 346, 391 / 373; 8 of
+  // 200..1000, 512 groups 147 / 133, 1024 189 / 193; 512 groups of 256 x 256 182 / 187, in
+  // fp32 161 / 190.
+  const i64 narrow = (i64)B * H * ((dv + 15) / 16);
+  const bool apart =
+      loads(256) && (i64)T >= 64 * (i64)B &&
+      narrow <= (known == LENS_UNEVEN && sizeof(S) == 2 && rpp <= 8 ? 768 : 256);
+  if (apart) {
+    grid.z = (dv + 15) / 16;
+    groups = narrow;
+  }
+  const dim3 ordered(H, grid.z, B);
   const int walk = (i64)T >= 64 * (i64)B ? LONGEST_FIRST    // see scan_sequence
                    : groups <= 256        ? HEADS_IN_TURN
                    : known == LENS_DIFFER ? LONGEST_FIRST_SHORT : IN_ORDER;
@@ -1596,19 +1630,20 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
       out, state, (const S*)q, (const S*)k, (const S*)v, (const S*)zl, zbias, \
       head_decay, inv_freq, positions, cu, q_start, sslot, q_scale, k_scale, \
       inv_tau, H, dk, dv, rot, ldq, ldk, ldv, ldz
-#define SCAN_PROMPT(RP, NT)                                                  \
+#define SCAN_PROMPT(RP, NT, COLS)                                                \
   do {                                                                       \
     if (zl)                                                                  \
-      linear_scan_prompt_kernel<S, RP, true, NT>                             \
+      linear_scan_prompt_kernel<S, RP, true, NT, COLS>                       \
           <<<walk ? ordered : grid, NT, sm, s>>>(SCAN_ARGS, walk);           \
     else                                                                     \
-      linear_scan_prompt_kernel<S, RP, false, NT>                            \
+      linear_scan_prompt_kernel<S, RP, false, NT, COLS>                      \
           <<<walk ? ordered : grid, NT, sm, s>>>(SCAN_ARGS, walk);           \
   } while (0)
 #define SCAN(RP)                                                             \
   do {                                                                       \
-    if (eight) SCAN_PROMPT((RP >= 8 ? RP : 8), 512);                         \
-    else if (prompt) SCAN_PROMPT(RP, 256);                                   \
+    if (apart) SCAN_PROMPT(RP, 512, 16);                                     \
+    else if (eight) SCAN_PROMPT((RP >= 8 ? RP : 8), 512, 32);                \
+    else if (prompt) SCAN_PROMPT(RP, 256, 32);                               \
     else if (single)                                                         \
       linear_scan_kernel<S, RP, 1><<<grid, 256, sm, s>>>(SCAN_ARGS);         \
     else                                                                     \

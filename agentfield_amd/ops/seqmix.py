@@ -616,10 +616,13 @@ def _one_each(md, T: int, B: int) -> bool:
 def _known_lens(md, T: int, B: int) -> int:
     """What the host knows of a step's lengths, for the recurrence's choice of blocks and
     of their order: 1 no sequence has more than one row, 2 up to 16 short ones differ by 16
-    rows or more, up to 32 by 64, and a longer one follows a shorter, 0 anything else."""
+    rows or more, up to 32 by 64, and a longer one follows a shorter, 3 the longest of long
+    ones (256 rows in the mean) has 1.25 times their mean, 0 anything else."""
     if _one_each(md, T, B):
         return 1
     lens = getattr(md, "seq_lens", None)
+    if lens and T >= 256 * B:
+        return 3 if 4 * B * max(lens) >= 5 * T else 0
     if not lens or B > 32 or T >= 64 * B:
         return 0
     unlike = max(lens) - min(lens) >= (16 if B <= 16 else 64)

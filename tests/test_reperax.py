@@ -1161,6 +1161,66 @@ def test_scan_knows_short_prompts_of_unlike_lengths():
     assert known(60, 3) == 0 == known(60, 3, seq_lens=None)
 
 
+def test_scan_knows_long_prompts_of_uneven_lengths():
+    def known(*lens):
+        return sm._known_lens(SimpleNamespace(seq_lens=list(lens)), sum(lens), len(lens))
+    assert known(1100, 300, 300, 300) == 3 == known(0, 512) == known(320, 256, 192)
+    assert known(300, 300) == 0 == known(319, 257, 192) == known(500, 10) == known(256)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("dk,dv,rot", [(16, 1, 0), (32, 16, 16), (56, 17, 0), (64, 40, 32),
+                                       (128, 31, 64), (128, 128, 0), (200, 33, 0),
+                                       (256, 16, 128)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_scan_staged_apart(dtype, dk, dv, rot, gated):
+    """Prompts of 64 tokens and more in the mean on few workgroups, half of whose waves
+    stage for the others: the bits of portions of one and nine tokens, which run on the token
+    kernel.  Around the blocks of tokens, next to empty and to short ones, with padded rows
+    and column tiles; and six uneven ones of 257 to 768 workgroups, known to be so or not."""
+    H = 2
+    g = torch.Generator(device="cuda").manual_seed(dk + dv)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+
+    def case(H, lens):
+        B, T = len(lens), sum(lens)
+        cu = [0, *itertools.accumulate(lens)]
+        q, k, v, z = ((torch.randn(T, n, generator=g, device="cuda") * s).to(dtype)
+                      for n, s in ((H * dk, dk ** -0.5), (H * dk, 0.3), (H * dv, 1.0),
+                                   (H * dk, 2.0)))
+        kw = dict(q_scale=0.5, k_scale=0.7)
+        if gated:
+            kw.update(inv_tau=1 / 16, decay_bias=torch.ones(H * dk, device="cuda"))
+        else:
+            kw.update(head_decay=torch.linspace(0.9, 0.99, H, device="cuda"))
+        if rot:
+            kw.update(inv_freq=sm.rotary_inv_freq(rot, 1e4, "cuda"))
+
+        def run(portion, **known):
+            state = torch.full((B, H, dk, dv), torch.nan, device="cuda")
+            out = torch.full((T, H * dv), torch.nan, device="cuda")
+            for at in range(0, max(lens), portion):
+                take = [max(0, min(portion, n - at)) for n in lens]
+                idx = torch.tensor([c + at + j for c, t in zip(cu, take) for j in range(t)],
+                                   device="cuda")
+                md = SimpleNamespace(cu_seqlens=i32([0, *itertools.accumulate(take)]),
+                                     q_start=i32([at] * B), state_slots=i32(range(B)), **known)
+                pos = i32([at + j for t in take for j in range(t)])
+                out[idx] = sm.linear_scan(q[idx], k[idx], v[idx], state, md, pos, H,
+                                          decay_logits=z[idx] if gated else None, **kw)
+            return out, state[[i for i in range(B) if lens[i]]]
+        return run
+    run = case(H, [1, 16, 0, 33, 300, 257, 15])
+    whole = run(1000)
+    assert all(torch.isfinite(t).all() for t in whole)
+    for portion in (1, 9):
+        assert all(map(torch.equal, run(portion), whole))
+    lens = [200, 210, 220, 230, 240, 500]
+    run = case(-(-50 // -(-dv // 16)), lens)
+    assert all(map(torch.equal, run(1000), run(1000, seq_lens=lens)))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("dk,dv", [(64, 40), (128, 128), (256, 64)])
