@@ -19,7 +19,8 @@
 //   The waves' sums meet once, in LDS; results do not depend on M within this kernel.
 //   The epilogue is the layer's next step: bf16 store, residual add in place,
 //   SwiGLU (a tile is 8 gate and 8 up rows), or rotary embedding + page append (a
-//   tile is 8 rotation pairs of a head).  RMSNorm (its weight is folded into W):
+//   tile is 8 rotation pairs of a head, or 12 in 24 weight rows, see launch_rows).
+//   RMSNorm (its weight is folded into W):
 //   the loop multiplies every X fragment with itself (diagonal of X X^T, one
 //   MFMA), so nobody has to leave row statistics behind.
 // More rows: X would be read once per 16 weight rows, so here four or eight waves
@@ -61,9 +62,9 @@
 // fp32 rounding between steps of different sizes.
 // Measured in us, alone and repeated (inside a step 5-25% more), against the split-K
 // kernel with two-stage buffers and its second launch (in brackets).  One row: 6144 x
-// 4096 with rotary and append 11.3 (21.3 in three launches), 4096 x 4096 7.2 and 4096 x
+// 4096 with rotary and append 10.7 (21.3 in three launches), 4096 x 4096 7.2 and 4096 x
 // 14336 19.5 (together 44.4), SwiGLU over 28672 x 4096 36.0 = 6.5 TB/s (58.2).  16
-// rows: 13.3, 8.0, 23.3, 41.2.  64 rows, without the closing launches: 13.1, 9.3,
+// rows: 11.0, 8.0, 23.3, 41.2.  64 rows, without the closing launches: 13.1, 9.3,
 // 23.3, 38.9 (16.7, o + down 44.8, 62.7).  128 rows: 16.9, 15.0, 27.5, 48.0 (library
 // 25.6 and 57.5 + 5.2 for the first and the last, o + down 63.1).
 #include "mfma_lines.h"
@@ -104,6 +105,13 @@ __device__ __forceinline__ int weight_row(const RowsArgs& a, int tile, int n) {
   return tile * 16 + n;
 }
 
+// The same of the 24-row tiles of EPI_ROPE, three groups of 8 rows: four rotation pairs of a
+// head each, or eight rows of v.
+__device__ __forceinline__ int rope_group_row(const RowsArgs& a, int group, int j) {
+  const int head = group >> 4, at = group & 15;
+  return head * 128 + (head >= a.Hq + a.Hk ? at * 8 + j : at * 4 + (j & 3) + (j & 4) * 16);
+}
+
 // Rotated q / k pair (dims d, d + 64) or plain v pair (dims d, d + 1) of row m to
 // its place.  head counts q, k, v heads in turn.
 __device__ __forceinline__ void put_rope(const RowsArgs& a, int m, int head, int d,
@@ -135,19 +143,20 @@ __device__ __forceinline__ void put_rope(const RowsArgs& a, int m, int head, int
 }
 
 // NORM: 0 none, 1 from ss, 2 computed from X.  PD pieces per wave in flight, with DRAIN
-// until the next is needed.
-template <int PD, int EPI, int NORM, int AUX, bool DRAIN>
+// until the next is needed.  Tiles of WL x 8 weight rows: 2, or 3 with EPI_ROPE.
+template <int PD, int EPI, int NORM, int AUX, bool DRAIN, int WL>
 __device__ __forceinline__ void rows_block(const RowsArgs& a, const int tile) {
   constexpr int NW = 8;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int n = lane & 15;
 
-  constexpr int PIECE = 2048;                    // 16 rows x 64 elements
-  constexpr int SLOT = PIECE * 2;                // of W and of X
+  static_assert(WL == 2 || (WL == 3 && EPI == EPI_ROPE), "tiles");
+  constexpr int PIECE = WL * 1024;               // 8 WL rows x 64 elements
+  constexpr int SLOT = PIECE + 2048;             // of W and of X
   constexpr int RS = 20;                         // column stride of the sums
   constexpr int RING = NW * PD * SLOT;
-  constexpr int SUMS = NW * 16 * RS * 4;
+  constexpr int SUMS = NW * WL * 8 * RS * 4;
   // one array for everything: with a second one the compiler waits for all loads
   // in front of the loop's reads
   constexpr int TAIL = SUMS + (NW + 1) * 16 * 4;
@@ -156,12 +165,13 @@ __device__ __forceinline__ void rows_block(const RowsArgs& a, const int tile) {
 
   // sources of this lane's chunks
   const int r8 = lane >> 3, ch = ((lane & 7) ^ r8) * 8 + wid * 64;
-  const u16 *wp[2], *xp[2];
+  const u16 *wp[WL], *xp[2];
 #pragma unroll
-  for (int g = 0; g < 2; ++g) {
-    wp[g] = a.W + (size_t)weight_row<EPI>(a, tile, g * 8 + r8) * a.K + ch;
-    xp[g] = a.X + (size_t)min(g * 8 + r8, a.M - 1) * a.K + ch;
-  }
+  for (int g = 0; g < WL; ++g)
+    wp[g] = a.W + (size_t)(WL == 3 ? rope_group_row(a, tile * 3 + g, r8)
+                                   : weight_row<EPI>(a, tile, g * 8 + r8)) * a.K + ch;
+#pragma unroll
+  for (int g = 0; g < 2; ++g) xp[g] = a.X + (size_t)min(g * 8 + r8, a.M - 1) * a.K + ch;
   const int cnt = ((a.K >> 6) - wid + NW - 1) / NW;  // this wave's pieces
   const int rot = cnt > 0 ? (tile >> 3) % cnt : 0;
   auto load = [&](int i) {
@@ -169,27 +179,31 @@ __device__ __forceinline__ void rows_block(const RowsArgs& a, const int tile) {
     const int p = i + rot < cnt ? i + rot : i + rot - cnt;
     const size_t off = (size_t)p * (NW * 64);
 #pragma unroll
-    for (int g = 0; g < 2; ++g) load_line8<AUX>(wp[g] + off, to + g * 1024);
+    for (int g = 0; g < WL; ++g) load_line8<AUX>(wp[g] + off, to + g * 1024);
 #pragma unroll
     for (int g = 0; g < 2; ++g)
       load_line8<KEEP>(xp[g] + off, to + PIECE + g * 1024);
   };
-  f32x4 acc = {0, 0, 0, 0}, sq = {0, 0, 0, 0};
+  f32x4 acc[WL - 1], sq = {0, 0, 0, 0};
+#pragma unroll
+  for (int t = 0; t < WL - 1; ++t) acc[t] = f32x4{0, 0, 0, 0};
 #pragma unroll
   for (int s = 0; s < PD; ++s)
     if (s < cnt) load(s);
   for (int i = 0; i < cnt; ++i) {
     // piece i has landed when only the loads of the PD - 1 behind it are out
     if (!DRAIN && i + PD <= cnt)
-      __builtin_amdgcn_s_waitcnt(vmcnt_only(4 * (PD - 1)));
+      __builtin_amdgcn_s_waitcnt(vmcnt_only((WL + 2) * (PD - 1)));
     else
       __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
     asm volatile("" ::: "memory");
     const lds_b* at = ring + (i % PD) * SLOT;
-    bf16x8r w[2], x[2];
+    // the second 16 rows of 24 end in the rows of X, whose products nobody stores
+    bf16x8r w[2][WL - 1], x[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      w[h] = frag(at, h);
+#pragma unroll
+      for (int t = 0; t < WL - 1; ++t) w[h][t] = frag(at + t * 2048, h);
       x[h] = frag(at + PIECE, h);
     }
     // the slot is read: fill it again
@@ -197,7 +211,9 @@ __device__ __forceinline__ void rows_block(const RowsArgs& a, const int tile) {
     if (i + PD < cnt) load(i + PD);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[h], w[h], acc, 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < WL - 1; ++t)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[h], w[h][t], acc[t], 0, 0, 0);
       if (NORM == 2)
         sq = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[h], x[h], sq, 0, 0, 0);
     }
@@ -205,10 +221,12 @@ __device__ __forceinline__ void rows_block(const RowsArgs& a, const int tile) {
 
   // meet in LDS: [wave][tile column][row]; + 4 spreads the columns over banks
   __syncthreads();
-  float (*red)[16][RS] = reinterpret_cast<float (*)[16][RS]>(lds);
+  float (*red)[WL * 8][RS] = reinterpret_cast<float (*)[WL * 8][RS]>(lds);
   float (*rsq)[16] = reinterpret_cast<float (*)[16]>(lds + SUMS);
   float* rstd = rsq[NW];
-  *reinterpret_cast<f32x4*>(&red[wid][n][(lane >> 4) * 4]) = acc;
+  *reinterpret_cast<f32x4*>(&red[wid][n][(lane >> 4) * 4]) = acc[0];
+  if (WL == 3 && n < 8)
+    *reinterpret_cast<f32x4*>(&red[wid][16 + n][(lane >> 4) * 4]) = acc[WL - 2];
   if (NORM == 2) {
 #pragma unroll
     for (int r = 0; r < 4; ++r)
@@ -238,6 +256,16 @@ __device__ __forceinline__ void rows_block(const RowsArgs& a, const int tile) {
   };
 
   // two values per thread: neighbours, or a gate / rotation pair
+  if constexpr (WL == 3) {
+    const int m = threadIdx.x / 12, j = threadIdx.x % 12, c = (j >> 2) * 8, i = j & 3;
+    if (m >= a.M) return;
+    const int group = tile * 3 + (j >> 2), head = group >> 4, at = group & 15;
+    if (head >= a.Hq + a.Hk)
+      put_rope(a, m, head, at * 8 + 2 * i, total(c + 2 * i, m), total(c + 2 * i + 1, m));
+    else
+      put_rope(a, m, head, at * 4 + i, total(c + i, m), total(c + 4 + i, m));
+    return;
+  }
   const int m = threadIdx.x >> 3, j = threadIdx.x & 7;
   if (m >= a.M) return;
   if (EPI == EPI_SWIGLU) {
@@ -263,9 +291,9 @@ __device__ __forceinline__ void rows_block(const RowsArgs& a, const int tile) {
   }
 }
 
-template <int PD, int EPI, int NORM, int AUX, bool DRAIN>
+template <int PD, int EPI, int NORM, int AUX, bool DRAIN, int WL = 2>
 __global__ void __launch_bounds__(512) gemm_rows_kernel(RowsArgs a) {
-  rows_block<PD, EPI, NORM, AUX, DRAIN>(a, blockIdx.x);
+  rows_block<PD, EPI, NORM, AUX, DRAIN, WL>(a, blockIdx.x);
 }
 
 // Several plain products of as many rows in one launch, the longest inner dimension first:
@@ -296,7 +324,7 @@ __global__ void __launch_bounds__(512) gemm_rows_group_kernel(RowsGroup g) {
   a.M = g.M;
   a.N = p.N;
   a.K = p.K;
-  rows_block<2, EPI_PLAIN, 0, AUX, false>(a, blockIdx.x - p.tile0);
+  rows_block<2, EPI_PLAIN, 0, AUX, false, 2>(a, blockIdx.x - p.tile0);
 }
 
 // All but N of a wave's loads have landed, its LDS reads are done, and so it is for
@@ -675,12 +703,34 @@ static bool streamed(const RowsArgs& a) { return (i64)a.N * a.K >= (8 << 20); }
 
 // With the norm computed, where some CUs have two blocks and others one, waves that wait
 // for all they have asked for are faster at few rows.  Rotary, in flight / drained in us:
-// 272 blocks, K 4096 11.5 / 10.9 at one row, 11.8 / 11.6 at 8, K 8192 20.0 / 17.7; 384
-// blocks, K 4096 12.6 / 11.9; 448 12.8 / 12.6; but 512 13.6 / 13.6, K 8192 24.1 / 25.7; 256
+// 272 blocks, K 4096 11.5 / 10.9 at one row, 11.8 / 11.6 at 8, K 8192 20.0 / 17.7; 448
+// blocks 12.8 / 12.6; but 512 13.6 / 13.6, K 8192 24.1 / 25.7; 256
 // 8.5 / 9.8; 576 16.5 / 18.4; K 2048 from 272 blocks on 0 to 3% slower.
+//
+// Rotary, tiles that leave half of the CUs one more than the others: of 24 rows instead of 16
+// all have as many, and X is read a third less often.  Blocks of 16 / 24 rows in us, one row
+// and 16: 384 / 256, K 4096 11.1 / 10.7 and 13.3 / 11.0, K 8192 19.2 / 18.1 and 23.9 / 18.2;
+// 264 / 176, K 4096 10.3 / 8.6 and 12.6 / 10.1; 768 / 512 18.0 / 17.8 and 20.2 / 18.4, K 2048
+// 12.0 / 10.3 and 12.9 / 11.0; K 1024 level.  Not where 16 rows fill their rounds as well: 240
+// / 160 7.7 / 8.3, 480 / 320 12.4 / 14.8, 960 / 640 21.7 / 22.1.  Longer rings (three and four
+// pieces) and, to 8 rows, 8 rows of X instead of 16 change nothing.
+static bool in_24s(const RowsArgs& a) {
+  const int g = a.N / 16, rounds = (a.N / 24 + ROWS_CUS - 1) / ROWS_CUS;
+  return a.N % 24 == 0 && g > rounds * ROWS_CUS && rounds <= 2;
+}
+
 template <int EPI, int NORM>
 static void launch_rows(const RowsArgs& a, hipStream_t st) {
   const int g = a.N / 16;
+  if constexpr (EPI == EPI_ROPE) {
+    if (in_24s(a)) {
+      if (streamed(a))
+        gemm_rows_kernel<2, EPI, NORM, STREAM, false, 3><<<a.N / 24, 512, 0, st>>>(a);
+      else
+        gemm_rows_kernel<2, EPI, NORM, KEEP, false, 3><<<a.N / 24, 512, 0, st>>>(a);
+      return;
+    }
+  }
   if (NORM == 2 && g > ROWS_CUS && g <= 448 && a.K >= 4096 && a.M <= 8)
     gemm_rows_kernel<2, EPI, NORM, STREAM, NORM == 2><<<g, 512, 0, st>>>(a);
   else if (streamed(a))

@@ -1080,6 +1080,19 @@ def test_rows_with_a_norm_between_one_and_two_blocks_per_cu(M, heads):
                  rtol=2 ** -7)
 
 
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("Hq,Hk,K", [
+    (31, 1, 4096),                 # 33 heads, 176 tiles: the fewest that go in 24s
+    (29, 2, 64), (32, 8, 1088),    # waves without a piece; 48 heads, a tile per CU
+    (64, 1, 256), (64, 16, 576),   # 66 and 96 heads, two rounds
+    (30, 1, 256), (32, 1, 256), (47, 2, 256), (62, 1, 256),   # tiles of 16 again
+])
+def test_qkv_rope_rows_in_tiles_of_24(M, Hq, Hk, K):
+    """Tiles of 24 weight rows, whose groups of 8 cross heads and reach from q into k and
+    from k into v.  Tolerance as there."""
+    test_qkv_rope_rows(M, Hq, Hk, K)
+
+
 @pytest.mark.parametrize("M", [3, 40])
 def test_qkv_rope_rows_refuses_other_geometries(M):
     """Head sizes other than 128, weights that are not whole heads, pages, stats
