@@ -610,11 +610,19 @@ __global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
   }
 }
 
-// The parts' sum + rotary positions + page append: grid (M, heads / 4), a head
-// per wave, a rotation (or value) pair per lane.
-__global__ void __launch_bounds__(256) rows_rope_kernel(RowsArgs a, int splits) {
-  const int m = blockIdx.x, lane = threadIdx.x & 63;
-  const int head = blockIdx.y * 4 + (threadIdx.x >> 6);
+// What adds the parts runs an eighth of the columns on each XCD (blockIdx.x): the tiles of
+// the products that wrote them there, every eighth, all splits of which are on one XCD where
+// the tiles are a multiple of 8.  With rows on the XCDs instead (row modulo 8, or any) the
+// products that write the same parts next were slower, 17.2 -> 16.9 us in the mean at 80 rows
+// and 17.4 -> 16.8 at 45, the launches themselves the same.  Steps of 16 layers: 16 x 5 rows
+// behind a history 2581 -> 2540 us, a prompt of 45 1794 -> 1764, 128 rows 3014 -> 2996; 64
+// rows level.
+
+// The parts' sum + rotary positions + page append: grid (8, M, heads / 64), every eighth head
+// a wave, a rotation (or value) pair per lane.
+__global__ void __launch_bounds__(512) rows_rope_kernel(RowsArgs a, int splits) {
+  const int m = blockIdx.y, lane = threadIdx.x & 63;
+  const int head = blockIdx.x + 8 * (blockIdx.z * 8 + (threadIdx.x >> 6));
   if (head >= a.Hq + 2 * a.Hk) return;
   const bool is_v = head >= a.Hq + a.Hk;
   const int d = is_v ? 2 * lane : lane, step = is_v ? 1 : 64;
@@ -632,15 +640,17 @@ __global__ void __launch_bounds__(256) rows_rope_kernel(RowsArgs a, int splits) 
 }
 
 // The parts' sum + residual (in place; a copy to `out` if given) + sums of squares
-// of the new rows (if ss is given): grid (M, 8), a block per eighth of a row.
+// of the new rows (if ss is given): grid (8, M), a block per eighth of a row, every eighth
+// tile of `tile` columns (0: neighbours).
 __global__ void __launch_bounds__(256) rows_residual_kernel(
     u16* __restrict__ residual, u16* __restrict__ out,
     const float* __restrict__ parts, float* __restrict__ ss, int M, int N,
-    int splits) {
-  const int m = blockIdx.x, nb = N / 8, c0 = blockIdx.y * nb;
+    int splits, int tile) {
+  const int m = blockIdx.y, nb = N / 8;
   __shared__ float red[4];
   float local = 0.f;
-  for (int c = c0 + threadIdx.x * 2; c < c0 + nb; c += 512) {
+  for (int i = threadIdx.x * 2; i < nb; i += 512) {
+    const int c = tile ? (i / tile * 8 + blockIdx.x) * tile + i % tile : blockIdx.x * nb + i;
     const u16x2 rv = *reinterpret_cast<const u16x2*>(residual + (size_t)m * N + c);
     float v0 = 0.f, v1 = 0.f;
 #pragma unroll 4
@@ -661,7 +671,7 @@ __global__ void __launch_bounds__(256) rows_residual_kernel(
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = local;
   __syncthreads();
   if (threadIdx.x == 0)
-    ss[m * 8 + blockIdx.y] = (red[0] + red[1]) + (red[2] + red[3]);
+    ss[m * 8 + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 // The parts' sum in bf16, rows optionally scaled by the RMSNorm scalar from ss.
@@ -793,21 +803,25 @@ static void launch_tile(const RowsArgs& a, hipStream_t st) {
 // 12 pieces of K each (6144 x 4096 in 5 at 64 rows: 11.2 us against 12.8, 4096 x 14336
 // in 8: 21.7 against 23.1; but 4096 x 4096 in 8, 8 pieces: 8.8 against 8.5 in 4), always
 // above 64 rows.
+static bool parts_in_128s(const RowsArgs& a, int splits) {
+  if (a.N % 128 || a.M > 64) return a.N % 128 == 0;
+  return a.N / 128 * splits >= 192 && a.K / 64 >= 12 * splits && (a.M > 32 || splits == 1);
+}
+
 template <int AUX>
 static void launch_parts_as(const RowsArgs& a, int splits, hipStream_t st) {
-  const dim3 g64(a.N / 64, splits), g128(a.N / 128, splits);
-  const bool wide = a.N % 128 == 0 && a.N / 128 * splits >= 192 &&
-                    a.K / 64 >= 12 * splits;
-  if (a.M <= 64 && wide && (a.M > 32 || splits == 1))
-    gemm_parts_kernel<4, 8, 4, 3, EPI_PARTS, AUX><<<g128, 512, 0, st>>>(a);
+  const bool wide = parts_in_128s(a, splits);
+  const dim3 g(a.N / (wide ? 128 : 64), splits);
+  if (a.M <= 64 && wide)
+    gemm_parts_kernel<4, 8, 4, 3, EPI_PARTS, AUX><<<g, 512, 0, st>>>(a);
   else if (a.M <= 32)
-    gemm_parts_kernel<2, 4, 1, 4, EPI_PARTS, AUX><<<g64, 256, 0, st>>>(a);
+    gemm_parts_kernel<2, 4, 1, 4, EPI_PARTS, AUX><<<g, 256, 0, st>>>(a);
   else if (a.M <= 64)
-    gemm_parts_kernel<4, 4, 2, 4, EPI_PARTS, AUX><<<g64, 256, 0, st>>>(a);
-  else if (a.N % 128 == 0)
-    gemm_parts_kernel<8, 8, 4, 3, EPI_PARTS, AUX><<<g128, 512, 0, st>>>(a);
+    gemm_parts_kernel<4, 4, 2, 4, EPI_PARTS, AUX><<<g, 256, 0, st>>>(a);
+  else if (wide)
+    gemm_parts_kernel<8, 8, 4, 3, EPI_PARTS, AUX><<<g, 512, 0, st>>>(a);
   else
-    gemm_parts_kernel<8, 4, 2, 3, EPI_PARTS, AUX><<<g64, 256, 0, st>>>(a);
+    gemm_parts_kernel<8, 4, 2, 3, EPI_PARTS, AUX><<<g, 256, 0, st>>>(a);
 }
 
 static void launch_parts(const RowsArgs& a, int splits, hipStream_t st) {
@@ -882,8 +896,9 @@ AF_EXPORT int af_rows_linear(void* out, void* residual, void* parts, void* ss_ou
     rows_sum_kernel<<<g, 256, 0, st>>>(a.out, a.parts, norm ? a.ss : nullptr, M, N,
                                        splits, 1.f / (float)K, eps);
   } else if (mode == 1 || mode == 4) {
-    rows_residual_kernel<<<dim3(M, 8), 256, 0, st>>>(
-        a.residual, a.out, a.parts, (float*)ss_out, M, N, splits);
+    const int tile = parts_in_128s(a, splits) ? 128 : 64;
+    rows_residual_kernel<<<dim3(8, M), 256, 0, st>>>(
+        a.residual, a.out, a.parts, (float*)ss_out, M, N, splits, N % (8 * tile) ? 0 : tile);
   } else {
     return 9008;
   }
@@ -958,6 +973,7 @@ AF_EXPORT int af_rows_qkv(void* q, void* parts, const void* X, const void* W,
   }
   if (!parts || !ss) return 9008;
   launch_parts(a, splits, st);
-  rows_rope_kernel<<<dim3(M, (Hq + 2 * Hk + 3) / 4), 256, 0, st>>>(a, splits);
+  const int heads = (Hq + 2 * Hk + 7) / 8;      // of an XCD
+  rows_rope_kernel<<<dim3(8, M, (heads + 7) / 8), 64 * min(heads, 8), 0, st>>>(a, splits);
   return af_last_err();
 }

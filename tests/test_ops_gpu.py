@@ -1093,6 +1093,32 @@ def test_qkv_rope_rows_in_tiles_of_24(M, Hq, Hk, K):
     test_qkv_rope_rows(M, Hq, Hk, K)
 
 
+@pytest.mark.parametrize("M", [17, 33, 65])
+@pytest.mark.parametrize("N,K", [
+    (512, 256), (1024, 256),       # one tile of 64, or of 128 above 64 rows, per XCD; two
+    (576, 128), (1152, 256),       # no multiple of 8 tiles: neighbours
+    (4096, 3072), (8192, 1024),    # tiles of 128 from 33 rows on; several turns of a block
+])
+def test_parts_meet_by_tiles(M, N, K):
+    """Every column once, whatever the tiles that an XCD adds up, and the rows' sums of
+    squares whole.  Tolerance: one bf16 rounding, and fp32 sums in another order."""
+    x, w = rnd(M, K, seed=M), rnd(N, K, seed=N, scale=1.0 / math.sqrt(K))
+    res, st = rnd(M, N, seed=5), torch.full((M, 8), -1.0, device=DEV)
+    want = res.float() + x.float() @ w.float().t()
+    out = ops.linear_rows(x, w, 4, res, ss_out=st)
+    assert torch.equal(out, res)
+    assert ((res.float() - want).abs() <= 2 ** -8 * want.abs() + 1e-4).all()
+    sq = res.double().pow(2).sum(1)
+    assert ((st.double().sum(1) - sq).abs() <= 2 ** -18 * sq).all()
+
+
+@pytest.mark.parametrize("M", [17, 128])
+@pytest.mark.parametrize("Hq,Hk", [(1, 1), (5, 1), (6, 1), (7, 1), (62, 1), (63, 1), (128, 3)])
+def test_rotary_parts_meet_by_heads(M, Hq, Hk):
+    """Fewer heads than XCDs, one more, and more than a block's 64; as test_qkv_rope_rows."""
+    test_qkv_rope_rows(M, Hq, Hk, 256)
+
+
 @pytest.mark.parametrize("M", [3, 40])
 def test_qkv_rope_rows_refuses_other_geometries(M):
     """Head sizes other than 128, weights that are not whole heads, pages, stats
