@@ -272,30 +272,38 @@ __device__ __forceinline__ void wide_tiles(const WideArgs& a, char* lds, int fir
     float* f4 = a.parts + ((size_t)at.split * a.M + at.row + r0) * cols + c0 + q * 8;
 #pragma unroll
     for (int m = 0; m < G; ++m) {
-      if (EXPERTS ? r0 + m * 16 < at.rows : r0 + m * 16 >= at.fresh) {
+      const bool mine = EXPERTS ? r0 + m * 16 < at.rows : r0 + m * 16 >= at.fresh;
+      if (PARTS) {
 #pragma unroll
-        for (int t = 0; t < (GLU ? 2 : 4); ++t) {
-          if (PARTS) {
-            if (c0 + t * 32 >= at.tn * OUT) {
-              *reinterpret_cast<f32x4*>(f4 + t * 32) = acc[t * 2][m];
-              *reinterpret_cast<f32x4*>(f4 + t * 32 + 4) = acc[t * 2 + 1][m];
-            }
-            continue;
+        for (int t = 0; t < 4; ++t)
+          if (mine && c0 + t * 32 >= at.tn * OUT) {
+            *reinterpret_cast<f32x4*>(f4 + t * 32) = acc[t * 2][m];
+            *reinterpret_cast<f32x4*>(f4 + t * 32 + 4) = acc[t * 2 + 1][m];
           }
-          bf16x8r v;
+        f4 += 16 * (size_t)cols;
+        continue;
+      }
+      // a group of rows at a time, converted by all lanes: behind the branch the compiler
+      // moved all sums to registers first, 256 of them instead of 140, and the experts'
+      // kernels spilled 56 (8 experts of 14336 x 4096, two per row: 4096 rows 2430 -> 2378 us,
+      // 1500 rows 1024 -> 1013, up to 1100 level; without experts nothing)
+      __builtin_amdgcn_sched_barrier(0);
+      bf16x8r v[GLU ? 2 : 4];
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            float f = acc[t * 2 + (j >> 2)][m][j & 3];
-            if (GLU)
-              f = f * __builtin_amdgcn_rcpf(1.f + __expf(-f)) *
-                  acc[(GLU ? 4 : 0) + t * 2 + (j >> 2)][m][j & 3];
-            v[j] = (__bf16)f;
-          }
-          if (c0 + t * 32 >= at.tn * OUT) *reinterpret_cast<bf16x8r*>(o + t * 32) = v;
+      for (int t = 0; t < (GLU ? 2 : 4); ++t) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          float f = acc[t * 2 + (j >> 2)][m][j & 3];
+          if (GLU)
+            f = f * __builtin_amdgcn_rcpf(1.f + __expf(-f)) *
+                acc[(GLU ? 4 : 0) + t * 2 + (j >> 2)][m][j & 3];
+          v[t][j] = (__bf16)f;
         }
       }
+#pragma unroll
+      for (int t = 0; t < (GLU ? 2 : 4); ++t)
+        if (mine && c0 + t * 32 >= at.tn * OUT) *reinterpret_cast<bf16x8r*>(o + t * 32) = v[t];
       o += 16 * (size_t)cols;
-      f4 += 16 * (size_t)cols;
     }
     if (next >= nt) break;
     p = next;
