@@ -770,14 +770,16 @@ def test_attn_decode_shares(G, page, nsplit, lens):
     check(ops.attn_decode(qd, kd, vd, btd, L, nsplit=nsplit), lens)
     scratch = tuple(torch.full((B, Hk, nsplit, G, n), torch.nan, device=DEV) for n in (D, 2))
     check(ops.attn_decode(qd, kd, vd, btd, L, nsplit=nsplit, scratch=scratch), lens)
-    graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        out = ops.attn_decode(qd, kd, vd, btd, L, nsplit=nsplit)
-    for turned in (lens[::-1], [min(n, 90) for n in lens], lens):
-        vd.copy_(values(turned))
-        L.copy_(torch.tensor(turned, dtype=torch.int32))
-        graph.replay()
-        check(out, turned)
+    # (torch's own state of captures is an inference tensor once one was made in that mode)
+    with torch.inference_mode():
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = ops.attn_decode(qd, kd, vd, btd, L, nsplit=nsplit)
+        for turned in (lens[::-1], [min(n, 90) for n in lens], lens):
+            vd.copy_(values(turned))
+            L.copy_(torch.tensor(turned, dtype=torch.int32))
+            graph.replay()
+            check(out, turned)
 
 
 @pytest.mark.parametrize("Hk,nsplit", [(3, 1), (4, 1), (4, 2), (8, 1), (8, 3), (11, 2)])
