@@ -92,7 +92,8 @@ __device__ __forceinline__ Visible visible(int L, int win) {
 // (a step of 16 layers 3205 / 2907), 9 of 1600..8000 in four 53 / 44, 24 of 800..4000 in two
 // 57 / 48, 5 of 300..3000 with 32 heads 36 / 31, 30 of up to 8000 with G = 8 113 / 86.  Four
 // rounds are what going on takes (3 us: a merge more, loads from the start); looking at the
-// lengths costs those that stay with nsplit parts 0.3 to 0.8 us (17 of 400 13.5 / 14.3).
+// lengths costs those that stay with nsplit parts 0.3 to 1.3 us (17 of 400 13.3 / 14.0, 16 of
+// 513..576 13.8 / 15.1, 24 of 900..1000 22.5 / 23.5).
 // Loads of a part before the cut is known: 0.2 us less there, 4 us more here.
 struct Cut { int mine, share; };   // rounds of the lane's sequence, of a slot (0: nsplit parts)
 __device__ __forceinline__ Cut find_cut(int L, int B, int nsplit, int slots, int win) {
@@ -105,8 +106,9 @@ __device__ __forceinline__ Cut find_cut(int L, int B, int nsplit, int slots, int
   return {mine, (__builtin_amdgcn_readfirstlane((int)total) + slots - 1) / slots};
 }
 
-// Rounds of each of n parts; n is 2, 3 or 4
+// Rounds of each of n parts; n is 2, 3, 4 or 5
 __device__ __forceinline__ int split_rounds(int rounds, int n) {
+  if (n == 5) return (int)(((uint64_t)(uint32_t)(rounds + 4) * 0xCCCCCCCDull) >> 34);
   if (n == 3) return (int)(((uint64_t)(uint32_t)(rounds + 2) * 0xAAAAAAABull) >> 33);
   return n == 2 ? (rounds + 1) >> 1 : (rounds + 3) >> 2;
 }
@@ -489,6 +491,10 @@ AF_EXPORT int af_attn_decode(void* out, void* po, void* pml, const void* q,
   const bool cut = nsplit > 1 && nsplit <= 4 && B > 1 && B <= 64 && win <= 0 &&
                    B * Hk * nsplit <= 256 * (G == 8 ? 2 : 3);
   const int slots = cut ? max(0, min(B * nsplit, cap - (B - 1))) : 0;
+  // The room for shares does for a fifth part of lengths alike, which makes up for the look
+  // at them where two blocks per CU hold all: four / five parts, 12 of 800..1000 17.2 / 16.3
+  // us, of 1500..3000 27.9 / 27.1, 9 of 1600..8000 44 / 40; but 16 of 500..4000 34.7 / 41.
+  if (slots > 0 && nsplit == 4 && cap >= B * 5 && B * Hk * 5 <= 512) nsplit = 5;
   const int faster = heads_first(Hk, nsplit) ? Hk : B;
   const dim3 grid(B * Hk, nsplit), blk(64 * AD_WAVES);
   hipStream_t st = (hipStream_t)stream;
