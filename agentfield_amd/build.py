@@ -72,7 +72,7 @@ MIX_GROUPS = {
 }
 MIX_SOURCES = [s for _lib, srcs in MIX_GROUPS.values() for s in srcs]
 MIX_LIB = MIX_GROUPS["seq"][0]
-HEADERS = ["common.h", "mfma_lines.h", "mix_attn.h", "mix_rows.h"]
+HEADERS = ["common.h", "decode_cut.h", "mfma_lines.h", "mix_attn.h", "mix_rows.h"]
 
 # hipcc -O3 may otherwise fuse scalar float code into packed-fp32 VALU ops
 HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",

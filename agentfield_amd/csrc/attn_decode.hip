@@ -30,23 +30,24 @@
 //   [dl*8, dl*8+8) and reads the same V rows whole, ~13 clocks per token at
 //   G = 4.
 //   Rows, then waves (through LDS), then splits (second kernel) merge once.
+// A sequence's result has nothing of the others, unless the step's cut (decode_cut.h) is
+// given: where that cuts unlike lengths in equal shares, the order of a sequence's fp32 sums
+// depends on the lengths beside it, and so may the last bit of its bf16 results.
 // Measured with 8 K/V heads, G = 4, against one lane group per token with a
 // shuffle reduction per score: 24 sequences of 1800..8100 tokens (513 MB)
-// 225 -> 108 us (4.7 TB/s), 128 of 545 101 -> 51 us (5.6 TB/s), 1 of 8000
-// 58 -> 22 us.  V is read with nontemporal loads, whole rows per instruction: 114
+// 225 -> 108 us (4.7 TB/s), in equal shares 84 (6.1), 128 of 545 101 -> 49 us (5.8 TB/s),
+// 1 of 8000 58 -> 16 us.  V is read with nontemporal loads, whole rows per instruction: 114
 // -> 108 and 57.3 -> 52.5 us.  K is not: two instructions share each of its lines,
 // and a line dropped between them is fetched twice (64 ragged sequences of up to
 // 2000 tokens 60 -> 65 us with both, 59 with V only).  Not the loads' latency: eight
 // waves per block (114 -> 125 us) and whole rows through LDS with two tiles per wave in
 // flight (110.5 -> 112) do not help, nor do pages in order.
-#include "common.h"
+#include "decode_cut.h"
 
 #include <type_traits>
 
 #define AD_D 128
 #define AD_MAXG 8
-#define AD_TILE 16   // tokens per wave iteration
-#define AD_WAVES 4
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8d;
 
@@ -71,80 +72,23 @@ __device__ __forceinline__ void each_head(F f) {
   }
 }
 
-// splits are whole rounds of the block's waves
-constexpr int ROUND = AD_TILE * AD_WAVES;
-
-// Visible tokens of a sequence are [first, L), its rounds begin at a whole tile.
-struct Visible { int first, tile0, rounds; };
-__device__ __forceinline__ Visible visible(int L, int win) {
-  // sliding window (Mistral): only the last `win` tokens
-  const int s0 = (win > 0 && L > win) ? L - win : 0;
-  const int a0 = s0 & ~(AD_TILE - 1);
-  return {s0, a0, (L - a0 + ROUND - 1) / ROUND};
-}
-
-// How the sequences of a step, a lane's each, are cut.  In nsplit parts each, the longest
-// decide: 24 of 1800..8100 tokens in two are blocks of 900 to 4050 tokens, 105 us where as
-// many tokens in sequences of one length take 86.  Where that leaves enough to win, all of
-// them are cut as one row of rounds into `slots` equal shares instead: a block goes on into
-// the next sequence, and its part of each is a piece, number slot + sequence.  Every block
-// and every merge finds the same cut.  In us, nsplit parts / equal shares: the above 105 / 90
-// (a step of 16 layers 3205 / 2907), 9 of 1600..8000 in four 53 / 44, 24 of 800..4000 in two
-// 57 / 48, 5 of 300..3000 with 32 heads 36 / 31, 30 of up to 8000 with G = 8 113 / 86.  Four
-// rounds are what going on takes (3 us: a merge more, loads from the start); looking at the
-// lengths costs those that stay with nsplit parts 0.3 to 1.3 us (17 of 400 13.3 / 14.0, 16 of
-// 513..576 13.8 / 15.1, 24 of 900..1000 22.5 / 23.5).
-// Loads of a part before the cut is known: 0.2 us less there, 4 us more here.
-struct Cut { int mine, share; };   // rounds of the lane's sequence, of a slot (0: nsplit parts)
-__device__ __forceinline__ Cut find_cut(int L, int B, int nsplit, int slots, int win) {
-  const int mine = (int)(threadIdx.x & 63) < B ? visible(L, win).rounds : 0;
-  const float total = wave_sum_f32((float)mine), most = wave_max_f32((float)mine);
-  // the largest part against a share, in products: this is on the way of every call
-  const int even =
-      most * (float)slots <= (float)nsplit * (total + 4.f * (float)slots);
-  if (__builtin_amdgcn_readfirstlane(even)) return {mine, 0};
-  return {mine, (__builtin_amdgcn_readfirstlane((int)total) + slots - 1) / slots};
-}
-
-// Rounds of each of n parts; n is 2, 3, 4 or 5
-__device__ __forceinline__ int split_rounds(int rounds, int n) {
-  if (n == 5) return (int)(((uint64_t)(uint32_t)(rounds + 4) * 0xCCCCCCCDull) >> 34);
-  if (n == 3) return (int)(((uint64_t)(uint32_t)(rounds + 2) * 0xAAAAAAABull) >> 33);
-  return n == 2 ? (rounds + 1) >> 1 : (rounds + 3) >> 2;
-}
-
-// Sums over the lanes up to a lane's own
-__device__ __forceinline__ int wave_scan(int v) {
-#define AD_ADD(CTRL, ROWS) \
-  v += __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false)
-  AD_ADD(0x111, 0xf);   // a row's lanes 1, 2, 4 and 8 below
-  AD_ADD(0x112, 0xf);
-  AD_ADD(0x114, 0xf);
-  AD_ADD(0x118, 0xf);
-  AD_ADD(0x142, 0xa);   // the last lane of rows 0 and 2, then of the lower half
-  AD_ADD(0x143, 0xc);
-#undef AD_ADD
-  return v;
-}
-
 // Partial layout: po [B, Hk, NSPLIT, G, D] f32; pml [B, Hk, NSPLIT, G, 2] f32
 // (maximum in units of log2, sum; a split without tokens leaves po unwritten);
 // CUT: [Hk, cap, G, ..], cap pieces, split s of sequence b at b * nsplit + s.
 //
 // TILED: page_size is a multiple of AD_TILE, so a tile lies in one page and its
 // index is a scalar load; otherwise every lane looks its tokens' pages up.
-// CUT: with find_cut, where the launcher says so.
-template <int G, bool TILED, bool CUT>
-__global__ void __launch_bounds__(64 * AD_WAVES, (G == 8 ? 3 : 4) - CUT) attn_decode_kernel(
+//
+// A block's part: rounds of sequence b from its skip'th on, sums to piece.  GO_ON: and `left`
+// rounds of the sequences behind it.
+template <int G, bool TILED, bool GO_ON>
+__device__ __forceinline__ void attn_part(
     u16* __restrict__ out, float* __restrict__ po, float* __restrict__ pml,
     const u16* __restrict__ q, const u16* __restrict__ kc, const u16* __restrict__ vc,
-    const i32* __restrict__ bt, const i32* __restrict__ len,
-    float scale, int B, int Hk, int page_size, int page_shift, int max_pages,
-    int nsplit, int slots, int cap, i64 qs, int win, int faster) {
-  // `faster`, the number of heads or of sequences, runs within x
-  const int hi = blockIdx.x / faster, lo = blockIdx.x - hi * faster, split = blockIdx.y;
-  const int kvh = faster == Hk ? lo : hi;
-  int b = faster == Hk ? hi : lo;
+    const i32* __restrict__ bt, const i32* __restrict__ len, float scale, int B, int Hk,
+    int page_size, int page_shift, int max_pages, int nsplit, i64 qs, int win,
+    float (*s_ml)[G][2], float (*s_o)[G][AD_D], int kvh, int b, int L, int skip, int rounds,
+    size_t piece, int left) {
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int tg = lane >> 4, dl = lane & 15;
@@ -158,42 +102,16 @@ __global__ void __launch_bounds__(64 * AD_WAVES, (G == 8 ? 3 : 4) - CUT) attn_de
   auto page_of = [&](int t) {
     return btrow[page_shift >= 0 ? t >> page_shift : t / page_size];
   };
-  // a part: its visible tokens [t0, t1), tile grid, place; this wave's tile and its page
+  // a part: its visible tokens [t0, t1), tile grid; this wave's tile and the next one's page
   int c0, t0, t1, t, pg_next = 0;
-  size_t piece = CUT ? (size_t)kvh * cap + b * nsplit + split
-                     : ((size_t)b * Hk + kvh) * nsplit + split;
   auto take = [&](int L, int skip, int rounds) {
     const Visible v = visible(L, win);
     c0 = v.tile0 + skip * ROUND;
     t1 = min(L, c0 + rounds * ROUND);
     t0 = max(v.first, c0);
     t = c0 + wid * AD_TILE;
-    if (CUT && TILED) pg_next = page_of(min(t, max(t1 - 1, 0)));
   };
-  int left = 0;                            // rounds of this slot behind the part
-  {
-    const int lens = CUT ? len[min(lane, B - 1)] : 0;
-    const int L = len[b], rounds = visible(L, win).rounds;
-    const int part = CUT ? split_rounds(rounds, nsplit) : (rounds + nsplit - 1) / nsplit;
-    take(L, split * part, part);
-    if (CUT) {
-      __builtin_amdgcn_sched_barrier(0);   // the page is looked up meanwhile
-      const Cut c = find_cut(lens, B, nsplit, slots, win);
-      if (c.share > 0) {
-        const int slot = split * B + b, at = slot * c.share;
-        const int sum = wave_scan(c.mine);
-        const unsigned long long behind = __ballot(sum > at);
-        if (slot >= slots || behind == 0) return;
-        b = (int)__ffsll(behind) - 1;
-        piece = (size_t)kvh * cap + slot + b;
-        btrow = tables + (size_t)b * max_pages;
-        const int skip = at - __builtin_amdgcn_readlane(sum - c.mine, b);
-        const int now = min(c.share, __builtin_amdgcn_readlane(c.mine, b) - skip);
-        left = c.share - now;
-        take(__builtin_amdgcn_readlane(lens, b), skip, now);
-      }
-    }
-  }
+  take(L, skip, rounds);
   if (c0 >= t1) {                          // no tokens (uniform in the block)
     if (nsplit > 1) {
       if (threadIdx.x < G) {
@@ -257,11 +175,9 @@ __global__ void __launch_bounds__(64 * AD_WAVES, (G == 8 ? 3 : 4) - CUT) attn_de
   auto begin = [&]() {                     // the wave's first tile
     load_q();
     if (t >= t1) return;
-    load_tile(t, CUT ? pg_next : TILED ? page_of(t) : 0, kf, vf);
+    load_tile(t, TILED ? page_of(t) : 0, kf, vf);
     if (TILED) pg_next = page_of(min(t + ROUND, t1 - 1));
   };
-  __shared__ float s_ml[AD_WAVES][G][2];
-  __shared__ float s_o[AD_WAVES][G][AD_D];
   begin();
   for (;;) {
     float m = AF_NEG_INF, l = 0.f, acc[G][8];
@@ -323,7 +239,7 @@ __global__ void __launch_bounds__(64 * AD_WAVES, (G == 8 ? 3 : 4) - CUT) attn_de
     const int of = b;
     const size_t to = piece;
     bool on = false;
-    if (CUT && left > 0) {
+    if (GO_ON && left > 0) {
       int L = 0;
       while (L <= 0 && b + 1 < B) {
         L = lengths[++b];
@@ -395,6 +311,50 @@ __global__ void __launch_bounds__(64 * AD_WAVES, (G == 8 ? 3 : 4) - CUT) attn_de
   }
 }
 
+// CUT: sequences are cut as the step's cut says (decode_cut.h).  The parts' code stands there
+// twice: with one body for nsplit parts and for shares, what goes on behind a part cost those
+// that do not 0.3 to 0.7 us.
+template <int G, bool TILED, bool CUT>
+__global__ void __launch_bounds__(64 * AD_WAVES, (G == 8 ? 3 : 4) - CUT) attn_decode_kernel(
+    u16* __restrict__ out, float* __restrict__ po, float* __restrict__ pml,
+    const u16* __restrict__ q, const u16* __restrict__ kc, const u16* __restrict__ vc,
+    const i32* __restrict__ bt, const i32* __restrict__ len, const CutRow* __restrict__ cut,
+    float scale, int B, int Hk, int page_size, int page_shift, int max_pages,
+    int nsplit, int cap, i64 qs, int win, int faster) {
+  __shared__ float s_ml[AD_WAVES][G][2];
+  __shared__ float s_o[AD_WAVES][G][AD_D];
+  // `faster`, the number of heads or of sequences, runs within x
+  const int hi = blockIdx.x / faster, lo = blockIdx.x - hi * faster, split = blockIdx.y;
+  const int kvh = faster == Hk ? lo : hi, b = faster == Hk ? hi : lo;
+#define AD_PART(GO_ON, ...)                                                               \
+  attn_part<G, TILED, GO_ON>(out, po, pml, q, kc, vc, bt, len, scale, B, Hk, page_size,   \
+                             page_shift, max_pages, nsplit, qs, win, s_ml, s_o, kvh,      \
+                             __VA_ARGS__)
+  if constexpr (!CUT) {
+    const int L = len[b], part = (visible(L, win).rounds + nsplit - 1) / nsplit;
+    AD_PART(false, b, L, split * part, part, ((size_t)b * Hk + kvh) * nsplit + split, 0);
+  } else {
+    typedef const __attribute__((address_space(4))) CutRow* rows;
+    const CutRow own = ((rows)cut)[b];
+    const int share = own[0], part = own[2];
+    if (share == 0) {
+      AD_PART(false, b, own[1], split * part, part,
+              (size_t)kvh * cap + b * nsplit + split, 0);
+    } else {
+      const int lane = threadIdx.x & 63, slot = split * B + b, at = slot * share;
+      const CutRow seq = cut[min(lane, B - 1)];
+      const unsigned long long behind = __ballot(lane < B && seq[3] > at);
+      if (behind == 0) return;
+      const int from = (int)__ffsll(behind) - 1;
+      const int begin = from > 0 ? __builtin_amdgcn_readlane(seq[3], max(from - 1, 0)) : 0;
+      const int now = min(share, __builtin_amdgcn_readlane(seq[3], from) - at);
+      AD_PART(true, from, __builtin_amdgcn_readlane(seq[1], from), at - begin, now,
+              (size_t)kvh * cap + slot + from, share - now);
+    }
+  }
+#undef AD_PART
+}
+
 // Combine split partials: grid (B, Hq), one wave, 2 dims per lane.  A launch that is all
 // latency: maxima, sums and partial outputs of up to NS splits (more go round again) are
 // asked for together and wait once, not split by split (a decode step of 16 layers, one
@@ -402,17 +362,15 @@ __global__ void __launch_bounds__(64 * AD_WAVES, (G == 8 ? 3 : 4) - CUT) attn_de
 // 2050).  Splits behind the last repeat it; those without tokens, whose po was not
 // written, are left out of the sum.
 // CUT: the parts are asked for as if there were nsplit each, and again where there are
-// shares (find_cut), so that the lengths are not waited for first.
+// shares, so that the cut is not waited for first.
 template <int NS, bool CUT>
 __global__ void __launch_bounds__(64) attn_decode_combine_kernel(
     u16* __restrict__ out, const float* __restrict__ po, const float* __restrict__ pml,
-    const i32* __restrict__ len, int B, int Hq, int G, int nsplit, int slots, int cap,
-    int win) {
+    const CutRow* __restrict__ cut, int Hq, int G, int nsplit, int cap) {
   const int b = blockIdx.x, h = blockIdx.y;
   const int kvh = h / G, g = h % G;
   const int Hk = Hq / G;
   const int lane = threadIdx.x;
-  const int lens = CUT ? len[min(lane, B - 1)] : 0;
   size_t first = CUT ? ((size_t)kvh * cap + b * nsplit) * G + g
                      : (((size_t)b * Hk + kvh) * nsplit) * G + g;
   int n = nsplit;
@@ -428,13 +386,11 @@ __global__ void __launch_bounds__(64) attn_decode_combine_kernel(
   };
   if (CUT) {
     ask(0);
-    __builtin_amdgcn_sched_barrier(0);
-    const Cut c = find_cut(lens, B, nsplit, slots, win);
-    if (c.share > 0) {
-      const int sum = wave_scan(c.mine);
-      const int rounds = __builtin_amdgcn_readlane(c.mine, b);
-      const int end = __builtin_amdgcn_readlane(sum, b), slot = (end - rounds) / c.share;
-      n = rounds > 0 ? (end - 1) / c.share - slot + 1 : 0;
+    const CutRow own = cut[b];
+    const int share = own[0];
+    if (share > 0) {
+      const int start = b > 0 ? cut[b - 1][3] : 0, end = own[3], slot = start / share;
+      n = end > start ? (end - 1) / share - slot + 1 : 0;
       first = ((size_t)kvh * cap + slot + b) * G + g;
       if (n > 0) ask(0);
     }
@@ -476,25 +432,17 @@ static bool heads_first(int Hk, int nsplit) {
 
 AF_EXPORT int af_attn_decode(void* out, void* po, void* pml, const void* q,
                              const void* kc, const void* vc, const void* bt,
-                             const void* len, float scale, int B, int Hq, int Hk,
-                             int D, int page_size, int max_pages, int nsplit,
-                             int cap, i64 qs, int win, void* stream) {
+                             const void* len, const void* cut, float scale, int B,
+                             int Hq, int Hk, int D, int page_size, int max_pages,
+                             int nsplit, int cap, i64 qs, int win, void* stream) {
   if (D != AD_D) return 9002;
   const int G = Hq / Hk;
   if (G < 1 || G > AD_MAXG || G * Hk != Hq) return 9003;
   if (B == 0) return 0;
   if (nsplit > 1 && cap < B * nsplit) return 9004;
-  // Equal shares: slots + B - 1 pieces at most.  A lane per sequence; all blocks have room
-  // at once, or the dispatch evens them out.  Beyond four parts a sequence is short, or the
-  // step is small (seven of 200..2000 in eight 14.7 us, 16 with a look at the lengths).  Long
-  // sequences behind a window are of one length.
-  const bool cut = nsplit > 1 && nsplit <= 4 && B > 1 && B <= 64 && win <= 0 &&
-                   B * Hk * nsplit <= 256 * (G == 8 ? 2 : 3);
-  const int slots = cut ? max(0, min(B * nsplit, cap - (B - 1))) : 0;
-  // The room for shares does for a fifth part of lengths alike, which makes up for the look
-  // at them where two blocks per CU hold all: four / five parts, 12 of 800..1000 17.2 / 16.3
-  // us, of 1500..3000 27.9 / 27.1, 9 of 1600..8000 44 / 40; but 16 of 500..4000 34.7 / 41.
-  if (slots > 0 && nsplit == 4 && cap >= B * 5 && B * Hk * 5 <= 512) nsplit = 5;
+  // B * nsplit shares are as many pieces and B - 1 at most
+  const bool shares = cut && nsplit > 1 && nsplit <= 4 && B > 1 && B <= CUT_MAX &&
+                      win <= 0 && cap >= B * (nsplit + 1) - 1;
   const int faster = heads_first(Hk, nsplit) ? Hk : B;
   const dim3 grid(B * Hk, nsplit), blk(64 * AD_WAVES);
   hipStream_t st = (hipStream_t)stream;
@@ -503,11 +451,11 @@ AF_EXPORT int af_attn_decode(void* out, void* po, void* pml, const void* q,
 #define AF_LAUNCH2(GG, TT, CUT)                                                  \
   attn_decode_kernel<GG, TT, CUT><<<grid, blk, 0, st>>>(                         \
       (u16*)out, (float*)po, (float*)pml, (const u16*)q, (const u16*)kc,         \
-      (const u16*)vc, (const i32*)bt, (const i32*)len, scale, B, Hk, page_size,  \
-      shift, max_pages, nsplit, slots, cap, qs, win, faster)
+      (const u16*)vc, (const i32*)bt, (const i32*)len, (const CutRow*)cut, scale, \
+      B, Hk, page_size, shift, max_pages, nsplit, cap, qs, win, faster)
 #define AF_LAUNCH1(GG, TT)                                                       \
   do {                                                                           \
-    if (slots > 0) AF_LAUNCH2(GG, TT, true);                                     \
+    if (shares) AF_LAUNCH2(GG, TT, true);                                        \
     else AF_LAUNCH2(GG, TT, false);                                              \
   } while (0)
 #define AF_LAUNCH(GG)                                                            \
@@ -529,15 +477,28 @@ AF_EXPORT int af_attn_decode(void* out, void* po, void* pml, const void* q,
     const dim3 g2(B, Hq);
 #define AF_COMBINE(NS)                                                           \
   do {                                                                           \
-    const auto merge = slots > 0 ? attn_decode_combine_kernel<NS, true>          \
-                                 : attn_decode_combine_kernel<NS, false>;        \
+    const auto merge = shares ? attn_decode_combine_kernel<NS, true>             \
+                              : attn_decode_combine_kernel<NS, false>;           \
     merge<<<g2, 64, 0, st>>>((u16*)out, (const float*)po, (const float*)pml,     \
-                             (const i32*)len, B, Hq, G, nsplit, slots, cap, win); \
+                             (const CutRow*)cut, Hq, G, nsplit, cap);             \
   } while (0)
     if (nsplit <= 4) AF_COMBINE(4);
     else if (nsplit <= 8) AF_COMBINE(8);
     else AF_COMBINE(16);
 #undef AF_COMBINE
   }
+  return af_last_err();
+}
+
+// The cut of a step whose embedding does not make it.
+__global__ void __launch_bounds__(64) decode_cut_kernel(CutRow* __restrict__ cut,
+                                                        const i32* __restrict__ len, int B,
+                                                        int nsplit) {
+  write_cut(cut, len, B, nsplit);
+}
+
+AF_EXPORT int af_decode_cut(void* cut, const void* len, int B, int nsplit, void* stream) {
+  if (B < 1 || B > CUT_MAX || nsplit < 1) return 9002;
+  decode_cut_kernel<<<1, 64, 0, (hipStream_t)stream>>>((CutRow*)cut, (const i32*)len, B, nsplit);
   return af_last_err();
 }

@@ -4,7 +4,7 @@
 // k, v      : [T, Hk*D] bf16 (post-RoPE)
 // kc, vc    : [npages, Hk, page_size, D] bf16
 // slot[t]   : global slot = page_index*page_size + in_page_offset (i64), -1 skips
-#include "common.h"
+#include "decode_cut.h"
 
 __global__ void __launch_bounds__(256) reshape_and_cache_kernel(
     const u16* __restrict__ k, const u16* __restrict__ v,
@@ -41,13 +41,19 @@ AF_EXPORT int af_reshape_and_cache(const void* k, const void* v, void* kc, void*
 // Gather rows of an i32 embedding-free path is not needed; but the engine uses
 // an embedding gather for input ids -> hidden states.
 // emb: [V, H] bf16, ids: [T] i32, out: [T, H] bf16.  ss (optional) gets the
-// per-row sum of squares, seeding the fused-norm decode path.
+// per-row sum of squares, seeding the fused-norm decode path.  A decode step's rows also
+// leave the cut of their attention (optional, decode_cut.h), in a block of its own.
 __global__ void __launch_bounds__(256) embedding_kernel(
     u16* __restrict__ out, const u16* __restrict__ emb, const i32* __restrict__ ids,
-    float* __restrict__ ss, int T, int H) {
-  const int per_row = H / 8;
+    float* __restrict__ ss, int T, int H, CutRow* __restrict__ cut,
+    const i32* __restrict__ len, int B, int nsplit) {
+  const int per_row = H / 8, blocks = cut ? gridDim.x - 1 : gridDim.x;
+  if (blockIdx.x == blocks) {
+    if (threadIdx.x < 64) write_cut(cut, len, B, nsplit);
+    return;
+  }
   __shared__ float red[4];
-  for (int t = blockIdx.x; t < T; t += gridDim.x) {
+  for (int t = blockIdx.x; t < T; t += blocks) {
     const u16* src = emb + (size_t)ids[t] * H;
     u16* dst = out + (size_t)t * H;
     float local = 0.f;
@@ -75,11 +81,14 @@ __global__ void __launch_bounds__(256) embedding_kernel(
 }
 
 AF_EXPORT int af_embedding(void* out, const void* emb, const void* ids,
-                           void* ss, int T, int H, void* stream) {
+                           void* ss, int T, int H, void* cut, const void* len, int B,
+                           int nsplit, void* stream) {
   if (H % 8) return 9001;
+  if (cut && (B < 1 || B > CUT_MAX || nsplit < 1)) return 9002;
   if (T == 0) return 0;
   int blocks = T < 2048 ? T : 2048;
-  embedding_kernel<<<blocks, 256, 0, (hipStream_t)stream>>>(
-      (u16*)out, (const u16*)emb, (const i32*)ids, (float*)ss, T, H);
+  embedding_kernel<<<blocks + (cut ? 1 : 0), 256, 0, (hipStream_t)stream>>>(
+      (u16*)out, (const u16*)emb, (const i32*)ids, (float*)ss, T, H, (CutRow*)cut,
+      (const i32*)len, B, nsplit);
   return af_last_err();
 }

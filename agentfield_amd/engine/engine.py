@@ -971,8 +971,10 @@ class LLMEngine:
             return None
         cfg = self.cfg
         G = cfg.num_heads // cfg.num_kv_heads
-        return ops.decode_scratch(bs, cfg.num_kv_heads, nsplit, G, self.device,
-                                  cfg.head_dim)
+        return ops.decode_scratch(
+            bs, cfg.num_kv_heads, nsplit, G, self.device, cfg.head_dim,
+            ops.decode_shares(bs, cfg.num_kv_heads, G, nsplit,
+                              getattr(cfg, "sliding_window", 0)))
 
     def _get_graph(self, bs: int, tkp: bool, lp: bool = False):
         key = (bs, tkp, lp)

@@ -11,6 +11,7 @@ Layout decisions (MI355X-first):
 """
 from __future__ import annotations
 
+import copy
 import math
 from dataclasses import dataclass
 
@@ -131,7 +132,8 @@ class AttnMetadata:
              lens), q_start [B] i32 (absolute chunk start; 0 unless chunked),
              block_table [B,maxp] i32, slots [T] i64.
     Decode:  block_table [B,maxp] i32, seq_lens_t [B] i32, slots [B] i64,
-             nsplit chosen by the engine.
+             nsplit chosen by the engine; decode_cut is the model's, of one
+             step.
     Models that keep per-sequence state besides K/V (recurrent mixers, token
     shift) also get state_slots [B] i32 and row_seq [T] i32 (the sequence
     index of every row); for them a decode step is the packed-chunk layout
@@ -146,6 +148,7 @@ class AttnMetadata:
     seq_lens_t: torch.Tensor | None = None
     nsplit: int = 1
     decode_scratch: tuple | None = None
+    decode_cut: ops.DecodeCut | None = None
     state_slots: torch.Tensor | None = None
     row_seq: torch.Tensor | None = None
     step_tiles: tuple | None = None     # row tiles that the step's layers share
@@ -202,7 +205,8 @@ class LlamaAttention(nn.Module):
         return ops.attn_decode(q, kv.k[self.layer_idx], kv.v[self.layer_idx],
                                md.block_table, md.seq_lens_t, self.scale,
                                nsplit=md.nsplit, scratch=md.decode_scratch,
-                               window=cfg.sliding_window)
+                               window=cfg.sliding_window,
+                               cut=md.decode_cut)
 
     def forward(self, x, positions, rope_tab, kv: KVCache, md: AttnMetadata):
         qkv = ops.linear(x, self.qkv)
@@ -459,14 +463,28 @@ class LlamaForCausalLM(nn.Module):
                 and self.embed.dtype == torch.bfloat16
                 and self.embed.shape[1] == cfg.hidden_size)
 
+    def _with_cut(self, kv: KVCache, md: AttnMetadata) -> AttnMetadata:
+        """md with the cut of this step's attention, to be made by the embedding.
+        The caller's md stays as it is: the next step has other lengths."""
+        cut, cfg = None, self.cfg
+        if not md.is_prefill and md.nsplit > 1:
+            cut = ops.decode_cut(md.seq_lens_t, kv.k[0].shape[1],
+                                 cfg.num_heads // cfg.num_kv_heads, md.nsplit,
+                                 cfg.sliding_window, fill=False)
+        if cut is not md.decode_cut:
+            md = copy.copy(md)
+            md.decode_cut = cut
+        return md
+
     def forward(self, ids, positions, kv: KVCache, md: AttnMetadata,
                 logit_rows: torch.Tensor | None = None):
         """ids/positions [T] -> logits [T or len(logit_rows), vocab]."""
         T = ids.numel()
+        md = self._with_cut(kv, md)
         if ids.is_cuda and self._can_fuse_rows(T):
             ss = (torch.empty(T, 8, dtype=torch.float32, device=ids.device)
                   if T > ops.ROWS_MAX else None)
-            residual = ops.embedding(ids, self.embed, ss=ss)
+            residual = ops.embedding(ids, self.embed, ss=ss, cut=md.decode_cut)
             pos = ops.qkv_step(T, self.cfg.head_dim, positions, self.rope_tab,
                                md.slots)
             for layer in self.layers:
@@ -483,7 +501,7 @@ class LlamaForCausalLM(nn.Module):
             if logit_rows is not None:
                 residual, ss = ops.gather_rows(residual, logit_rows), None
             return self._logits_rows_fused(residual, ss)
-        h = ops.embedding(ids, self.embed)
+        h = ops.embedding(ids, self.embed, cut=md.decode_cut)
         residual = None
         for layer in self.layers:
             h, residual = layer(h, residual, positions, self.rope_tab, kv, md)

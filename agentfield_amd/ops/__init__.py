@@ -136,7 +136,10 @@ def reshape_and_cache(k: torch.Tensor, v: torch.Tensor, kcache: torch.Tensor,
 
 
 def embedding(ids: torch.Tensor, table: torch.Tensor,
-              ss: torch.Tensor | None = None) -> torch.Tensor:
+              ss: torch.Tensor | None = None,
+              cut: "DecodeCut | None" = None) -> torch.Tensor:
+    """table[ids]; ss [T, 8] gets the rows' sums of squares, and cut, a decode
+    step's (decode_cut with fill=False), is made in the same launch."""
     if not _on_gpu(table):
         out = table[ids.long()]
         if ss is not None:
@@ -148,6 +151,7 @@ def embedding(ids: torch.Tensor, table: torch.Tensor,
     out = torch.empty(T, H, dtype=table.dtype, device=table.device)
     rc = _lib.lib().af_embedding(_lib.ptr(out), _lib.ptr(table),
                                  _lib.ptr(ids.int()), _lib.ptr(ss), T, H,
+                                 *(cut.args() if cut else (None, None, 0, 0)),
                                  _lib.cur_stream())
     _lib.check(rc, "af_embedding")
     return out
@@ -159,10 +163,17 @@ def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
                 scale: float | None = None, nsplit: int = 1,
                 scratch: tuple[torch.Tensor, torch.Tensor] | None = None,
                 out: torch.Tensor | None = None,
-                window: int = 0) -> torch.Tensor:
+                window: int = 0,
+                cut: "DecodeCut | None" = None) -> torch.Tensor:
     """Paged decode attention. q [B, Hq*D] (strided rows ok) -> out [B, Hq*D].
     window > 0: sliding-window (Mistral) — only the last `window` cached
-    tokens are attended."""
+    tokens are attended.
+
+    cut: how the step's sequences are cut (decode_cut).  Without one a sequence
+    is summed in nsplit parts of its own, whatever is beside it.  With one,
+    lengths unlike enough are cut in equal shares of all tokens: where a sequence
+    is cut, and so the order of its fp32 sums and its last bit in bf16, then
+    depends on the lengths beside it."""
     _, Hk, page, D = kcache.shape
     B = q.shape[0]
     Hq = q.shape[1] // D
@@ -177,23 +188,68 @@ def attn_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
     G = Hq // Hk
     po = pml = None
     cap = 0
+    if cut is not None:
+        _need(cut.B == B and cut.nsplit == nsplit and cut.data.device == q.device,
+              f"decode attention: {B} sequences in {nsplit} parts, cut as {cut.B} in "
+              f"{cut.nsplit}")
     if nsplit > 1:
-        po, pml = decode_scratch(B, Hk, nsplit, G, q.device) if scratch is None else scratch
+        if scratch is None:
+            scratch = decode_scratch(B, Hk, nsplit, G, q.device, shares=cut is not None)
+        po, pml = scratch
         cap = min(po.numel() // (Hk * G * D), pml.numel() // (Hk * G * 2))
     rc = _lib.lib().af_attn_decode(
         _lib.ptr(out), _lib.ptr(po), _lib.ptr(pml), _lib.ptr(q),
         _lib.ptr(kcache), _lib.ptr(vcache), _lib.ptr(block_table),
-        _lib.ptr(seq_lens), scale, B, Hq, Hk, D, page, block_table.shape[1],
-        nsplit, cap, q.stride(0), window, _lib.cur_stream())
+        _lib.ptr(seq_lens), _lib.ptr(cut.data if cut else None), scale, B, Hq, Hk, D,
+        page, block_table.shape[1], nsplit, cap, q.stride(0), window,
+        _lib.cur_stream())
     _lib.check(rc, "af_attn_decode")
     return out
 
 
-def decode_scratch(B: int, Hk: int, nsplit: int, G: int, device, D: int = 128):
-    """Scratch of attn_decode: room for nsplit parts of every sequence, and for one more
-    each, with which unlike lengths can be cut evenly."""
-    return tuple(torch.empty(B, Hk, nsplit + 1, G, n, dtype=torch.float32, device=device)
-                 for n in (D, 2))
+def decode_shares(B: int, Hk: int, G: int, nsplit: int, window: int = 0) -> bool:
+    """Whether a decode step's sequences may be cut in equal shares: a lane per
+    sequence, and room for all blocks at once, or the dispatch evens them out.
+    Beyond four parts a sequence is short, or the step is small.  Long sequences
+    behind a window are of one length."""
+    return (2 <= nsplit <= 4 and 2 <= B <= 64 and window <= 0
+            and B * Hk * nsplit <= 256 * (2 if G == 8 else 3))
+
+
+def decode_scratch(B: int, Hk: int, nsplit: int, G: int, device, D: int = 128,
+                   shares: bool = False):
+    """Scratch of attn_decode: room for nsplit parts of every sequence, and with
+    shares (decode_shares) for one more each."""
+    return tuple(torch.empty(B, Hk, nsplit + shares, G, n, dtype=torch.float32,
+                             device=device) for n in (D, 2))
+
+
+class DecodeCut:
+    """How the sequences of one decode step are cut, for attn_decode in each of its
+    layers: made from the lengths on the device, once a step."""
+
+    def __init__(self, seq_lens: torch.Tensor, nsplit: int):
+        self.seq_lens, self.B, self.nsplit = seq_lens, seq_lens.numel(), nsplit
+        self.data = torch.empty(self.B, 4, dtype=torch.int32, device=seq_lens.device)
+
+    def args(self):
+        return (_lib.ptr(self.data), _lib.ptr(self.seq_lens), self.B, self.nsplit)
+
+
+def decode_cut(seq_lens: torch.Tensor, Hk: int, G: int, nsplit: int,
+               window: int = 0, fill: bool = True) -> DecodeCut | None:
+    """The cut of a step of sequences of seq_lens [B] tokens, None where it would
+    stay with nsplit parts of each anyway.  fill=False leaves it to be made by
+    `embedding`."""
+    if not (seq_lens.is_cuda and seq_lens.dtype is torch.int32
+            and seq_lens.is_contiguous()
+            and decode_shares(seq_lens.numel(), Hk, G, nsplit, window)):
+        return None
+    cut = DecodeCut(seq_lens, nsplit)
+    if fill:
+        rc = _lib.lib().af_decode_cut(*cut.args(), _lib.cur_stream())
+        _lib.check(rc, "af_decode_cut")
+    return cut
 
 
 def prefill_split(seq_lens: list[int], G: int, Hk: int, max_keys: int):

@@ -47,9 +47,10 @@ def _declare(l: ctypes.CDLL) -> None:
     l.af_silu_mul.argtypes = [p, p, p, f, f, i64, i64, p]
     l.af_add.argtypes = [p, p, p, i64, p]
     l.af_reshape_and_cache.argtypes = [p, p, p, p, p, i, i, i, i, p]
-    l.af_embedding.argtypes = [p, p, p, p, i, i, p]
-    l.af_attn_decode.argtypes = [p, p, p, p, p, p, p, p, f, i, i, i, i, i, i, i, i,
-                                 i64, i, p]
+    l.af_embedding.argtypes = [p, p, p, p, i, i, p, p, i, i, p]
+    l.af_attn_decode.argtypes = [p, p, p, p, p, p, p, p, p, f, i, i, i, i, i, i, i,
+                                 i, i64, i, p]
+    l.af_decode_cut.argtypes = [p, p, i, i, p]
     l.af_attn_prefill.argtypes = [p, p, p, p, p, p, p, p, p, f, i, i, i, i, i,
                                   i, i, i, i64, i, i, i, p]
     l.af_gemm_bf16.argtypes = [p, p, p, i, i, i, p]
@@ -86,7 +87,7 @@ def _declare(l: ctypes.CDLL) -> None:
     l.af_axpy.argtypes = [p, p, f, i, p]
     l.af_device_sync.argtypes = []
     for fn in ("af_rmsnorm", "af_rope_cache", "af_silu_mul", "af_add",
-               "af_reshape_and_cache", "af_embedding", "af_attn_decode",
+               "af_reshape_and_cache", "af_embedding", "af_attn_decode", "af_decode_cut",
                "af_attn_prefill", "af_gemm_bf16", "af_gemm_bf16_ring", "af_gemm_bf16_q8", "af_gemm_mxfp8", "af_oneshot_allreduce",
                "af_gemm_skinny", "af_rows_linear", "af_rows_group", "af_rows_qkv",
                "af_moe_route", "af_moe_combine", "af_moe_gemm", "af_gemm_wide",

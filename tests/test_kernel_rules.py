@@ -358,3 +358,18 @@ def test_wide_split_without_room_for_its_parts(monkeypatch):
     monkeypatch.setattr(ops, "launch_wide_split", full)
     x, w = (Operand(**vars(mat(n, 14336))) for n in (300, 4096))
     assert ops.linear(x, w) == "torch"
+
+
+@pytest.mark.parametrize("B,Hk,G,nsplit,window,shares", [
+    (24, 8, 4, 2, 0, True), (48, 8, 4, 2, 0, True), (49, 8, 4, 2, 0, False),
+    (32, 8, 8, 2, 0, True), (33, 8, 8, 2, 0, False), (64, 1, 4, 4, 0, True),
+    (65, 1, 4, 2, 0, False), (1, 8, 4, 4, 0, False), (2, 8, 4, 1, 0, False),
+    (9, 8, 4, 5, 0, False), (24, 8, 4, 2, 4096, False)])
+def test_decode_steps_that_may_be_cut_in_shares(B, Hk, G, nsplit, window, shares):
+    """Room for all blocks at once, a lane per sequence, two to four parts, no window; the
+    scratch has room for one piece more of each sequence there, and only there."""
+    assert ops.decode_shares(B, Hk, G, nsplit, window) == shares
+    po, pml = ops.decode_scratch(B, Hk, nsplit, G, "cpu", shares=shares)
+    assert po.shape == (B, Hk, nsplit + shares, G, 128)
+    assert pml.shape == (B, Hk, nsplit + shares, G, 2)
+    assert ops.decode_cut(torch.ones(B, dtype=torch.int32), Hk, G, nsplit, window) is None

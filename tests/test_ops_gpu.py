@@ -489,6 +489,32 @@ def test_embedding_and_gather():
     assert close(g, out.cpu()[rows.cpu().long()], atol=0)
 
 
+@pytest.mark.parametrize("nsplit", [2, 3, 4])
+@pytest.mark.parametrize("lens", [
+    [7, 4000], [0, 0], [64] * 9, [0, 3000, 0, 65, 64, 1], [1600, 1500, 1400],
+    list(range(0, 64 * 90, 90)), [2900 if i == 40 else 7 * i for i in range(64)]])
+def test_embedding_makes_the_cut(nsplit, lens):
+    """The step's cut beside the rows of the embedding and on its own: for every sequence the
+    rounds of 64 tokens of a share, where the largest of nsplit parts has four more than
+    that, its tokens, the rounds of one of its parts, and those up to its end."""
+    tab, B = rnd(64, 256, seed=3), len(lens)
+    ids = torch.randint(0, 64, (B,), dtype=torch.int32, device=DEV)
+    L = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    rounds = [-(-n // 64) for n in lens]
+    total, slots = sum(rounds), B * nsplit
+    share = -(-total // slots) if max(rounds) / nsplit > total / slots + 4 else 0
+    want = [[share, lens[i], -(-rounds[i] // nsplit), sum(rounds[:i + 1])] for i in range(B)]
+    assert ops.decode_cut(L, 1, 4, nsplit).data.tolist() == want
+    ss = torch.full((B, 8), -1.0, device=DEV)
+    for stats in (None, ss):
+        cut = ops.decode_cut(L, 1, 4, nsplit, fill=False)
+        cut.data.fill_(-1)
+        assert torch.equal(ops.embedding(ids, tab, ss=stats, cut=cut), tab[ids.long()])
+        assert cut.data.tolist() == want
+    sq = tab[ids.long()].double().pow(2).sum(1)
+    assert ((ss.double().sum(1) - sq).abs() <= 2 ** -18 * sq).all()
+
+
 def test_sample_topk_topp():
     torch.manual_seed(7)
     B, V = 4, 50000
@@ -726,21 +752,28 @@ def test_attn_decode_merges_splits(nsplit):
     assert close(got, want, atol=2 ** -7, rtol=2 ** -8)
 
 
-@pytest.mark.parametrize("G,page,nsplit,lens", [
-    (4, 64, 2, [6000, 1, 700, 64, 65]),            # through three sequences and more
-    (4, 64, 2, [0, 3000, 0, 0, 2, 1100, 0]),       # empty ones first, between and last
-    (1, 16, 3, [5, 4096, 17, 2048]),               # shares that end with a sequence
-    (2, 64, 4, [9000, 300, 300]),
-    (8, 24, 2, [2500, 100, 33]),                   # tiles over two pages
-    (8, 64, 4, [64 * 150, 1, 1, 1, 1, 1]),
-    (4, 32, 2, [2900 if i == 40 else 7 * i for i in range(64)]),   # a lane each
-    (4, 32, 2, [2900 if i == 40 else 7 * i for i in range(65)]),   # one too many
-    (4, 64, 2, [1600, 1500, 1400])])               # alike: nsplit parts each
-def test_attn_decode_shares(G, page, nsplit, lens):
+@pytest.mark.parametrize("Hk,G,page,nsplit,lens", [
+    (2, 4, 64, 2, [6000, 1, 700, 64, 65]),            # through three sequences and more
+    (8, 4, 64, 2, [6000, 1, 700, 64, 65]),            # heads first in the grid
+    (2, 4, 64, 2, [0, 3000, 0, 0, 2, 1100, 0]),       # empty ones first, between and last
+    (8, 4, 64, 4, [0, 3000, 0, 0, 2, 1100, 0]),
+    (2, 1, 16, 3, [5, 4096, 17, 2048]),               # shares that end with a sequence
+    (32, 1, 64, 3, [5, 4096, 17]),
+    (2, 2, 64, 4, [9000, 300, 300]),
+    (2, 8, 24, 2, [2500, 100, 33]),                   # tiles over two pages
+    (8, 8, 24, 2, [2500, 100, 33]),
+    (2, 8, 64, 4, [64 * 150, 1, 1, 1, 1, 1]),
+    (2, 4, 32, 2, [2900 if i == 40 else 7 * i for i in range(64)]),   # a lane each
+    (2, 4, 32, 2, [2900 if i == 40 else 7 * i for i in range(65)]),   # one too many
+    (8, 4, 64, 4, [800 + 17 * i for i in range(12)]),  # alike: nsplit parts each, of several
+    (2, 4, 64, 4, [1500, 1601, 1700]),                 # rounds and uneven remainders
+    (8, 2, 64, 3, [1600, 1500, 1400])])
+def test_attn_decode_shares(Hk, G, page, nsplit, lens):
     """Sequences of unlike lengths, cut in equal shares of all their tokens; replayed with
-    other lengths, and with scratch for nsplit parts of each only.  What is not visible is
-    NaN in the values.  Tolerance: bf16 rounding of outputs below 4 (2^-9 * 4)."""
-    D, Hk, B = 128, 2, len(lens)
+    other lengths, with scratch for nsplit parts of each only, and without a cut.  What is
+    not visible is NaN in the values.  Tolerance: bf16 rounding of outputs below 4 (2^-9 *
+    4)."""
+    D, B = 128, len(lens)
     torch.manual_seed(len(lens) + G)
     maxp = -(-max(lens) // page)
     bt = (torch.randperm(B * maxp) + 1).view(B, maxp).to(torch.int32)
@@ -767,19 +800,103 @@ def test_attn_decode_shares(G, page, nsplit, lens):
         assert all((got[b] == 0).all() for b in range(B) if not lens[b])
 
     vd, L = values(lens).to(DEV), torch.tensor(lens, dtype=torch.int32, device=DEV)
-    check(ops.attn_decode(qd, kd, vd, btd, L, nsplit=nsplit), lens)
+
+    def attn(scratch=None):
+        cut = ops.decode_cut(L, Hk, G, nsplit)
+        assert (cut is not None) == (B <= 64)
+        return ops.attn_decode(qd, kd, vd, btd, L, nsplit=nsplit, scratch=scratch, cut=cut)
+    check(attn(), lens)
+    plain = ops.attn_decode(qd, kd, vd, btd, L, nsplit=nsplit)
+    check(plain, lens)
     scratch = tuple(torch.full((B, Hk, nsplit, G, n), torch.nan, device=DEV) for n in (D, 2))
-    check(ops.attn_decode(qd, kd, vd, btd, L, nsplit=nsplit, scratch=scratch), lens)
+    assert torch.equal(attn(scratch), plain)
     # (torch's own state of captures is an inference tensor once one was made in that mode)
     with torch.inference_mode():
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph):
-            out = ops.attn_decode(qd, kd, vd, btd, L, nsplit=nsplit)
+            out = attn()
         for turned in (lens[::-1], [min(n, 90) for n in lens], lens):
             vd.copy_(values(turned))
             L.copy_(torch.tensor(turned, dtype=torch.int32))
             graph.replay()
             check(out, turned)
+
+
+@pytest.mark.parametrize("Hk,G,nsplit,mine", [(8, 4, 2, 700), (2, 4, 4, 2000),
+                                              (8, 8, 4, 130), (2, 1, 3, 4096)])
+def test_attn_decode_beside_other_lengths(Hk, G, nsplit, mine):
+    """What a sequence's result has of the lengths beside it: nothing without a cut, the
+    order of its fp32 sums with one.  These differ by 1e-5 of the outputs, which are below
+    4: at most two neighbouring bf16 values (2^-7 of the larger)."""
+    D, page, B, top = 128, 64, 5, 6000
+    torch.manual_seed(mine)
+    maxp = -(-top // page)
+    bt = (torch.randperm(B * maxp) + 1).view(B, maxp).int().to(DEV)
+    kc, vc = (torch.randn(B * maxp + 1, Hk, page, D).bfloat16().to(DEV) for _ in range(2))
+    q = torch.randn(B, Hk * G * D).bfloat16().to(DEV)
+    rows = {False: [], True: []}
+    for other in ([700, 650, 800, 600], [6000, 1, 1, 1], [64, 3000, 0, 5], [1, 1, 1, 6000]):
+        L = torch.tensor(other[:2] + [mine] + other[2:], dtype=torch.int32, device=DEV)
+        for shares in rows:
+            cut = ops.decode_cut(L, Hk, G, nsplit) if shares else None
+            rows[shares].append(ops.attn_decode(q, kc, vc, bt, L, nsplit=nsplit,
+                                                cut=cut)[2].float())
+    for a in rows[False]:
+        assert torch.equal(a, rows[False][0])
+    for a in rows[True]:
+        d = (a - rows[False][0]).abs()
+        assert (d <= 2 ** -7 * torch.maximum(a.abs(), rows[False][0].abs()) + 4e-5).all()
+
+
+def test_attn_decode_refuses_another_steps_cut():
+    """A cut made for other parts or another number of sequences would leave tokens out."""
+    kc = torch.zeros(4, 2, 16, 128, dtype=torch.bfloat16, device=DEV)
+    q = torch.zeros(3, 8 * 128, dtype=torch.bfloat16, device=DEV)
+    bt = torch.zeros(3, 1, dtype=torch.int32, device=DEV)
+    L = torch.tensor([5, 6, 7], dtype=torch.int32, device=DEV)
+    for cut in (ops.decode_cut(L, 2, 4, 4), ops.decode_cut(L[:2], 2, 4, 2)):
+        with pytest.raises(ops.AfOpsError):
+            ops.attn_decode(q, kc, kc, bt, L, nsplit=2, cut=cut)
+
+
+@pytest.mark.parametrize("fused", [True, False])
+def test_decode_steps_with_a_cut(fused):
+    """A captured decode step of unlike lengths, whose embedding cuts them anew at each
+    replay, against the unsplit step: 1% of the logits' norm, as both are bf16 roundings of
+    the same two layers.  The caller's metadata is left as it was."""
+    from agentfield_amd.models.llama import (AttnMetadata, KVCache, LlamaConfig,
+                                             LlamaForCausalLM)
+    cfg = LlamaConfig(hidden_size=512, intermediate_size=256, num_layers=2, num_heads=16,
+                      num_kv_heads=8, vocab_size=512, max_position=4096)
+    page, top = 64, 3000
+    m = LlamaForCausalLM(cfg, device=DEV).init_random(5).fold_norm_weights()
+    m.no_fused_decode = not fused
+    B, maxp = 4, -(-top // page)
+    bt = torch.arange(1, B * maxp + 1, device=DEV, dtype=torch.int32).view(B, maxp)
+    kv = KVCache(cfg, B * maxp + 1, page, DEV)
+    for t in (*kv.k, *kv.v):
+        t.normal_(generator=torch.Generator(device=DEV).manual_seed(1))
+    ids = torch.randint(0, 512, (B,), device=DEV, dtype=torch.int32)
+    L = torch.tensor([700, 3000, 1, 64], device=DEV, dtype=torch.int32)
+    pos, slots = L - 1, torch.zeros(B, device=DEV, dtype=torch.int64)
+
+    def step(nsplit):
+        md = AttnMetadata(is_prefill=False, slots=slots, block_table=bt, seq_lens_t=L,
+                          nsplit=nsplit)
+        logits = m(ids, pos, kv, md)
+        assert md.decode_cut is None
+        return logits.float()
+    with torch.inference_mode():
+        step(4)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got = step(4)
+        for lens in ([700, 3000, 1, 64], [1, 2, 3000, 2999], [900, 950, 1000, 980]):
+            L.copy_(torch.tensor(lens))
+            pos.copy_(L - 1)
+            graph.replay()
+            want = step(1)
+            assert (got - want).norm() <= 1e-2 * want.norm()
 
 
 @pytest.mark.parametrize("Hk,nsplit", [(3, 1), (4, 1), (4, 2), (8, 1), (8, 3), (11, 2)])
