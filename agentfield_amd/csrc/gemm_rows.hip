@@ -722,11 +722,17 @@ static bool streamed(const RowsArgs& a) { return (i64)a.N * a.K >= (8 << 20); }
 // and 16: 384 / 256, K 4096 11.1 / 10.7 and 13.3 / 11.0, K 8192 19.2 / 18.1 and 23.9 / 18.2;
 // 264 / 176, K 4096 10.3 / 8.6 and 12.6 / 10.1; 768 / 512 18.0 / 17.8 and 20.2 / 18.4, K 2048
 // 12.0 / 10.3 and 12.9 / 11.0; K 1024 level.  Not where 16 rows fill their rounds as well: 240
-// / 160 7.7 / 8.3, 480 / 320 12.4 / 14.8, 960 / 640 21.7 / 22.1.  Longer rings (three and four
-// pieces) and, to 8 rows, 8 rows of X instead of 16 change nothing.
+// / 160 7.7 / 8.3, 480 / 320 12.4 / 14.8, 960 / 640 21.7 / 22.1.  Nor where the second round
+// of 24 is half empty and K long, one rule for all M, so that results do not depend on it: 1,
+// 4, 8 and 16 rows, 528 / 352, K 5120 19.0 18.9 19.9 23.1 / 19.7 18.7 19.3 21.4; 576 / 384 19.7
+// 19.8 21.0 23.6 / 20.0 20.5 21.6 21.9, K 6144 22.2 22.3 23.6 26.7 / 22.8 23.4 24.7 24.8; but
+// K 3584 0.91 to 0.99 of the time at 352 to 384, K 4096 0.92 to 1.03, and from 416 tiles of 24
+// on 0.90 to 0.99 at every K and M.  Longer rings (three and four pieces) and, to 8 rows, 8 rows
+// of X instead of 16 change nothing.
 static bool in_24s(const RowsArgs& a) {
-  const int g = a.N / 16, rounds = (a.N / 24 + ROWS_CUS - 1) / ROWS_CUS;
-  return a.N % 24 == 0 && g > rounds * ROWS_CUS && rounds <= 2;
+  const int g = a.N / 16, g24 = a.N / 24, rounds = (g24 + ROWS_CUS - 1) / ROWS_CUS;
+  return a.N % 24 == 0 && g > rounds * ROWS_CUS && rounds <= 2 &&
+         (rounds == 1 || a.K < 4096 || g24 > 400);
 }
 
 template <int EPI, int NORM>

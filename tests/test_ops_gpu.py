@@ -1212,6 +1212,26 @@ def test_qkv_rope_rows_in_tiles_of_24(M, Hq, Hk, K):
     test_qkv_rope_rows(M, Hq, Hk, K)
 
 
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("heads,K,same", [(66, 4096, True), (75, 5120, True),
+                                          (66, 4032, False), (78, 5120, False)])
+def test_qkv_rope_rows_where_tiles_of_24_do_not_pay(M, heads, K, same):
+    """With a half-empty second round of long tiles, 16 weight rows again: the bits of a
+    projection of the first heads only, whose tiles of 16 start in the same pieces.  In 24s
+    they start elsewhere, and bits differ where products cancel up to their rounding."""
+    D, page = 128, 16
+    x, w = rnd(M, K // 2, seed=M), rnd(heads * D, K // 2, seed=heads)
+    x, w = torch.cat([x, x], 1), torch.cat([w, -w], 1)
+    tab = ops.rope_table(64, D, device=DEV)
+    pos, slots = torch.arange(M, device=DEV).int(), torch.arange(M, device=DEV)
+
+    def q_of(w):
+        kc, vc = (torch.zeros(2, 1, page, D, dtype=torch.bfloat16, device=DEV)
+                  for _ in range(2))
+        return ops.qkv_rope_rows(x, w, 1e-5, None, pos, tab, kc, vc, slots)[:, :30 * D]
+    assert torch.equal(q_of(w), q_of(w[:32 * D].contiguous())) == same
+
+
 @pytest.mark.parametrize("M", [17, 33, 65])
 @pytest.mark.parametrize("N,K", [
     (512, 256), (1024, 256),       # one tile of 64, or of 128 above 64 rows, per XCD; two
