@@ -2,6 +2,10 @@
 take.  The rules are about sizes, types and addresses, so they are checked here
 on stand-ins, without a GPU: whatever the row GEMMs take, for instance, is read by
 kernels that know only x's sizes and the number of weight rows."""
+import ctypes
+import re
+from collections import defaultdict
+from pathlib import Path
 from types import SimpleNamespace
 
 import pytest
@@ -373,3 +377,52 @@ def test_decode_steps_that_may_be_cut_in_shares(B, Hk, G, nsplit, window, shares
     assert po.shape == (B, Hk, nsplit + shares, G, 128)
     assert pml.shape == (B, Hk, nsplit + shares, G, 2)
     assert ops.decode_cut(torch.ones(B, dtype=torch.int32), Hk, G, nsplit, window) is None
+
+
+ROOT = Path(__file__).resolve().parent.parent
+
+
+def prototypes(text, mark):
+    """{name: kinds of its arguments} of the C entry points that are declared or defined
+    behind mark."""
+    kinds = {"int": "i", "long": "l", "i64": "l", "int64_t": "l", "float": "f", "u32": "u", "uint32_t": "u",
+             "unsigned long long": "q", "uint64_t": "q"}
+    out = {}
+    for name, args in re.findall(mark + r"int (af_\w+)\(([^)]*)\)", text):
+        args = [a.replace("const", " ").strip() for a in args.split(",")]
+        out[name] = "".join(
+            "" if a in ("", "void") else "p" if "*" in a
+            else kinds[" ".join(a.split()[:-1]) or a] for a in args)
+    return out
+
+
+def defined():
+    text = "".join(f.read_text() for f in (ROOT / "agentfield_amd" / "csrc").glob("*.hip"))
+    return prototypes(text, "AF_EXPORT ")
+
+
+@pytest.mark.parametrize("path", sorted((ROOT / "tools").glob("*.cpp")), ids=lambda p: p.name)
+def test_tools_call_the_kernels_as_they_are(path):
+    """A declaration of other arguments links all the same, and passes sizes for streams."""
+    want, got = defined(), prototypes(path.read_text(), r"(?m)^")
+    assert got and {n: want[n] for n in got} == got
+
+
+def test_bindings_call_the_kernels_as_they_are():
+    """The loader's argument types against the entry points' own."""
+    from agentfield_amd.ops import _lib
+    fake = defaultdict(SimpleNamespace)
+
+    class Library:
+        def __getattr__(self, name):
+            return fake[name]
+    _lib._declare(Library())
+    kinds = {ctypes.c_void_p: "p", ctypes.c_int: "i", ctypes.c_int64: "l",
+             ctypes.c_float: "f", ctypes.c_uint32: "u"}
+    want = defined()
+    got = {n: "".join(kinds.get(t, "?") for t in f.argtypes) for n, f in fake.items()
+           if hasattr(f, "argtypes")}
+    assert len(got) > 30
+    for name, args in got.items():
+        if "?" not in args:
+            assert args == want[name], name

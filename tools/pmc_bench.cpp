@@ -12,21 +12,28 @@
 #include <vector>
 
 extern "C" {
-int af_attn_prefill(void*, const void*, const void*, const void*, const void*,
-                    const void*, const void*, const void*, const void*, float,
-                    int, int, int, int, long, int, int, void*);
-int af_attn_decode(void*, void*, void*, const void*, const void*, const void*,
-                   const void*, const void*, float, int, int, int, int, int,
-                   int, int, long, void*);
-int af_gemm_skinny(void*, void*, void*, const void*, const void*, int, int,
-                   int, int, int, const void*, float, void*, void*);
-int af_gemm_bf16(void*, const void*, const void*, int, int, int, void*);
-int af_rmsnorm(void*, void*, const void*, const void*, const void*, float,
-               int, int, void*);
+int af_attn_prefill(void* out, void* po, void* pml, const void* q, const void* kc,
+                    const void* vc, const void* bt, const void* qstart,
+                    const void* cu_seqlens, float scale, int nseq, int items, int few,
+                    int few_cols, int nsplit, int Hq, int Hk, int D, long qs,
+                    int page_size, int max_pages, int win, void* stream);
+int af_attn_decode(void* out, void* po, void* pml, const void* q, const void* kc,
+                   const void* vc, const void* bt, const void* len, const void* cut,
+                   float scale, int B, int Hq, int Hk, int D, int page_size,
+                   int max_pages, int nsplit, int cap, long qs, int win, void* stream);
+int af_gemm_skinny(void* out, void* partial, void* residual, const void* X,
+                   const void* W, int M, int N, int K, int SK, int mode,
+                   const void* scale_ss, float eps, void* ss_out, void* stream);
+int af_gemm_bf16(void* C, const void* A, const void* W, int M, int N, int K,
+                 void* stream);
+int af_rmsnorm(void* out, void* res_out, const void* x, const void* res, const void* w,
+               float eps, int T, int H, void* stream);
 }
 
 #define CK(x) do { hipError_t e = (x); if (e != hipSuccess) { \
   fprintf(stderr, "HIP error %d at line %d\n", e, __LINE__); exit(1); } } while (0)
+#define AF(x) do { int rc = (x); if (rc != 0) { \
+  fprintf(stderr, "kernel refused: %d at line %d\n", rc, __LINE__); exit(1); } } while (0)
 
 static void* dz(size_t bytes) {
   void* p = nullptr;
@@ -54,17 +61,15 @@ int main() {
     void* kc = dz((size_t)npages * Hk * page * D * 2);
     void* vc = dz((size_t)npages * Hk * page * D * 2);
     void* out = dz((size_t)T * Hq * D * 2);
-    std::vector<int> bt(B * maxp), cu(B + 1), qs(B, 0), ts, tq;
+    std::vector<int> bt(B * maxp), cu(B + 1), qs(B, 0);
     for (int i = 0; i < B * maxp; ++i) bt[i] = 1 + i;
     for (int i = 0; i <= B; ++i) cu[i] = i * S;
-    for (int b = 0; b < B; ++b)
-      for (int q0 = 0; q0 < S; q0 += 16) { ts.push_back(b); tq.push_back(q0); }
-    void *d_bt = d_i32(bt), *d_cu = d_i32(cu), *d_qs = d_i32(qs),
-         *d_ts = d_i32(ts), *d_tq = d_i32(tq);
+    void *d_bt = d_i32(bt), *d_cu = d_i32(cu), *d_qs = d_i32(qs);
+    // items of 128 columns, a column per row and query head of a K/V head
+    const int items = B * (S * (Hq / Hk) / 128);
     for (int it = 0; it < 3; ++it)
-      af_attn_prefill(out, q, kc, vc, d_bt, d_qs, d_cu, d_ts, d_tq,
-                      0.0883f, (int)ts.size(), Hq, Hk, D, (long)Hq * D, page,
-                      maxp, s);
+      AF(af_attn_prefill(out, nullptr, nullptr, q, kc, vc, d_bt, d_qs, d_cu, 0.0883f, B,
+                         items, 0, 32, 1, Hq, Hk, D, (long)Hq * D, page, maxp, 0, s));
     CK(hipDeviceSynchronize());
     printf("prefill ok\n");
   }
@@ -77,8 +82,8 @@ int main() {
     void* out = dz((size_t)M * N * 2);
     void* part = dz((size_t)SK * M * N * 4);
     for (int it = 0; it < 3; ++it)
-      af_gemm_skinny(out, part, nullptr, x, w, M, N, K, SK, 0, nullptr, 0.f,
-                     nullptr, s);
+      AF(af_gemm_skinny(out, part, nullptr, x, w, M, N, K, SK, 0, nullptr, 0.f,
+                        nullptr, s));
     CK(hipDeviceSynchronize());
     printf("skinny ok\n");
   }
@@ -97,8 +102,8 @@ int main() {
     for (int i = 0; i < B * maxp; ++i) bt[i] = 1 + i;
     void *d_bt = d_i32(bt), *d_len = d_i32(len);
     for (int it = 0; it < 3; ++it)
-      af_attn_decode(out, po, pml, q, kc, vc, d_bt, d_len, 0.0883f, B, Hq, Hk,
-                     D, page, maxp, ns, (long)Hq * D, s);
+      AF(af_attn_decode(out, po, pml, q, kc, vc, d_bt, d_len, nullptr, 0.0883f, B, Hq,
+                        Hk, D, page, maxp, ns, B * ns, (long)Hq * D, 0, s));
     CK(hipDeviceSynchronize());
     printf("decode ok\n");
   }
@@ -109,7 +114,7 @@ int main() {
     void* a = dz((size_t)N * N * 2);
     void* w = dz((size_t)N * N * 2);
     void* c = dz((size_t)N * N * 2);
-    for (int it = 0; it < 3; ++it) af_gemm_bf16(c, a, w, N, N, N, s);
+    for (int it = 0; it < 3; ++it) AF(af_gemm_bf16(c, a, w, N, N, N, s));
     CK(hipDeviceSynchronize());
     printf("gemm ok\n");
   }
@@ -122,7 +127,7 @@ int main() {
     void* w = dz((size_t)H * 2);
     void* out = dz((size_t)T * H * 2);
     for (int it = 0; it < 3; ++it)
-      af_rmsnorm(out, res, x, res, w, 1e-5f, T, H, s);
+      AF(af_rmsnorm(out, res, x, res, w, 1e-5f, T, H, s));
     CK(hipDeviceSynchronize());
     printf("rmsnorm ok\n");
   }
