@@ -1236,11 +1236,16 @@ def test_qkv_rope_rows_where_tiles_of_24_do_not_pay(M, heads, K, same):
 @pytest.mark.parametrize("N,K", [
     (512, 256), (1024, 256),       # one tile of 64, or of 128 above 64 rows, per XCD; two
     (576, 128), (1152, 256),       # no multiple of 8 tiles: neighbours
-    (4096, 3072), (8192, 1024),    # tiles of 128 from 33 rows on; several turns of a block
+    (4096, 3072), (8192, 1024),    # several turns of a block
+    (4096, 11008), (8192, 3072),   # tiles of 128 from 33 rows on, in 8 and 4 splits
 ])
 def test_parts_meet_by_tiles(M, N, K):
     """Every column once, whatever the tiles that an XCD adds up, and the rows' sums of
     squares whole.  Tolerance: one bf16 rounding, and fp32 sums in another order."""
+    splits = ops.rows_splits(M, N, K)
+    if K in (11008, 3072) and M == 33:
+        in_128s = splits > 1 and N // 128 * splits >= 192 and K // 64 >= 12 * splits
+        assert in_128s == ((N, K) != (4096, 3072))
     x, w = rnd(M, K, seed=M), rnd(N, K, seed=N, scale=1.0 / math.sqrt(K))
     res, st = rnd(M, N, seed=5), torch.full((M, 8), -1.0, device=DEV)
     want = res.float() + x.float() @ w.float().t()
