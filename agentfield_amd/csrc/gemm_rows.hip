@@ -612,11 +612,15 @@ __global__ void __launch_bounds__(64 * NW) gemm_tile_kernel(RowsArgs a) {
 
 // What adds the parts runs an eighth of the columns on each XCD (blockIdx.x): the tiles of
 // the products that wrote them there, every eighth, all splits of which are on one XCD where
-// the tiles are a multiple of 8.  With rows on the XCDs instead (row modulo 8, or any) the
-// products that write the same parts next were slower, 17.2 -> 16.9 us in the mean at 80 rows
-// and 17.4 -> 16.8 at 45, the launches themselves the same.  Steps of 16 layers: 16 x 5 rows
-// behind a history 2581 -> 2540 us, a prompt of 45 1794 -> 1764, 128 rows 3014 -> 2996; 64
-// rows level.
+// the tiles are a multiple of 8.  The rotary launch walks heads, tiles of 128 columns; of
+// tiles of 64 (QKV of 17 to 32 rows in several splits) a head is two XCDs', as its rotation
+// pairs are.  With rows on the XCDs instead (row modulo 8, or any) the products that write the
+// same parts next were slower, the launches themselves faster.  In us under the profiler, rows
+// / columns, 20, 45, 80 and 128 rows: 6144 x 4096 11.0 12.7 15.2 17.2 / 11.0 11.4 13.5 14.8 and
+// rotary 4.0 4.1 4.6 5.3 / 4.7 4.6 4.6 4.8; 4096 x 4096 8.3 9.4 13.1 15.1 / 8.2 9.0 10.5 12.2
+// and its residual 2.8 4.0 4.1 4.8 / 4.0 4.7 4.8 4.8; 4096 x 14336 and its residual level.  A
+// layer's four products with these, replayed: 17 rows 86.0 / 85.4, 32 89.3 / 88.7, 45 94.8 /
+// 92.9, 64 99.2 / 97.2, 80 110.8 / 105.6, 128 125.8 / 121.9.
 
 // The parts' sum + rotary positions + page append: grid (8, M, heads / 64), every eighth head
 // a wave, a rotation (or value) pair per lane.

@@ -1092,7 +1092,9 @@ __device__ __forceinline__ ScanRows scan_sequence(const i32* __restrict__ cu, in
 // of two waves and then their staging (28 vector instructions each and a quarter); so it is
 // the arithmetic of one, beside the staging: 140 -> 100 ns a token with decays per channel,
 // 124 -> 87 with one per head.  Every column is staged for twice as often, which costs where
-// the chip is full.  (All four waves of 16 columns staging 267 -> 226 us.)
+// the chip is full.  (All four waves of 16 columns staging 267 -> 226 us.)  One loop holds both
+// roles, and the registers of both: in bf16 with decays per channel 18 more than the 128 of RP
+// = 8 (68 bytes of scratch a lane), elsewhere none.
 template <typename S, int RP, bool ZL, int NT, int COLS>
 __global__ void __launch_bounds__(NT, RP == 8 && sizeof(S) == 2 ? (NT == 512 ? 4 : 3) : 2)
 linear_scan_prompt_kernel(
@@ -1601,8 +1603,8 @@ static int launch_scan(float* out, float* state, const void* q, const void* k,
                                               T >= 128 * B)));
   const bool prompt = eight || loads(256);
   // Half of eight waves staging for the other half, 16 columns to a workgroup, where the
-  // longest sequences decide: up to a workgroup per CU of these, or three where the caller
-  // knows them to be uneven.  All waves staging / apart in us: one sequence of 1900 tokens, 8
+  // longest sequences decide: up to a workgroup per CU of these, or three (of which two are
+  // there at once) where the caller knows them to be uneven.  All waves staging / apart in us: one sequence of 1900 tokens, 8
   // heads of 128 x 128 with decays per channel 267 / 190, 16 heads, one decay per head 235 /
   // 165; 4 of 300..700, 4 heads of 64 x 64 79 / 47, 8 of 256 x 256 222 / 158, in fp32 8 of 128
   // x 128 161 / 135; 3 of 58..82 19.2 / 18.2, but 4 of 49..58 16.2 / 16.7.  6 of 500..1900,

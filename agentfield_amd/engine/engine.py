@@ -36,9 +36,10 @@ def _bucket_for(n: int, max_bs: int) -> int:
 def choose_nsplit(bs: int, hk: int) -> int:
     """Decode attention split-K factor: about 512 workgroups, two per CU,
     whose waves keep enough K/V in flight.  Measured, 8 K/V heads: 64 sequences
-    of 545 tokens 28.3 us unsplit (31.8 in two), 8 of 300..3000 20.9 us in 8
-    (21.1 in 4, 23.4 in 16), 24 of 1800..8100 108 us in 2 (158 unsplit, 105 in
-    4 or 8, 111 in 16)."""
+    of 545 tokens 27.3 us unsplit (29.0 in two), 8 of 300..3000 19.7 us in 8
+    (20.2 in 4, 20.1 in 16), 24 of 1800..8100 83 us in 2 (134 unsplit, 85 in
+    4, 90 in 8, 86 in 16), 9 of 1600..8000 41 in 4 (62 in 2, 42 in 8); two to
+    four parts with the step's cut, which makes shares of these."""
     target = 512
     ns = max(1, min(16, target // max(1, bs * hk)))
     return 1 << (ns.bit_length() - 1)
